@@ -136,8 +136,8 @@ size_t mi355_mul_mat_q_ws_bytes(int64_t N, int64_t K, int64_t B);
 int mi355_mul_mat_q_ws(void *stream, int type, const void *W, const void *act, float *dst, int64_t N, int64_t K, int64_t B,
                        int64_t dst_stride, void *ws, size_t ws_bytes);
 
-/* MUL_MAT for 1..32 activation rows as one weight-streaming launch on the int8 matrix cores (every weight type; K a
- * multiple of 256; 16-byte aligned rows: mi355_mul_mat_skinny_supported says whether a product qualifies).  Same operands
+/* MUL_MAT for 1..32 activation rows as one weight-streaming launch on the int8 matrix cores (every weight type and K, the
+ * matrix at an even address: mi355_mul_mat_skinny_supported says whether a product qualifies).  Same operands
  * as mi355_mul_mat_vec_q (`act` from mi355_quantize_act) plus an optional residual added to the result (may alias dst).
  * It is what mi355_mul_mat uses between the batch-1 kernels and the tile kernels (ggml's MUL_MAT with src1->ne[1] of
  * 5..32, ggml_compute_forward_mul_mat, ggml/src/ggml-cpu/ggml-cpu.c:7380-7560).  `ws` of mi355_mul_mat_skinny_ws_bytes
@@ -329,10 +329,10 @@ int mi355_mul_mat_id_q8k(void *stream, int type, const void *as, const void *act
                          int64_t N, int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T, void *route_ws,
                          size_t route_ws_bytes);
 
-/* The same for experts of the per-32-block types (Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL, Q8_0): the routed form of mi355_mul_mat_q's tile
- * kernel on 128-slot column tiles.  `act` holds the nb1*T rows of b in the mi355_quantize_act (Q8_1) layout; route_ws as above.
- * K a multiple of 128, expert rows 16-byte aligned, at most 256 experts (mi355_mul_mat_id_q_supported); mi355_mul_mat_id picks
- * this path from 32 slots on. */
+/* The same for experts of the per-32-block types (Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL, Q8_0) and, at the precision of Q8_1 activations, of
+ * Q6_K and IQ4_XS: the routed form of mi355_mul_mat_q's tile kernel on 128-slot column tiles.  `act` holds the nb1*T rows of b in the mi355_quantize_act (Q8_1) layout; route_ws as above.
+ * K a multiple of the block size, the stack at an even address, at most 256 experts (mi355_mul_mat_id_q_supported);
+ * mi355_mul_mat_id picks this path from 32 slots on (Q6_K and IQ4_XS: where their rows are no multiple of 16 bytes). */
 int mi355_mul_mat_id_q_supported(int type, const void *as, int64_t N, int64_t K, int64_t n_expert);
 int mi355_mul_mat_id_q(void *stream, int type, const void *as, const void *act, const int32_t *ids, int64_t ids_stride, float *dst,
                        int64_t N, int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T, void *route_ws,

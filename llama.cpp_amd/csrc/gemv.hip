@@ -525,7 +525,7 @@ __global__ void __launch_bounds__(256) k_gemv_id(const uint8_t *__restrict__ as,
     gemv_body<TYPE, 1, RPW, false, false, LDSA>(m, blockIdx.x, aq + arow * K, ads + arow * (K >> 5), K, nullptr, s_act_dyn);
 }
 
-// Same routing for weight rows that are not 16-byte aligned (byte loads): one wave per (row, slot).
+// Same routing for expert stacks at an odd address (byte loads): one wave per (row, slot).
 template <int TYPE>
 __global__ void __launch_bounds__(64) k_gemv_id_unaligned(const uint8_t *__restrict__ as, const int8_t *__restrict__ aq,
                                                           const act_ds *__restrict__ ads, const int32_t *__restrict__ ids,
@@ -676,23 +676,19 @@ int mi355_mul_mat_vec_q_multi(void *stream, int n_mats, const mi355_gemv_mat *ma
     MI355_REQUIRE(B >= 1 && B <= 32, "mul_mat_vec_q: batch %lld outside 1..32", (long long)B);
     MI355_REQUIRE(((uintptr_t)act & 15) == 0, "mul_mat_vec_q: activation workspace is not 16-byte aligned");
     int64_t total_rows = 0;
-    bool aligned = true;
+    bool loadable = true;
     for (int i = 0; i < n_mats; i++) {
-        MI355_REQUIRE(is_weight_type(mats[i].type) && K > 0 && K % type_block_elems(mats[i].type) == 0, "mul_mat_vec_q: unsupported type %d or K=%lld not a multiple of its block size", mats[i].type, (long long)K);
-        aligned = aligned && layout_aligned(mats[i].W, make_row_layout(mats[i].type, K));
+        MI355_REQUIRE(is_weight_type(mats[i].type) && K > 0 && K < (int64_t(1) << 30) && K % type_block_elems(mats[i].type) == 0, "mul_mat_vec_q: unsupported type %d or K=%lld not a multiple of its block size", mats[i].type, (long long)K);
+        MI355_REQUIRE(mats[i].N > 0 && mats[i].dst_stride >= mats[i].N, "mul_mat_vec_q: bad shape");
+        loadable = loadable && layout_loadable(mats[i].W);
+        total_rows += mats[i].N;
     }
-    if (!aligned) {   // tiny / odd shapes only: byte-load kernel, one matrix at a time
+    if (!loadable) {   // a matrix at an odd address: byte-load kernel, one matrix at a time
         for (int i = 0; i < n_mats; i++) {
-            MI355_REQUIRE(mats[i].N > 0 && mats[i].dst_stride >= mats[i].N, "mul_mat_vec_q: bad shape");
             int rc = gemv_unaligned((hipStream_t)stream, mats[i].type, mats[i].W, act, mats[i].dst, mats[i].residual, mats[i].N, K, B, mats[i].dst_stride);
             if (rc != MI355_OK) return rc;
         }
         return MI355_OK;
-    }
-    for (int i = 0; i < n_mats; i++) {
-        int rc = check_gemv_args("mul_mat_vec_q", mats[i].type, mats[i].W, mats[i].N, K, mats[i].dst_stride);
-        if (rc != MI355_OK) return rc;
-        total_rows += mats[i].N;
     }
     // From five activation rows on the matrix-core kernel (skinny.hip) is ahead wherever it supports the product; a single
     // Q4_0/Q8_0/Q4_K matrix already at four (14336 x 4096 Q4_K: 14.3 -> 12.0 us, 4096 x 14336: 18.0 -> 14.6 us).
@@ -707,7 +703,7 @@ int mi355_mul_mat_vec_q_multi(void *stream, int n_mats, const mi355_gemv_mat *ma
             return MI355_OK;
         }
     }
-    MI355_REQUIRE(B <= 8, "mul_mat_vec_q: batch %lld needs the matrix-core kernel, which does not support this product (K a multiple of 256, aligned rows)", (long long)B);
+    MI355_REQUIRE(B <= 8, "mul_mat_vec_q: batch %lld needs the matrix-core kernel, which does not support this product", (long long)B);
     int rpw = pick_rpw(total_rows);
     if (B > 4 && rpw > 2) rpw = 2;   // keep the accumulator tile in registers
     {   // per-type corrections, measured on the 8B shapes
@@ -988,7 +984,7 @@ int mi355_mul_mat_id_vec(void *stream, int type, const void *as, const void *act
     hipStream_t s = (hipStream_t)stream;
     const int8_t *aq = (const int8_t *)act;
     const act_ds *ads = (const act_ds *)(aq + nb1 * T * K);
-    if (!layout_aligned(as, L)) {
+    if (!layout_loadable(as)) {
         const dim3 ugrid((unsigned)N, (unsigned)(n_used * T));
 #define MI355_ID_UNALIGNED_LAUNCH(TY) MI355_LAUNCH(k_gemv_id_unaligned<TY>, ugrid, dim3(64), 0, s, (const uint8_t *)as, aq, ads, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, L);
         MI355_WEIGHT_TYPE_SWITCH(type, MI355_ID_UNALIGNED_LAUNCH)

@@ -14,10 +14,9 @@
 //   Q8_0 : level as int8, scale d
 //   Q5_0 : level - 16 as int8, scale d;  IQ4_NL : the table value of the nibble as int8, scale d
 //   IQ4_XS : as IQ4_NL, scale d * (ls - 32) from the super-block's header
-//   Q4_1, Q5_1 : level 0..15 / 0..31 as int8, scale d; the "+ m * d_x * sum(q)" term of the stage's four blocks is added with one
-//          v_mfma_f32_32x32x16_f16 on (fp16 dx*sum(q), the reference's `s` field of block_q8_1) x (fp16 m)
-//   Q4_K, Q5_K : level 0..15 / 0..31 as int8, scale d*sc; the "- dmin*m*sum(q)" term of all blocks is
-//          added with one v_mfma_f32_32x32x16_f16 per stage on (fp16 dx*sum(q)) x (fp16 dmin*m)
+//   Q4_1, Q5_1 : level 0..15 / 0..31 as int8, scale d; the "+ m * d_x * sum(q)" term of the stage's four blocks is added with two
+//          v_mfma_f32_32x32x2_f32 on (dx * sum(q)) x m
+//   Q4_K, Q5_K : level 0..15 / 0..31 as int8, scale d*sc; the "- dmin*m*sum(q)" term of the blocks the same way
 //   Q6_K : level - 32 as int8, scale d*sc per 16 elements (v_mfma_i32_32x32x16_i8, two per block)
 //
 // MFMA operand mapping used here (A = activations, B = weights, D[i][j], i = activation
@@ -47,54 +46,18 @@ template <int TYPE> struct mmq_cfg {
     // 16 bytes of nibbles per block with a per-block scale: one request / commit form serves them all
     static constexpr bool NIBBLE32 = TYPE == MI355_Q4_0 || TYPE == MI355_Q4_1 || TYPE == MI355_Q5_0 || TYPE == MI355_Q5_1 || TYPE == MI355_IQ4_NL ||
                                      TYPE == MI355_IQ4_XS;
-    static constexpr bool PREFETCH = NIBBLE32 || TYPE == MI355_Q8_0;
+    static constexpr bool PREFETCH = NIBBLE32 || TYPE == MI355_Q8_0 || TYPE == MI355_Q6_K;
 };
 
 // ---- stage loaders: global (device layout) -> int8 rows + scales in LDS ----------------
 // sW  : int8 [MMQ_BM][MMQ_LDK]
 // sWs : float [NG][MMQ_BM]   (scale g of row r at sWs[g*MMQ_BM + r])
-// sWo : fp16  [MMQ_BM][4]    (Q4_K only: dmin*m of the 4 sub-blocks of the stage)
+// sWo : float [4][MMQ_BM]    (types with a block minimum: what multiplies d_x * sum(q) of the stage's 4 blocks)
 template <int TYPE>
 __device__ __forceinline__ void load_weight_stage(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0,
-                                                  int64_t N, int64_t k0, int8_t *sW, float *sWs, _Float16 *sWo) {
+                                                  int64_t N, int64_t k0, int8_t *sW, float *sWs, float *sWo) {
     const int tid = threadIdx.x;
-    if constexpr (TYPE == MI355_Q4_0) {
-        // 128 rows x 4 blocks of 16 B
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 2, b = idx & 3;
-            const int64_t row = row0 + r < N ? row0 + r : N - 1;
-            const uint8_t *wrow = W + row * L.row_bytes;
-            const int64_t blk = (k0 >> 5) + b;
-            const u32x4 q = load16(wrow + blk * 16);
-            u32x4 lo, hi;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                // nibble - 8 per byte without cross-byte borrow
-                lo[i] = (((q[i] & 0x0F0F0F0Fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-                hi[i] = ((((q[i] >> 4) & 0x0F0F0F0Fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-            }
-            *(u32x4 *)(sW + r * MMQ_LDK + b * 32) = lo;
-            *(u32x4 *)(sW + r * MMQ_LDK + b * 32 + 16) = hi;
-            sWs[b * MMQ_BM + r] = half_bits_to_float(*(const unsigned short *)(wrow + L.off_b + blk * 2));
-        }
-    } else if constexpr (TYPE == MI355_Q8_0) {
-        // 128 rows x 4 blocks x 2 halves of 16 B
-#pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 3, c = idx & 7;   // c: 16-byte piece of the stage
-            const int64_t row = row0 + r < N ? row0 + r : N - 1;
-            const uint8_t *wrow = W + row * L.row_bytes;
-            const u32x4 q = load16(wrow + k0 + c * 16);
-            *(u32x4 *)(sW + r * MMQ_LDK + c * 16) = q;
-            if ((c & 1) == 0) {
-                const int b = c >> 1;
-                sWs[b * MMQ_BM + r] = half_bits_to_float(*(const unsigned short *)(wrow + L.off_b + ((k0 >> 5) + b) * 2));
-            }
-        }
-    } else if constexpr (TYPE == MI355_Q4_K || TYPE == MI355_Q5_K) {
+    {
         // stage = half a super-block: sub-blocks j0..j0+3, 64 B of qs per row = 4 pieces of 16 B (Q5_K: bit j of qh[l] is the fifth
         // bit of element l of sub-block j, dequantize_row_q5_K, ggml/src/ggml-quants.c:1482-1507)
         constexpr int BB = TYPE == MI355_Q4_K ? Q4_K_BYTES : Q5_K_BYTES, QS = TYPE == MI355_Q4_K ? 16 : 48;
@@ -107,7 +70,7 @@ __device__ __forceinline__ void load_weight_stage(const uint8_t *__restrict__ W,
             const int gl = p >> 1, h = p & 1;
             const int64_t row = row0 + r < N ? row0 + r : N - 1;
             const uint8_t *blk = W + row * L.row_bytes + sb * BB;
-            const u32x4 q = load16(blk + QS + (half * 2 + gl) * 32 + h * 16);
+            const u32x4 q = load16w(blk + QS + (half * 2 + gl) * 32 + h * 16);
             u32x4 lo, hi;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -115,7 +78,7 @@ __device__ __forceinline__ void load_weight_stage(const uint8_t *__restrict__ W,
                 hi[i] = (q[i] >> 4) & 0x0F0F0F0Fu;
             }
             if constexpr (TYPE == MI355_Q5_K) {
-                const u32x4 qh = load16(blk + 16 + h * 16);
+                const u32x4 qh = load16w(blk + 16 + h * 16);
                 const int ja = half * 4 + 2 * gl;         // sub-block of the low nibbles; the high nibbles are the next one
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
@@ -126,53 +89,22 @@ __device__ __forceinline__ void load_weight_stage(const uint8_t *__restrict__ W,
             *(u32x4 *)(sW + r * MMQ_LDK + (2 * gl) * 32 + h * 16) = lo;
             *(u32x4 *)(sW + r * MMQ_LDK + (2 * gl + 1) * 32 + h * 16) = hi;
             // this thread also owns the (scale, min) of sub-block p of the stage
-            const u32x4 hdr = load16(blk);
+            const u32x4 hdr = load16w(blk);
             const float d = half_bits_to_float((unsigned short)(hdr[0] & 0xFFFFu));
             const float dmin = half_bits_to_float((unsigned short)(hdr[0] >> 16));
             int sc, mn;
             q4k_scale_min(hdr[1], hdr[2], hdr[3], half * 4 + p, sc, mn);
             sWs[p * MMQ_BM + r] = d * (float)sc;
-            sWo[r * 4 + p] = (_Float16)(dmin * (float)mn);
-        }
-    } else {   // Q6_K: stage = half hf of a super-block: 64 B ql + 32 B qh, 8 scales
-        const int64_t sb = k0 >> 8;
-        const int hf = (int)((k0 >> 7) & 1);
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 2, p = idx & 3;          // p: 16-byte piece of this half's ql
-            const int l0 = 16 * (p & 1), qa = p >> 1;
-            const int64_t row = row0 + r < N ? row0 + r : N - 1;
-            const uint8_t *wrow = W + row * L.row_bytes;
-            const u32x4 ql = load16(wrow + sb * 128 + hf * 64 + p * 16);
-            const u32x4 qh = load16(wrow + L.off_b + sb * 64 + hf * 32 + l0);
-            u32x4 vA, vB;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const u32 a = (ql[i] & 0x0F0F0F0Fu) | (((qh[i] >> (2 * qa)) & 0x03030303u) << 4);
-                const u32 b = ((ql[i] >> 4) & 0x0F0F0F0Fu) | (((qh[i] >> (2 * qa + 4)) & 0x03030303u) << 4);
-                // level - 32 per byte: flip bit 5, then sign-extend it into bits 6..7
-                const u32 ta = a ^ 0x20202020u, tb = b ^ 0x20202020u;
-                const u32 ma = ta & 0x20202020u, mb = tb & 0x20202020u;
-                vA[i] = ta | (ma << 1) | (ma << 2);
-                vB[i] = tb | (mb << 1) | (mb << 2);
-            }
-            *(u32x4 *)(sW + r * MMQ_LDK + qa * 32 + l0) = vA;
-            *(u32x4 *)(sW + r * MMQ_LDK + (qa + 2) * 32 + l0) = vB;
-            // scales of 16-element groups 2p and 2p+1 of the stage
-            const float d = half_bits_to_float(*(const unsigned short *)(wrow + L.off_d + sb * 2));
-            const int8_t *sc = (const int8_t *)(wrow + L.off_c + sb * 16 + hf * 8);
-            sWs[(2 * p) * MMQ_BM + r] = d * (float)sc[2 * p];
-            sWs[(2 * p + 1) * MMQ_BM + r] = d * (float)sc[2 * p + 1];
+            sWo[p * MMQ_BM + r] = -(dmin * (float)mn);
         }
     }
 }
 
-// sA  : int8 [BN][MMQ_LDK];  sAd : float [4][BN] block scales;  sAs : fp16 [BN][4]  dx*sum(q) (Q4_K)
+// sA  : int8 [BN][MMQ_LDK];  sAd : float [4][BN] block scales;  sAs : float [4][BN]  dx*sum(q) (types with a block minimum)
 template <int TYPE, int BN>
 __device__ __forceinline__ void load_act_stage(const int8_t *__restrict__ aq, const act_ds *__restrict__ ads,
                                                int64_t col0, int64_t B, int64_t K, int64_t k0, int8_t *sA, float *sAd,
-                                               _Float16 *sAs) {
+                                               float *sAs) {
     const int tid = threadIdx.x;
     const int64_t nblk = K >> 5;
     // BN rows x 8 pieces of 16 B
@@ -192,13 +124,13 @@ __device__ __forceinline__ void load_act_stage(const int8_t *__restrict__ aq, co
             const int64_t col = col0 + r < B ? col0 + r : B - 1;
             const act_ds s = ads[col * nblk + (k0 >> 5) + b];
             sAd[b * BN + r] = s.d;
-            if constexpr (TYPE == MI355_Q4_K || TYPE == MI355_Q5_K) sAs[r * 4 + b] = (_Float16)(s.d * (float)s.sum);
+            if constexpr (TYPE == MI355_Q4_K || TYPE == MI355_Q5_K) sAs[b * BN + r] = s.d * (float)s.sum;
         }
     }
 }
 
 // ---- the same stages split into "request" (global -> registers) and "commit" (unpack -> LDS), so that the next stage's bytes
-// travel while the current stage is contracted (Q4_0 / Q8_0, whose per-32 scales keep them on this kernel)
+// travel while the current stage is contracted (all types but Q4_K and Q5_K, whose batches run on the super-block kernels)
 template <int TYPE, bool NIB = mmq_cfg<TYPE>::NIBBLE32> struct mmq_wregs {};
 // Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL, IQ4_XS: thread t owns blocks (row, b) = (idx >> 2, idx & 3), idx = t and t + 256
 template <int TYPE> struct mmq_wregs<TYPE, true> {
@@ -207,25 +139,28 @@ template <int TYPE> struct mmq_wregs<TYPE, true> {
     u32x4 q[2];
     u32 qh[2];
     u32 dm[2];   // fp16 d in the low half, fp16 m above it (HAS_MIN); IQ4_XS: the bits of the f32 block scale
-    __device__ __forceinline__ void fetch(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int64_t k0, int tid) {
+    __device__ __forceinline__ void fetch(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int64_t k0, int64_t nblk, int tid) {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
             const int idx = tid + it * 256;
             const int r = idx >> 2, b = idx & 3;
             const int64_t row = row0 + r < N ? row0 + r : N - 1;
             const uint8_t *wrow = W + row * L.row_bytes;
-            const int64_t blk = (k0 >> 5) + b;
-            q[it] = load16(wrow + blk * 16);
-            if constexpr (HAS_QH) qh[it] = *(const u32 *)(wrow + L.off_b + blk * 4);
+            int64_t blk = (k0 >> 5) + b;
+            const bool live = blk < nblk;   // K is a multiple of 32: the last stage may hold fewer than four blocks
+            blk = live ? blk : nblk - 1;
+            q[it] = load16w(wrow + blk * 16);
+            if constexpr (HAS_QH) qh[it] = load4w(wrow + L.off_b + blk * 4);
             const int so = HAS_QH ? L.off_c : L.off_b;   // the scales follow the fifth bits where there are any
             if constexpr (TYPE == MI355_IQ4_XS) {
-                const uint2 h = *(const uint2 *)(wrow + L.off_b + (blk >> 3) * 8);
-                dm[it] = __builtin_bit_cast(u32, iq4xs_block_scale(h.x, h.y, (int)(blk & 7)));
-            } else if constexpr (HAS_MIN) dm[it] = *(const u32 *)(wrow + so + blk * 4);
+                const u32x2 h = load8w(wrow + L.off_b + (blk >> 3) * 8);
+                dm[it] = __builtin_bit_cast(u32, iq4xs_block_scale(h[0], h[1], (int)(blk & 7)));
+            } else if constexpr (HAS_MIN) dm[it] = load4w(wrow + so + blk * 4);
             else dm[it] = *(const unsigned short *)(wrow + so + blk * 2);
+            if (!live) dm[it] = 0;          // scale (and minimum) 0: the block adds nothing
         }
     }
-    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, _Float16 *sWo, int tid) const {
+    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *sWo, int tid) const {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
             const int idx = tid + it * 256;
@@ -255,35 +190,79 @@ template <int TYPE> struct mmq_wregs<TYPE, true> {
             *(u32x4 *)(sW + r * MMQ_LDK + b * 32 + 16) = hi;
             if constexpr (TYPE == MI355_IQ4_XS) sWs[b * MMQ_BM + r] = __builtin_bit_cast(float, dm[it]);
             else sWs[b * MMQ_BM + r] = half_bits_to_float((unsigned short)(dm[it] & 0xFFFFu));
-            if constexpr (HAS_MIN) {
-                union { unsigned short u; _Float16 f; } m;
-                m.u = (unsigned short)(dm[it] >> 16);
-                sWo[r * 4 + b] = m.f;
-            }
+            if constexpr (HAS_MIN) sWo[b * MMQ_BM + r] = half_bits_to_float((unsigned short)(dm[it] >> 16));
         }
     }
 };
 template <> struct mmq_wregs<MI355_Q8_0, false> {
     u32x4 q[4];
     unsigned short d[4];
-    __device__ __forceinline__ void fetch(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int64_t k0, int tid) {
+    __device__ __forceinline__ void fetch(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int64_t k0, int64_t nblk, int tid) {
 #pragma unroll
         for (int it = 0; it < 4; it++) {
             const int idx = tid + it * 256;
             const int r = idx >> 3, c = idx & 7;   // c: 16-byte piece of the stage
             const int64_t row = row0 + r < N ? row0 + r : N - 1;
             const uint8_t *wrow = W + row * L.row_bytes;
-            q[it] = load16(wrow + k0 + c * 16);
-            d[it] = *(const unsigned short *)(wrow + L.off_b + ((k0 >> 5) + (c >> 1)) * 2);   // both pieces of a block read its scale
+            int64_t blk = (k0 >> 5) + (c >> 1);   // both pieces of a block read its scale
+            const bool live = blk < nblk;
+            blk = live ? blk : nblk - 1;
+            q[it] = load16w(wrow + blk * 32 + (c & 1) * 16);
+            d[it] = *(const unsigned short *)(wrow + L.off_b + blk * 2);
+            if (!live) d[it] = 0;
         }
     }
-    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, _Float16 *, int tid) const {
+    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *, int tid) const {
 #pragma unroll
         for (int it = 0; it < 4; it++) {
             const int idx = tid + it * 256;
             const int r = idx >> 3, c = idx & 7;
             *(u32x4 *)(sW + r * MMQ_LDK + c * 16) = q[it];
             if ((c & 1) == 0) sWs[(c >> 1) * MMQ_BM + r] = half_bits_to_float(d[it]);
+        }
+    }
+};
+// stage = half hf of a super-block: 64 B of ql + 32 B of qh, 8 scales of 16 elements; thread t owns the 16-byte pieces (row, p) = (idx >> 2, idx & 3)
+template <> struct mmq_wregs<MI355_Q6_K, false> {
+    u32x4 ql[2], qh[2];
+    unsigned short d[2], sc[2];   // super-block scale; the int8 scales of groups 2p and 2p + 1
+    __device__ __forceinline__ void fetch(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int64_t k0, int64_t, int tid) {
+        const int64_t sb = k0 >> 8;
+        const int hf = (int)((k0 >> 7) & 1);
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int idx = tid + it * 256;
+            const int r = idx >> 2, p = idx & 3;
+            const int64_t row = row0 + r < N ? row0 + r : N - 1;
+            const uint8_t *wrow = W + row * L.row_bytes;
+            ql[it] = load16w(wrow + sb * 128 + hf * 64 + p * 16);
+            qh[it] = load16w(wrow + L.off_b + sb * 64 + hf * 32 + 16 * (p & 1));
+            sc[it] = *(const unsigned short *)(wrow + L.off_c + sb * 16 + hf * 8 + 2 * p);
+            d[it] = *(const unsigned short *)(wrow + L.off_d + sb * 2);
+        }
+    }
+    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *, int tid) const {
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int idx = tid + it * 256;
+            const int r = idx >> 2, p = idx & 3;
+            const int l0 = 16 * (p & 1), qa = p >> 1;
+            u32x4 vA, vB;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const u32 a = (ql[it][i] & 0x0F0F0F0Fu) | (((qh[it][i] >> (2 * qa)) & 0x03030303u) << 4);
+                const u32 b = ((ql[it][i] >> 4) & 0x0F0F0F0Fu) | (((qh[it][i] >> (2 * qa + 4)) & 0x03030303u) << 4);
+                // level - 32 per byte: flip bit 5, then sign-extend it into bits 6..7
+                const u32 ta = a ^ 0x20202020u, tb = b ^ 0x20202020u;
+                const u32 ma = ta & 0x20202020u, mb = tb & 0x20202020u;
+                vA[i] = ta | (ma << 1) | (ma << 2);
+                vB[i] = tb | (mb << 1) | (mb << 2);
+            }
+            *(u32x4 *)(sW + r * MMQ_LDK + qa * 32 + l0) = vA;
+            *(u32x4 *)(sW + r * MMQ_LDK + (qa + 2) * 32 + l0) = vB;
+            const float df = half_bits_to_float(d[it]);
+            sWs[(2 * p) * MMQ_BM + r] = df * (float)(int)(signed char)(sc[it] & 0xFFu);
+            sWs[(2 * p + 1) * MMQ_BM + r] = df * (float)(int)(signed char)(sc[it] >> 8);
         }
     }
 };
@@ -302,7 +281,8 @@ template <int BN, bool WITH_SUM> struct mmq_aregs {
             const int r = idx >> 3, c = idx & 7;
             int64_t col = col0 + r < B ? col0 + r : B - 1;
             if (row_of) col = row_of[col];
-            q[it] = load16(aq + col * K + k0 + c * 16);
+            const int64_t k = k0 + c * 16 < K ? k0 + c * 16 : K - 16;   // past the end: any bytes, the weight scales there are 0
+            q[it] = load16(aq + col * K + k);
         }
 #pragma unroll
         for (int it = 0; it < NS; it++) {
@@ -310,12 +290,13 @@ template <int BN, bool WITH_SUM> struct mmq_aregs {
             const int r = (idx >> 2) < BN ? (idx >> 2) : BN - 1, b = idx & 3;
             int64_t col = col0 + r < B ? col0 + r : B - 1;
             if (row_of) col = row_of[col];
-            const act_ds e = ads[col * nblk + (k0 >> 5) + b];
+            const int64_t blk = (k0 >> 5) + b < nblk ? (k0 >> 5) + b : nblk - 1;
+            const act_ds e = ads[col * nblk + blk];
             d[it] = e.d;
             if constexpr (WITH_SUM) sum[it] = e.sum;
         }
     }
-    __device__ __forceinline__ void commit(int8_t *sA, float *sAd, _Float16 *sAs, int tid) const {
+    __device__ __forceinline__ void commit(int8_t *sA, float *sAd, float *sAs, int tid) const {
 #pragma unroll
         for (int it = 0; it < NQ; it++) {
             const int idx = tid + it * 256;
@@ -327,7 +308,7 @@ template <int BN, bool WITH_SUM> struct mmq_aregs {
             const int idx = tid + it * 256;
             if (idx < BN * 4) {
                 sAd[(idx & 3) * BN + (idx >> 2)] = d[it];
-                if constexpr (WITH_SUM) sAs[idx] = (_Float16)(d[it] * (float)sum[it]);   // [row][block of the stage]
+                if constexpr (WITH_SUM) sAs[(idx & 3) * BN + (idx >> 2)] = d[it] * (float)sum[it];
             }
         }
     }
@@ -349,14 +330,14 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
                                              int64_t K, int64_t B, int64_t dst_stride, row_layout L, int n_col_tiles,
                                              int n_groups, int n_groups_padded, mmq32_route route) {
     typedef mmq_cfg<TYPE> C;
-    static_assert(!ID || C::PREFETCH, "the routed form exists for the per-32-block types");
+    static_assert(!ID || C::PREFETCH, "the routed form gathers activation rows in the register-staged loads");
     constexpr int BN = 64 * TN;
     __shared__ __attribute__((aligned(16))) int8_t sW[MMQ_BM * MMQ_LDK];
     __shared__ __attribute__((aligned(16))) int8_t sA[BN * MMQ_LDK];
     __shared__ __attribute__((aligned(16))) float sWs[C::NG * MMQ_BM];
     __shared__ __attribute__((aligned(16))) float sAd[4 * BN];
-    __shared__ __attribute__((aligned(16))) _Float16 sWo[C::MIN ? MMQ_BM * 4 : 4];
-    __shared__ __attribute__((aligned(16))) _Float16 sAs[C::MIN ? BN * 4 : 4];
+    __shared__ __attribute__((aligned(16))) float sWo[C::MIN ? MMQ_BM * 4 : 4];
+    __shared__ __attribute__((aligned(16))) float sAs[C::MIN ? BN * 4 : 4];
 
     // XCD-aware id: hardware deals group ids round-robin over 8 XCDs; make logical neighbours share an XCD
     const int per_xcd = n_groups_padded >> 3;
@@ -388,7 +369,7 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
             for (int r = 0; r < 16; r++) acc[tb][tw][r] = 0.0f;
 
     // split K: grid row y walks stages [k_lo, k_hi) and writes its sums to slice y of `dst` (a workspace then, see launch_mmq)
-    const int64_t stages = K / MMQ_BK, st_per = (stages + gridDim.y - 1) / gridDim.y;
+    const int64_t nblk = K >> 5, stages = (K + MMQ_BK - 1) / MMQ_BK, st_per = (stages + gridDim.y - 1) / gridDim.y;
     const int64_t k_lo = (int64_t)blockIdx.y * st_per * MMQ_BK;
     const int64_t k_hi = k_lo + st_per * MMQ_BK < K ? k_lo + st_per * MMQ_BK : K;
     if (gridDim.y > 1) dst += (int64_t)blockIdx.y * B * dst_stride;
@@ -397,7 +378,7 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
     mmq_wregs<TYPE> wregs;
     mmq_aregs<BN, C::MIN> aregs;
     if constexpr (PREFETCH) {
-        wregs.fetch(W, L, row0, N, k_lo, threadIdx.x);
+        wregs.fetch(W, L, row0, N, k_lo, nblk, threadIdx.x);
         aregs.fetch(aq, ads, col0, B, K, k_lo, threadIdx.x, row_of);
     }
     for (int64_t k0 = k_lo; k0 < k_hi; k0 += MMQ_BK) {
@@ -413,7 +394,7 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
         if constexpr (PREFETCH) {
             // past the end the last stage is requested again and never committed: no branch, the loads stay here
             const int64_t k1 = k0 + MMQ_BK < k_hi ? k0 + MMQ_BK : k0;
-            wregs.fetch(W, L, row0, N, k1, threadIdx.x);
+            wregs.fetch(W, L, row0, N, k1, nblk, threadIdx.x);
             aregs.fetch(aq, ads, col0, B, K, k1, threadIdx.x, row_of);
             __builtin_amdgcn_sched_barrier(0);   // requested now, a whole stage ahead of their commit
         }
@@ -472,25 +453,21 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
         }
 
         if constexpr (C::MIN) {
-            // acc -= sum_b (dx*sum q)[i][b] * (dmin*m)[j][b] over the 4 blocks of the stage (Q4_K; Q4_1 and Q5_1: acc += ... * m[j][b]):
-            // a 32x32x16 f16 MFMA whose k slots 0..3 hold the blocks (lanes 32..63 and slots 4..7 are zero)
-            f16x8 af[TN], bf[2];
+            // acc += sum_b (dx * sum q)[i][b] * m[j][b] over the 4 blocks of the stage (Q4_K, Q5_K: m = -dmin * 6-bit minimum): two
+            // v_mfma_f32_32x32x2_f32 per tile on the matrix pipe, which waits for the vector ALUs anyway; k = lane / 32.  In f32 as the
+            // batch-1 kernels do it (as f16 operands the term carried 3.6e-4 of the result).
 #pragma unroll
-            for (int tb = 0; tb < TN; tb++) {
-                const f16x4 v = *(const f16x4 *)(sAs + (wcol0 + tb * 32 + l32) * 4);
+            for (int p = 0; p < 2; p++) {
+                float af[TN], bf[2];
 #pragma unroll
-                for (int i = 0; i < 8; i++) af[tb][i] = (i < 4 && lhi == 0) ? (TYPE == MI355_Q4_K || TYPE == MI355_Q5_K ? (_Float16)(-(float)v[i & 3]) : v[i & 3]) : (_Float16)0.0f;
+                for (int tb = 0; tb < TN; tb++) af[tb] = sAs[(2 * p + lhi) * BN + wcol0 + tb * 32 + l32];
+#pragma unroll
+                for (int tw = 0; tw < 2; tw++) bf[tw] = sWo[(2 * p + lhi) * MMQ_BM + wrow0 + tw * 32 + l32];
+#pragma unroll
+                for (int tb = 0; tb < TN; tb++)
+#pragma unroll
+                    for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
             }
-#pragma unroll
-            for (int tw = 0; tw < 2; tw++) {
-                const f16x4 v = *(const f16x4 *)(sWo + (wrow0 + tw * 32 + l32) * 4);
-#pragma unroll
-                for (int i = 0; i < 8; i++) bf[tw][i] = (i < 4 && lhi == 0) ? v[i & 3] : (_Float16)0.0f;
-            }
-#pragma unroll
-            for (int tb = 0; tb < TN; tb++)
-#pragma unroll
-                for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
         }
     }
 
@@ -513,7 +490,7 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
 // eight slices, at most two groups per compute unit.
 static int mmq_slices(int64_t N, int64_t K, int64_t B) {
     const int64_t bn = B <= 64 ? 64 : 128;
-    const int64_t groups = ((N + MMQ_BM - 1) / MMQ_BM) * ((B + bn - 1) / bn), stages = K / MMQ_BK;
+    const int64_t groups = ((N + MMQ_BM - 1) / MMQ_BM) * ((B + bn - 1) / bn), stages = (K + MMQ_BK - 1) / MMQ_BK;
     int64_t n = 512 / groups;
     if (n > stages / 4) n = stages / 4;
     if (n > 8) n = 8;
@@ -587,10 +564,10 @@ static void launch_mmq_id(hipStream_t s, const void *as, const void *act, int64_
 using namespace mi355;
 
 extern "C" int mi355_mul_mat_id_q_supported(int type, const void *as, int64_t N, int64_t K, int64_t n_expert) {
-    const bool typed = type == MI355_Q4_0 || type == MI355_Q4_1 || type == MI355_Q5_0 || type == MI355_Q5_1 || type == MI355_IQ4_NL || type == MI355_Q8_0;
-    if (!typed || N <= 0 || K <= 0 || K % MMQ_BK != 0 || n_expert <= 0 || n_expert > 256) return 0;
-    const row_layout L = make_row_layout(type, K);
-    return layout_aligned(as, L) && (N * L.row_bytes) % 16 == 0 ? 1 : 0;
+    const bool typed = type == MI355_Q4_0 || type == MI355_Q4_1 || type == MI355_Q5_0 || type == MI355_Q5_1 || type == MI355_IQ4_NL ||
+                       type == MI355_Q8_0 || type == MI355_Q6_K || type == MI355_IQ4_XS;
+    if (!typed || N <= 0 || K <= 0 || K % type_block_elems(type) != 0 || n_expert <= 0 || n_expert > 256) return 0;
+    return layout_loadable(as) ? 1 : 0;
 }
 
 extern "C" int mi355_mul_mat_id_q(void *stream, int type, const void *as, const void *act, const int32_t *ids, int64_t ids_stride, float *dst, int64_t N,
@@ -612,6 +589,8 @@ extern "C" int mi355_mul_mat_id_q(void *stream, int type, const void *as, const 
         case MI355_Q4_1: launch_mmq_id<MI355_Q4_1>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
         case MI355_Q5_0: launch_mmq_id<MI355_Q5_0>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
         case MI355_Q5_1: launch_mmq_id<MI355_Q5_1>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
+        case MI355_Q6_K: launch_mmq_id<MI355_Q6_K>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
+        case MI355_IQ4_XS: launch_mmq_id<MI355_IQ4_XS>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
         case MI355_IQ4_NL: launch_mmq_id<MI355_IQ4_NL>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
         default: launch_mmq_id<MI355_Q8_0>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
     }
@@ -619,7 +598,7 @@ extern "C" int mi355_mul_mat_id_q(void *stream, int type, const void *as, const 
 }
 
 extern "C" size_t mi355_mul_mat_q_ws_bytes(int64_t N, int64_t K, int64_t B) {
-    if (N <= 0 || K <= 0 || B <= 0 || K % MMQ_BK != 0) return 0;
+    if (N <= 0 || K <= 0 || B <= 0 || K % QK != 0) return 0;
     const int n = mmq_slices(N, K, B);
     return n > 1 ? (size_t)n * (size_t)N * (size_t)B * sizeof(float) : 0;
 }
@@ -635,8 +614,7 @@ extern "C" int mi355_mul_mat_q_ws(void *stream, int type, const void *W, const v
     MI355_REQUIRE(N > 0 && K > 0 && B > 0, "mul_mat_q: bad shape N=%lld K=%lld B=%lld", (long long)N, (long long)K, (long long)B);
     MI355_REQUIRE(K % type_block_elems(type) == 0, "mul_mat_q: K=%lld is not a multiple of the block size", (long long)K);
     MI355_REQUIRE(dst_stride >= N, "mul_mat_q: dst_stride < N");
-    const row_layout L = make_row_layout(type, K);
-    if (!layout_aligned(W, L) || K % MMQ_BK != 0)   // tiny / odd shapes only
+    if (!layout_loadable(W))   // a matrix at an odd address
         return gemv_unaligned((hipStream_t)stream, type, W, act, dst, nullptr, N, K, B, dst_stride);
     MI355_REQUIRE(((uintptr_t)act & 15) == 0, "mul_mat_q: activation workspace is not 16-byte aligned");
     MI355_REQUIRE((N + MMQ_BM - 1) / MMQ_BM * ((B + 63) / 64) < (1 << 30), "mul_mat_q: too many tiles");

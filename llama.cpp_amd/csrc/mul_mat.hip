@@ -1,6 +1,6 @@
 // MUL_MAT host entry: quantize activations on the device, then dispatch to the GEMV (few activation rows), the
 // weight-streaming matrix-core kernel (up to 32 rows) or the int8-MFMA tile kernels.  Also the byte-load fallback for
-// weight rows that are not 16-byte aligned.
+// weight matrices at an odd address.
 #include "common.hpp"
 #include "qdot.hpp"
 

@@ -43,7 +43,21 @@ __host__ inline bool layout_aligned(const void *W, const row_layout &L) {
     return ((uintptr_t)W & 15) == 0 && (L.row_bytes & 15) == 0 && (L.off_b & 15) == 0 && (L.off_c & 15) == 0;
 }
 
-// Byte-load GEMV for weight rows that are not 16-byte aligned, any batch (mul_mat.hip).
+// Rows whose length is no multiple of 16 bytes (Q6_K and IQ4_XS with an odd number of super-blocks, Q4_0 / Q5_x / Q8_0 with a number of
+// blocks that is no multiple of 8) start at any even address.  The weight loads below are typed for 2-byte alignment: global loads of 4
+// and 16 bytes need no more than that (the compiler emits the same global_load_dwordx4 for them), so every such row runs on the same
+// kernels as an aligned one.  Only a matrix at an odd address is left to the byte loads of gemv_unaligned.
+typedef u32 u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef u32 u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));   // two neighbouring {d, sum} pairs of an activation row
+typedef u32 u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef u32 u32_a2 __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 load16w(const void *p) { return *(const u32x4_a2 *)p; }
+__device__ __forceinline__ u32x4 load_stream16w(const void *p) { return __builtin_nontemporal_load((const u32x4_a2 *)p); }
+__device__ __forceinline__ u32x2 load8w(const void *p) { return *(const u32x2_a2 *)p; }
+__device__ __forceinline__ u32 load4w(const void *p) { return *(const u32_a2 *)p; }
+__host__ inline bool layout_loadable(const void *W) { return ((uintptr_t)W & 1) == 0; }
+
+// Byte-load GEMV for weight matrices at an odd address, any batch (mul_mat.hip).
 // act: split activation layout holding B rows of K; residual may be null or alias dst.
 int gemv_unaligned(hipStream_t s, int type, const void *W, const void *act, float *dst, const float *residual, int64_t N,
                    int64_t K, int64_t B, int64_t dst_stride);
@@ -79,7 +93,7 @@ template <> struct wq<MI355_Q4_0> {
     struct act { u32x4 a0, a1; float d; int sum; };
     static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &L, int c) {
         chunk w;
-        w.qs = load_stream16(row + c * 16);
+        w.qs = load_stream16w(row + c * 16);
         w.d = half_bits_to_float(*(const unsigned short *)(row + L.off_b + c * 2));
         return w;
     }
@@ -117,8 +131,8 @@ template <> struct wq<MI355_Q8_0> {
         chunk w;
         // the two loads of a wave interleave 16-byte pieces of the same 128-byte lines: a streaming
         // (non-temporal) hint would fetch each line from HBM twice, so these stay ordinary loads
-        w.q0 = load16(row + c * 32);
-        w.q1 = load16(row + c * 32 + 16);
+        w.q0 = load16w(row + c * 32);
+        w.q1 = load16w(row + c * 32 + 16);
         w.d = half_bits_to_float(*(const unsigned short *)(row + L.off_b + c * 2));
         return w;
     }
@@ -193,9 +207,9 @@ template <> struct wq<MI355_IQ4_XS> {
     typedef wq<MI355_Q8_0>::act act;
     static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &L, int c) {
         chunk w;
-        w.qs = load_stream16(row + c * 16);
-        const uint2 h = *(const uint2 *)(row + L.off_b + (c >> 3) * 8);   // the same eight bytes for the eight lanes of a super-block
-        w.d = iq4xs_block_scale(h.x, h.y, c & 7);
+        w.qs = load_stream16w(row + c * 16);
+        const u32x2 h = load8w(row + L.off_b + (c >> 3) * 8);   // the same eight bytes for the eight lanes of a super-block
+        w.d = iq4xs_block_scale(h[0], h[1], c & 7);
         return w;
     }
     static __device__ __forceinline__ act load_a(const int8_t *__restrict__ q, const act_ds *__restrict__ ds, int c) { return wq<MI355_Q8_0>::load_a(q, ds, c); }
@@ -218,8 +232,8 @@ template <> struct wq<MI355_Q4_1> {
     typedef wq<MI355_Q4_0>::act act;
     static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &L, int c) {
         chunk w;
-        w.qs = load_stream16(row + c * 16);
-        const u32 dm = *(const u32 *)(row + L.off_b + c * 4);
+        w.qs = load_stream16w(row + c * 16);
+        const u32 dm = load4w(row + L.off_b + c * 4);
         w.d = half_bits_to_float((unsigned short)(dm & 0xFFFFu));
         w.m = half_bits_to_float((unsigned short)(dm >> 16));
         return w;
@@ -246,8 +260,8 @@ template <> struct wq<MI355_Q5_0> {
     typedef wq<MI355_Q4_0>::act act;
     static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &L, int c) {
         chunk w;
-        w.qs = load_stream16(row + c * 16);
-        w.qh = *(const u32 *)(row + L.off_b + c * 4);
+        w.qs = load_stream16w(row + c * 16);
+        w.qh = load4w(row + L.off_b + c * 4);
         w.d = half_bits_to_float(*(const unsigned short *)(row + L.off_c + c * 2));
         return w;
     }
@@ -276,9 +290,9 @@ template <> struct wq<MI355_Q5_1> {
     typedef wq<MI355_Q4_0>::act act;
     static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &L, int c) {
         chunk w;
-        w.qs = load_stream16(row + c * 16);
-        w.qh = *(const u32 *)(row + L.off_b + c * 4);
-        const u32 dm = *(const u32 *)(row + L.off_c + c * 4);
+        w.qs = load_stream16w(row + c * 16);
+        w.qh = load4w(row + L.off_b + c * 4);
+        const u32 dm = load4w(row + L.off_c + c * 4);
         w.d = half_bits_to_float((unsigned short)(dm & 0xFFFFu));
         w.m = half_bits_to_float((unsigned short)(dm >> 16));
         return w;
@@ -305,9 +319,9 @@ template <> struct wq<MI355_Q4_K> {
         const uint8_t *blk = row + sb * Q4_K_BYTES;
         // header and both qs loads touch the same 128-byte lines from three instructions: ordinary
         // (temporal) loads, so the line is fetched from HBM once and the other two hit in cache
-        const u32x4 hdr = load16(blk);   // d, dmin, 12 scale bytes: same address for the 4 lanes of a super-block
-        w.q0 = load16(blk + 16 + g * 32);
-        w.q1 = load16(blk + 32 + g * 32);
+        const u32x4 hdr = load16w(blk);   // d, dmin, 12 scale bytes: same address for the 4 lanes of a super-block
+        w.q0 = load16w(blk + 16 + g * 32);
+        w.q1 = load16w(blk + 32 + g * 32);
         w.d = half_bits_to_float((unsigned short)(hdr[0] & 0xFFFFu));
         w.dmin = half_bits_to_float((unsigned short)(hdr[0] >> 16));
         // all eight 6-bit (scale, min) pairs at once, branch-free (get_scale_min_k4, ggml-quants.c:631-638)
@@ -369,11 +383,11 @@ template <> struct wq<MI355_Q5_K> {
         chunk w;
         const int sb = c >> 2, g = c & 3;
         const uint8_t *blk = row + sb * Q5_K_BYTES;
-        const u32x4 hdr = load16(blk);   // d, dmin, 12 scale bytes: same address for the 4 lanes of a super-block
-        w.h0 = load16(blk + 16);         // qh: also shared by the 4 lanes
-        w.h1 = load16(blk + 32);
-        w.q0 = load16(blk + 48 + g * 32);
-        w.q1 = load16(blk + 64 + g * 32);
+        const u32x4 hdr = load16w(blk);   // d, dmin, 12 scale bytes: same address for the 4 lanes of a super-block
+        w.h0 = load16w(blk + 16);         // qh: also shared by the 4 lanes
+        w.h1 = load16w(blk + 32);
+        w.q0 = load16w(blk + 48 + g * 32);
+        w.q1 = load16w(blk + 64 + g * 32);
         w.g = g;
         w.d = half_bits_to_float((unsigned short)(hdr[0] & 0xFFFFu));
         w.dmin = half_bits_to_float((unsigned short)(hdr[0] >> 16));
@@ -422,8 +436,8 @@ template <> struct wq<MI355_Q6_K> {
         chunk w;
         const int sb = c >> 3, cc = c & 7, hf = cc >> 2, r = cc & 3;
         const int l0 = 16 * (r & 1), qa = r >> 1;
-        w.ql = load_stream16(row + sb * 128 + cc * 16);
-        w.qh = load_stream16(row + L.off_b + sb * 64 + hf * 32 + l0);
+        w.ql = load_stream16w(row + sb * 128 + cc * 16);
+        w.qh = load_stream16w(row + L.off_b + sb * 64 + hf * 32 + l0);
         const int8_t *sc = (const int8_t *)(row + L.off_c + sb * 16 + hf * 8 + (l0 >> 4));
         w.scA = (float)sc[2 * qa];
         w.scB = (float)sc[2 * qa + 4];
@@ -472,8 +486,7 @@ template <> struct wq<MI355_Q6_K> {
 
 // ---------------------------------------------------------------- scalar element access
 // Dequantized weight element e of a row stored in device layout.  Byte loads only, so it
-// works for rows that are not 16-byte aligned (K not a multiple of 256 for Q4_0/Q8_0, of
-// 2048 for Q6_K).  Semantics: dequantize_row_* of ggml/src/ggml-quants.c:255-347, 349-363,
+// works for rows at any address.  Semantics: dequantize_row_* of ggml/src/ggml-quants.c:255-347, 349-363,
 // 1280-1302, 1482-1507, 1690-1719, 2436-2475.
 template <int TYPE>
 __device__ __forceinline__ float weight_value(const uint8_t *__restrict__ row, const row_layout &L, int64_t e) {

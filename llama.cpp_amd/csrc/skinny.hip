@@ -74,8 +74,9 @@ template <int TYPE, int NI> struct sk_regs {
 };
 
 // grid.x = 32-row tiles of the weight matrix, grid.y = slices of K (partial sums to `dst` as [slice][B][dst_stride] then).
-// The group's four waves split the slice's steps.
-template <int TYPE, int NI>
+// The group's four waves split the slice's steps.  TAIL: K is no multiple of 256 (per-32-block types; a form of its own, since the branch
+// and its registers cost the others 7 %: Q8_0 28672 x 8192, 8 rows, 53.7 -> 57.6 us).
+template <int TYPE, int NI, bool TAIL>
 __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads,
                                                    float *__restrict__ dst, const float *__restrict__ residual, int64_t N, int K, int B,
                                                    int64_t dst_stride, int steps_per_slice, int steps_per_wave) {
@@ -99,7 +100,7 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     uint8_t *s_qh = s_w + 32 * WPAD;
 
     const row_layout L = make_row_layout(TYPE, K);
-    const int nsteps = K >> 8;
+    const int nsteps = TAIL ? (K + 255) >> 8 : K >> 8;
     const int nblk = K >> 5;
     const int64_t row0 = (int64_t)blockIdx.x * 32;
 
@@ -142,43 +143,89 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
         t_src[u] = ads + (int64_t)c * nblk + 2 * t_piece;
     }
 
+    // The last step of a row whose K is no multiple of 256: blocks past the end repeat the last one (nothing is read behind the row) and
+    // get scale and minimum 0; the activation bytes they meet are those of the last block too, hence finite.
+    auto fetch_tail = [&](int s, R &g) {
+        constexpr int BLOCK_Q = T::ROW_BYTES / 8;   // level bytes per block
+        const int last = nblk - 1;
+#pragma unroll
+        for (int u = 0; u < R::NW; u++) {
+            const int blk = s * 8 + 16 * w_piece / BLOCK_Q;
+            g.w[u] = load16w(w_src[u] + s * T::STEP_BYTES - (blk > last ? (blk - last) * BLOCK_Q : 0));
+        }
+        const int so = T::FIFTH32 ? L.off_c : L.off_b;
+        u32 sc[8], fw[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int blk = s * 8 + j < nblk ? s * 8 + j : last;
+            if constexpr (T::PAIR) sc[j] = load4w(w_mine + so + blk * 4);
+            else sc[j] = *(const unsigned short *)(w_mine + so + blk * 2);
+            fw[j] = 0;
+            if constexpr (T::FIFTH32) fw[j] = load4w(w_mine + L.off_b + blk * 4);
+            if (s * 8 + j > last) sc[j] = 0;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            g.qh[0][j] = fw[j];
+            g.qh[1][j] = fw[4 + j];
+            g.hdr[j] = T::PAIR ? sc[j] : sc[2 * j] | (sc[2 * j + 1] << 16);
+            g.hdr2[j] = sc[4 + j];
+        }
+#pragma unroll
+        for (int u = 0; u < R::NA; u++) {
+            const int blk = s * 8 + (a_piece >> 1);
+            g.a[u] = load16(a_src[u] + s * 256 - (blk > last ? (blk - last) * 32 : 0));
+        }
+#pragma unroll
+        for (int u = 0; u < R::NT; u++) {   // two blocks per piece; 16-byte loads of {d, sum} pairs would straddle the end of the row
+            const int b0 = s * 8 + 2 * t_piece;
+            const uint2 e0 = *(const uint2 *)(t_src[u] + s * 8 - (b0 > last ? b0 - last : 0)), e1 = *(const uint2 *)(t_src[u] + s * 8 + 1 - (b0 + 1 > last ? b0 + 1 - last : 0));
+            g.t[u] = u32x4{e0.x, e0.y, e1.x, e1.y};
+        }
+    };
     // loads of one step into the register set `g`
     auto fetch = [&](int step, R &g) {
         const int s = step < nsteps ? step : nsteps - 1;
+        if constexpr (TAIL) {
+            if (s * 8 + 8 > nblk) {   // uniform
+                fetch_tail(s, g);
+                return;
+            }
+        }
         const int w_off = s * T::STEP_BYTES;   // < 2^31: rows are shorter than that
 #pragma unroll
-        for (int u = 0; u < R::NW; u++) g.w[u] = load16(w_src[u] + w_off);
+        for (int u = 0; u < R::NW; u++) g.w[u] = load16w(w_src[u] + w_off);
         if constexpr (T::KQ) {
-            g.hdr = load16(w_mine + w_off);
-            if constexpr (TYPE == MI355_Q5_K) g.qh[0] = load16(w_mine + w_off + 16 + 16 * kh);
+            g.hdr = load16w(w_mine + w_off);
+            if constexpr (TYPE == MI355_Q5_K) g.qh[0] = load16w(w_mine + w_off + 16 + 16 * kh);
         } else if constexpr (T::FIFTH32) {
-            g.qh[0] = load16(w_mine + L.off_b + s * 32);
-            g.qh[1] = load16(w_mine + L.off_b + s * 32 + 16);
+            g.qh[0] = load16w(w_mine + L.off_b + s * 32);
+            g.qh[1] = load16w(w_mine + L.off_b + s * 32 + 16);
             if constexpr (T::PAIR) {
-                g.hdr = load16(w_mine + L.off_c + s * 32);
-                g.hdr2 = load16(w_mine + L.off_c + s * 32 + 16);
+                g.hdr = load16w(w_mine + L.off_c + s * 32);
+                g.hdr2 = load16w(w_mine + L.off_c + s * 32 + 16);
             } else {
-                g.hdr = load16(w_mine + L.off_c + s * 16);
+                g.hdr = load16w(w_mine + L.off_c + s * 16);
             }
         } else if constexpr (T::PAIR) {
-            g.hdr = load16(w_mine + L.off_b + s * 32);
-            g.hdr2 = load16(w_mine + L.off_b + s * 32 + 16);
+            g.hdr = load16w(w_mine + L.off_b + s * 32);
+            g.hdr2 = load16w(w_mine + L.off_b + s * 32 + 16);
         } else if constexpr (TYPE == MI355_IQ4_XS) {
-            const uint2 h = *(const uint2 *)(w_mine + L.off_b + s * 8);   // the super-block's d, scales_h, scales_l
-            g.hdr[0] = h.x;
-            g.hdr[1] = h.y;
+            const u32x2 h = load8w(w_mine + L.off_b + s * 8);   // the super-block's d, scales_h, scales_l
+            g.hdr[0] = h[0];
+            g.hdr[1] = h[1];
         } else if constexpr (Q6) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) g.qh[u] = load16(qh_src[u] + s * 64);
-            g.hdr = load16(w_mine + L.off_c + s * 16);                            // sixteen int8 scales
+            for (int u = 0; u < 2; u++) g.qh[u] = load16w(qh_src[u] + s * 64);
+            g.hdr = load16w(w_mine + L.off_c + s * 16);                            // sixteen int8 scales
             g.d6 = *(const unsigned short *)(w_mine + L.off_d + s * 2);
         } else {
-            g.hdr = load16(w_mine + L.off_b + s * 16);   // eight f16 block scales
+            g.hdr = load16w(w_mine + L.off_b + s * 16);   // eight f16 block scales
         }
 #pragma unroll
         for (int u = 0; u < R::NA; u++) g.a[u] = load16(a_src[u] + s * 256);
 #pragma unroll
-        for (int u = 0; u < R::NT; u++) g.t[u] = load16(t_src[u] + s * 8);
+        for (int u = 0; u < R::NT; u++) g.t[u] = *(const u32x4_a8 *)(t_src[u] + s * 8);
     };
 
     float acc[NI][4];
@@ -391,16 +438,19 @@ __global__ void __launch_bounds__(256) k_skinny_slices(const float *__restrict__
 template <int TYPE, int NI>
 void launch_skinny(hipStream_t s, const void *W, const int8_t *aq, const act_ds *ads, float *dst, const float *residual, int64_t N, int K, int B,
                    int64_t dst_stride, int slices, float *part) {
-    const int nsteps = K >> 8;
+    const int nsteps = (K + 255) >> 8;
     const int steps_per_slice = (nsteps + slices - 1) / slices;
     const int steps_per_wave = (steps_per_slice + 3) / 4;
     const dim3 grid((unsigned)((N + 31) / 32), (unsigned)slices);
-    if (slices == 1) {
-        MI355_LAUNCH((k_mm_skinny<TYPE, NI>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, dst, residual, N, K, B, dst_stride, steps_per_slice,
-                           steps_per_wave);
-    } else {
-        MI355_LAUNCH((k_mm_skinny<TYPE, NI>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, part, (const float *)nullptr, N, K, B, N, steps_per_slice,
-                           steps_per_wave);
+    float *out = slices == 1 ? dst : part;
+    const float *res = slices == 1 ? residual : nullptr;
+    const int64_t stride = slices == 1 ? dst_stride : N;
+    constexpr bool BLOCKS32 = (sk_traits<TYPE>::NIB32 && TYPE != MI355_IQ4_XS) || TYPE == MI355_Q8_0;
+    if (BLOCKS32 && K % 256 != 0)
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave);
+    else
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, false>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave);
+    if (slices > 1) {
         MI355_LAUNCH(k_skinny_slices, dim3((unsigned)((N + 255) / 256), (unsigned)B), dim3(256), 0, s, part, dst, residual, N, B, dst_stride, slices);
     }
 }
@@ -417,7 +467,7 @@ void launch_skinny_nt(hipStream_t s, const void *W, const int8_t *aq, const act_
 // slices of K: launches with fewer than ~1.5 groups per compute unit split K over several groups (and pay a second launch
 // that adds the slices), as long as a slice keeps 4 steps; a short K with at most 8 activation rows is quicker in one go.
 int skinny_slices(int64_t N, int64_t K, int64_t B) {
-    const int64_t tiles = (N + 31) / 32, nsteps = K >> 8;
+    const int64_t tiles = (N + 31) / 32, nsteps = (K + 255) >> 8;
     if (tiles >= 384 || (B <= 8 && nsteps <= 16)) return 1;
     int s = 1;
     while (s < 8 && tiles * s < 512 && nsteps / (s * 2) >= 4) s *= 2;
@@ -433,8 +483,7 @@ using namespace mi355;
 extern "C" {
 
 int mi355_mul_mat_skinny_supported(int type, const void *W, int64_t K, int64_t B) {
-    return is_weight_type(type) && B >= 1 && B <= 32 && K > 0 && K % 256 == 0 && K < (int64_t(1) << 30) &&
-           layout_aligned(W, make_row_layout(type, K));
+    return is_weight_type(type) && B >= 1 && B <= 32 && K > 0 && K % type_block_elems(type) == 0 && K < (int64_t(1) << 30) && layout_loadable(W);
 }
 
 size_t mi355_mul_mat_skinny_ws_bytes(int64_t N, int64_t K, int64_t B) {

@@ -351,6 +351,25 @@ def test_unaligned_rows_fallback(dev, name, t):
         assert orc.nmse(got, want) < (1e-6 if (t == orc.Q5_K and B > 8) else 1e-9)
 
 
+@pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t not in (orc.Q4_K, orc.Q5_K)])   # those two are 16-byte aligned at any K
+@pytest.mark.parametrize("blocks", [1, 7, 9, 43, 47])
+def test_ragged_rows(dev, name, t, blocks):
+    """rows that start at any even address and whose length is no whole number of the kernels' K steps: GEMV, weight-streaming and tile
+    kernels, with and without slices along K, against exact integer block dots (f32 sums: NMSE of some 1e-14)"""
+    import mi355
+    rng = np.random.default_rng(blocks)
+    K = orc.BLOCK[t][0] * blocks
+    N = 150
+    Wq = _weights(rng, t, N, K)
+    Wd = mi355.upload_weights(t, _to_dev(dev, Wq))
+    for B in (1, 3, 4, 8, 9, 32, 33, 130):
+        x = rng.standard_normal((B, K)).astype(np.float32)
+        want = orc.mul_mat("q8_1", t, Wq, x)
+        for split in (False, True):
+            got = mi355.mul_mat(t, Wd, _to_dev(dev, x), split=split).cpu().numpy()
+            assert orc.nmse(got, want) < 1e-11, (B, split)
+
+
 KQ_TYPES = [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q6_K)]
 TILED_TYPES = [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q5_K, orc.Q6_K, orc.IQ4_XS)]   # types with tile images for the wide-tile GEMM
 

@@ -135,3 +135,19 @@ def test_mul_mat_id_on_tile_images_skewed_routing(dev, pattern):
     got = mi355.mul_mat_id_tiled(t, tiles, N, torch.from_numpy(b).to(dev), idd, n_used).cpu().numpy()
     want = expected_per_expert("cpu", t, Wq, b, np.clip(ids, 0, n_expert - 1), n_expert, n_used, 1, N)
     assert orc.nmse(got, want) < 1e-9
+
+
+@pytest.mark.parametrize("name,t,blocks", [("q6_k", orc.Q6_K, 3), ("iq4_xs", orc.IQ4_XS, 5), ("q4_0", orc.Q4_0, 3), ("q8_0", orc.Q8_0, 9), ("q5_1", orc.Q5_1, 7)])
+@pytest.mark.parametrize("T", [3, 16, 130])
+def test_mul_mat_id_ragged_rows(dev, name, t, blocks, T):
+    """expert rows that start at any even address, K no whole number of the tile kernel's stages: per-slot GEMV and routed tiles"""
+    import torch
+    import mi355
+    n_expert, n_used, N, K = 5, 2, 70, orc.BLOCK[t][0] * blocks
+    rng = np.random.default_rng(T)
+    Wq = orc.quantize("oracle", t, (rng.standard_normal((n_expert * N, K)) * 0.02).astype(np.float32))
+    b = rng.standard_normal((T, 1, K)).astype(np.float32)
+    ids = np.stack([rng.permutation(n_expert) for _ in range(T)]).astype(np.int32)
+    Wd = mi355.upload_weights(t, torch.from_numpy(Wq).to(dev)).reshape(n_expert, N, -1)
+    got = mi355.mul_mat_id(t, Wd, torch.from_numpy(b).to(dev), torch.from_numpy(ids).to(dev)[:, :n_used], n_used).cpu().numpy()
+    assert orc.nmse(got, expected_per_expert("q8_1", t, Wq, b, ids, n_expert, n_used, 1, N)) < 1e-11
