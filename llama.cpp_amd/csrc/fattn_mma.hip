@@ -28,36 +28,53 @@ namespace {
 constexpr int FM_BC = 64;            // kv cells per tile
 constexpr float FM_NEG = -FLT_MAX / 2;
 
+// O^T is accumulated in tiles of 32 elements of the head: head sizes that are no multiple of 32 (80, 112) leave the last tile partly
+// unused - its upper rows meet whatever the padding columns of the V tile hold and are never stored.
+template <int D> constexpr int fm_dtiles() { return (D + 31) / 32; }
+template <int D> constexpr int fm_vpitch() { return 32 * fm_dtiles<D>() + 16; }   // f16 pitch of a V row in LDS: rows 8 banks apart, so the four rows of a transposing read miss each other
+
 // ---- staging of one 64-cell K tile and the matching V tile through registers, both row-major ----
 template <int D, int NTH, int BC = FM_BC> struct kv_stage {
     static constexpr int KP = D + 8;        // f16 pitch of a K row in LDS (16 bytes of padding spread the banks)
-    static constexpr int VP = D + 16;       // f16 pitch of a V row in LDS: rows 8 banks apart, so the four rows of a transposing read miss each other
+    static constexpr int VP = fm_vpitch<D>();
     static constexpr int KCH = D / 8;       // 16-byte chunks per K/V row
-    static constexpr int KIT = BC * KCH / NTH;            // chunks per thread per tile, K and V each
-    static_assert(D % 32 == 0 && KIT >= 1, "head size not served by this kernel");
-    static_assert(NTH % KCH == 0, "a thread keeps its chunk position over the rows it loads");
+    static constexpr int UNITS = BC * KCH;
+    static constexpr int KIT = (UNITS + NTH - 1) / NTH;   // chunks per thread per tile, K and V each
+    static constexpr bool EVEN = NTH % KCH == 0 && UNITS % NTH == 0;   // a thread keeps its chunk position over the rows it loads
+    static_assert(D % 16 == 0, "head size not served by this kernel");
     u32x4 k[KIT], v[KIT];
 
     // A tile that lies inside the cache is addressed as (uniform base of the tile and of the thread's it-th row block) + (one
     // 32-bit offset per thread, the same for every tile): thread tid loads rows tid / KCH + it * (NTH / KCH), chunk tid % KCH.
     // The uniform part is scalar arithmetic; per-row 64-bit products in vector registers cost as many instructions per tile
-    // step as the soft-max.  The launcher checks that a tile's span fits 32 bits.  The last, partial tile clamps row by row.
+    // step as the soft-max.  The launcher checks that a tile's span fits 32 bits.  Head sizes whose chunks do not divide the group
+    // evenly (80, 96, 112) keep one offset per chunk instead.  The last, partial tile clamps row by row.
     __device__ __forceinline__ void fetch(const fattn_args &a, int64_t hk, int64_t kv0, int tid) {
         if (kv0 + BC <= a.Nkv) {   // uniform
-            const unsigned r0 = (unsigned)(tid / KCH), ch16 = (unsigned)(tid % KCH) * 16;
-            const unsigned ko = r0 * (unsigned)a.k_nb1 + ch16, vo = r0 * (unsigned)a.v_nb1 + ch16;
             const uint8_t *kb = a.k + kv0 * a.k_nb1 + hk * a.k_nb2, *vb = a.v + kv0 * a.v_nb1 + hk * a.v_nb2;
+            if constexpr (EVEN) {
+                const unsigned r0 = (unsigned)(tid / KCH), ch16 = (unsigned)(tid % KCH) * 16;
+                const unsigned ko = r0 * (unsigned)a.k_nb1 + ch16, vo = r0 * (unsigned)a.v_nb1 + ch16;
 #pragma unroll
-            for (int it = 0; it < KIT; it++) {
-                k[it] = load16(kb + (size_t)it * (NTH / KCH) * a.k_nb1 + ko);
-                v[it] = load16(vb + (size_t)it * (NTH / KCH) * a.v_nb1 + vo);
+                for (int it = 0; it < KIT; it++) {
+                    k[it] = load16(kb + (size_t)it * (NTH / KCH) * a.k_nb1 + ko);
+                    v[it] = load16(vb + (size_t)it * (NTH / KCH) * a.v_nb1 + vo);
+                }
+            } else {
+#pragma unroll
+                for (int it = 0; it < KIT; it++) {
+                    const unsigned unit = tid + it * NTH < UNITS ? tid + it * NTH : UNITS - 1;
+                    const unsigned row = unit / KCH, ch16 = unit % KCH * 16;
+                    k[it] = load16(kb + (row * (unsigned)a.k_nb1 + ch16));
+                    v[it] = load16(vb + (row * (unsigned)a.v_nb1 + ch16));
+                }
             }
             return;
         }
         const int64_t last = a.Nkv - 1;
 #pragma unroll
         for (int it = 0; it < KIT; it++) {
-            const int unit = tid + it * NTH;
+            const int unit = EVEN || tid + it * NTH < UNITS ? tid + it * NTH : UNITS - 1;
             const int row = unit / KCH, ch = unit % KCH;
             const int64_t c = kv0 + row < last ? kv0 + row : last;   // rows past the end repeat the last cell; their scores are dropped
             k[it] = load16(a.k + c * a.k_nb1 + hk * a.k_nb2 + ch * 16);
@@ -68,6 +85,7 @@ template <int D, int NTH, int BC = FM_BC> struct kv_stage {
 #pragma unroll
         for (int it = 0; it < KIT; it++) {
             const int unit = tid + it * NTH;
+            if (UNITS % NTH != 0 && unit >= UNITS) continue;
             const int row = unit / KCH, ch = unit % KCH;
             *(u32x4 *)(sK + row * KP + ch * 8) = k[it];
             *(u32x4 *)(sV + row * VP + ch * 8) = v[it];
@@ -230,7 +248,7 @@ __device__ __forceinline__ float alibi_slope(const fattn_args &a, int64_t head) 
 // + 12 point at, so lane 4 r + q of a group points at row c + r, elements 16 (group % 2) + 4 q .. + 3 of the tile's 32.
 template <int D, int NDT>
 __device__ __forceinline__ void accumulate_pv(f32x16 (&o)[NDT], const f32x16 &S, const _Float16 *sV, int dt0, int u, int l32, int lhi) {
-    constexpr int VP = D + 16;
+    constexpr int VP = fm_vpitch<D>();
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     const int li = l32 & 15;
     const _Float16 *lane_base = sV + (32 * u + 4 * lhi + (li >> 2)) * VP + 16 * (l32 >> 4) + 4 * (li & 3);
@@ -330,9 +348,10 @@ __device__ __forceinline__ grid_pos xcd_grid_pos() {
 }
 
 template <int D, int HPW>
-__global__ void __launch_bounds__(256, 2) k_fattn_mma(fattn_args a) {
+__global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a) {
     typedef kv_stage<D, 256> stage_t;
     constexpr int QTW = 4 / HPW;   // query tiles per group
+    constexpr int NDT = fm_dtiles<D>();
     __shared__ __attribute__((aligned(16))) _Float16 sK[FM_BC * stage_t::KP];
     __shared__ __attribute__((aligned(16))) _Float16 sVt[FM_BC * stage_t::VP];
 
@@ -355,9 +374,9 @@ __global__ void __launch_bounds__(256, 2) k_fattn_mma(fattn_args a) {
     const unsigned short *mrow = a.mask ? (const unsigned short *)(a.mask + iq * a.mask_nb1) : nullptr;
     const bool mask_aligned = (((uintptr_t)a.mask | a.mask_nb1) & 7) == 0;
 
-    f32x16 o[D / 32];
+    f32x16 o[NDT];
 #pragma unroll
-    for (int dt = 0; dt < D / 32; dt++)
+    for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[dt][r] = 0.0f;
     float m = FM_NEG, l = 0.0f;
@@ -423,21 +442,22 @@ __global__ void __launch_bounds__(256, 2) k_fattn_mma(fattn_args a) {
         m = m_new;
         if (__ballot(alpha != 1.0f) != 0) {   // wave-uniform
 #pragma unroll
-            for (int dt = 0; dt < D / 32; dt++)
+            for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
         }
 #pragma unroll
-        for (int u = 0; u < 2; u++) accumulate_pv<D, D / 32>(o, S[u], sVt, 0, u, l32, lhi);
+        for (int u = 0; u < 2; u++) accumulate_pv<D, NDT>(o, S[u], sVt, 0, u, l32, lhi);
     }
 
     if (q0 + l32 < a.Nq) {
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
         float *dp = a.dst + ((q0 + l32) * a.Hq + head) * D;
 #pragma unroll
-        for (int dt = 0; dt < D / 32; dt++)
+        for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
             for (int g = 0; g < 4; g++) {
+                if (32 * dt + 8 * g >= D) continue;
                 f32x4 w;
 #pragma unroll
                 for (int i = 0; i < 4; i++) w[i] = o[dt][4 * g + i] * inv;
@@ -454,13 +474,14 @@ __global__ void __launch_bounds__(256, 2) k_fattn_mma(fattn_args a) {
 // with half the work per wave and tile; NU = 4 (eight waves, 128-cell tiles) when even those leave one group per compute
 // unit: two waves per SIMD, so that one wave's matrix instructions run under the other's soft-max arithmetic, and half the
 // tile steps.
-template <int D, int NU>
-__global__ void __launch_bounds__(128 * NU, NU == 2 ? 2 : 1) k_fattn_mma_half(fattn_args a) {
+// PQ: the two columns of waves are neighbouring query tiles of one head instead of two heads (an odd number of query heads per kv head)
+template <int D, int NU, bool PQ>
+__global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn_mma_half(fattn_args a) {
     constexpr int NTH = 128 * NU, BC = 32 * NU;
     typedef kv_stage<D, NTH, BC> stage_t;
-    constexpr int NDT = D / 32;
+    constexpr int NDT = fm_dtiles<D>(), DP = 32 * NDT;
     constexpr int KV_HALVES = BC * stage_t::KP + BC * stage_t::VP;                    // f16 elements of the K tile and the V tile
-    constexpr int MERGE_FLOATS = NU * (D + 2) * 32;                                   // per (head, pair of waves): O^T [D][32], max, sum
+    constexpr int MERGE_FLOATS = NU * (DP + 2) * 32;                                   // per (head, pair of waves): O^T [D][32], max, sum
     constexpr int SMEM_BYTES = KV_HALVES * 2 > MERGE_FLOATS * 4 ? KV_HALVES * 2 : MERGE_FLOATS * 4;
     __shared__ __attribute__((aligned(16))) uint8_t smem[SMEM_BYTES];
     _Float16 *sK = (_Float16 *)smem, *sVt = sK + BC * stage_t::KP;
@@ -470,11 +491,12 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 ? 2 : 1) k_fattn_mma_half(fa
     const int lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, lhi = lane >> 5;
     const int u = wave % NU, hp = wave / NU;
-    const int pairs = (int)(a.Hq / a.Hkv) / 2;   // head pairs per kv head
+    const int R = (int)(a.Hq / a.Hkv);
+    const int pairs = PQ ? R : R / 2;   // heads or head pairs per kv head
     const grid_pos gp = xcd_grid_pos();
-    const int64_t hk = gp.y / pairs, hg = gp.y % pairs;
-    const int64_t head = (hk * pairs + hg) * 2 + hp;
-    const int64_t q0 = (int64_t)gp.x * 32;
+    const int64_t hk = gp.y / pairs;
+    const int64_t head = PQ ? gp.y : 2 * (int64_t)gp.y + hp;
+    const int64_t q0 = PQ ? ((int64_t)gp.x * 2 + hp) * 32 : (int64_t)gp.x * 32;
     const int64_t iq = q0 + l32 < a.Nq ? q0 + l32 : a.Nq - 1;   // clamped: rows past Nq are computed and dropped
 
     f16x8 qf[D / 16];
@@ -506,7 +528,7 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 ? 2 : 1) k_fattn_mma_half(fa
         for (int g = 0; g < 4; g++) mcur[g] = mnext[g];
         __syncthreads();
         if (kv0 + BC < a.Nkv) prefetch(kv0 + BC);
-        f32x16 S = scores<D, true>(qf, sK, u, l32, lhi);
+        f32x16 S = scores<D, (D <= 128)>(qf, sK, u, l32, lhi);
         float mx = finish_scores(S, mcur, a, scale, slope, kv0 + 32 * u, lhi, a.Nkv);
         mx = half_pair_max(mx);
         if (__ballot(mx > FM_NEG) == 0) continue;   // all 32 cells masked for all 32 queries (wave-uniform; barriers are at the loop head)
@@ -537,7 +559,7 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 ? 2 : 1) k_fattn_mma_half(fa
     // ---- the states of a head's waves are joined pairwise: u + step hands its state to u (step = 1, then 2)
 #pragma unroll
     for (int step = 1; step < NU; step *= 2) {
-        float *mg = s_merge + (hp * (NU / 2) + (u >> 1) / step) * (D + 2) * 32;   // [d][query], then max, sum
+        float *mg = s_merge + (hp * (NU / 2) + (u >> 1) / step) * (DP + 2) * 32;   // [d][query], then max, sum
         __syncthreads();
         if ((u & (2 * step - 1)) == step) {
 #pragma unroll
@@ -545,13 +567,13 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 ? 2 : 1) k_fattn_mma_half(fa
 #pragma unroll
                 for (int r = 0; r < 16; r++) mg[(32 * dt + 8 * (r >> 2) + 4 * lhi + (r & 3)) * 32 + l32] = o[dt][r];
             if (lhi == 0) {
-                mg[D * 32 + l32] = m;
-                mg[(D + 1) * 32 + l32] = l;
+                mg[DP * 32 + l32] = m;
+                mg[(DP + 1) * 32 + l32] = l;
             }
         }
         __syncthreads();
         if ((u & (2 * step - 1)) == 0) {
-            const float m1 = mg[D * 32 + l32], l1 = mg[(D + 1) * 32 + l32];
+            const float m1 = mg[DP * 32 + l32], l1 = mg[(DP + 1) * 32 + l32];
             const float M = fmaxf(m, m1);
             const float f0 = __expf(m - M), f1 = __expf(m1 - M);
             l = l * f0 + l1 * f1;
@@ -569,6 +591,7 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 ? 2 : 1) k_fattn_mma_half(fa
     for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
         for (int g = 0; g < 4; g++) {
+            if (32 * dt + 8 * g >= D) continue;
             f32x4 w;
 #pragma unroll
             for (int i = 0; i < 4; i++) w[i] = o[dt][4 * g + i] * inv;
@@ -576,14 +599,19 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 ? 2 : 1) k_fattn_mma_half(fa
         }
 }
 
-template <int D>
+template <int D, bool PQ>
 int launch_half(hipStream_t s, const fattn_args &a) {
-    const int64_t pairs = (a.Hq / a.Hkv) / 2;
-    const dim3 grid((unsigned)((a.Nq + 31) / 32), (unsigned)(a.Hkv * pairs));
+    const int64_t R = a.Hq / a.Hkv, n_tiles = (a.Nq + 31) / 32;
+    const dim3 grid((unsigned)(PQ ? (n_tiles + 1) / 2 : n_tiles), (unsigned)(a.Hkv * (PQ ? R : R / 2)));
     // at most one group per compute unit and a long cache: eight waves on 128-cell tiles (512 rows: 4096 cells 112 -> 103 us,
     // 512 cells 24.8 -> 26.2 us)
-    if ((int64_t)grid.x * grid.y <= 256 && a.Nkv >= 1024) MI355_LAUNCH((k_fattn_mma_half<D, 4>), grid, dim3(512), 0, s, a);
-    else MI355_LAUNCH((k_fattn_mma_half<D, 2>), grid, dim3(256), 0, s, a);
+    if constexpr (D <= 128) {   // (head size 256: the eight waves' registers do not fit)
+        if ((int64_t)grid.x * grid.y <= 256 && a.Nkv >= 1024) {
+            MI355_LAUNCH((k_fattn_mma_half<D, 4, PQ>), grid, dim3(512), 0, s, a);
+            return launch_status("k_fattn_mma_half");
+        }
+    }
+    MI355_LAUNCH((k_fattn_mma_half<D, 2, PQ>), grid, dim3(256), 0, s, a);
     return launch_status("k_fattn_mma_half");
 }
 
@@ -790,7 +818,6 @@ int launch_dec(hipStream_t s, const fattn_args &a) {
 int launch_fattn_mma(hipStream_t s, fattn_args &a, int64_t D, size_t ws_bytes) {
     if (a.Hkv * (a.Hq / a.Hkv) > 65535 || (a.Nq + 31) / 32 > 0x7fffffff) return 1;
     if ((a.q_nb1 % 16) != 0 || (a.q_nb2 % 16) != 0) return 1;
-    if (D != 64 && D != 128) return 1;
     if (a.k_nb1 >= (size_t(1) << 24) || a.v_nb1 >= (size_t(1) << 24)) return 1;   // kv_stage: a tile's rows within 32-bit offsets
     a.kv_extent = nullptr;
     const int64_t n_tiles = (a.Nq + 31) / 32;
@@ -806,17 +833,21 @@ int launch_fattn_mma(hipStream_t s, fattn_args &a, int64_t D, size_t ws_bytes) {
     }
     // few query tiles (a batch of a few hundred rows): twice the groups with half a K/V tile per wave, while the chip is not full
     const int64_t R = a.Hq / a.Hkv;
-    if (R % 2 == 0 && n_tiles * a.Hkv * (R / 2) <= 512) {
-        switch (D) {
-            case 64: return launch_half<64>(s, a);
-            case 128: return launch_half<128>(s, a);
-        }
-    }
+    // (an odd number of query heads per kv head pairs neighbouring query tiles: 512 rows over 1024 cells, 32 heads, D 128: 40 -> 31 us).
+    // Against the vector kernel, which served these head sizes before: 512 x 512 cells, 32 / 32 heads, D 80: 192 -> 16 us (launch and
+    // latency of eight tile steps); 2048 x 2048, 32 / 8 heads: D 80 2053 -> 95 us, D 112 2055 -> 117 us, D 256 4370 -> 325 us.
+    const bool pq = R % 2 != 0, half = (pq ? (n_tiles + 1) / 2 * a.Hq : n_tiles * a.Hq / 2) <= 512;
+#define MI355_FM_HEAD(D_) return !half ? launch_hpw<D_>(s, a) : pq ? launch_half<D_, true>(s, a) : launch_half<D_, false>(s, a);
     switch (D) {
-        case 64: return launch_hpw<64>(s, a);
-        case 128: return launch_hpw<128>(s, a);
-        default: return 1;   // other head sizes stay on the vector kernel
+        case 64: MI355_FM_HEAD(64)
+        case 80: MI355_FM_HEAD(80)
+        case 96: MI355_FM_HEAD(96)
+        case 112: MI355_FM_HEAD(112)
+        case 128: MI355_FM_HEAD(128)
+        case 256: MI355_FM_HEAD(256)
+        default: return 1;
     }
+#undef MI355_FM_HEAD
 }
 
 // Few query rows: returns 1 when the shape is not served.  a.n_splits / a.cells_per_split (a multiple of 64) are set by the caller.

@@ -227,3 +227,20 @@ def test_prefill_mask_extent_prepass(dev, kind):
         ms = np.concatenate([mask[rows], np.full((64 - len(rows), Nkv), -np.inf, dtype=np.float16)])
         f64 = orc.flash_attn("f64", q[h:h + 1][:, rows], k[h // 4:h // 4 + 1].view(np.uint16), v[h // 4:h // 4 + 1].view(np.uint16), ms.view(np.uint16), scale)
         assert orc.nmse(with_pass[rows][:, h:h + 1], f64) < 1e-5
+
+
+@pytest.mark.parametrize("D", [80, 96, 112, 256])
+@pytest.mark.parametrize("Nq,Nkv,Hq,Hkv", [(16, 40, 4, 4), (33, 96, 6, 2), (65, 1090, 8, 2), (130, 1056, 3, 1), (545, 600, 64, 16), (545, 600, 66, 66)])
+def test_prefill_head_sizes(dev, D, Nq, Nkv, Hq, Hkv):
+    """the matrix-core kernels at head sizes whose 16-byte chunks do not divide the group (80, 96, 112), that fill the last 32-element
+    output tile in part (80, 112) or need the whole register file (256): query tiles and cell tiles with remainders, one, two and four
+    heads per group, few and many groups.  f16 probabilities and values: 2^-11 per term, averaged to some 3e-4 of the result (NMSE 1e-7)."""
+    rng = np.random.default_rng(D + Nq + Hq)
+    q, k, v, mask = _inputs(rng, D, Nq, Nkv, Hq, Hkv, causal=True, rand_mask=True)
+    scale = 1.0 / np.sqrt(D)
+    got = _run(dev, q, k, v, mask, scale, llama_layout=True)
+    kk, vv = (np.repeat(a.astype(np.float64), Hq // Hkv, axis=0) for a in (k, v))
+    s = np.einsum("hqd,hkd->hqk", q.astype(np.float16).astype(np.float64), kk) * scale + mask[:Nq].astype(np.float64)
+    p = np.exp(s - s.max(axis=-1, keepdims=True))
+    want = np.einsum("hqk,hkd->qhd", p / p.sum(axis=-1, keepdims=True), vv)
+    assert orc.nmse(got, want) < 1e-6
