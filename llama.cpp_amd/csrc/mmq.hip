@@ -3,25 +3,25 @@
 //
 // A 256-thread group (4 waves, 2 x 2) owns a 128 (weight rows) x BN (activation rows)
 // tile of dst and walks K in stages of 128 elements.  Per stage the weight rows are
-// unpacked from their 4/6/8-bit blocks to int8 in LDS (16-byte streaming loads from HBM,
-// each weight byte is unpacked once per group and reused for BN activation rows), the
-// activation int8 rows are copied to LDS, and each wave contracts its 64 x (BN/2)
+// unpacked from their 4/6/8-bit blocks to int8 in LDS (each weight byte is unpacked once per
+// group and reused for BN activation rows), the activation int8 rows are copied to LDS - into the
+// other of two buffers, so that a stage costs one barrier - and each wave contracts its 64 x (BN/2)
 // sub-tile with v_mfma_i32_32x32x32_i8, one instruction per 32-element quantization block,
 // so every MFMA result is an exact per-block integer dot.  Block results are scaled by
 // (weight block scale) x (activation block scale) and accumulated in f32 registers.
 //
-//   Q4_0 : level - 8 as int8, scale d                    (one MFMA per block)
+//   Q4_0 : 16 * (level - 8) as int8, scale d / 16        (one MFMA per block)
 //   Q8_0 : level as int8, scale d
 //   Q5_0 : level - 16 as int8, scale d;  IQ4_NL : the table value of the nibble as int8, scale d
 //   IQ4_XS : as IQ4_NL, scale d * (ls - 32) from the super-block's header
 //   Q4_1, Q5_1 : level 0..15 / 0..31 as int8, scale d; the "+ m * d_x * sum(q)" term of the stage's four blocks is added with two
 //          v_mfma_f32_32x32x2_f32 on (dx * sum(q)) x m
 //   Q4_K, Q5_K : level 0..15 / 0..31 as int8, scale d*sc; the "- dmin*m*sum(q)" term of the blocks the same way
-//   Q6_K : level - 32 as int8, scale d*sc per 16 elements (v_mfma_i32_32x32x16_i8, two per block)
+//   Q6_K : level - 32 as int8, scale d*sc per 16 elements (two MFMAs per block, each on the lane half that holds its elements)
 //
 // MFMA operand mapping used here (A = activations, B = weights, D[i][j], i = activation
 // row, j = weight row): lane l supplies row/column l % 32 and the k bytes
-// [16*(l/32), 16*(l/32)+16) of the 32-wide step (8-byte halves for the 16-wide step);
+// [16*(l/32), 16*(l/32)+16) of the 32-wide step;
 // D register r of lane l is element i = 8*(r/4) + 4*(l/32) + r%4, j = l % 32.  Both
 // operands use the same k split, so the contraction is independent of how the hardware
 // numbers k internally.
@@ -36,7 +36,22 @@ namespace mi355 {
 
 constexpr int MMQ_BM = 128;          // weight rows per group
 constexpr int MMQ_BK = 128;          // K elements per stage
-constexpr int MMQ_LDK = MMQ_BK + 16; // LDS row pitch in bytes (pad to spread banks)
+// byte offset of 16-byte chunk c (0..7) of row r of a stage in LDS: rows of 128 bytes, the chunks of eight neighbouring rows in different
+// banks (a pad of 16 bytes per row does the same, but two stages of the types with minima then leave one group per compute unit)
+__device__ __forceinline__ int mmq_chunk(int r, int c) { return r * MMQ_BK + ((c ^ (r & 7)) << 4); }
+
+// Scaling of the block sums, the larger part of the kernel's work (16 sums per lane and v_mfma_i32_32x32x32_i8, which itself takes 32 of
+// the 4 x 16 x n cycles that n instructions per sum cost): the accumulator of each matrix instruction starts at the bits of
+// M = 1.5 * 2^23, so that its integer result (|sum| < 2^22: 32 * 127 * 128 at most) read as a float is M + sum, without a conversion.  Then
+//     t = fma(M + sum, dw, -M dw)      = sum * dw rounded once: M * dw is exact, dw has at most 19 significant bits
+//     acc = fma(t, dx, acc)            dx as f16 (what block_q8_1 holds), widened inside the instruction (v_fma_mix_f32)
+// two instructions per sum instead of three (convert, dw * dx shared, fma): see the figures at launch_mmq.
+constexpr float MMQ_MAGIC = 12582912.0f;
+constexpr int MMQ_MAGIC_BITS = 0x4B400000;
+
+// place of activation row r's scale in a block's row of sAd: the 16 rows of a lane (i = 8 (j / 4) + 4 (lane / 32) + j % 4 of a 32-row
+// tile, j = 0..15) side by side
+__device__ __forceinline__ int mmq_dx_slot(int r) { return (r & ~31) + ((r >> 2) & 1) * 16 + ((r >> 3) & 3) * 4 + (r & 3); }
 
 template <int TYPE> struct mmq_cfg {
     static constexpr int G = TYPE == MI355_Q6_K ? 16 : 32;   // elements per weight scale
@@ -46,121 +61,50 @@ template <int TYPE> struct mmq_cfg {
     // 16 bytes of nibbles per block with a per-block scale: one request / commit form serves them all
     static constexpr bool NIBBLE32 = TYPE == MI355_Q4_0 || TYPE == MI355_Q4_1 || TYPE == MI355_Q5_0 || TYPE == MI355_Q5_1 || TYPE == MI355_IQ4_NL ||
                                      TYPE == MI355_IQ4_XS;
-    static constexpr bool PREFETCH = NIBBLE32 || TYPE == MI355_Q8_0 || TYPE == MI355_Q6_K;
 };
 
-// ---- stage loaders: global (device layout) -> int8 rows + scales in LDS ----------------
-// sW  : int8 [MMQ_BM][MMQ_LDK]
+// ---- a stage is requested (global -> registers) one stage ahead and committed (unpack -> LDS) while the stage before it is contracted
+// sW  : int8 [MMQ_BM][MMQ_BK] (mmq_chunk)
 // sWs : float [NG][MMQ_BM]   (scale g of row r at sWs[g*MMQ_BM + r])
 // sWo : float [4][MMQ_BM]    (types with a block minimum: what multiplies d_x * sum(q) of the stage's 4 blocks)
-template <int TYPE>
-__device__ __forceinline__ void load_weight_stage(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0,
-                                                  int64_t N, int64_t k0, int8_t *sW, float *sWs, float *sWo) {
-    const int tid = threadIdx.x;
-    {
-        // stage = half a super-block: sub-blocks j0..j0+3, 64 B of qs per row = 4 pieces of 16 B (Q5_K: bit j of qh[l] is the fifth
-        // bit of element l of sub-block j, dequantize_row_q5_K, ggml/src/ggml-quants.c:1482-1507)
-        constexpr int BB = TYPE == MI355_Q4_K ? Q4_K_BYTES : Q5_K_BYTES, QS = TYPE == MI355_Q4_K ? 16 : 48;
-        const int64_t sb = k0 >> 8;
-        const int half = (int)((k0 >> 7) & 1);
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 2, p = idx & 3;          // p: piece -> group gl = p>>1 of the stage, half h = p&1
-            const int gl = p >> 1, h = p & 1;
-            const int64_t row = row0 + r < N ? row0 + r : N - 1;
-            const uint8_t *blk = W + row * L.row_bytes + sb * BB;
-            const u32x4 q = load16w(blk + QS + (half * 2 + gl) * 32 + h * 16);
-            u32x4 lo, hi;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                lo[i] = q[i] & 0x0F0F0F0Fu;
-                hi[i] = (q[i] >> 4) & 0x0F0F0F0Fu;
-            }
-            if constexpr (TYPE == MI355_Q5_K) {
-                const u32x4 qh = load16w(blk + 16 + h * 16);
-                const int ja = half * 4 + 2 * gl;         // sub-block of the low nibbles; the high nibbles are the next one
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    lo[i] |= ((qh[i] >> ja) & 0x01010101u) << 4;
-                    hi[i] |= ((qh[i] >> (ja + 1)) & 0x01010101u) << 4;
-                }
-            }
-            *(u32x4 *)(sW + r * MMQ_LDK + (2 * gl) * 32 + h * 16) = lo;
-            *(u32x4 *)(sW + r * MMQ_LDK + (2 * gl + 1) * 32 + h * 16) = hi;
-            // this thread also owns the (scale, min) of sub-block p of the stage
-            const u32x4 hdr = load16w(blk);
-            const float d = half_bits_to_float((unsigned short)(hdr[0] & 0xFFFFu));
-            const float dmin = half_bits_to_float((unsigned short)(hdr[0] >> 16));
-            int sc, mn;
-            q4k_scale_min(hdr[1], hdr[2], hdr[3], half * 4 + p, sc, mn);
-            sWs[p * MMQ_BM + r] = d * (float)sc;
-            sWo[p * MMQ_BM + r] = -(dmin * (float)mn);
-        }
-    }
-}
-
-// sA  : int8 [BN][MMQ_LDK];  sAd : float [4][BN] block scales;  sAs : float [4][BN]  dx*sum(q) (types with a block minimum)
-template <int TYPE, int BN>
-__device__ __forceinline__ void load_act_stage(const int8_t *__restrict__ aq, const act_ds *__restrict__ ads,
-                                               int64_t col0, int64_t B, int64_t K, int64_t k0, int8_t *sA, float *sAd,
-                                               float *sAs) {
-    const int tid = threadIdx.x;
-    const int64_t nblk = K >> 5;
-    // BN rows x 8 pieces of 16 B
-#pragma unroll
-    for (int it = 0; it < BN * 8 / 256; it++) {
-        const int idx = tid + it * 256;
-        const int r = idx >> 3, c = idx & 7;
-        const int64_t col = col0 + r < B ? col0 + r : B - 1;
-        *(u32x4 *)(sA + r * MMQ_LDK + c * 16) = load16(aq + col * K + k0 + c * 16);
-    }
-    // BN rows x 4 block scales
-#pragma unroll
-    for (int it = 0; it < (BN * 4 + 255) / 256; it++) {
-        const int idx = tid + it * 256;
-        if (idx < BN * 4) {
-            const int r = idx >> 2, b = idx & 3;
-            const int64_t col = col0 + r < B ? col0 + r : B - 1;
-            const act_ds s = ads[col * nblk + (k0 >> 5) + b];
-            sAd[b * BN + r] = s.d;
-            if constexpr (TYPE == MI355_Q4_K || TYPE == MI355_Q5_K) sAs[b * BN + r] = s.d * (float)s.sum;
-        }
-    }
-}
-
-// ---- the same stages split into "request" (global -> registers) and "commit" (unpack -> LDS), so that the next stage's bytes
-// travel while the current stage is contracted (all types but Q4_K and Q5_K, whose batches run on the super-block kernels)
+// sA  : int8 [BN][MMQ_BK] (mmq_chunk);  sAd : f16 [4][BN] block scales (mmq_dx_slot);  sAs : float [4][BN]  dx*sum(q) (types with a block minimum)
 template <int TYPE, bool NIB = mmq_cfg<TYPE>::NIBBLE32> struct mmq_wregs {};
 // Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL, IQ4_XS: thread t owns blocks (row, b) = (idx >> 2, idx & 3), idx = t and t + 256
 template <int TYPE> struct mmq_wregs<TYPE, true> {
     static constexpr bool HAS_QH = TYPE == MI355_Q5_0 || TYPE == MI355_Q5_1;
     static constexpr bool HAS_MIN = TYPE == MI355_Q4_1 || TYPE == MI355_Q5_1;
+    const uint8_t *wrow[2];
     u32x4 q[2];
     u32 qh[2];
-    u32 dm[2];   // fp16 d in the low half, fp16 m above it (HAS_MIN); IQ4_XS: the bits of the f32 block scale
-    __device__ __forceinline__ void fetch(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int64_t k0, int64_t nblk, int tid) {
+    u32 dm[2];   // fp16 d in the low half, fp16 m above it (HAS_MIN); IQ4_XS: the first word of the super-block's header, the second in qh
+    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int64_t row = row0 + ((tid + it * 256) >> 2);
+            wrow[it] = W + (row < N ? row : N - 1) * L.row_bytes;
+        }
+    }
+    __device__ __forceinline__ void fetch(const row_layout &L, int k0, int nblk, int tid) {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
             const int idx = tid + it * 256;
-            const int r = idx >> 2, b = idx & 3;
-            const int64_t row = row0 + r < N ? row0 + r : N - 1;
-            const uint8_t *wrow = W + row * L.row_bytes;
-            int64_t blk = (k0 >> 5) + b;
-            const bool live = blk < nblk;   // K is a multiple of 32: the last stage may hold fewer than four blocks
-            blk = live ? blk : nblk - 1;
+            const int b = idx & 3;
+            const uint8_t *wrow = this->wrow[it];
+            int blk = (k0 >> 5) + b;        // K is a multiple of 32: the last stage may hold fewer than four blocks, commit() zeroes the scales
+            blk = blk < nblk ? blk : nblk - 1;
             q[it] = load16w(wrow + blk * 16);
             if constexpr (HAS_QH) qh[it] = load4w(wrow + L.off_b + blk * 4);
             const int so = HAS_QH ? L.off_c : L.off_b;   // the scales follow the fifth bits where there are any
             if constexpr (TYPE == MI355_IQ4_XS) {
                 const u32x2 h = load8w(wrow + L.off_b + (blk >> 3) * 8);
-                dm[it] = __builtin_bit_cast(u32, iq4xs_block_scale(h[0], h[1], (int)(blk & 7)));
+                dm[it] = h[0];
+                qh[it] = h[1];
             } else if constexpr (HAS_MIN) dm[it] = load4w(wrow + so + blk * 4);
             else dm[it] = *(const unsigned short *)(wrow + so + blk * 2);
-            if (!live) dm[it] = 0;          // scale (and minimum) 0: the block adds nothing
         }
     }
-    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *sWo, int tid) const {
+    // k0: the stage that was fetched.  Nothing of a loaded value is touched before this point: a conversion at the load would wait for it.
+    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *sWo, int k0, int nblk, int tid) const {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
             const int idx = tid + it * 256;
@@ -173,9 +117,9 @@ template <int TYPE> struct mmq_wregs<TYPE, true> {
                     a |= spread4(qh[it] >> (4 * i));
                     c |= spread4(qh[it] >> (16 + 4 * i));
                 }
-                if constexpr (TYPE == MI355_Q4_0) {          // nibble - 8 per byte without cross-byte borrow
-                    a = ((a | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-                    c = ((c | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
+                if constexpr (TYPE == MI355_Q4_0) {          // 16 * (nibble - 8): the nibble in the upper half of the byte, its top bit flipped
+                    a = ((q[it][i] << 4) & 0xF0F0F0F0u) ^ 0x80808080u;
+                    c = (q[it][i] & 0xF0F0F0F0u) ^ 0x80808080u;
                 } else if constexpr (TYPE == MI355_Q5_0) {   // level - 16
                     a = ((a | 0x80808080u) - 0x10101010u) ^ 0x80808080u;
                     c = ((c | 0x80808080u) - 0x10101010u) ^ 0x80808080u;
@@ -186,67 +130,135 @@ template <int TYPE> struct mmq_wregs<TYPE, true> {
                 lo[i] = a;
                 hi[i] = c;
             }
-            *(u32x4 *)(sW + r * MMQ_LDK + b * 32) = lo;
-            *(u32x4 *)(sW + r * MMQ_LDK + b * 32 + 16) = hi;
-            if constexpr (TYPE == MI355_IQ4_XS) sWs[b * MMQ_BM + r] = __builtin_bit_cast(float, dm[it]);
-            else sWs[b * MMQ_BM + r] = half_bits_to_float((unsigned short)(dm[it] & 0xFFFFu));
-            if constexpr (HAS_MIN) sWo[b * MMQ_BM + r] = half_bits_to_float((unsigned short)(dm[it] >> 16));
+            *(u32x4 *)(sW + mmq_chunk(r, 2 * b)) = lo;
+            *(u32x4 *)(sW + mmq_chunk(r, 2 * b + 1)) = hi;
+            const u32 dm = (k0 >> 5) + b < nblk ? this->dm[it] : 0;   // past the end: scale (and minimum) 0, the block adds nothing
+            if constexpr (TYPE == MI355_IQ4_XS) sWs[b * MMQ_BM + r] = iq4xs_block_scale(dm, qh[it], ((k0 >> 5) + b) & 7);
+            else if constexpr (TYPE == MI355_Q4_0) sWs[b * MMQ_BM + r] = half_bits_to_float((unsigned short)(dm & 0xFFFFu)) * 0.0625f;
+            else sWs[b * MMQ_BM + r] = half_bits_to_float((unsigned short)(dm & 0xFFFFu));
+            if constexpr (HAS_MIN) sWo[b * MMQ_BM + r] = half_bits_to_float((unsigned short)(dm >> 16));
         }
     }
 };
 template <> struct mmq_wregs<MI355_Q8_0, false> {
+    const uint8_t *wrow[4];
     u32x4 q[4];
     unsigned short d[4];
-    __device__ __forceinline__ void fetch(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int64_t k0, int64_t nblk, int tid) {
+    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
+#pragma unroll
+        for (int it = 0; it < 4; it++) {
+            const int64_t row = row0 + ((tid + it * 256) >> 3);
+            wrow[it] = W + (row < N ? row : N - 1) * L.row_bytes;
+        }
+    }
+    __device__ __forceinline__ void fetch(const row_layout &L, int k0, int nblk, int tid) {
 #pragma unroll
         for (int it = 0; it < 4; it++) {
             const int idx = tid + it * 256;
-            const int r = idx >> 3, c = idx & 7;   // c: 16-byte piece of the stage
-            const int64_t row = row0 + r < N ? row0 + r : N - 1;
-            const uint8_t *wrow = W + row * L.row_bytes;
-            int64_t blk = (k0 >> 5) + (c >> 1);   // both pieces of a block read its scale
-            const bool live = blk < nblk;
-            blk = live ? blk : nblk - 1;
+            const int c = idx & 7;   // 16-byte piece of the stage
+            const uint8_t *wrow = this->wrow[it];
+            int blk = (k0 >> 5) + (c >> 1);   // both pieces of a block read its scale
+            blk = blk < nblk ? blk : nblk - 1;
             q[it] = load16w(wrow + blk * 32 + (c & 1) * 16);
             d[it] = *(const unsigned short *)(wrow + L.off_b + blk * 2);
-            if (!live) d[it] = 0;
         }
     }
-    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *, int tid) const {
+    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *, int k0, int nblk, int tid) const {
 #pragma unroll
         for (int it = 0; it < 4; it++) {
             const int idx = tid + it * 256;
             const int r = idx >> 3, c = idx & 7;
-            *(u32x4 *)(sW + r * MMQ_LDK + c * 16) = q[it];
-            if ((c & 1) == 0) sWs[(c >> 1) * MMQ_BM + r] = half_bits_to_float(d[it]);
+            *(u32x4 *)(sW + mmq_chunk(r, c)) = q[it];
+            if ((c & 1) == 0) sWs[(c >> 1) * MMQ_BM + r] = half_bits_to_float((k0 >> 5) + (c >> 1) < nblk ? d[it] : (unsigned short)0);
         }
     }
 };
+// Q4_K, Q5_K: stage = half a super-block, sub-blocks 4 half .. + 4, 64 B of qs per row = 4 pieces of 16 B; thread t owns the pieces
+// (row, p) = (idx >> 2, idx & 3) and the (scale, min) of sub-block p of the stage.  Q5_K: bit j of qh[l] is the fifth bit of element l of
+// sub-block j (dequantize_row_q5_K, ggml/src/ggml-quants.c:1482-1507)
+template <int TYPE> struct mmq_wregs_k45 {
+    static constexpr int BB = TYPE == MI355_Q4_K ? Q4_K_BYTES : Q5_K_BYTES, QS = TYPE == MI355_Q4_K ? 16 : 48;
+    const uint8_t *wrow[2];
+    u32x4 q[2], hdr[2], qh[2];
+    int half;
+    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int64_t row = row0 + ((tid + it * 256) >> 2);
+            wrow[it] = W + (row < N ? row : N - 1) * L.row_bytes;
+        }
+    }
+    __device__ __forceinline__ void fetch(const row_layout &L, int k0, int, int tid) {
+        half = (int)((k0 >> 7) & 1);
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int idx = tid + it * 256;
+            const int p = idx & 3;
+            const uint8_t *blk = wrow[it] + (k0 >> 8) * BB;
+            q[it] = load16w(blk + QS + (half * 2 + (p >> 1)) * 32 + (p & 1) * 16);
+            hdr[it] = load16w(blk);
+            if constexpr (TYPE == MI355_Q5_K) qh[it] = load16w(blk + 16 + (p & 1) * 16);
+        }
+    }
+    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *sWo, int, int, int tid) const {
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int idx = tid + it * 256;
+            const int r = idx >> 2, p = idx & 3, gl = p >> 1, h = p & 1;   // piece p: half h of group gl of the stage
+            u32x4 lo, hi;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                lo[i] = q[it][i] & 0x0F0F0F0Fu;
+                hi[i] = (q[it][i] >> 4) & 0x0F0F0F0Fu;
+                if constexpr (TYPE == MI355_Q5_K) {
+                    const int ja = half * 4 + 2 * gl;   // sub-block of the low nibbles; the high nibbles are the next one
+                    lo[i] |= ((qh[it][i] >> ja) & 0x01010101u) << 4;
+                    hi[i] |= ((qh[it][i] >> (ja + 1)) & 0x01010101u) << 4;
+                }
+            }
+            *(u32x4 *)(sW + mmq_chunk(r, 4 * gl + h)) = lo;
+            *(u32x4 *)(sW + mmq_chunk(r, 4 * gl + 2 + h)) = hi;
+            int sc, mn;
+            q4k_scale_min(hdr[it][1], hdr[it][2], hdr[it][3], half * 4 + p, sc, mn);
+            sWs[p * MMQ_BM + r] = half_bits_to_float((unsigned short)(hdr[it][0] & 0xFFFFu)) * (float)sc;
+            sWo[p * MMQ_BM + r] = -(half_bits_to_float((unsigned short)(hdr[it][0] >> 16)) * (float)mn);
+        }
+    }
+};
+template <> struct mmq_wregs<MI355_Q4_K, false> : mmq_wregs_k45<MI355_Q4_K> {};
+template <> struct mmq_wregs<MI355_Q5_K, false> : mmq_wregs_k45<MI355_Q5_K> {};
 // stage = half hf of a super-block: 64 B of ql + 32 B of qh, 8 scales of 16 elements; thread t owns the 16-byte pieces (row, p) = (idx >> 2, idx & 3)
 template <> struct mmq_wregs<MI355_Q6_K, false> {
+    const uint8_t *wrow[2];
     u32x4 ql[2], qh[2];
     unsigned short d[2], sc[2];   // super-block scale; the int8 scales of groups 2p and 2p + 1
-    __device__ __forceinline__ void fetch(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int64_t k0, int64_t, int tid) {
-        const int64_t sb = k0 >> 8;
+    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int64_t row = row0 + ((tid + it * 256) >> 2);
+            wrow[it] = W + (row < N ? row : N - 1) * L.row_bytes;
+        }
+    }
+    __device__ __forceinline__ void fetch(const row_layout &L, int k0, int, int tid) {
+        const int sb = k0 >> 8;
         const int hf = (int)((k0 >> 7) & 1);
 #pragma unroll
         for (int it = 0; it < 2; it++) {
             const int idx = tid + it * 256;
-            const int r = idx >> 2, p = idx & 3;
-            const int64_t row = row0 + r < N ? row0 + r : N - 1;
-            const uint8_t *wrow = W + row * L.row_bytes;
+            const int p = idx & 3;
+            const uint8_t *wrow = this->wrow[it];
             ql[it] = load16w(wrow + sb * 128 + hf * 64 + p * 16);
             qh[it] = load16w(wrow + L.off_b + sb * 64 + hf * 32 + 16 * (p & 1));
             sc[it] = *(const unsigned short *)(wrow + L.off_c + sb * 16 + hf * 8 + 2 * p);
             d[it] = *(const unsigned short *)(wrow + L.off_d + sb * 2);
         }
     }
-    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *, int tid) const {
+    __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *, int k0, int nblk, int tid) const {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
             const int idx = tid + it * 256;
             const int r = idx >> 2, p = idx & 3;
-            const int l0 = 16 * (p & 1), qa = p >> 1;
+            const int qa = p >> 1;
             u32x4 vA, vB;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -258,8 +270,8 @@ template <> struct mmq_wregs<MI355_Q6_K, false> {
                 vA[i] = ta | (ma << 1) | (ma << 2);
                 vB[i] = tb | (mb << 1) | (mb << 2);
             }
-            *(u32x4 *)(sW + r * MMQ_LDK + qa * 32 + l0) = vA;
-            *(u32x4 *)(sW + r * MMQ_LDK + (qa + 2) * 32 + l0) = vB;
+            *(u32x4 *)(sW + mmq_chunk(r, 2 * qa + (p & 1))) = vA;
+            *(u32x4 *)(sW + mmq_chunk(r, 2 * qa + 4 + (p & 1))) = vB;
             const float df = half_bits_to_float(d[it]);
             sWs[(2 * p) * MMQ_BM + r] = df * (float)(int)(signed char)(sc[it] & 0xFFu);
             sWs[(2 * p + 1) * MMQ_BM + r] = df * (float)(int)(signed char)(sc[it] >> 8);
@@ -268,46 +280,55 @@ template <> struct mmq_wregs<MI355_Q6_K, false> {
 };
 template <int BN, bool WITH_SUM> struct mmq_aregs {
     static constexpr int NQ = BN * 8 / 256, NS = (BN * 4 + 255) / 256;
+    const int8_t *arow[NQ];
+    const act_ds *srow[NS];
     u32x4 q[NQ];
     float d[NS];
     int sum[NS];
     // row_of: null, or the activation row of every column (the routed form: columns are (token, expert slot) pairs sorted by expert)
-    __device__ __forceinline__ void fetch(const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, int64_t col0, int64_t B, int64_t K, int64_t k0,
-                                          int tid, const int32_t *__restrict__ row_of = nullptr) {
-        const int64_t nblk = K >> 5;
+    __device__ __forceinline__ void init(const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, int64_t col0, int64_t B, int64_t K, int tid,
+                                         const int32_t *__restrict__ row_of) {
 #pragma unroll
         for (int it = 0; it < NQ; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 3, c = idx & 7;
+            const int r = (tid + it * 256) >> 3;
             int64_t col = col0 + r < B ? col0 + r : B - 1;
             if (row_of) col = row_of[col];
-            const int64_t k = k0 + c * 16 < K ? k0 + c * 16 : K - 16;   // past the end: any bytes, the weight scales there are 0
-            q[it] = load16(aq + col * K + k);
+            arow[it] = aq + col * K;
         }
 #pragma unroll
         for (int it = 0; it < NS; it++) {
-            const int idx = tid + it * 256;
-            const int r = (idx >> 2) < BN ? (idx >> 2) : BN - 1, b = idx & 3;
+            const int i = (tid + it * 256) >> 2, r = i < BN ? i : BN - 1;
             int64_t col = col0 + r < B ? col0 + r : B - 1;
             if (row_of) col = row_of[col];
-            const int64_t blk = (k0 >> 5) + b < nblk ? (k0 >> 5) + b : nblk - 1;
-            const act_ds e = ads[col * nblk + blk];
+            srow[it] = ads + col * (K >> 5);
+        }
+    }
+    __device__ __forceinline__ void fetch(int k0, int nblk, int tid) {
+#pragma unroll
+        for (int it = 0; it < NQ; it++) {
+            const int k = k0 + (tid & 7) * 16, last = nblk * 32 - 16;
+            q[it] = load16(arow[it] + (k < last ? k : last));   // past the end: any bytes, the weight scales there are 0
+        }
+#pragma unroll
+        for (int it = 0; it < NS; it++) {
+            const int blk = (k0 >> 5) + (tid & 3);
+            const act_ds e = srow[it][blk < nblk ? blk : nblk - 1];
             d[it] = e.d;
             if constexpr (WITH_SUM) sum[it] = e.sum;
         }
     }
-    __device__ __forceinline__ void commit(int8_t *sA, float *sAd, float *sAs, int tid) const {
+    __device__ __forceinline__ void commit(int8_t *sA, _Float16 *sAd, float *sAs, int tid) const {
 #pragma unroll
         for (int it = 0; it < NQ; it++) {
             const int idx = tid + it * 256;
             const int r = idx >> 3, c = idx & 7;
-            *(u32x4 *)(sA + r * MMQ_LDK + c * 16) = q[it];
+            *(u32x4 *)(sA + mmq_chunk(r, c)) = q[it];
         }
 #pragma unroll
         for (int it = 0; it < NS; it++) {
             const int idx = tid + it * 256;
             if (idx < BN * 4) {
-                sAd[(idx & 3) * BN + (idx >> 2)] = d[it];
+                sAd[(idx & 3) * BN + mmq_dx_slot(idx >> 2)] = (_Float16)d[it];   // exact: d is f16-rounded
                 if constexpr (WITH_SUM) sAs[(idx & 3) * BN + (idx >> 2)] = d[it] * (float)sum[it];
             }
         }
@@ -325,19 +346,21 @@ struct mmq32_route {
 };
 
 template <int TYPE, int TN, bool ID = false>
-__global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq,
+__global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq,
                                              const act_ds *__restrict__ ads, float *__restrict__ dst, int64_t N,
                                              int64_t K, int64_t B, int64_t dst_stride, row_layout L, int n_col_tiles,
                                              int n_groups, int n_groups_padded, mmq32_route route) {
     typedef mmq_cfg<TYPE> C;
-    static_assert(!ID || C::PREFETCH, "the routed form gathers activation rows in the register-staged loads");
     constexpr int BN = 64 * TN;
-    __shared__ __attribute__((aligned(16))) int8_t sW[MMQ_BM * MMQ_LDK];
-    __shared__ __attribute__((aligned(16))) int8_t sA[BN * MMQ_LDK];
-    __shared__ __attribute__((aligned(16))) float sWs[C::NG * MMQ_BM];
-    __shared__ __attribute__((aligned(16))) float sAd[4 * BN];
-    __shared__ __attribute__((aligned(16))) float sWo[C::MIN ? MMQ_BM * 4 : 4];
-    __shared__ __attribute__((aligned(16))) float sAs[C::MIN ? BN * 4 : 4];
+    struct stage_mem {
+        __attribute__((aligned(16))) int8_t w[MMQ_BM * MMQ_BK];
+        __attribute__((aligned(16))) int8_t a[BN * MMQ_BK];
+        __attribute__((aligned(16))) float ws[C::NG * MMQ_BM];
+        __attribute__((aligned(16))) _Float16 ad[4 * BN];
+        __attribute__((aligned(16))) float wo[C::MIN ? MMQ_BM * 4 : 4];
+        __attribute__((aligned(16))) float as[C::MIN ? BN * 4 : 4];
+    };
+    __shared__ stage_mem sm[2];
 
     // XCD-aware id: hardware deals group ids round-robin over 8 XCDs; make logical neighbours share an XCD
     const int per_xcd = n_groups_padded >> 3;
@@ -368,90 +391,108 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[tb][tw][r] = 0.0f;
 
+    i32x16 magic;
+#pragma unroll
+    for (int r = 0; r < 16; r++) magic[r] = MMQ_MAGIC_BITS;
+
     // split K: grid row y walks stages [k_lo, k_hi) and writes its sums to slice y of `dst` (a workspace then, see launch_mmq)
-    const int64_t nblk = K >> 5, stages = (K + MMQ_BK - 1) / MMQ_BK, st_per = (stages + gridDim.y - 1) / gridDim.y;
-    const int64_t k_lo = (int64_t)blockIdx.y * st_per * MMQ_BK;
-    const int64_t k_hi = k_lo + st_per * MMQ_BK < K ? k_lo + st_per * MMQ_BK : K;
+    const int nblk = (int)(K >> 5), stages = (nblk + MMQ_BK / QK - 1) / (MMQ_BK / QK), st_per = (stages + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int s_lo = (int)blockIdx.y * st_per, s_hi = s_lo + st_per < stages ? s_lo + st_per : stages;
     if (gridDim.y > 1) dst += (int64_t)blockIdx.y * B * dst_stride;
 
-    constexpr bool PREFETCH = C::PREFETCH;
     mmq_wregs<TYPE> wregs;
     mmq_aregs<BN, C::MIN> aregs;
-    if constexpr (PREFETCH) {
-        wregs.fetch(W, L, row0, N, k_lo, nblk, threadIdx.x);
-        aregs.fetch(aq, ads, col0, B, K, k_lo, threadIdx.x, row_of);
-    }
-    for (int64_t k0 = k_lo; k0 < k_hi; k0 += MMQ_BK) {
-        __syncthreads();
-        if constexpr (PREFETCH) {
-            wregs.commit(sW, sWs, sWo, threadIdx.x);
-            aregs.commit(sA, sAd, sAs, threadIdx.x);
-        } else {
-            load_weight_stage<TYPE>(W, L, row0, N, k0, sW, sWs, sWo);
-            load_act_stage<TYPE, BN>(aq, ads, col0, B, K, k0, sA, sAd, sAs);
-        }
-        __syncthreads();
-        if constexpr (PREFETCH) {
-            // past the end the last stage is requested again and never committed: no branch, the loads stay here
-            const int64_t k1 = k0 + MMQ_BK < k_hi ? k0 + MMQ_BK : k0;
-            wregs.fetch(W, L, row0, N, k1, nblk, threadIdx.x);
-            aregs.fetch(aq, ads, col0, B, K, k1, threadIdx.x, row_of);
-            __builtin_amdgcn_sched_barrier(0);   // requested now, a whole stage ahead of their commit
-        }
+    wregs.init(W, L, row0, N, threadIdx.x);
+    aregs.init(aq, ads, col0, B, K, threadIdx.x, row_of);
+    auto fetch = [&](int st) {
+        wregs.fetch(L, st * MMQ_BK, nblk, threadIdx.x);
+        aregs.fetch(st * MMQ_BK, nblk, threadIdx.x);
+    };
+    auto commit = [&](stage_mem &m, int st) {
+        wregs.commit(m.w, m.ws, m.wo, st * MMQ_BK, nblk, threadIdx.x);
+        aregs.commit(m.a, m.ad, m.as, threadIdx.x);
+    };
 
+    // operands and scales of one Q8_1 block for the wave's tiles
+    constexpr int NS = C::G == 32 ? 1 : 2;   // scale groups per block
+    struct block_ops { i32x4 a[TN], w[2]; };
+    struct block_scales {
+        f16x8 dx[TN][2];     // activation block scales of this lane's 16 rows per tile
+        float dw[2][NS];
+    };
+    const int a_at = mmq_chunk(wcol0 + l32, lhi), w_at = mmq_chunk(wrow0 + l32, lhi);
+    auto load_ops = [&](const stage_mem &m, int ks) {
+        block_ops f;
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) {   // one Q8_1 block per step
-            // activation block scales for this lane's 16 D rows: i = 8*(r/4) + 4*lhi + r%4
-            f32x4 dx[TN][4];
+        for (int tb = 0; tb < TN; tb++) f.a[tb] = *(const i32x4 *)(m.a + tb * 32 * MMQ_BK + (a_at ^ (ks << 5)));   // chunk 2 ks + lhi
 #pragma unroll
-            for (int tb = 0; tb < TN; tb++)
+        for (int tw = 0; tw < 2; tw++) f.w[tw] = *(const i32x4 *)(m.w + tw * 32 * MMQ_BK + (w_at ^ (ks << 5)));
+        return f;
+    };
+    auto load_scales = [&](const stage_mem &m, int ks) {
+        block_scales f;
 #pragma unroll
-                for (int q = 0; q < 4; q++) dx[tb][q] = *(const f32x4 *)(sAd + ks * BN + wcol0 + tb * 32 + 8 * q + 4 * lhi);
+        for (int tb = 0; tb < TN; tb++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) f.dx[tb][h] = *(const f16x8 *)(m.ad + ks * BN + wcol0 + tb * 32 + 16 * lhi + 8 * h);
+#pragma unroll
+        for (int tw = 0; tw < 2; tw++)
+#pragma unroll
+            for (int h = 0; h < NS; h++) f.dw[tw][h] = m.ws[(ks * NS + h) * MMQ_BM + wrow0 + tw * 32 + l32];
+        return f;
+    };
+    // matrix instruction n of a block: tile (tb, tw), scale group h.  Two groups of 16 (Q6_K): the operands hold 16 consecutive elements
+    // per lane half, so group h is the half lhi == h, and the other half of the weights is zeroed.
+    constexpr int NM = TN * 2 * NS;
+    auto mma = [&](const block_ops &f, int n) {
+        const int tb = n / NS % TN, tw = n / NS / TN, h = n % NS;
+        i32x4 w = f.w[tw];
+        if constexpr (NS == 2) {
+            const int keep = lhi == h ? -1 : 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[i] &= keep;
+        }
+        return __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[tb], w, magic, 0, 0, 0);
+    };
+    auto scale = [&](const block_scales &f, int n, const i32x16 &I) {
+        const int tb = n / NS % TN, tw = n / NS / TN, h = n % NS;
+        const float dw = f.dw[tw][h], mdw = -MMQ_MAGIC * dw;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int bits = I[r];
+            acc[tb][tw][r] = __builtin_fmaf(__builtin_fmaf(__builtin_bit_cast(float, bits), dw, mdw), (float)f.dx[tb][r >> 3][r & 7], acc[tb][tw][r]);
+        }
+    };
 
-            if constexpr (C::G == 32) {
-                i32x4 af[TN], bf[2];
+    fetch(s_lo);
+    commit(sm[0], s_lo);
+    fetch(s_lo + 1 < s_hi ? s_lo + 1 : s_lo);
+    __syncthreads();
+    int buf = 0;
+    for (int st = s_lo; st < s_hi; st++, buf ^= 1) {
+        const stage_mem &m = sm[buf];
+        // One matrix instruction is always in flight: its successor is issued before its sums are scaled, so that neither waits for the
+        // other (left to the compiler, all of them write the same registers one after the other); the next block's operands are read
+        // from LDS while the last sums of this one are scaled.
+        block_ops f = load_ops(m, 0);
+        block_scales sc = load_scales(m, 0);
+        i32x16 I = mma(f, 0);
 #pragma unroll
-                for (int tb = 0; tb < TN; tb++) af[tb] = *(const i32x4 *)(sA + (wcol0 + tb * 32 + l32) * MMQ_LDK + ks * 32 + 16 * lhi);
+        for (int ks = 0; ks < 4; ks++) {
+            block_scales sc_next = sc;
 #pragma unroll
-                for (int tw = 0; tw < 2; tw++) bf[tw] = *(const i32x4 *)(sW + (wrow0 + tw * 32 + l32) * MMQ_LDK + ks * 32 + 16 * lhi);
-#pragma unroll
-                for (int tw = 0; tw < 2; tw++) {
-                    const float dw = sWs[ks * MMQ_BM + wrow0 + tw * 32 + l32];
-#pragma unroll
-                    for (int tb = 0; tb < TN; tb++) {
-                        i32x16 z;
-#pragma unroll
-                        for (int r = 0; r < 16; r++) z[r] = 0;
-                        const i32x16 I = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[tb], bf[tw], z, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 16; r++) acc[tb][tw][r] += (float)I[r] * (dw * dx[tb][r >> 2][r & 3]);
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int hs = 0; hs < 2; hs++) {   // two 16-element scale groups per block
-                    long af[TN], bf[2];
-#pragma unroll
-                    for (int tb = 0; tb < TN; tb++) af[tb] = *(const long *)(sA + (wcol0 + tb * 32 + l32) * MMQ_LDK + ks * 32 + hs * 16 + 8 * lhi);
-#pragma unroll
-                    for (int tw = 0; tw < 2; tw++) bf[tw] = *(const long *)(sW + (wrow0 + tw * 32 + l32) * MMQ_LDK + ks * 32 + hs * 16 + 8 * lhi);
-#pragma unroll
-                    for (int tw = 0; tw < 2; tw++) {
-                        const float dw = sWs[(ks * 2 + hs) * MMQ_BM + wrow0 + tw * 32 + l32];
-#pragma unroll
-                        for (int tb = 0; tb < TN; tb++) {
-                            i32x16 z;
-#pragma unroll
-                            for (int r = 0; r < 16; r++) z[r] = 0;
-                            const i32x16 I = __builtin_amdgcn_mfma_i32_32x32x16_i8(af[tb], bf[tw], z, 0, 0, 0);
-#pragma unroll
-                            for (int r = 0; r < 16; r++) acc[tb][tw][r] += (float)I[r] * (dw * dx[tb][r >> 2][r & 3]);
-                        }
-                    }
-                }
+            for (int n = 0; n < NM; n++) {
+                const i32x16 cur = I;
+                I = mma(f, n + 1 < NM ? n + 1 : 0);   // (the last one of a stage is not used)
+                __builtin_amdgcn_sched_barrier(0);
+                if (n == NM - 2 && ks < 3) f = load_ops(m, ks + 1);
+                if (n == NM - 1 && ks < 3) sc_next = load_scales(m, ks + 1);
+                scale(sc, n, cur);
+                asm volatile("" : "+v"(acc[n / NS % TN][n / NS / TN]));   // formed here, and not behind the matrix instructions of the whole stage
+                __builtin_amdgcn_sched_barrier(0);
             }
+            sc = sc_next;
         }
-
         if constexpr (C::MIN) {
             // acc += sum_b (dx * sum q)[i][b] * m[j][b] over the 4 blocks of the stage (Q4_K, Q5_K: m = -dmin * 6-bit minimum): two
             // v_mfma_f32_32x32x2_f32 per tile on the matrix pipe, which waits for the vector ALUs anyway; k = lane / 32.  In f32 as the
@@ -460,15 +501,19 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
             for (int p = 0; p < 2; p++) {
                 float af[TN], bf[2];
 #pragma unroll
-                for (int tb = 0; tb < TN; tb++) af[tb] = sAs[(2 * p + lhi) * BN + wcol0 + tb * 32 + l32];
+                for (int tb = 0; tb < TN; tb++) af[tb] = m.as[(2 * p + lhi) * BN + wcol0 + tb * 32 + l32];
 #pragma unroll
-                for (int tw = 0; tw < 2; tw++) bf[tw] = sWo[(2 * p + lhi) * MMQ_BM + wrow0 + tw * 32 + l32];
+                for (int tw = 0; tw < 2; tw++) bf[tw] = m.wo[(2 * p + lhi) * MMQ_BM + wrow0 + tw * 32 + l32];
 #pragma unroll
                 for (int tb = 0; tb < TN; tb++)
 #pragma unroll
                     for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
             }
         }
+        // the next stage, requested one stage ago, goes to the other buffer; past the end the last stage is requested again and never used
+        commit(sm[buf ^ 1], st + 1);
+        fetch(st + 2 < s_hi ? st + 2 : st);
+        __syncthreads();
     }
 
     // store: lane holds weight row j = l32 of each 32-wide tile, 16 activation rows
@@ -485,6 +530,12 @@ __global__ void __launch_bounds__(256) k_mmq(const uint8_t *__restrict__ W, cons
         }
 }
 
+// What bounds the kernel is the vector ALU: a wave issues 637 of its instructions per stage, 512 of them the two per block sum and 16
+// matrix instructions, which are busy a quarter of that time (counters, Q4_0 14336 x 4096, 512 rows; 4 cycles each = 2550 cycles of the
+// 2800 a stage takes with one group per compute unit).  Before the two-instruction form, the double-buffered stages and the f32 minima, by
+// type (14336 x 4096, 512 rows with the quantization launch, us): Q4_0 139 -> 116, Q4_1 228 -> 128, Q5_0 149 -> 124, Q5_1 229 -> 140,
+// IQ4_NL 149 -> 128, Q8_0 146 -> 130; 64 rows: Q4_0 34.3 -> 32.3.
+//
 // A product with few tiles leaves most of the chip idle while each group walks all of K: such launches are cut along K into
 // slices that run side by side and a second launch adds the slices in fixed order.  At least four stages per slice, at most
 // eight slices, at most two groups per compute unit.
