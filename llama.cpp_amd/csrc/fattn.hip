@@ -590,8 +590,11 @@ int mi355_flash_attn_ext_quant(void *stream, const float *q, const void *k, cons
     if (frc != MI355_OK) return frc;
     const int R = (int)(Hq / Hkv);
     hipStream_t s = (hipStream_t)stream;
-    if (Nq >= 16 && act == nullptr) {   // prefill: f16 matrix cores
+    if (Nq >= 16) {   // prefill: f16 matrix cores
         const int rc = launch_fattn_mma(s, a, D, ws_bytes);
+        // the quantized rows by a launch of their own: a few us, where the vector kernel, which writes them itself, takes ten times as
+        // long as the matrix-core one (512 x 512 cells, 32 / 8 heads: 200 against 20 us)
+        if (rc == MI355_OK && act != nullptr) return mi355_quantize_act(stream, dst, act, Hq * D, Nq, Hq * D);
         if (rc <= 0) return rc;
     }
     // Decode and small batches over a long context: matrix cores with (token, head) columns, which read a kv head's

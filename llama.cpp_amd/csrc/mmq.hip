@@ -68,47 +68,59 @@ template <int TYPE> struct mmq_cfg {
 // sWs : float [NG][MMQ_BM]   (scale g of row r at sWs[g*MMQ_BM + r])
 // sWo : float [4][MMQ_BM]    (types with a block minimum: what multiplies d_x * sum(q) of the stage's 4 blocks)
 // sA  : int8 [BN][MMQ_BK] (mmq_chunk);  sAd : f16 [4][BN] block scales (mmq_dx_slot);  sAs : float [4][BN]  dx*sum(q) (types with a block minimum)
+// The rows a thread loads from: uniform base of the tile + a 32-bit offset per row (64-bit pointers per row are twice the registers, and
+// the spills they caused took Q8_0 14336 x 4096 at 512 rows from 130 to 193 us).  A tile of 128 rows spans less than 4 GiB: launch_mmq.
+__device__ __forceinline__ uint64_t uniform_addr(const void *p) {   // into scalar registers: 64-bit products of uniform values are formed by the vector ALU
+    const uint64_t u = (uint64_t)p;
+    return (uint64_t)(u32)__builtin_amdgcn_readfirstlane((u32)u) | ((uint64_t)(u32)__builtin_amdgcn_readfirstlane((u32)(u >> 32)) << 32);
+}
+template <class T> __device__ __forceinline__ T global_load(uint64_t base, u32 off) {
+    return *(const T __attribute__((address_space(1))) *)(base + off);
+}
+template <int NR, int TPR> struct mmq_rows {
+    uint64_t base;
+    u32 off[NR];
+    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
+        base = uniform_addr(W + row0 * L.row_bytes);
+        const int last = (int)(N - 1 - row0 < MMQ_BM - 1 ? N - 1 - row0 : MMQ_BM - 1);   // rows past the end repeat the last one and are not stored
+#pragma unroll
+        for (int it = 0; it < NR; it++) {
+            const int r = tid / TPR + it * (256 / TPR);
+            off[it] = (u32)(r < last ? r : last) * (u32)L.row_bytes;
+        }
+    }
+};
 template <int TYPE, bool NIB = mmq_cfg<TYPE>::NIBBLE32> struct mmq_wregs {};
-// Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL, IQ4_XS: thread t owns blocks (row, b) = (idx >> 2, idx & 3), idx = t and t + 256
-template <int TYPE> struct mmq_wregs<TYPE, true> {
+// Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL, IQ4_XS: thread t owns blocks (row, b) = (t >> 2, t & 3) and (64 + (t >> 2), t & 3)
+template <int TYPE> struct mmq_wregs<TYPE, true> : mmq_rows<2, 4> {
     static constexpr bool HAS_QH = TYPE == MI355_Q5_0 || TYPE == MI355_Q5_1;
     static constexpr bool HAS_MIN = TYPE == MI355_Q4_1 || TYPE == MI355_Q5_1;
-    const uint8_t *wrow[2];
     u32x4 q[2];
     u32 qh[2];
     u32 dm[2];   // fp16 d in the low half, fp16 m above it (HAS_MIN); IQ4_XS: the first word of the super-block's header, the second in qh
-    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-            const int64_t row = row0 + ((tid + it * 256) >> 2);
-            wrow[it] = W + (row < N ? row : N - 1) * L.row_bytes;
-        }
-    }
     __device__ __forceinline__ void fetch(const row_layout &L, int k0, int nblk, int tid) {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int b = idx & 3;
-            const uint8_t *wrow = this->wrow[it];
+            const int b = tid & 3;
+            const u32 wrow = off[it];
             int blk = (k0 >> 5) + b;        // K is a multiple of 32: the last stage may hold fewer than four blocks, commit() zeroes the scales
             blk = blk < nblk ? blk : nblk - 1;
-            q[it] = load16w(wrow + blk * 16);
-            if constexpr (HAS_QH) qh[it] = load4w(wrow + L.off_b + blk * 4);
+            q[it] = global_load<u32x4_a2>(base, wrow + blk * 16);
+            if constexpr (HAS_QH) qh[it] = global_load<u32_a2>(base, wrow + L.off_b + blk * 4);
             const int so = HAS_QH ? L.off_c : L.off_b;   // the scales follow the fifth bits where there are any
             if constexpr (TYPE == MI355_IQ4_XS) {
-                const u32x2 h = load8w(wrow + L.off_b + (blk >> 3) * 8);
+                const u32x2 h = global_load<u32x2_a2>(base, wrow + L.off_b + (blk >> 3) * 8);
                 dm[it] = h[0];
                 qh[it] = h[1];
-            } else if constexpr (HAS_MIN) dm[it] = load4w(wrow + so + blk * 4);
-            else dm[it] = *(const unsigned short *)(wrow + so + blk * 2);
+            } else if constexpr (HAS_MIN) dm[it] = global_load<u32_a2>(base, wrow + so + blk * 4);
+            else dm[it] = global_load<unsigned short>(base, wrow + so + blk * 2);
         }
     }
     // k0: the stage that was fetched.  Nothing of a loaded value is touched before this point: a conversion at the load would wait for it.
     __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *sWo, int k0, int nblk, int tid) const {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 2, b = idx & 3;
+            const int r = (tid >> 2) + 64 * it, b = tid & 3;
             u32x4 lo, hi;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -140,71 +152,51 @@ template <int TYPE> struct mmq_wregs<TYPE, true> {
         }
     }
 };
-template <> struct mmq_wregs<MI355_Q8_0, false> {
-    const uint8_t *wrow[4];
+template <> struct mmq_wregs<MI355_Q8_0, false> : mmq_rows<4, 8> {
     u32x4 q[4];
     unsigned short d[4];
-    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
-#pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int64_t row = row0 + ((tid + it * 256) >> 3);
-            wrow[it] = W + (row < N ? row : N - 1) * L.row_bytes;
-        }
-    }
     __device__ __forceinline__ void fetch(const row_layout &L, int k0, int nblk, int tid) {
 #pragma unroll
         for (int it = 0; it < 4; it++) {
-            const int idx = tid + it * 256;
-            const int c = idx & 7;   // 16-byte piece of the stage
-            const uint8_t *wrow = this->wrow[it];
+            const int c = tid & 7;   // 16-byte piece of the stage
+            const u32 wrow = off[it];
             int blk = (k0 >> 5) + (c >> 1);   // both pieces of a block read its scale
             blk = blk < nblk ? blk : nblk - 1;
-            q[it] = load16w(wrow + blk * 32 + (c & 1) * 16);
-            d[it] = *(const unsigned short *)(wrow + L.off_b + blk * 2);
+            q[it] = global_load<u32x4_a2>(base, wrow + blk * 32 + (c & 1) * 16);
+            d[it] = global_load<unsigned short>(base, wrow + L.off_b + blk * 2);
         }
     }
     __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *, int k0, int nblk, int tid) const {
 #pragma unroll
         for (int it = 0; it < 4; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 3, c = idx & 7;
+            const int r = (tid >> 3) + 32 * it, c = tid & 7;
             *(u32x4 *)(sW + mmq_chunk(r, c)) = q[it];
             if ((c & 1) == 0) sWs[(c >> 1) * MMQ_BM + r] = half_bits_to_float((k0 >> 5) + (c >> 1) < nblk ? d[it] : (unsigned short)0);
         }
     }
 };
 // Q4_K, Q5_K: stage = half a super-block, sub-blocks 4 half .. + 4, 64 B of qs per row = 4 pieces of 16 B; thread t owns the pieces
-// (row, p) = (idx >> 2, idx & 3) and the (scale, min) of sub-block p of the stage.  Q5_K: bit j of qh[l] is the fifth bit of element l of
+// (row, p) = (t >> 2, t & 3), (64 + (t >> 2), t & 3) and the (scale, min) of sub-block p of the stage.  Q5_K: bit j of qh[l] is the fifth bit of element l of
 // sub-block j (dequantize_row_q5_K, ggml/src/ggml-quants.c:1482-1507)
-template <int TYPE> struct mmq_wregs_k45 {
+template <int TYPE> struct mmq_wregs_k45 : mmq_rows<2, 4> {
     static constexpr int BB = TYPE == MI355_Q4_K ? Q4_K_BYTES : Q5_K_BYTES, QS = TYPE == MI355_Q4_K ? 16 : 48;
-    const uint8_t *wrow[2];
     u32x4 q[2], hdr[2], qh[2];
     int half;
-    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-            const int64_t row = row0 + ((tid + it * 256) >> 2);
-            wrow[it] = W + (row < N ? row : N - 1) * L.row_bytes;
-        }
-    }
     __device__ __forceinline__ void fetch(const row_layout &L, int k0, int, int tid) {
         half = (int)((k0 >> 7) & 1);
 #pragma unroll
         for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int p = idx & 3;
-            const uint8_t *blk = wrow[it] + (k0 >> 8) * BB;
-            q[it] = load16w(blk + QS + (half * 2 + (p >> 1)) * 32 + (p & 1) * 16);
-            hdr[it] = load16w(blk);
-            if constexpr (TYPE == MI355_Q5_K) qh[it] = load16w(blk + 16 + (p & 1) * 16);
+            const int p = tid & 3;
+            const u32 blk = off[it] + (k0 >> 8) * BB;
+            q[it] = global_load<u32x4_a2>(base, blk + QS + (half * 2 + (p >> 1)) * 32 + (p & 1) * 16);
+            hdr[it] = global_load<u32x4_a2>(base, blk);
+            if constexpr (TYPE == MI355_Q5_K) qh[it] = global_load<u32x4_a2>(base, blk + 16 + (p & 1) * 16);
         }
     }
     __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *sWo, int, int, int tid) const {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 2, p = idx & 3, gl = p >> 1, h = p & 1;   // piece p: half h of group gl of the stage
+            const int r = (tid >> 2) + 64 * it, p = tid & 3, gl = p >> 1, h = p & 1;   // piece p: half h of group gl of the stage
             u32x4 lo, hi;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -227,37 +219,27 @@ template <int TYPE> struct mmq_wregs_k45 {
 };
 template <> struct mmq_wregs<MI355_Q4_K, false> : mmq_wregs_k45<MI355_Q4_K> {};
 template <> struct mmq_wregs<MI355_Q5_K, false> : mmq_wregs_k45<MI355_Q5_K> {};
-// stage = half hf of a super-block: 64 B of ql + 32 B of qh, 8 scales of 16 elements; thread t owns the 16-byte pieces (row, p) = (idx >> 2, idx & 3)
-template <> struct mmq_wregs<MI355_Q6_K, false> {
-    const uint8_t *wrow[2];
+// stage = half hf of a super-block: 64 B of ql + 32 B of qh, 8 scales of 16 elements; thread t owns the 16-byte pieces (row, p) = (t >> 2, t & 3), (64 + (t >> 2), t & 3)
+template <> struct mmq_wregs<MI355_Q6_K, false> : mmq_rows<2, 4> {
     u32x4 ql[2], qh[2];
     unsigned short d[2], sc[2];   // super-block scale; the int8 scales of groups 2p and 2p + 1
-    __device__ __forceinline__ void init(const uint8_t *__restrict__ W, const row_layout &L, int64_t row0, int64_t N, int tid) {
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-            const int64_t row = row0 + ((tid + it * 256) >> 2);
-            wrow[it] = W + (row < N ? row : N - 1) * L.row_bytes;
-        }
-    }
     __device__ __forceinline__ void fetch(const row_layout &L, int k0, int, int tid) {
         const int sb = k0 >> 8;
         const int hf = (int)((k0 >> 7) & 1);
 #pragma unroll
         for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int p = idx & 3;
-            const uint8_t *wrow = this->wrow[it];
-            ql[it] = load16w(wrow + sb * 128 + hf * 64 + p * 16);
-            qh[it] = load16w(wrow + L.off_b + sb * 64 + hf * 32 + 16 * (p & 1));
-            sc[it] = *(const unsigned short *)(wrow + L.off_c + sb * 16 + hf * 8 + 2 * p);
-            d[it] = *(const unsigned short *)(wrow + L.off_d + sb * 2);
+            const int p = tid & 3;
+            const u32 wrow = off[it];
+            ql[it] = global_load<u32x4_a2>(base, wrow + sb * 128 + hf * 64 + p * 16);
+            qh[it] = global_load<u32x4_a2>(base, wrow + L.off_b + sb * 64 + hf * 32 + 16 * (p & 1));
+            sc[it] = global_load<unsigned short>(base, wrow + L.off_c + sb * 16 + hf * 8 + 2 * p);
+            d[it] = global_load<unsigned short>(base, wrow + L.off_d + sb * 2);
         }
     }
     __device__ __forceinline__ void commit(int8_t *sW, float *sWs, float *, int k0, int nblk, int tid) const {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 2, p = idx & 3;
+            const int r = (tid >> 2) + 64 * it, p = tid & 3;
             const int qa = p >> 1;
             u32x4 vA, vB;
 #pragma unroll
@@ -278,59 +260,58 @@ template <> struct mmq_wregs<MI355_Q6_K, false> {
         }
     }
 };
-template <int BN, bool WITH_SUM> struct mmq_aregs {
-    static constexpr int NQ = BN * 8 / 256, NS = (BN * 4 + 255) / 256;
-    const int8_t *arow[NQ];
-    const act_ds *srow[NS];
+template <int BN, bool WITH_SUM, bool ID> struct mmq_aregs {
+    static_assert(BN == 64 || BN == 128, "columns of a tile");
+    static constexpr int NQ = BN * 8 / 256, NS = BN * 4 / 256;
+    uint64_t qbase, sbase;      // uniform: first row of the tile (ID: row 0)
+    u32 qoff[NQ], soff[NS];     // the row as bytes / entries from there; ID: as blocks from row 0, since the gathered rows lie anywhere
     u32x4 q[NQ];
     float d[NS];
     int sum[NS];
-    // row_of: null, or the activation row of every column (the routed form: columns are (token, expert slot) pairs sorted by expert)
-    __device__ __forceinline__ void init(const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, int64_t col0, int64_t B, int64_t K, int tid,
+    // row_of (ID): the activation row of every column (columns are (token, expert slot) pairs sorted by expert)
+    __device__ __forceinline__ void init(const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, int64_t col0, int64_t B, int nblk, int tid,
                                          const int32_t *__restrict__ row_of) {
+        qbase = ID ? (uint64_t)aq : uniform_addr(aq + col0 * nblk * QK);
+        sbase = ID ? (uint64_t)ads : uniform_addr(ads + col0 * nblk);
+        const int last = (int)(B - 1 - col0 < BN - 1 ? B - 1 - col0 : BN - 1);   // rows past the end repeat the last one and are not stored
 #pragma unroll
         for (int it = 0; it < NQ; it++) {
-            const int r = (tid + it * 256) >> 3;
-            int64_t col = col0 + r < B ? col0 + r : B - 1;
-            if (row_of) col = row_of[col];
-            arow[it] = aq + col * K;
+            const int r = (tid >> 3) + 32 * it, row = r < last ? r : last;
+            qoff[it] = ID ? (u32)row_of[col0 + row] * (u32)nblk : (u32)row * (u32)(nblk * QK);
         }
 #pragma unroll
         for (int it = 0; it < NS; it++) {
-            const int i = (tid + it * 256) >> 2, r = i < BN ? i : BN - 1;
-            int64_t col = col0 + r < B ? col0 + r : B - 1;
-            if (row_of) col = row_of[col];
-            srow[it] = ads + col * (K >> 5);
+            const int r = (tid >> 2) + 64 * it, row = r < last ? r : last;
+            soff[it] = (ID ? (u32)row_of[col0 + row] : (u32)row) * (u32)nblk;
         }
     }
     __device__ __forceinline__ void fetch(int k0, int nblk, int tid) {
+        const int k = k0 + (tid & 7) * 16, k_last = nblk * QK - 16;   // past the end: any bytes, the weight scales there are 0
+        const u32 kk = (u32)(k < k_last ? k : k_last);
 #pragma unroll
-        for (int it = 0; it < NQ; it++) {
-            const int k = k0 + (tid & 7) * 16, last = nblk * 32 - 16;
-            q[it] = load16(arow[it] + (k < last ? k : last));   // past the end: any bytes, the weight scales there are 0
-        }
+        for (int it = 0; it < NQ; it++) q[it] = ID ? global_load<u32x4>(qbase + (uint64_t)qoff[it] * QK, kk) : global_load<u32x4>(qbase, qoff[it] + kk);
+        const int blk = (k0 >> 5) + (tid & 3);
+        const u32 bb = (u32)(blk < nblk ? blk : nblk - 1);
 #pragma unroll
         for (int it = 0; it < NS; it++) {
-            const int blk = (k0 >> 5) + (tid & 3);
-            const act_ds e = srow[it][blk < nblk ? blk : nblk - 1];
-            d[it] = e.d;
-            if constexpr (WITH_SUM) sum[it] = e.sum;
+            const uint64_t at = ID ? sbase + (uint64_t)(soff[it] + bb) * sizeof(act_ds) : sbase;
+            const u32 o = ID ? 0 : (soff[it] + bb) * (u32)sizeof(act_ds);
+            static_assert(sizeof(act_ds) == 8, "{float d; int sum;}");
+            d[it] = global_load<float>(at, o);
+            if constexpr (WITH_SUM) sum[it] = global_load<int>(at, o + 4);
         }
     }
     __device__ __forceinline__ void commit(int8_t *sA, _Float16 *sAd, float *sAs, int tid) const {
 #pragma unroll
         for (int it = 0; it < NQ; it++) {
-            const int idx = tid + it * 256;
-            const int r = idx >> 3, c = idx & 7;
+            const int r = (tid >> 3) + 32 * it, c = tid & 7;
             *(u32x4 *)(sA + mmq_chunk(r, c)) = q[it];
         }
 #pragma unroll
         for (int it = 0; it < NS; it++) {
-            const int idx = tid + it * 256;
-            if (idx < BN * 4) {
-                sAd[(idx & 3) * BN + mmq_dx_slot(idx >> 2)] = (_Float16)d[it];   // exact: d is f16-rounded
-                if constexpr (WITH_SUM) sAs[(idx & 3) * BN + (idx >> 2)] = d[it] * (float)sum[it];
-            }
+            const int r = (tid >> 2) + 64 * it, b = tid & 3;   // (BN is 64 or 128: every thread has a row)
+            sAd[b * BN + mmq_dx_slot(r)] = (_Float16)d[it];   // exact: d is f16-rounded
+            if constexpr (WITH_SUM) sAs[b * BN + r] = d[it] * (float)sum[it];
         }
     }
 };
@@ -345,11 +326,22 @@ struct mmq32_route {
     int64_t expert_bytes;      // from one expert's matrix to the next
 };
 
+// The matrices of a launch (up to three of one type that share the activation: Q, K and V; gate and up): their row tiles are numbered one
+// matrix after the other, so that small ones fill the compute units together and pay one launch (and one sum of slices).
+constexpr int MMQ_MATS = 3;
+struct mmq_mat {
+    const uint8_t *W;
+    float *dst;
+    const float *residual;     // may be null; dst's shape and stride; may be dst
+    int64_t N, dst_stride;
+    int first_row_tile;        // unused entries: INT_MAX
+};
+struct mmq_mats { mmq_mat m[MMQ_MATS]; };
+
 template <int TYPE, int TN, bool ID = false>
-__global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq,
-                                             const act_ds *__restrict__ ads, float *__restrict__ dst, int64_t N,
-                                             int64_t K, int64_t B, int64_t dst_stride, row_layout L, int n_col_tiles,
-                                             int n_groups, int n_groups_padded, mmq32_route route) {
+__global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, int64_t K, int64_t B,
+                                             row_layout L, int n_col_tiles, int n_groups, int n_groups_padded, int64_t slice_stride,
+                                             mmq32_route route) {
     typedef mmq_cfg<TYPE> C;
     constexpr int BN = 64 * TN;
     struct stage_mem {
@@ -366,11 +358,21 @@ __global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, c
     const int per_xcd = n_groups_padded >> 3;
     const int lid = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
     if (lid >= n_groups) return;   // uniform for the whole group
-    const int64_t row0 = (int64_t)(lid / n_col_tiles) * MMQ_BM;
-    int64_t col0 = (int64_t)(lid % n_col_tiles) * BN;
+    // (uniform: kept in scalar registers, although the division goes through the vector ALU)
+    const int row_tile = __builtin_amdgcn_readfirstlane(lid / n_col_tiles), col_tile = lid - row_tile * n_col_tiles;
+    int mi = 0;
+#pragma unroll
+    for (int j = 1; j < MMQ_MATS; j++)
+        if (!ID && row_tile >= mats.m[j].first_row_tile) mi = j;
+    const uint8_t *W = mats.m[mi].W;
+    float *dst = mats.m[mi].dst;
+    const float *residual = mats.m[mi].residual;
+    const int64_t N = mats.m[mi].N, dst_stride = mats.m[mi].dst_stride;
+    const int64_t row0 = (int64_t)(row_tile - mats.m[mi].first_row_tile) * MMQ_BM;
+    int64_t col0 = (int64_t)col_tile * BN;
     const int32_t *row_of = nullptr;
     if constexpr (ID) {
-        const int ct = lid % n_col_tiles;
+        const int ct = col_tile;
         if (ct >= *route.n_tiles) return;   // uniform for the whole group
         W += (int64_t)route.tiles[4 * ct] * route.expert_bytes;
         col0 = route.tiles[4 * ct + 1];
@@ -398,12 +400,12 @@ __global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, c
     // split K: grid row y walks stages [k_lo, k_hi) and writes its sums to slice y of `dst` (a workspace then, see launch_mmq)
     const int nblk = (int)(K >> 5), stages = (nblk + MMQ_BK / QK - 1) / (MMQ_BK / QK), st_per = (stages + (int)gridDim.y - 1) / (int)gridDim.y;
     const int s_lo = (int)blockIdx.y * st_per, s_hi = s_lo + st_per < stages ? s_lo + st_per : stages;
-    if (gridDim.y > 1) dst += (int64_t)blockIdx.y * B * dst_stride;
+    if (gridDim.y > 1) dst += (int64_t)blockIdx.y * slice_stride;
 
     mmq_wregs<TYPE> wregs;
-    mmq_aregs<BN, C::MIN> aregs;
+    mmq_aregs<BN, C::MIN, ID> aregs;
     wregs.init(W, L, row0, N, threadIdx.x);
-    aregs.init(aq, ads, col0, B, K, threadIdx.x, row_of);
+    aregs.init(aq, ads, col0, B, nblk, threadIdx.x, row_of);
     auto fetch = [&](int st) {
         wregs.fetch(L, st * MMQ_BK, nblk, threadIdx.x);
         aregs.fetch(st * MMQ_BK, nblk, threadIdx.x);
@@ -420,7 +422,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, c
         f16x8 dx[TN][2];     // activation block scales of this lane's 16 rows per tile
         float dw[2][NS];
     };
-    const int a_at = mmq_chunk(wcol0 + l32, lhi), w_at = mmq_chunk(wrow0 + l32, lhi);
+    int a_at = mmq_chunk(wcol0 + l32, lhi), w_at = mmq_chunk(wrow0 + l32, lhi);
     auto load_ops = [&](const stage_mem &m, int ks) {
         block_ops f;
 #pragma unroll
@@ -471,6 +473,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, c
     int buf = 0;
     for (int st = s_lo; st < s_hi; st++, buf ^= 1) {
         const stage_mem &m = sm[buf];
+        asm volatile("" : "+v"(a_at), "+v"(w_at));   // the four chunk addresses of a stage are formed in the loop: kept across it they cost spills
         // One matrix instruction is always in flight: its successor is issued before its sums are scaled, so that neither waits for the
         // other (left to the compiler, all of them write the same registers one after the other); the next block's operands are read
         // from LDS while the last sums of this one are scaled.
@@ -510,10 +513,11 @@ __global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, c
                     for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
             }
         }
-        // the next stage, requested one stage ago, goes to the other buffer; past the end the last stage is requested again and never used
-        commit(sm[buf ^ 1], st + 1);
-        fetch(st + 2 < s_hi ? st + 2 : st);
-        __syncthreads();
+        if (st + 1 < s_hi) {   // the next stage, requested one stage ago, goes to the other buffer (uniform)
+            commit(sm[buf ^ 1], st + 1);
+            fetch(st + 2 < s_hi ? st + 2 : st + 1);   // past the end the last stage is requested again and never used
+            __syncthreads();
+        }
     }
 
     // store: lane holds weight row j = l32 of each 32-wide tile, 16 activation rows
@@ -525,7 +529,10 @@ __global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, c
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int64_t b = col0 + wcol0 + tb * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-                if (n < N && b < B) dst[(ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n] = acc[tb][tw][r];
+                if (n < N && b < B) {
+                    const int64_t o = (ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n;
+                    dst[o] = residual ? acc[tb][tw][r] + residual[o] : acc[tb][tw][r];
+                }
             }
         }
 }
@@ -539,9 +546,9 @@ __global__ void __launch_bounds__(256, 2) k_mmq(const uint8_t *__restrict__ W, c
 // A product with few tiles leaves most of the chip idle while each group walks all of K: such launches are cut along K into
 // slices that run side by side and a second launch adds the slices in fixed order.  At least four stages per slice, at most
 // eight slices, at most two groups per compute unit.
-static int mmq_slices(int64_t N, int64_t K, int64_t B) {
+static int mmq_slices(int64_t row_tiles, int64_t K, int64_t B) {
     const int64_t bn = B <= 64 ? 64 : 128;
-    const int64_t groups = ((N + MMQ_BM - 1) / MMQ_BM) * ((B + bn - 1) / bn), stages = (K + MMQ_BK - 1) / MMQ_BK;
+    const int64_t groups = row_tiles * ((B + bn - 1) / bn), stages = (K + MMQ_BK - 1) / MMQ_BK;
     int64_t n = 512 / groups;
     if (n > stages / 4) n = stages / 4;
     if (n > 8) n = 8;
@@ -549,44 +556,70 @@ static int mmq_slices(int64_t N, int64_t K, int64_t B) {
     const int64_t per = (stages + n - 1) / n;
     return (int)((stages + per - 1) / per);   // no empty slice
 }
+static int64_t mmq_row_tiles(int n_mats, const int64_t *Ns) {
+    int64_t t = 0;
+    for (int i = 0; i < n_mats; i++) t += (Ns[i] + MMQ_BM - 1) / MMQ_BM;
+    return t;
+}
+static size_t mmq_ws_bytes(int n_mats, const int64_t *Ns, int64_t K, int64_t B) {
+    const int n = mmq_slices(mmq_row_tiles(n_mats, Ns), K, B);
+    int64_t rows = 0;
+    for (int i = 0; i < n_mats; i++) rows += Ns[i];
+    return n > 1 ? (size_t)n * (size_t)rows * (size_t)B * sizeof(float) : 0;
+}
 
-__global__ void __launch_bounds__(256) k_mmq_split_sum(const float *__restrict__ part, float *__restrict__ dst, int64_t N, int64_t B, int64_t dst_stride,
-                                                       int n_slices) {
+// dst[b][n] of every matrix = sum of its slices in ascending order (+ residual).  part: [slice][B][rows of all matrices]
+__global__ void __launch_bounds__(256) k_mmq_split_sum(const float *__restrict__ part, mmq_mats mats, int64_t rows, int64_t B, int n_slices) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= N * B) return;
+    if (i >= rows * B) return;
     float acc = part[i];
-    for (int sl = 1; sl < n_slices; sl++) acc = add_rn(acc, part[(int64_t)sl * N * B + i]);
-    dst[(i / N) * dst_stride + i % N] = acc;
+    for (int sl = 1; sl < n_slices; sl++) acc = add_rn(acc, part[(int64_t)sl * rows * B + i]);
+    const int64_t b = i / rows;
+    int64_t n = i % rows;
+    int j = 0;
+    while (j < MMQ_MATS - 1 && n >= mats.m[j].N) n -= mats.m[j++].N;
+    const mmq_mat &m = mats.m[j];
+    const int64_t o = b * m.dst_stride + n;
+    m.dst[o] = m.residual ? add_rn(acc, m.residual[o]) : acc;
 }
 
 template <int TYPE, int TN>
-static void launch_mmq(hipStream_t s, const void *W, const void *act, float *dst, int64_t N, int64_t K, int64_t B,
-                       int64_t dst_stride, void *ws, size_t ws_bytes) {
+static void launch_mmq(hipStream_t s, int n_mats, const mi355_gemv_mat *mats, const void *act, int64_t K, int64_t B, void *ws, size_t ws_bytes) {
     constexpr int BN = 64 * TN;
     const row_layout L = make_row_layout(TYPE, K);
     const int8_t *aq = (const int8_t *)act;
     const act_ds *ads = (const act_ds *)(aq + B * K);
-    const int n_row_tiles = (int)((N + MMQ_BM - 1) / MMQ_BM);
-    const int n_col_tiles = (int)((B + BN - 1) / BN);
-    const int n_groups = n_row_tiles * n_col_tiles;
-    const int n_groups_padded = (n_groups + 7) & ~7;
-    int n_slices = mmq_slices(N, K, B);
-    if (n_slices > 1 && (ws == nullptr || ((uintptr_t)ws & 15) != 0 || ws_bytes < (size_t)n_slices * (size_t)N * (size_t)B * sizeof(float))) n_slices = 1;
-    if (n_slices > 1) {
-        MI355_LAUNCH((k_mmq<TYPE, TN>), dim3((unsigned)n_groups_padded, (unsigned)n_slices), dim3(256), 0, s, (const uint8_t *)W, aq, ads,
-                           (float *)ws, N, K, B, N, L, n_col_tiles, n_groups, n_groups_padded, mmq32_route{});
-        MI355_LAUNCH(k_mmq_split_sum, dim3((unsigned)((N * B + 255) / 256)), dim3(256), 0, s, (const float *)ws, dst, N, B, dst_stride, n_slices);
-        return;
+    mmq_mats a, part;
+    int64_t Ns[MMQ_MATS], rows = 0;
+    int row_tiles = 0;
+    for (int i = 0; i < MMQ_MATS; i++) {
+        if (i >= n_mats) {
+            a.m[i] = mmq_mat{nullptr, nullptr, nullptr, 0, 0, 0x7fffffff};
+            part.m[i] = a.m[i];
+            continue;
+        }
+        const mi355_gemv_mat &m = mats[i];
+        a.m[i] = mmq_mat{(const uint8_t *)m.W, m.dst, m.residual, m.N, m.dst_stride, row_tiles};
+        part.m[i] = mmq_mat{(const uint8_t *)m.W, (float *)ws + rows, nullptr, m.N, 0, row_tiles};
+        Ns[i] = m.N;
+        rows += m.N;
+        row_tiles += (int)((m.N + MMQ_BM - 1) / MMQ_BM);
     }
-    MI355_LAUNCH((k_mmq<TYPE, TN>), dim3((unsigned)n_groups_padded), dim3(256), 0, s, (const uint8_t *)W, aq, ads,
-                       dst, N, K, B, dst_stride, L, n_col_tiles, n_groups, n_groups_padded, mmq32_route{});
+    for (int i = 0; i < n_mats; i++) part.m[i].dst_stride = rows;
+    const int n_col_tiles = (int)((B + BN - 1) / BN);
+    const int n_groups = row_tiles * n_col_tiles;
+    const int n_groups_padded = (n_groups + 7) & ~7;
+    int n_slices = mmq_slices(row_tiles, K, B);
+    if (n_slices > 1 && (ws == nullptr || ((uintptr_t)ws & 15) != 0 || ws_bytes < mmq_ws_bytes(n_mats, Ns, K, B))) n_slices = 1;
+    const dim3 grid((unsigned)n_groups_padded, (unsigned)n_slices);
+    MI355_LAUNCH((k_mmq<TYPE, TN>), grid, dim3(256), 0, s, n_slices > 1 ? part : a, aq, ads, K, B, L, n_col_tiles, n_groups, n_groups_padded, rows * B, mmq32_route{});
+    if (n_slices > 1) MI355_LAUNCH(k_mmq_split_sum, dim3((unsigned)((rows * B + 255) / 256)), dim3(256), 0, s, (const float *)ws, a, rows, B, n_slices);
 }
 
 template <int TYPE>
-static void launch_mmq_tn(hipStream_t s, const void *W, const void *act, float *dst, int64_t N, int64_t K, int64_t B,
-                          int64_t dst_stride, void *ws, size_t ws_bytes) {
-    if (B <= 64) launch_mmq<TYPE, 1>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes);
-    else launch_mmq<TYPE, 2>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes);
+static void launch_mmq_tn(hipStream_t s, int n_mats, const mi355_gemv_mat *mats, const void *act, int64_t K, int64_t B, void *ws, size_t ws_bytes) {
+    if (B <= 64) launch_mmq<TYPE, 1>(s, n_mats, mats, act, K, B, ws, ws_bytes);
+    else launch_mmq<TYPE, 2>(s, n_mats, mats, act, K, B, ws, ws_bytes);
 }
 
 // the routed launch: 128-column tiles over the slot list sorted by expert; the routing workspace is laid out as for the
@@ -606,8 +639,9 @@ static void launch_mmq_id(hipStream_t s, const void *as, const void *act, int64_
     const int n_groups = n_row_tiles * max_tiles;
     const int n_groups_padded = (n_groups + 7) & ~7;
     const mmq32_route route = {act_row, dst_row, tiles, n_tiles, N * L.row_bytes};
-    MI355_LAUNCH((k_mmq<TYPE, 2, true>), dim3((unsigned)n_groups_padded), dim3(256), 0, s, (const uint8_t *)as, aq, ads, dst, N, K, S, N, L, max_tiles,
-                 n_groups, n_groups_padded, route);
+    mmq_mats a;
+    for (int i = 0; i < MMQ_MATS; i++) a.m[i] = i ? mmq_mat{nullptr, nullptr, nullptr, 0, 0, 0x7fffffff} : mmq_mat{(const uint8_t *)as, dst, nullptr, N, N, 0};
+    MI355_LAUNCH((k_mmq<TYPE, 2, true>), dim3((unsigned)n_groups_padded), dim3(256), 0, s, a, aq, ads, K, S, L, max_tiles, n_groups, n_groups_padded, (int64_t)0, route);
 }
 
 }  // namespace mi355
@@ -617,7 +651,7 @@ using namespace mi355;
 extern "C" int mi355_mul_mat_id_q_supported(int type, const void *as, int64_t N, int64_t K, int64_t n_expert) {
     const bool typed = type == MI355_Q4_0 || type == MI355_Q4_1 || type == MI355_Q5_0 || type == MI355_Q5_1 || type == MI355_IQ4_NL ||
                        type == MI355_Q8_0 || type == MI355_Q6_K || type == MI355_IQ4_XS;
-    if (!typed || N <= 0 || K <= 0 || K % type_block_elems(type) != 0 || n_expert <= 0 || n_expert > 256) return 0;
+    if (!typed || N <= 0 || K <= 0 || K >= (int64_t(1) << 24) || K % type_block_elems(type) != 0 || n_expert <= 0 || n_expert > 256) return 0;
     return layout_loadable(as) ? 1 : 0;
 }
 
@@ -626,7 +660,7 @@ extern "C" int mi355_mul_mat_id_q(void *stream, int type, const void *as, const 
     MI355_REQUIRE(mi355_mul_mat_id_q_supported(type, as, N, K, n_expert), "mul_mat_id_q: type %d, K=%lld, %lld experts or the weight alignment is not supported",
                   type, (long long)K, (long long)n_expert);
     MI355_REQUIRE(n_used > 0 && nb1 > 0 && T > 0 && ids_stride >= n_used, "mul_mat_id_q: bad shape");
-    MI355_REQUIRE(T * n_used < (1 << 24) && nb1 * T < (1 << 24), "mul_mat_id_q: too many slots");
+    MI355_REQUIRE(T * n_used < (1 << 24) && nb1 * T < (1 << 24) && nb1 * T * (K / QK) < (int64_t(1) << 32), "mul_mat_id_q: too many slots");
     MI355_REQUIRE(((uintptr_t)act & 15) == 0, "mul_mat_id_q: activation workspace is not 16-byte aligned");
     const size_t need = mi355_mul_mat_id_q8k_route_bytes(n_expert, n_used, T);
     if (route_ws == nullptr || route_ws_bytes < need || ((uintptr_t)route_ws & 15) != 0) {
@@ -648,11 +682,13 @@ extern "C" int mi355_mul_mat_id_q(void *stream, int type, const void *as, const 
     return launch_status("k_mmq (routed)");
 }
 
-extern "C" size_t mi355_mul_mat_q_ws_bytes(int64_t N, int64_t K, int64_t B) {
-    if (N <= 0 || K <= 0 || B <= 0 || K % QK != 0) return 0;
-    const int n = mmq_slices(N, K, B);
-    return n > 1 ? (size_t)n * (size_t)N * (size_t)B * sizeof(float) : 0;
+extern "C" size_t mi355_mul_mat_q_multi_ws_bytes(int n_mats, const int64_t *Ns, int64_t K, int64_t B) {
+    if (n_mats < 1 || n_mats > MMQ_MATS || K <= 0 || B <= 0 || K % QK != 0) return 0;
+    for (int i = 0; i < n_mats; i++)
+        if (Ns[i] <= 0) return 0;
+    return mmq_ws_bytes(n_mats, Ns, K, B);
 }
+extern "C" size_t mi355_mul_mat_q_ws_bytes(int64_t N, int64_t K, int64_t B) { return mi355_mul_mat_q_multi_ws_bytes(1, &N, K, B); }
 
 extern "C" int mi355_mul_mat_q(void *stream, int type, const void *W, const void *act, float *dst, int64_t N, int64_t K,
                                int64_t B, int64_t dst_stride) {
@@ -661,26 +697,37 @@ extern "C" int mi355_mul_mat_q(void *stream, int type, const void *W, const void
 
 extern "C" int mi355_mul_mat_q_ws(void *stream, int type, const void *W, const void *act, float *dst, int64_t N, int64_t K,
                                   int64_t B, int64_t dst_stride, void *ws, size_t ws_bytes) {
+    const mi355_gemv_mat m = {type, W, N, dst, dst_stride, nullptr};
+    return mi355_mul_mat_q_multi(stream, type, 1, &m, act, K, B, ws, ws_bytes);
+}
+
+extern "C" int mi355_mul_mat_q_multi(void *stream, int type, int n_mats, const mi355_gemv_mat *mats, const void *act, int64_t K, int64_t B, void *ws,
+                                     size_t ws_bytes) {
     MI355_REQUIRE(is_weight_type(type), "mul_mat_q: unsupported weight type %d", type);
-    MI355_REQUIRE(N > 0 && K > 0 && B > 0, "mul_mat_q: bad shape N=%lld K=%lld B=%lld", (long long)N, (long long)K, (long long)B);
+    MI355_REQUIRE(n_mats >= 1 && n_mats <= MMQ_MATS, "mul_mat_q: 1..%d matrices per launch, got %d", MMQ_MATS, n_mats);
+    MI355_REQUIRE(K > 0 && B > 0 && K < (int64_t(1) << 24), "mul_mat_q: bad shape K=%lld B=%lld", (long long)K, (long long)B);
     MI355_REQUIRE(K % type_block_elems(type) == 0, "mul_mat_q: K=%lld is not a multiple of the block size", (long long)K);
-    MI355_REQUIRE(dst_stride >= N, "mul_mat_q: dst_stride < N");
-    if (!layout_loadable(W))   // a matrix at an odd address
-        return gemv_unaligned((hipStream_t)stream, type, W, act, dst, nullptr, N, K, B, dst_stride);
-    MI355_REQUIRE(((uintptr_t)act & 15) == 0, "mul_mat_q: activation workspace is not 16-byte aligned");
-    MI355_REQUIRE((N + MMQ_BM - 1) / MMQ_BM * ((B + 63) / 64) < (1 << 30), "mul_mat_q: too many tiles");
-    hipStream_t s = (hipStream_t)stream;
-    switch (type) {
-        case MI355_Q4_0: launch_mmq_tn<MI355_Q4_0>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        case MI355_Q8_0: launch_mmq_tn<MI355_Q8_0>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        case MI355_Q4_K: launch_mmq_tn<MI355_Q4_K>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        case MI355_Q5_K: launch_mmq_tn<MI355_Q5_K>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        case MI355_Q4_1: launch_mmq_tn<MI355_Q4_1>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        case MI355_Q5_0: launch_mmq_tn<MI355_Q5_0>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        case MI355_Q5_1: launch_mmq_tn<MI355_Q5_1>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        case MI355_IQ4_NL: launch_mmq_tn<MI355_IQ4_NL>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        case MI355_IQ4_XS: launch_mmq_tn<MI355_IQ4_XS>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
-        default: launch_mmq_tn<MI355_Q6_K>(s, W, act, dst, N, K, B, dst_stride, ws, ws_bytes); break;
+    int64_t row_tiles = 0;
+    bool loadable = true;
+    for (int i = 0; i < n_mats; i++) {
+        MI355_REQUIRE(mats[i].type == type, "mul_mat_q: the matrices of a launch have one type");
+        MI355_REQUIRE(mats[i].N > 0, "mul_mat_q: bad shape N=%lld", (long long)mats[i].N);
+        MI355_REQUIRE(mats[i].dst_stride >= mats[i].N, "mul_mat_q: dst_stride < N");
+        row_tiles += (mats[i].N + MMQ_BM - 1) / MMQ_BM;
+        loadable = loadable && layout_loadable(mats[i].W);
     }
+    if (!loadable) {   // a matrix at an odd address
+        for (int i = 0; i < n_mats; i++) {
+            const int rc = gemv_unaligned((hipStream_t)stream, type, mats[i].W, act, mats[i].dst, mats[i].residual, mats[i].N, K, B, mats[i].dst_stride);
+            if (rc != MI355_OK) return rc;
+        }
+        return MI355_OK;
+    }
+    MI355_REQUIRE(((uintptr_t)act & 15) == 0, "mul_mat_q: activation workspace is not 16-byte aligned");
+    MI355_REQUIRE(row_tiles * ((B + 63) / 64) < (1 << 30), "mul_mat_q: too many tiles");
+    hipStream_t s = (hipStream_t)stream;
+#define MI355_MMQ_LAUNCH(TY) launch_mmq_tn<TY>(s, n_mats, mats, act, K, B, ws, ws_bytes);
+    MI355_WEIGHT_TYPE_SWITCH(type, MI355_MMQ_LAUNCH)
+#undef MI355_MMQ_LAUNCH
     return launch_status("k_mmq");
 }

@@ -69,6 +69,8 @@ _SIGNATURES = {
     "mi355_mul_mat_q": (_int, [_p, _int, _p, _p, _p, _i64, _i64, _i64, _i64]),
     "mi355_mul_mat_q_ws_bytes": (_sz, [_i64, _i64, _i64]),
     "mi355_mul_mat_q_ws": (_int, [_p, _int, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _sz]),
+    "mi355_mul_mat_q_multi_ws_bytes": (_sz, [_int, _p, _i64, _i64]),
+    "mi355_mul_mat_q_multi": (_int, [_p, _int, _int, _p, _p, _i64, _i64, _p, _sz]),
     "mi355_mul_mat_skinny_supported": (_int, [_int, _p, _i64, _i64]),
     "mi355_mul_mat_skinny_ws_bytes": (_sz, [_i64, _i64, _i64]),
     "mi355_mul_mat_skinny": (_int, [_p, _int, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _sz]),

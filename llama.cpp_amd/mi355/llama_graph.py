@@ -275,6 +275,14 @@ class LlamaRunner:
                     self.split_ws = torch.empty(need + 256, dtype=torch.uint8, device=self.dev)
                 check(self.lib.mi355_mul_mat_mid_multi(_stream(), Q4_K, len(mats), arr, _ptr(act), K, T, _ptr(self.split_ws) if need else None, need))
                 mats = []
+            if not q8k:   # Q8_1 blocks: the weight-streaming kernel up to 32 rows, then the per-block tile kernel, neighbours of one type in one launch
+                while mats:
+                    n = 1
+                    if T > 32:
+                        while n < min(3, len(mats)) and mats[n][0][0] == mats[0][0][0]:
+                            n += 1
+                    self._mm_q8_1(mats[:n], act, K, T, residual)
+                    mats = mats[n:]
             for (t, W), out in mats:
                 if q8k == 3:
                     N = out.shape[1]
@@ -308,10 +316,25 @@ class LlamaRunner:
                     else:
                         check(self.lib.mi355_mul_mat_q8k_ws(_stream(), t, _ptr(W), _ptr(act), _ptr(out), res, N, K, T, out.stride(0), sw, sn))
                     continue
-                dst = out if residual is None else self.t1[:T]
-                check(self.lib.mi355_mul_mat_q(_stream(), t, _ptr(W), _ptr(act), _ptr(dst), out.shape[1], K, T, dst.stride(0)))
-                if residual is not None:
-                    self._bin(0, dst, residual, out)
+
+    def _mm_q8_1(self, mats, act, K, T, residual):
+        """products of more than eight rows on Q8_1 activations: one matrix (up to 32 rows), or up to three of one type in one launch"""
+        t = mats[0][0][0]
+        arr = (GemvMat * len(mats))()
+        for i, ((_, W), out) in enumerate(mats):
+            arr[i].type, arr[i].W, arr[i].N, arr[i].dst, arr[i].dst_stride = t, W.data_ptr(), out.shape[1], out.data_ptr(), out.stride(0)
+            arr[i].residual = residual.data_ptr() if residual is not None else None
+        if T <= 32:
+            need = int(self.lib.mi355_mul_mat_skinny_ws_bytes(arr[0].N, K, T))
+        else:
+            need = int(self.lib.mi355_mul_mat_q_multi_ws_bytes(len(mats), (C.c_int64 * len(mats))(*[out.shape[1] for _, out in mats]), K, T))
+        if self.split_ws is None or self.split_ws.numel() < need:
+            self.split_ws = torch.empty(need + 256, dtype=torch.uint8, device=self.dev)
+        ws = _ptr(self.split_ws) if need else None
+        if T <= 32:
+            check(self.lib.mi355_mul_mat_skinny(_stream(), t, arr[0].W, _ptr(act), arr[0].dst, arr[0].residual, arr[0].N, K, T, arr[0].dst_stride, ws, need))
+        else:
+            check(self.lib.mi355_mul_mat_q_multi(_stream(), t, len(mats), arr, _ptr(act), K, T, ws, need))
 
     def forward(self, T, n_kv, last_only=True):
         """fused launch sequence: 10 launches per layer instead of 25, same arithmetic per node"""

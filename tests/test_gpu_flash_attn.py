@@ -244,3 +244,16 @@ def test_prefill_head_sizes(dev, D, Nq, Nkv, Hq, Hkv):
     p = np.exp(s - s.max(axis=-1, keepdims=True))
     want = np.einsum("hqk,hkd->qhd", p / p.sum(axis=-1, keepdims=True), vv)
     assert orc.nmse(got, want) < 1e-6
+
+
+@pytest.mark.parametrize("D,Nq", [(64, 16), (128, 100)])
+def test_prefill_quantized_output(dev, D, Nq):
+    """the Q8_1 rows that accompany a prompt batch's output are the quantization of that output, byte for byte"""
+    import torch
+    import mi355
+    rng = np.random.default_rng(D)
+    q, k, v, mask = _inputs(rng, D, Nq, 256, 8, 2)
+    args = [torch.from_numpy(a).to(dev) for a in (q, k, v, mask)]
+    dst, act = mi355.flash_attn_ext(*args, 1.0 / np.sqrt(D), quantized=True)
+    assert torch.equal(dst, mi355.flash_attn_ext(*args, 1.0 / np.sqrt(D)))
+    assert torch.equal(act, mi355.quantize_act(dst.reshape(Nq, 8 * D)))

@@ -577,3 +577,35 @@ def test_mmq_tiled_multi(dev, name, t, Ns, K, B):
         Nt, Bt = min(N, 40), min(B, 16)
         assert orc.nmse(multi[i][:Bt, :Nt], orc.mul_mat("cpu", t, Wq[i][:Nt], x[:Bt])) < 1e-9
         assert orc.nmse(multi[i][B - 5:, N - 7:], orc.mul_mat("cpu", t, Wq[i][N - 7:], x[B - 5:])) < 1e-9
+
+
+@pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t in (orc.Q4_0, orc.Q5_1, orc.Q8_0, orc.Q6_K)])
+@pytest.mark.parametrize("K,B", [(512, 33), (2048, 65), (1024, 300)])
+def test_mul_mat_q_multi(dev, name, t, K, B):
+    """up to three matrices in one launch of the per-block tile kernel, ragged row counts, a residual that is the destination, with and
+    without slices along K: the product of each matrix alone plus the residual (f32 sums in another order: NMSE of some 1e-14)"""
+    import ctypes as C
+    import torch
+    import mi355
+    lib = mi355.load()
+    rng = np.random.default_rng(K + B)
+    Ns = [300, 64, 129]
+    Ws = [mi355.upload_weights(t, _to_dev(dev, _weights(rng, t, N, K))) for N in Ns]
+    act = mi355.quantize_act(_to_dev(dev, rng.standard_normal((B, K)).astype(np.float32)))
+    res = [_to_dev(dev, rng.standard_normal((B, N)).astype(np.float32)) for N in Ns]
+    want = []
+    for W, r, N in zip(Ws, res, Ns):
+        d = torch.empty((B, N), dtype=torch.float32, device=dev)
+        mi355.check(lib.mi355_mul_mat_q(None, t, W.data_ptr(), act.data_ptr(), d.data_ptr(), N, K, B, N))
+        want.append((d.double() + r.double()).cpu().numpy())
+    need = lib.mi355_mul_mat_q_multi_ws_bytes(3, (C.c_int64 * 3)(*Ns), K, B)
+    for nws in {0, int(need)}:
+        ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dev)
+        dst = [r.clone() for r in res]
+        arr = (mi355.GemvMat * 3)()
+        for i in range(3):
+            arr[i].type, arr[i].W, arr[i].N, arr[i].dst, arr[i].dst_stride, arr[i].residual = t, Ws[i].data_ptr(), Ns[i], dst[i].data_ptr(), Ns[i], dst[i].data_ptr()
+        mi355.check(lib.mi355_mul_mat_q_multi(None, t, 3, arr, act.data_ptr(), K, B, ws.data_ptr() if nws else None, nws))
+        torch.cuda.synchronize()
+        for d, w in zip(dst, want):
+            assert orc.nmse(d.cpu().numpy(), w) < 1e-11, nws
