@@ -336,6 +336,14 @@ int mi355_mul_mat_id_q8k(void *stream, int type, const void *as, const void *act
                          int64_t N, int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T, void *route_ws,
                          size_t route_ws_bytes);
 
+/* MUL_MAT_ID for a few slots per expert on the weight-streaming kernel of mi355_mul_mat_skinny: every group of the launch collects the slots
+ * of its expert from the ids itself, so an expert's matrix is read once however many of the (at most 1024) slots chose it.  Operands as
+ * mi355_mul_mat_id_vec (`act`: the nb1*T rows of b in the mi355_quantize_act layout); every weight type and K, the stack at an even address.
+ * mi355_mul_mat_id takes it between the per-slot GEMV and the routed tile kernels. */
+int mi355_mul_mat_id_skinny_supported(int type, const void *as, int64_t K, int64_t n_expert, int64_t n_used, int64_t T);
+int mi355_mul_mat_id_skinny(void *stream, int type, const void *as, const void *act, const int32_t *ids, int64_t ids_stride, float *dst, int64_t N,
+                            int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T);
+
 /* The same for experts of the per-32-block types (Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL, Q8_0) and, at the precision of Q8_1 activations, of
  * Q6_K and IQ4_XS: the routed form of mi355_mul_mat_q's tile kernel on 128-slot column tiles.  `act` holds the nb1*T rows of b in the mi355_quantize_act (Q8_1) layout; route_ws as above.
  * K a multiple of the block size, the stack at an even address, at most 256 experts (mi355_mul_mat_id_q_supported);

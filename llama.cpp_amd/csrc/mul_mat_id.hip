@@ -1,8 +1,10 @@
 // MUL_MAT_ID host entry: quantize the nb1*T rows of b once, then route every
 // (token, expert slot) pair to its expert's weights on the device: per-slot GEMV for a few slots,
-// slots sorted by expert and one tile launch over all experts for many.
+// the weight-streaming kernel for a few per expert, slots sorted by expert and one tile launch over all experts for many.
 #include "common.hpp"
 #include "qdot.hpp"
+
+#include <math.h>
 
 using namespace mi355;
 
@@ -18,6 +20,18 @@ static bool use_routed_tiles(int type, const void *as, int64_t N, int64_t K, int
         return false;
     const row_layout L = make_row_layout(type, K);
     return layout_aligned(as, L) && (N * L.row_bytes) % 16 == 0;
+}
+
+// Between the two: the weight-streaming kernel, which reads every chosen expert's matrix once.  It pays from where the slots outnumber the
+// experts they choose (on average E (1 - (1 - 1/E)^S) of E) by as much as it streams slower than the GEMV: 8 experts of 14336 x 4096,
+// 8 / 12 / 24 slots: Q4_0 46 / 67 / 125 us with a GEMV per slot, 43 / 57 / 64 streamed; Q6_K 68 / 98 / 196 against 87 / 102 / 116.
+// Up to 32 slots per expert it is ahead of the routed tile kernel (Q4_0, 32 / 64 / 256 / 512 slots: 214 / 208 / 215 / 245 us against
+// 65 / 78 / 192 / 304; 16 experts of 2048 x 2048, 512 slots: 63 against 28).
+static bool use_skinny(int type, const void *as, int64_t K, int64_t n_expert, int64_t n_used, int64_t T) {
+    const int64_t S = T * n_used;
+    if (!mi355_mul_mat_id_skinny_supported(type, as, K, n_expert, n_used, T) || S > 32 * n_expert) return false;
+    const double chosen = (double)n_expert * (1.0 - pow(1.0 - 1.0 / (double)n_expert, (double)S));
+    return (double)S >= (type == MI355_Q6_K ? 2.1 : 1.7) * chosen;
 }
 
 size_t mi355_mul_mat_id_ws_bytes(int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T) {
@@ -45,6 +59,7 @@ int mi355_mul_mat_id(void *stream, int type, const void *as, const float *b, con
     }
     int rc = mi355_quantize_act(stream, b, ws, K, nb1 * T, K);
     if (rc != MI355_OK) return rc;
+    if (use_skinny(type, as, K, n_expert, n_used, T)) return mi355_mul_mat_id_skinny(stream, type, as, ws, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T);
     if (T * n_used >= ROUTED_MIN_SLOTS && mi355_mul_mat_id_q_supported(type, as, N, K, n_expert)) {   // per-32-block types and the super-block types whose rows are no multiple of 16 bytes: the routed form of the per-block tile kernel
         const size_t act = (mi355_act_bytes(K, nb1 * T) + 255) & ~(size_t)255;
         return mi355_mul_mat_id_q(stream, type, as, ws, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, (uint8_t *)ws + act, ws_bytes - act);

@@ -76,10 +76,20 @@ template <int TYPE, int NI> struct sk_regs {
 // grid.x = 32-row tiles of the weight matrix, grid.y = slices of K (partial sums to `dst` as [slice][B][dst_stride] then).
 // The group's four waves split the slice's steps.  TAIL: K is no multiple of 256 (per-32-block types; a form of its own, since the branch
 // and its registers cost the others 7 %: Q8_0 28672 x 8192, 8 rows, 53.7 -> 57.6 us).
-template <int TYPE, int NI, bool TAIL>
+//
+// ID: MUL_MAT_ID with a few slots per expert.  grid.z = experts; a group collects its expert's (token, expert slot) pairs from the ids
+// itself (at most SK_MAX_SLOTS of them in all: two reads of a few KiB from L2, no routing launch) and takes them 8 NI columns at a time,
+// so that an expert's matrix is read from memory once however many slots chose it; the passes over further columns find their 32 rows in L2.
+constexpr int SK_MAX_SLOTS = 1024;
+struct sk_id {
+    const int32_t *ids;        // expert of slot t * n_used + e at ids[t * ids_stride + e]
+    int64_t ids_stride, expert_bytes;
+    int n_used, nb1, n_slots;
+};
+template <int TYPE, int NI, bool TAIL, bool ID = false>
 __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads,
                                                    float *__restrict__ dst, const float *__restrict__ residual, int64_t N, int K, int B,
-                                                   int64_t dst_stride, int steps_per_slice, int steps_per_wave) {
+                                                   int64_t dst_stride, int steps_per_slice, int steps_per_wave, sk_id id) {
     typedef sk_traits<TYPE> T;
     typedef sk_regs<TYPE, NI> R;
     constexpr int WPAD = T::ROW_BYTES + 16;
@@ -98,6 +108,23 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     float2 *s_t = (float2 *)(s_a + A_BYTES);
     int *s_g = (int *)(s_a + A_BYTES + T_BYTES);
     uint8_t *s_qh = s_w + 32 * WPAD;
+
+    __shared__ unsigned short s_slot[ID ? SK_MAX_SLOTS : 1];
+    int n_cols = B;
+    if constexpr (ID) {
+        __shared__ int s_n;
+        if (threadIdx.x == 0) s_n = 0;
+        __syncthreads();
+        for (int sl = threadIdx.x; sl < id.n_slots; sl += 256) {
+            int ex = id.ids[(int64_t)(sl / id.n_used) * id.ids_stride + sl % id.n_used];
+            ex = ex < 0 ? 0 : (ex >= (int)gridDim.z ? (int)gridDim.z - 1 : ex);   // never index outside the expert stack
+            if (ex == (int)blockIdx.z) s_slot[atomicAdd(&s_n, 1)] = (unsigned short)sl;   // (any order: a column's sums do not depend on its neighbours)
+        }
+        __syncthreads();
+        n_cols = __builtin_amdgcn_readfirstlane(s_n);
+        if (n_cols == 0) return;   // uniform for the whole group
+        W += (int64_t)blockIdx.z * id.expert_bytes;
+    }
 
     const row_layout L = make_row_layout(TYPE, K);
     const int nsteps = TAIL ? (K + 255) >> 8 : K >> 8;
@@ -128,20 +155,22 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     }
     const int64_t my_row = row0 + r < N ? row0 + r : N - 1;
     const uint8_t *w_mine = W + my_row * L.row_bytes;   // the row whose results this lane holds: its scales go to registers
+    int c_lo = 0;   // ID: first column of the pass
+    auto act_row = [&](int i) -> int64_t {   // activation row of column i of the pass; columns past the end repeat the last one
+        const int c = c_lo + i < n_cols ? c_lo + i : n_cols - 1;
+        if constexpr (!ID) return c;
+        const int sl = s_slot[c];
+        return (int64_t)(sl / id.n_used) * id.nb1 + sl % id.n_used % id.nb1;
+    };
+    do {
     const int a_piece = lane & 15, a_row = lane >> 4;
     const int8_t *a_src[R::NA];
 #pragma unroll
-    for (int u = 0; u < R::NA; u++) {
-        const int c = a_row + 4 * u < B ? a_row + 4 * u : B - 1;   // activation rows past the end repeat the last one
-        a_src[u] = aq + (int64_t)c * K + 16 * a_piece;
-    }
+    for (int u = 0; u < R::NA; u++) a_src[u] = aq + act_row(a_row + 4 * u) * K + 16 * a_piece;
     const int t_piece = lane & 3, t_row = lane >> 2;   // {d, sum} pairs: 4 lanes x 16 bytes per activation row and step
     const act_ds *t_src[R::NT];
 #pragma unroll
-    for (int u = 0; u < R::NT; u++) {
-        const int c = t_row + 16 * u < B ? t_row + 16 * u : B - 1;
-        t_src[u] = ads + (int64_t)c * nblk + 2 * t_piece;
-    }
+    for (int u = 0; u < R::NT; u++) t_src[u] = ads + act_row(t_row + 16 * u) * nblk + 2 * t_piece;
 
     // The last step of a row whose K is no multiple of 256: blocks past the end repeat the last one (nothing is read behind the row) and
     // get scale and minimum 0; the activation bytes they meet are those of the last block too, hence finite.
@@ -415,12 +444,15 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
         const float sum = ((s_red[(0 * NI * 4 + v) * 64 + lane] + s_red[(1 * NI * 4 + v) * 64 + lane]) + s_red[(2 * NI * 4 + v) * 64 + lane]) +
                           s_red[(3 * NI * 4 + v) * 64 + lane];
         const int q = v >> 2, i = v & 3;
-        const int c = 8 * q + 4 * kh + i;
-        if (c < B && row0 + r < N) {
-            const int64_t o = ((int64_t)blockIdx.y * B + c) * dst_stride + row0 + r;
+        const int c = c_lo + 8 * q + 4 * kh + i;
+        if (c < n_cols && row0 + r < N) {
+            const int64_t o = (ID ? (int64_t)s_slot[c] : (int64_t)blockIdx.y * B + c) * dst_stride + row0 + r;
             dst[o] = residual ? sum + residual[o] : sum;
         }
     }
+    if constexpr (ID) __syncthreads();   // the partial sums have been read: the next pass reuses the memory
+    c_lo += 8 * NI;
+    } while (ID && c_lo < n_cols);
 }
 
 // sum of the K slices: dst[c][n] = sum_s part[s][c][n] (+ residual), slices in ascending order
@@ -447,9 +479,9 @@ void launch_skinny(hipStream_t s, const void *W, const int8_t *aq, const act_ds 
     const int64_t stride = slices == 1 ? dst_stride : N;
     constexpr bool BLOCKS32 = (sk_traits<TYPE>::NIB32 && TYPE != MI355_IQ4_XS) || TYPE == MI355_Q8_0;
     if (BLOCKS32 && K % 256 != 0)
-        MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave);
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave, sk_id{});
     else
-        MI355_LAUNCH((k_mm_skinny<TYPE, NI, false>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave);
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, false>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave, sk_id{});
     if (slices > 1) {
         MI355_LAUNCH(k_skinny_slices, dim3((unsigned)((N + 255) / 256), (unsigned)B), dim3(256), 0, s, part, dst, residual, N, B, dst_stride, slices);
     }
@@ -464,6 +496,17 @@ void launch_skinny_nt(hipStream_t s, const void *W, const int8_t *aq, const act_
     else launch_skinny<TYPE, 4>(s, W, aq, ads, dst, residual, N, K, B, dst_stride, slices, part);
 }
 
+template <int TYPE, int NI>
+void launch_skinny_id(hipStream_t s, const void *as, const int8_t *aq, const act_ds *ads, float *dst, int64_t N, int K, int64_t n_expert, const sk_id &id) {
+    const int nsteps = (K + 255) >> 8;
+    const dim3 grid((unsigned)((N + 31) / 32), 1, (unsigned)n_expert);
+    constexpr bool BLOCKS32 = (sk_traits<TYPE>::NIB32 && TYPE != MI355_IQ4_XS) || TYPE == MI355_Q8_0;
+    if (BLOCKS32 && K % 256 != 0)
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32, true>), grid, dim3(256), 0, s, (const uint8_t *)as, aq, ads, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id);
+    else
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, false, true>), grid, dim3(256), 0, s, (const uint8_t *)as, aq, ads, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id);
+}
+
 // slices of K: launches with fewer than ~1.5 groups per compute unit split K over several groups (and pay a second launch
 // that adds the slices), as long as a slice keeps 4 steps; a short K with at most 8 activation rows is quicker in one go.
 int skinny_slices(int64_t N, int64_t K, int64_t B) {
@@ -473,6 +516,10 @@ int skinny_slices(int64_t N, int64_t K, int64_t B) {
     while (s < 8 && tiles * s < 512 && nsteps / (s * 2) >= 4) s *= 2;
     return s;
 }
+
+// Columns per pass of the expert form (8, 16 or 32) by the average number of slots per expert: a few more than the average, since a second
+// pass costs as much matrix work as the first, and no more than that, since every column is copied and scaled whether a slot fills it or not
+constexpr int64_t SK_ID_NARROW = 5, SK_ID_WIDE = 12;
 
 }  // namespace
 
@@ -506,6 +553,31 @@ int mi355_mul_mat_skinny(void *stream, int type, const void *W, const void *act,
     MI355_WEIGHT_TYPE_SWITCH(type, X)
 #undef X
     return launch_status("k_mm_skinny");
+}
+
+int mi355_mul_mat_id_skinny_supported(int type, const void *as, int64_t K, int64_t n_expert, int64_t n_used, int64_t T) {
+    return is_weight_type(type) && K > 0 && K % type_block_elems(type) == 0 && K < (int64_t(1) << 30) && n_expert > 0 && n_expert <= 65535 && n_used > 0 && T > 0 &&
+           T * n_used <= SK_MAX_SLOTS && layout_loadable(as);
+}
+
+int mi355_mul_mat_id_skinny(void *stream, int type, const void *as, const void *act, const int32_t *ids, int64_t ids_stride, float *dst, int64_t N, int64_t K,
+                            int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T) {
+    MI355_REQUIRE(mi355_mul_mat_id_skinny_supported(type, as, K, n_expert, n_used, T), "mul_mat_id_skinny: type %d, K=%lld, %lld slots or the weight alignment is not supported",
+                  type, (long long)K, (long long)(T * n_used));
+    MI355_REQUIRE(N > 0 && nb1 > 0 && ids_stride >= n_used, "mul_mat_id_skinny: bad shape");
+    MI355_REQUIRE(((uintptr_t)act & 15) == 0, "mul_mat_id_skinny: activation workspace is not 16-byte aligned");
+    hipStream_t s = (hipStream_t)stream;
+    const int8_t *aq = (const int8_t *)act;
+    const act_ds *ads = (const act_ds *)(aq + nb1 * T * K);
+    const sk_id id = {ids, ids_stride, N * make_row_layout(type, K).row_bytes, (int)n_used, (int)nb1, (int)(T * n_used)};
+    const int64_t avg = T * n_used / n_expert;   // slots per expert
+#define X(TY)                                                                                 \
+    if (avg <= SK_ID_NARROW) launch_skinny_id<TY, 1>(s, as, aq, ads, dst, N, (int)K, n_expert, id); \
+    else if (avg <= SK_ID_WIDE) launch_skinny_id<TY, 2>(s, as, aq, ads, dst, N, (int)K, n_expert, id); \
+    else launch_skinny_id<TY, 4>(s, as, aq, ads, dst, N, (int)K, n_expert, id);
+    MI355_WEIGHT_TYPE_SWITCH(type, X)
+#undef X
+    return launch_status("k_mm_skinny (experts)");
 }
 
 }  // extern "C"

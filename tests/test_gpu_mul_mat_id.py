@@ -138,7 +138,7 @@ def test_mul_mat_id_on_tile_images_skewed_routing(dev, pattern):
 
 
 @pytest.mark.parametrize("name,t,blocks", [("q6_k", orc.Q6_K, 3), ("iq4_xs", orc.IQ4_XS, 5), ("q4_0", orc.Q4_0, 3), ("q8_0", orc.Q8_0, 9), ("q5_1", orc.Q5_1, 7)])
-@pytest.mark.parametrize("T", [3, 16, 130])
+@pytest.mark.parametrize("T", [3, 16, 60, 130])
 def test_mul_mat_id_ragged_rows(dev, name, t, blocks, T):
     """expert rows that start at any even address, K no whole number of the tile kernel's stages: per-slot GEMV and routed tiles"""
     import torch
@@ -151,3 +151,32 @@ def test_mul_mat_id_ragged_rows(dev, name, t, blocks, T):
     Wd = mi355.upload_weights(t, torch.from_numpy(Wq).to(dev)).reshape(n_expert, N, -1)
     got = mi355.mul_mat_id(t, Wd, torch.from_numpy(b).to(dev), torch.from_numpy(ids).to(dev)[:, :n_used], n_used).cpu().numpy()
     assert orc.nmse(got, expected_per_expert("q8_1", t, Wq, b, ids, n_expert, n_used, 1, N)) < 1e-11
+
+
+@pytest.mark.parametrize("name,t", list(orc.WEIGHT_TYPES.items()))
+@pytest.mark.parametrize("n_expert,n_used,bcast,T,pattern", [(8, 2, True, 7, "spread"), (4, 3, False, 33, "spread"), (6, 2, True, 150, "spread"), (8, 2, True, 90, "one_expert"),
+                                                             (3, 2, True, 20, "out_of_range")])
+def test_mul_mat_id_skinny(dev, name, t, n_expert, n_used, bcast, T, pattern):
+    """the weight-streaming kernel over experts: none, one and several passes over an expert's columns, a ragged last row tile, ids outside
+    [0, n_expert) clamped; against exact integer block dots (f32 sums: NMSE of some 1e-14)"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    N, K = 70, 1024
+    nb1 = 1 if bcast else n_used
+    rng = np.random.default_rng(T)
+    Wq = orc.quantize("oracle", t, (rng.standard_normal((n_expert * N, K)) * 0.02).astype(np.float32))
+    b = rng.standard_normal((T, nb1, K)).astype(np.float32)
+    ids = np.stack([rng.permutation(max(n_expert, n_used))[:n_used] for _ in range(T)]).astype(np.int32)
+    if pattern == "one_expert":
+        ids[:] = 5
+    elif pattern == "out_of_range":
+        ids = rng.integers(-2, n_expert + 2, size=ids.shape).astype(np.int32)
+    Wd = mi355.upload_weights(t, torch.from_numpy(Wq).to(dev))
+    act = mi355.quantize_act(torch.from_numpy(b.reshape(T * nb1, K)).to(dev))
+    idd = torch.from_numpy(ids).to(dev)
+    got = torch.full((T, n_used, N), float("nan"), device=dev)
+    mi355.check(lib.mi355_mul_mat_id_skinny(None, t, Wd.data_ptr(), act.data_ptr(), idd.data_ptr(), idd.stride(0), got.data_ptr(), N, K, n_expert, n_used, nb1, T))
+    torch.cuda.synchronize()
+    want = expected_per_expert("q8_1", t, Wq, b, np.clip(ids, 0, n_expert - 1), n_expert, n_used, nb1, N)
+    assert orc.nmse(got.cpu().numpy(), want) < 1e-11
