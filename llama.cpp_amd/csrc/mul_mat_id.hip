@@ -25,11 +25,14 @@ static bool use_routed_tiles(int type, const void *as, int64_t N, int64_t K, int
 // Between the two: the weight-streaming kernel, which reads every chosen expert's matrix once.  It pays from where the slots outnumber the
 // experts they choose (on average E (1 - (1 - 1/E)^S) of E) by as much as it streams slower than the GEMV: 8 experts of 14336 x 4096,
 // 8 / 12 / 24 slots: Q4_0 46 / 67 / 125 us with a GEMV per slot, 43 / 57 / 64 streamed; Q6_K 68 / 98 / 196 against 87 / 102 / 116.
-// Up to 32 slots per expert it is ahead of the routed tile kernel (Q4_0, 32 / 64 / 256 / 512 slots: 214 / 208 / 215 / 245 us against
-// 65 / 78 / 192 / 304; 16 experts of 2048 x 2048, 512 slots: 63 against 28).
-static bool use_skinny(int type, const void *as, int64_t K, int64_t n_expert, int64_t n_used, int64_t T) {
+// Up to 32 slots per expert it is ahead of the routed tile kernels (Q4_0, 32 / 64 / 256 / 512 slots: 214 / 208 / 215 / 245 us against
+// 65 / 78 / 192 / 304; 16 experts of 2048 x 2048, 256 slots: 63 against 28; IQ4_XS 226 / 225 / 235 / 253 against 75 / 86 / 172 / 278); for the
+// types whose routed kernel has 64-column tiles (routed, Q4_K and Q6_K) up to 16 (Q4_K, 32 / 64 / 128 / 256 slots: 147 / 146 / 149 / 154 us
+// against 72 / 91 / 130 / 192; Q6_K 211 / 212 / 221 / 228 against 112 / 130 / 168 / 257).
+static bool use_skinny(int type, const void *as, int64_t K, int64_t n_expert, int64_t n_used, int64_t T, bool routed) {
     const int64_t S = T * n_used;
-    if (!mi355_mul_mat_id_skinny_supported(type, as, K, n_expert, n_used, T) || S > 32 * n_expert) return false;
+    const int64_t most = routed && (type == MI355_Q4_K || type == MI355_Q6_K) ? 16 : 32;
+    if (!mi355_mul_mat_id_skinny_supported(type, as, K, n_expert, n_used, T) || S > most * n_expert) return false;
     const double chosen = (double)n_expert * (1.0 - pow(1.0 - 1.0 / (double)n_expert, (double)S));
     return (double)S >= (type == MI355_Q6_K ? 2.1 : 1.7) * chosen;
 }
@@ -53,13 +56,14 @@ int mi355_mul_mat_id(void *stream, int type, const void *as, const float *b, con
     if (use_routed_tiles(type, as, N, K, n_expert, n_used, T)) {
         int rc = mi355_quantize_act_q8k(stream, b, ws, K, nb1 * T, K);
         if (rc != MI355_OK) return rc;
+        if (use_skinny(type, as, K, n_expert, n_used, T, true)) return mi355_mul_mat_id_skinny_q8k(stream, type, as, ws, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T);
         const size_t act = (mi355_act_bytes(K, nb1 * T) + 255) & ~(size_t)255;
         return mi355_mul_mat_id_q8k(stream, type, as, ws, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, (uint8_t *)ws + act,
                                     ws_bytes - act);
     }
     int rc = mi355_quantize_act(stream, b, ws, K, nb1 * T, K);
     if (rc != MI355_OK) return rc;
-    if (use_skinny(type, as, K, n_expert, n_used, T)) return mi355_mul_mat_id_skinny(stream, type, as, ws, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T);
+    if (use_skinny(type, as, K, n_expert, n_used, T, false)) return mi355_mul_mat_id_skinny(stream, type, as, ws, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T);
     if (T * n_used >= ROUTED_MIN_SLOTS && mi355_mul_mat_id_q_supported(type, as, N, K, n_expert)) {   // per-32-block types and the super-block types whose rows are no multiple of 16 bytes: the routed form of the per-block tile kernel
         const size_t act = (mi355_act_bytes(K, nb1 * T) + 255) & ~(size_t)255;
         return mi355_mul_mat_id_q(stream, type, as, ws, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, (uint8_t *)ws + act, ws_bytes - act);

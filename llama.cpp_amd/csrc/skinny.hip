@@ -19,6 +19,7 @@
 // Activations are the Q8_1 workspace of mi355_quantize_act (ggml-cpu quantizes to Q8_0/Q8_1 for Q4_0/Q8_0 weights and to
 // Q8_K for Q4_K, ggml-cpu.c:7420-7450; the NMSE bound of the product is what is checked for Q4_K).
 #include "qdot.hpp"
+#include "q8k.hpp"
 
 namespace mi355 {
 
@@ -71,6 +72,8 @@ template <int TYPE, int NI> struct sk_regs {
     u32x4 qh[2];                            // Q6_K: the high bit pairs, 32 rows x 64 bytes (on their way to LDS); Q5_0 / Q5_1: the
                                             // eight fifth-bit words of the lane's row; Q5_K ([0] only): qh bytes 16 (lane / 32) .. + 16
     u32 d6;                                 // Q6_K: the f16 super-block scale of the lane's row (hdr holds its 16 int8 scales)
+    u32x4 t1;                               // Q8K: the second half of the column's block sums; its scale
+    float d8;
 };
 
 // grid.x = 32-row tiles of the weight matrix, grid.y = slices of K (partial sums to `dst` as [slice][B][dst_stride] then).
@@ -86,17 +89,25 @@ struct sk_id {
     int64_t ids_stride, expert_bytes;
     int n_used, nb1, n_slots;
 };
-template <int TYPE, int NI, bool TAIL, bool ID = false>
+//
+// Q8K: activations in the per-super-block form of mi355_quantize_act_q8k (one scale per 256 elements, the sums of its eight 32-element
+// blocks), the format ggml-cpu multiplies the super-block types with: aux1 = scales, aux2 = sums.  The integer block scales multiply the
+// block sums in 24-bit integer multiply-adds and a value meets f32 once per super-block (ggml_vec_dot_q4_K_q8_K / _q5_K_ / _q6_K_ / _iq4_xs_q8_K,
+// ggml/src/ggml-cpu/ggml-cpu-quants.c:6817-6848, 7539-7592, 8262-8283, 11381): 21 vector instructions per value and super-block for Q4_K
+// against 32 of the Q8_1 form.
+struct sk_q8k { const float *d; const _Float16 *bs; };
+__device__ __forceinline__ int mul24(int a, int b) { return ((a << 8) >> 8) * ((b << 8) >> 8); }   // v_mul_i32_i24 / v_mad_i32_i24
+template <int TYPE, int NI, bool TAIL, bool ID = false, bool Q8K = false>
 __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads,
                                                    float *__restrict__ dst, const float *__restrict__ residual, int64_t N, int K, int B,
-                                                   int64_t dst_stride, int steps_per_slice, int steps_per_wave, sk_id id) {
+                                                   int64_t dst_stride, int steps_per_slice, int steps_per_wave, sk_id id, sk_q8k q8) {
     typedef sk_traits<TYPE> T;
     typedef sk_regs<TYPE, NI> R;
     constexpr int WPAD = T::ROW_BYTES + 16;
     constexpr int QHPAD = 64 + 16;
     constexpr bool Q6 = TYPE == MI355_Q6_K;
     constexpr int W_BYTES = 32 * WPAD + (Q6 ? 32 * QHPAD : 0), A_BYTES = 8 * NI * SK_APAD, T_BYTES = 8 * 8 * NI * 8;
-    constexpr int G_BYTES = Q6 ? 16 * 8 * NI * 4 : 0;   // Q6_K: integer sums of the activation levels per 16 elements
+    constexpr int G_BYTES = Q6 && !Q8K ? 16 * 8 * NI * 4 : 0;   // Q6_K: integer sums of the activation levels per 16 elements
     constexpr int WAVE_BYTES = W_BYTES + A_BYTES + T_BYTES + G_BYTES;
     constexpr int RED_BYTES = 4 * NI * 4 * 64 * 4;
     __shared__ __attribute__((aligned(16))) uint8_t s_mem[4 * WAVE_BYTES > RED_BYTES ? 4 * WAVE_BYTES : RED_BYTES];
@@ -107,6 +118,8 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     uint8_t *s_a = s_w + W_BYTES;
     float2 *s_t = (float2 *)(s_a + A_BYTES);
     int *s_g = (int *)(s_a + A_BYTES + T_BYTES);
+    int *s_b = (int *)s_t;                        // Q8K: the sums of the eight blocks [8][8 NI], then the scales [8 NI] (T_BYTES hold them)
+    float *s_d8 = (float *)s_t + 8 * 8 * NI;
     uint8_t *s_qh = s_w + 32 * WPAD;
 
     __shared__ unsigned short s_slot[ID ? SK_MAX_SLOTS : 1];
@@ -170,7 +183,9 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     const int t_piece = lane & 3, t_row = lane >> 2;   // {d, sum} pairs: 4 lanes x 16 bytes per activation row and step
     const act_ds *t_src[R::NT];
 #pragma unroll
-    for (int u = 0; u < R::NT; u++) t_src[u] = ads + act_row(t_row + 16 * u) * nblk + 2 * t_piece;
+    for (int u = 0; u < R::NT; u++) t_src[u] = Q8K ? nullptr : ads + act_row(t_row + 16 * u) * nblk + 2 * t_piece;
+    // Q8K: lane c < 8 NI brings the scale and the block sums of column c
+    const int64_t q8_row = Q8K ? act_row(lane < 8 * NI ? lane : 0) * (K >> 8) : 0;
 
     // The last step of a row whose K is no multiple of 256: blocks past the end repeat the last one (nothing is read behind the row) and
     // get scale and minimum 0; the activation bytes they meet are those of the last block too, hence finite.
@@ -253,8 +268,14 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
         }
 #pragma unroll
         for (int u = 0; u < R::NA; u++) g.a[u] = load16(a_src[u] + s * 256);
+        if constexpr (Q8K) {
+            g.t[0] = load16(q8.bs + (q8_row + s) * 16);
+            g.t1 = load16(q8.bs + (q8_row + s) * 16 + 8);
+            g.d8 = q8.d[q8_row + s];
+        } else {
 #pragma unroll
-        for (int u = 0; u < R::NT; u++) g.t[u] = *(const u32x4_a8 *)(t_src[u] + s * 8);
+            for (int u = 0; u < R::NT; u++) g.t[u] = *(const u32x4_a8 *)(t_src[u] + s * 8);
+        }
     };
 
     float acc[NI][4];
@@ -278,13 +299,21 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
 #pragma unroll
         for (int u = 0; u < R::NA; u++) {
             *(u32x4 *)(s_a + (a_row + 4 * u) * SK_APAD + 16 * a_piece) = cur.a[u];
-            if constexpr (Q6) {   // the lane's 16 bytes are one 16-element group of its activation row
+            if constexpr (Q6 && !Q8K) {   // the lane's 16 bytes are one 16-element group of its activation row
                 int sum = 0;
 #pragma unroll
                 for (int i = 0; i < 4; i++) sum = dot4(0x01010101, (int)cur.a[u][i], sum);
                 s_g[a_piece * (8 * NI) + a_row + 4 * u] = sum;
             }
         }
+        if constexpr (Q8K) {
+            if (lane < 8 * NI) {
+                const f16x8 lo = __builtin_bit_cast(f16x8, cur.t[0]), hi = __builtin_bit_cast(f16x8, cur.t1);   // sum = 64 hi + lo
+#pragma unroll
+                for (int j = 0; j < 8; j++) s_b[j * (8 * NI) + lane] = (int)(float)lo[j] + 64 * (int)(float)hi[j];
+                s_d8[lane] = cur.d8;
+            }
+        } else {
 #pragma unroll
         for (int u = 0; u < R::NT; u++) {
             if (t_row + 16 * u < 8 * NI) {
@@ -300,6 +329,7 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
                 }
             }
         }
+        }
         const u32x4 hdr = cur.hdr, hdr2 = cur.hdr2;
         const u32x4 fifth[2] = {cur.qh[0], cur.qh[1]};   // (Q6_K's went to LDS above)
         const u32 d6 = cur.d6;
@@ -307,7 +337,106 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
         if (step + 1 < s_hi) fetch(step + 1, cur);
 
         const int am = r < 8 * NI ? r : r & 7;   // operand rows past the copied ones repeat copied ones; their results are not used
-        if constexpr (Q6) {
+        if constexpr (Q8K) {
+            int isum[NI][4], msum[NI][4];   // sum of scale * block sum; sum of minimum * sum of levels (Q4_K, Q5_K)
+#pragma unroll
+            for (int qq = 0; qq < NI; qq++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) isum[qq][i] = msum[qq][i] = 0;
+            i32x16 z;
+#pragma unroll
+            for (int i = 0; i < 16; i++) z[i] = 0;
+            float dw, dmin = 0.0f;
+            if constexpr (Q6) {
+                dw = half_bits_to_float((unsigned short)d6);
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+                    for (int is = 0; is < 2; is++) {
+                        const u32x2 qh8 = *(const u32x2 *)(s_qh + r * QHPAD + 32 * hf + 16 * is + 8 * kh);
+#pragma unroll
+                        for (int qlo = 0; qlo < 2; qlo++) {
+                            const u32x2 ql8 = *(const u32x2 *)(s_w + r * WPAD + 64 * hf + 32 * qlo + 16 * is + 8 * kh);
+#pragma unroll
+                            for (int qhi = 0; qhi < 2; qhi++) {
+                                const int q = qlo + 2 * qhi, g = 8 * hf + 2 * q + is;   // as in the Q8_1 form below
+                                u32x2 lv;
+#pragma unroll
+                                for (int i = 0; i < 2; i++) {   // level - 32 per byte: flip bit 5, then sign-extend it into bits 6 and 7
+                                    const u32 t = (((ql8[i] >> (4 * qhi)) & 0x0F0F0F0Fu) | (((qh8[i] >> (2 * q)) & 0x03030303u) << 4)) ^ 0x20202020u;
+                                    const u32 m = t & 0x20202020u;
+                                    lv[i] = t | (m << 1) | (m << 2);
+                                }
+                                const u32x2 a8 = *(const u32x2 *)(s_a + am * SK_APAD + 128 * hf + 32 * q + 16 * is + 8 * kh);
+                                const i32x16 D = __builtin_amdgcn_mfma_i32_32x32x16_i8(__builtin_bit_cast(long, a8), __builtin_bit_cast(long, lv), z, 0, 0, 0);
+                                const u32 sc_word = hdr[g >> 2];
+                                const int sc = (int)(signed char)((sc_word >> (8 * (g & 3))) & 0xFFu);
+#pragma unroll
+                                for (int qq = 0; qq < NI; qq++)
+#pragma unroll
+                                    for (int i = 0; i < 4; i++) isum[qq][i] += mul24(sc, D[4 * qq + i]);
+                            }
+                        }
+                    }
+            } else {
+                int sc[8], mn[8];
+                if constexpr (T::KQ) {
+                    dw = half_bits_to_float((unsigned short)(hdr[0] & 0xFFFFu));
+                    dmin = half_bits_to_float((unsigned short)(hdr[0] >> 16));
+                    const u32 u0 = hdr[1], u1 = hdr[2], u2 = hdr[3];
+                    const u32 s_lo = u0 & 0x3F3F3F3Fu, m_lo = u1 & 0x3F3F3F3Fu;
+                    const u32 s_hi = (u2 & 0x0F0F0F0Fu) | (((u0 >> 6) & 0x03030303u) << 4);
+                    const u32 m_hi = ((u2 >> 4) & 0x0F0F0F0Fu) | (((u1 >> 6) & 0x03030303u) << 4);
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        sc[j] = (int)(((j < 4 ? s_lo : s_hi) >> (8 * (j & 3))) & 0xFFu);
+                        mn[j] = (int)(((j < 4 ? m_lo : m_hi) >> (8 * (j & 3))) & 0xFFu);
+                    }
+                } else {   // IQ4_XS
+                    dw = half_bits_to_float((unsigned short)(hdr[0] & 0xFFFFu));
+#pragma unroll
+                    for (int j = 0; j < 8; j++) sc[j] = (int)(((hdr[1] >> (4 * j)) & 0xFu) | (((hdr[0] >> (16 + 2 * j)) & 3u) << 4)) - 32;
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    i32x4 wop;
+                    if constexpr (T::KQ) {
+                        const u32x4 v = *(const u32x4 *)(s_w + r * WPAD + 32 * (j >> 1) + 16 * kh);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            wop[i] = (int)((v[i] >> (4 * (j & 1))) & 0x0F0F0F0Fu);
+                            if constexpr (TYPE == MI355_Q5_K) wop[i] |= (int)(((fifth[0][i] >> j) & 0x01010101u) << 4);
+                        }
+                    } else {
+                        const u32x4 v = *(const u32x4 *)(s_w + r * WPAD + 16 * j);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) wop[i] = (int)iq4nl_lookup4((v[i] >> (4 * kh)) & 0x0F0F0F0Fu);
+                    }
+                    const i32x4 aop = *(const i32x4 *)(s_a + am * SK_APAD + 32 * j + 16 * kh);
+                    const i32x16 D = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop, wop, z, 0, 0, 0);
+#pragma unroll
+                    for (int qq = 0; qq < NI; qq++) {
+                        if constexpr (T::KQ) {
+                            const i32x4 b = *(const i32x4 *)(s_b + j * (8 * NI) + 8 * qq + 4 * kh);
+#pragma unroll
+                            for (int i = 0; i < 4; i++) msum[qq][i] += mul24(mn[j], b[i]);
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; i++) isum[qq][i] += mul24(sc[j], D[4 * qq + i]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int qq = 0; qq < NI; qq++) {
+                const f32x4 d8 = *(const f32x4 *)(s_d8 + 8 * qq + 4 * kh);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float v = dw * (float)isum[qq][i];
+                    if constexpr (T::KQ) v = __builtin_fmaf(-dmin, (float)msum[qq][i], v);
+                    acc[qq][i] = __builtin_fmaf(d8[i], v, acc[qq][i]);
+                }
+            }
+        } else if constexpr (Q6) {
             // 16 groups of 16 levels, each with its own int8 scale: one v_mfma_i32_32x32x16_i8 per group (8 levels per lane).
             // Group (hf, q, is): levels 128 hf + 32 q + 16 is .. + 16; level l of it = nibble q / 2 of ql byte 64 hf + 32 (q % 2) + 16 is + l
             // plus bits 2q, 2q + 1 of qh byte 32 hf + 16 is + l, minus 32 (dequantize_row_q6_K, ggml/src/ggml-quants.c:1690-1719).
@@ -479,9 +608,9 @@ void launch_skinny(hipStream_t s, const void *W, const int8_t *aq, const act_ds 
     const int64_t stride = slices == 1 ? dst_stride : N;
     constexpr bool BLOCKS32 = (sk_traits<TYPE>::NIB32 && TYPE != MI355_IQ4_XS) || TYPE == MI355_Q8_0;
     if (BLOCKS32 && K % 256 != 0)
-        MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave, sk_id{});
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave, sk_id{}, sk_q8k{});
     else
-        MI355_LAUNCH((k_mm_skinny<TYPE, NI, false>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave, sk_id{});
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, false>), grid, dim3(256), 0, s, (const uint8_t *)W, aq, ads, out, res, N, K, B, stride, steps_per_slice, steps_per_wave, sk_id{}, sk_q8k{});
     if (slices > 1) {
         MI355_LAUNCH(k_skinny_slices, dim3((unsigned)((N + 255) / 256), (unsigned)B), dim3(256), 0, s, part, dst, residual, N, B, dst_stride, slices);
     }
@@ -502,9 +631,16 @@ void launch_skinny_id(hipStream_t s, const void *as, const int8_t *aq, const act
     const dim3 grid((unsigned)((N + 31) / 32), 1, (unsigned)n_expert);
     constexpr bool BLOCKS32 = (sk_traits<TYPE>::NIB32 && TYPE != MI355_IQ4_XS) || TYPE == MI355_Q8_0;
     if (BLOCKS32 && K % 256 != 0)
-        MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32, true>), grid, dim3(256), 0, s, (const uint8_t *)as, aq, ads, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id);
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32, true>), grid, dim3(256), 0, s, (const uint8_t *)as, aq, ads, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id, sk_q8k{});
     else
-        MI355_LAUNCH((k_mm_skinny<TYPE, NI, false, true>), grid, dim3(256), 0, s, (const uint8_t *)as, aq, ads, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id);
+        MI355_LAUNCH((k_mm_skinny<TYPE, NI, false, true>), grid, dim3(256), 0, s, (const uint8_t *)as, aq, ads, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id, sk_q8k{});
+}
+
+template <int TYPE, int NI>
+void launch_skinny_id_q8k(hipStream_t s, const void *as, const int8_t *aq, const sk_q8k &q8, float *dst, int64_t N, int K, int64_t n_expert, const sk_id &id) {
+    const int nsteps = K >> 8;
+    MI355_LAUNCH((k_mm_skinny<TYPE, NI, false, true, true>), dim3((unsigned)((N + 31) / 32), 1, (unsigned)n_expert), dim3(256), 0, s, (const uint8_t *)as, aq,
+                 (const act_ds *)nullptr, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id, q8);
 }
 
 // slices of K: launches with fewer than ~1.5 groups per compute unit split K over several groups (and pay a second launch
@@ -576,6 +712,31 @@ int mi355_mul_mat_id_skinny(void *stream, int type, const void *as, const void *
     else if (avg <= SK_ID_WIDE) launch_skinny_id<TY, 2>(s, as, aq, ads, dst, N, (int)K, n_expert, id); \
     else launch_skinny_id<TY, 4>(s, as, aq, ads, dst, N, (int)K, n_expert, id);
     MI355_WEIGHT_TYPE_SWITCH(type, X)
+#undef X
+    return launch_status("k_mm_skinny (experts)");
+}
+
+int mi355_mul_mat_id_skinny_q8k(void *stream, int type, const void *as, const void *act, const int32_t *ids, int64_t ids_stride, float *dst, int64_t N,
+                                int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T) {
+    MI355_REQUIRE((type == MI355_Q4_K || type == MI355_Q5_K || type == MI355_Q6_K || type == MI355_IQ4_XS) && mi355_mul_mat_id_skinny_supported(type, as, K, n_expert, n_used, T),
+                  "mul_mat_id_skinny_q8k: type %d, K=%lld, %lld slots or the weight alignment is not supported", type, (long long)K, (long long)(T * n_used));
+    MI355_REQUIRE(N > 0 && nb1 > 0 && ids_stride >= n_used, "mul_mat_id_skinny_q8k: bad shape");
+    MI355_REQUIRE(((uintptr_t)act & 15) == 0 && (q8k_bs_offset(K, nb1 * T) & 15) == 0, "mul_mat_id_skinny_q8k: activation workspace is not 16-byte aligned");
+    hipStream_t s = (hipStream_t)stream;
+    const int8_t *aq = (const int8_t *)act;
+    const sk_q8k q8 = {(const float *)(aq + q8k_d_offset(K, nb1 * T)), (const _Float16 *)(aq + q8k_bs_offset(K, nb1 * T))};
+    const sk_id id = {ids, ids_stride, N * make_row_layout(type, K).row_bytes, (int)n_used, (int)nb1, (int)(T * n_used)};
+    const int64_t avg = T * n_used / n_expert;   // slots per expert
+#define X(TY)                                                                                           \
+    if (avg <= SK_ID_NARROW) launch_skinny_id_q8k<TY, 1>(s, as, aq, q8, dst, N, (int)K, n_expert, id); \
+    else if (avg <= SK_ID_WIDE) launch_skinny_id_q8k<TY, 2>(s, as, aq, q8, dst, N, (int)K, n_expert, id); \
+    else launch_skinny_id_q8k<TY, 4>(s, as, aq, q8, dst, N, (int)K, n_expert, id);
+    switch (type) {
+        case MI355_Q4_K: X(MI355_Q4_K) break;
+        case MI355_Q5_K: X(MI355_Q5_K) break;
+        case MI355_IQ4_XS: X(MI355_IQ4_XS) break;
+        default: X(MI355_Q6_K) break;
+    }
 #undef X
     return launch_status("k_mm_skinny (experts)");
 }

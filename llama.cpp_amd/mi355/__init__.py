@@ -136,6 +136,7 @@ _SIGNATURES = {
     "mi355_moe_combine": (_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64]),
     "mi355_mul_mat_id_skinny_supported": (_int, [_int, _p, _i64, _i64, _i64, _i64]),
     "mi355_mul_mat_id_skinny": (_int, [_p, _int, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64]),
+    "mi355_mul_mat_id_skinny_q8k": (_int, [_p, _int, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64]),
     "mi355_mul_mat_id_q_supported": (_int, [_int, _p, _i64, _i64, _i64]),
     "mi355_mul_mat_id_q": (_int, [_p, _int, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p, _sz]),
     "mi355_mul_mat_id_vec": (_int, [_p, _int, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64]),

@@ -180,3 +180,10 @@ def test_mul_mat_id_skinny(dev, name, t, n_expert, n_used, bcast, T, pattern):
     torch.cuda.synchronize()
     want = expected_per_expert("q8_1", t, Wq, b, np.clip(ids, 0, n_expert - 1), n_expert, n_used, nb1, N)
     assert orc.nmse(got.cpu().numpy(), want) < 1e-11
+    if t in (orc.Q4_K, orc.Q5_K, orc.Q6_K, orc.IQ4_XS):   # the form on Q8_K activations: the CPU path's integer sums
+        act = mi355.quantize_act_q8k(torch.from_numpy(b.reshape(T * nb1, K)).to(dev))
+        got.fill_(float("nan"))
+        mi355.check(lib.mi355_mul_mat_id_skinny_q8k(None, t, Wd.data_ptr(), act.data_ptr(), idd.data_ptr(), idd.stride(0), got.data_ptr(), N, K, n_expert, n_used, nb1, T))
+        torch.cuda.synchronize()
+        want = expected_per_expert("cpu", t, Wq, b, np.clip(ids, 0, n_expert - 1), n_expert, n_used, nb1, N)
+        assert orc.nmse(got.cpu().numpy(), want) < 1e-11
