@@ -17,7 +17,7 @@
 //   Q4_1, Q5_1 : level 0..15 / 0..31 as int8, scale d; the "+ m * d_x * sum(q)" term of the stage's four blocks is added with two
 //          v_mfma_f32_32x32x2_f32 on (dx * sum(q)) x m
 //   Q4_K, Q5_K : level 0..15 / 0..31 as int8, scale d*sc; the "- dmin*m*sum(q)" term of the blocks the same way
-//   Q6_K : level - 32 as int8, scale d*sc per 16 elements (two MFMAs per block, each on the lane half that holds its elements)
+//   Q6_K : level - 32 as int8, scale d*sc per 16 elements (two v_mfma_i32_32x32x16_i8 per block)
 //
 // MFMA operand mapping used here (A = activations, B = weights, D[i][j], i = activation
 // row, j = weight row): lane l supplies row/column l % 32 and the k bytes
@@ -338,19 +338,24 @@ struct mmq_mat {
 };
 struct mmq_mats { mmq_mat m[MMQ_MATS]; };
 
-template <int TYPE, int TN, bool ID = false>
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ long pair64(int lo, int hi) { return (long)((uint64_t)(u32)lo | (uint64_t)(u32)hi << 32); }
+
+template <int V> struct mmq_int { static constexpr int value = V; };
+
+template <int TYPE, int TNK, bool ID = false>
 __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, int64_t K, int64_t B,
                                              row_layout L, int n_col_tiles, int n_groups, int n_groups_padded, int64_t slice_stride,
                                              mmq32_route route) {
     typedef mmq_cfg<TYPE> C;
-    constexpr int BN = 64 * TN;
+    constexpr int BNK = 64 * TNK;
     struct stage_mem {
         __attribute__((aligned(16))) int8_t w[MMQ_BM * MMQ_BK];
-        __attribute__((aligned(16))) int8_t a[BN * MMQ_BK];
+        __attribute__((aligned(16))) int8_t a[BNK * MMQ_BK];
         __attribute__((aligned(16))) float ws[C::NG * MMQ_BM];
-        __attribute__((aligned(16))) _Float16 ad[4 * BN];
+        __attribute__((aligned(16))) _Float16 ad[4 * BNK];
         __attribute__((aligned(16))) float wo[C::MIN ? MMQ_BM * 4 : 4];
-        __attribute__((aligned(16))) float as[C::MIN ? BN * 4 : 4];
+        __attribute__((aligned(16))) float as[C::MIN ? BNK * 4 : 4];
     };
     __shared__ stage_mem sm[2];
 
@@ -369,7 +374,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
     const float *residual = mats.m[mi].residual;
     const int64_t N = mats.m[mi].N, dst_stride = mats.m[mi].dst_stride;
     const int64_t row0 = (int64_t)(row_tile - mats.m[mi].first_row_tile) * MMQ_BM;
-    int64_t col0 = (int64_t)col_tile * BN;
+    int64_t col0 = (int64_t)col_tile * BNK;
     const int32_t *row_of = nullptr;
     if constexpr (ID) {
         const int ct = col_tile;
@@ -383,165 +388,184 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l32 = lane & 31, lhi = lane >> 5;
     const int wrow0 = (wave & 1) * 64;           // weight rows of this wave inside the tile
-    const int wcol0 = (wave >> 1) * (32 * TN);   // activation rows of this wave inside the tile
-
-    f32x16 acc[TN][2];
-#pragma unroll
-    for (int tb = 0; tb < TN; tb++)
-#pragma unroll
-        for (int tw = 0; tw < 2; tw++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[tb][tw][r] = 0.0f;
-
-    i32x16 magic;
-#pragma unroll
-    for (int r = 0; r < 16; r++) magic[r] = MMQ_MAGIC_BITS;
 
     // split K: grid row y walks stages [k_lo, k_hi) and writes its sums to slice y of `dst` (a workspace then, see launch_mmq)
     const int nblk = (int)(K >> 5), stages = (nblk + MMQ_BK / QK - 1) / (MMQ_BK / QK), st_per = (stages + (int)gridDim.y - 1) / (int)gridDim.y;
     const int s_lo = (int)blockIdx.y * st_per, s_hi = s_lo + st_per < stages ? s_lo + st_per : stages;
     if (gridDim.y > 1) dst += (int64_t)blockIdx.y * slice_stride;
 
-    mmq_wregs<TYPE> wregs;
-    mmq_aregs<BN, C::MIN, ID> aregs;
-    wregs.init(W, L, row0, N, threadIdx.x);
-    aregs.init(aq, ads, col0, B, nblk, threadIdx.x, row_of);
-    auto fetch = [&](int st) {
-        wregs.fetch(L, st * MMQ_BK, nblk, threadIdx.x);
-        aregs.fetch(st * MMQ_BK, nblk, threadIdx.x);
-    };
-    auto commit = [&](stage_mem &m, int st) {
-        wregs.commit(m.w, m.ws, m.wo, st * MMQ_BK, nblk, threadIdx.x);
-        aregs.commit(m.a, m.ad, m.as, threadIdx.x);
-    };
-
-    // operands and scales of one Q8_1 block for the wave's tiles
-    constexpr int NS = C::G == 32 ? 1 : 2;   // scale groups per block
-    struct block_ops { i32x4 a[TN], w[2]; };
-    struct block_scales {
-        f16x8 dx[TN][2];     // activation block scales of this lane's 16 rows per tile
-        float dw[2][NS];
-    };
-    int a_at = mmq_chunk(wcol0 + l32, lhi), w_at = mmq_chunk(wrow0 + l32, lhi);
-    auto load_ops = [&](const stage_mem &m, int ks) {
-        block_ops f;
-#pragma unroll
-        for (int tb = 0; tb < TN; tb++) f.a[tb] = *(const i32x4 *)(m.a + tb * 32 * MMQ_BK + (a_at ^ (ks << 5)));   // chunk 2 ks + lhi
-#pragma unroll
-        for (int tw = 0; tw < 2; tw++) f.w[tw] = *(const i32x4 *)(m.w + tw * 32 * MMQ_BK + (w_at ^ (ks << 5)));
-        return f;
-    };
-    auto load_scales = [&](const stage_mem &m, int ks) {
-        block_scales f;
-#pragma unroll
+    // ID: a tile whose columns all lie in its first half (the second tile of an expert that is routed a few more than 128 slots) runs with
+    // half the columns per wave: half the matrix instructions and sums to scale (8 experts of 14336 x 4096: Q8_0, 1400 slots 463 -> 377 us,
+    // Q4_0, 1024 slots 342 -> 330).  Uniform for the whole group.  Not for batches: their groups mostly run in one round, whose time is
+    // that of the full tiles (Q4_0 14336 x 4096, 160 rows: 63 us with and without, 512 rows 99.5 -> 100.2 for the larger kernel).
+    auto walk = [&](auto tn) __attribute__((always_inline)) {
+        constexpr int TN = decltype(tn)::value, BN = 64 * TN;
+        const int wcol0 = (wave >> 1) * (32 * TN);   // activation rows of this wave inside the tile
+        f32x16 acc[TN][2];
+    #pragma unroll
         for (int tb = 0; tb < TN; tb++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) f.dx[tb][h] = *(const f16x8 *)(m.ad + ks * BN + wcol0 + tb * 32 + 16 * lhi + 8 * h);
-#pragma unroll
-        for (int tw = 0; tw < 2; tw++)
-#pragma unroll
-            for (int h = 0; h < NS; h++) f.dw[tw][h] = m.ws[(ks * NS + h) * MMQ_BM + wrow0 + tw * 32 + l32];
-        return f;
-    };
-    // matrix instruction n of a block: tile (tb, tw), scale group h.  Two groups of 16 (Q6_K): the operands hold 16 consecutive elements
-    // per lane half, so group h is the half lhi == h, and the other half of the weights is zeroed.
-    constexpr int NM = TN * 2 * NS;
-    auto mma = [&](const block_ops &f, int n) {
-        const int tb = n / NS % TN, tw = n / NS / TN, h = n % NS;
-        i32x4 w = f.w[tw];
-        if constexpr (NS == 2) {
-            const int keep = lhi == h ? -1 : 0;
-#pragma unroll
-            for (int i = 0; i < 4; i++) w[i] &= keep;
-        }
-        return __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[tb], w, magic, 0, 0, 0);
-    };
-    auto scale = [&](const block_scales &f, int n, const i32x16 &I) {
-        const int tb = n / NS % TN, tw = n / NS / TN, h = n % NS;
-        const float dw = f.dw[tw][h], mdw = -MMQ_MAGIC * dw;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int bits = I[r];
-            acc[tb][tw][r] = __builtin_fmaf(__builtin_fmaf(__builtin_bit_cast(float, bits), dw, mdw), (float)f.dx[tb][r >> 3][r & 7], acc[tb][tw][r]);
-        }
-    };
+    #pragma unroll
+            for (int tw = 0; tw < 2; tw++)
+    #pragma unroll
+                for (int r = 0; r < 16; r++) acc[tb][tw][r] = 0.0f;
 
-    fetch(s_lo);
-    commit(sm[0], s_lo);
-    fetch(s_lo + 1 < s_hi ? s_lo + 1 : s_lo);
-    __syncthreads();
-    int buf = 0;
-    for (int st = s_lo; st < s_hi; st++, buf ^= 1) {
-        const stage_mem &m = sm[buf];
-        asm volatile("" : "+v"(a_at), "+v"(w_at));   // the four chunk addresses of a stage are formed in the loop: kept across it they cost spills
-        // One matrix instruction is always in flight: its successor is issued before its sums are scaled, so that neither waits for the
-        // other (left to the compiler, all of them write the same registers one after the other); the next block's operands are read
-        // from LDS while the last sums of this one are scaled.
-        block_ops f = load_ops(m, 0);
-        block_scales sc = load_scales(m, 0);
-        i32x16 I = mma(f, 0);
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            block_scales sc_next = sc;
-#pragma unroll
-            for (int n = 0; n < NM; n++) {
-                const i32x16 cur = I;
-                I = mma(f, n + 1 < NM ? n + 1 : 0);   // (the last one of a stage is not used)
-                __builtin_amdgcn_sched_barrier(0);
-                if (n == NM - 2 && ks < 3) f = load_ops(m, ks + 1);
-                if (n == NM - 1 && ks < 3) sc_next = load_scales(m, ks + 1);
-                scale(sc, n, cur);
-                asm volatile("" : "+v"(acc[n / NS % TN][n / NS / TN]));   // formed here, and not behind the matrix instructions of the whole stage
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            sc = sc_next;
-        }
-        if constexpr (C::MIN) {
-            // acc += sum_b (dx * sum q)[i][b] * m[j][b] over the 4 blocks of the stage (Q4_K, Q5_K: m = -dmin * 6-bit minimum): two
-            // v_mfma_f32_32x32x2_f32 per tile on the matrix pipe, which waits for the vector ALUs anyway; k = lane / 32.  In f32 as the
-            // batch-1 kernels do it (as f16 operands the term carried 3.6e-4 of the result).
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                float af[TN], bf[2];
-#pragma unroll
-                for (int tb = 0; tb < TN; tb++) af[tb] = m.as[(2 * p + lhi) * BN + wcol0 + tb * 32 + l32];
-#pragma unroll
-                for (int tw = 0; tw < 2; tw++) bf[tw] = m.wo[(2 * p + lhi) * MMQ_BM + wrow0 + tw * 32 + l32];
-#pragma unroll
-                for (int tb = 0; tb < TN; tb++)
-#pragma unroll
-                    for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
-            }
-        }
-        if (st + 1 < s_hi) {   // the next stage, requested one stage ago, goes to the other buffer (uniform)
-            commit(sm[buf ^ 1], st + 1);
-            fetch(st + 2 < s_hi ? st + 2 : st + 1);   // past the end the last stage is requested again and never used
-            __syncthreads();
-        }
-    }
+        i32x16 magic;
+    #pragma unroll
+        for (int r = 0; r < 16; r++) magic[r] = MMQ_MAGIC_BITS;
 
-    // store: lane holds weight row j = l32 of each 32-wide tile, 16 activation rows
-#pragma unroll
-    for (int tb = 0; tb < TN; tb++)
-#pragma unroll
-        for (int tw = 0; tw < 2; tw++) {
-            const int64_t n = row0 + wrow0 + tw * 32 + l32;
-#pragma unroll
+        mmq_wregs<TYPE> wregs;
+        mmq_aregs<BN, C::MIN, ID> aregs;
+        wregs.init(W, L, row0, N, threadIdx.x);
+        aregs.init(aq, ads, col0, B, nblk, threadIdx.x, row_of);
+        auto fetch = [&](int st) {
+            wregs.fetch(L, st * MMQ_BK, nblk, threadIdx.x);
+            aregs.fetch(st * MMQ_BK, nblk, threadIdx.x);
+        };
+        auto commit = [&](stage_mem &m, int st) {
+            wregs.commit(m.w, m.ws, m.wo, st * MMQ_BK, nblk, threadIdx.x);
+            aregs.commit(m.a, m.ad, m.as, threadIdx.x);
+        };
+
+        // operands and scales of one Q8_1 block for the wave's tiles
+        constexpr int NS = C::G == 32 ? 1 : 2;   // scale groups per block
+        struct block_ops { i32x4 a[TN], w[2]; };
+        struct block_scales {
+            f16x8 dx[TN][2];     // activation block scales of this lane's 16 rows per tile
+            float dw[2][NS];
+        };
+        int a_at = NS == 1 ? mmq_chunk(wcol0 + l32, lhi) : mmq_chunk(wcol0 + l32, 0) + 8 * lhi;
+        int w_at = NS == 1 ? mmq_chunk(wrow0 + l32, lhi) : mmq_chunk(wrow0 + l32, 0) + 8 * lhi;
+        // one 16-byte chunk per lane half (2 ks + lhi); two groups of 16 (Q6_K): this lane half's 8 bytes of both groups' chunks
+        auto load_op = [&](const int8_t *m, int at, int ks) {
+            if constexpr (NS == 1) return *(const i32x4 *)(m + (at ^ (ks << 5)));
+            else {
+                const i32x2 g0 = *(const i32x2 *)(m + (at ^ (ks << 5))), g1 = *(const i32x2 *)(m + (at ^ (ks << 5) ^ 16));
+                return i32x4{g0[0], g0[1], g1[0], g1[1]};
+            }
+        };
+        auto load_ops = [&](const stage_mem &m, int ks) {
+            block_ops f;
+    #pragma unroll
+            for (int tb = 0; tb < TN; tb++) f.a[tb] = load_op(m.a + tb * 32 * MMQ_BK, a_at, ks);
+    #pragma unroll
+            for (int tw = 0; tw < 2; tw++) f.w[tw] = load_op(m.w + tw * 32 * MMQ_BK, w_at, ks);
+            return f;
+        };
+        auto load_scales = [&](const stage_mem &m, int ks) {
+            block_scales f;
+    #pragma unroll
+            for (int tb = 0; tb < TN; tb++)
+    #pragma unroll
+                for (int h = 0; h < 2; h++) f.dx[tb][h] = *(const f16x8 *)(m.ad + ks * BN + wcol0 + tb * 32 + 16 * lhi + 8 * h);
+    #pragma unroll
+            for (int tw = 0; tw < 2; tw++)
+    #pragma unroll
+                for (int h = 0; h < NS; h++) f.dw[tw][h] = m.ws[(ks * NS + h) * MMQ_BM + wrow0 + tw * 32 + l32];
+            return f;
+        };
+        // matrix instruction n of a block: tile (tb, tw), scale group h.  Two groups of 16 (Q6_K): one v_mfma_i32_32x32x16_i8 each (the
+        // 32-element form with half of the weights zeroed costs the vector ALU four more instructions).
+        constexpr int NM = TN * 2 * NS;
+        auto mma = [&](const block_ops &f, int n) {
+            const int tb = n / NS % TN, tw = n / NS / TN, h = n % NS;
+            if constexpr (NS == 1) return __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[tb], f.w[tw], magic, 0, 0, 0);
+            else return __builtin_amdgcn_mfma_i32_32x32x16_i8(pair64(f.a[tb][2 * h], f.a[tb][2 * h + 1]), pair64(f.w[tw][2 * h], f.w[tw][2 * h + 1]), magic, 0, 0, 0);
+        };
+        auto scale = [&](const block_scales &f, int n, const i32x16 &I) {
+            const int tb = n / NS % TN, tw = n / NS / TN, h = n % NS;
+            const float dw = f.dw[tw][h], mdw = -MMQ_MAGIC * dw;
+    #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const int64_t b = col0 + wcol0 + tb * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-                if (n < N && b < B) {
-                    const int64_t o = (ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n;
-                    dst[o] = residual ? acc[tb][tw][r] + residual[o] : acc[tb][tw][r];
+                const int bits = I[r];
+                acc[tb][tw][r] = __builtin_fmaf(__builtin_fmaf(__builtin_bit_cast(float, bits), dw, mdw), (float)f.dx[tb][r >> 3][r & 7], acc[tb][tw][r]);
+            }
+        };
+
+        fetch(s_lo);
+        commit(sm[0], s_lo);
+        fetch(s_lo + 1 < s_hi ? s_lo + 1 : s_lo);
+        __syncthreads();
+        int buf = 0;
+        for (int st = s_lo; st < s_hi; st++, buf ^= 1) {
+            const stage_mem &m = sm[buf];
+            asm volatile("" : "+v"(a_at), "+v"(w_at));   // the four chunk addresses of a stage are formed in the loop: kept across it they cost spills
+            // One matrix instruction is always in flight: its successor is issued before its sums are scaled, so that neither waits for the
+            // other (left to the compiler, all of them write the same registers one after the other); the next block's operands are read
+            // from LDS while the last sums of this one are scaled.
+            block_ops f = load_ops(m, 0);
+            block_scales sc = load_scales(m, 0);
+            i32x16 I = mma(f, 0);
+    #pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                block_scales sc_next = sc;
+    #pragma unroll
+                for (int n = 0; n < NM; n++) {
+                    const i32x16 cur = I;
+                    I = mma(f, n + 1 < NM ? n + 1 : 0);   // (the last one of a stage is not used)
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (n == NM - 2 && ks < 3) f = load_ops(m, ks + 1);
+                    if (n == NM - 1 && ks < 3) sc_next = load_scales(m, ks + 1);
+                    scale(sc, n, cur);
+                    asm volatile("" : "+v"(acc[n / NS % TN][n / NS / TN]));   // formed here, and not behind the matrix instructions of the whole stage
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                sc = sc_next;
+            }
+            if constexpr (C::MIN) {
+                // acc += sum_b (dx * sum q)[i][b] * m[j][b] over the 4 blocks of the stage (Q4_K, Q5_K: m = -dmin * 6-bit minimum): two
+                // v_mfma_f32_32x32x2_f32 per tile on the matrix pipe, which waits for the vector ALUs anyway; k = lane / 32.  In f32 as the
+                // batch-1 kernels do it (as f16 operands the term carried 3.6e-4 of the result).
+    #pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    float af[TN], bf[2];
+    #pragma unroll
+                    for (int tb = 0; tb < TN; tb++) af[tb] = m.as[(2 * p + lhi) * BN + wcol0 + tb * 32 + l32];
+    #pragma unroll
+                    for (int tw = 0; tw < 2; tw++) bf[tw] = m.wo[(2 * p + lhi) * MMQ_BM + wrow0 + tw * 32 + l32];
+    #pragma unroll
+                    for (int tb = 0; tb < TN; tb++)
+    #pragma unroll
+                        for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
                 }
             }
+            if (st + 1 < s_hi) {   // the next stage, requested one stage ago, goes to the other buffer (uniform)
+                commit(sm[buf ^ 1], st + 1);
+                fetch(st + 2 < s_hi ? st + 2 : st + 1);   // past the end the last stage is requested again and never used
+                __syncthreads();
+            }
         }
+
+        // store: lane holds weight row j = l32 of each 32-wide tile, 16 activation rows
+    #pragma unroll
+        for (int tb = 0; tb < TN; tb++)
+    #pragma unroll
+            for (int tw = 0; tw < 2; tw++) {
+                const int64_t n = row0 + wrow0 + tw * 32 + l32;
+    #pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int64_t b = col0 + wcol0 + tb * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
+                    if (n < N && b < B) {
+                        const int64_t o = (ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n;
+                        dst[o] = residual ? acc[tb][tw][r] + residual[o] : acc[tb][tw][r];
+                    }
+                }
+            }
+    };
+    if constexpr (ID) {
+        if (B - col0 <= BNK / 2) {
+            walk(mmq_int<1>{});
+            return;
+        }
+    }
+    walk(mmq_int<TNK>{});
 }
 
 // What bounds the kernel is the vector ALU: a wave issues 637 of its instructions per stage, 512 of them the two per block sum and 16
 // matrix instructions, which are busy a quarter of that time (counters, Q4_0 14336 x 4096, 512 rows; 4 cycles each = 2550 cycles of the
 // 2800 a stage takes with one group per compute unit).  Before the two-instruction form, the double-buffered stages and the f32 minima, by
 // type (14336 x 4096, 512 rows with the quantization launch, us): Q4_0 139 -> 116, Q4_1 228 -> 128, Q5_0 149 -> 124, Q5_1 229 -> 140,
-// IQ4_NL 149 -> 128, Q8_0 146 -> 130; 64 rows: Q4_0 34.3 -> 32.3.
+// IQ4_NL 149 -> 128, Q8_0 146 -> 130; 64 rows: Q4_0 34.3 -> 32.3.  Q6_K with 16-element instead of masked 32-element matrix
+// instructions: 4096 x 11008, 64 rows 41.2 -> 39.5.
 //
 // A product with few tiles leaves most of the chip idle while each group walks all of K: such launches are cut along K into
 // slices that run side by side and a second launch adds the slices in fixed order.  At least four stages per slice, at most

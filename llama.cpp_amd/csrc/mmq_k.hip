@@ -537,6 +537,8 @@ __device__ __forceinline__ void kp_dma_slot(int it, int &row, int &chunk) {
     chunk = (lane & 7) ^ ((row >> 1) & 7);
 }
 
+template <int V> struct kp_int { static constexpr int value = V; };
+
 template <int TYPE, bool ID>
 __global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const float *__restrict__ ad8,
                                                    const _Float16 *__restrict__ abs_, float *dst, const float *residual,
@@ -574,7 +576,6 @@ __global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W
     const int lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, lhi = lane >> 5;
     const int wrow0 = (wave & 1) * 32;    // weight rows of this wave inside the tile
-    const int wcol0 = (wave >> 1) * 64;   // activation rows of this wave inside the tile
     const int64_t nsb = K >> 8;
     // split K: group y of gridDim.y walks super-blocks [sb_lo, sb_hi) and writes its sums to its own slice of `dst` (see launch)
     const int64_t sb_per = (nsb + gridDim.y - 1) / gridDim.y;
@@ -587,179 +588,189 @@ __global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W
     // this thread's weight row, the activation rows of its four transfers, and the column whose scales it copies
     const int64_t wr = row0 + (tid >> 2) < N ? row0 + (tid >> 2) : N - 1;
     const uint8_t *wrow = W + wr * L.row_bytes;
-    unsigned aofs[4];
-#pragma unroll
-    for (int it = 0; it < 4; it++) {
-        int r, c;
-        kp_dma_slot<4>(it, r, c);
-        const int64_t col = col0 + r;
-        const int64_t cc = col < B ? col : B - 1;
-        aofs[it] = (unsigned)((int64_t)(ID ? route.act_row[cc] : (int)cc) * K + c * 16);
-    }
-    int srow;
-    {
-        const int64_t col = col0 + (tid >> 1);
-        const int64_t cc = col < B ? col : B - 1;
-        srow = ID ? route.act_row[cc] : (int)cc;
-    }
-
-    f32x16 acc[2];
-#pragma unroll
-    for (int tb = 0; tb < 2; tb++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[tb][r] = 0.0f;
-
-    // per super-block scales of the weights come with the piece (Q4_K header / Q6_K d); those of the activations are fetched
-    // by two threads per column: 16 bytes of the sub-block sums each, the even thread also the scale
-    auto fetch_scales = [&](int64_t sb, float &d8, u32x4 &bs) {
-        d8 = ad8[(int64_t)srow * nsb + sb];
-        if constexpr (Q4) bs = *(const u32x4 *)(abs_ + ((int64_t)srow * nsb + sb) * 16 + 8 * (tid & 1));
-    };
-    auto store_scales = [&](int sbuf, float d8, const u32x4 &bs, const kp_h<TYPE> &H) {
-        sAd[sbuf][tid >> 1] = d8;   // both threads of the column write the same value: an unconditional use keeps the load where it was issued
-        if constexpr (Q4) {
-            *(u32x4 *)(sAs[sbuf] + (tid >> 1) * 16 + 8 * (tid & 1)) = bs;
-            // the four threads of a row share the work (and all use the header, so its load stays where it was issued):
-            // each writes d, dmin (same values) and the mins of sub-blocks 2p, 2p + 1
-            const int r = tid >> 2, p2 = 2 * (tid & 3);
-            sWd[sbuf][r] = half_bits_to_float((unsigned short)(H.hdr[0] & 0xFFFFu));
-            sWn[sbuf][r] = half_bits_to_float((unsigned short)(H.hdr[0] >> 16));
-            int sc, mn0, mn1;
-            q4k_scale_min(H.hdr[1], H.hdr[2], H.hdr[3], p2, sc, mn0);
-            q4k_scale_min(H.hdr[1], H.hdr[2], H.hdr[3], p2 + 1, sc, mn1);
-            typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-            const f16x2 m1 = {(_Float16)(float)mn0, (_Float16)(float)mn1};
-            const f16x2 m64 = {(_Float16)(float)(64 * mn0), (_Float16)(float)(64 * mn1)};
-            *(f16x2 *)(sWm[sbuf] + r * 16 + p2) = m1;
-            *(f16x2 *)(sWm[sbuf] + r * 16 + 8 + p2) = m64;
-        } else {
-            sWd[sbuf][tid >> 2] = half_bits_to_float(H.d);   // the four threads of a row write the same value
+    // A tile whose columns all lie in its first half (the ragged end of a batch; the second tile of an expert that is routed a few more
+    // than 128 slots) runs with 32 x 32 per wave: half the matrix instructions, activation transfers and scaling, the same unpack.  Uniform
+    // for the whole group, so each form keeps a branch-free stage.  8 experts of 14336 x 4096, 1024 slots (about half of the experts with a
+    // second tile of some ten slots): Q4_K 336 -> 318 us; Q5_K 4096 x 4096, 1400 slots 131 -> 126; one-round products 0 .. 1.5 % quicker.
+    auto walk = [&](auto ntb) __attribute__((always_inline)) {
+        constexpr int NTB = decltype(ntb)::value;   // 32-column result tiles per wave
+        const int wcol0 = (wave >> 1) * (32 * NTB); // activation rows of this wave inside the tile
+        unsigned aofs[2 * NTB];
+    #pragma unroll
+        for (int it = 0; it < 2 * NTB; it++) {
+            int r, c;
+            kp_dma_slot<2 * NTB>(it, r, c);
+            const int64_t col = col0 + r;
+            const int64_t cc = col < B ? col : B - 1;
+            aofs[it] = (unsigned)((int64_t)(ID ? route.act_row[cc] : (int)cc) * K + c * 16);
         }
-    };
+        int srow;
+        {
+            const int64_t col = col0 + (tid >> 1);
+            const int64_t cc = col < B ? col : B - 1;
+            srow = ID ? route.act_row[cc] : (int)cc;
+        }
 
-    kp_w<TYPE> R0, R1;   // pieces of the even / odd stages
-    kp_h<TYPE> Hc, Hn;   // super-block data in use / of the next super-block
-    float d8n = 0.0f;
-    u32x4 bsn = {0, 0, 0, 0};
-    // prologue: stage 0 into the "a" buffers, pieces of stage 1 in flight
-    kp_fetch_w<TYPE>(R0, wrow, L, sb_lo, 0);
-    kp_fetch_w<TYPE>(R1, wrow, L, sb_lo, 1);
-    kp_fetch_h<TYPE>(Hc, wrow, L, sb_lo);
-    kp_dma_a<4>(aq + sb_lo * QKK, aofs, sAa);
-    fetch_scales(sb_lo, d8n, bsn);
-    {
-        kp_planes P;
-#pragma unroll
-        for (int i = 0; i < 4; i++) kp_unpack<TYPE>(R0, Hc, 0, i, P);
-        kp_store<TYPE>(P, sW1a, sW0a);
-        store_scales(0, d8n, bsn, Hc);
-    }
-    Hn = Hc;
-    __syncthreads();
+        f32x16 acc[NTB];
+    #pragma unroll
+        for (int tb = 0; tb < NTB; tb++)
+    #pragma unroll
+            for (int r = 0; r < 16; r++) acc[tb][r] = 0.0f;
 
-    for (int64_t sb = sb_lo; sb < sb_hi; sb++) {
-        i32x16 hi[2], lo[2];
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            const int8_t *cA = half == 0 ? sAa : sAb_;
-            const int8_t *cW1 = half == 0 ? sW1a : sW1b;
-            const int8_t *cW0 = half == 0 ? sW0a : sW0b;
-            int8_t *nA = half == 0 ? sAb_ : sAa;
-            int8_t *nW1 = half == 0 ? sW1b : sW1a;
-            int8_t *nW0 = half == 0 ? sW0b : sW0a;
-            kp_w<TYPE> &Rn = half == 0 ? R1 : R0;    // piece of the next stage: unpacked during this one
-            kp_w<TYPE> &Rf = half == 0 ? R0 : R1;    // held this stage's piece (unpacked one stage ago): refilled for the stage after next
-            // Past the end of K the same work is done on the last super-block again and never read: no branches in the stage,
-            // so the compiler schedules it as one block.
-            const int64_t sb1 = sb + 1 < sb_hi ? sb + 1 : sb;
-            kp_dma_a<4>(aq + (half == 0 ? sb * QKK + 128 : sb1 * QKK), aofs, nA);
-            if (half == 1) fetch_scales(sb1, d8n, bsn);
-            kp_fetch_w<TYPE>(Rf, wrow, L, sb1, half);
-            if (half == 0) kp_fetch_h<TYPE>(Hn, wrow, L, sb1);   // used from the next stage on
-            __builtin_amdgcn_sched_barrier(0);   // the loads stay here, a whole stage ahead of their first use
+        // per super-block scales of the weights come with the piece (Q4_K header / Q6_K d); those of the activations are fetched
+        // by two threads per column: 16 bytes of the sub-block sums each, the even thread also the scale
+        auto fetch_scales = [&](int64_t sb, float &d8, u32x4 &bs) {
+            d8 = ad8[(int64_t)srow * nsb + sb];
+            if constexpr (Q4) bs = *(const u32x4 *)(abs_ + ((int64_t)srow * nsb + sb) * 16 + 8 * (tid & 1));
+        };
+        auto store_scales = [&](int sbuf, float d8, const u32x4 &bs, const kp_h<TYPE> &H) {
+            sAd[sbuf][tid >> 1] = d8;   // both threads of the column write the same value: an unconditional use keeps the load where it was issued
+            if constexpr (Q4) {
+                *(u32x4 *)(sAs[sbuf] + (tid >> 1) * 16 + 8 * (tid & 1)) = bs;
+                // the four threads of a row share the work (and all use the header, so its load stays where it was issued):
+                // each writes d, dmin (same values) and the mins of sub-blocks 2p, 2p + 1
+                const int r = tid >> 2, p2 = 2 * (tid & 3);
+                sWd[sbuf][r] = half_bits_to_float((unsigned short)(H.hdr[0] & 0xFFFFu));
+                sWn[sbuf][r] = half_bits_to_float((unsigned short)(H.hdr[0] >> 16));
+                int sc, mn0, mn1;
+                q4k_scale_min(H.hdr[1], H.hdr[2], H.hdr[3], p2, sc, mn0);
+                q4k_scale_min(H.hdr[1], H.hdr[2], H.hdr[3], p2 + 1, sc, mn1);
+                typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+                const f16x2 m1 = {(_Float16)(float)mn0, (_Float16)(float)mn1};
+                const f16x2 m64 = {(_Float16)(float)(64 * mn0), (_Float16)(float)(64 * mn1)};
+                *(f16x2 *)(sWm[sbuf] + r * 16 + p2) = m1;
+                *(f16x2 *)(sWm[sbuf] + r * 16 + 8 + p2) = m64;
+            } else {
+                sWd[sbuf][tid >> 2] = half_bits_to_float(H.d);   // the four threads of a row write the same value
+            }
+        };
 
+        kp_w<TYPE> R0, R1;   // pieces of the even / odd stages
+        kp_h<TYPE> Hc, Hn;   // super-block data in use / of the next super-block
+        float d8n = 0.0f;
+        u32x4 bsn = {0, 0, 0, 0};
+        // prologue: stage 0 into the "a" buffers, pieces of stage 1 in flight
+        kp_fetch_w<TYPE>(R0, wrow, L, sb_lo, 0);
+        kp_fetch_w<TYPE>(R1, wrow, L, sb_lo, 1);
+        kp_fetch_h<TYPE>(Hc, wrow, L, sb_lo);
+        kp_dma_a<2 * NTB>(aq + sb_lo * QKK, aofs, sAa);
+        fetch_scales(sb_lo, d8n, bsn);
+        {
             kp_planes P;
-            i32x4 af[2][2], b1[2], b0[2];
-            auto load_frags = [&](int ks, int slot) {
-#pragma unroll
-                for (int tb = 0; tb < 2; tb++) af[slot][tb] = *(const i32x4 *)(cA + kp_off(wcol0 + tb * 32 + l32, ks * 2 + lhi));
-                b1[slot] = *(const i32x4 *)(cW1 + kp_off(wrow0 + l32, ks * 2 + lhi));
-                b0[slot] = *(const i32x4 *)(cW0 + kp_off(wrow0 + l32, ks * 2 + lhi));
-            };
-            load_frags(0, 0);
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                if (ks < 3) load_frags(ks + 1, (ks + 1) & 1);   // operands of the next step are in flight during this step's matrix instructions
-                const int sl = ks & 1;
-#pragma unroll
-                for (int tb = 0; tb < 2; tb++) {
-                    if (half == 0 && ks == 0) {
-                        i32x16 z;
-#pragma unroll
-                        for (int r = 0; r < 16; r++) z[r] = 0;
-                        hi[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b1[sl], z, 0, 0, 0);
-                        lo[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b0[sl], z, 0, 0, 0);
-                    } else {
-                        hi[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b1[sl], hi[tb], 0, 0, 0);
-                        lo[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b0[sl], lo[tb], 0, 0, 0);
-                    }
-                }
-                kp_unpack<TYPE>(Rn, half == 0 ? Hc : Hn, half ^ 1, ks, P);   // a quarter of the next stage's piece between the matrix instructions
-            }
-            kp_store<TYPE>(P, nW1, nW0);
+    #pragma unroll
+            for (int i = 0; i < 4; i++) kp_unpack<TYPE>(R0, Hc, 0, i, P);
+            kp_store<TYPE>(P, sW1a, sW0a);
+            store_scales(0, d8n, bsn, Hc);
+        }
+        Hn = Hc;
+        __syncthreads();
 
-            if (half == 1) {   // end of the super-block: scale the integer sums into the f32 accumulators
-                const int sbuf = (int)((sb - sb_lo) & 1);
-#pragma unroll
-                for (int tb = 0; tb < 2; tb++) {
-                    f32x4 d8[4];
-#pragma unroll
-                    for (int q = 0; q < 4; q++) d8[q] = *(const f32x4 *)(sAd[sbuf] + wcol0 + tb * 32 + 8 * q + 4 * lhi);
-                    const int wr_ = wrow0 + l32;
-                    const float dw = sWd[sbuf][wr_];
-                    if constexpr (Q4) {
-                        const float dn = sWn[sbuf][wr_];
-                        const f16x8 am = *(const f16x8 *)(sAs[sbuf] + (wcol0 + tb * 32 + l32) * 16 + 8 * lhi);
-                        const f16x8 bm = *(const f16x8 *)(sWm[sbuf] + wr_ * 16 + 8 * lhi);
-                        f32x16 z;
-#pragma unroll
-                        for (int r = 0; r < 16; r++) z[r] = 0.0f;
-                        const f32x16 M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, z, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const int t = (hi[tb][r] << RADIX_SHIFT) + lo[tb][r];
-                            acc[tb][r] += d8[r >> 2][r & 3] * (dw * (float)t - dn * M[r]);
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const int t = (hi[tb][r] << RADIX_SHIFT) + lo[tb][r];
-                            acc[tb][r] += d8[r >> 2][r & 3] * (dw * (float)t);
+        for (int64_t sb = sb_lo; sb < sb_hi; sb++) {
+            i32x16 hi[NTB], lo[NTB];
+    #pragma unroll
+            for (int half = 0; half < 2; half++) {
+                const int8_t *cA = half == 0 ? sAa : sAb_;
+                const int8_t *cW1 = half == 0 ? sW1a : sW1b;
+                const int8_t *cW0 = half == 0 ? sW0a : sW0b;
+                int8_t *nA = half == 0 ? sAb_ : sAa;
+                int8_t *nW1 = half == 0 ? sW1b : sW1a;
+                int8_t *nW0 = half == 0 ? sW0b : sW0a;
+                kp_w<TYPE> &Rn = half == 0 ? R1 : R0;    // piece of the next stage: unpacked during this one
+                kp_w<TYPE> &Rf = half == 0 ? R0 : R1;    // held this stage's piece (unpacked one stage ago): refilled for the stage after next
+                // Past the end of K the same work is done on the last super-block again and never read: no branches in the stage,
+                // so the compiler schedules it as one block.
+                const int64_t sb1 = sb + 1 < sb_hi ? sb + 1 : sb;
+                kp_dma_a<2 * NTB>(aq + (half == 0 ? sb * QKK + 128 : sb1 * QKK), aofs, nA);
+                if (half == 1) fetch_scales(sb1, d8n, bsn);
+                kp_fetch_w<TYPE>(Rf, wrow, L, sb1, half);
+                if (half == 0) kp_fetch_h<TYPE>(Hn, wrow, L, sb1);   // used from the next stage on
+                __builtin_amdgcn_sched_barrier(0);   // the loads stay here, a whole stage ahead of their first use
+
+                kp_planes P;
+                i32x4 af[2][NTB], b1[2], b0[2];
+                auto load_frags = [&](int ks, int slot) {
+    #pragma unroll
+                    for (int tb = 0; tb < NTB; tb++) af[slot][tb] = *(const i32x4 *)(cA + kp_off(wcol0 + tb * 32 + l32, ks * 2 + lhi));
+                    b1[slot] = *(const i32x4 *)(cW1 + kp_off(wrow0 + l32, ks * 2 + lhi));
+                    b0[slot] = *(const i32x4 *)(cW0 + kp_off(wrow0 + l32, ks * 2 + lhi));
+                };
+                load_frags(0, 0);
+    #pragma unroll
+                for (int ks = 0; ks < 4; ks++) {
+                    if (ks < 3) load_frags(ks + 1, (ks + 1) & 1);   // operands of the next step are in flight during this step's matrix instructions
+                    const int sl = ks & 1;
+    #pragma unroll
+                    for (int tb = 0; tb < NTB; tb++) {
+                        if (half == 0 && ks == 0) {
+                            i32x16 z;
+    #pragma unroll
+                            for (int r = 0; r < 16; r++) z[r] = 0;
+                            hi[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b1[sl], z, 0, 0, 0);
+                            lo[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b0[sl], z, 0, 0, 0);
+                        } else {
+                            hi[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b1[sl], hi[tb], 0, 0, 0);
+                            lo[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b0[sl], lo[tb], 0, 0, 0);
                         }
                     }
+                    kp_unpack<TYPE>(Rn, half == 0 ? Hc : Hn, half ^ 1, ks, P);   // a quarter of the next stage's piece between the matrix instructions
+                }
+                kp_store<TYPE>(P, nW1, nW0);
+
+                if (half == 1) {   // end of the super-block: scale the integer sums into the f32 accumulators
+                    const int sbuf = (int)((sb - sb_lo) & 1);
+    #pragma unroll
+                    for (int tb = 0; tb < NTB; tb++) {
+                        f32x4 d8[4];
+    #pragma unroll
+                        for (int q = 0; q < 4; q++) d8[q] = *(const f32x4 *)(sAd[sbuf] + wcol0 + tb * 32 + 8 * q + 4 * lhi);
+                        const int wr_ = wrow0 + l32;
+                        const float dw = sWd[sbuf][wr_];
+                        if constexpr (Q4) {
+                            const float dn = sWn[sbuf][wr_];
+                            const f16x8 am = *(const f16x8 *)(sAs[sbuf] + (wcol0 + tb * 32 + l32) * 16 + 8 * lhi);
+                            const f16x8 bm = *(const f16x8 *)(sWm[sbuf] + wr_ * 16 + 8 * lhi);
+                            f32x16 z;
+    #pragma unroll
+                            for (int r = 0; r < 16; r++) z[r] = 0.0f;
+                            const f32x16 M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, z, 0, 0, 0);
+    #pragma unroll
+                            for (int r = 0; r < 16; r++) {
+                                const int t = (hi[tb][r] << RADIX_SHIFT) + lo[tb][r];
+                                acc[tb][r] += d8[r >> 2][r & 3] * (dw * (float)t - dn * M[r]);
+                            }
+                        } else {
+    #pragma unroll
+                            for (int r = 0; r < 16; r++) {
+                                const int t = (hi[tb][r] << RADIX_SHIFT) + lo[tb][r];
+                                acc[tb][r] += d8[r >> 2][r & 3] * (dw * (float)t);
+                            }
+                        }
+                    }
+                }
+                if (half == 1) {   // last, so that the loads had the whole stage (the barrier keeps the scheduler from hoisting the wait)
+                    __builtin_amdgcn_sched_barrier(0);
+                    store_scales((int)((sb - sb_lo + 1) & 1), d8n, bsn, Hn);
+                    Hc = Hn;
+                }
+                __syncthreads();   // also waits for this stage's transfers and loads (issued a whole stage ago)
+            }
+        }
+
+    #pragma unroll
+        for (int tb = 0; tb < NTB; tb++) {
+            const int64_t n = row0 + wrow0 + l32;
+    #pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int64_t b = col0 + wcol0 + tb * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
+                if (n < N && b < B) {
+                    const int64_t o = (ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n;
+                    dst[o] = residual ? acc[tb][r] + residual[o] : acc[tb][r];   // residual may be dst itself: one reader and writer per element
                 }
             }
-            if (half == 1) {   // last, so that the loads had the whole stage (the barrier keeps the scheduler from hoisting the wait)
-                __builtin_amdgcn_sched_barrier(0);
-                store_scales((int)((sb - sb_lo + 1) & 1), d8n, bsn, Hn);
-                Hc = Hn;
-            }
-            __syncthreads();   // also waits for this stage's transfers and loads (issued a whole stage ago)
         }
-    }
-
-#pragma unroll
-    for (int tb = 0; tb < 2; tb++) {
-        const int64_t n = row0 + wrow0 + l32;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int64_t b = col0 + wcol0 + tb * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-            if (n < N && b < B) {
-                const int64_t o = (ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n;
-                dst[o] = residual ? acc[tb][r] + residual[o] : acc[tb][r];   // residual may be dst itself: one reader and writer per element
-            }
-        }
-    }
+    };
+    if (B - col0 > BN / 2) walk(kp_int<2>{});
+    else walk(kp_int<1>{});
 }
 
 // ---- planes kept in HBM ----------------------------------------------------------------------------------------------------

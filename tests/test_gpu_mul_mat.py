@@ -370,6 +370,26 @@ def test_ragged_rows(dev, name, t, blocks):
             assert orc.nmse(got, want) < 1e-11, (B, split)
 
 
+@pytest.mark.parametrize("name,t", TYPES)
+@pytest.mark.parametrize("K", [1280, 2048])
+def test_ragged_last_column_tile(dev, name, t, K):
+    """batches whose last 128-column tile holds 1, 64, 65 and 128 columns (up to 64 it runs with half the columns per wave): every column
+    against the same arithmetic on the CPU; integer sums are exact, f32 sums over at most 64 blocks leave an NMSE of some 1e-14"""
+    import mi355
+    rng = np.random.default_rng(K)
+    N = 130
+    Wq = _weights(rng, t, N, K)
+    Wd = mi355.upload_weights(t, _to_dev(dev, Wq))
+    x = rng.standard_normal((384, K)).astype(np.float32)
+    for B in (129, 192, 193, 256, 257, 320, 321):
+        aligned = K % 2048 == 0 or t in (orc.Q4_K, orc.Q5_K)
+        q8k = (t in (orc.Q4_K, orc.Q5_K, orc.Q6_K) or (t == orc.IQ4_XS and B >= 256)) and aligned
+        want = orc.mul_mat("cpu" if q8k else "q8_1", t, Wq, x[:B])
+        for split in (False, True):
+            got = mi355.mul_mat(t, Wd, _to_dev(dev, x[:B]), split=split).cpu().numpy()
+            assert orc.nmse(got, want) < 1e-11, (B, split)
+
+
 KQ_TYPES = [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q6_K)]
 TILED_TYPES = [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q5_K, orc.Q6_K, orc.IQ4_XS)]   # types with tile images for the wide-tile GEMM
 

@@ -85,6 +85,24 @@ def test_mul_mat_id_skewed_routing(dev, name, t, pattern):
     assert orc.nmse(got, want) < (1e-6 if t in (orc.Q4_1, orc.Q5_1) else 1e-9)   # the block minimum meets fp16(d_x * sum(q)) in the tile kernel
 
 
+@pytest.mark.parametrize("name,t", list(orc.WEIGHT_TYPES.items()))
+@pytest.mark.parametrize("K", [1280, 2048])
+def test_mul_mat_id_last_column_tiles(dev, name, t, K):
+    """experts whose second 128-column tile holds 1, 64 and 65 slots (up to 64 it runs with half the columns per wave)"""
+    import torch
+    import mi355
+    counts, N = (129, 192, 193, 64), 70
+    T = sum(counts)
+    rng = np.random.default_rng(K)
+    Wq = orc.quantize("oracle", t, (rng.standard_normal((len(counts) * N, K)) * 0.02).astype(np.float32))
+    b = rng.standard_normal((T, 1, K)).astype(np.float32)
+    ids = rng.permutation(np.repeat(np.arange(len(counts)), counts)).astype(np.int32).reshape(T, 1)
+    Wd = mi355.upload_weights(t, torch.from_numpy(Wq).to(dev)).reshape(len(counts), N, -1)
+    got = mi355.mul_mat_id(t, Wd, torch.from_numpy(b).to(dev), torch.from_numpy(ids).to(dev), 1).cpu().numpy()
+    want = expected_per_expert("cpu" if routed(t, 1, T, K) else "q8_1", t, Wq, b, ids, len(counts), 1, 1, N)
+    assert orc.nmse(got, want) < 1e-11   # exact integer sums, f32 sums over at most 64 blocks
+
+
 @pytest.mark.parametrize("name,t", [("q4_k", orc.Q4_K), ("q5_k", orc.Q5_K), ("q6_k", orc.Q6_K)])
 @pytest.mark.parametrize("n_expert,n_used,nb1_bcast,T,N,K", [(8, 2, True, 512, 192, 2048), (8, 2, False, 300, 64, 4096), (4, 4, True, 70, 256, 2048),
                                                               (8, 1, False, 3, 130, 2048)])   # Q6_K rows are 16-byte aligned from K = 2048 on
