@@ -148,6 +148,26 @@ __device__ __forceinline__ void fs_output(unsigned v_addr, unsigned p_rd, fs_sta
     }
 }
 
+// The same for one half of the elements (H = 0: lane, 1: 64 + lane), same sums
+template <int H> __device__ __forceinline__ void fs_output_half(unsigned v_addr, unsigned p_rd, f32x4 &o) {
+    constexpr int NJ = 16;
+    u32x2 v[NJ], pa[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const unsigned addr = v_addr + (unsigned)(j * 4 * FS_ROW);
+        asm volatile("ds_read_b64 %0, %1" : "=v"(pa[j]) : "v"(p_rd + (unsigned)(j * 8)));
+        if constexpr (H == 0) asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v[j]) : "v"(addr));
+        else asm volatile("ds_read_b64_tr_b16 %0, %1 offset:128" : "=v"(v[j]) : "v"(addr));
+    }
+#pragma unroll
+    for (int jb = 0; jb < NJ; jb += 8)
+        asm volatile("s_waitcnt lgkmcnt(0)"
+                     : "+v"(v[jb]), "+v"(v[jb + 1]), "+v"(v[jb + 2]), "+v"(v[jb + 3]), "+v"(v[jb + 4]), "+v"(v[jb + 5]), "+v"(v[jb + 6]), "+v"(v[jb + 7]),
+                       "+v"(pa[jb]), "+v"(pa[jb + 1]), "+v"(pa[jb + 2]), "+v"(pa[jb + 3]), "+v"(pa[jb + 4]), "+v"(pa[jb + 5]), "+v"(pa[jb + 6]), "+v"(pa[jb + 7]));
+#pragma unroll
+    for (int j = 0; j < NJ; j++) o = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pa[j]), __builtin_bit_cast(f16x4, v[j]), o, 0, 0, 0);
+}
+
 __global__ void __launch_bounds__(FS_WAVES * 64, 1) k_fattn_dec_stream(fattn_args a, int tiles_per_wave, int n_tiles, int R) {
     __shared__ __attribute__((aligned(1024))) uint8_t ring_buf[FS_WAVES * 2 * FS_STAGE];
     __shared__ __attribute__((aligned(16))) unsigned short pbuf[FS_WAVES][4][FS_TILE];
@@ -681,36 +701,47 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
 }
 
 // ---- short caches: at most 512 cells, one launch -------------------------------------------------------------------------------
-// One group per kv head, one wave per 64-cell tile (up to eight).  Nothing here is bound by bytes: the time is one trip to memory
+// Two groups per kv head, one for each half of the output elements, one wave per 64-cell tile (up to eight).  Nothing here is bound by bytes: the time is one trip to memory
 // plus the arithmetic of one tile, so a wave requests everything at once - its K and V tiles as coalesced 16-byte loads into
 // registers (four whole rows per instruction), q, its mask value - and then passes first K, then V through its own 16 KiB of
 // LDS to bring them into operand form: K rows with their chunks XOR-ed across the banks, so that each lane reads back the row of
 // its cell; V row-major for the transposing reads.  (A lane loading its own K row directly would touch 64 cache lines per
 // instruction: measured 2.8 us per wave of the group.)  The waves' states meet in LDS; the group normalises and writes the output
 // (and its Q8_1 form where the next product wants it), so no second launch merges anything.
+// Both groups of a kv head form the same scores; a group then reads only its half of every V row.  In a model the cache comes from HBM and a
+// compute unit's own requests are what takes the time: 512 cells are 256 KiB for one group per kv head (12.0 us per layer, 8B model),
+// 192 KiB for one of two (10.4 us; K reaches the second one through L2), with the same bits.
 constexpr int FSS_MAX_WAVES = 8;
 
 __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn_args a, int R) {
     __shared__ __attribute__((aligned(1024))) uint8_t tbuf[FSS_MAX_WAVES * FS_KT];
     __shared__ __attribute__((aligned(16))) unsigned short pbuf[FSS_MAX_WAVES][4][FS_TILE];
     __shared__ float s_m[FSS_MAX_WAVES][4], s_l[FSS_MAX_WAVES][4];
-    __shared__ float s_o[FSS_MAX_WAVES][4][FS_D];
+    __shared__ float s_o[FSS_MAX_WAVES][4][FS_D / 2];
     __shared__ __attribute__((aligned(16))) unsigned short qbuf[FSS_MAX_WAVES][4][FS_D];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int n_waves = (int)(blockDim.x >> 6);
     const int64_t hk = blockIdx.x;
+    const int part = (int)blockIdx.y;   // elements 64 part .. + 63 of the output
     const int64_t c0 = (int64_t)wave * FS_TILE;
     const int rsub = lane >> 4, pos = lane & 15;
 
     // load i: rows 4i .. 4i + 3, lane -> row 4i + lane / 16, chunk lane % 16 (rows past the end repeat the last cell; their weights are zero)
-    u32x4 kraw[16], vraw[16];
+    // (half rows of V: rows 8i .. 8i + 7, lane -> row 8i + lane / 8, chunk lane % 8 of the half)
+    const int vsub = lane >> 3, vpos = (lane & 7) + 8 * part;
+    u32x4 kraw[16], vraw[8];
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         int64_t cell = c0 + 4 * i + rsub;
         if (cell >= a.Nkv) cell = a.Nkv - 1;
         kraw[i] = load16(a.k + cell * a.k_nb1 + hk * a.k_nb2 + (pos << 4));
-        vraw[i] = load16(a.v + cell * a.v_nb1 + hk * a.v_nb2 + (pos << 4));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        int64_t cell = c0 + 8 * i + vsub;
+        if (cell >= a.Nkv) cell = a.Nkv - 1;
+        vraw[i] = load16(a.v + cell * a.v_nb1 + hk * a.v_nb2 + (vpos << 4));
     }
     const int64_t cell = c0 + lane;
     unsigned short mbits = 0xFC00;   // -inf
@@ -763,9 +794,11 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
 
     // V through the same bytes, row-major (the K rows are in registers)
 #pragma unroll
-    for (int i = 0; i < 16; i++) *(u32x4 *)(tb + (4 * i + rsub) * FS_ROW + (pos << 4)) = vraw[i];
+    for (int i = 0; i < 8; i++) *(u32x4 *)(tb + (8 * i + vsub) * FS_ROW + (vpos << 4)) = vraw[i];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // fs_output reads LDS through inline assembly: nothing may be moved across
-    fs_output((unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)tb + fs_v_lane(lane), p_base + (unsigned)(lane & 3) * (FS_TILE * 2), S);
+    const unsigned v_addr = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)tb + fs_v_lane(lane), p_rd = p_base + (unsigned)(lane & 3) * (FS_TILE * 2);
+    if (part == 0) fs_output_half<0>(v_addr, p_rd, S.o0);   // uniform
+    else fs_output_half<1>(v_addr, p_rd, S.o0);
 
     // ---- the waves' states meet in LDS
 #pragma unroll
@@ -776,11 +809,10 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
             s_l[wave][r] = L;
         }
         s_o[wave][r][lane] = S.o0[r];
-        s_o[wave][r][64 + lane] = S.o1[r];
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < R * FS_D; idx += (int)blockDim.x) {   // whole waves: R * 128 and the group size are multiples of 64
-        const int r = idx / FS_D, d = idx % FS_D;
+    for (int idx = threadIdx.x; idx < R * (FS_D / 2); idx += (int)blockDim.x) {   // whole waves: R * 64 and the group size are multiples of 64
+        const int r = idx / (FS_D / 2), d = idx % (FS_D / 2);
         float M = s_m[0][r];
         for (int w = 1; w < n_waves; w++) M = fmaxf(M, s_m[w][r]);
         float L = 0.0f, O = 0.0f;
@@ -791,8 +823,9 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
         }
         const int64_t head = hk * R + r;
         const float o = O / L;
-        a.dst[head * FS_D + d] = o;
-        if (a.act_q) quantize_lane32(o, a.act_q, a.act_s, head * FS_D + d);
+        const int64_t at = head * FS_D + 64 * part + d;
+        a.dst[at] = o;
+        if (a.act_q) quantize_lane32(o, a.act_q, a.act_s, at);
     }
 }
 
@@ -801,7 +834,7 @@ int launch_fattn_dec_short(hipStream_t s, fattn_args &a, int64_t D) {
     if (D != FS_D || a.Nq != 1 || R > 4 || a.Hkv > 65535 || a.Nkv > FSS_MAX_WAVES * FS_TILE) return 1;
     if ((a.q_nb2 % 16) != 0 || (a.k_nb1 % 16) != 0 || (a.k_nb2 % 16) != 0 || (a.v_nb1 % 16) != 0 || (a.v_nb2 % 16) != 0) return 1;
     const int n_waves = (int)((a.Nkv + FS_TILE - 1) / FS_TILE);
-    MI355_LAUNCH(k_fattn_dec_short, dim3((unsigned)a.Hkv), dim3((unsigned)n_waves * 64), 0, s, a, (int)R);
+    MI355_LAUNCH(k_fattn_dec_short, dim3((unsigned)a.Hkv, 2), dim3((unsigned)n_waves * 64), 0, s, a, (int)R);
     return launch_status("k_fattn_dec_short");
 }
 
