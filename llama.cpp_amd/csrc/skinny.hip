@@ -26,7 +26,7 @@ namespace mi355 {
 namespace {
 
 // What goes through LDS per step (256 elements) and weight row: the 4-bit (Q8_0: 8-bit) plane of the levels - 128 bytes of
-// nibbles for every type but Q8_0; Q6_K copies its 64 bytes of high bit pairs beside them.  Everything a lane needs of ITS row
+// nibbles for every type but Q8_0 (256, in one or two halves); Q6_K copies its 64 bytes of high bit pairs beside them.  Everything a lane needs of ITS row
 // only (block scales and minima, the K-quants' 16-byte header, the fifth bits of Q5_0 / Q5_1 / Q5_K) goes straight to registers.
 template <int TYPE> struct sk_traits {
     static constexpr int ROW_BYTES = TYPE == MI355_Q8_0 ? 256 : 128;
@@ -62,9 +62,16 @@ __device__ __forceinline__ float f16_of(const u32x4 &v, int j) {   // j is a com
     return half_bits_to_float((unsigned short)((j & 1) ? (u >> 16) : (u & 0xFFFFu)));
 }
 
+// Q8_0 with nine and more activation rows, and its experts: the 256 bytes of a step go through the same 128 bytes of LDS per row, four
+// blocks at a time.  With all of them in LDS a group of 16-row form takes 55 KiB, two groups per compute unit.  28672 x 8192, 16 / 32 rows
+// 62.7 / 79.4 -> 62.2 / 76.6 us, 4096 x 14336, 24 rows 23.6 -> 22.4, 8 experts of 14336 x 4096, 32 slots 95.5 -> 91.4; up to eight rows the
+// whole step is quicker (28672 x 8192, 8 rows 55.1 against 56.0; 32768 x 2080, 6 rows 21.3 against 23.8).
+constexpr int sk_halves(int type, int ni, bool tail, bool id) { return type == MI355_Q8_0 && !tail && (ni > 1 || id) ? 2 : 1; }
+
 // registers of one step in flight
-template <int TYPE, int NI> struct sk_regs {
+template <int TYPE, int NI, int HALVES> struct sk_regs {
     static constexpr int NW = 32 * sk_traits<TYPE>::ROW_BYTES / 1024;   // 16-byte loads per lane for the weights
+    static constexpr int NWH = NW / HALVES;                             // ... for those that are in LDS together
     static constexpr int NA = 2 * NI;                                   // ... for 8 NI activation rows of 256 bytes
     static constexpr int NT = (NI + 1) / 2;                             // ... for their 8 {d, sum} pairs each
     u32x4 w[NW], a[NA], t[NT], hdr;
@@ -102,8 +109,10 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
                                                    float *__restrict__ dst, const float *__restrict__ residual, int64_t N, int K, int B,
                                                    int64_t dst_stride, int steps_per_slice, int steps_per_wave, sk_id id, sk_q8k q8) {
     typedef sk_traits<TYPE> T;
-    typedef sk_regs<TYPE, NI> R;
-    constexpr int WPAD = T::ROW_BYTES + 16;
+    constexpr int HALVES = sk_halves(TYPE, NI, TAIL, ID);
+    typedef sk_regs<TYPE, NI, HALVES> R;
+    constexpr int LDS_ROW = T::ROW_BYTES / HALVES;   // bytes of a weight row in LDS
+    constexpr int WPAD = LDS_ROW + 16;
     constexpr int QHPAD = 64 + 16;
     constexpr bool Q6 = TYPE == MI355_Q6_K;
     constexpr int W_BYTES = 32 * WPAD + (Q6 ? 32 * QHPAD : 0), A_BYTES = 8 * NI * SK_APAD, T_BYTES = 8 * 8 * NI * 8;
@@ -150,11 +159,11 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     const int s_hi = s_lo + steps_per_wave < slice_hi ? s_lo + steps_per_wave : slice_hi;   // may be <= s_lo: a wave without steps
 
     // copy assignments: weights: a lane reads 16 bytes along a row, LPR lanes per row; activation rows: 16 lanes per row
-    constexpr int LPR = T::ROW_BYTES / 16, RPL = 64 / LPR;   // lanes per row, rows per load
+    constexpr int LPR = LDS_ROW / 16, RPL = 64 / LPR;   // lanes per row, rows per load
     const int w_piece = lane % LPR, w_row = lane / LPR;
-    const uint8_t *w_src[R::NW];
+    const uint8_t *w_src[R::NWH];
 #pragma unroll
-    for (int u = 0; u < R::NW; u++) {
+    for (int u = 0; u < R::NWH; u++) {
         int64_t row = row0 + w_row + u * RPL;
         row = row < N ? row : N - 1;   // clamp: rows past the end repeat the last row and are not stored
         w_src[u] = W + row * L.row_bytes + 16 * w_piece + T::QS_OFF;
@@ -187,13 +196,19 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     // Q8K: lane c < 8 NI brings the scale and the block sums of column c
     const int64_t q8_row = Q8K ? act_row(lane < 8 * NI ? lane : 0) * (K >> 8) : 0;
 
+    // the weights of one half of a step (HALVES == 2)
+    auto fetch_half = [&](int step, R &g, int half) {
+        const int s = step < nsteps ? step : nsteps - 1;
+#pragma unroll
+        for (int u = 0; u < R::NWH; u++) g.w[half * R::NWH + u] = load16w(w_src[u] + s * T::STEP_BYTES + half * LDS_ROW);
+    };
     // The last step of a row whose K is no multiple of 256: blocks past the end repeat the last one (nothing is read behind the row) and
     // get scale and minimum 0; the activation bytes they meet are those of the last block too, hence finite.
     auto fetch_tail = [&](int s, R &g) {
         constexpr int BLOCK_Q = T::ROW_BYTES / 8;   // level bytes per block
         const int last = nblk - 1;
 #pragma unroll
-        for (int u = 0; u < R::NW; u++) {
+        for (int u = 0; u < R::NWH; u++) {
             const int blk = s * 8 + 16 * w_piece / BLOCK_Q;
             g.w[u] = load16w(w_src[u] + s * T::STEP_BYTES - (blk > last ? (blk - last) * BLOCK_Q : 0));
         }
@@ -227,7 +242,7 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
             g.t[u] = u32x4{e0.x, e0.y, e1.x, e1.y};
         }
     };
-    // loads of one step into the register set `g`
+    // loads of one step into the register set `g` (HALVES == 2: without the weights, fetch_half)
     auto fetch = [&](int step, R &g) {
         const int s = step < nsteps ? step : nsteps - 1;
         if constexpr (TAIL) {
@@ -237,8 +252,10 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
             }
         }
         const int w_off = s * T::STEP_BYTES;   // < 2^31: rows are shorter than that
+        if constexpr (HALVES == 1) {
 #pragma unroll
-        for (int u = 0; u < R::NW; u++) g.w[u] = load16w(w_src[u] + w_off);
+            for (int u = 0; u < R::NW; u++) g.w[u] = load16w(w_src[u] + w_off);
+        }
         if constexpr (T::KQ) {
             g.hdr = load16w(w_mine + w_off);
             if constexpr (TYPE == MI355_Q5_K) g.qh[0] = load16w(w_mine + w_off + 16 + 16 * kh);
@@ -287,11 +304,13 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     // One set of load registers: as soon as a step's loads have been copied to LDS, the same registers take the next step's
     // loads, which are then in flight while this step is contracted.  Only the weight scales of the lane's row stay behind.
     R cur = {};
+    if constexpr (HALVES == 2) fetch_half(s_lo, cur, 0);
     fetch(s_lo, cur);
+    if constexpr (HALVES == 2) fetch_half(s_lo, cur, 1);
     for (int step = s_lo; step < s_hi; step++) {
         // ---- registers -> the wave's LDS
 #pragma unroll
-        for (int u = 0; u < R::NW; u++) *(u32x4 *)(s_w + (w_row + u * RPL) * WPAD + 16 * w_piece) = cur.w[u];
+        for (int u = 0; u < R::NWH; u++) *(u32x4 *)(s_w + (w_row + u * RPL) * WPAD + 16 * w_piece) = cur.w[u];
         if constexpr (Q6) {
 #pragma unroll
             for (int u = 0; u < 2; u++) *(u32x4 *)(s_qh + ((lane >> 2) + 16 * u) * QHPAD + 16 * (lane & 3)) = cur.qh[u];
@@ -334,7 +353,10 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
         const u32x4 fifth[2] = {cur.qh[0], cur.qh[1]};   // (Q6_K's went to LDS above)
         const u32 d6 = cur.d6;
         wave_lds_sync();
-        if (step + 1 < s_hi) fetch(step + 1, cur);
+        if (step + 1 < s_hi) {
+            if constexpr (HALVES == 2) fetch_half(step + 1, cur, 0);
+            fetch(step + 1, cur);
+        }
 
         const int am = r < 8 * NI ? r : r & 7;   // operand rows past the copied ones repeat copied ones; their results are not used
         if constexpr (Q8K) {
@@ -508,10 +530,24 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
             }
     #pragma unroll
             for (int j = 0; j < 8; j++) {
+                if constexpr (HALVES == 2) {
+                    if (j == 4) {   // the second half takes the first one's place
+                        // the first half's sums are formed here, not behind the branch below: sixteen registers per block less
+#pragma unroll
+                        for (int q = 0; q < NI; q++)
+#pragma unroll
+                            for (int i = 0; i < 4; i++) asm volatile("" : "+v"(acc[q][i]));
+                        wave_lds_sync();
+#pragma unroll
+                        for (int u = 0; u < R::NWH; u++) *(u32x4 *)(s_w + (w_row + u * RPL) * WPAD + 16 * w_piece) = cur.w[R::NWH + u];
+                        wave_lds_sync();
+                        if (step + 1 < s_hi) fetch_half(step + 1, cur, 1);
+                    }
+                }
                 // operand B: levels 16 kh .. + 16 of block j of weight row r
                 i32x4 wop;
                 if constexpr (TYPE == MI355_Q8_0) {
-                    wop = *(const i32x4 *)(s_w + r * WPAD + 32 * j + 16 * kh);
+                    wop = *(const i32x4 *)(s_w + r * WPAD + 32 * (HALVES == 2 ? j & 3 : j) + 16 * kh);
                 } else if constexpr (T::NIB32) {   // byte b of the block's 16: level b in the low nibble, level 16 + b in the high one
                     const u32x4 v = *(const u32x4 *)(s_w + r * WPAD + 16 * j);
                     const u32 fw = j < 4 ? fifth[0][j & 3] : fifth[1][j & 3];   // Q5_0 / Q5_1: bit e = fifth bit of element e
