@@ -494,8 +494,8 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
     const int R = (int)(a.Hq / a.Hkv);
     const int pairs = PQ ? R : R / 2;   // heads or head pairs per kv head
     const grid_pos gp = xcd_grid_pos();
-    const int64_t hk = gp.y / pairs;
-    const int64_t head = PQ ? gp.y : 2 * (int64_t)gp.y + hp;
+    const int64_t hk = gp.y / pairs, hg = gp.y % pairs;
+    const int64_t head = PQ ? hk * pairs + hg : (hk * pairs + hg) * 2 + hp;
     const int64_t q0 = PQ ? ((int64_t)gp.x * 2 + hp) * 32 : (int64_t)gp.x * 32;
     const int64_t iq = q0 + l32 < a.Nq ? q0 + l32 : a.Nq - 1;   // clamped: rows past Nq are computed and dropped
 
