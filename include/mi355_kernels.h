@@ -106,6 +106,8 @@ int mi355_quantize_act(void *stream, const float *x, void *act, int64_t k, int64
  * runs it on mi355_mul_mat_q8k, and it has tile images for mi355_mul_mat_q8k_tiled.
  * `ws` is scratch of at least mi355_mul_mat_ws_bytes(K, B) bytes. */
 size_t mi355_mul_mat_ws_bytes(int64_t K, int64_t B);
+/* ... with the room that lets a product with few tiles run as slices along K, whatever the weight type. */
+size_t mi355_mul_mat_split_ws_bytes(int64_t N, int64_t K, int64_t B);
 int mi355_mul_mat(void *stream, int type, const void *W, const float *x, float *dst, int64_t N, int64_t K, int64_t B,
                   int64_t x_stride, int64_t dst_stride, void *ws, size_t ws_bytes);
 

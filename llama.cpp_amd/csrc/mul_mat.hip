@@ -83,6 +83,12 @@ size_t mi355_mul_mat_ws_bytes(int64_t K, int64_t B) {
     return (n + 255) & ~(size_t)255;
 }
 
+size_t mi355_mul_mat_split_ws_bytes(int64_t N, int64_t K, int64_t B) {
+    size_t n = mi355_mul_mat_q_ws_bytes(N, K, B);
+    for (const size_t s : {mi355_mul_mat_q8k_ws_bytes(N, K, B), mi355_mul_mat_skinny_ws_bytes(N, K, B), mi355_mul_mat_mid_ws_bytes(N, K, B)}) n = s > n ? s : n;
+    return mi355_mul_mat_ws_bytes(K, B) + n;
+}
+
 // 4 or 5 (Q6_K) to 32 activation rows: the weight-streaming matrix-core kernel (skinny.hip) where it supports the product.
 static bool use_skinny(int type, const void *W, int64_t K, int64_t B) {
     return B >= (type == MI355_Q6_K ? 5 : 4) && B <= 32 && mi355_mul_mat_skinny_supported(type, W, K, B);
