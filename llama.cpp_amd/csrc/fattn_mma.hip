@@ -140,7 +140,29 @@ __device__ __forceinline__ float half_pair_sum(float x) {
 // most, far inside the f16 range of the matrix operand.
 constexpr float FM_LAZY = 8.0f;
 constexpr float FM_LOG2E = 1.4426950408889634f;
-__device__ __forceinline__ float lazy_max(float m, float mx) { return mx > m + FM_LAZY ? mx : m; }
+//
+// PX: probabilities of f32 precision, for the calls whose other form (the vector kernel) multiplies f32 probabilities: the matrix operand
+// is f16, so a probability goes in as 2^10 p = hi + lo, two f16 values, and every V fragment meets two matrix instructions.  The factor
+// (exact, taken back at the end) keeps lo of a small probability from being subnormal: with probabilities of at most e^4 (2^10 e^4 < 65504)
+// the pair is within 2^-22 p or 2^-35 of one at the reference point.  Error against 64-bit arithmetic and time: see launch_fattn_mma.
+constexpr float FM_PX_SCALE = 1024.0f;
+template <int D> constexpr int fm_px_chains() { return D == 64 || D == 128 ? 4 : 2; }   // partial sums of a score (one chain: D 128, 512 x 512 cells 1.48e-7, four 1.26e-7; vector kernel 1.28e-7)
+template <bool PX> __device__ __forceinline__ float lazy_max(float m, float mx) { return mx > m + (PX ? 4.0f : FM_LAZY) ? mx : m; }
+// the reference point as a power of two.  PX: rounded once and used as it is wherever exponents are compared, so that old and new terms of a sum agree
+template <bool PX> __device__ __forceinline__ float exponent_of(float m) { return PX ? mul_rn(m, FM_LOG2E) : m * FM_LOG2E; }
+// what a state with reference point m is multiplied with when the point moves to m_new
+template <bool PX> __device__ __forceinline__ float rescale(float m, float m_new) {
+    return PX ? __builtin_amdgcn_exp2f(sub_rn(exponent_of<true>(m), exponent_of<true>(m_new))) : __builtin_amdgcn_exp2f((m - m_new) * FM_LOG2E);
+}
+// ... and when two finished states are joined
+template <bool PX> __device__ __forceinline__ float merge_factor(float m, float M) { return PX ? rescale<true>(m, M) : __expf(m - M); }
+// O / sum with inv = reciprocal of the sum.  PX: rounded once (one correction step); a row without a visible cell is 0 / 0, as in the vector kernel
+template <bool PX> __device__ __forceinline__ float sum_of(float l) { return PX ? l * FM_PX_SCALE : l; }
+template <bool PX> __device__ __forceinline__ float reciprocal_of(float l) { return PX || l > 0.0f ? 1.0f / l : 0.0f; }
+template <bool PX> __device__ __forceinline__ float quotient(float o, float l, float inv) {
+    const float q = o * inv;
+    return PX ? fmaf(fmaf(-q, l, o), inv, q) : q;
+}
 // exp(s - m) as one multiply-add and one exponential: 2^(s log2(e) - m log2(e)); m2 = m log2(e)
 __device__ __forceinline__ float exp_rel(float s, float m2) { return __builtin_amdgcn_exp2f(fmaf(s, FM_LOG2E, -m2)); }
 
@@ -246,39 +268,95 @@ __device__ __forceinline__ float alibi_slope(const fattn_args &a, int64_t head) 
 // element 32 dt + l32 of cells c .. c + 3 and c + 8 .. c + 11, c = 32 u + 16 t + 4 lhi - comes from the row-major V tile by two
 // transposing reads: in each group of 16 lanes, lane i receives element i % 4 of the four rows that lanes i / 4, i / 4 + 4, + 8 and
 // + 12 point at, so lane 4 r + q of a group points at row c + r, elements 16 (group % 2) + 4 q .. + 3 of the tile's 32.
+template <int D>
+__device__ __forceinline__ const _Float16 *v_lane_base(const _Float16 *sV, int u, int l32, int lhi) {
+    const int li = l32 & 15;
+    return sV + (32 * u + 4 * lhi + (li >> 2)) * fm_vpitch<D>() + 16 * (l32 >> 4) + 4 * (li & 3);
+}
+template <int VP>
+__device__ __forceinline__ f16x8 v_fragment(const _Float16 *vp) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)vp);
+    const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(vp + 8 * VP));
+    const f16x4 h0 = __builtin_bit_cast(f16x4, v0), h1 = __builtin_bit_cast(f16x4, v1);
+    f16x8 vf;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        vf[i] = h0[i];
+        vf[4 + i] = h1[i];
+    }
+    return vf;
+}
 template <int D, int NDT>
 __device__ __forceinline__ void accumulate_pv(f32x16 (&o)[NDT], const f32x16 &S, const _Float16 *sV, int dt0, int u, int l32, int lhi) {
     constexpr int VP = fm_vpitch<D>();
-    typedef short s16x4 __attribute__((ext_vector_type(4)));
-    const int li = l32 & 15;
-    const _Float16 *lane_base = sV + (32 * u + 4 * lhi + (li >> 2)) * VP + 16 * (l32 >> 4) + 4 * (li & 3);
+    const _Float16 *lane_base = v_lane_base<D>(sV, u, l32, lhi);
 #pragma unroll
     for (int t = 0; t < 2; t++) {
         f16x8 pf;
 #pragma unroll
         for (int i = 0; i < 8; i++) pf[i] = (_Float16)S[8 * t + i];
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) {
-            const _Float16 *vp = lane_base + 16 * t * VP + 32 * (dt0 + dt);
-            const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)vp);
-            const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(vp + 8 * VP));
-            const f16x4 h0 = __builtin_bit_cast(f16x4, v0), h1 = __builtin_bit_cast(f16x4, v1);
-            f16x8 vf;
+        for (int dt = 0; dt < NDT; dt++)
+            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_fragment<VP>(lane_base + 16 * t * VP + 32 * (dt0 + dt)), pf, o[dt], 0, 0, 0);
+    }
+}
+// PX: the same for the NS halves u0 .. of a tile, with probabilities as pairs.  A tile's terms are added up from zero and meet the long sum
+// once: of the roundings of O those are the ones that count (one per tile of 64 cells where the vector kernel has one per 16 or 32 cells).
+template <int D, int NDT, int NS>
+__device__ __forceinline__ void accumulate_pv_px(f32x16 (&o)[NDT], const f32x16 (&S)[NS], const _Float16 *sV, int u0, int l32, int lhi) {
+    constexpr int VP = fm_vpitch<D>();
+    f16x8 hi[2 * NS], lo[2 * NS];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                vf[i] = h0[i];
-                vf[4 + i] = h1[i];
-            }
-            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf, o[dt], 0, 0, 0);
+    for (int t = 0; t < 2 * NS; t++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float p = S[t / 2][8 * (t & 1) + i];
+            hi[t][i] = (_Float16)(p * FM_PX_SCALE);
+            lo[t][i] = (_Float16)fmaf(p, FM_PX_SCALE, -(float)hi[t][i]);   // exact before the conversion
         }
+    const _Float16 *lane_base = v_lane_base<D>(sV, u0, l32, lhi);
+#pragma unroll
+    for (int dt = 0; dt < NDT; dt++) {
+        f32x16 sum;
+#pragma unroll
+        for (int r = 0; r < 16; r++) sum[r] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 2 * NS; t++) {
+            const f16x8 vf = v_fragment<VP>(lane_base + 16 * t * VP + 32 * dt);
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, lo[t], sum, 0, 0, 0);
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, hi[t], sum, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[dt][r] += sum[r];
     }
 }
 
 // EAGER: all of the row's fragments are requested before the first matrix instruction (D / 2 more registers), so the chain of
 // dependent instructions does not stop for an LDS round trip after every second one.
-template <int D, bool EAGER = false>
+// CHAINS: independent partial sums of D / CHAINS elements each, added at the end (smaller sums, smaller roundings)
+template <int D, bool EAGER = false, int CHAINS = 1>
 __device__ __forceinline__ f32x16 scores(const f16x8 (&qf)[D / 16], const _Float16 *sK, int u, int l32, int lhi) {
     constexpr int KP = D + 8;
+    if constexpr (CHAINS > 1) {
+        f32x16 part[CHAINS];
+#pragma unroll
+        for (int c = 0; c < CHAINS; c++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) part[c][r] = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < D / 16; kk++) {
+            const f16x8 kf = *(const f16x8 *)(sK + (32 * u + l32) * KP + 16 * kk + 8 * lhi);
+            part[kk % CHAINS] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[kk], part[kk % CHAINS], 0, 0, 0);
+        }
+#pragma unroll
+        for (int step = 1; step < CHAINS; step *= 2)
+#pragma unroll
+            for (int c = 0; c + step < CHAINS; c += 2 * step)
+#pragma unroll
+                for (int r = 0; r < 16; r++) part[c][r] += part[c + step][r];
+        return part[0];
+    }
     f32x16 S;
 #pragma unroll
     for (int r = 0; r < 16; r++) S[r] = 0.0f;
@@ -347,7 +425,7 @@ __device__ __forceinline__ grid_pos xcd_grid_pos() {
     return grid_pos{nx - 1 - (unsigned)(L % nx), (unsigned)(L / nx)};
 }
 
-template <int D, int HPW>
+template <int D, int HPW, bool PX>
 __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a) {
     typedef kv_stage<D, 256> stage_t;
     constexpr int QTW = 4 / HPW;   // query tiles per group
@@ -418,16 +496,16 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
         float mx = FM_NEG;
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            S[u] = scores<D>(qf, sK, u, l32, lhi);
+            S[u] = scores<D, false, PX ? fm_px_chains<D>() : 1>(qf, sK, u, l32, lhi);
             mx = fmaxf(mx, finish_scores(S[u], mcur[u], a, scale, slope, kv0 + 32 * u, lhi, a.Nkv));
         }
         mx = half_pair_max(mx);
         if (__ballot(mx > FM_NEG) == 0) continue;   // every cell of the tile is masked for all 32 queries (wave-uniform)
-        const float m_new = lazy_max(m, mx);
-        const float alpha = __builtin_amdgcn_exp2f((m - m_new) * FM_LOG2E);   // exactly 1 while the reference point stays
+        const float m_new = lazy_max<PX>(m, mx);
+        const float alpha = rescale<PX>(m, m_new);   // exactly 1 while the reference point stays
         // dropped scores are exactly FM_NEG: exp(FM_NEG - m) is 0 for any real maximum; a column that has seen no cell yet
         // (maximum still FM_NEG) subtracts 0 instead, so its dropped scores give 0 as well and not exp(0)
-        const float m2 = m_new > FM_NEG ? m_new * FM_LOG2E : 0.0f;
+        const float m2 = m_new > FM_NEG ? exponent_of<PX>(m_new) : 0.0f;
         float rs = 0.0f;
 #pragma unroll
         for (int u = 0; u < 2; u++)
@@ -446,12 +524,15 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
         }
+        if constexpr (PX) accumulate_pv_px<D, NDT, 2>(o, S, sVt, 0, l32, lhi);
+        else {
 #pragma unroll
-        for (int u = 0; u < 2; u++) accumulate_pv<D, NDT>(o, S[u], sVt, 0, u, l32, lhi);
+            for (int u = 0; u < 2; u++) accumulate_pv<D, NDT>(o, S[u], sVt, 0, u, l32, lhi);
+        }
     }
 
     if (q0 + l32 < a.Nq) {
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        const float sum = sum_of<PX>(l), inv = reciprocal_of<PX>(sum);
         float *dp = a.dst + ((q0 + l32) * a.Hq + head) * D;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++)
@@ -460,7 +541,7 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
                 if (32 * dt + 8 * g >= D) continue;
                 f32x4 w;
 #pragma unroll
-                for (int i = 0; i < 4; i++) w[i] = o[dt][4 * g + i] * inv;
+                for (int i = 0; i < 4; i++) w[i] = quotient<PX>(o[dt][4 * g + i], sum, inv);
                 *(f32x4 *)(dp + 32 * dt + 8 * g + 4 * lhi) = w;
             }
     }
@@ -475,7 +556,7 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
 // unit: two waves per SIMD, so that one wave's matrix instructions run under the other's soft-max arithmetic, and half the
 // tile steps.
 // PQ: the two columns of waves are neighbouring query tiles of one head instead of two heads (an odd number of query heads per kv head)
-template <int D, int NU, bool PQ>
+template <int D, int NU, bool PQ, bool PX>
 __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn_mma_half(fattn_args a) {
     constexpr int NTH = 128 * NU, BC = 32 * NU;
     typedef kv_stage<D, NTH, BC> stage_t;
@@ -513,30 +594,42 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
         for (int r = 0; r < 16; r++) o[dt][r] = 0.0f;
     float m = FM_NEG, l = 0.0f;
 
+    // cells past kv_limit are masked for every query of this group
+    int64_t kv_limit = a.Nkv;
+    if constexpr (PX) {
+        if (a.kv_extent) {
+            int e = a.kv_extent[PQ ? 2 * gp.x : gp.x];
+            if (PQ && (int64_t)(2 * gp.x + 1) * 32 < a.Nq) e = max(e, a.kv_extent[2 * gp.x + 1]);
+            kv_limit = e < a.Nkv ? e : a.Nkv;
+        }
+    }
+
     stage_t st;
     u32x2 mnext[4];
     auto prefetch = [&](int64_t kv0) {
         st.fetch(a, hk, kv0, tid);
         fetch_mask<4>(mnext, mrow, mask_aligned && kv0 + BC <= a.Nkv, kv0 + 32 * u + 4 * lhi, a.Nkv);
     };
-    prefetch(0);
-    for (int64_t kv0 = 0; kv0 < a.Nkv; kv0 += BC) {
+    if (!PX || kv_limit > 0) prefetch(0);
+    for (int64_t kv0 = 0; kv0 < kv_limit; kv0 += BC) {
         __syncthreads();   // the previous tile has been consumed
         st.commit(sK, sVt, tid);
         u32x2 mcur[4];
 #pragma unroll
         for (int g = 0; g < 4; g++) mcur[g] = mnext[g];
         __syncthreads();
-        if (kv0 + BC < a.Nkv) prefetch(kv0 + BC);
-        f32x16 S = scores<D, (D <= 128)>(qf, sK, u, l32, lhi);
+        if (kv0 + BC < kv_limit) prefetch(kv0 + BC);
+        f32x16 S1[1];
+        f32x16 &S = S1[0];
+        S = scores<D, (D <= 128), PX ? fm_px_chains<D>() : 1>(qf, sK, u, l32, lhi);
         float mx = finish_scores(S, mcur, a, scale, slope, kv0 + 32 * u, lhi, a.Nkv);
         mx = half_pair_max(mx);
         if (__ballot(mx > FM_NEG) == 0) continue;   // all 32 cells masked for all 32 queries (wave-uniform; barriers are at the loop head)
-        const float m_new = lazy_max(m, mx);
-        const float alpha = __builtin_amdgcn_exp2f((m - m_new) * FM_LOG2E);   // exactly 1 while the reference point stays
+        const float m_new = lazy_max<PX>(m, mx);
+        const float alpha = rescale<PX>(m, m_new);   // exactly 1 while the reference point stays
         // dropped scores are exactly FM_NEG: exp(FM_NEG - m) is 0 for any real maximum; a column that has seen no cell yet
         // (maximum still FM_NEG) subtracts 0 instead, so its dropped scores give 0 as well and not exp(0)
-        const float m2 = m_new > FM_NEG ? m_new * FM_LOG2E : 0.0f;
+        const float m2 = m_new > FM_NEG ? exponent_of<PX>(m_new) : 0.0f;
         float rs = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
@@ -553,7 +646,8 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
         }
-        accumulate_pv<D, NDT>(o, S, sVt, 0, u, l32, lhi);
+        if constexpr (PX) accumulate_pv_px<D, NDT, 1>(o, S1, sVt, u, l32, lhi);
+        else accumulate_pv<D, NDT>(o, S, sVt, 0, u, l32, lhi);
     }
 
     // ---- the states of a head's waves are joined pairwise: u + step hands its state to u (step = 1, then 2)
@@ -575,7 +669,7 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
         if ((u & (2 * step - 1)) == 0) {
             const float m1 = mg[DP * 32 + l32], l1 = mg[(DP + 1) * 32 + l32];
             const float M = fmaxf(m, m1);
-            const float f0 = __expf(m - M), f1 = __expf(m1 - M);
+            const float f0 = merge_factor<PX>(m, M), f1 = merge_factor<PX>(m1, M);
             l = l * f0 + l1 * f1;
             m = M;
 #pragma unroll
@@ -585,7 +679,7 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
         }
     }
     if (u != 0 || q0 + l32 >= a.Nq) return;
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const float sum = sum_of<PX>(l), inv = reciprocal_of<PX>(sum);
     float *dp = a.dst + ((q0 + l32) * a.Hq + head) * D;
 #pragma unroll
     for (int dt = 0; dt < NDT; dt++)
@@ -594,12 +688,12 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
             if (32 * dt + 8 * g >= D) continue;
             f32x4 w;
 #pragma unroll
-            for (int i = 0; i < 4; i++) w[i] = o[dt][4 * g + i] * inv;
+            for (int i = 0; i < 4; i++) w[i] = quotient<PX>(o[dt][4 * g + i], sum, inv);
             *(f32x4 *)(dp + 32 * dt + 8 * g + 4 * lhi) = w;
         }
 }
 
-template <int D, bool PQ>
+template <int D, bool PQ, bool PX>
 int launch_half(hipStream_t s, const fattn_args &a) {
     const int64_t R = a.Hq / a.Hkv, n_tiles = (a.Nq + 31) / 32;
     const dim3 grid((unsigned)(PQ ? (n_tiles + 1) / 2 : n_tiles), (unsigned)(a.Hkv * (PQ ? R : R / 2)));
@@ -607,29 +701,40 @@ int launch_half(hipStream_t s, const fattn_args &a) {
     // 512 cells 24.8 -> 26.2 us)
     if constexpr (D <= 128) {   // (head size 256: the eight waves' registers do not fit)
         if ((int64_t)grid.x * grid.y <= 256 && a.Nkv >= 1024) {
-            MI355_LAUNCH((k_fattn_mma_half<D, 4, PQ>), grid, dim3(512), 0, s, a);
+            MI355_LAUNCH((k_fattn_mma_half<D, 4, PQ, PX>), grid, dim3(512), 0, s, a);
             return launch_status("k_fattn_mma_half");
         }
     }
-    MI355_LAUNCH((k_fattn_mma_half<D, 2, PQ>), grid, dim3(256), 0, s, a);
+    MI355_LAUNCH((k_fattn_mma_half<D, 2, PQ, PX>), grid, dim3(256), 0, s, a);
     return launch_status("k_fattn_mma_half");
 }
 
-template <int D, int HPW>
+template <int D, int HPW, bool PX>
 int launch(hipStream_t s, const fattn_args &a) {
     constexpr int QTW = 4 / HPW;
     const int64_t groups = (a.Hq / a.Hkv) / HPW;
     const dim3 grid((unsigned)((a.Nq + 32 * QTW - 1) / (32 * QTW)), (unsigned)(a.Hkv * groups));
-    MI355_LAUNCH((k_fattn_mma<D, HPW>), grid, dim3(256), 0, s, a);
+    MI355_LAUNCH((k_fattn_mma<D, HPW, PX>), grid, dim3(256), 0, s, a);
     return launch_status("k_fattn_mma");
 }
 
-template <int D>
+template <int D, bool PX>
 int launch_hpw(hipStream_t s, const fattn_args &a) {
     const int64_t R = a.Hq / a.Hkv;
-    if (R % 4 == 0) return launch<D, 4>(s, a);
-    if (R % 2 == 0) return launch<D, 2>(s, a);
-    return launch<D, 1>(s, a);
+    if (R % 4 == 0) return launch<D, 4, PX>(s, a);
+    if (R % 2 == 0) return launch<D, 2, PX>(s, a);
+    return launch<D, 1, PX>(s, a);
+}
+
+// Pairs of probabilities: head sizes 112 and 128 always in halves (the registers of whole tiles do not fit: 50 and 33 spills; 2048 x 2048 cells,
+// 32 / 8 heads: 165 -> 139 and 160 -> 155 us), head size 64 too (the error of its longer sums would exceed the vector kernel's, 1.39e-7 against 1.36e-7; halves 1.34e-7)
+template <int D, bool PX>
+int launch_head(hipStream_t s, const fattn_args &a, bool pq, bool half) {
+    constexpr bool HALVES_ONLY = PX && (D == 64 || D == 112 || D == 128);
+    if constexpr (!HALVES_ONLY) {
+        if (!half) return launch_hpw<D, PX>(s, a);
+    }
+    return pq ? launch_half<D, true, PX>(s, a) : launch_half<D, false, PX>(s, a);
 }
 
 // ---- decode / small batches: the 32 MFMA columns are (token, head of the GQA group) pairs -------
@@ -834,17 +939,20 @@ int launch_fattn_mma(hipStream_t s, fattn_args &a, int64_t D, size_t ws_bytes) {
     // few query tiles (a batch of a few hundred rows): twice the groups with half a K/V tile per wave, while the chip is not full
     const int64_t R = a.Hq / a.Hkv;
     // (an odd number of query heads per kv head pairs neighbouring query tiles: 512 rows over 1024 cells, 32 heads, D 128: 40 -> 31 us).
-    // Against the vector kernel, which served these head sizes before: 512 x 512 cells, 32 / 32 heads, D 80: 192 -> 16 us (launch and
-    // latency of eight tile steps); 2048 x 2048, 32 / 8 heads: D 80 2053 -> 95 us, D 112 2055 -> 117 us, D 256 4370 -> 325 us.
+    // Against the vector kernel, which served the other head sizes and the quantized output before (us; error against 64-bit arithmetic on the
+    // same operands; f16 probabilities would be 1.5e-4 .. 2.1e-4): 512 x 512 cells, 32 / 32 heads, D 80: 203 -> 18.3, 1.28e-7 -> 1.25e-7;
+    // 2048 x 2048, 32 / 8 heads: D 80 2046 -> 111, 1.56e-7 -> 1.49e-7; D 112 2049 -> 139, 1.55e-7 -> 1.47e-7; D 256 4346 -> 252, 1.71e-7 -> 1.59e-7;
+    // D 128 with quantized output 2056 -> 155, 1.55e-7 -> 1.44e-7, 768 x 2048 812 -> 91, 2.49e-7 -> 2.05e-7.
+    const bool px = a.act_q != nullptr;   // head sizes 64 and 128: f16 probabilities, except where the output is also quantized
     const bool pq = R % 2 != 0, half = (pq ? (n_tiles + 1) / 2 * a.Hq : n_tiles * a.Hq / 2) <= 512;
-#define MI355_FM_HEAD(D_) return !half ? launch_hpw<D_>(s, a) : pq ? launch_half<D_, true>(s, a) : launch_half<D_, false>(s, a);
+#define MI355_FM_HEAD(D_, PX_) return launch_head<D_, PX_>(s, a, pq, half);
     switch (D) {
-        case 64: MI355_FM_HEAD(64)
-        case 80: MI355_FM_HEAD(80)
-        case 96: MI355_FM_HEAD(96)
-        case 112: MI355_FM_HEAD(112)
-        case 128: MI355_FM_HEAD(128)
-        case 256: MI355_FM_HEAD(256)
+        case 64: if (px) MI355_FM_HEAD(64, true) else MI355_FM_HEAD(64, false)
+        case 80: MI355_FM_HEAD(80, true)
+        case 96: MI355_FM_HEAD(96, true)
+        case 112: MI355_FM_HEAD(112, true)
+        case 128: if (px) MI355_FM_HEAD(128, true) else MI355_FM_HEAD(128, false)
+        case 256: MI355_FM_HEAD(256, true)
         default: return 1;
     }
 #undef MI355_FM_HEAD
