@@ -920,10 +920,20 @@ int launch_dec(hipStream_t s, const fattn_args &a) {
 
 }  // namespace
 
+// From how many (query, head) pairs on the matrix-core kernels are ahead of the vector kernel, which splits the cells over groups and so
+// fills the chip with any number of pairs, while a tile of 32 queries walks all cells in one serial chain (1.1 us per 64 cells of D 80).
+// Smallest sizes at which no call of the grid {4 .. 64 heads} x {16 .. 384 rows} x {64 .. 16384 cells} x head sizes was slower: us, vector / matrix,
+// 16384 cells: D 80, 4 heads, 16 rows 35 / 291; D 256, 8 heads, 64 rows 318 / 818; D 64, 16 heads, 64 rows 146 / 253, 96 rows 232 / 252;
+// D 80, 32 heads, 48 rows 465 / 295; 64 cells, D 256, 32 heads, 48 rows 11 / 15, 64 rows 13.6 / 15.2.
+static int64_t px_min_pairs(int64_t D, int64_t Nkv) { return Nkv < 512 ? 2049 : D == 64 ? 1537 : 1152; }
+
 int launch_fattn_mma(hipStream_t s, fattn_args &a, int64_t D, size_t ws_bytes) {
     if (a.Hkv * (a.Hq / a.Hkv) > 65535 || (a.Nq + 31) / 32 > 0x7fffffff) return 1;
     if ((a.q_nb1 % 16) != 0 || (a.q_nb2 % 16) != 0) return 1;
     if (a.k_nb1 >= (size_t(1) << 24) || a.v_nb1 >= (size_t(1) << 24)) return 1;   // kv_stage: a tile's rows within 32-bit offsets
+    // head sizes 64 and 128: f16 probabilities, except where the output is also quantized
+    const bool px = a.act_q != nullptr || (D != 64 && D != 128);
+    if (px && a.Nq * a.Hq < px_min_pairs(D, a.Nkv)) return 1;
     a.kv_extent = nullptr;
     const int64_t n_tiles = (a.Nq + 31) / 32;
     // The pre-pass pays when there are more groups than the chip holds at once (two per compute unit): then a group that stops
@@ -943,7 +953,6 @@ int launch_fattn_mma(hipStream_t s, fattn_args &a, int64_t D, size_t ws_bytes) {
     // same operands; f16 probabilities would be 1.5e-4 .. 2.1e-4): 512 x 512 cells, 32 / 32 heads, D 80: 203 -> 18.3, 1.28e-7 -> 1.25e-7;
     // 2048 x 2048, 32 / 8 heads: D 80 2046 -> 111, 1.56e-7 -> 1.49e-7; D 112 2049 -> 139, 1.55e-7 -> 1.47e-7; D 256 4346 -> 252, 1.71e-7 -> 1.59e-7;
     // D 128 with quantized output 2056 -> 155, 1.55e-7 -> 1.44e-7, 768 x 2048 812 -> 91, 2.49e-7 -> 2.05e-7.
-    const bool px = a.act_q != nullptr;   // head sizes 64 and 128: f16 probabilities, except where the output is also quantized
     const bool pq = R % 2 != 0, half = (pq ? (n_tiles + 1) / 2 * a.Hq : n_tiles * a.Hq / 2) <= 512;
 #define MI355_FM_HEAD(D_, PX_) return launch_head<D_, PX_>(s, a, pq, half);
     switch (D) {

@@ -277,3 +277,29 @@ def test_prefill_f32_probabilities(dev, D, quantized, Nq, Nkv, Hq, Hkv):
     got = mi355.flash_attn_ext(*(torch.from_numpy(a).to(dev) for a in (q, k, v, mask)), scale, quantized=quantized)
     got = (got[0] if quantized else got).cpu().numpy()
     assert orc.nmse(got, _textbook(q, k, v, mask, scale)) < 1e-12
+
+
+@pytest.mark.parametrize("D,quantized", [(80, False), (256, False), (64, True), (128, True)])
+@pytest.mark.parametrize("Nkv,pairs", [(64, 2049), (508, 2049), (2048, 1152)])
+def test_prefill_few_pairs_stay_on_the_vector_kernel(dev, D, quantized, Nkv, pairs):
+    """with few (query, head) pairs a serial walk over the cells takes several times as long as the vector kernel: both sides of the line,
+    told apart by the launches (vector kernel: the output's quantization inside, a merge launch where the cells are split)"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    if D == 64 and Nkv == 2048:
+        pairs = 1537
+    rng = np.random.default_rng(D + Nkv)
+    for Hq in (8, 32):
+        most = (pairs - 1) // Hq
+        for Nq, matrix in ((most, False), (most + 1, True)):
+            q, k, v, _ = _inputs(rng, D, Nq, Nkv, Hq, Hq // 4, causal=False)
+            mask = np.zeros(((Nq + 63) // 64 * 64, Nkv), dtype=np.float16)
+            args = [torch.from_numpy(a).to(dev) for a in (q, k, v, mask)]
+            before = lib.mi355_launch_count()
+            got = mi355.flash_attn_ext(*args, 1.0 / np.sqrt(D), quantized=quantized)
+            launches = lib.mi355_launch_count() - before
+            splits = min(max(1, min((Nkv + 255) // 256, 2048 // (Hq // 4 * Nq))), 256)
+            assert launches == ((2 if quantized else 1) if matrix else (2 if splits > 1 else 1)), (Hq, Nq)
+            got = (got[0] if quantized else got).cpu().numpy()
+            assert orc.nmse(got, _textbook(q, k, v, mask, 1.0 / np.sqrt(D))) < 1e-12
