@@ -71,7 +71,7 @@ int fattn_vec_kv(hipStream_t s, const float *q, const void *k, int type_k, const
                  size_t ws_bytes, void *act);
 
 // one query token over at most 512 cells of an f16 cache, head size 128, up to four query heads per kv head: one launch, two
-// groups per kv head (halves of the output), one wave per 64 cells, states merged in LDS (fattn_stream.hip); returns 1 when the shape is not served
+// groups per kv head up to 128 of those (halves of the output), one wave per 64 cells, states merged in LDS (fattn_stream.hip); returns 1 when the shape is not served
 int launch_fattn_dec_short(hipStream_t s, fattn_args &a, int64_t D);
 // one query token over a long f16 cache, head size 128, up to four query heads per kv head: per-wave streaming through LDS
 // (fattn_stream.hip); sets a.n_splits for k_fattn_combine; returns 1 when the shape is not served

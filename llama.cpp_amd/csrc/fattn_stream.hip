@@ -701,7 +701,7 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
 }
 
 // ---- short caches: at most 512 cells, one launch -------------------------------------------------------------------------------
-// Two groups per kv head, one for each half of the output elements, one wave per 64-cell tile (up to eight).  Nothing here is bound by bytes: the time is one trip to memory
+// Two groups per kv head, one for each half of the output elements (PARTS), one wave per 64-cell tile (up to eight).  Nothing here is bound by bytes: the time is one trip to memory
 // plus the arithmetic of one tile, so a wave requests everything at once - its K and V tiles as coalesced 16-byte loads into
 // registers (four whole rows per instruction), q, its mask value - and then passes first K, then V through its own 16 KiB of
 // LDS to bring them into operand form: K rows with their chunks XOR-ed across the banks, so that each lane reads back the row of
@@ -710,27 +710,31 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
 // (and its Q8_1 form where the next product wants it), so no second launch merges anything.
 // Both groups of a kv head form the same scores; a group then reads only its half of every V row.  In a model the cache comes from HBM and a
 // compute unit's own requests are what takes the time: 512 cells are 256 KiB for one group per kv head (12.0 us per layer, 8B model),
-// 192 KiB for one of two (10.4 us; K reaches the second one through L2), with the same bits.
+// 192 KiB for one of two (10.4 us; K reaches the second one through L2), with the same bits.  A group takes a compute unit's LDS: with
+// more than 128 kv heads two groups each would take a second round (256 kv heads, 512 cells: 16.4 us with one group per head, 23.9 with two).
 constexpr int FSS_MAX_WAVES = 8;
 
+template <int PARTS>
 __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn_args a, int R) {
+    static_assert(PARTS == 1 || PARTS == 2, "whole rows of V or halves");
+    constexpr int DO = FS_D / PARTS, VIT = 16 / PARTS, VCH = 16 / PARTS;   // output elements of the group; V loads; 16-byte chunks of V per row
     __shared__ __attribute__((aligned(1024))) uint8_t tbuf[FSS_MAX_WAVES * FS_KT];
     __shared__ __attribute__((aligned(16))) unsigned short pbuf[FSS_MAX_WAVES][4][FS_TILE];
     __shared__ float s_m[FSS_MAX_WAVES][4], s_l[FSS_MAX_WAVES][4];
-    __shared__ float s_o[FSS_MAX_WAVES][4][FS_D / 2];
+    __shared__ float s_o[FSS_MAX_WAVES][4][DO];
     __shared__ __attribute__((aligned(16))) unsigned short qbuf[FSS_MAX_WAVES][4][FS_D];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int n_waves = (int)(blockDim.x >> 6);
     const int64_t hk = blockIdx.x;
-    const int part = (int)blockIdx.y;   // elements 64 part .. + 63 of the output
+    const int part = (int)blockIdx.y;   // PARTS == 2: elements 64 part .. + 63 of the output
     const int64_t c0 = (int64_t)wave * FS_TILE;
     const int rsub = lane >> 4, pos = lane & 15;
 
     // load i: rows 4i .. 4i + 3, lane -> row 4i + lane / 16, chunk lane % 16 (rows past the end repeat the last cell; their weights are zero)
     // (half rows of V: rows 8i .. 8i + 7, lane -> row 8i + lane / 8, chunk lane % 8 of the half)
-    const int vsub = lane >> 3, vpos = (lane & 7) + 8 * part;
-    u32x4 kraw[16], vraw[8];
+    const int vsub = lane / VCH, vpos = lane % VCH + VCH * part;
+    u32x4 kraw[16], vraw[VIT];
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         int64_t cell = c0 + 4 * i + rsub;
@@ -738,8 +742,8 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
         kraw[i] = load16(a.k + cell * a.k_nb1 + hk * a.k_nb2 + (pos << 4));
     }
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        int64_t cell = c0 + 8 * i + vsub;
+    for (int i = 0; i < VIT; i++) {
+        int64_t cell = c0 + (64 / VIT) * i + vsub;
         if (cell >= a.Nkv) cell = a.Nkv - 1;
         vraw[i] = load16(a.v + cell * a.v_nb1 + hk * a.v_nb2 + (vpos << 4));
     }
@@ -794,10 +798,11 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
 
     // V through the same bytes, row-major (the K rows are in registers)
 #pragma unroll
-    for (int i = 0; i < 8; i++) *(u32x4 *)(tb + (8 * i + vsub) * FS_ROW + (vpos << 4)) = vraw[i];
+    for (int i = 0; i < VIT; i++) *(u32x4 *)(tb + ((64 / VIT) * i + vsub) * FS_ROW + (vpos << 4)) = vraw[i];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // fs_output reads LDS through inline assembly: nothing may be moved across
     const unsigned v_addr = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)tb + fs_v_lane(lane), p_rd = p_base + (unsigned)(lane & 3) * (FS_TILE * 2);
-    if (part == 0) fs_output_half<0>(v_addr, p_rd, S.o0);   // uniform
+    if constexpr (PARTS == 1) fs_output(v_addr, p_rd, S);
+    else if (part == 0) fs_output_half<0>(v_addr, p_rd, S.o0);   // uniform
     else fs_output_half<1>(v_addr, p_rd, S.o0);
 
     // ---- the waves' states meet in LDS
@@ -809,10 +814,11 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
             s_l[wave][r] = L;
         }
         s_o[wave][r][lane] = S.o0[r];
+        if constexpr (PARTS == 1) s_o[wave][r][64 + lane] = S.o1[r];
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < R * (FS_D / 2); idx += (int)blockDim.x) {   // whole waves: R * 64 and the group size are multiples of 64
-        const int r = idx / (FS_D / 2), d = idx % (FS_D / 2);
+    for (int idx = threadIdx.x; idx < R * DO; idx += (int)blockDim.x) {   // whole waves: R * DO and the group size are multiples of 64
+        const int r = idx / DO, d = idx % DO;
         float M = s_m[0][r];
         for (int w = 1; w < n_waves; w++) M = fmaxf(M, s_m[w][r]);
         float L = 0.0f, O = 0.0f;
@@ -834,7 +840,8 @@ int launch_fattn_dec_short(hipStream_t s, fattn_args &a, int64_t D) {
     if (D != FS_D || a.Nq != 1 || R > 4 || a.Hkv > 65535 || a.Nkv > FSS_MAX_WAVES * FS_TILE) return 1;
     if ((a.q_nb2 % 16) != 0 || (a.k_nb1 % 16) != 0 || (a.k_nb2 % 16) != 0 || (a.v_nb1 % 16) != 0 || (a.v_nb2 % 16) != 0) return 1;
     const int n_waves = (int)((a.Nkv + FS_TILE - 1) / FS_TILE);
-    MI355_LAUNCH(k_fattn_dec_short, dim3((unsigned)a.Hkv, 2), dim3((unsigned)n_waves * 64), 0, s, a, (int)R);
+    if (a.Hkv <= 128) MI355_LAUNCH(k_fattn_dec_short<2>, dim3((unsigned)a.Hkv, 2), dim3((unsigned)n_waves * 64), 0, s, a, (int)R);
+    else MI355_LAUNCH(k_fattn_dec_short<1>, dim3((unsigned)a.Hkv), dim3((unsigned)n_waves * 64), 0, s, a, (int)R);
     return launch_status("k_fattn_dec_short");
 }
 

@@ -303,3 +303,18 @@ def test_prefill_few_pairs_stay_on_the_vector_kernel(dev, D, quantized, Nkv, pai
             assert launches == ((2 if quantized else 1) if matrix else (2 if splits > 1 else 1)), (Hq, Nq)
             got = (got[0] if quantized else got).cpu().numpy()
             assert orc.nmse(got, _textbook(q, k, v, mask, 1.0 / np.sqrt(D))) < 1e-12
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(128, 128), (129, 129), (258, 129), (520, 130), (256, 256)])
+@pytest.mark.parametrize("Nkv", [257, 320, 511, 512])
+def test_decode_short_cache_many_kv_heads(dev, Hq, Hkv, Nkv):
+    """one token over 257 .. 512 cells: two groups per kv head up to 128 of them, one beyond; f16 probabilities leave some 2e-4 (NMSE 4e-8)"""
+    import torch
+    import mi355
+    rng = np.random.default_rng(Hq + Nkv)
+    q, k, v, mask = _inputs(rng, 128, 1, Nkv, Hq, Hkv, causal=False, rand_mask=True)
+    mask[0, rng.integers(0, Nkv, 40)] = -np.inf
+    args = [torch.from_numpy(a).to(dev) for a in (q, k, v, mask)]
+    dst, act = mi355.flash_attn_ext(*args, 0.09, quantized=True)
+    assert orc.nmse(dst.cpu().numpy(), _textbook(q, k, v, mask, 0.09)) < 1e-6
+    assert torch.equal(act, mi355.quantize_act(dst.reshape(1, Hq * 128)))
