@@ -166,9 +166,16 @@ template <bool PX> __device__ __forceinline__ float quotient(float o, float l, f
 // exp(s - m) as one multiply-add and one exponential: 2^(s log2(e) - m log2(e)); m2 = m log2(e)
 __device__ __forceinline__ float exp_rel(float s, float m2) { return __builtin_amdgcn_exp2f(fmaf(s, FM_LOG2E, -m2)); }
 
-// scale [+ softcap], add the mask, mark dropped cells with FM_NEG; returns the largest surviving score.
-// A masked cell (-inf; slopes are positive) and a NaN score of a stale cell both end as FM_NEG in fmaxf(s, FM_NEG); the test against
-// the end of the range is made only in a tile that reaches past it (uniform over the group), on 32-bit offsets.
+// the larger of two, NaN if one of them is (v_maximum3_f32)
+__device__ __forceinline__ float max_or_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float half_pair_max_or_nan(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return max_or_nan(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// scale [+ softcap], add the mask; returns the largest score, NaN if there is one (such a tile is not skipped).  A masked cell (-inf) and one past the end of the range end as -inf, a
+// probability of exactly 0.  A NaN stays one and shows in the column's sum (store_rows).  The test against the end of the range is
+// made only in a tile that reaches past it (uniform over the group), on 32-bit offsets.
 __device__ __forceinline__ float finish_scores(f32x16 &S, const u32x2 (&mw)[4], const fattn_args &a, float scale, float slope,
                                                 int64_t c_first, int lhi, int64_t c_end) {
     float mx = FM_NEG;
@@ -178,10 +185,8 @@ __device__ __forceinline__ float finish_scores(f32x16 &S, const u32x2 (&mw)[4], 
         for (int g = 0; g < 4; g++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                float s = fmaf(S[4 * g + i], scale, mask_value(mw[g], i));
-                s = fmaxf(s, FM_NEG);   // -inf and NaN become FM_NEG
-                S[4 * g + i] = s;
-                mx = fmaxf(mx, s);
+                S[4 * g + i] = fmaf(S[4 * g + i], scale, mask_value(mw[g], i));
+                mx = max_or_nan(mx, S[4 * g + i]);
             }
         return mx;
     }
@@ -192,31 +197,17 @@ __device__ __forceinline__ float finish_scores(f32x16 &S, const u32x2 (&mw)[4], 
 #pragma unroll
         for (int r = 0; r < 16; r++) S[r] *= scale;
     }
-    if (room >= 32) {   // every cell of this half tile lies inside the range
+    const int left = room < 32 ? (int)room - 4 * lhi : 32;   // cells of the range from this lane's first one on (may be <= 0)
 #pragma unroll
-        for (int g = 0; g < 4; g++)
+    for (int g = 0; g < 4; g++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float s = S[4 * g + i] + slope * mask_value(mw[g], i);
-                s = fmaxf(s, FM_NEG);   // -inf and NaN become FM_NEG
-                S[4 * g + i] = s;
-                mx = fmaxf(mx, s);
-            }
-    } else {
-        const int left = (int)room - 4 * lhi;   // cells of the range from this lane's first one on (may be <= 0)
-#pragma unroll
-        for (int g = 0; g < 4; g++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float s = S[4 * g + i] + slope * mask_value(mw[g], i);
-                s = 8 * g + i < left ? fmaxf(s, FM_NEG) : FM_NEG;
-                S[4 * g + i] = s;
-                mx = fmaxf(mx, s);
-            }
-    }
+        for (int i = 0; i < 4; i++) {
+            const float mv = mask_value(mw[g], i);
+            S[4 * g + i] = 8 * g + i < left && mv != -INFINITY ? S[4 * g + i] + slope * mv : -INFINITY;
+            mx = max_or_nan(mx, S[4 * g + i]);
+        }
     return mx;
 }
-
 // The decode kernel keeps the plain form (every score tested against the end of its kv range): with its two tile bodies the
 // split into a full-tile and an end-of-range variant cost it 10 % at 131072 cells (115 -> 127 us) for 2 % gained at 32768.
 __device__ __forceinline__ float finish_scores_dec(f32x16 &S, const u32x2 (&mw)[4], const fattn_args &a, float scale, float slope,
@@ -378,6 +369,91 @@ __device__ __forceinline__ f32x16 scores(const f16x8 (&qf)[D / 16], const _Float
     return S;
 }
 
+// One row again, as the vector kernel computes it: no term of a masked cell, whatever the cache holds there; f32 probabilities.  By a whole wave,
+// a lane per cell for the scores and per element for the output.
+template <int D, bool PX>
+__device__ __forceinline__ void exact_row(const fattn_args &a, int64_t hk, int64_t head, int64_t iq, float slope, float scale, int lane) {
+    constexpr int E = (D + 63) / 64;
+    const float *qp = (const float *)(a.q + iq * a.q_nb1 + head * a.q_nb2);
+    const unsigned short *mrow = a.mask ? (const unsigned short *)(a.mask + iq * a.mask_nb1) : nullptr;
+    const uint8_t *kh = a.k + hk * a.k_nb2, *vh = a.v + hk * a.v_nb2;
+    float m = FM_NEG, l = 0.0f, acc[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) acc[e] = 0.0f;
+#pragma unroll 1
+    for (int64_t c0 = 0; c0 < a.Nkv; c0 += 64) {
+        const int64_t c = c0 + lane;
+        const float mv = c >= a.Nkv ? -INFINITY : mrow ? half_bits_to_float(mrow[c]) : 0.0f;
+        const bool valid = mv != -INFINITY;
+        const uint64_t live = __ballot(valid);
+        float s = FM_NEG;
+        if (valid) {
+            float dot = 0.0f;
+#pragma unroll 1
+            for (int ch = 0; ch < D / 8; ch++) {
+                const f16x8 kk = *(const f16x8 *)(kh + c * a.k_nb1 + 16 * ch);
+#pragma unroll
+                for (int i = 0; i < 8; i++) dot = fmaf((float)(_Float16)qp[8 * ch + i], (float)kk[i], dot);
+            }
+            s = dot * scale;
+            if (a.softcap != 0.0f) s = a.softcap * tanhf(s);
+            s += slope * mv;
+        }
+        const float m_new = fmaxf(m, wave_max(s)), f = __expf(m - m_new), p = valid ? __expf(s - m_new) : 0.0f;
+        l = l * f + wave_sum(p);
+        m = m_new;
+#pragma unroll
+        for (int e = 0; e < E; e++) acc[e] *= f;
+#pragma unroll 1
+        for (uint64_t w = live; w != 0; w &= w - 1) {
+            const int j = __builtin_ctzll(w);
+            const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), j));
+            const _Float16 *vp = (const _Float16 *)(vh + (c0 + j) * a.v_nb1);
+#pragma unroll
+            for (int e = 0; e < E; e++)
+                if (64 * e + lane < D) acc[e] = fmaf(pj, (float)vp[64 * e + lane], acc[e]);
+        }
+    }
+    float *dp = a.dst + (iq * a.Hq + head) * D;
+#pragma unroll
+    for (int e = 0; e < E; e++)
+        if (64 * e + lane < D) dp[64 * e + lane] = !PX && l == 0.0f ? 0.0f : acc[e] / l;
+}
+
+// The finished rows of a wave.  The matrix instructions multiply every cell of a tile that some query of the 32 sees, for the others by a
+// probability of 0; where the cache holds something that is not finite (a cell never written, or of another sequence) that is NaN and not 0.
+// Such a column cannot hide: its sum or an element is not finite.  It is computed again by exact_row, as is one whose result is rightly so.
+template <int D, bool PX, int NDT>
+__device__ __forceinline__ void store_rows(const fattn_args &a, const f32x16 (&o)[NDT], float l, int64_t hk, int64_t head, int64_t q0, float slope, float scale,
+                                           int lane) {
+    const int l32 = lane & 31, lhi = lane >> 5;
+    float z = l * 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            if (32 * dt + 8 * (r >> 2) < D) z = fmaf(o[dt][r], 0.0f, z);
+    const bool live = q0 + l32 < a.Nq;
+    const uint64_t bad = __ballot(live && z != 0.0f);
+    u32 again = (u32)bad | (u32)(bad >> 32);   // columns
+    if (live && ((again >> l32) & 1) == 0) {
+        const float sum = sum_of<PX>(l), inv = reciprocal_of<PX>(sum);
+        float *dp = a.dst + ((q0 + l32) * a.Hq + head) * D;
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                if (32 * dt + 8 * g >= D) continue;
+                f32x4 w;
+#pragma unroll
+                for (int i = 0; i < 4; i++) w[i] = quotient<PX>(o[dt][4 * g + i], sum, inv);
+                *(f32x4 *)(dp + 32 * dt + 8 * g + 4 * lhi) = w;
+            }
+    }
+#pragma unroll 1
+    for (; again != 0; again &= again - 1) exact_row<D, PX>(a, hk, head, q0 + __builtin_ctz(again), slope, scale, lane);   // uniform
+}
+
 // ---- prefill --------------------------------------------------------------------------------
 // How far each tile of 32 queries can see: extent[t] = 1 + the last cell whose mask entry is not -inf in any of the tile's
 // rows (0 when there is none).  With llama.cpp's causal mask the tiles of a prompt see a growing prefix of the cache, and the
@@ -497,15 +573,13 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             S[u] = scores<D, false, PX ? fm_px_chains<D>() : 1>(qf, sK, u, l32, lhi);
-            mx = fmaxf(mx, finish_scores(S[u], mcur[u], a, scale, slope, kv0 + 32 * u, lhi, a.Nkv));
+            mx = max_or_nan(mx, finish_scores(S[u], mcur[u], a, scale, slope, kv0 + 32 * u, lhi, a.Nkv));
         }
-        mx = half_pair_max(mx);
-        if (__ballot(mx > FM_NEG) == 0) continue;   // every cell of the tile is masked for all 32 queries (wave-uniform)
+        mx = half_pair_max_or_nan(mx);
+        if (__ballot(!(mx <= FM_NEG)) == 0) continue;   // every cell of the tile is masked for all 32 queries (wave-uniform)
         const float m_new = lazy_max<PX>(m, mx);
         const float alpha = rescale<PX>(m, m_new);   // exactly 1 while the reference point stays
-        // dropped scores are exactly FM_NEG: exp(FM_NEG - m) is 0 for any real maximum; a column that has seen no cell yet
-        // (maximum still FM_NEG) subtracts 0 instead, so its dropped scores give 0 as well and not exp(0)
-        const float m2 = m_new > FM_NEG ? exponent_of<PX>(m_new) : 0.0f;
+        const float m2 = exponent_of<PX>(m_new);   // finite also for a column that has seen no cell yet: exp(-inf) is 0 there too
         float rs = 0.0f;
 #pragma unroll
         for (int u = 0; u < 2; u++)
@@ -531,20 +605,7 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
         }
     }
 
-    if (q0 + l32 < a.Nq) {
-        const float sum = sum_of<PX>(l), inv = reciprocal_of<PX>(sum);
-        float *dp = a.dst + ((q0 + l32) * a.Hq + head) * D;
-#pragma unroll
-        for (int dt = 0; dt < NDT; dt++)
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                if (32 * dt + 8 * g >= D) continue;
-                f32x4 w;
-#pragma unroll
-                for (int i = 0; i < 4; i++) w[i] = quotient<PX>(o[dt][4 * g + i], sum, inv);
-                *(f32x4 *)(dp + 32 * dt + 8 * g + 4 * lhi) = w;
-            }
-    }
+    store_rows<D, PX, NDT>(a, o, l, hk, head, q0, slope, scale, lane);
 }
 
 // ---- prefill with few query tiles: the 32-cell parts of every K/V tile go to different waves -----------------------------------
@@ -623,13 +684,11 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
         f32x16 &S = S1[0];
         S = scores<D, (D <= 128), PX ? fm_px_chains<D>() : 1>(qf, sK, u, l32, lhi);
         float mx = finish_scores(S, mcur, a, scale, slope, kv0 + 32 * u, lhi, a.Nkv);
-        mx = half_pair_max(mx);
-        if (__ballot(mx > FM_NEG) == 0) continue;   // all 32 cells masked for all 32 queries (wave-uniform; barriers are at the loop head)
+        mx = half_pair_max_or_nan(mx);
+        if (__ballot(!(mx <= FM_NEG)) == 0) continue;   // all 32 cells masked for all 32 queries (wave-uniform; barriers are at the loop head)
         const float m_new = lazy_max<PX>(m, mx);
         const float alpha = rescale<PX>(m, m_new);   // exactly 1 while the reference point stays
-        // dropped scores are exactly FM_NEG: exp(FM_NEG - m) is 0 for any real maximum; a column that has seen no cell yet
-        // (maximum still FM_NEG) subtracts 0 instead, so its dropped scores give 0 as well and not exp(0)
-        const float m2 = m_new > FM_NEG ? exponent_of<PX>(m_new) : 0.0f;
+        const float m2 = exponent_of<PX>(m_new);   // finite also for a column that has seen no cell yet: exp(-inf) is 0 there too
         float rs = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
@@ -678,19 +737,8 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
                 for (int r = 0; r < 16; r++) o[dt][r] = o[dt][r] * f0 + mg[(32 * dt + 8 * (r >> 2) + 4 * lhi + (r & 3)) * 32 + l32] * f1;
         }
     }
-    if (u != 0 || q0 + l32 >= a.Nq) return;
-    const float sum = sum_of<PX>(l), inv = reciprocal_of<PX>(sum);
-    float *dp = a.dst + ((q0 + l32) * a.Hq + head) * D;
-#pragma unroll
-    for (int dt = 0; dt < NDT; dt++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            if (32 * dt + 8 * g >= D) continue;
-            f32x4 w;
-#pragma unroll
-            for (int i = 0; i < 4; i++) w[i] = quotient<PX>(o[dt][4 * g + i], sum, inv);
-            *(f32x4 *)(dp + 32 * dt + 8 * g + 4 * lhi) = w;
-        }
+    if (u != 0) return;
+    store_rows<D, PX, NDT>(a, o, l, hk, head, q0, slope, scale, lane);
 }
 
 template <int D, bool PQ, bool PX>

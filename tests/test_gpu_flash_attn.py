@@ -318,3 +318,72 @@ def test_decode_short_cache_many_kv_heads(dev, Hq, Hkv, Nkv):
     dst, act = mi355.flash_attn_ext(*args, 0.09, quantized=True)
     assert orc.nmse(dst.cpu().numpy(), _textbook(q, k, v, mask, 0.09)) < 1e-6
     assert torch.equal(act, mi355.quantize_act(dst.reshape(1, Hq * 128)))
+
+
+@pytest.mark.parametrize("D,quantized", [(64, False), (80, False), (96, False), (112, False), (128, False), (256, False), (64, True), (128, True)])
+@pytest.mark.parametrize("Nq,Nkv,Hq,Hkv", [(300, 1100, 8, 2), (200, 520, 12, 12), (600, 640, 32, 8), (40, 600, 70, 70)])
+def test_prefill_non_finite_masked_cells(dev, D, quantized, Nq, Nkv, Hq, Hkv):
+    """-inf mask entries contribute nothing, whatever the cache holds there: NaN and infinities in K and V of masked cells, in tiles that some
+    queries see in part and in tiles nobody sees, against the same call on a cache with zeros in their place"""
+    import torch
+    import mi355
+    rng = np.random.default_rng(D + Nq)
+    q, k, v, mask = _inputs(rng, D, Nq, Nkv, Hq, Hkv)
+    scale = 1.0 / np.sqrt(D)
+    dead = np.concatenate([np.arange(70, 75), np.arange(128, 192), [5, 233]])     # never written: masked for everybody, a whole tile among them
+    mask[:, dead] = -np.inf
+    stale = np.arange(Nkv - Nq + 1, Nkv)                                           # causal: masked for the queries before them
+    late = stale[-Nq // 3:]
+    mask[:, late] = -np.inf                                                        # ... and the last ones for everybody
+    k[:, np.concatenate([dead, late])], v[:, np.concatenate([dead, late])] = 0, 0
+    clean = [torch.from_numpy(a).to(dev) for a in (q, k, v, mask)]
+    bad_k, bad_v = k.copy(), v.copy()
+    for i, c in enumerate(np.concatenate([dead, late])):
+        bad_k[:, c, i % D], bad_v[:, c, (3 * i) % D] = (np.nan, np.inf, -np.inf)[i % 3], (np.inf, np.nan, -np.inf, np.nan)[i % 4]
+    dirty = [clean[0], torch.from_numpy(bad_k).to(dev), torch.from_numpy(bad_v).to(dev), clean[3]]
+    want, got = (mi355.flash_attn_ext(*x, scale, quantized=quantized) for x in (clean, dirty))
+    want, got = ((x[0] if quantized else x).cpu().numpy() for x in (want, got))
+    assert np.isfinite(got).all()
+    f16 = D in (64, 128) and not quantized                  # f16 probabilities on clean tiles, f32 where a row is computed again
+    assert orc.nmse(got, want) < (1e-6 if f16 else 1e-12)
+    assert orc.nmse(got, _textbook(q, k, v, mask, scale)) < (1e-6 if f16 else 1e-12)
+
+
+@pytest.mark.parametrize("D,quantized", [(64, False), (80, False), (112, False), (128, False), (256, False), (128, True)])
+@pytest.mark.parametrize("max_bias,softcap", [(0.0, 0.0), (8.0, 0.0), (0.0, 10.0)])
+def test_prefill_non_finite_visible_cells(dev, D, quantized, max_bias, softcap):
+    """a NaN key or value of a visible cell, and an infinite value, reach exactly the rows that see them (f32 reference on the CPU)"""
+    import torch
+    import mi355
+    rng = np.random.default_rng(D)
+    Hq, Hkv, Nq, Nkv = 40, 8, 70, 530
+    q, k, v, mask = _inputs(rng, D, Nq, Nkv, Hq, Hkv)
+    scale = 1.0 / np.sqrt(D)
+    k[1, Nkv - 30, 7] = np.nan          # seen by the last 30 queries
+    v[2, Nkv - 20, 3] = np.inf
+    v[3, Nkv - 10, 5] = np.nan
+    got = mi355.flash_attn_ext(*(torch.from_numpy(a).to(dev) for a in (q, k, v, mask)), scale, max_bias, softcap, quantized=quantized)
+    got = (got[0] if quantized else got).cpu().numpy()
+    nan, inf = np.zeros((Nq, Hq, D), bool), np.zeros((Nq, Hq, D), bool)
+    g = Hq // Hkv
+    nan[Nq - 30:, g:2 * g] = True
+    inf[Nq - 20:, 2 * g:3 * g, 3] = True
+    nan[Nq - 10:, 3 * g:4 * g, 5] = True
+    assert np.array_equal(np.isnan(got), nan) and np.array_equal(np.isposinf(got), inf)
+    k[1, Nkv - 30, 7], v[2, Nkv - 20, 3], v[3, Nkv - 10, 5] = 0, 0, 0
+    f64 = orc.flash_attn("f64", q, k.view(np.uint16), v.view(np.uint16), mask.view(np.uint16), scale, max_bias, softcap)
+    keep = ~np.isnan(got).any(axis=(2,)) & ~np.isinf(got).any(axis=(2,))
+    assert orc.nmse(got[keep], f64[keep]) < 1e-5
+
+
+@pytest.mark.parametrize("D", [64, 80, 96, 112, 128, 256])
+@pytest.mark.parametrize("max_bias,softcap,masked", [(8.0, 0.0, True), (0.0, 10.0, True), (0.0, 0.0, False), (0.0, 10.0, False)])
+def test_prefill_alibi_softcap_no_mask(dev, D, max_bias, softcap, masked):
+    rng = np.random.default_rng(D + 1)
+    Hq, Hkv, Nq, Nkv = 24, 8, 100, 530
+    q, k, v, mask = _inputs(rng, D, Nq, Nkv, Hq, Hkv, causal=False, rand_mask=True)
+    mask = mask if masked else None
+    scale = 1.0 / np.sqrt(D)
+    got = _run(dev, q, k, v, mask, scale, max_bias, softcap)
+    f64 = orc.flash_attn("f64", q, k.view(np.uint16), v.view(np.uint16), None if mask is None else mask.view(np.uint16), scale, max_bias, softcap)
+    assert orc.nmse(got, f64) < 1e-5         # q's f16 rounding
