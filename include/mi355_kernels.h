@@ -352,7 +352,8 @@ int mi355_mul_mat_id_skinny_q8k(void *stream, int type, const void *as, const vo
 /* The same for experts of the per-32-block types (Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL, Q8_0) and, at the precision of Q8_1 activations, of
  * Q6_K and IQ4_XS: the routed form of mi355_mul_mat_q's tile kernel on 128-slot column tiles.  `act` holds the nb1*T rows of b in the mi355_quantize_act (Q8_1) layout; route_ws as above.
  * K a multiple of the block size, the stack at an even address, at most 256 experts (mi355_mul_mat_id_q_supported);
- * mi355_mul_mat_id picks this path from 32 slots on (Q6_K and IQ4_XS: where their rows are no multiple of 16 bytes). */
+ * mi355_mul_mat_id picks this path from 32 slots on where the weight-streaming form above is not ahead (more than 32 slots per expert on average, or more than 1024 in all; Q6_K and IQ4_XS:
+ * where their rows are no multiple of 16 bytes). */
 int mi355_mul_mat_id_q_supported(int type, const void *as, int64_t N, int64_t K, int64_t n_expert);
 int mi355_mul_mat_id_q(void *stream, int type, const void *as, const void *act, const int32_t *ids, int64_t ids_stride, float *dst,
                        int64_t N, int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T, void *route_ws,

@@ -10,8 +10,8 @@ using namespace mi355;
 
 extern "C" {
 
-// Above this many (token, expert slot) pairs the slots are sorted by expert and run through the tile kernel,
-// which reads every expert's matrix once; below it each slot streams its expert's matrix through the GEMV.
+// From this many (token, expert slot) pairs on the slots may be sorted by expert and run through the routed tile kernels, which read every
+// expert's matrix once; with fewer each slot streams its expert's matrix through the GEMV.  use_skinny takes calls from both.
 static constexpr int64_t ROUTED_MIN_SLOTS = 32;   // measured cross-over on 8 experts of 14336 x 4096
 
 static bool use_routed_tiles(int type, const void *as, int64_t N, int64_t K, int64_t n_expert, int64_t n_used, int64_t T) {
@@ -29,6 +29,9 @@ static bool use_routed_tiles(int type, const void *as, int64_t N, int64_t K, int
 // 65 / 78 / 192 / 304; 16 experts of 2048 x 2048, 256 slots: 63 against 28; IQ4_XS 226 / 225 / 235 / 253 against 75 / 86 / 172 / 278); for the
 // types whose routed kernel has 64-column tiles (routed, Q4_K and Q6_K) up to 16 (Q4_K, 32 / 64 / 128 / 256 slots: 147 / 146 / 149 / 154 us
 // against 72 / 91 / 130 / 192; Q6_K 211 / 212 / 221 / 228 against 112 / 130 / 168 / 257).
+// Those figures are for slots spread evenly.  Choices by Zipf's law: 8 experts of 14336 x 4096, 128 slots, Q4_K 134 us routed, 124 streamed; 256 of
+// 512 x 2048, 8 per token, 1024 slots 89 / 51.  All tokens choosing the same two (eight) experts, where the routed kernel has full tiles: 8 experts, 64 /
+// 128 slots Q4_K 56 / 58 routed, 47 / 68 streamed, Q4_0 148 / 154 against 44 / 67; 256 experts, 1024 slots Q4_K 40 / 50, Q6_K 43 / 73, Q4_0 100 / 52.
 static bool use_skinny(int type, const void *as, int64_t K, int64_t n_expert, int64_t n_used, int64_t T, bool routed) {
     const int64_t S = T * n_used;
     const int64_t most = routed && (type == MI355_Q4_K || type == MI355_Q6_K) ? 16 : 32;

@@ -87,8 +87,8 @@ template <int TYPE, int NI, int HALVES> struct sk_regs {
 // The group's four waves split the slice's steps.  TAIL: K is no multiple of 256 (per-32-block types; a form of its own, since the branch
 // and its registers cost the others 7 %: Q8_0 28672 x 8192, 8 rows, 53.7 -> 57.6 us).
 //
-// ID: MUL_MAT_ID with a few slots per expert.  grid.z = experts; a group collects its expert's (token, expert slot) pairs from the ids
-// itself (at most SK_MAX_SLOTS of them in all: two reads of a few KiB from L2, no routing launch) and takes them 8 NI columns at a time,
+// ID: MUL_MAT_ID with a few slots per expert.  grid.y = experts, grid.z = groups that share an expert's passes (skinny_id_groups); a group
+// collects its expert's (token, expert slot) pairs from the ids itself (at most SK_MAX_SLOTS of them in all: two reads of a few KiB from L2, no routing launch) and takes them 8 NI columns at a time,
 // so that an expert's matrix is read from memory once however many slots chose it; the passes over further columns find their 32 rows in L2.
 constexpr int SK_MAX_SLOTS = 1024;
 struct sk_id {
@@ -133,27 +133,58 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
 
     __shared__ unsigned short s_slot[ID ? SK_MAX_SLOTS : 1];
     int n_cols = B;
+    int c_lo = 0;   // ID: first column of the pass
     if constexpr (ID) {
-        __shared__ int s_n;
-        if (threadIdx.x == 0) s_n = 0;
-        __syncthreads();
-        for (int sl = threadIdx.x; sl < id.n_slots; sl += 256) {
-            int ex = id.ids[(int64_t)(sl / id.n_used) * id.ids_stride + sl % id.n_used];
-            ex = ex < 0 ? 0 : (ex >= (int)gridDim.z ? (int)gridDim.z - 1 : ex);   // never index outside the expert stack
-            if (ex == (int)blockIdx.z) s_slot[atomicAdd(&s_n, 1)] = (unsigned short)sl;   // (any order: a column's sums do not depend on its neighbours)
+        auto expert_of = [&](unsigned sl) {
+            const unsigned t = sl / (unsigned)id.n_used;
+            const int ex = id.ids[t * id.ids_stride + (sl - t * (unsigned)id.n_used)];
+            return ex < 0 ? 0 : (ex >= (int)gridDim.y ? (int)gridDim.y - 1 : ex);   // never index outside the expert stack
+        };
+        constexpr int ROUNDS = SK_MAX_SLOTS / 256;
+        __shared__ int s_hits[ROUNDS][4];
+        if (!Q8K || gridDim.z == 1) {   // any order: a column's sums do not depend on its neighbours
+            if (threadIdx.x == 0) s_hits[0][0] = 0;
+            __syncthreads();
+            for (unsigned sl = threadIdx.x; sl < (unsigned)id.n_slots; sl += 256)
+                if (expert_of(sl) == (int)blockIdx.y) s_slot[atomicAdd(&s_hits[0][0], 1)] = (unsigned short)sl;
+            __syncthreads();
+            n_cols = s_hits[0][0];
+        } else {   // ascending, so that the groups that share an expert's passes agree on their columns
+            uint64_t hit[ROUNDS];
+#pragma unroll
+            for (int i = 0; i < ROUNDS; i++) {
+                const unsigned sl = (unsigned)(i * 256) + threadIdx.x;
+                hit[i] = __ballot(sl < (unsigned)id.n_slots && expert_of(sl) == (int)blockIdx.y);
+                if (lane == 0) s_hits[i][wave] = __popcll(hit[i]);
+            }
+            __syncthreads();
+            int at[ROUNDS];
+            n_cols = 0;
+#pragma unroll
+            for (int i = 0; i < ROUNDS; i++)
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    if (w == wave) at[i] = n_cols;
+                    n_cols += s_hits[i][w];
+                }
+#pragma unroll
+            for (int i = 0; i < ROUNDS; i++)
+                if ((hit[i] >> lane) & 1) s_slot[at[i] + __popcll(hit[i] & ((1ull << lane) - 1))] = (unsigned short)(i * 256 + threadIdx.x);
+            __syncthreads();
         }
-        __syncthreads();
-        n_cols = __builtin_amdgcn_readfirstlane(s_n);
-        if (n_cols == 0) return;   // uniform for the whole group
-        W += (int64_t)blockIdx.z * id.expert_bytes;
+        n_cols = __builtin_amdgcn_readfirstlane(n_cols);
+        c_lo = (int)blockIdx.z * (8 * NI);
+        if (n_cols <= c_lo) return;   // uniform for the whole group
+        W += (int64_t)blockIdx.y * id.expert_bytes;
     }
+    const int slice = ID ? 0 : (int)blockIdx.y;
 
     const row_layout L = make_row_layout(TYPE, K);
     const int nsteps = TAIL ? (K + 255) >> 8 : K >> 8;
     const int nblk = K >> 5;
     const int64_t row0 = (int64_t)blockIdx.x * 32;
 
-    const int slice_lo = blockIdx.y * steps_per_slice;
+    const int slice_lo = slice * steps_per_slice;
     const int slice_hi = slice_lo + steps_per_slice < nsteps ? slice_lo + steps_per_slice : nsteps;
     const int s_lo = slice_lo + wave * steps_per_wave;
     const int s_hi = s_lo + steps_per_wave < slice_hi ? s_lo + steps_per_wave : slice_hi;   // may be <= s_lo: a wave without steps
@@ -177,7 +208,6 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
     }
     const int64_t my_row = row0 + r < N ? row0 + r : N - 1;
     const uint8_t *w_mine = W + my_row * L.row_bytes;   // the row whose results this lane holds: its scales go to registers
-    int c_lo = 0;   // ID: first column of the pass
     auto act_row = [&](int i) -> int64_t {   // activation row of column i of the pass; columns past the end repeat the last one
         const int c = c_lo + i < n_cols ? c_lo + i : n_cols - 1;
         if constexpr (!ID) return c;
@@ -611,12 +641,12 @@ __global__ void __launch_bounds__(256) k_mm_skinny(const uint8_t *__restrict__ W
         const int q = v >> 2, i = v & 3;
         const int c = c_lo + 8 * q + 4 * kh + i;
         if (c < n_cols && row0 + r < N) {
-            const int64_t o = (ID ? (int64_t)s_slot[c] : (int64_t)blockIdx.y * B + c) * dst_stride + row0 + r;
+            const int64_t o = (ID ? (int64_t)s_slot[c] : (int64_t)slice * B + c) * dst_stride + row0 + r;
             dst[o] = residual ? sum + residual[o] : sum;
         }
     }
     if constexpr (ID) __syncthreads();   // the partial sums have been read: the next pass reuses the memory
-    c_lo += 8 * NI;
+    c_lo += ID ? 8 * NI * (int)gridDim.z : 8 * NI;
     } while (ID && c_lo < n_cols);
 }
 
@@ -661,10 +691,19 @@ void launch_skinny_nt(hipStream_t s, const void *W, const int8_t *aq, const act_
     else launch_skinny<TYPE, 4>(s, W, aq, ads, dst, residual, N, K, B, dst_stride, slices, part);
 }
 
+// Groups that share an expert's passes over its columns (Q8K form; the routed tile kernels of the other types are slower than one group's
+// passes).  A token chooses an expert once, so an expert has up to T columns where the average leaves it T n_used / n_expert: with one group
+// per expert and row tile its passes run one after the other while the others' compute units idle.  Every token choosing the same two of 16
+// experts of 2048 x 2048, 256 slots, one / two groups / routed tile kernel: Q4_K 31.0 / 25.0 / 27.0 us, Q6_K 37.2 / 28.7 / 30.0.  The second groups
+// find nothing to do where the slots are spread: 25.5 -> 26.3 us there, but 48 -> 53 at 64 experts of 1024 x 2048 and 45 -> 55 at 256 of
+// 512 x 2048, 1024 slots (one group, the same eight experts for every token: 33.6 and 50 us; routed 31 and 40, spread 55 and 100); up to 64 tokens
+// one group is ahead of the routed kernel in either case.
+int skinny_id_groups(int64_t N, int64_t n_expert, int64_t T) { return T > 64 && (N + 31) / 32 * n_expert <= 1024 ? 2 : 1; }
+
 template <int TYPE, int NI>
 void launch_skinny_id(hipStream_t s, const void *as, const int8_t *aq, const act_ds *ads, float *dst, int64_t N, int K, int64_t n_expert, const sk_id &id) {
     const int nsteps = (K + 255) >> 8;
-    const dim3 grid((unsigned)((N + 31) / 32), 1, (unsigned)n_expert);
+    const dim3 grid((unsigned)((N + 31) / 32), (unsigned)n_expert);
     constexpr bool BLOCKS32 = (sk_traits<TYPE>::NIB32 && TYPE != MI355_IQ4_XS) || TYPE == MI355_Q8_0;
     if (BLOCKS32 && K % 256 != 0)
         MI355_LAUNCH((k_mm_skinny<TYPE, NI, BLOCKS32, true>), grid, dim3(256), 0, s, (const uint8_t *)as, aq, ads, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id, sk_q8k{});
@@ -675,7 +714,7 @@ void launch_skinny_id(hipStream_t s, const void *as, const int8_t *aq, const act
 template <int TYPE, int NI>
 void launch_skinny_id_q8k(hipStream_t s, const void *as, const int8_t *aq, const sk_q8k &q8, float *dst, int64_t N, int K, int64_t n_expert, const sk_id &id) {
     const int nsteps = K >> 8;
-    MI355_LAUNCH((k_mm_skinny<TYPE, NI, false, true, true>), dim3((unsigned)((N + 31) / 32), 1, (unsigned)n_expert), dim3(256), 0, s, (const uint8_t *)as, aq,
+    MI355_LAUNCH((k_mm_skinny<TYPE, NI, false, true, true>), dim3((unsigned)((N + 31) / 32), (unsigned)n_expert, (unsigned)skinny_id_groups(N, n_expert, id.n_slots / id.n_used)), dim3(256), 0, s, (const uint8_t *)as, aq,
                  (const act_ds *)nullptr, dst, (const float *)nullptr, N, K, 0, N, nsteps, (nsteps + 3) / 4, id, q8);
 }
 

@@ -205,3 +205,34 @@ def test_mul_mat_id_skinny(dev, name, t, n_expert, n_used, bcast, T, pattern):
         torch.cuda.synchronize()
         want = expected_per_expert("cpu", t, Wq, b, np.clip(ids, 0, n_expert - 1), n_expert, n_used, nb1, N)
         assert orc.nmse(got.cpu().numpy(), want) < 1e-11
+
+
+@pytest.mark.parametrize("name,t", [("q4_0", orc.Q4_0), ("q4_k", orc.Q4_K), ("q5_k", orc.Q5_K), ("q6_k", orc.Q6_K), ("iq4_xs", orc.IQ4_XS)])
+@pytest.mark.parametrize("n_expert,n_used,T,N", [(16, 2, 128, 2048), (16, 2, 65, 2080), (256, 4, 66, 128), (256, 4, 66, 129), (5, 3, 300, 33), (5, 3, 64, 33)])
+def test_mul_mat_id_skinny_same_experts_for_all_tokens(dev, name, t, n_expert, n_used, T, N):
+    """every token chooses the same experts, and spread-out routing, where one or two groups share an expert's passes (32-row tiles times
+    experts on both sides of 1024, tokens on both sides of 64): every slot exactly once; exact integer dots, f32 sums over 32 blocks"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    K = 1024
+    rng = np.random.default_rng(N + T)
+    Wq = orc.quantize("oracle", t, (rng.standard_normal((64, K)) * 0.02).astype(np.float32))
+    pick = rng.integers(0, 64, n_expert * N)          # the experts' rows are drawn from 64
+    Wd = mi355.upload_weights(t, torch.from_numpy(Wq[pick]).to(dev))
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    same = np.tile(rng.permutation(n_expert)[:n_used].astype(np.int32), (T, 1))
+    spread = np.stack([rng.permutation(n_expert)[:n_used] for _ in range(T)]).astype(np.int32)
+    forms = [("q8_1", mi355.quantize_act, lib.mi355_mul_mat_id_skinny)]
+    if t != orc.Q4_0:
+        forms.append(("cpu", mi355.quantize_act_q8k, lib.mi355_mul_mat_id_skinny_q8k))
+    for kind, quantize, product in forms:
+        act = quantize(torch.from_numpy(x).to(dev))
+        rows = orc.mul_mat(kind, t, Wq, x)
+        for ids in (same, spread):
+            idd = torch.from_numpy(ids).to(dev)
+            got = torch.full((T, n_used, N), float("nan"), device=dev)
+            mi355.check(product(None, t, Wd.data_ptr(), act.data_ptr(), idd.data_ptr(), n_used, got.data_ptr(), N, K, n_expert, n_used, 1, T))
+            torch.cuda.synchronize()
+            want = rows[np.arange(T)[:, None, None], pick.reshape(n_expert, N)[ids]]
+            assert orc.nmse(got.cpu().numpy(), want) < 1e-11
