@@ -590,7 +590,8 @@ int mi355_flash_attn_ext_quant(void *stream, const float *q, const void *k, cons
     if (frc != MI355_OK) return frc;
     const int R = (int)(Hq / Hkv);
     hipStream_t s = (hipStream_t)stream;
-    if (Nq >= 16) {   // prefill: f16 matrix cores
+    // prefill: f16 matrix cores; a quantized output takes its launch of 16-byte loads from dst (any other address: the vector kernel)
+    if (Nq >= 16 && (act == nullptr || ((uintptr_t)dst & 15) == 0)) {
         const int rc = launch_fattn_mma(s, a, D, ws_bytes);
         // the quantized rows by a launch of their own: a few us, where the vector kernel, which writes them itself, takes ten times as
         // long as the matrix-core one (512 x 512 cells, 32 / 8 heads: 200 against 20 us)

@@ -387,3 +387,30 @@ def test_prefill_alibi_softcap_no_mask(dev, D, max_bias, softcap, masked):
     got = _run(dev, q, k, v, mask, scale, max_bias, softcap)
     f64 = orc.flash_attn("f64", q, k.view(np.uint16), v.view(np.uint16), None if mask is None else mask.view(np.uint16), scale, max_bias, softcap)
     assert orc.nmse(got, f64) < 1e-5         # q's f16 rounding
+
+
+@pytest.mark.parametrize("D,quantized", [(64, True), (128, True), (256, True), (80, False), (128, False)])
+@pytest.mark.parametrize("floats", [1, 2, 3])
+def test_prefill_output_at_any_float_address(dev, D, quantized, floats):
+    """an output that starts at a multiple of 4 bytes only, with and without its quantized form: the rows of the aligned call"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    Nq, Nkv, Hq, Hkv = 130, 200, 32, 8
+    rng = np.random.default_rng(D + floats)
+    q, k, v, mask = (torch.from_numpy(a).to(dev) for a in _inputs(rng, D, Nq, Nkv, Hq, Hkv))
+    want = mi355.flash_attn_ext(q, k, v, mask, 0.1)
+    out = torch.full((Nq * Hq * D + 8,), float("nan"), device=dev)
+    dst = out[floats:floats + Nq * Hq * D]
+    act = torch.empty(int(lib.mi355_act_bytes(Hq * D, Nq)), dtype=torch.uint8, device=dev) if quantized else None
+    ws = torch.empty(int(lib.mi355_flash_attn_ws_bytes(D, Nq, Nkv, Hq)), dtype=torch.uint8, device=dev)
+    es = [t.element_size() for t in (q, k, v, mask)]
+    mi355.check(lib.mi355_flash_attn_ext_quant(None, q.data_ptr(), k.data_ptr(), v.data_ptr(), mask.data_ptr(), dst.data_ptr(), D, Nq, Nkv, Hq, Hkv,
+                                               q.stride(1) * es[0], q.stride(0) * es[0], k.stride(1) * es[1], k.stride(0) * es[1], v.stride(1) * es[2],
+                                               v.stride(0) * es[2], mask.stride(0) * es[3], 0.1, 0.0, 0.0, ws.data_ptr(), ws.numel(),
+                                               act.data_ptr() if quantized else None))
+    torch.cuda.synchronize()
+    assert orc.nmse(dst.cpu().numpy(), want.cpu().numpy().reshape(-1)) < 1e-6           # f16 against f32 probabilities at most
+    assert torch.isnan(out[:floats]).all() and torch.isnan(out[floats + Nq * Hq * D:]).all()
+    if quantized:
+        assert torch.equal(act, mi355.quantize_act(dst.clone().reshape(Nq, Hq * D)))
