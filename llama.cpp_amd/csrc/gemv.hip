@@ -678,12 +678,13 @@ int mi355_mul_mat_vec_q_multi(void *stream, int n_mats, const mi355_gemv_mat *ma
     int64_t total_rows = 0;
     bool loadable = true;
     for (int i = 0; i < n_mats; i++) {
-        MI355_REQUIRE(is_weight_type(mats[i].type) && K > 0 && K < (int64_t(1) << 30) && K % type_block_elems(mats[i].type) == 0, "mul_mat_vec_q: unsupported type %d or K=%lld not a multiple of its block size", mats[i].type, (long long)K);
+        MI355_REQUIRE(is_weight_type(mats[i].type) && K > 0 && K % type_block_elems(mats[i].type) == 0, "mul_mat_vec_q: unsupported type %d or K=%lld not a multiple of its block size", mats[i].type, (long long)K);
         MI355_REQUIRE(mats[i].N > 0 && mats[i].dst_stride >= mats[i].N, "mul_mat_vec_q: bad shape");
-        loadable = loadable && layout_loadable(mats[i].W);
+        MI355_REQUIRE(K < (int64_t(1) << 30) || !layout_aligned(mats[i].W, make_row_layout(mats[i].type, K)), "mul_mat_vec_q: bad shape K=%lld", (long long)K);
+        loadable = loadable && layout_loadable(mats[i].W) && K < (int64_t(1) << 30);
         total_rows += mats[i].N;
     }
-    if (!loadable) {   // a matrix at an odd address: byte-load kernel, one matrix at a time
+    if (!loadable) {   // a matrix at an odd address, rows of 2^30 elements and more: byte-load kernel, one matrix at a time
         for (int i = 0; i < n_mats; i++) {
             int rc = gemv_unaligned((hipStream_t)stream, mats[i].type, mats[i].W, act, mats[i].dst, mats[i].residual, mats[i].N, K, B, mats[i].dst_stride);
             if (rc != MI355_OK) return rc;

@@ -607,6 +607,12 @@ __global__ void __launch_bounds__(256) k_mmq_split_sum(const float *__restrict__
     m.dst[o] = m.residual ? add_rn(acc, m.residual[o]) : acc;
 }
 
+// The kernel reaches the 128 rows of a tile by 32-bit offsets from its first one: K up to some 2^25.  Longer rows run on the byte-load kernels.
+static bool mmq_rows_fit(int type, int64_t K) {
+    const int64_t row = make_row_layout(type, K).row_bytes;
+    return MMQ_BM * (row > K ? row : K) <= (int64_t(1) << 32);
+}
+
 template <int TYPE, int TN>
 static void launch_mmq(hipStream_t s, int n_mats, const mi355_gemv_mat *mats, const void *act, int64_t K, int64_t B, void *ws, size_t ws_bytes) {
     constexpr int BN = 64 * TN;
@@ -649,16 +655,14 @@ static void launch_mmq_tn(hipStream_t s, int n_mats, const mi355_gemv_mat *mats,
 // the routed launch: 128-column tiles over the slot list sorted by expert; the routing workspace is laid out as for the
 // super-block kernel's routed form (act_row[S], dst_row[S], tiles[4 x ((S + 63) / 64 + n_expert)], n_tiles)
 template <int TYPE>
-static void launch_mmq_id(hipStream_t s, const void *as, const void *act, int64_t act_rows, const int32_t *ids, int64_t ids_stride, float *dst, int64_t N,
-                          int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T, void *route_ws) {
+static void launch_mmq_id(hipStream_t s, const void *as, const int8_t *aq, const act_ds *ads, const int32_t *ids, int64_t ids_stride, float *dst, int64_t N, int64_t K,
+                          int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T, void *route_ws) {
     constexpr int BN = 128;
     const int64_t S = T * n_used;
     const int max_tiles = (int)((S + BN - 1) / BN + n_expert);
     int32_t *act_row = (int32_t *)route_ws, *dst_row = act_row + S, *tiles = dst_row + S, *n_tiles = tiles + 4 * ((S + 63) / 64 + n_expert);
     launch_route_slots(s, ids, ids_stride, n_expert, n_used, nb1, T, BN, act_row, dst_row, tiles, n_tiles);
     const row_layout L = make_row_layout(TYPE, K);
-    const int8_t *aq = (const int8_t *)act;
-    const act_ds *ads = (const act_ds *)(aq + act_rows * K);
     const int n_row_tiles = (int)((N + MMQ_BM - 1) / MMQ_BM);
     const int n_groups = n_row_tiles * max_tiles;
     const int n_groups_padded = (n_groups + 7) & ~7;
@@ -675,7 +679,7 @@ using namespace mi355;
 extern "C" int mi355_mul_mat_id_q_supported(int type, const void *as, int64_t N, int64_t K, int64_t n_expert) {
     const bool typed = type == MI355_Q4_0 || type == MI355_Q4_1 || type == MI355_Q5_0 || type == MI355_Q5_1 || type == MI355_IQ4_NL ||
                        type == MI355_Q8_0 || type == MI355_Q6_K || type == MI355_IQ4_XS;
-    if (!typed || N <= 0 || K <= 0 || K >= (int64_t(1) << 24) || K % type_block_elems(type) != 0 || n_expert <= 0 || n_expert > 256) return 0;
+    if (!typed || N <= 0 || K <= 0 || K >= (int64_t(1) << 30) || K % type_block_elems(type) != 0 || n_expert <= 0 || n_expert > 256) return 0;
     return layout_loadable(as) ? 1 : 0;
 }
 
@@ -686,23 +690,19 @@ extern "C" int mi355_mul_mat_id_q(void *stream, int type, const void *as, const 
     MI355_REQUIRE(n_used > 0 && nb1 > 0 && T > 0 && ids_stride >= n_used, "mul_mat_id_q: bad shape");
     MI355_REQUIRE(T * n_used < (1 << 24) && nb1 * T < (1 << 24) && nb1 * T * (K / QK) < (int64_t(1) << 32), "mul_mat_id_q: too many slots");
     MI355_REQUIRE(((uintptr_t)act & 15) == 0, "mul_mat_id_q: activation workspace is not 16-byte aligned");
+    if (!mmq_rows_fit(type, K)) return mi355_mul_mat_id_vec(stream, type, as, act, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T);
     const size_t need = mi355_mul_mat_id_q8k_route_bytes(n_expert, n_used, T);
     if (route_ws == nullptr || route_ws_bytes < need || ((uintptr_t)route_ws & 15) != 0) {
         set_error("mul_mat_id_q: routing workspace of %zu bytes, need %zu (16-byte aligned)", route_ws_bytes, need);
         return MI355_ERR_WORKSPACE;
     }
     hipStream_t s = (hipStream_t)stream;
-    const int64_t rows = nb1 * T;
-    switch (type) {
-        case MI355_Q4_0: launch_mmq_id<MI355_Q4_0>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-        case MI355_Q4_1: launch_mmq_id<MI355_Q4_1>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-        case MI355_Q5_0: launch_mmq_id<MI355_Q5_0>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-        case MI355_Q5_1: launch_mmq_id<MI355_Q5_1>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-        case MI355_Q6_K: launch_mmq_id<MI355_Q6_K>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-        case MI355_IQ4_XS: launch_mmq_id<MI355_IQ4_XS>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-        case MI355_IQ4_NL: launch_mmq_id<MI355_IQ4_NL>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-        default: launch_mmq_id<MI355_Q8_0>(s, as, act, rows, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-    }
+    const int8_t *aq = (const int8_t *)act;
+    const act_ds *ads = (const act_ds *)(aq + nb1 * T * K);
+#define X(TY) \
+    case TY: launch_mmq_id<TY>(s, as, aq, ads, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
+    switch (type) { X(MI355_Q4_0) X(MI355_Q4_1) X(MI355_Q5_0) X(MI355_Q5_1) X(MI355_Q6_K) X(MI355_IQ4_XS) X(MI355_IQ4_NL) X(MI355_Q8_0) }
+#undef X
     return launch_status("k_mmq (routed)");
 }
 
@@ -729,18 +729,18 @@ extern "C" int mi355_mul_mat_q_multi(void *stream, int type, int n_mats, const m
                                      size_t ws_bytes) {
     MI355_REQUIRE(is_weight_type(type), "mul_mat_q: unsupported weight type %d", type);
     MI355_REQUIRE(n_mats >= 1 && n_mats <= MMQ_MATS, "mul_mat_q: 1..%d matrices per launch, got %d", MMQ_MATS, n_mats);
-    MI355_REQUIRE(K > 0 && B > 0 && K < (int64_t(1) << 24), "mul_mat_q: bad shape K=%lld B=%lld", (long long)K, (long long)B);
+    MI355_REQUIRE(K > 0 && B > 0, "mul_mat_q: bad shape K=%lld B=%lld", (long long)K, (long long)B);
     MI355_REQUIRE(K % type_block_elems(type) == 0, "mul_mat_q: K=%lld is not a multiple of the block size", (long long)K);
     int64_t row_tiles = 0;
-    bool loadable = true;
+    bool fit = mmq_rows_fit(type, K);
     for (int i = 0; i < n_mats; i++) {
         MI355_REQUIRE(mats[i].type == type, "mul_mat_q: the matrices of a launch have one type");
         MI355_REQUIRE(mats[i].N > 0, "mul_mat_q: bad shape N=%lld", (long long)mats[i].N);
         MI355_REQUIRE(mats[i].dst_stride >= mats[i].N, "mul_mat_q: dst_stride < N");
         row_tiles += (mats[i].N + MMQ_BM - 1) / MMQ_BM;
-        loadable = loadable && layout_loadable(mats[i].W);
+        fit = fit && layout_loadable(mats[i].W);
     }
-    if (!loadable) {   // a matrix at an odd address
+    if (!fit) {   // a matrix at an odd address, rows beyond 32-bit offsets
         for (int i = 0; i < n_mats; i++) {
             const int rc = gemv_unaligned((hipStream_t)stream, type, mats[i].W, act, mats[i].dst, mats[i].residual, mats[i].N, K, B, mats[i].dst_stride);
             if (rc != MI355_OK) return rc;

@@ -629,3 +629,37 @@ def test_mul_mat_q_multi(dev, name, t, K, B):
         torch.cuda.synchronize()
         for d, w in zip(dst, want):
             assert orc.nmse(d.cpu().numpy(), w) < 1e-11, nws
+
+
+@pytest.mark.parametrize("name,t", [("q4_0", orc.Q4_0), ("q8_0", orc.Q8_0)])
+@pytest.mark.parametrize("K", [(1 << 24) + 96, (1 << 25) + 128])
+def test_batches_over_very_long_rows(dev, name, t, K):
+    """rows on both sides of what the tile kernel's 32-bit offsets reach, as a batch and through experts: integer weights and activations with
+    scales of 1, exact block dots; f32 sums of 2^20 blocks whose magnitude grows with the square root leave some 2^-24 * 2^10 of the result"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    N, B, lim = 3, 33, (7 if t == orc.Q4_0 else 127)
+    g = torch.Generator(device=dev).manual_seed(1)
+    W = torch.randint(-lim, lim + 1, (N, K), device=dev, generator=g, dtype=torch.int32).float()
+    W[:, ::32] = -8 if t == orc.Q4_0 else 127
+    x = torch.randint(-127, 128, (B, K), device=dev, generator=g, dtype=torch.int32).float()
+    # (the first of 32 sets the scale.  Its sign is random: terms of one sign and size are all rounded the same way once a lane's f32 sum is 2^13 times larger)
+    x[:, ::32] = 127 * torch.sign(x[:, 1::32] + 0.5)
+    Wd = mi355.upload_weights(t, mi355.quantize_weights(t, W))
+    act = mi355.quantize_act(x)
+    want = torch.zeros((B, N), dtype=torch.float64, device=dev)
+    for k in range(0, K, 1 << 22):
+        want += x[:, k:k + (1 << 22)].double() @ W[:, k:k + (1 << 22)].double().T.contiguous()
+    del x, W
+    got = torch.full((B, N), float("nan"), device=dev)
+    mi355.check(lib.mi355_mul_mat_q(None, t, Wd.data_ptr(), act.data_ptr(), got.data_ptr(), N, K, B, N))
+    torch.cuda.synchronize()
+    assert orc.nmse(got.cpu().numpy(), want.cpu().numpy()) < 1e-7
+    assert lib.mi355_mul_mat_id_q_supported(t, Wd.data_ptr(), 1, K, N) == 1      # three experts of one row
+    ids = torch.tensor([[b % 3, (b + 1) % 3] for b in range(B)], dtype=torch.int32, device=dev)
+    got = torch.full((B, 2, 1), float("nan"), device=dev)
+    route = torch.empty(int(lib.mi355_mul_mat_id_q8k_route_bytes(N, 2, B)), dtype=torch.uint8, device=dev)
+    mi355.check(lib.mi355_mul_mat_id_q(None, t, Wd.data_ptr(), act.data_ptr(), ids.data_ptr(), 2, got.data_ptr(), 1, K, N, 2, 1, B, route.data_ptr(), route.numel()))
+    torch.cuda.synchronize()
+    assert orc.nmse(got[..., 0].cpu().numpy(), want.gather(1, ids.long()).cpu().numpy()) < 1e-7
