@@ -688,7 +688,7 @@ extern "C" int mi355_mul_mat_id_q(void *stream, int type, const void *as, const 
     MI355_REQUIRE(mi355_mul_mat_id_q_supported(type, as, N, K, n_expert), "mul_mat_id_q: type %d, K=%lld, %lld experts or the weight alignment is not supported",
                   type, (long long)K, (long long)n_expert);
     MI355_REQUIRE(n_used > 0 && nb1 > 0 && T > 0 && ids_stride >= n_used, "mul_mat_id_q: bad shape");
-    MI355_REQUIRE(T * n_used < (1 << 24) && nb1 * T < (1 << 24) && nb1 * T * (K / QK) < (int64_t(1) << 32), "mul_mat_id_q: too many slots");
+    MI355_REQUIRE(T * n_used < (1 << 24) && nb1 * T < (1 << 24), "mul_mat_id_q: too many slots");
     MI355_REQUIRE(((uintptr_t)act & 15) == 0, "mul_mat_id_q: activation workspace is not 16-byte aligned");
     if (!mmq_rows_fit(type, K)) return mi355_mul_mat_id_vec(stream, type, as, act, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T);
     const size_t need = mi355_mul_mat_id_q8k_route_bytes(n_expert, n_used, T);
@@ -699,10 +699,16 @@ extern "C" int mi355_mul_mat_id_q(void *stream, int type, const void *as, const 
     hipStream_t s = (hipStream_t)stream;
     const int8_t *aq = (const int8_t *)act;
     const act_ds *ads = (const act_ds *)(aq + nb1 * T * K);
+    // the kernel counts the activation's blocks in 32 bits: tokens in runs of fewer than 2^32 of them (one run up to 137 GB of activations)
+    const int64_t run = ((int64_t(1) << 32) - 1) / (nb1 * (K / QK));
+    MI355_REQUIRE(run > 0, "mul_mat_id_q: nb1=%lld rows per token are too many", (long long)nb1);
+    for (int64_t t0 = 0; t0 < T; t0 += run) {
+        const int64_t n = T - t0 < run ? T - t0 : run;
 #define X(TY) \
-    case TY: launch_mmq_id<TY>(s, as, aq, ads, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws); break;
-    switch (type) { X(MI355_Q4_0) X(MI355_Q4_1) X(MI355_Q5_0) X(MI355_Q5_1) X(MI355_Q6_K) X(MI355_IQ4_XS) X(MI355_IQ4_NL) X(MI355_Q8_0) }
+    case TY: launch_mmq_id<TY>(s, as, aq + t0 * nb1 * K, ads + t0 * nb1 * (K / QK), ids + t0 * ids_stride, ids_stride, dst + t0 * n_used * N, N, K, n_expert, n_used, nb1, n, route_ws); break;
+        switch (type) { X(MI355_Q4_0) X(MI355_Q4_1) X(MI355_Q5_0) X(MI355_Q5_1) X(MI355_Q6_K) X(MI355_IQ4_XS) X(MI355_IQ4_NL) X(MI355_Q8_0) }
 #undef X
+    }
     return launch_status("k_mmq (routed)");
 }
 

@@ -236,3 +236,31 @@ def test_mul_mat_id_skinny_same_experts_for_all_tokens(dev, name, t, n_expert, n
             torch.cuda.synchronize()
             want = rows[np.arange(T)[:, None, None], pick.reshape(n_expert, N)[ids]]
             assert orc.nmse(got.cpu().numpy(), want) < 1e-11
+
+
+def test_routed_tiles_over_more_than_2_32_activation_blocks(dev):
+    """the last of 2^24 - 1 tokens lie beyond 2^32 blocks: zeros but for the first and last 64, whose levels are all 1"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    t, K, T, N, E = orc.Q8_0, 8320, (1 << 24) - 1, 1, 2
+    if torch.cuda.mem_get_info()[0] < 200 << 30:
+        pytest.skip("needs 174 GB of activations")
+    W = torch.ones((E, K), device=dev) * torch.tensor([[127.0], [254.0]], device=dev)         # levels 127, scales 1 and 2
+    Wd = mi355.upload_weights(t, mi355.quantize_weights(t, W))
+    act = torch.zeros(int(lib.mi355_act_bytes(K, T)), dtype=torch.uint8, device=dev)
+    ends = torch.cat([torch.arange(64), torch.arange(T - 64, T)]).to(dev)
+    act[:T * K].view(T, K)[ends] = 1
+    ds = act[T * K:T * K + T * (K // 32) * 8].view(torch.int32).view(T, K // 32, 2)
+    ds[ends, :, 0] = 0x3F800000                                                                 # scale 1.0f
+    ds[ends, :, 1] = 32
+    ids = torch.arange(T, dtype=torch.int32, device=dev) % E
+    got = torch.full((T,), float("nan"), device=dev)
+    route = torch.empty(int(lib.mi355_mul_mat_id_q8k_route_bytes(E, 1, T)), dtype=torch.uint8, device=dev)
+    mi355.check(lib.mi355_mul_mat_id_q(None, t, Wd.data_ptr(), act.data_ptr(), ids.data_ptr(), 1, got.data_ptr(), N, K, E, 1, 1, T, route.data_ptr(), route.numel()))
+    torch.cuda.synchronize()
+    want = torch.zeros(T, device=dev)
+    want[ends] = 127.0 * K * (1 + ids[ends].float())
+    assert torch.equal(got, want)                                                               # whole numbers below 2^24
+    del act, ds
+    torch.cuda.empty_cache()
