@@ -45,7 +45,12 @@ __device__ __forceinline__ int mmq_chunk(int r, int c) { return r * MMQ_BK + ((c
 // M = 1.5 * 2^23, so that its integer result (|sum| < 2^22: 32 * 127 * 128 at most) read as a float is M + sum, without a conversion.  Then
 //     t = fma(M + sum, dw, -M dw)      = sum * dw rounded once: M * dw is exact, dw has at most 19 significant bits
 //     acc = fma(t, dx, acc)            dx as f16 (what block_q8_1 holds), widened inside the instruction (v_fma_mix_f32)
-// two instructions per sum instead of three (convert, dw * dx shared, fma): see the figures at launch_mmq.
+// two instructions per sum instead of three (convert, dw * dx, fma): see the figures at launch_mmq.  The error against 64-bit arithmetic
+// stays that of three where sum * dw rarely needs more than 24 bits (Q4_0, Q5_0: 2.042e-7, 2.018e-7 of the result at K = 4096 either way; the
+// types with minima gained more by their f32 form).  With levels of eight bits it would grow (Q8_0 2.027e-7 -> 2.037e-7, IQ4_NL 2.026e-7 ->
+// 2.038e-7, IQ4_XS 2.030e-7 -> 2.037e-7), so for those types (mmq_cfg::WIDE) the last stage has sums of its own, which takes at least as much off
+// the rounding of the long ones (it has the registers: nothing is requested any more): 1.994e-7, 1.995e-7, 1.995e-7; K = 1024, three / two
+// instructions / with that: Q8_0 1.030e-7 / 1.055e-7 / 0.979e-7.  Time 114.3 -> 114.8 us (14336 x 4096, 512 rows); three instructions take 137.
 constexpr float MMQ_MAGIC = 12582912.0f;
 constexpr int MMQ_MAGIC_BITS = 0x4B400000;
 
@@ -61,6 +66,8 @@ template <int TYPE> struct mmq_cfg {
     // 16 bytes of nibbles per block with a per-block scale: one request / commit form serves them all
     static constexpr bool NIBBLE32 = TYPE == MI355_Q4_0 || TYPE == MI355_Q4_1 || TYPE == MI355_Q5_0 || TYPE == MI355_Q5_1 || TYPE == MI355_IQ4_NL ||
                                      TYPE == MI355_IQ4_XS;
+    // levels of eight bits: the last stage has sums of its own
+    static constexpr bool WIDE = TYPE == MI355_Q8_0 || TYPE == MI355_IQ4_NL || TYPE == MI355_IQ4_XS;
 };
 
 // ---- a stage is requested (global -> registers) one stage ahead and committed (unpack -> LDS) while the stage before it is contracted
@@ -471,7 +478,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
             if constexpr (NS == 1) return __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[tb], f.w[tw], magic, 0, 0, 0);
             else return __builtin_amdgcn_mfma_i32_32x32x16_i8(pair64(f.a[tb][2 * h], f.a[tb][2 * h + 1]), pair64(f.w[tw][2 * h], f.w[tw][2 * h + 1]), magic, 0, 0, 0);
         };
-        auto scale = [&](const block_scales &f, int n, const i32x16 &I) {
+        auto scale = [&](f32x16 (&acc)[TN][2], const block_scales &f, int n, const i32x16 &I) {
             const int tb = n / NS % TN, tw = n / NS / TN, h = n % NS;
             const float dw = f.dw[tw][h], mdw = -MMQ_MAGIC * dw;
     #pragma unroll
@@ -485,9 +492,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
         commit(sm[0], s_lo);
         fetch(s_lo + 1 < s_hi ? s_lo + 1 : s_lo);
         __syncthreads();
-        int buf = 0;
-        for (int st = s_lo; st < s_hi; st++, buf ^= 1) {
-            const stage_mem &m = sm[buf];
+        auto contract = [&](const stage_mem &m, f32x16 (&acc)[TN][2]) __attribute__((always_inline)) {
             asm volatile("" : "+v"(a_at), "+v"(w_at));   // the four chunk addresses of a stage are formed in the loop: kept across it they cost spills
             // One matrix instruction is always in flight: its successor is issued before its sums are scaled, so that neither waits for the
             // other (left to the compiler, all of them write the same registers one after the other); the next block's operands are read
@@ -505,7 +510,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
                     __builtin_amdgcn_sched_barrier(0);
                     if (n == NM - 2 && ks < 3) f = load_ops(m, ks + 1);
                     if (n == NM - 1 && ks < 3) sc_next = load_scales(m, ks + 1);
-                    scale(sc, n, cur);
+                    scale(acc, sc, n, cur);
                     asm volatile("" : "+v"(acc[n / NS % TN][n / NS / TN]));   // formed here, and not behind the matrix instructions of the whole stage
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -528,11 +533,37 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
                         for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
                 }
             }
+        };
+        int buf = 0, st = s_lo;
+        const bool two = C::WIDE && (nblk & 3) == 1 && s_hi == stages && s_hi - s_lo > 1;   // the last stage holds one block: two stages
+        const int loop_end = C::WIDE ? s_hi - 1 - two : s_hi;
+        for (; st < loop_end; st++, buf ^= 1) {
+            contract(sm[buf], acc);
             if (st + 1 < s_hi) {   // the next stage, requested one stage ago, goes to the other buffer (uniform)
                 commit(sm[buf ^ 1], st + 1);
                 fetch(st + 2 < s_hi ? st + 2 : st + 1);   // past the end the last stage is requested again and never used
                 __syncthreads();
             }
+        }
+        if constexpr (C::WIDE) {   // the last stage on its own sums
+            f32x16 last[TN][2];
+    #pragma unroll
+            for (int tb = 0; tb < TN; tb++)
+    #pragma unroll
+                for (int tw = 0; tw < 2; tw++)
+    #pragma unroll
+                    for (int r = 0; r < 16; r++) last[tb][tw][r] = 0.0f;
+            if (two) {   // (both buffers before the sums: the requested stage's registers make room for them)
+                commit(sm[buf ^ 1], s_hi - 1);
+                __syncthreads();
+            }
+            for (; st < s_hi; st++, buf ^= 1) contract(sm[buf], last);
+    #pragma unroll
+            for (int tb = 0; tb < TN; tb++)
+    #pragma unroll
+                for (int tw = 0; tw < 2; tw++)
+    #pragma unroll
+                    for (int r = 0; r < 16; r++) acc[tb][tw][r] += last[tb][tw][r];
         }
 
         // store: lane holds weight row j = l32 of each 32-wide tile, 16 activation rows

@@ -663,3 +663,54 @@ def test_batches_over_very_long_rows(dev, name, t, K):
     mi355.check(lib.mi355_mul_mat_id_q(None, t, Wd.data_ptr(), act.data_ptr(), ids.data_ptr(), 2, got.data_ptr(), 1, K, N, 2, 1, B, route.data_ptr(), route.numel()))
     torch.cuda.synchronize()
     assert orc.nmse(got[..., 0].cpu().numpy(), want.gather(1, ids.long()).cpu().numpy()) < 1e-7
+
+
+@pytest.mark.parametrize("name,t,bound", [("q8_0", orc.Q8_0, 1.04e-7), ("iq4_nl", orc.IQ4_NL, 1.04e-7), ("iq4_xs", orc.IQ4_XS, 1.04e-7), ("q4_0", orc.Q4_0, 1.04e-7),
+                                          ("q5_0", orc.Q5_0, 1.04e-7)])
+def test_tile_kernel_sums_against_f64(dev, name, t, bound):
+    """the error of the tile kernel's f32 sums over 32 blocks (2-norm, 2 M sums; their own scatter is 0.05 %): block sums converted and multiplied by both scales at
+    once leave 1.030e-7; rounded once more, 1.055e-7 where levels have eight bits"""
+    import torch
+    import mi355
+    rng = np.random.default_rng(1)
+    N, K, B = 4096, 1024, 512
+    Wq = _weights(rng, t, N, K)
+    Wd = mi355.upload_weights(t, _to_dev(dev, Wq))
+    act = mi355.quantize_act(_to_dev(dev, rng.standard_normal((B, K)).astype(np.float32)))
+    a = act[:B * K].view(torch.int8).reshape(B, K // 32, 32).double() * act[B * K:B * K + B * K // 4].view(torch.float32).reshape(B, K // 32, 2)[..., :1].double()
+    want = a.reshape(B, K) @ _to_dev(dev, orc.dequantize("oracle", t, Wq, K)).double().T.contiguous()
+    got = torch.empty((B, N), dtype=torch.float32, device=dev)
+    mi355.check(mi355.load().mi355_mul_mat_q(None, t, Wd.data_ptr(), act.data_ptr(), got.data_ptr(), N, K, B, N))
+    torch.cuda.synchronize()
+    assert float((got.double() - want).norm() / want.norm()) < bound
+
+
+@pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t in (orc.Q8_0, orc.IQ4_NL, orc.IQ4_XS)])
+@pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5, 6, 8, 9, 13, 16, 17, 21])
+def test_tile_kernel_last_stage(dev, name, t, blocks):
+    """one to six stages of four blocks whose last holds one to four, where the last stage, or the last two, are summed on their own; alone and
+    through experts (one column tile, and a second one of a few columns); exact block dots, f32 sums"""
+    import torch
+    import mi355
+    rng = np.random.default_rng(blocks)
+    K, N = (32 if t != orc.IQ4_XS else 256) * blocks, 130
+    Wq = _weights(rng, t, 2 * N, K)
+    Wd = mi355.upload_weights(t, _to_dev(dev, Wq))
+    for B in (33, 65, 130):
+        x = rng.standard_normal((B, K)).astype(np.float32)
+        want = orc.mul_mat("q8_1", t, Wq, x)
+        act = mi355.quantize_act(_to_dev(dev, x))
+        for split in (False, True):
+            need = int(mi355.load().mi355_mul_mat_q_ws_bytes(2 * N, K, B)) if split else 0
+            ws = torch.empty(need + 16, dtype=torch.uint8, device=dev)
+            got = torch.full((B, 2 * N), float("nan"), device=dev)
+            mi355.check(mi355.load().mi355_mul_mat_q_ws(None, t, Wd.data_ptr(), act.data_ptr(), got.data_ptr(), 2 * N, K, B, 2 * N, ws.data_ptr(), need))
+            torch.cuda.synchronize()
+            assert orc.nmse(got.cpu().numpy(), want) < 1e-11, (B, split)
+        ids = torch.arange(B, dtype=torch.int32, device=dev).reshape(B, 1) % 31 // 30          # expert 1: every 31st row
+        route = torch.empty(int(mi355.load().mi355_mul_mat_id_q8k_route_bytes(2, 1, B)), dtype=torch.uint8, device=dev)
+        got = torch.full((B, N), float("nan"), device=dev)
+        mi355.check(mi355.load().mi355_mul_mat_id_q(None, t, Wd.data_ptr(), act.data_ptr(), ids.data_ptr(), 1, got.data_ptr(), N, K, 2, 1, 1, B, route.data_ptr(), route.numel()))
+        torch.cuda.synchronize()
+        pick = ids.cpu().numpy().astype(bool)
+        assert orc.nmse(got.cpu().numpy(), np.where(pick, want[:, N:], want[:, :N])) < 1e-11, B
