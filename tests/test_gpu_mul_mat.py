@@ -714,3 +714,55 @@ def test_tile_kernel_last_stage(dev, name, t, blocks):
         torch.cuda.synchronize()
         pick = ids.cpu().numpy().astype(bool)
         assert orc.nmse(got.cpu().numpy(), np.where(pick, want[:, N:], want[:, :N])) < 1e-11, B
+
+
+@pytest.mark.parametrize("name,t", TYPES)
+@pytest.mark.parametrize("B", [40, 130])
+def test_tile_kernel_infinite_scales(dev, name, t, B):
+    """a weight block whose f16 scale is infinite gives plus or minus infinity by the sign of the block's sum, in its row alone; with and without
+    slices along K, through experts, and beside NaN activation rows, which stay NaN"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    rng = np.random.default_rng(B)
+    be, bb = orc.BLOCK[t]
+    K, N = 2048, 150
+    Wf = (np.abs(rng.standard_normal((N, K))) * 0.02 + 0.002).astype(np.float32)      # one sign: the groups of a super-block agree
+    Wq = orc.quantize("oracle", t, Wf)
+    x = (np.abs(rng.standard_normal((B, K))) + 0.1).astype(np.float32) * np.where(np.arange(B) % 3 == 0, -1, 1)[:, None].astype(np.float32)
+    at = 208 if t == orc.Q6_K else 0                                                     # where a block's f16 scale lies
+    clean = orc.mul_mat("q8_1", t, Wq, x)
+    bad = Wq.copy()
+    want = clean.copy()
+    for row, block, bits in ((3, 0, 0x7C00), (70, K // be // 2, 0xFC00), (149, K // be - 1, 0x7C00)):
+        d = bad[row].reshape(K // be, bb)[block, at:at + 2].view(np.uint16)
+        sign = (-1.0 if d[0] & 0x8000 else 1.0) * (-1.0 if bits & 0x8000 else 1.0)      # the levels carry the sign of the scale they were made for
+        d[0] = bits
+        want[:, row] = np.where(np.arange(B) % 3 == 0, -1, 1) * sign * np.inf
+    Wd = mi355.upload_weights(t, _to_dev(dev, bad))
+    for spoiled in (False, True):
+        act = mi355.quantize_act(_to_dev(dev, x))
+        if spoiled:                                                                      # activation row 5: a NaN scale
+            act[B * K:B * K + B * K // 4].view(torch.float32).reshape(B, K // 32, 2)[5, 7, 0] = float("nan")
+            want[5] = np.nan
+        results = []
+        for split in (False, True):
+            need = int(lib.mi355_mul_mat_q_ws_bytes(N, K, B)) if split else 0
+            ws = torch.empty(need + 16, dtype=torch.uint8, device=dev)
+            got = torch.full((B, N), 1.0, device=dev)
+            m = (mi355.GemvMat * 1)()
+            m[0].type, m[0].W, m[0].N, m[0].dst, m[0].dst_stride, m[0].residual = t, Wd.data_ptr(), N, got.data_ptr(), N, got.data_ptr()
+            mi355.check(lib.mi355_mul_mat_q_multi(None, t, 1, m, act.data_ptr(), K, B, ws.data_ptr() if need else None, need))
+            torch.cuda.synchronize()
+            results.append(got.cpu().numpy() - 1.0)
+        if lib.mi355_mul_mat_id_q_supported(t, Wd.data_ptr(), N, K, 1):
+            ids = torch.zeros((B, 1), dtype=torch.int32, device=dev)
+            route = torch.empty(int(lib.mi355_mul_mat_id_q8k_route_bytes(1, 1, B)), dtype=torch.uint8, device=dev)
+            got = torch.full((B, N), 1.0, device=dev)
+            mi355.check(lib.mi355_mul_mat_id_q(None, t, Wd.data_ptr(), act.data_ptr(), ids.data_ptr(), 1, got.data_ptr(), N, K, 1, 1, 1, B, route.data_ptr(), route.numel()))
+            torch.cuda.synchronize()
+            results.append(got.cpu().numpy())
+        for got in results:
+            finite = np.isfinite(want)
+            assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+            assert orc.nmse(got[finite], want[finite]) < 1e-11
