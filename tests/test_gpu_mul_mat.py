@@ -158,9 +158,7 @@ def test_mmq_matches_oracle(dev, name, t, N, K, B):
         want = orc.mul_mat("cpu", t, Wq[:Nt], x[:Bt])
     else:
         want = orc.mul_mat("q8_1", t, Wq[:Nt], x[:Bt])
-    # Q4_1 / Q5_1 batches add "m * d_x * sum(q)" through fp16 operands (fp16 d_x * sum(q) is the `s` field the reference's own dot
-    # uses); Q5_K batches on packed rows subtract "dmin * m * d_x * sum(q)" the same way
-    assert orc.nmse(got[:Bt, :Nt], want) < (1e-6 if (B > 8 and t in (orc.Q4_1, orc.Q5_1, orc.Q5_K)) else 1e-9)
+    assert orc.nmse(got[:Bt, :Nt], want) < 1e-11      # exact block dots, f32 sums over at most 448 blocks (an f16 block minimum would leave 1e-7)
     if orc.ref is not None:
         cpu = orc.mul_mat("ref", t, Wq, x)
         assert orc.nmse(got, cpu) <= 5e-4
@@ -296,9 +294,8 @@ def test_mmq_llama8b_ffn_shapes(dev, name, t, N, K):
         kind = "cpu" if (kq and (t != orc.IQ4_XS or B >= 256)) else "q8_1"
         corner = orc.mul_mat(kind, t, Wq[:64], x[:24])
         edge = orc.mul_mat(kind, t, Wq[N - 9:], x[B - 3:])
-        tol = 1e-6 if t in (orc.Q4_1, orc.Q5_1, orc.Q5_K) else 1e-9    # the block minimum meets fp16(d_x * sum(q)), as in the reference's dot
-        assert orc.nmse(got[:24, :64], corner) < tol
-        assert orc.nmse(got[B - 3:, N - 9:], edge) < tol
+        assert orc.nmse(got[:24, :64], corner) < 1e-11      # exact block dots, f32 sums over at most 448 blocks
+        assert orc.nmse(got[B - 3:, N - 9:], edge) < 1e-11
         assert orc.ref is not None, "the reference build (oracle/_ref) is the whole-output check of this test"
         want = orc.mul_mat("ref", t, Wq, x, n_threads=16)
         assert orc.nmse(got, want) <= 5e-4
@@ -328,13 +325,13 @@ def test_mmq_q8_1_path_for_k_quants(dev, name, t, N, K, B):
     dst = torch.empty((B, N), dtype=torch.float32, device=dev)
     mi355.check(mi355.load().mi355_mul_mat_q(None, t, Wd.data_ptr(), act.data_ptr(), dst.data_ptr(), N, K, B, N))
     torch.cuda.synchronize()
-    tol = 1e-6 if t == orc.Q4_K else 1e-9    # Q4_K adds its min term through fp16 operands
-    assert orc.nmse(dst.cpu().numpy()[:24, :64], orc.mul_mat("q8_1", t, Wq[:64], x[:24])) < tol
+    assert orc.nmse(dst.cpu().numpy()[:24, :64], orc.mul_mat("q8_1", t, Wq[:64], x[:24])) < 1e-11
 
 
 @pytest.mark.parametrize("name,t", TYPES)
 def test_unaligned_rows_fallback(dev, name, t):
-    """K for which the device-layout rows are not 16-byte multiples (byte-load kernel)"""
+    """a matrix at an odd address (byte-load kernel), with rows that are no 16-byte multiples, and the same rows at an even one"""
+    import torch
     import mi355
     rng = np.random.default_rng(5)
     be = orc.BLOCK[t][0]
@@ -343,12 +340,17 @@ def test_unaligned_rows_fallback(dev, name, t):
         Wq = _weights(rng, t, 19, K)
         x = rng.standard_normal((B, K)).astype(np.float32)
         Wd = mi355.upload_weights(t, _to_dev(dev, Wq))
+        odd = torch.empty(Wd.numel() + 17, dtype=torch.uint8, device=dev)
+        odd = odd[1 + (-odd.data_ptr()) % 2:][:Wd.numel()].reshape(Wd.shape)
+        odd.copy_(Wd)
+        assert odd.data_ptr() % 2 == 1
+        got = mi355.mul_mat(t, odd, _to_dev(dev, x)).cpu().numpy()
+        assert orc.nmse(got, orc.mul_mat("q8_1", t, Wq, x)) < 1e-11      # f32 products of f32 weights and activations
         got = mi355.mul_mat(t, Wd, _to_dev(dev, x)).cpu().numpy()
-        # Q4_K rows are always aligned, so B > 32 takes the super-block tile kernel and the CPU's activation format
+        # Q4_K and Q5_K rows are always 16-byte aligned, so B > 32 takes the super-block tile kernels and the CPU's activation format
         # (5..32 rows: the weight-streaming kernel with Q8_1 activations)
         want = orc.mul_mat("cpu" if (t in (orc.Q4_K, orc.Q5_K) and B > 32) else "q8_1", t, Wq, x)
-        # Q5_K rows are always aligned too: its batches run the per-32-block tile kernel, whose minimum term goes through fp16 operands
-        assert orc.nmse(got, want) < (1e-6 if (t == orc.Q5_K and B > 8) else 1e-9)
+        assert orc.nmse(got, want) < 1e-11
 
 
 @pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t not in (orc.Q4_K, orc.Q5_K)])   # those two are 16-byte aligned at any K

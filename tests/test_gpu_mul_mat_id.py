@@ -49,9 +49,7 @@ def test_mul_mat_id(dev, name, t, n_expert, n_used, nb1_bcast, T, N, K):
         want = np.zeros((T, n_used, N), dtype=np.float32)
         assert orc.oracle.orc_mul_mat_id_q8_1(t, orc._ptr(Wq), orc._ptr(b), orc._ptr(ids_full), n_expert, orc._ptr(want), N, K,
                                               n_expert, n_used, nb1, T) == 0
-    # per-32-block experts with 32+ slots run the routed form of their tile kernel, where the block minimum of Q4_1 / Q5_1 meets
-    # fp16(d_x * sum(q)), the `s` field the reference's own dot uses
-    assert orc.nmse(got, want) < (1e-6 if (t in (orc.Q4_1, orc.Q5_1) and T * n_used >= 32) else 1e-9)
+    assert orc.nmse(got, want) < 1e-11      # exact block dots, f32 sums over at most 128 blocks (an f16 block minimum would leave 1e-7)
     if orc.ref is not None:
         cpu = np.zeros_like(want)
         assert orc.ref.ref_mul_mat_id(t, orc._ptr(Wq), orc._ptr(b), orc._ptr(ids_full), orc._ptr(cpu), N, K, n_expert, n_used,
@@ -82,7 +80,7 @@ def test_mul_mat_id_skewed_routing(dev, name, t, pattern):
     got = mi355.mul_mat_id(t, Wd, torch.from_numpy(b).to(dev), idd, n_used).cpu().numpy()
     kind = "cpu" if t in (orc.Q4_K, orc.Q6_K, orc.Q5_K, orc.IQ4_XS) else "q8_1"   # the activation format of the type's routed tile kernel
     want = expected_per_expert(kind, t, Wq, b, np.clip(ids, 0, n_expert - 1), n_expert, n_used, 1, N)
-    assert orc.nmse(got, want) < (1e-6 if t in (orc.Q4_1, orc.Q5_1) else 1e-9)   # the block minimum meets fp16(d_x * sum(q)) in the tile kernel
+    assert orc.nmse(got, want) < 1e-11
 
 
 @pytest.mark.parametrize("name,t", list(orc.WEIGHT_TYPES.items()))
@@ -264,3 +262,32 @@ def test_routed_tiles_over_more_than_2_32_activation_blocks(dev):
     assert torch.equal(got, want)                                                               # whole numbers below 2^24
     del act, ds
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("name,t", [(n, t) for n, t in orc.WEIGHT_TYPES.items() if t not in (orc.Q4_K, orc.Q5_K)])
+@pytest.mark.parametrize("n_expert,n_used,T,N", [(4, 1, 32, 130), (4, 4, 32, 64), (8, 2, 128, 70), (16, 2, 128, 33), (16, 3, 65, 129)])
+def test_routed_tiles_with_few_slots_per_expert(dev, name, t, n_expert, n_used, T, N):
+    """mi355_mul_mat_id_q called directly where mi355_mul_mat_id prefers the weight-streaming kernel; and the stack at an odd address, where
+    mi355_mul_mat_id falls back to byte loads"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    K = 1280
+    rng = np.random.default_rng(T + N)
+    Wq = orc.quantize("oracle", t, (rng.standard_normal((n_expert * N, K)) * 0.02).astype(np.float32))
+    b = rng.standard_normal((T, 1, K)).astype(np.float32)
+    ids = np.stack([rng.permutation(n_expert)[:n_used] for _ in range(T)]).astype(np.int32)
+    Wd = mi355.upload_weights(t, torch.from_numpy(Wq).to(dev))
+    act, idd = mi355.quantize_act(torch.from_numpy(b[:, 0]).to(dev)), torch.from_numpy(ids).to(dev)
+    got = torch.full((T, n_used, N), float("nan"), device=dev)
+    route = torch.empty(int(lib.mi355_mul_mat_id_q8k_route_bytes(n_expert, n_used, T)), dtype=torch.uint8, device=dev)
+    mi355.check(lib.mi355_mul_mat_id_q(None, t, Wd.data_ptr(), act.data_ptr(), idd.data_ptr(), n_used, got.data_ptr(), N, K, n_expert, n_used, 1, T,
+                                       route.data_ptr(), route.numel()))
+    torch.cuda.synchronize()
+    want = expected_per_expert("q8_1", t, Wq, b, ids, n_expert, n_used, 1, N)
+    assert orc.nmse(got.cpu().numpy(), want) < 1e-11
+    odd = torch.empty(Wd.numel() + 1, dtype=torch.uint8, device=dev)[1:].reshape(n_expert, N, -1)
+    odd.copy_(Wd.reshape(odd.shape))
+    assert odd.data_ptr() % 2 == 1
+    got = mi355.mul_mat_id(t, odd, torch.from_numpy(b).to(dev), idd, n_used).cpu().numpy()
+    assert orc.nmse(got, want) < 1e-11
