@@ -598,51 +598,54 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
                     for (int r = 0; r < 16; r++) acc[tb][tw][r] += last[tb][tw][r];
         }
 
-        // store: lane holds weight row j = l32 of each 32-wide tile, 16 activation rows
-        uint64_t nans = 0;   // of the lane's sums: bit r + 16 (tw + 2 tb)
-        auto store = [&](auto checked) __attribute__((always_inline)) {
-    #pragma unroll
-            for (int tb = 0; tb < TN; tb++)
-    #pragma unroll
-                for (int tw = 0; tw < 2; tw++) {
-                    const int64_t n = row0 + wrow0 + tw * 32 + l32;
-    #pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int64_t b = col0 + wcol0 + tb * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-                        if (n < N && b < B) {
-                            const int64_t o = (ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n;
-                            if (decltype(checked)::value && acc[tb][tw][r] != acc[tb][tw][r]) nans |= 1ull << (r + 16 * (tw + 2 * tb));
-                            else dst[o] = residual ? acc[tb][tw][r] + residual[o] : acc[tb][tw][r];
-                        }
-                    }
-                }
-        };
-        float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // (four chains; with the test at each store instead the call takes 2 to 4 % longer, this way up to 1: Q4_0 4096 x 4096, 512 rows 47.3 us, 49.6, 47.3)
+        // An infinite weight scale makes a sum M * inf - M * inf: where a wave's sums are not all finite, the NaNs of rows with such a scale are
+        // formed again, block by block (a NaN of another origin stays one).  Four chains; the test takes up to 1 % of a call, at each store 2 to 4.
+        float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     #pragma unroll
         for (int tb = 0; tb < TN; tb++)
     #pragma unroll
             for (int tw = 0; tw < 2; tw++)
     #pragma unroll
                 for (int r = 0; r < 16; r++) zero[r & 3] = __builtin_fmaf(acc[tb][tw][r], 0.0f, zero[r & 3]);
-        if (__ballot((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.0f) == 0) {   // uniform: every sum is finite
-            store(mmq_int<0>{});
-            return;
+        if (__ballot((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.0f) != 0) {   // uniform
+            const int k_lo = s_lo * MMQ_BK, k_hi = s_hi * MMQ_BK < K ? s_hi * MMQ_BK : (int)K;
+            bool infinite[2];
+    #pragma unroll
+            for (int tw = 0; tw < 2; tw++) {
+                const int64_t n = row0 + wrow0 + tw * 32 + l32;
+                infinite[tw] = n < N && infinite_scale<TYPE>(W + n * L.row_bytes, L, k_lo, k_hi);
+            }
+            if (__ballot(infinite[0] || infinite[1]) != 0) {   // uniform
+    #pragma unroll 1
+                for (int i = 0; i < TN * 32; i++) {   // sum r of tile (tb, tw)
+                    const int r = i & 15, tw = (i >> 4) & 1;
+                    const int64_t n = row0 + wrow0 + tw * 32 + l32, b = col0 + wcol0 + (i >> 5) * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
+                    if (!(tw ? infinite[1] : infinite[0]) || b >= B) continue;
+                    const int64_t arow = ID ? (int64_t)row_of[b] : b;
+                    const float sum = plain_sum<TYPE>(W + n * L.row_bytes, L, aq + arow * K, ads + arow * nblk, k_lo, k_hi);
+    #pragma unroll
+                    for (int j = 0; j < TN * 32; j++) {
+                        const float at = acc[j >> 5][(j >> 4) & 1][j & 15];
+                        acc[j >> 5][(j >> 4) & 1][j & 15] = j == i && at != at ? sum : at;
+                    }
+                }
+            }
         }
-        store(mmq_int<1>{});
-        if (nans == 0) return;
-        // An infinite weight scale makes a sum M * inf - M * inf.  The row's sums are formed again, block by block (a NaN of another origin stays one)
-        u32 infinite = 0;
-        for (int tw = 0; tw < 2; tw++)
-            if ((nans >> (16 * tw)) & 0x0000FFFF0000FFFFull) infinite |= (u32)infinite_scale<TYPE>(W + (row0 + wrow0 + tw * 32 + l32) * L.row_bytes, L, s_lo * MMQ_BK, s_hi * MMQ_BK < K ? s_hi * MMQ_BK : (int)K) << tw;
-        for (; nans != 0; nans &= nans - 1) {
-            const int i = __builtin_ctzll(nans), r = i & 15, tw = (i >> 4) & 1;
-            const int64_t n = row0 + wrow0 + tw * 32 + l32, b = col0 + wcol0 + (i >> 5) * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-            const int64_t o = (ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n;
-            const int64_t arow = ID ? (int64_t)row_of[b] : b;
-            float sum = __builtin_nanf("");
-            if ((infinite >> tw) & 1) sum = plain_sum<TYPE>(W + n * L.row_bytes, L, aq + arow * K, ads + arow * nblk, s_lo * MMQ_BK, s_hi * MMQ_BK < K ? s_hi * MMQ_BK : (int)K);
-            dst[o] = residual ? sum + residual[o] : sum;
-        }
+        // store: lane holds weight row j = l32 of each 32-wide tile, 16 activation rows
+    #pragma unroll
+        for (int tb = 0; tb < TN; tb++)
+    #pragma unroll
+            for (int tw = 0; tw < 2; tw++) {
+                const int64_t n = row0 + wrow0 + tw * 32 + l32;
+    #pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int64_t b = col0 + wcol0 + tb * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
+                    if (n < N && b < B) {
+                        const int64_t o = (ID ? (int64_t)route.dst_row[b] : b) * dst_stride + n;
+                        dst[o] = residual ? acc[tb][tw][r] + residual[o] : acc[tb][tw][r];
+                    }
+                }
+            }
     };
     if constexpr (ID) {
         if (B - col0 <= BNK / 2) {
@@ -656,7 +659,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
 // What bounds the kernel is the vector ALU: a wave issues 637 of its instructions per stage, 512 of them the two per block sum and 16
 // matrix instructions, which are busy a quarter of that time (counters, Q4_0 14336 x 4096, 512 rows; 4 cycles each = 2550 cycles of the
 // 2800 a stage takes with one group per compute unit).  Before the two-instruction form, the double-buffered stages and the f32 minima, by
-// type (14336 x 4096, 512 rows with the quantization launch, us): Q4_0 139 -> 116, Q4_1 228 -> 128, Q5_0 149 -> 124, Q5_1 229 -> 140,
+// type (14336 x 4096, 512 rows with the quantization launch, us): Q4_0 124 -> 98, Q4_1 228 -> 128, Q5_0 149 -> 124, Q5_1 229 -> 140,
 // IQ4_NL 149 -> 128, Q8_0 146 -> 130; 64 rows: Q4_0 34.3 -> 32.3.  Q6_K with 16-element instead of masked 32-element matrix
 // instructions: 4096 x 11008, 64 rows 41.2 -> 39.5.
 //

@@ -591,7 +591,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W
     // A tile whose columns all lie in its first half (the ragged end of a batch; the second tile of an expert that is routed a few more
     // than 128 slots) runs with 32 x 32 per wave: half the matrix instructions, activation transfers and scaling, the same unpack.  Uniform
     // for the whole group, so each form keeps a branch-free stage.  8 experts of 14336 x 4096, 1024 slots (about half of the experts with a
-    // second tile of some ten slots): Q4_K 336 -> 318 us; Q5_K 4096 x 4096, 1400 slots 131 -> 126; one-round products 0 .. 1.5 % quicker.
+    // second tile of some ten slots): Q4_K 325 -> 308 us, runs differing by some 10 %; Q5_K 4096 x 4096, 1400 slots 131 -> 126; one-round products 0 .. 1.5 % quicker.
     auto walk = [&](auto ntb) __attribute__((always_inline)) {
         constexpr int NTB = decltype(ntb)::value;   // 32-column result tiles per wave
         const int wcol0 = (wave >> 1) * (32 * NTB); // activation rows of this wave inside the tile
