@@ -510,7 +510,7 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
             if constexpr (NS == 1) return __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[tb], f.w[tw], magic, 0, 0, 0);
             else return __builtin_amdgcn_mfma_i32_32x32x16_i8(pair64(f.a[tb][2 * h], f.a[tb][2 * h + 1]), pair64(f.w[tw][2 * h], f.w[tw][2 * h + 1]), magic, 0, 0, 0);
         };
-        auto scale = [&](f32x16 (&acc)[TN][2], const block_scales &f, int n, const i32x16 &I) {
+        auto scale = [&](const block_scales &f, int n, const i32x16 &I) {
             const int tb = n / NS % TN, tw = n / NS / TN, h = n % NS;
             const float dw = f.dw[tw][h], mdw = -MMQ_MAGIC * dw;
     #pragma unroll
@@ -524,78 +524,85 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
         commit(sm[0], s_lo);
         fetch(s_lo + 1 < s_hi ? s_lo + 1 : s_lo);
         __syncthreads();
-        auto contract = [&](const stage_mem &m, f32x16 (&acc)[TN][2]) __attribute__((always_inline)) {
-            asm volatile("" : "+v"(a_at), "+v"(w_at));   // the four chunk addresses of a stage are formed in the loop: kept across it they cost spills
-            // One matrix instruction is always in flight: its successor is issued before its sums are scaled, so that neither waits for the
-            // other (left to the compiler, all of them write the same registers one after the other); the next block's operands are read
-            // from LDS while the last sums of this one are scaled.
-            block_ops f = load_ops(m, 0);
-            block_scales sc = load_scales(m, 0);
-            i32x16 I = mma(f, 0);
+        int buf = 0, st = s_lo;
+        f32x16 before[C::WIDE ? TN : 1][2];   // WIDE: the sums of all but the last stage
+        const bool two = C::WIDE && (nblk & 3) == 1 && s_hi == stages && s_hi - s_lo > 1;   // ... the last two, where the last holds one block
     #pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                block_scales sc_next = sc;
-    #pragma unroll
-                for (int n = 0; n < NM; n++) {
-                    const i32x16 cur = I;
-                    I = mma(f, n + 1 < NM ? n + 1 : 0);   // (the last one of a stage is not used)
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (n == NM - 2 && ks < 3) f = load_ops(m, ks + 1);
-                    if (n == NM - 1 && ks < 3) sc_next = load_scales(m, ks + 1);
-                    scale(acc, sc, n, cur);
-                    asm volatile("" : "+v"(acc[n / NS % TN][n / NS / TN]));   // formed here, and not behind the matrix instructions of the whole stage
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                sc = sc_next;
-            }
-            if constexpr (C::MIN) {
-                // acc += sum_b (dx * sum q)[i][b] * m[j][b] over the 4 blocks of the stage (Q4_K, Q5_K: m = -dmin * 6-bit minimum): two
-                // v_mfma_f32_32x32x2_f32 per tile on the matrix pipe, which waits for the vector ALUs anyway; k = lane / 32.  In f32 as the
-                // batch-1 kernels do it (as f16 operands the term carried 3.6e-4 of the result).
-    #pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    float af[TN], bf[2];
-    #pragma unroll
-                    for (int tb = 0; tb < TN; tb++) af[tb] = m.as[(2 * p + lhi) * BN + wcol0 + tb * 32 + l32];
-    #pragma unroll
-                    for (int tw = 0; tw < 2; tw++) bf[tw] = m.wo[(2 * p + lhi) * MMQ_BM + wrow0 + tw * 32 + l32];
+        for (int part = 0; part < (C::WIDE ? 2 : 1); part++) {
+            const int part_end = C::WIDE && part == 0 ? s_hi - 1 - two : s_hi;
+            if constexpr (C::WIDE) {
+                if (part == 1) {
     #pragma unroll
                     for (int tb = 0; tb < TN; tb++)
     #pragma unroll
-                        for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
+                        for (int tw = 0; tw < 2; tw++)
+    #pragma unroll
+                            for (int r = 0; r < 16; r++) {
+                                before[tb][tw][r] = acc[tb][tw][r];
+                                acc[tb][tw][r] = 0.0f;
+                            }
+                    if (two) {   // (both buffers before the sums: the requested stage's registers make room for them)
+                        commit(sm[buf ^ 1], s_hi - 1);
+                        __syncthreads();
+                    }
                 }
             }
-        };
-        int buf = 0, st = s_lo;
-        const bool two = C::WIDE && (nblk & 3) == 1 && s_hi == stages && s_hi - s_lo > 1;   // the last stage holds one block: two stages
-        const int loop_end = C::WIDE ? s_hi - 1 - two : s_hi;
-        for (; st < loop_end; st++, buf ^= 1) {
-            contract(sm[buf], acc);
-            if (st + 1 < s_hi) {   // the next stage, requested one stage ago, goes to the other buffer (uniform)
-                commit(sm[buf ^ 1], st + 1);
-                fetch(st + 2 < s_hi ? st + 2 : st + 1);   // past the end the last stage is requested again and never used
-                __syncthreads();
+            for (; st < part_end; st++, buf ^= 1) {
+                const stage_mem &m = sm[buf];
+                asm volatile("" : "+v"(a_at), "+v"(w_at));   // the four chunk addresses of a stage are formed in the loop: kept across it they cost spills
+                // One matrix instruction is always in flight: its successor is issued before its sums are scaled, so that neither waits for the
+                // other (left to the compiler, all of them write the same registers one after the other); the next block's operands are read
+                // from LDS while the last sums of this one are scaled.
+                block_ops f = load_ops(m, 0);
+                block_scales sc = load_scales(m, 0);
+                i32x16 I = mma(f, 0);
+    #pragma unroll
+                for (int ks = 0; ks < 4; ks++) {
+                    block_scales sc_next = sc;
+    #pragma unroll
+                    for (int n = 0; n < NM; n++) {
+                        const i32x16 cur = I;
+                        I = mma(f, n + 1 < NM ? n + 1 : 0);   // (the last one of a stage is not used)
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (n == NM - 2 && ks < 3) f = load_ops(m, ks + 1);
+                        if (n == NM - 1 && ks < 3) sc_next = load_scales(m, ks + 1);
+                        scale(sc, n, cur);
+                        asm volatile("" : "+v"(acc[n / NS % TN][n / NS / TN]));   // formed here, and not behind the matrix instructions of the whole stage
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    sc = sc_next;
+                }
+                if constexpr (C::MIN) {
+                    // acc += sum_b (dx * sum q)[i][b] * m[j][b] over the 4 blocks of the stage (Q4_K, Q5_K: m = -dmin * 6-bit minimum): two
+                    // v_mfma_f32_32x32x2_f32 per tile on the matrix pipe, which waits for the vector ALUs anyway; k = lane / 32.  In f32 as the
+                    // batch-1 kernels do it (as f16 operands the term carried 3.6e-4 of the result).
+    #pragma unroll
+                    for (int p = 0; p < 2; p++) {
+                        float af[TN], bf[2];
+    #pragma unroll
+                        for (int tb = 0; tb < TN; tb++) af[tb] = m.as[(2 * p + lhi) * BN + wcol0 + tb * 32 + l32];
+    #pragma unroll
+                        for (int tw = 0; tw < 2; tw++) bf[tw] = m.wo[(2 * p + lhi) * MMQ_BM + wrow0 + tw * 32 + l32];
+    #pragma unroll
+                        for (int tb = 0; tb < TN; tb++)
+    #pragma unroll
+                            for (int tw = 0; tw < 2; tw++) acc[tb][tw] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[tb], bf[tw], acc[tb][tw], 0, 0, 0);
+                    }
+                }
+                if (part == 0 && st + 1 < s_hi) {   // the next stage, requested one stage ago, goes to the other buffer (uniform)
+                    commit(sm[buf ^ 1], st + 1);
+                    fetch(st + 2 < s_hi ? st + 2 : st + 1);   // past the end the last stage is requested again and never used
+                    __syncthreads();
+                }
             }
         }
-        if constexpr (C::WIDE) {   // the last stage on its own sums
-            f32x16 last[TN][2];
+        if constexpr (C::WIDE) {
     #pragma unroll
             for (int tb = 0; tb < TN; tb++)
     #pragma unroll
                 for (int tw = 0; tw < 2; tw++)
     #pragma unroll
-                    for (int r = 0; r < 16; r++) last[tb][tw][r] = 0.0f;
-            if (two) {   // (both buffers before the sums: the requested stage's registers make room for them)
-                commit(sm[buf ^ 1], s_hi - 1);
-                __syncthreads();
-            }
-            for (; st < s_hi; st++, buf ^= 1) contract(sm[buf], last);
-    #pragma unroll
-            for (int tb = 0; tb < TN; tb++)
-    #pragma unroll
-                for (int tw = 0; tw < 2; tw++)
-    #pragma unroll
-                    for (int r = 0; r < 16; r++) acc[tb][tw][r] += last[tb][tw][r];
+                    for (int r = 0; r < 16; r++) acc[tb][tw][r] += before[tb][tw][r];
         }
 
         // An infinite weight scale makes a sum M * inf - M * inf: where a wave's sums are not all finite, the NaNs of rows with such a scale are
