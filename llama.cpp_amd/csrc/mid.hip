@@ -25,23 +25,24 @@
 #include "qdot.hpp"
 #include "tiles.hpp"
 
+#include <type_traits>
+
 namespace mi355 {
 
 namespace {
 
 // A wave's ring of weight stages in LDS, filled by global-to-LDS transfers (no registers in between): per super-block four
 // transfers of 8 rows x 128 bytes of nibbles (1 KiB each, placed 16 bytes further apart so that rows 8 apart fall into different
-// banks) and one of the 32 rows' 16-byte headers (lanes 32..63 repeat them).  Slot p (16 bytes) of a nibble transfer holds piece
-// (p & 7) ^ (p >> 3) of row p >> 3: lanes that read the same piece of 32 different rows then hit different banks.
-constexpr int MID_STAGES = 3;
+// banks), one of the 32 rows' 16-byte headers (lanes 32..63 repeat them) and one of the set's activation scales (a float per lane).  Slot p
+// (16 bytes) of a nibble transfer holds piece (p & 7) ^ (p >> 3) of row p >> 3: lanes that read the same piece of 32 different rows
+// then hit different banks.
+constexpr int MID_STAGES = 2;
 constexpr int MID_SPAN = 1024 + 16;
-constexpr int MID_STAGE = 4 * MID_SPAN + 1024;
+constexpr int MID_HDR = 4 * MID_SPAN, MID_D8 = MID_HDR + 1024;
+constexpr int MID_STAGE = MID_D8 + 256;
 
-// chunks (64 columns = two 32-element blocks) of activation operands a wave holds ahead: a whole super-block with one activation
-// tile per wave, half of one with two (registers)
-template <int NB> constexpr int mid_ring() { return NB == 1 ? 4 : 2; }
 template <int NB> struct mid_act {
-    u32x4 a[NB][2 * mid_ring<NB>()];   // the lane's operand chunks of the ring's 32-element blocks, per activation tile
+    u32x4 a[NB][8];   // the lane's operand chunks of a super-block's 32-element blocks, per activation tile
     f16x8 bs[NB];     // its rows' {bsum_j & 63} (kh = 0) or {bsum_j >> 6} (kh = 1)
 };
 
@@ -89,77 +90,65 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
     const int s_lo = slice_lo + part * steps_per_wave;
     const int s_hi = s_lo + steps_per_wave < slice_hi ? s_lo + steps_per_wave : slice_hi;   // may be <= s_lo: a wave without steps
 
-    // sources of the transfers: 32-bit offsets from W (the launcher keeps matrices below 4 GiB); rows past the end repeat the
-    // last row and are not stored
-    const int64_t row_bytes = (int64_t)nsteps * Q4_K_BYTES;
-    unsigned w_off[4], h_off;
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        int64_t row = row0 + 8 * u + (lane >> 3);
-        row = row < N ? row : N - 1;
-        w_off[u] = (unsigned)(row * row_bytes + 16 + 16 * ((lane & 7) ^ ((lane >> 3) & 7)));
-    }
-    {
-        const int64_t my_row = row0 + r < N ? row0 + r : N - 1;
-        h_off = (unsigned)(my_row * row_bytes);
-    }
-    auto dma = [&](const uint8_t *g, unsigned off, uint8_t *l) {   // g, l: wave-uniform
-        asm volatile("" : "+v"(off));   // keeps the sum from being formed per lane ahead of the loop (two registers per source)
-        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(g + off), (void __attribute__((address_space(3))) *)l, 16, 0, 0);
-    };
-    auto issue = [&](int step, int slot) {   // super-block `step` of the wave's rows into stage `slot`
-        const uint8_t *g = W + (int64_t)step * Q4_K_BYTES;
-        uint8_t *st = ring + slot * MID_STAGE;
-#pragma unroll
-        for (int u = 0; u < 4; u++) dma(g, w_off[u], st + u * MID_SPAN);
-        dma(g, h_off, st + 4 * MID_SPAN);
-    };
-    // what the lane reads back: its own row's header, and piece 2 g + kh of its row for chunk g
-    const unsigned rd_hdr = 4 * MID_SPAN + r * 16;
-    unsigned rd_w[4];
-#pragma unroll
-    for (int g = 0; g < 4; g++) rd_w[g] = (unsigned)((r >> 3) * MID_SPAN + ((r & 7) * 8 + ((2 * g + kh) ^ (r & 7))) * 16);
-
-    // activation operands: lane (r, kh) supplies levels 16 kh .. + 16 of a 32-element block of activation row 32 (NB set + nb) + r
+    // sources of the transfers: 32-bit offsets from W (the launcher keeps matrices and images below 4 GiB), formed anew for every stage from the
+    // lane number (registers); rows past the end repeat the last row and are not stored
+    const u32 row_bytes = (u32)nsteps * Q4_K_BYTES;
+    const int last_row = (int)(N - 1);
     const int64_t b16 = ((int64_t)B + 15) & ~(int64_t)15;
     const int64_t cb_pad = wt_cb_pad(B);
-    const int64_t aux0 = b16 * K;   // the records behind the image
-    // 32-bit offsets from `act` (the launcher keeps images below 4 GiB): a uniform base plus one register per address
-    u32 a_tile[NB];   // the lane's row inside its 16-row block's first tile
-    u32 a_rec[NB];    // its sums in the block's record, super-block 0
-    int a_sw[NB];     // chunk swizzle of that row
-    u32 d_rec[NB][2];   // scales of the tile's two 16-row blocks, first row of the lane's four; the lane's 16 results
-                        // of a tile are activation rows 8 q + 4 kh + i (q, i = 0..3) of the tile
+    const int64_t aux0 = b16 * K;   // the records behind the activation image
+    const u32 rec_step = (u32)(cb_pad * WT_A_AUX);
+    // Buffer loads, not global ones: with a global-to-LDS load in flight the compiler turns every wait for an ordinary load into a wait
+    // for everything (it counts the former as a flat access), which put each stage's whole trip from HBM into every step.
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)W, 0, 0xFFFFFFFFu, 0x00020000);
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)act, 0, 0xFFFFFFFFu, 0x00020000);
+    typedef __attribute__((address_space(3))) void *lds_ptr;
+    auto issue = [&](int step, int slot) {   // super-block `step` of the wave's rows, and its activation scales, into stage `slot`
+        const u32 g = (u32)step * Q4_K_BYTES;
+        uint8_t *st = ring + slot * MID_STAGE;
+        int ln;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            int row = (int)row0 + 8 * u + (ln >> 3);
+            row = row < last_row ? row : last_row;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr)(st + u * MID_SPAN), 16, (u32)row * row_bytes + (16 + 16 * ((ln & 7) ^ (ln >> 3))), g, 0, 0);
+        }
+        int row = (int)row0 + (ln & 31);
+        row = row < last_row ? row : last_row;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr)(st + MID_HDR), 16, (u32)row * row_bytes, g, 0, 0);
+        int rb = 2 * NB * set + (ln >> 4);   // scale of activation row 32 NB set + lane
+        rb = rb < (int)cb_pad ? rb : (int)cb_pad - 1;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr)(st + MID_D8), 4, (u32)(rb * WT_A_AUX + (ln & 15) * 4), (u32)aux0 + (u32)step * rec_step, 0, 0);
+    };
+    // what the lane reads back: its own row's header, and piece 2 g + kh of its row for chunk g
+    const unsigned rd_hdr = MID_HDR + r * 16;
+    const unsigned rd_w = (unsigned)((r >> 3) * MID_SPAN + (r & 7) * 128), rd_p = (unsigned)((kh ^ (r & 7)) << 4);
+
+    // activation operands: lane (r, kh) supplies levels 16 kh .. + 16 of a 32-element block of activation row 32 (NB set + nb) + r
+    // the lane's offset inside the image (its chunk of the first tile's even and odd blocks, the two swizzled) in a register, the place
+    // of the 64-column tile in a scalar: no vector arithmetic per request
+    u32 a_off[NB][2], a_rec[NB];   // a_rec: its sums in the block's record, super-block 0
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
         int64_t arow = (int64_t)32 * (NB * set + nb) + r;
         arow = arow < b16 ? arow : b16 - 1;   // rows past the image repeat its last row; their results are not stored
         const int r16 = (int)(arow & 15);
-        a_tile[nb] = (u32)((arow >> 4) * (int64_t)(K >> 6) * WT_TILE + r16 * 64);
-        a_sw[nb] = (r16 >> 2) & 3;
-        a_rec[nb] = (u32)(aux0 + (arow >> 4) * WT_A_AUX + 64 + r16 * 32 + kh * 16);
 #pragma unroll
-        for (int hb = 0; hb < 2; hb++) {
-            int64_t rb = (int64_t)2 * (NB * set + nb) + hb;
-            rb = rb < cb_pad ? rb : cb_pad - 1;
-            d_rec[nb][hb] = (u32)(aux0 + rb * WT_A_AUX + 4 * kh * 4);
-        }
+        for (int h = 0; h < 2; h++)
+            a_off[nb][h] = (u32)((arow >> 4) * (int64_t)(K >> 6) * WT_TILE + r16 * 64) + (u32)(((2 * h + kh) ^ ((r16 >> 2) & 3)) << 4);
+        a_rec[nb] = (u32)((arow >> 4) * WT_A_AUX + 64 + r16 * 32 + kh * 16);
     }
-    const u32 rec_step = (u32)(cb_pad * WT_A_AUX);
 
-    constexpr int RING = mid_ring<NB>();
-    auto fetch_a = [&](int step, int g, mid_act<NB> &A) {   // the two blocks of chunk g (one 64-column tile) into ring slot g % RING
-        const int s = step < nsteps ? step : nsteps - 1;
+    auto fetch_a = [&](int s, int g, mid_act<NB> &A) {   // the two blocks of chunk g (one 64-column tile)
 #pragma unroll
         for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-            for (int h = 0; h < 2; h++)
-                A.a[nb][2 * (g % RING) + h] = load16(act + (a_tile[nb] + (u32)(s * 4 + g) * WT_TILE + (u32)(((2 * h + kh) ^ a_sw[nb]) << 4)));
+            for (int h = 0; h < 2; h++) A.a[nb][2 * g + h] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[nb][h] + g * WT_TILE, s * 4 * WT_TILE, 0);
     };
-    auto fetch_s = [&](int step, mid_act<NB> &A) {
-        const int s = step < nsteps ? step : nsteps - 1;
+    auto fetch_s = [&](int s, mid_act<NB> &A) {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) A.bs[nb] = *(const f16x8 *)(act + (a_rec[nb] + (u32)s * rec_step));
+        for (int nb = 0; nb < NB; nb++) A.bs[nb] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_rec[nb], (u32)aux0 + (u32)s * rec_step, 0));
     };
 
     f32x16 accf[NB];
@@ -169,23 +158,23 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
         for (int i = 0; i < 16; i++) accf[nb][i] = 0.0f;
 
     mid_act<NB> A;
-    // order of the requests: the weight stages first, then the activation operands of the same super-block, so that the arrival
-    // of a super-block's first activation operand (loads complete in order) says that its weight stage has landed
-#pragma unroll
-    for (int p = 0; p < MID_STAGES - 1; p++)
-        if (s_lo + p < s_hi) issue(s_lo + p, p);
+    // Loads complete in order, so the order of the requests decides what a wait waits for: a super-block's weight stage, then its
+    // activation operands, then the stage of the super-block after it.  The arrival of the first operand then says that its weight
+    // stage has landed, and no operand queues behind a weight stage that is wanted later than itself.  (With the stage two
+    // super-blocks on requested at the start of a step, in front of the step's second half of activation operands, every step
+    // waited for that stage's whole trip from HBM.)
     if (s_lo < s_hi) {
+        issue(s_lo, 0);
 #pragma unroll
-        for (int g = 0; g < RING; g++) fetch_a(s_lo, g, A);
+        for (int g = 0; g < 4; g++) fetch_a(s_lo, g, A);
         fetch_s(s_lo, A);
+        issue(s_lo + 1 < s_hi ? s_lo + 1 : s_lo, 1);
     }
-    int slot = 0;   // stage of the current super-block
-    for (int step = s_lo; step < s_hi; step++) {
-        {   // the stage read last step takes the super-block MID_STAGES - 1 on
-            const int ahead = step + MID_STAGES - 1;
-            const int aslot = slot == 0 ? MID_STAGES - 1 : slot - 1;
-            if (ahead < s_hi) issue(ahead, aslot);
-        }
+    // AHEAD: super-blocks of the wave that follow this one (2: two or more).  A request under a run-time condition would make the
+    // compiler's counts of what is in flight those of the path without it, i.e. every wait behind it a wait for everything; so the
+    // last two steps are copies of their own.
+    auto body = [&](auto ahead, int step, int slot) {
+        constexpr int AHEAD = decltype(ahead)::value;
         // ---- the lane's header and its four operand pieces out of the stage (inline assembly: the compiler would wait for every
         //      transfer in flight before an LDS read it can see).  The first read names an activation operand of this super-block
         //      as an input, which puts the compiler's wait for that operand - and with it the arrival of the stage - in front.
@@ -193,9 +182,8 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
         u32x4 hdr, wq[4];
         asm volatile("ds_read_b128 %0, %1" : "=v"(hdr) : "v"(st + rd_hdr), "v"(A.a[0][0]) : "memory");
 #pragma unroll
-        for (int g = 0; g < 4; g++) asm volatile("ds_read_b128 %0, %1" : "=v"(wq[g]) : "v"(st + rd_w[g]) : "memory");
+        for (int g = 0; g < 4; g++) asm volatile("ds_read_b128 %0, %1" : "=v"(wq[g]) : "v"(st + rd_w + (rd_p ^ (32 * g))) : "memory");
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(hdr), "+v"(wq[0]), "+v"(wq[1]), "+v"(wq[2]), "+v"(wq[3]) : : "memory");
-        slot = slot == MID_STAGES - 1 ? 0 : slot + 1;
 
         // all eight 6-bit (scale, min) pairs as the bytes of four words (get_scale_min_k4, ggml-quants.c:631-638)
         const float d = half_bits_to_float((unsigned short)(hdr[0] & 0xFFFFu));
@@ -209,11 +197,16 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
         //      {bsum_j & 63} (kh = 0) or {bsum_j >> 6} (kh = 1): sum over the 16 products = sum_j m_j bsum_j, exact in f32
         f16x8 mop;
         {
-            const float f = kh ? 64.0f : 1.0f;
+            // a byte in front of 0x64 is the f16 1024 + m: two of them per permute, one packed subtraction and one packed product
+            const _Float16 f = (_Float16)(kh ? 64.0f : 1.0f);
+            const f16x2 k1024 = {(_Float16)1024.0f, (_Float16)1024.0f}, ff = {f, f};
+            f16x2 mp[4];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const u32 M = j < 4 ? m_lo : m_hi;
-                mop[j] = (_Float16)(f * (float)((M >> (8 * (j & 3))) & 0xFFu));
+            for (int j = 0; j < 4; j++) {
+                const u32 M = j < 2 ? m_lo : m_hi;
+                mp[j] = (__builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, M, j & 1 ? 0x04030402u : 0x04010400u)) - k1024) * ff;
+                mop[2 * j] = mp[j][0];
+                mop[2 * j + 1] = mp[j][1];
             }
         }
         i32x16 hi[NB], lo[NB];
@@ -221,15 +214,8 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
         for (int nb = 0; nb < NB; nb++)
 #pragma unroll
             for (int i = 0; i < 16; i++) { hi[nb][i] = 0; lo[nb][i] = 0; }
-        f32x4 d8[NB][4];   // the scales of the rows this lane finishes: wanted at the end of the step, requested before its last chunk
 #pragma unroll
         for (int g = 0; g < 4; g++) {   // chunk g: sub-blocks 2 g (low nibbles) and 2 g + 1 (high nibbles), one 64-column tile
-            if (g == 3) {
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) d8[nb][q] = *(const f32x4 *)(act + (d_rec[nb][q >> 1] + (u32)step * rec_step + (u32)((8 * (q & 1)) * 4)));
-            }
             const u32x4 v = wq[g];
 #pragma unroll
             for (int h = 0; h < 2; h++) {
@@ -241,18 +227,19 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const u32 n = (v[i] >> (4 * h)) & 0x0F0F0F0Fu;
-                    wh[i] = (int)(n * a);   // bytes <= 15 * 7: no carries between them
-                    wl[i] = (int)(n * b);
+                    wh[i] = (int)mul_bytes(n, a);
+                    wl[i] = (int)mul_bytes(n, b);
                 }
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++) {
-                    hi[nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, A.a[nb][2 * (g % RING) + h]), wh, hi[nb], 0, 0, 0);
-                    lo[nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, A.a[nb][2 * (g % RING) + h]), wl, lo[nb], 0, 0, 0);
+                    hi[nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, A.a[nb][2 * g + h]), wh, hi[nb], 0, 0, 0);
+                    lo[nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, A.a[nb][2 * g + h]), wl, lo[nb], 0, 0, 0);
                 }
             }
-            // the chunk's registers take the operands RING chunks on
-            if (g + RING < 4) fetch_a(step, g + RING, A);
-            else if (step + 1 < s_hi) fetch_a(step + 1, g + RING - 4, A);
+            if constexpr (AHEAD >= 1) {
+                fetch_a(step + 1, g, A);   // the chunk's registers take the next super-block's operands
+                __builtin_amdgcn_sched_barrier(1);   // arithmetic may pass; the requests stay here (the scheduler moves them behind the chunks)
+            }
         }
         // ---- finish the super-block: accf += d8 (d (8 HI + LO) - dmin MS)
 #pragma unroll
@@ -260,17 +247,32 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
             f32x16 z;
 #pragma unroll
             for (int i = 0; i < 16; i++) z[i] = 0.0f;
+            f32x4 d8[4];   // the lane's 16 results of a tile are activation rows 8 q + 4 kh + i (q, i = 0..3) of the tile
+#pragma unroll
+            for (int q = 0; q < 4; q++) asm volatile("ds_read_b128 %0, %1" : "=v"(d8[q]) : "v"(st + MID_D8 + (32 * nb + 8 * q + 4 * kh) * 4) : "memory");
             const f32x16 ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(A.bs[nb], mop, z, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; q++) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(d8[q]) : : "memory");
 #pragma unroll
             for (int q = 0; q < 4; q++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float isum = (float)(8 * hi[nb][4 * q + i] + lo[nb][4 * q + i]);
                     const float t = __builtin_fmaf(d, isum, -(dmin * ms[4 * q + i]));
-                    accf[nb][4 * q + i] = __builtin_fmaf(d8[nb][q][i], t, accf[nb][4 * q + i]);
+                    accf[nb][4 * q + i] = __builtin_fmaf(d8[q][i], t, accf[nb][4 * q + i]);
                 }
         }
-        if (step + 1 < s_hi) fetch_s(step + 1, A);
+        if constexpr (AHEAD >= 1) fetch_s(step + 1, A);
+        if constexpr (AHEAD >= 2) issue(step + 2, slot);   // this step's stage has been read
+    };
+    if (s_lo < s_hi) {
+        int step = s_lo;
+        for (; step + 2 < s_hi; step++) body(std::integral_constant<int, 2>(), step, (step - s_lo) & 1);
+        if (step + 1 < s_hi) {
+            body(std::integral_constant<int, 1>(), step, (step - s_lo) & 1);
+            step++;
+        }
+        body(std::integral_constant<int, 0>(), step, (step - s_lo) & 1);
     }
 
     // the parts of K: fixed order 0, 1, ...

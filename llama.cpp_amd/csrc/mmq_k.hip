@@ -34,7 +34,6 @@
 
 namespace mi355 {
 
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef short i16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int KQ_BK = 128;            // K elements per stage (half a super-block)
@@ -118,14 +117,6 @@ struct mmq_route {
     const int32_t *n_tiles;        // number of column tiles in use (device value)
     int64_t expert_bytes;          // bytes from one expert's matrix to the next
 };
-
-// 4 packed bytes (each <= 15) times a small factor (<= 7): no byte overflows, so two 16-bit multiplies do it
-__device__ __forceinline__ u32 mul_bytes(u32 x, u32 f) {
-    const u16x2 v = __builtin_bit_cast(u16x2, x);
-    const u16x2 m = {(unsigned short)f, (unsigned short)f};
-    const u16x2 p = v * m;
-    return __builtin_bit_cast(u32, p);
-}
 
 // Q5_K: four levels 0..31 (bytes of a) times the sub-block scale 0..63 -> value = 16*hi + lo, hi <= 122, lo <= 15
 __device__ __forceinline__ void q5k_planes(u32 a, int sc, u32 &hi, u32 &lo) {
