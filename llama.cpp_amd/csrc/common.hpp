@@ -110,6 +110,36 @@ __device__ __forceinline__ u32x4 load_stream16(const void *p) {
 }
 __device__ __forceinline__ u32x4 load16(const void *p) { return *(const u32x4 *)p; }
 
+// Buffer loads: base and soff are wave-uniform (scalars), voff the lane's byte offset; together below 4 GiB from base.  Against an ordinary
+// load: one register of address per lane and no arithmetic to form it.  And next to global-to-LDS transfers they are the only form that
+// can stay in flight: while a global_load_lds is, the compiler makes every wait for an ordinary load a wait for everything (it counts the
+// transfer as a flat access), with buffer transfers it counts exactly.
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *base) { return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 0xFFFFFFFFu, 0x00020000); }
+__device__ __forceinline__ u32x4 buf_load16(const void *base, u32 voff, u32 soff) { return __builtin_amdgcn_raw_buffer_load_b128(buf_rsrc(base), voff, soff, 0); }
+__device__ __forceinline__ u32x2 buf_load8(const void *base, u32 voff, u32 soff) {
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(buf_rsrc(base), voff, soff, 0));
+}
+__device__ __forceinline__ u32 buf_load4(const void *base, u32 voff, u32 soff) { return __builtin_amdgcn_raw_buffer_load_b32(buf_rsrc(base), voff, soff, 0); }
+__device__ __forceinline__ unsigned short buf_load2(const void *base, u32 voff, u32 soff) { return __builtin_amdgcn_raw_buffer_load_b16(buf_rsrc(base), voff, soff, 0); }
+__device__ __forceinline__ unsigned char buf_load1(const void *base, u32 voff, u32 soff) { return __builtin_amdgcn_raw_buffer_load_b8(buf_rsrc(base), voff, soff, 0); }
+// global memory -> LDS, 16 (4) bytes per lane to lds + 16 (4) * lane; lds: wave-uniform
+__device__ __forceinline__ void buf_to_lds16(const void *base, u32 voff, u32 soff, void *lds) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf_rsrc(base), (void __attribute__((address_space(3))) *)lds, 16, voff, soff, 0, 0);
+}
+__device__ __forceinline__ void buf_to_lds4(const void *base, u32 voff, u32 soff, void *lds) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf_rsrc(base), (void __attribute__((address_space(3))) *)lds, 4, voff, soff, 0, 0);
+}
+#else   // the host pass knows neither the builtins nor the resource type
+__device__ u32x4 buf_load16(const void *, u32, u32);
+__device__ u32x2 buf_load8(const void *, u32, u32);
+__device__ u32 buf_load4(const void *, u32, u32);
+__device__ unsigned short buf_load2(const void *, u32, u32);
+__device__ unsigned char buf_load1(const void *, u32, u32);
+__device__ void buf_to_lds16(const void *, u32, u32, void *);
+__device__ void buf_to_lds4(const void *, u32, u32, void *);
+#endif
+
 // Single roundings that stay single: the compiler may not merge these into fused multiply-adds, whatever surrounds the call.
 // (The CUDA-style __fmul_rn / __fadd_rn of the HIP headers are plain operators and do get merged.)  For results that several
 // kernels must reproduce bit for bit.

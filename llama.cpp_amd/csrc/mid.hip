@@ -98,11 +98,7 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
     const int64_t cb_pad = wt_cb_pad(B);
     const int64_t aux0 = b16 * K;   // the records behind the activation image
     const u32 rec_step = (u32)(cb_pad * WT_A_AUX);
-    // Buffer loads, not global ones: with a global-to-LDS load in flight the compiler turns every wait for an ordinary load into a wait
-    // for everything (it counts the former as a flat access), which put each stage's whole trip from HBM into every step.
-    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)W, 0, 0xFFFFFFFFu, 0x00020000);
-    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)act, 0, 0xFFFFFFFFu, 0x00020000);
-    typedef __attribute__((address_space(3))) void *lds_ptr;
+    // (buffer loads, see common.hpp)
     auto issue = [&](int step, int slot) {   // super-block `step` of the wave's rows, and its activation scales, into stage `slot`
         const u32 g = (u32)step * Q4_K_BYTES;
         uint8_t *st = ring + slot * MID_STAGE;
@@ -112,14 +108,14 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
         for (int u = 0; u < 4; u++) {
             int row = (int)row0 + 8 * u + (ln >> 3);
             row = row < last_row ? row : last_row;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr)(st + u * MID_SPAN), 16, (u32)row * row_bytes + (16 + 16 * ((ln & 7) ^ (ln >> 3))), g, 0, 0);
+            buf_to_lds16(W, (u32)row * row_bytes + (16 + 16 * ((ln & 7) ^ (ln >> 3))), g, st + u * MID_SPAN);
         }
         int row = (int)row0 + (ln & 31);
         row = row < last_row ? row : last_row;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr)(st + MID_HDR), 16, (u32)row * row_bytes, g, 0, 0);
+        buf_to_lds16(W, (u32)row * row_bytes, g, st + MID_HDR);
         int rb = 2 * NB * set + (ln >> 4);   // scale of activation row 32 NB set + lane
         rb = rb < (int)cb_pad ? rb : (int)cb_pad - 1;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr)(st + MID_D8), 4, (u32)(rb * WT_A_AUX + (ln & 15) * 4), (u32)aux0 + (u32)step * rec_step, 0, 0);
+        buf_to_lds4(act, (u32)(rb * WT_A_AUX + (ln & 15) * 4), (u32)aux0 + (u32)step * rec_step, st + MID_D8);
     };
     // what the lane reads back: its own row's header, and piece 2 g + kh of its row for chunk g
     const unsigned rd_hdr = MID_HDR + r * 16;
@@ -144,11 +140,11 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
 #pragma unroll
         for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) A.a[nb][2 * g + h] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[nb][h] + g * WT_TILE, s * 4 * WT_TILE, 0);
+            for (int h = 0; h < 2; h++) A.a[nb][2 * g + h] = buf_load16(act, a_off[nb][h] + g * WT_TILE, s * 4 * WT_TILE);
     };
     auto fetch_s = [&](int s, mid_act<NB> &A) {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) A.bs[nb] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_rec[nb], (u32)aux0 + (u32)s * rec_step, 0));
+        for (int nb = 0; nb < NB; nb++) A.bs[nb] = __builtin_bit_cast(f16x8, buf_load16(act, a_rec[nb], (u32)aux0 + (u32)s * rec_step));
     };
 
     f32x16 accf[NB];

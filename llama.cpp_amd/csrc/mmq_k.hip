@@ -16,14 +16,11 @@
 // per 32.  The Q4_K min term is one v_mfma_f32_32x32x16_f16 per super-block on exact small
 // integers: k slots 0..7 carry (bsum & 63) x m_j, slots 8..15 carry (bsum >> 6) x 64*m_j.
 //
-// A 256-thread group (4 waves, 2 x 2) owns a 64 (weight rows) x 128 (activation rows) tile of
-// dst; each wave a 32 x 64 sub-tile (1 x 2 MFMA tiles).  K is walked in stages of 128 elements.  k_mmq_kp is the kernel
-// of the full-width tile: double-buffered LDS, one barrier per stage, activations by direct global-to-LDS transfers, the
-// weight unpack interleaved with the matrix instructions.  (Keeping the unpacked weights in the registers of the lane that
-// feeds them to the matrix cores, with no LDS round trip, measured the same: the unpack is then repeated by the two waves
-// that share rows, and the vector ALU is the limit either way at ~11 instructions per matrix instruction.)  k_mmq_k is
-// the single-buffered kernel (register prefetch, two barriers per stage) kept for the 64 x 64 tile that sparse expert
-// routing uses.
+// k_mmq_kp, the kernel of the full-width tile: a group owns 128 (weight rows) x 128 (activation rows) of dst, or 64 x 128 where the
+// launch has at most one such tile per compute unit; each wave a 32 x 64 sub-tile (1 x 2 MFMA tiles).  K is walked in stages of 128
+// elements, see there.  (Keeping the unpacked weights in the registers of the lane that feeds them to the matrix cores, with no LDS round
+// trip, measured the same: the unpack is then repeated by the two waves that share rows.)  k_mmq_k is the single-buffered kernel (register
+// prefetch, two barriers per stage) of a 64 x 64 tile that sparse expert routing uses.
 //
 // MFMA operand mapping (A = activations, B = weights, D[i][j]): lane l supplies row l % 32
 // and k bytes [16*(l/32), +16) (f16: k slots [8*(l/32), +8)); D register r of lane l is
@@ -389,22 +386,25 @@ __global__ void __launch_bounds__(256, OCC) k_mmq_k(const uint8_t *__restrict__ 
         }
 }
 
-// ---- pipelined variant of the 64 x 128 tile ---------------------------------------------------------------------------
-// Two LDS buffers per operand, one barrier per 128-element stage.  While the matrix cores work on stage s from
-// buffer s % 2, the same waves unpack the weights of stage s + 1 (fetched to registers during stage s - 1) into the other
-// buffer, and the activations of stage s + 1 go from global memory straight to LDS (global_load_lds, no registers, no
-// vector-ALU work).  LDS rows are 128 bytes without padding; the 16-byte chunk c of row r lives at chunk c ^ ((r >> 1) & 7),
-// which keeps every 16-lane group of a ds_read_b128 on distinct banks.  A super-block is two stages, so the buffer of a
-// stage is its half: every LDS access names its array statically and the compiler can tell the buffer being filled from
-// the one being read.
+// ---- pipelined kernel of the 128-column tile ----------------------------------------------------------------------------
+// Stage s works on 128 elements of K: the matrix cores read its weight planes and activations from LDS while the same waves unpack the
+// weight piece of stage s + 1 into the other pair of plane buffers; the activations of stage s + 3 start from memory to LDS (a ring of
+// four stages) and the weight piece of stage s + 3 to registers.  One barrier per stage, which waits for the next stage's transfers and
+// for nothing younger: a trip to L2 or HBM is longer than a stage.  LDS rows are 128 bytes without padding; the 16-byte chunk c of row r
+// lives at chunk c ^ ((r >> 1) & 7), which keeps every 16-lane group of a ds_read_b128 on distinct banks.
+// What bounds it (14336 x 4096, 512 rows, Q4_K): LDS is active 53 % of the compute units' busy time, the vector ALU 39 %, the matrix pipes
+// 34 %; two waves per SIMD do not overlap them further.  With two stages in flight, waits for everything in flight at every stage and two
+// groups of 64 rows per compute unit: whole calls, us, before / now: Q4_K 14336 x 4096 x 512 102.8 / 96.9, 4096 x 14336 x 512 104.7 / 97.2;
+// IQ4_XS 8192 x 4096 x 512 67.6 / 58.6; Q5_K 14336 x 4096 x 200 62.2 / 59.0; Q6_K 4096 x 4096 x 100 24.8 / 24.1; experts (8 of 14336 x 4096,
+// 1024 slots) Q4_K 284 / 264, Q6_K 399 / 333.  The 64-row tile: Q5_K 1024 x 4096 x 50 14.6 / 13.7, 16.1 on 128-row tiles (half the units idle).
 constexpr int KP_ROW = 128;
 __device__ __forceinline__ int kp_off(int row, int chunk) { return row * KP_ROW + ((chunk ^ ((row >> 1) & 7)) << 4); }
 
 template <int TYPE> struct kp_w;   // the 16-byte weight piece of one stage that this thread unpacks (row tid / 4, piece tid % 4)
 template <> struct kp_w<MI355_Q4_K> { u32x4 q; };
-template <> struct kp_w<MI355_Q6_K> { u32x4 ql, qh; int scA, scB; };
+template <> struct kp_w<MI355_Q6_K> { u32x4 ql, qh; unsigned char scA, scB; };   // raw bytes: widening at the load would wait for it
 template <> struct kp_w<MI355_Q5_K> { u32x4 q, qh; };
-template <> struct kp_w<MI355_IQ4_XS> { u32x4 q; int ls; };   // ls: the block's scale, -32..31
+template <> struct kp_w<MI355_IQ4_XS> { u32x4 q; u32x2 hdr; };
 // the two forms of the kernel: with a min term and an unsigned product (Q4_K, Q5_K) / signed products and no min term (Q6_K, IQ4_XS)
 template <int TYPE> struct kp_form {
     static constexpr bool MIN = TYPE == MI355_Q4_K || TYPE == MI355_Q5_K;
@@ -417,36 +417,44 @@ template <> struct kp_h<MI355_Q6_K> { unsigned short d; };   // raw fp16 bits: c
 template <> struct kp_h<MI355_Q5_K> { u32x4 hdr; };
 template <> struct kp_h<MI355_IQ4_XS> { unsigned short d; };
 
+// Every request of the kernel's loop is a buffer load (common.hpp): a scalar place along K, one register of per-lane offset.
+struct kp_addr { u32 q, q2, sc, h; };   // byte offsets from the wave's first weight row: levels, further level bits, scales, block header / d
 template <int TYPE>
-__device__ __forceinline__ void kp_fetch_h(kp_h<TYPE> &H, const uint8_t *__restrict__ wrow, const row_layout &L, int64_t sb) {
-    if constexpr (TYPE == MI355_Q4_K) H.hdr = load16(wrow + sb * Q4_K_BYTES);
-    else if constexpr (TYPE == MI355_Q5_K) H.hdr = load16(wrow + sb * Q5_K_BYTES);
-    else if constexpr (TYPE == MI355_IQ4_XS) H.d = *(const unsigned short *)(wrow + L.off_b + sb * 8);
-    else H.d = *(const unsigned short *)(wrow + L.off_d + sb * 2);
+__device__ __forceinline__ kp_addr kp_addr_of(u32 row_off, const row_layout &L) {   // row_off: (row of the thread - first row of its wave) * row_bytes
+    const u32 p = threadIdx.x & 3;
+    if constexpr (TYPE == MI355_Q4_K) return {row_off + 16 + (p >> 1) * 32 + (p & 1) * 16, 0, 0, row_off};
+    else if constexpr (TYPE == MI355_Q5_K) return {row_off + 48 + (p >> 1) * 32 + (p & 1) * 16, row_off + 16 + (p & 1) * 16, 0, row_off};
+    else if constexpr (TYPE == MI355_IQ4_XS) return {row_off + p * 16, 0, 0, row_off + (u32)L.off_b};
+    else return {row_off + p * 16, row_off + (u32)L.off_b + 16 * (p & 1), row_off + (u32)L.off_c + (p & 1) + 2 * (p >> 1), row_off + (u32)L.off_d};
+}
+
+// requests of kp_fetch_h / kp_fetch_w, in instructions
+template <int TYPE> struct kp_loads { static constexpr int H = 1, W = TYPE == MI355_Q4_K ? 1 : TYPE == MI355_Q6_K ? 4 : 2; };
+
+template <int TYPE>
+__device__ __forceinline__ void kp_fetch_h(kp_h<TYPE> &H, const uint8_t *w, const kp_addr &A, u32 sb) {
+    if constexpr (TYPE == MI355_Q4_K) H.hdr = buf_load16(w, A.h, sb * Q4_K_BYTES);
+    else if constexpr (TYPE == MI355_Q5_K) H.hdr = buf_load16(w, A.h, sb * Q5_K_BYTES);
+    else if constexpr (TYPE == MI355_IQ4_XS) H.d = buf_load2(w, A.h, sb * 8);
+    else H.d = buf_load2(w, A.h, sb * 2);
 }
 
 template <int TYPE>
-__device__ __forceinline__ void kp_fetch_w(kp_w<TYPE> &R, const uint8_t *__restrict__ wrow, const row_layout &L, int64_t sb, int half) {
-    const int p = threadIdx.x & 3;
+__device__ __forceinline__ void kp_fetch_w(kp_w<TYPE> &R, const uint8_t *w, const kp_addr &A, u32 sb, int half) {
+    asm volatile("" : "+s"(sb));   // two halves of a super-block share Q5_K's fifth bits: each requests them, the requests are counted
     if constexpr (TYPE == MI355_Q4_K) {
-        const uint8_t *blk = wrow + sb * Q4_K_BYTES;
-        R.q = load16(blk + 16 + (half * 2 + (p >> 1)) * 32 + (p & 1) * 16);
+        R.q = buf_load16(w, A.q, sb * Q4_K_BYTES + half * 64);
     } else if constexpr (TYPE == MI355_Q5_K) {   // the Q4_K geometry behind 32 bytes of fifth bits (bit j of qh[l]: sub-block j, level l)
-        const uint8_t *blk = wrow + sb * Q5_K_BYTES;
-        R.q = load16(blk + 48 + (half * 2 + (p >> 1)) * 32 + (p & 1) * 16);
-        R.qh = load16(blk + 16 + (p & 1) * 16);
+        R.q = buf_load16(w, A.q, sb * Q5_K_BYTES + half * 64);
+        R.qh = buf_load16(w, A.q2, sb * Q5_K_BYTES);
     } else if constexpr (TYPE == MI355_IQ4_XS) {   // block 4 half + p: 16 bytes of table indices, its six-bit scale from the header
-        const int ib = half * 4 + p;
-        R.q = load16(wrow + sb * 128 + ib * 16);
-        const uint2 h = *(const uint2 *)(wrow + L.off_b + sb * 8);
-        R.ls = (int)(((h.y >> (4 * ib)) & 0xFu) | (((h.x >> (16 + 2 * ib)) & 3u) << 4)) - 32;
+        R.q = buf_load16(w, A.q, sb * 128 + half * 64);
+        R.hdr = buf_load8(w, A.h, sb * 8);
     } else {
-        const int l0 = 16 * (p & 1), qa = p >> 1;
-        R.ql = load16(wrow + sb * 128 + half * 64 + p * 16);
-        R.qh = load16(wrow + L.off_b + sb * 64 + half * 32 + l0);
-        const int8_t *sc = (const int8_t *)(wrow + L.off_c + sb * 16 + half * 8 + (l0 >> 4));
-        R.scA = sc[2 * qa];
-        R.scB = sc[2 * qa + 4];
+        R.ql = buf_load16(w, A.q, sb * 128 + half * 64);
+        R.qh = buf_load16(w, A.q2, sb * 64 + half * 32);
+        R.scA = buf_load1(w, A.sc, sb * 16 + half * 8);
+        R.scB = buf_load1(w, A.sc + 4, sb * 16 + half * 8);
     }
 }
 
@@ -480,19 +488,21 @@ __device__ __forceinline__ void kp_unpack(const kp_w<TYPE> &R, const kp_h<TYPE> 
         q5k_planes(nh, sch, hi, lo);
         P.b1[i] = hi; P.b0[i] = lo;
     } else if constexpr (TYPE == MI355_IQ4_XS) {
+        const int ib = half * 4 + p;
+        const int ls = (int)(((R.hdr[1] >> (4 * ib)) & 0xFu) | (((R.hdr[0] >> (16 + 2 * ib)) & 3u) << 4)) - 32;   // the block's scale
         u32 hi, lo;
-        iq4xs_planes(iq4nl_lookup4(R.q[i] & 0x0F0F0F0Fu), R.ls, hi, lo);
+        iq4xs_planes(iq4nl_lookup4(R.q[i] & 0x0F0F0F0Fu), ls, hi, lo);
         P.a1[i] = hi; P.a0[i] = lo;
-        iq4xs_planes(iq4nl_lookup4((R.q[i] >> 4) & 0x0F0F0F0Fu), R.ls, hi, lo);
+        iq4xs_planes(iq4nl_lookup4((R.q[i] >> 4) & 0x0F0F0F0Fu), ls, hi, lo);
         P.b1[i] = hi; P.b0[i] = lo;
     } else {
         const int qa = p >> 1;
         const u32 va = (R.ql[i] & 0x0F0F0F0Fu) | (((R.qh[i] >> (2 * qa)) & 0x03030303u) << 4);
         const u32 vb = ((R.ql[i] >> 4) & 0x0F0F0F0Fu) | (((R.qh[i] >> (2 * qa + 4)) & 0x03030303u) << 4);
         u32 hi, lo;
-        q6k_planes(va, R.scA, hi, lo);
+        q6k_planes(va, (int8_t)R.scA, hi, lo);
         P.a1[i] = hi; P.a0[i] = lo;
-        q6k_planes(vb, R.scB, hi, lo);
+        q6k_planes(vb, (int8_t)R.scB, hi, lo);
         P.b1[i] = hi; P.b0[i] = lo;
     }
 }
@@ -511,14 +521,13 @@ __device__ __forceinline__ void kp_store(const kp_planes &P, int8_t *__restrict_
 }
 
 // activations of one stage: 32 * AI rows x 128 bytes, AI wave-wide 16-byte transfers per wave.  aofs: per-lane byte offsets of
-// the 16 bytes this lane moves (row * K + swizzled chunk, fixed for the whole kernel); base: uniform pointer to the stage.
+// the 16 bytes this lane moves (row * K + swizzled chunk, fixed for the whole kernel); k0: the stage's place along K.
 template <int AI>
-__device__ __forceinline__ void kp_dma_a(const int8_t *__restrict__ base, const unsigned (&aofs)[AI], int8_t *__restrict__ sA) {
-    const int wave = threadIdx.x >> 6;
+__device__ __forceinline__ void kp_dma_a(const int8_t *base, u32 k0, const unsigned (&aofs)[AI], int8_t *__restrict__ sA) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
     for (int it = 0; it < AI; it++)
-        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(base + aofs[it]),
-                                         (void __attribute__((address_space(3))) *)(sA + (wave * AI + it) * 1024), 16, 0, 0);
+        buf_to_lds16(base, aofs[it], k0, sA + (wave * AI + it) * 1024);
 }
 // row of transfer `it` of this lane and the logical chunk that belongs at the lane's LDS position
 template <int AI>
@@ -530,76 +539,100 @@ __device__ __forceinline__ void kp_dma_slot(int it, int &row, int &chunk) {
 
 template <int V> struct kp_int { static constexpr int value = V; };
 
-template <int TYPE, bool ID>
-__global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const float *__restrict__ ad8,
+// 16 bytes of LDS on their way to registers, and the wait for all that are (every result of kp_lds_request passes through it before its use)
+template <int OFF>
+__device__ __forceinline__ i32x4 kp_lds_request(unsigned addr) {
+    i32x4 v;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
+    return v;
+}
+__device__ __forceinline__ void kp_lds_wait(i32x4 &a, i32x4 &b, i32x4 &c, i32x4 &d) {
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : : "memory");
+}
+__device__ __forceinline__ void kp_lds_wait(i32x4 &a, i32x4 &b, i32x4 &c) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b), "+v"(c) : : "memory"); }
+
+template <int TYPE, bool ID, int BM>
+__global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const float *__restrict__ ad8,
                                                    const _Float16 *__restrict__ abs_, float *dst, const float *residual,
                                                    int64_t N, int64_t K, int64_t B, int64_t dst_stride, row_layout L, int n_col_tiles,
                                                    int n_groups, int n_groups_padded, mmq_route route) {
     constexpr bool Q4 = kp_form<TYPE>::MIN;   // the form with a min term (Q4_K, Q5_K)
     constexpr int RADIX_SHIFT = kp_form<TYPE>::RADIX_SHIFT;
-    constexpr int BM = 64, BN = 128;
-    __shared__ __attribute__((aligned(16))) int8_t sW1a[BM * KP_ROW], sW1b[BM * KP_ROW];
-    __shared__ __attribute__((aligned(16))) int8_t sW0a[BM * KP_ROW], sW0b[BM * KP_ROW];
-    __shared__ __attribute__((aligned(16))) int8_t sAa[BN * KP_ROW], sAb_[BN * KP_ROW];
+    constexpr int BN = 128, WW = BM / 32;   // waves along the weight rows (two along the columns)
+    constexpr int CT = 4 * BM / BN;         // threads that share a column's scales
+    constexpr int W_BUF = BM * KP_ROW, A_BUF = BN * KP_ROW;
+    __shared__ __attribute__((aligned(16))) int8_t sW[4 * W_BUF];   // [half][hi, lo plane]
+    __shared__ __attribute__((aligned(16))) int8_t sA[4 * A_BUF];   // ring of four stages
     __shared__ __attribute__((aligned(16))) float sWd[2][BM];
     __shared__ __attribute__((aligned(16))) float sWn[2][Q4 ? BM : 4];
     __shared__ __attribute__((aligned(16))) _Float16 sWm[2][Q4 ? BM * 16 : 8];
     __shared__ __attribute__((aligned(16))) float sAd[2][BN];
     __shared__ __attribute__((aligned(16))) _Float16 sAs[2][Q4 ? BN * 16 : 8];
-    // sAa / sAb_ are written by global-to-LDS transfers only; a transfer names the wave's first 16 bytes, so to the compiler most
-    // of these arrays is never stored to.  The empty asm makes them memory that unknown code may have written.
-    asm volatile("" ::"v"((void *)sAa), "v"((void *)sAb_) : "memory");
-
     const int per_xcd = n_groups_padded >> 3;
-    const int lid = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    const int lid = ID ? (int)blockIdx.x : (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
     if (lid >= n_groups) return;
-    const int64_t row0 = (int64_t)(lid / n_col_tiles) * BM;
-    int64_t col0 = (int64_t)(lid % n_col_tiles) * BN;
-    if constexpr (ID) {
-        const int ct = lid % n_col_tiles;
+    int64_t row0, col0;
+    if constexpr (!ID) {
+        row0 = (int64_t)(lid / n_col_tiles) * BM;
+        col0 = (int64_t)(lid % n_col_tiles) * BN;
+    } else {
+        // column tile by column tile over the whole chip, in the order of their work (k_route_slots): the last groups are the short ones
+        const int n_row_tiles = n_groups / n_col_tiles, ct = (int)blockIdx.x / n_row_tiles;
+        row0 = (int64_t)((int)blockIdx.x - ct * n_row_tiles) * BM;
         if (ct >= *route.n_tiles) return;
-        W += (int64_t)route.tiles[4 * ct] * route.expert_bytes;
-        col0 = route.tiles[4 * ct + 1];
-        B = route.tiles[4 * ct + 2];
+        // the same for every lane: scalars, as the base of the weight loads has to be
+        W += (int64_t)__builtin_amdgcn_readfirstlane(route.tiles[4 * ct]) * route.expert_bytes;
+        col0 = __builtin_amdgcn_readfirstlane(route.tiles[4 * ct + 1]);
+        B = __builtin_amdgcn_readfirstlane(route.tiles[4 * ct + 2]);
     }
 
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lhi = lane >> 5;
-    const int wrow0 = (wave & 1) * 32;    // weight rows of this wave inside the tile
+    const int wrow0 = (wave % WW) * 32;    // weight rows of this wave inside the tile
     const int64_t nsb = K >> 8;
     // split K: group y of gridDim.y walks super-blocks [sb_lo, sb_hi) and writes its sums to its own slice of `dst` (see launch)
     const int64_t sb_per = (nsb + gridDim.y - 1) / gridDim.y;
-    const int64_t sb_lo = (int64_t)blockIdx.y * sb_per, sb_hi = sb_lo + sb_per < nsb ? sb_lo + sb_per : nsb;
+    const int sb_lo = (int)((int64_t)blockIdx.y * sb_per), sb_hi = (int)(sb_lo + sb_per < nsb ? sb_lo + sb_per : nsb);
     if (gridDim.y > 1) {
         dst += (int64_t)blockIdx.y * B * dst_stride;
         residual = nullptr;
     }
 
-    // this thread's weight row, the activation rows of its four transfers, and the column whose scales it copies
-    const int64_t wr = row0 + (tid >> 2) < N ? row0 + (tid >> 2) : N - 1;
-    const uint8_t *wrow = W + wr * L.row_bytes;
+    // this thread's weight row (four threads each)
+    // offsets from the wave's first row: 16 rows stay below 4 GiB for any K whose activations do
+    const int64_t wr = row0 + (tid >> 2) < N ? row0 + (tid >> 2) : N - 1, wr0 = row0 + 16 * wave < N ? row0 + 16 * wave : N - 1;
+    const uint8_t *w_tile = W + wr0 * L.row_bytes;
+    const kp_addr wa = kp_addr_of<TYPE>((u32)((wr - wr0) * L.row_bytes), L);
     // A tile whose columns all lie in its first half (the ragged end of a batch; the second tile of an expert that is routed a few more
     // than 128 slots) runs with 32 x 32 per wave: half the matrix instructions, activation transfers and scaling, the same unpack.  Uniform
-    // for the whole group, so each form keeps a branch-free stage.  8 experts of 14336 x 4096, 1024 slots (about half of the experts with a
-    // second tile of some ten slots): Q4_K 325 -> 308 us, runs differing by some 10 %; Q5_K 4096 x 4096, 1400 slots 131 -> 126; one-round products 0 .. 1.5 % quicker.
+    // for the whole group, so each form keeps a branch-free stage.
     auto walk = [&](auto ntb) __attribute__((always_inline)) {
         constexpr int NTB = decltype(ntb)::value;   // 32-column result tiles per wave
-        const int wcol0 = (wave >> 1) * (32 * NTB); // activation rows of this wave inside the tile
-        unsigned aofs[2 * NTB];
+        const int wcol0 = (wave / WW) * (32 * NTB); // activation rows of this wave inside the tile
+        constexpr int AI = NTB * 4 / WW;            // transfers of a wave per stage
+        unsigned aofs[AI];
     #pragma unroll
-        for (int it = 0; it < 2 * NTB; it++) {
+        for (int it = 0; it < AI; it++) {
             int r, c;
-            kp_dma_slot<2 * NTB>(it, r, c);
+            kp_dma_slot<AI>(it, r, c);
             const int64_t col = col0 + r;
             const int64_t cc = col < B ? col : B - 1;
             aofs[it] = (unsigned)((int64_t)(ID ? route.act_row[cc] : (int)cc) * K + c * 16);
         }
         int srow;
         {
-            const int64_t col = col0 + (tid >> 1);
+            const int64_t col = col0 + tid / CT;
             const int64_t cc = col < B ? col : B - 1;
             srow = ID ? route.act_row[cc] : (int)cc;
+        }
+
+        // LDS addresses of this lane's operands of the stage's four 32-element steps (first tile / hi plane of the first buffer)
+        unsigned a_rd[4], w_rd[4];
+    #pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            a_rd[ks] = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)sA + kp_off(wcol0 + l32, ks * 2 + lhi);
+            w_rd[ks] = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)sW + kp_off(wrow0 + l32, ks * 2 + lhi);
         }
 
         f32x16 acc[NTB];
@@ -609,26 +642,27 @@ __global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W
             for (int r = 0; r < 16; r++) acc[tb][r] = 0.0f;
 
         // per super-block scales of the weights come with the piece (Q4_K header / Q6_K d); those of the activations are fetched
-        // by two threads per column: 16 bytes of the sub-block sums each, the even thread also the scale
-        auto fetch_scales = [&](int64_t sb, float &d8, u32x4 &bs) {
-            d8 = ad8[(int64_t)srow * nsb + sb];
-            if constexpr (Q4) bs = *(const u32x4 *)(abs_ + ((int64_t)srow * nsb + sb) * 16 + 8 * (tid & 1));
+        // by two or four threads per column: the scale, and 16 bytes of the sub-block sums (threads 2, 3 the same as 0, 1)
+        const u32 d_off = (u32)srow * (u32)nsb * 4, s_off = (u32)srow * (u32)nsb * 32 + 16 * (tid & 1);
+        auto fetch_scales = [&](int sb, float &d8, u32x4 &bs) {
+            d8 = __builtin_bit_cast(float, buf_load4(ad8, d_off, (u32)sb * 4));
+            if constexpr (Q4) bs = buf_load16(abs_, s_off, (u32)sb * 32);
         };
         auto store_scales = [&](int sbuf, float d8, const u32x4 &bs, const kp_h<TYPE> &H) {
-            sAd[sbuf][tid >> 1] = d8;   // both threads of the column write the same value: an unconditional use keeps the load where it was issued
+            sAd[sbuf][tid / CT] = d8;   // the threads of a column write the same value: an unconditional use keeps the load where it was issued
             if constexpr (Q4) {
-                *(u32x4 *)(sAs[sbuf] + (tid >> 1) * 16 + 8 * (tid & 1)) = bs;
+                *(u32x4 *)(sAs[sbuf] + (tid / CT) * 16 + 8 * (tid & 1)) = bs;
                 // the four threads of a row share the work (and all use the header, so its load stays where it was issued):
                 // each writes d, dmin (same values) and the mins of sub-blocks 2p, 2p + 1
                 const int r = tid >> 2, p2 = 2 * (tid & 3);
                 sWd[sbuf][r] = half_bits_to_float((unsigned short)(H.hdr[0] & 0xFFFFu));
                 sWn[sbuf][r] = half_bits_to_float((unsigned short)(H.hdr[0] >> 16));
-                int sc, mn0, mn1;
-                q4k_scale_min(H.hdr[1], H.hdr[2], H.hdr[3], p2, sc, mn0);
-                q4k_scale_min(H.hdr[1], H.hdr[2], H.hdr[3], p2 + 1, sc, mn1);
-                typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-                const f16x2 m1 = {(_Float16)(float)mn0, (_Float16)(float)mn1};
-                const f16x2 m64 = {(_Float16)(float)(64 * mn0), (_Float16)(float)(64 * mn1)};
+                // (get_scale_min_k4 on whole words; a byte under 0x64 is the f16 1024 + m)
+                const u32 m_lo = H.hdr[2] & 0x3F3F3F3Fu, m_hi = ((H.hdr[3] >> 4) & 0x0F0F0F0Fu) | (((H.hdr[2] >> 6) & 0x03030303u) << 4);
+                const u32 mm = ((tid & 2) ? m_hi : m_lo) >> (16 * (tid & 1));
+                const f16x2 k1024 = {(_Float16)1024.0f, (_Float16)1024.0f}, k64 = {(_Float16)64.0f, (_Float16)64.0f};
+                const f16x2 m1 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, mm, 0x04010400u)) - k1024;
+                const f16x2 m64 = m1 * k64;
                 *(f16x2 *)(sWm[sbuf] + r * 16 + p2) = m1;
                 *(f16x2 *)(sWm[sbuf] + r * 16 + 8 + p2) = m64;
             } else {
@@ -636,116 +670,157 @@ __global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W
             }
         };
 
-        kp_w<TYPE> R0, R1;   // pieces of the even / odd stages
-        kp_h<TYPE> Hc, Hn;   // super-block data in use / of the next super-block
+        // Requests of a stage, in this order: the activation transfers of the stage three on; the scales of the next super-block (first half)
+        // or the header of the one after it (second half); the weight piece of the stage three on.
+        constexpr int LW = kp_loads<TYPE>::W, E0 = (Q4 ? 2 : 1) + LW, E1 = kp_loads<TYPE>::H + LW;
+        // End of a stage: the next stage's transfers of this wave, issued two stages ago, have landed - all but the YOUNGER requests behind
+        // them - and its LDS accesses are done; then the group's.
+        auto stage_end = [=](auto younger) {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(younger)::value) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);   // or work on the next stage's loads moves up, and the wait for them with it
+        };
+        auto last = [&](int sb) { return sb < sb_hi ? sb : sb_hi - 1; };   // past the end the last super-block is requested again and never read: no branches in a stage
+
+        kp_w<TYPE> R0, R1, R2, R3;   // pieces, by stage number modulo 4
+        kp_h<TYPE> H0, H1;           // super-block headers, by super-block number modulo 2 (numbers count from sb_lo)
         float d8n = 0.0f;
         u32x4 bsn = {0, 0, 0, 0};
-        // prologue: stage 0 into the "a" buffers, pieces of stage 1 in flight
-        kp_fetch_w<TYPE>(R0, wrow, L, sb_lo, 0);
-        kp_fetch_w<TYPE>(R1, wrow, L, sb_lo, 1);
-        kp_fetch_h<TYPE>(Hc, wrow, L, sb_lo);
-        kp_dma_a<2 * NTB>(aq + sb_lo * QKK, aofs, sAa);
+        // prologue: the requests of the three stages before the first, and what they leave in LDS
+        kp_dma_a<AI>(aq, (u32)sb_lo * QKK, aofs, sA);
+        __builtin_amdgcn_sched_barrier(0);
+        kp_fetch_h<TYPE>(H0, w_tile, wa, (u32)sb_lo);
+        kp_fetch_w<TYPE>(R0, w_tile, wa, (u32)sb_lo, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        kp_dma_a<AI>(aq, (u32)sb_lo * QKK + 128, aofs, sA + A_BUF);
+        __builtin_amdgcn_sched_barrier(0);
         fetch_scales(sb_lo, d8n, bsn);
+        kp_fetch_w<TYPE>(R1, w_tile, wa, (u32)sb_lo, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        kp_dma_a<AI>(aq, (u32)last(sb_lo + 1) * QKK, aofs, sA + 2 * A_BUF);
+        __builtin_amdgcn_sched_barrier(0);
+        kp_fetch_h<TYPE>(H1, w_tile, wa, (u32)last(sb_lo + 1));
+        kp_fetch_w<TYPE>(R2, w_tile, wa, (u32)last(sb_lo + 1), 0);
+        __builtin_amdgcn_sched_barrier(0);
         {
             kp_planes P;
     #pragma unroll
-            for (int i = 0; i < 4; i++) kp_unpack<TYPE>(R0, Hc, 0, i, P);
-            kp_store<TYPE>(P, sW1a, sW0a);
-            store_scales(0, d8n, bsn, Hc);
+            for (int i = 0; i < 4; i++) kp_unpack<TYPE>(R0, H0, 0, i, P);
+            kp_store<TYPE>(P, sW, sW + W_BUF);
+            store_scales(0, d8n, bsn, H0);
         }
-        Hn = Hc;
-        __syncthreads();
+        stage_end(kp_int<0>{});
 
-        for (int64_t sb = sb_lo; sb < sb_hi; sb++) {
-            i32x16 hi[NTB], lo[NTB];
-    #pragma unroll
-            for (int half = 0; half < 2; half++) {
-                const int8_t *cA = half == 0 ? sAa : sAb_;
-                const int8_t *cW1 = half == 0 ? sW1a : sW1b;
-                const int8_t *cW0 = half == 0 ? sW0a : sW0b;
-                int8_t *nA = half == 0 ? sAb_ : sAa;
-                int8_t *nW1 = half == 0 ? sW1b : sW1a;
-                int8_t *nW0 = half == 0 ? sW0b : sW0a;
-                kp_w<TYPE> &Rn = half == 0 ? R1 : R0;    // piece of the next stage: unpacked during this one
-                kp_w<TYPE> &Rf = half == 0 ? R0 : R1;    // held this stage's piece (unpacked one stage ago): refilled for the stage after next
-                // Past the end of K the same work is done on the last super-block again and never read: no branches in the stage,
-                // so the compiler schedules it as one block.
-                const int64_t sb1 = sb + 1 < sb_hi ? sb + 1 : sb;
-                kp_dma_a<2 * NTB>(aq + (half == 0 ? sb * QKK + 128 : sb1 * QKK), aofs, nA);
-                if (half == 1) fetch_scales(sb1, d8n, bsn);
-                kp_fetch_w<TYPE>(Rf, wrow, L, sb1, half);
-                if (half == 0) kp_fetch_h<TYPE>(Hn, wrow, L, sb1);   // used from the next stage on
-                __builtin_amdgcn_sched_barrier(0);   // the loads stay here, a whole stage ahead of their first use
-
-                kp_planes P;
-                i32x4 af[2][NTB], b1[2], b0[2];
-                auto load_frags = [&](int ks, int slot) {
-    #pragma unroll
-                    for (int tb = 0; tb < NTB; tb++) af[slot][tb] = *(const i32x4 *)(cA + kp_off(wcol0 + tb * 32 + l32, ks * 2 + lhi));
-                    b1[slot] = *(const i32x4 *)(cW1 + kp_off(wrow0 + l32, ks * 2 + lhi));
-                    b0[slot] = *(const i32x4 *)(cW0 + kp_off(wrow0 + l32, ks * 2 + lhi));
-                };
-                load_frags(0, 0);
-    #pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    if (ks < 3) load_frags(ks + 1, (ks + 1) & 1);   // operands of the next step are in flight during this step's matrix instructions
-                    const int sl = ks & 1;
-    #pragma unroll
-                    for (int tb = 0; tb < NTB; tb++) {
-                        if (half == 0 && ks == 0) {
-                            i32x16 z;
-    #pragma unroll
-                            for (int r = 0; r < 16; r++) z[r] = 0;
-                            hi[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b1[sl], z, 0, 0, 0);
-                            lo[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b0[sl], z, 0, 0, 0);
-                        } else {
-                            hi[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b1[sl], hi[tb], 0, 0, 0);
-                            lo[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b0[sl], lo[tb], 0, 0, 0);
-                        }
-                    }
-                    kp_unpack<TYPE>(Rn, half == 0 ? Hc : Hn, half ^ 1, ks, P);   // a quarter of the next stage's piece between the matrix instructions
-                }
-                kp_store<TYPE>(P, nW1, nW0);
-
-                if (half == 1) {   // end of the super-block: scale the integer sums into the f32 accumulators
-                    const int sbuf = (int)((sb - sb_lo) & 1);
-    #pragma unroll
-                    for (int tb = 0; tb < NTB; tb++) {
-                        f32x4 d8[4];
-    #pragma unroll
-                        for (int q = 0; q < 4; q++) d8[q] = *(const f32x4 *)(sAd[sbuf] + wcol0 + tb * 32 + 8 * q + 4 * lhi);
-                        const int wr_ = wrow0 + l32;
-                        const float dw = sWd[sbuf][wr_];
-                        if constexpr (Q4) {
-                            const float dn = sWn[sbuf][wr_];
-                            const f16x8 am = *(const f16x8 *)(sAs[sbuf] + (wcol0 + tb * 32 + l32) * 16 + 8 * lhi);
-                            const f16x8 bm = *(const f16x8 *)(sWm[sbuf] + wr_ * 16 + 8 * lhi);
-                            f32x16 z;
-    #pragma unroll
-                            for (int r = 0; r < 16; r++) z[r] = 0.0f;
-                            const f32x16 M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, z, 0, 0, 0);
-    #pragma unroll
-                            for (int r = 0; r < 16; r++) {
-                                const int t = (hi[tb][r] << RADIX_SHIFT) + lo[tb][r];
-                                acc[tb][r] += d8[r >> 2][r & 3] * (dw * (float)t - dn * M[r]);
-                            }
-                        } else {
-    #pragma unroll
-                            for (int r = 0; r < 16; r++) {
-                                const int t = (hi[tb][r] << RADIX_SHIFT) + lo[tb][r];
-                                acc[tb][r] += d8[r >> 2][r & 3] * (dw * (float)t);
-                            }
-                        }
-                    }
-                }
-                if (half == 1) {   // last, so that the loads had the whole stage (the barrier keeps the scheduler from hoisting the wait)
-                    __builtin_amdgcn_sched_barrier(0);
-                    store_scales((int)((sb - sb_lo + 1) & 1), d8n, bsn, Hn);
-                    Hc = Hn;
-                }
-                __syncthreads();   // also waits for this stage's transfers and loads (issued a whole stage ago)
+        i32x16 hi[NTB], lo[NTB];
+        // one stage; its position in the ring of four (0, 2: first half of a super-block) is known at compile time
+        // LEFT: super-blocks from this one to the end, 3 for more than two.  The last stages request nothing that nobody uses (the compiler
+        // would drop such loads, and stage_end's count with them).
+        auto stage = [&](auto pos, auto left, const int sb) __attribute__((always_inline)) {
+            constexpr int POS = decltype(pos)::value, half = POS & 1, ODD = POS >> 1, LEFT = decltype(left)::value;
+            constexpr bool REQ = LEFT == 3 || (LEFT == 2 && half == 0), NEXT = LEFT > 1 || half == 0;   // NEXT: there is a next stage
+            kp_w<TYPE> &Rn = POS == 0 ? R1 : POS == 1 ? R2 : POS == 2 ? R3 : R0;   // piece of the next stage: unpacked during this one
+            kp_w<TYPE> &Rf = POS == 0 ? R3 : POS == 1 ? R0 : POS == 2 ? R1 : R2;   // receives the piece of the stage three on
+            kp_h<TYPE> &Hn = (half == 0) == (ODD == 0) ? H0 : H1;   // header of the piece being unpacked: this super-block's, then the next one's
+            kp_h<TYPE> &Hf = ODD == 0 ? H0 : H1;                    // second half: this super-block's header is done with
+            if constexpr (REQ) {
+                const int sb3 = last(half == 0 ? sb + 1 : sb + 2);
+                kp_dma_a<AI>(aq, (u32)sb3 * QKK + (half == 0 ? 128 : 0), aofs, sA + ((POS + 3) & 3) * A_BUF);
+                __builtin_amdgcn_sched_barrier(0);   // the order of the requests is what stage_end counts on
+                if constexpr (half == 0) fetch_scales(last(sb + 1), d8n, bsn);
+                else kp_fetch_h<TYPE>(Hf, w_tile, wa, (u32)sb3);
+                kp_fetch_w<TYPE>(Rf, w_tile, wa, (u32)sb3, half ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
+
+            kp_planes P;
+            // Operand reads in inline assembly: for an LDS read it can see, the compiler waits for transfers in flight that may have written
+            // there, and it does not tell the stages of the ring apart.  A step waits for its operands, issues the next step's, computes.
+            i32x4 af[2][NTB], b1[2], b0[2];
+            auto load_frags = [&](int ks, int slot) {
+                af[slot][0] = kp_lds_request<POS * A_BUF>(a_rd[ks]);
+                if constexpr (NTB == 2) af[slot][NTB - 1] = kp_lds_request<POS * A_BUF + 32 * KP_ROW>(a_rd[ks]);
+                b1[slot] = kp_lds_request<(2 * half) * W_BUF>(w_rd[ks]);
+                b0[slot] = kp_lds_request<(2 * half + 1) * W_BUF>(w_rd[ks]);
+            };
+            load_frags(0, 0);
+    #pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                const int sl = ks & 1;
+                if constexpr (NTB == 2) kp_lds_wait(af[sl][0], af[sl][NTB - 1], b1[sl], b0[sl]);
+                else kp_lds_wait(af[sl][0], b1[sl], b0[sl]);
+                if (ks < 3) load_frags(ks + 1, sl ^ 1);
+    #pragma unroll
+                for (int tb = 0; tb < NTB; tb++) {
+                    if (half == 0 && ks == 0) {
+                        i32x16 z;
+    #pragma unroll
+                        for (int r = 0; r < 16; r++) z[r] = 0;
+                        hi[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b1[sl], z, 0, 0, 0);
+                        lo[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b0[sl], z, 0, 0, 0);
+                    } else {
+                        hi[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b1[sl], hi[tb], 0, 0, 0);
+                        lo[tb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[sl][tb], b0[sl], lo[tb], 0, 0, 0);
+                    }
+                }
+                if constexpr (NEXT) kp_unpack<TYPE>(Rn, Hn, half ^ 1, ks, P);   // a quarter of the next stage's piece between the matrix instructions
+            }
+            if constexpr (NEXT) kp_store<TYPE>(P, sW + 2 * (half ^ 1) * W_BUF, sW + (2 * (half ^ 1) + 1) * W_BUF);
+
+            if constexpr (half == 1) {   // end of the super-block: scale the integer sums into the f32 accumulators
+    #pragma unroll
+                for (int tb = 0; tb < NTB; tb++) {
+                    f32x4 d8[4];
+    #pragma unroll
+                    for (int q = 0; q < 4; q++) d8[q] = *(const f32x4 *)(sAd[ODD] + wcol0 + tb * 32 + 8 * q + 4 * lhi);
+                    const int wr_ = wrow0 + l32;
+                    const float dw = sWd[ODD][wr_];
+                    if constexpr (Q4) {
+                        const float dn = sWn[ODD][wr_];
+                        const f16x8 am = *(const f16x8 *)(sAs[ODD] + (wcol0 + tb * 32 + l32) * 16 + 8 * lhi);
+                        const f16x8 bm = *(const f16x8 *)(sWm[ODD] + wr_ * 16 + 8 * lhi);
+                        f32x16 z;
+    #pragma unroll
+                        for (int r = 0; r < 16; r++) z[r] = 0.0f;
+                        const f32x16 M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, z, 0, 0, 0);
+    #pragma unroll
+                        for (int r = 0; r < 16; r++) {
+                            const int t = (hi[tb][r] << RADIX_SHIFT) + lo[tb][r];
+                            acc[tb][r] += d8[r >> 2][r & 3] * (dw * (float)t - dn * M[r]);
+                        }
+                    } else {
+    #pragma unroll
+                        for (int r = 0; r < 16; r++) {
+                            const int t = (hi[tb][r] << RADIX_SHIFT) + lo[tb][r];
+                            acc[tb][r] += d8[r >> 2][r & 3] * (dw * (float)t);
+                        }
+                    }
+                }
+                // last, so that the loads had two stages (the barrier keeps the scheduler from hoisting the wait)
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (NEXT) store_scales(ODD ^ 1, d8n, bsn, ODD == 0 ? H1 : H0);
+            }
+            if constexpr (REQ) stage_end(kp_int<2 * AI + (half == 0 ? 2 * E0 + E1 : 2 * E1 + E0)>{});
+            else if constexpr (LEFT == 2) stage_end(kp_int<AI + E0>{});
+            else if constexpr (NEXT) stage_end(kp_int<0>{});
+        };
+        int sb = sb_lo;
+        for (; sb + 2 < sb_hi; sb += 2) {   // no exit in the middle: a second way round the loop would have the compiler wait for younger loads
+            stage(kp_int<0>{}, kp_int<3>{}, sb);
+            stage(kp_int<1>{}, kp_int<3>{}, sb);
+            stage(kp_int<2>{}, kp_int<3>{}, sb + 1);
+            stage(kp_int<3>{}, kp_int<3>{}, sb + 1);
         }
+        if (sb + 1 < sb_hi) {
+            stage(kp_int<0>{}, kp_int<2>{}, sb);
+            stage(kp_int<1>{}, kp_int<2>{}, sb);
+            stage(kp_int<2>{}, kp_int<1>{}, sb + 1);
+            stage(kp_int<3>{}, kp_int<1>{}, sb + 1);
+        } else {
+            stage(kp_int<0>{}, kp_int<1>{}, sb);
+            stage(kp_int<1>{}, kp_int<1>{}, sb);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no transfer into this group's LDS outlives it
 
     #pragma unroll
         for (int tb = 0; tb < NTB; tb++) {
@@ -976,14 +1051,14 @@ __global__ void __launch_bounds__(256, 2) k_mmq_pl(const int8_t *__restrict__ pl
     float d8n = 0.0f;
     u32x4 bsn = {0, 0, 0, 0};
     // both planes of a stage: 64 rows x 128 bytes each, two wave-wide transfers per wave and plane, swizzled like the activations
-    auto dma_w = [&](int64_t k0, int8_t *s1, int8_t *s0) {
-        kp_dma_a<2>(plane1 + k0, pofs, s1);
-        kp_dma_a<2>(plane0 + k0, pofs, s0);
+    auto dma_w = [&](u32 k0, int8_t *s1, int8_t *s0) {
+        kp_dma_a<2>(plane1, k0, pofs, s1);
+        kp_dma_a<2>(plane0, k0, pofs, s0);
     };
     // prologue: stage 0 into the "a" buffers
     pl_fetch_h<TYPE>(Hc, aux_row, sb_lo);
-    kp_dma_a<4>(aq + sb_lo * QKK, aofs, sAa);
-    dma_w(sb_lo * QKK, sW1a, sW0a);
+    kp_dma_a<4>(aq, (u32)sb_lo * QKK, aofs, sAa);
+    dma_w((u32)sb_lo * QKK, sW1a, sW0a);
     fetch_scales(sb_lo, d8n, bsn);
     store_scales(0, d8n, bsn, Hc);
     Hn = Hc;
@@ -1001,8 +1076,8 @@ __global__ void __launch_bounds__(256, 2) k_mmq_pl(const int8_t *__restrict__ pl
             int8_t *nW0 = half == 0 ? sW0b : sW0a;
             // Past the end of K the same work is done on the last super-block again and never read: no branches in the stage.
             const int64_t sb1 = sb + 1 < sb_hi ? sb + 1 : sb;
-            const int64_t k1 = half == 0 ? sb * QKK + 128 : sb1 * QKK;   // the next stage
-            kp_dma_a<4>(aq + k1, aofs, nA);
+            const u32 k1 = half == 0 ? (u32)sb * QKK + 128 : (u32)sb1 * QKK;   // the next stage
+            kp_dma_a<4>(aq, k1, aofs, nA);
             dma_w(k1, nW1, nW0);
             if (half == 1) fetch_scales(sb1, d8n, bsn);
             if (half == 0) pl_fetch_h<TYPE>(Hn, aux_row, sb1);   // used from the next stage on
@@ -1139,27 +1214,31 @@ static void launch_split_sum(hipStream_t s, const float *part, float *dst, const
     MI355_LAUNCH(k_split_sum, dim3((unsigned)((N * B / 4 + 255) / 256)), dim3(256), 0, s, part, dst, residual, N, B, dst_stride, n);
 }
 
+// tiles of 64 rows fit on the chip at once
+static bool kp_one_round(int64_t N, int64_t cols) { return (N + 63) / 64 * cols <= 256; }
+
 template <int TYPE>
 static void launch_mmq_k(hipStream_t s, const void *W, const void *act, float *dst, const float *residual, int64_t N, int64_t K, int64_t B,
                          int64_t dst_stride, void *ws, size_t ws_bytes) {
-    constexpr int BM = 64, BN = 128;
     const row_layout L = make_row_layout(TYPE, K);
     const int8_t *aq = (const int8_t *)act;
     const float *ad8 = (const float *)(aq + q8k_d_offset(K, B));
     const _Float16 *abs_ = (const _Float16 *)(aq + q8k_bs_offset(K, B));
-    const int n_row_tiles = (int)((N + BM - 1) / BM);
-    const int n_col_tiles = (int)((B + BN - 1) / BN);
-    const int n_groups = n_row_tiles * n_col_tiles;
-    const int n_groups_padded = (n_groups + 7) & ~7;
+    const int n_col_tiles = (int)((B + 127) / 128);
     const int n_slices = usable_slices(N, K, B, ws, ws_bytes);
-    if (n_slices > 1) {
-        MI355_LAUNCH((k_mmq_kp<TYPE, false>), dim3((unsigned)n_groups_padded, (unsigned)n_slices), dim3(256), 0, s, (const uint8_t *)W, aq, ad8, abs_,
-                           (float *)ws, nullptr, N, K, B, N, L, n_col_tiles, n_groups, n_groups_padded, mmq_route{});
-        launch_split_sum(s, (const float *)ws, dst, residual, N, B, dst_stride, n_slices);
-        return;
-    }
-    MI355_LAUNCH((k_mmq_kp<TYPE, false>), dim3((unsigned)n_groups_padded), dim3(256), 0, s, (const uint8_t *)W, aq, ad8, abs_, dst, residual, N, K,
-                       B, dst_stride, L, n_col_tiles, n_groups, n_groups_padded, mmq_route{});
+    float *out = n_slices > 1 ? (float *)ws : dst;
+    const int64_t out_stride = n_slices > 1 ? N : dst_stride;
+    const float *add = n_slices > 1 ? nullptr : residual;
+    auto launch = [&](auto bm) {
+        constexpr int BM = decltype(bm)::value;
+        const int n_groups = (int)((N + BM - 1) / BM) * n_col_tiles, n_groups_padded = (n_groups + 7) & ~7;
+        MI355_LAUNCH((k_mmq_kp<TYPE, false, BM>), dim3((unsigned)n_groups_padded, (unsigned)n_slices), dim3(4 * BM), 0, s, (const uint8_t *)W, aq, ad8, abs_,
+                           out, add, N, K, B, out_stride, L, n_col_tiles, n_groups, n_groups_padded, mmq_route{});
+    };
+    // a group of 64 rows on every compute unit beats one of 128 on every second one
+    if (kp_one_round(N, n_col_tiles * n_slices)) launch(kp_int<64>{});
+    else launch(kp_int<128>{});
+    if (n_slices > 1) launch_split_sum(s, (const float *)ws, dst, residual, N, B, dst_stride, n_slices);
 }
 
 // ---- MUL_MAT_ID with many slots: sort the slots by expert, then one tile launch over all experts ----
@@ -1182,19 +1261,28 @@ __global__ void __launch_bounds__(1024) k_route_slots(const int32_t *__restrict_
         atomicAdd(&cnt[ex], 1);
     }
     __syncthreads();
-    if (tid == 0) {
-        int col = 0, nt = 0;
+    // Column tiles in the order of their work: the full ones of all experts, the ends of more than half a tile, the others.  Launches that
+    // start their tiles in this order end with the short ones.  One thread per expert, sums over the experts before it from LDS.
+    if (tid < n_expert) {
+        const int sh = 31 - __clz(bn);   // bn: 64 or 128
+        int col = 0, n_full = 0, n_big = 0, n_small = 0, full0 = 0, big0 = 0, small0 = 0;
         for (int ex = 0; ex < n_expert; ex++) {
-            first[ex] = col;
-            for (int c = 0; c < cnt[ex]; c += bn, nt++) {
-                tiles[4 * nt] = ex;
-                tiles[4 * nt + 1] = col + c;
-                tiles[4 * nt + 2] = col + cnt[ex];
-                tiles[4 * nt + 3] = 0;
-            }
-            col += cnt[ex];
+            if (ex == tid) { first[ex] = col; full0 = n_full; big0 = n_big; small0 = n_small; }
+            const int c = cnt[ex], f = c >> sh, r = c - (f << sh);
+            col += c;
+            n_full += f;
+            n_big += r > bn / 2;
+            n_small += r > 0 && r <= bn / 2;
         }
-        *n_tiles = nt;
+        const int c = cnt[tid], f = c >> sh, r = c - (f << sh);
+        for (int k = 0; k * bn < c; k++) {
+            int32_t *t = tiles + 4 * (k < f ? full0 + k : r > bn / 2 ? n_full + big0 : n_full + n_big + small0);
+            t[0] = tid;
+            t[1] = first[tid] + k * bn;
+            t[2] = first[tid] + c;
+            t[3] = 0;
+        }
+        if (tid == 0) *n_tiles = n_full + n_big + n_small;
     }
     __syncthreads();
     for (int64_t sl = tid; sl < S; sl += 1024) {
@@ -1234,19 +1322,22 @@ static void launch_mmq_k_id(hipStream_t s, const void *as, const void *act, int6
     const int8_t *aq = (const int8_t *)act;
     const float *ad8 = (const float *)(aq + q8k_d_offset(K, act_rows));
     const _Float16 *abs_ = (const _Float16 *)(aq + q8k_bs_offset(K, act_rows));
-    const int n_row_tiles = (int)((N + 63) / 64);
-    const int n_groups = n_row_tiles * max_tiles;
-    const int n_groups_padded = (n_groups + 7) & ~7;
     const mmq_route route = {act_row, dst_row, tiles, n_tiles, N * L.row_bytes};
+    auto groups = [&](int bm) { return (int)((N + bm - 1) / bm) * max_tiles; };
+    auto padded = [&](int bm) { return (groups(bm) + 7) & ~7; };
     if constexpr (BOTH) {
         if (bn == 64) {
-            MI355_LAUNCH((k_mmq_k<TYPE, 1, 1, 2, true>), dim3((unsigned)n_groups_padded), dim3(256), 0, s, (const uint8_t *)as, aq, ad8, abs_,
-                               dst, nullptr, N, K, S, N, L, max_tiles, n_groups, n_groups_padded, route);
+            MI355_LAUNCH((k_mmq_k<TYPE, 1, 1, 2, true>), dim3((unsigned)padded(64)), dim3(256), 0, s, (const uint8_t *)as, aq, ad8, abs_,
+                               dst, nullptr, N, K, S, N, L, max_tiles, groups(64), padded(64), route);
             return;
         }
     }
-    MI355_LAUNCH((k_mmq_kp<TYPE, true>), dim3((unsigned)n_groups_padded), dim3(256), 0, s, (const uint8_t *)as, aq, ad8, abs_, dst, nullptr, N, K,
-                           S, N, L, max_tiles, n_groups, n_groups_padded, route);
+    if (kp_one_round(N, max_tiles))
+        MI355_LAUNCH((k_mmq_kp<TYPE, true, 64>), dim3((unsigned)groups(64)), dim3(256), 0, s, (const uint8_t *)as, aq, ad8, abs_, dst, nullptr, N, K,
+                               S, N, L, max_tiles, groups(64), groups(64), route);
+    else
+        MI355_LAUNCH((k_mmq_kp<TYPE, true, 128>), dim3((unsigned)groups(128)), dim3(512), 0, s, (const uint8_t *)as, aq, ad8, abs_, dst, nullptr, N, K,
+                               S, N, L, max_tiles, groups(128), groups(128), route);
 }
 
 }  // namespace mi355

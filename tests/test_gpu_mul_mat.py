@@ -392,6 +392,33 @@ def test_ragged_last_column_tile(dev, name, t, K):
             assert orc.nmse(got, want) < 1e-11, (B, split)
 
 
+@pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q5_K, orc.Q6_K, orc.IQ4_XS)])
+@pytest.mark.parametrize("nsb", [1, 2, 3, 4, 5, 8, 16])
+def test_q8k_tile_stages_and_rows(dev, name, t, nsb):
+    """the super-block tile kernel walks K in pairs of super-blocks with the last one or two apart, on tiles of 64 rows (few of them) or
+    128, with half or all of the columns per wave: integer sums are exact, f32 sums over at most 16 super-blocks leave an NMSE of some
+    1e-14.  The large matrix repeats 65 rows, so every output has an equal among the checked ones."""
+    import torch
+    import mi355
+    K = 256 * nsb
+    if (t == orc.Q6_K and K % 2048) or (t == orc.IQ4_XS and K % 512):
+        pytest.skip("rows of no multiple of 16 bytes do not run here")
+    rng = np.random.default_rng(nsb)
+    Wq = _weights(rng, t, 65, K)
+    x = rng.standard_normal((100, K)).astype(np.float32)
+    want = orc.mul_mat("cpu", t, Wq, x)
+    for reps, N in ((2, 130), (260, 65 * 260)):
+        Wd = mi355.upload_weights(t, _to_dev(dev, np.tile(Wq, (reps, 1))))
+        for B in (1, 33, 64, 65, 100):
+            act = mi355.quantize_act_q8k(_to_dev(dev, x[:B]))
+            got = torch.empty((B, N), dtype=torch.float32, device=dev)
+            mi355.check(mi355.load().mi355_mul_mat_q8k(None, t, Wd.data_ptr(), act.data_ptr(), got.data_ptr(), N, K, B, N))
+            torch.cuda.synchronize()
+            first = got[:, :65].cpu().numpy()
+            assert orc.nmse(first, want[:B]) < 1e-11, (N, B)
+            assert torch.equal(got.view(B, reps, 65), got[:, None, :65].expand(B, reps, 65)), (N, B)
+
+
 KQ_TYPES = [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q6_K)]
 TILED_TYPES = [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q5_K, orc.Q6_K, orc.IQ4_XS)]   # types with tile images for the wide-tile GEMM
 
