@@ -795,3 +795,30 @@ def test_tile_kernel_infinite_scales(dev, name, t, B):
             finite = np.isfinite(want)
             assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
             assert orc.nmse(got[finite], want[finite]) < 1e-11
+
+
+@pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q5_K, orc.Q6_K, orc.IQ4_XS)])
+@pytest.mark.parametrize("N", [129, 130, 131, 132])
+def test_slices_of_any_number_of_rows(dev, name, t, N):
+    """a product cut along K whose slabs pad their rows to 16 bytes: integer sums are exact, f32 sums over 16 super-blocks leave an NMSE
+    of some 1e-14; with a residual, and without touching what lies behind a row of dst"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    K, B = 4096, 37
+    rng = np.random.default_rng(N)
+    Wq = _weights(rng, t, N, K)
+    W = mi355.upload_weights(t, _to_dev(dev, Wq))
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    res = rng.standard_normal((B, N + 5)).astype(np.float32)
+    act = mi355.quantize_act_q8k(_to_dev(dev, x))
+    need = int(lib.mi355_mul_mat_q8k_ws_bytes(N, K, B))
+    assert need > 0
+    ws = torch.full((need,), 255, dtype=torch.uint8, device=dev)     # NaNs where nothing is written
+    dst = torch.full((B, N + 5), 7.0, device=dev)
+    r = _to_dev(dev, res)
+    mi355.check(lib.mi355_mul_mat_q8k_ws(None, t, W.data_ptr(), act.data_ptr(), dst.data_ptr(), r.data_ptr(), N, K, B, N + 5, ws.data_ptr(), need))
+    torch.cuda.synchronize()
+    want = orc.mul_mat("cpu", t, Wq, x)
+    assert orc.nmse(dst[:, :N].cpu().numpy(), want + res[:, :N]) < 1e-11
+    assert (dst[:, N:] == 7.0).all()
