@@ -126,6 +126,13 @@ int mi355_mul_mat_static_init(void);
 int mi355_mul_mat_static(void *stream, int type, const void *W, const float *x, float *dst, int64_t N, int64_t K, int64_t B,
                          int64_t x_stride, int64_t dst_stride);
 
+/* MUL_MAT of one to three f32 activation rows as one launch without a workspace: every group quantizes the rows to Q8_1 for itself
+ * (quantize_row_q8_1_ref's bytes), so the result is mi355_mul_mat's bit for bit.  _supported: the product is one that this form serves
+ * quicker than a quantization launch and a product launch; mi355_mul_mat asks it too.  x as for mi355_quantize_act. */
+int mi355_mul_mat_vec_f32_supported(int type, const void *W, int64_t N, int64_t K, int64_t B);
+int mi355_mul_mat_vec_f32(void *stream, int type, const void *W, const float *x, float *dst, int64_t N, int64_t K, int64_t B, int64_t x_stride,
+                          int64_t dst_stride);
+
 /* The two halves of mi355_mul_mat for callers that reuse one quantized activation for
  * several weight matrices (Q/K/V or gate/up projections): `act` from mi355_quantize_act. */
 int mi355_mul_mat_vec_q(void *stream, int type, const void *W, const void *act, float *dst, int64_t N, int64_t K,

@@ -114,6 +114,7 @@ int mi355_mul_mat(void *stream, int type, const void *W, const float *x, float *
         set_error("mul_mat: workspace of %zu bytes, need %zu", ws_bytes, mi355_mul_mat_ws_bytes(K, B));
         return MI355_ERR_WORKSPACE;
     }
+    if (mi355_mul_mat_vec_f32_supported(type, W, N, K, B)) return mi355_mul_mat_vec_f32(stream, type, W, x, dst, N, K, B, x_stride, dst_stride);
     if (use_mid(type, W, K, B)) {
         int rc = mi355_quantize_act_q8k_tiled(stream, x, ws, K, B, x_stride);
         if (rc != MI355_OK) return rc;

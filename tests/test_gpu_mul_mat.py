@@ -797,6 +797,43 @@ def test_tile_kernel_infinite_scales(dev, name, t, B):
             assert orc.nmse(got[finite], want[finite]) < 1e-11
 
 
+@pytest.mark.parametrize("name,t", TYPES)
+def test_few_rows_in_one_launch(dev, name, t):
+    """one to three activation rows quantized inside the product launch: the bytes of a quantization launch and a product launch, at the
+    edges of a group's rows (8 and 16), of one and two rows per wave (2048), of a pass over K (4096 elements) and with padded rows of x"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    be = mi355.BLOCK[t][0]
+    gen = torch.Generator(device=dev).manual_seed(t)
+    shapes = [(1, be, 1), (7, 3 * be, 3), (9, 4096, 2), (2047, 2048, 2), (2049, 1024 + be, 3), (4096, 4096, 3), (4095, 4096 + be, 1), (33, 8192, 1), (14336, 4096, 1)]
+    for N, K, B in shapes:
+        raw = np.random.default_rng(N + K).standard_normal((min(N, 64), K)).astype(np.float32) * 0.02
+        Wq = np.resize(orc.quantize("oracle", t, raw), (N, orc.row_bytes(t, K)))
+        W = mi355.upload_weights(t, _to_dev(dev, Wq))
+        wide = torch.randn(B, K + 8, device=dev, generator=gen)
+        wide[0, :be] = 0.0
+        if B > 1:
+            wide[1, K - 3] = float("inf")
+        x = wide[:, :K]
+        assert lib.mi355_mul_mat_vec_f32_supported(t, W.data_ptr(), N, K, B), (N, K, B)
+        act = torch.empty(int(lib.mi355_act_bytes(K, B)), dtype=torch.uint8, device=dev)
+        want = torch.empty(B, N, device=dev)
+        mi355.check(lib.mi355_quantize_act(None, x.data_ptr(), act.data_ptr(), K, B, x.stride(0)))
+        mi355.check(lib.mi355_mul_mat_vec_q(None, t, W.data_ptr(), act.data_ptr(), want.data_ptr(), N, K, B, N))
+        guard = torch.full((B, N + 3), 7.0, device=dev)
+        mi355.check(lib.mi355_mul_mat_vec_f32(None, t, W.data_ptr(), x.data_ptr(), guard.data_ptr(), N, K, B, x.stride(0), N + 3))
+        torch.cuda.synchronize()
+        assert torch.equal(guard[:, :N].contiguous().view(torch.int32), want.view(torch.int32)), (N, K, B)
+        assert (guard[:, N:] == 7.0).all()
+        assert torch.equal(mi355.mul_mat(t, W, x).view(torch.int32), want.view(torch.int32)), (N, K, B)
+    assert not lib.mi355_mul_mat_vec_f32_supported(t, W.data_ptr(), 4096, 4096, 4)      # more rows, longer rows, many groups: two launches
+    assert not lib.mi355_mul_mat_vec_f32_supported(t, W.data_ptr(), 4096, 14336, 1)
+    assert not lib.mi355_mul_mat_vec_f32_supported(t, W.data_ptr() + 1, 4096, 4096, 1)
+    with pytest.raises(mi355.Mi355Error, match="aligned"):
+        mi355.check(lib.mi355_mul_mat_vec_f32(None, t, W.data_ptr(), x.data_ptr() + 4, guard.data_ptr(), N, K, 1, K, N))
+
+
 @pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q5_K, orc.Q6_K, orc.IQ4_XS)])
 @pytest.mark.parametrize("N", [129, 130, 131, 132])
 def test_slices_of_any_number_of_rows(dev, name, t, N):
