@@ -617,7 +617,8 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
 // unit: two waves per SIMD, so that one wave's matrix instructions run under the other's soft-max arithmetic, and half the
 // tile steps.
 // PQ: the two columns of waves are neighbouring query tiles of one head instead of two heads (an odd number of query heads per kv head)
-template <int D, int NU, bool PQ, bool PX>
+// SPLIT: the cells are cut into a.n_splits ranges of a.cells_per_split (whole tiles), one per group; k_fattn_half_merge joins their states
+template <int D, int NU, bool PQ, bool PX, bool SPLIT = false>
 __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn_mma_half(fattn_args a) {
     constexpr int NTH = 128 * NU, BC = 32 * NU;
     typedef kv_stage<D, NTH, BC> stage_t;
@@ -665,14 +666,17 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
         }
     }
 
+    const int64_t kv_lo = SPLIT ? (int64_t)blockIdx.z * a.cells_per_split : 0;
+    if (SPLIT && kv_lo + a.cells_per_split < kv_limit) kv_limit = kv_lo + a.cells_per_split;
+
     stage_t st;
     u32x2 mnext[4];
     auto prefetch = [&](int64_t kv0) {
         st.fetch(a, hk, kv0, tid);
         fetch_mask<4>(mnext, mrow, mask_aligned && kv0 + BC <= a.Nkv, kv0 + 32 * u + 4 * lhi, a.Nkv);
     };
-    if (!PX || kv_limit > 0) prefetch(0);
-    for (int64_t kv0 = 0; kv0 < kv_limit; kv0 += BC) {
+    if (!PX || kv_lo < kv_limit) prefetch(kv_lo);
+    for (int64_t kv0 = kv_lo; kv0 < kv_limit; kv0 += BC) {
         __syncthreads();   // the previous tile has been consumed
         st.commit(sK, sVt, tid);
         u32x2 mcur[4];
@@ -738,23 +742,130 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
         }
     }
     if (u != 0) return;
-    store_rows<D, PX, NDT>(a, o, l, hk, head, q0, slope, scale, lane);
+    if constexpr (SPLIT) {
+        if (q0 + l32 >= a.Nq) return;
+        const int64_t rows = a.Nq * a.Hq, at = (int64_t)blockIdx.z * rows + (q0 + l32) * a.Hq + head;
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                if (32 * dt + 8 * g >= D) continue;
+                f32x4 w;
+#pragma unroll
+                for (int i = 0; i < 4; i++) w[i] = o[dt][4 * g + i];
+                *(f32x4 *)(a.ws + at * D + 32 * dt + 8 * g + 4 * lhi) = w;
+            }
+        if (lhi == 0) ((float2 *)(a.ws + a.n_splits * rows * D))[at] = float2{m, l};
+    } else {
+        store_rows<D, PX, NDT>(a, o, l, hk, head, q0, slope, scale, lane);
+    }
+}
+
+// Joins the states of a row's ranges of cells, one wave per (query, head) row, in the terms of store_rows: a row that is not finite is
+// computed again by exact_row.
+template <int D, bool PX>
+__global__ void __launch_bounds__(256) k_fattn_half_merge(fattn_args a) {
+    constexpr int E = (D + 63) / 64;
+    const int lane = threadIdx.x & 63;
+    const int64_t rows = a.Nq * a.Hq, row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;   // whole wave
+    const float2 *ml = (const float2 *)(a.ws + a.n_splits * rows * D);
+    const float2 mine = lane < a.n_splits ? ml[lane * rows + row] : float2{FM_NEG, 0.0f};
+    const float f = merge_factor<PX>(mine.x, wave_max_dpp(mine.x));
+    const float l = wave_sum_dpp(lane < a.n_splits ? mine.y * f : 0.0f);
+    float o[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) o[e] = 0.0f;
+    for (int s0 = 0; s0 < a.n_splits; s0 += 4) {   // four ranges' values requested together; past the end the last one again, times 0
+        float v[4][E];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                const int sp = s0 + j < a.n_splits ? s0 + j : a.n_splits - 1, d = 64 * e + lane;
+                v[j][e] = d < D ? a.ws[(sp * rows + row) * D + d] : 0.0f;
+            }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float fs = s0 + j < a.n_splits ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), s0 + j)) : 0.0f;
+#pragma unroll
+            for (int e = 0; e < E; e++) o[e] = fmaf(v[j][e], fs, o[e]);
+        }
+    }
+    float z = l * 0.0f;
+#pragma unroll
+    for (int e = 0; e < E; e++) z = fmaf(o[e], 0.0f, z);
+    const int64_t iq = row / a.Hq, head = row % a.Hq;
+    if (__ballot(z != 0.0f) != 0) {
+        exact_row<D, PX>(a, head / (a.Hq / a.Hkv), head, iq, alibi_slope(a, head), a.softcap != 0.0f ? a.scale / a.softcap : a.scale, lane);
+        return;
+    }
+    const float sum = sum_of<PX>(l), inv = reciprocal_of<PX>(sum);
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int d = 64 * e + lane;
+        if (d < D) a.dst[row * D + d] = quotient<PX>(o[e], sum, inv);
+    }
+}
+
+// How many ranges the cells are cut into.  A group's walk is a serial chain, so a launch of few groups takes as long as one of them however idle
+// the chip is; the states of more ranges cost a merge launch and their way through memory.  The time in us of n ranges, from a sweep over
+// (64 .. 256 head size, 24 .. 256 groups, 2 .. 256 tiles of 64 cells, n = 1 .. 16), which it meets within some 15 %: a tile step takes
+// 0.95 (D 64), 1.4 (up to 128) or 3.4 us (256: one group per compute unit), 1.34 times that with a second group on the compute unit; the merge 4
+// and 8 bytes per value and range at 4 TB/s.  Before / after, us: 64 rows over 8192 cells, 32 / 8 heads, D 128 146 -> 32; 343 x 3840, 4 / 4 heads, D 64
+// 51 -> 18; 268 x 3776, 32 / 8, D 128 77 -> 50; 512 x 4096 81 -> 72 (n = 2); 300 x 2500, 8 / 8, D 256 136 -> 41; not cut: 560 x 672, 16 / 4 (22.5; 27 in three).
+// (probabilities of f32 precision: one launch up to 2048 cells)
+static bool half_may_split(const fattn_args &a, bool px) { return (!px || a.Nkv > 2048) && a.ws != nullptr && ((uintptr_t)a.ws & 15) == 0; }
+struct half_plan { int64_t n; float us; };
+static half_plan plan_half(int64_t D, int64_t groups, int64_t rows, int64_t tiles, bool wide, size_t ws_bytes) {
+    const float step = D == 64 ? 0.95f : D <= 128 ? 1.4f : 3.4f;
+    half_plan best = {1, 0.0f};
+    float whole = 0.0f;
+    for (int64_t n = 1; n <= 64 && n <= tiles; n++) {
+        if (n > 1 && ws_bytes < (size_t)n * (size_t)rows * (size_t)(D + 2) * sizeof(float)) break;
+        const int64_t g = groups * n, slots = D <= 128 ? 512 : 256;
+        const float busy = g <= 256 ? 1.0f : (float)((g + slots - 1) / slots) * (D <= 128 ? 1.34f : 1.0f);
+        float us = (float)((tiles + n - 1) / n) * step * busy;
+        if (n == 1 && wide) us *= 0.9f;   // eight waves on 128-cell tiles
+        if (n > 1) us += 4.0f + (float)(rows * n * D) * 8.0f / 4e6f;
+        if (n == 1) whole = us;
+        if (n == 1 || (us < best.us && us < 0.9f * whole)) best = {n, us};
+    }
+    return best;
+}
+
+// groups of the launch below
+static dim3 half_grid(const fattn_args &a, bool pq) {
+    const int64_t R = a.Hq / a.Hkv, n_tiles = (a.Nq + 31) / 32;
+    return dim3((unsigned)(pq ? (n_tiles + 1) / 2 : n_tiles), (unsigned)(a.Hkv * (pq ? R : R / 2)));
 }
 
 template <int D, bool PQ, bool PX>
-int launch_half(hipStream_t s, const fattn_args &a) {
-    const int64_t R = a.Hq / a.Hkv, n_tiles = (a.Nq + 31) / 32;
-    const dim3 grid((unsigned)(PQ ? (n_tiles + 1) / 2 : n_tiles), (unsigned)(a.Hkv * (PQ ? R : R / 2)));
+int launch_half(hipStream_t s, fattn_args a, size_t ws_bytes) {
+    dim3 grid = half_grid(a, PQ);
+    const int64_t groups = (int64_t)grid.x * grid.y, rows = a.Nq * a.Hq, tiles = (a.Nkv + 63) / 64;
     // at most one group per compute unit and a long cache: eight waves on 128-cell tiles (512 rows: 4096 cells 112 -> 103 us,
-    // 512 cells 24.8 -> 26.2 us)
-    if constexpr (D <= 128) {   // (head size 256: the eight waves' registers do not fit)
-        if ((int64_t)grid.x * grid.y <= 256 && a.Nkv >= 1024) {
+    // 512 cells 24.8 -> 26.2 us).  Head size 256: the eight waves' registers do not fit.
+    const bool wide = D <= 128 && groups <= 256 && a.Nkv >= 1024;
+    const int64_t n = half_may_split(a, PX) ? plan_half(D, groups, rows, tiles, wide, ws_bytes).n : 1;
+    a.cells_per_split = (tiles + n - 1) / n * 64;
+    a.n_splits = (int)((a.Nkv + a.cells_per_split - 1) / a.cells_per_split);   // no empty range
+    grid.z = (unsigned)a.n_splits;
+    if constexpr (D <= 128) {
+        if (wide && a.n_splits == 1) {
             MI355_LAUNCH((k_fattn_mma_half<D, 4, PQ, PX>), grid, dim3(512), 0, s, a);
             return launch_status("k_fattn_mma_half");
         }
     }
-    MI355_LAUNCH((k_fattn_mma_half<D, 2, PQ, PX>), grid, dim3(256), 0, s, a);
-    return launch_status("k_fattn_mma_half");
+    if (a.n_splits == 1) {
+        MI355_LAUNCH((k_fattn_mma_half<D, 2, PQ, PX>), grid, dim3(256), 0, s, a);
+        return launch_status("k_fattn_mma_half");
+    }
+    MI355_LAUNCH((k_fattn_mma_half<D, 2, PQ, PX, true>), grid, dim3(256), 0, s, a);
+    const int rc = launch_status("k_fattn_mma_half");
+    if (rc != MI355_OK) return rc;
+    MI355_LAUNCH((k_fattn_half_merge<D, PX>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, a);
+    return launch_status("k_fattn_half_merge");
 }
 
 template <int D, int HPW, bool PX>
@@ -777,12 +888,12 @@ int launch_hpw(hipStream_t s, const fattn_args &a) {
 // Pairs of probabilities: head sizes 112 and 128 always in halves (the registers of whole tiles do not fit: 50 and 33 spills; 2048 x 2048 cells,
 // 32 / 8 heads: 165 -> 139 and 160 -> 155 us), head size 64 too (the error of its longer sums would exceed the vector kernel's, 1.39e-7 against 1.36e-7; halves 1.34e-7)
 template <int D, bool PX>
-int launch_head(hipStream_t s, const fattn_args &a, bool pq, bool half) {
+int launch_head(hipStream_t s, const fattn_args &a, size_t ws_bytes, bool pq, bool half) {
     constexpr bool HALVES_ONLY = PX && (D == 64 || D == 112 || D == 128);
     if constexpr (!HALVES_ONLY) {
         if (!half) return launch_hpw<D, PX>(s, a);
     }
-    return pq ? launch_half<D, true, PX>(s, a) : launch_half<D, false, PX>(s, a);
+    return pq ? launch_half<D, true, PX>(s, a, ws_bytes) : launch_half<D, false, PX>(s, a, ws_bytes);
 }
 
 // ---- decode / small batches: the 32 MFMA columns are (token, head of the GQA group) pairs -------
@@ -1002,7 +1113,7 @@ int launch_fattn_mma(hipStream_t s, fattn_args &a, int64_t D, size_t ws_bytes) {
     // 2048 x 2048, 32 / 8 heads: D 80 2046 -> 111, 1.56e-7 -> 1.49e-7; D 112 2049 -> 139, 1.55e-7 -> 1.47e-7; D 256 4346 -> 252, 1.71e-7 -> 1.59e-7;
     // D 128 with quantized output 2056 -> 155, 1.55e-7 -> 1.44e-7, 768 x 2048 812 -> 91, 2.49e-7 -> 2.05e-7.
     const bool pq = R % 2 != 0, half = (pq ? (n_tiles + 1) / 2 * a.Hq : n_tiles * a.Hq / 2) <= 512;
-#define MI355_FM_HEAD(D_, PX_) return launch_head<D_, PX_>(s, a, pq, half);
+#define MI355_FM_HEAD(D_, PX_) return launch_head<D_, PX_>(s, a, ws_bytes, pq, half);
     switch (D) {
         case 64: if (px) MI355_FM_HEAD(64, true) else MI355_FM_HEAD(64, false)
         case 80: MI355_FM_HEAD(80, true)
