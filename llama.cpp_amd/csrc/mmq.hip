@@ -674,29 +674,51 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
 // IQ4_NL 149 -> 128, Q8_0 146 -> 130; 64 rows: Q4_0 34.3 -> 32.3.  Q6_K with 16-element instead of masked 32-element matrix
 // instructions: 4096 x 11008, 64 rows 41.2 -> 39.5.
 //
+static size_t mmq_slab_bytes(int n, int64_t rows, int64_t B) { return (size_t)n * (size_t)rows * (size_t)B * sizeof(float); }
+
 // A product with few tiles leaves most of the chip idle while each group walks all of K: such launches are cut along K into
 // slices that run side by side and a second launch adds the slices in fixed order.  At least four stages per slice, at most
-// eight slices, at most two groups per compute unit.
-static int mmq_slices(int64_t row_tiles, int64_t K, int64_t B) {
+// eight slices, at most two groups per compute unit; more of them, up to sixteen, where a model of the time in us says so, which a sweep of n = 1 .. 16 over
+// (1024 .. 21603 rows, 10 .. 112 stages, 50 .. 512 columns) meets within some 15 %: a stage takes 1.2 (64 columns) or 2.1 (128), Q6_K 1.7 times that; 1.4
+// times with a second group on the compute unit; the sum 4, and 8 bytes per value and slice at 4 TB/s.  A call, us: Q6_K 1135 x 7424, 65 rows
+// 41.2 -> 30.9 (16 slices instead of 8), Q5_1 3509 x 1216, 73 rows 23.6 -> 18.9 (5 instead of 2).  (Fewer slices than these would be quicker here
+// and there, Q5_0 8491 x 2016, 316 rows 49.9 -> 44.5 with one instead of two, but make longer f32 sums.)
+// ws_bytes: what is there for the partial sums; none of them fits: one slice.
+static int mmq_slices(int type, int64_t row_tiles, int64_t K, int64_t B, int64_t rows, size_t ws_bytes) {
     const int64_t bn = B <= 64 ? 64 : 128;
     const int64_t groups = row_tiles * ((B + bn - 1) / bn), stages = (K + MMQ_BK - 1) / MMQ_BK;
-    int64_t n = 512 / groups;
-    if (n > stages / 4) n = stages / 4;
-    if (n > 8) n = 8;
-    if (n < 2) return 1;
-    const int64_t per = (stages + n - 1) / n;
-    return (int)((stages + per - 1) / per);   // no empty slice
+    int64_t least = 512 / groups;
+    if (least > stages / 4) least = stages / 4;
+    if (least > 8) least = 8;
+    if (least < 1) least = 1;
+    least = (stages + (stages + least - 1) / least - 1) / ((stages + least - 1) / least);   // no empty slice
+    const float stage = (bn == 64 ? 1.2f : 2.1f) * (type == MI355_Q6_K ? 1.7f : 1.0f);
+    int64_t best = 1;
+    float best_us = 0.0f;
+    for (int64_t n = least; n <= 16 && n <= stages; n++) {
+        const int64_t per = (stages + n - 1) / n, g = groups * n;
+        if (n > 1 && mmq_slab_bytes((int)n, rows, B) > ws_bytes) break;
+        if ((stages + per - 1) / per != n) continue;
+        const float busy = g <= 256 ? 1.0f : 1.4f * (float)((g + 511) / 512);
+        const float us = (float)per * stage * busy + (n > 1 ? 4.0f + (float)(n * rows * B) * 8.0f / 4e6f : 0.0f);
+        if (n == least || us < 0.95f * best_us) {
+            best = n;
+            best_us = us;
+        }
+    }
+    return (int)best;
 }
 static int64_t mmq_row_tiles(int n_mats, const int64_t *Ns) {
     int64_t t = 0;
     for (int i = 0; i < n_mats; i++) t += (Ns[i] + MMQ_BM - 1) / MMQ_BM;
     return t;
 }
-static size_t mmq_ws_bytes(int n_mats, const int64_t *Ns, int64_t K, int64_t B) {
-    const int n = mmq_slices(mmq_row_tiles(n_mats, Ns), K, B);
+static size_t mmq_ws_bytes(int n_mats, const int64_t *Ns, int64_t K, int64_t B) {   // for any type
     int64_t rows = 0;
     for (int i = 0; i < n_mats; i++) rows += Ns[i];
-    return n > 1 ? (size_t)n * (size_t)rows * (size_t)B * sizeof(float) : 0;
+    const int64_t row_tiles = mmq_row_tiles(n_mats, Ns);
+    const int a = mmq_slices(MI355_Q4_0, row_tiles, K, B, rows, SIZE_MAX), b = mmq_slices(MI355_Q6_K, row_tiles, K, B, rows, SIZE_MAX), n = a > b ? a : b;
+    return n > 1 ? mmq_slab_bytes(n, rows, B) : 0;
 }
 
 // dst[b][n] of every matrix = sum of its slices in ascending order (+ residual).  part: [slice][B][rows of all matrices]
@@ -746,8 +768,7 @@ static void launch_mmq(hipStream_t s, int n_mats, const mi355_gemv_mat *mats, co
     const int n_col_tiles = (int)((B + BN - 1) / BN);
     const int n_groups = row_tiles * n_col_tiles;
     const int n_groups_padded = (n_groups + 7) & ~7;
-    int n_slices = mmq_slices(row_tiles, K, B);
-    if (n_slices > 1 && (ws == nullptr || ((uintptr_t)ws & 15) != 0 || ws_bytes < mmq_ws_bytes(n_mats, Ns, K, B))) n_slices = 1;
+    const int n_slices = mmq_slices(TYPE, row_tiles, K, B, rows, ws == nullptr || ((uintptr_t)ws & 15) != 0 ? 0 : ws_bytes);
     const dim3 grid((unsigned)n_groups_padded, (unsigned)n_slices);
     MI355_LAUNCH((k_mmq<TYPE, TN>), grid, dim3(256), 0, s, n_slices > 1 ? part : a, aq, ads, K, B, L, n_col_tiles, n_groups, n_groups_padded, rows * B, mmq32_route{});
     if (n_slices > 1) MI355_LAUNCH(k_mmq_split_sum, dim3((unsigned)((rows * B + 255) / 256)), dim3(256), 0, s, (const float *)ws, a, rows, B, n_slices);
