@@ -430,10 +430,21 @@ __global__ void __launch_bounds__(512) k_fattn_combine(const float *__restrict__
     }
 }
 
-static int pick_splits(int64_t Nkv, int64_t Hkv, int64_t Nq) {
-    int64_t by_len = (Nkv + 255) / 256;
-    int64_t by_fill = 2048 / (Hkv * Nq > 0 ? Hkv * Nq : 1);
+// query heads a group serves from one pass over the kv head's bytes
+static int heads_per_group(int64_t R) { return R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1; }
+
+// Ranges of cells, one per group.  At least one per 256 cells while that makes 2048 groups at most; as short as 64 cells while there are no
+// more than 512 groups, two per compute unit: a group's walk is a serial chain (some 3 us per 32 cells of D 256), and with 256 cells each a
+// launch of few kv heads took as long as a chain of eight such steps on a nearly idle chip.  One row, 32 / 8 heads of 256, us a call, 256 cells each / this
+// rule (n: ranges): 2048 cells 28.9 / 13.7 (32), 4096 29.7 / 18.4 (64; 20.0 with 32, 23.8 with 128); 64 / 8 heads, 4096 29.6 / 22.1 (32; 24.9 with 64);
+// 32 / 32 heads, 4096 28.5 either way (16; 32.4 with 64).  D 80 at 2048 and 4096 cells is the host's 13.5 us for two launches.  A Q8_0 cache, 64 / 8 heads of 128:
+// 512 cells 15.1 / 11.5, 1024 15.3 / 11.6, 2048 15.3 / 11.6.
+static int pick_splits(int64_t Nkv, int64_t Hkv, int64_t Hq, int64_t Nq) {
+    const int64_t by_len = (Nkv + 255) / 256, by_fill = 2048 / (Hkv * Nq);
+    const int64_t fine_len = (Nkv + 63) / 64, fine_fill = 512 / (Hq / heads_per_group(Hq / Hkv) * Nq);
     int64_t n = by_len < by_fill ? by_len : by_fill;
+    const int64_t fine = fine_len < fine_fill ? fine_len : fine_fill;
+    if (n < fine) n = fine;
     if (n < 1) n = 1;
     if (n > 256) n = 256;
     return (int)n;
@@ -471,7 +482,7 @@ template <int D>
 static int launch_vec_r(hipStream_t s, fattn_args &a, int R) {
     // R = query heads served per group from one pass over the kv head's bytes.  A short context is not bandwidth-bound but
     // a serial chain of soft-max updates per (step, head): one head per group then spreads it over R times as many waves.
-    // Up to 1024 cells and few (token, head) pairs: one head per group, eight waves per group (32 cells of a D = 128 head per step,
+    // Up to some hundred cells and few (token, head) pairs: one head per group, eight waves per group (32 cells of a D = 128 head per step,
     // four steps' loads in flight) and no split of the cells over groups, so no second launch.  Measured per decoded token of
     // the 8B model at 256 cells: 4 waves 1.897 ms, 8 waves 1.856 ms, 16 waves 1.875 ms; requesting K and V together with the mask
     // instead of after it (one round trip less per step, but masked cells - rows of the cache that may never have been written - then
@@ -481,16 +492,25 @@ static int launch_vec_r(hipStream_t s, fattn_args &a, int R) {
     // (quantized operands cost more arithmetic per cell: from 257 cells on their cells are split over groups)
     const bool quantized = a.type_k != MI355_F16 || a.type_v != MI355_F16;
     if (a.Nkv <= one_head_max && !(quantized && a.Nkv > 256 && a.n_splits > 1)) {
-        if (a.Nq * a.Hq <= 512) {   // few (token, head) pairs: the chip is far from full
+        if (a.Nq * a.Hq > 512) return launch_vec<D, 1>(s, a);
+        // few (token, head) pairs: the chip is far from full
+        constexpr int64_t step = 8 * 4 * (D <= 64 ? 8 : D <= 128 ? 4 : 2);   // cells a group of eight waves takes per step
+        // One launch against ranges of cells and a merge launch, us a call: D 256 (step 64), 32 / 8 heads, 448 cells 11.8 / 13.4, 512 14.9 / 13.5,
+        // 1024 29.5 / 13.1; 16 / 8 heads, 512 cells 12.9 / 14.1, 640 15.2 / 14.1, 1024 25.6 / 14.0; D 80 (step 128), 32 / 8 heads, 768 cells 10.7 / -,
+        // 896 14.9 / 13.3, 1024 17.1 / 13.6; 8 / 8 heads, 1024 cells 12.3 / 13.4: neighbouring heads of a kv head run on different XCDs and
+        // each fetches the rows, so more heads are slower.
+        const int64_t lim = a.Hq <= 16 ? 8 : D > 128 ? 7 : 6;
+        if (quantized || a.Nkv <= lim * step || a.n_splits < 4) {
             a.n_splits = 1;
             a.cells_per_split = a.Nkv;
             return launch_vec<D, 1, 8>(s, a);
         }
-        return launch_vec<D, 1>(s, a);
     }
-    if (R % 4 == 0) return launch_vec<D, 4>(s, a);
-    if (R % 2 == 0) return launch_vec<D, 2>(s, a);
-    return launch_vec<D, 1>(s, a);
+    switch (heads_per_group(R)) {
+        case 4: return launch_vec<D, 4>(s, a);
+        case 2: return launch_vec<D, 2>(s, a);
+        default: return launch_vec<D, 1>(s, a);
+    }
 }
 
 // checks shared by the entry points and the argument block of the kernels; quantized operands skip the f16 row checks
@@ -519,12 +539,12 @@ static int fattn_fill(fattn_args &a, const float *q, const void *k, const void *
     a.n_head_log2 = n2;
     a.m0 = powf(2.0f, -(max_bias) / n2);
     a.m1 = powf(2.0f, -(max_bias / 2.0f) / n2);
-    a.n_splits = pick_splits(Nkv, Hkv, Nq);
-    if (a.n_splits > 1) {
-        const size_t need = (size_t)Nq * (size_t)Hq * (size_t)a.n_splits * (size_t)(D + 2) * sizeof(float);
-        if (ws == nullptr || ws_bytes < need) a.n_splits = 1;   // no scratch: run unsplit
-    }
-    a.cells_per_split = (Nkv + a.n_splits - 1) / a.n_splits;
+    const size_t per_split = (size_t)Nq * (size_t)Hq * (size_t)(D + 2) * sizeof(float);
+    const int64_t fit = ws ? (int64_t)(ws_bytes / per_split) : 0;   // as many as the scratch holds; none: run unsplit
+    int64_t n = pick_splits(Nkv, Hkv, Hq, Nq);
+    if (n > fit) n = fit > 1 ? fit : 1;
+    a.cells_per_split = (Nkv + n - 1) / n;
+    a.n_splits = (int)((Nkv + a.cells_per_split - 1) / a.cells_per_split);   // no empty range
     return MI355_OK;
 }
 

@@ -457,3 +457,41 @@ def test_prefill_ranges_of_cells(dev, D, Nkv, Nq, Hq, Hkv):
     bound = 1e-6 if D in (64, 128) else 1e-12
     assert orc.nmse(whole[seen], want) < bound
     assert orc.nmse(got[seen], want) < bound
+
+
+@pytest.mark.parametrize("Nq", [1, 3])
+@pytest.mark.parametrize("D,Hq,Hkv,one", [(80, 32, 8, 768), (80, 16, 16, 1024), (112, 6, 3, 1024), (256, 32, 8, 448), (256, 16, 2, 512), (256, 33, 11, 448)])
+def test_decode_ranges_of_cells(dev, D, Hq, Hkv, one, Nq):
+    """few rows of a head size that only the vector kernel takes: one launch up to `one` cells, ranges as short as 64 cells and a merge
+    beyond; ragged ends, ranges without a visible cell, masked cells that hold anything, and scratch memory for fewer ranges than the rule
+    asks for.  f32 probabilities: some 3e-7 of the result (NMSE 1e-13)"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    rng = np.random.default_rng(D + Hq)
+    scale = 1.0 / np.sqrt(D)
+    for Nkv, launches in ((one, 1), (one + 1, 2), (1090, 2), (2049, 2), (4160, 2)):
+        q, k, v, mask = _inputs(rng, D, Nq, Nkv, Hq, Hkv, rand_mask=True)
+        mask[:, 130:260] = -np.inf
+        v[:, 140] = np.nan
+        k[:, 150] = np.inf
+        args = [torch.from_numpy(a).to(dev) for a in (q, k, v, mask)]
+        before = lib.mi355_launch_count()
+        got = mi355.flash_attn_ext(*args, scale).cpu().numpy()
+        assert lib.mi355_launch_count() - before == launches, Nkv
+        whole = mi355.flash_attn_ext(*args, scale, workspace=False).cpu().numpy()
+        qd, kd, vd, md = args
+        ws = torch.empty(3 * Nq * Hq * (D + 2) * 4, dtype=torch.uint8, device=dev)   # three ranges
+        dst = torch.empty((Nq, Hq, D), dtype=torch.float32, device=dev)
+        mi355.check(lib.mi355_flash_attn_ext(torch.cuda.current_stream().cuda_stream, qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), md.data_ptr(), dst.data_ptr(),
+                                             D, Nq, Nkv, Hq, Hkv, qd.stride(1) * 4, qd.stride(0) * 4, kd.stride(1) * 2, kd.stride(0) * 2, vd.stride(1) * 2,
+                                             vd.stride(0) * 2, md.stride(0) * 2, scale, 0.0, 0.0, ws.data_ptr(), ws.numel()))
+        v[:, 140] = 0
+        k[:, 150] = 0
+        want = _textbook(q, k, v, mask, scale)
+        for out in (got, whole, dst.cpu().numpy()):
+            assert orc.nmse(out, want) < 1e-12, Nkv
+        if D % 32 == 0:
+            rows, act = mi355.flash_attn_ext(*args, scale, quantized=True)
+            assert np.array_equal(rows.cpu().numpy(), got)
+            assert torch.equal(act, mi355.quantize_act(rows.reshape(Nq, Hq * D)))
