@@ -125,7 +125,9 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
     __shared__ float s_o[NW][R][D];
 
     const int split = blockIdx.x;
-    const int64_t hk = blockIdx.y / a.groups, hg = blockIdx.y % a.groups, iq = blockIdx.z;
+    // neighbouring groups are different kv heads: workgroups go to the XCDs in turn, so the groups of one kv head (a multiple of 8 apart where there are
+    // 8 kv heads, or 16) share an L2 and its rows are fetched once (64 / 8 heads of 256, 448 cells: 15.5 -> 11.6 us; 32 / 8 heads of 80, 1024: 17.0 -> 12.1)
+    const int64_t hk = blockIdx.y % (unsigned)a.Hkv, hg = blockIdx.y / (unsigned)a.Hkv, iq = blockIdx.z;
     const int64_t head0 = (hk * a.groups + hg) * R;   // first of this group's R query heads
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sub = lane % LPR, slot = wave * CPW + lane / LPR;
@@ -495,11 +497,10 @@ static int launch_vec_r(hipStream_t s, fattn_args &a, int R) {
         if (a.Nq * a.Hq > 512) return launch_vec<D, 1>(s, a);
         // few (token, head) pairs: the chip is far from full
         constexpr int64_t step = 8 * 4 * (D <= 64 ? 8 : D <= 128 ? 4 : 2);   // cells a group of eight waves takes per step
-        // One launch against ranges of cells and a merge launch, us a call: D 256 (step 64), 32 / 8 heads, 448 cells 11.8 / 13.4, 512 14.9 / 13.5,
-        // 1024 29.5 / 13.1; 16 / 8 heads, 512 cells 12.9 / 14.1, 640 15.2 / 14.1, 1024 25.6 / 14.0; D 80 (step 128), 32 / 8 heads, 768 cells 10.7 / -,
-        // 896 14.9 / 13.3, 1024 17.1 / 13.6; 8 / 8 heads, 1024 cells 12.3 / 13.4: neighbouring heads of a kv head run on different XCDs and
-        // each fetches the rows, so more heads are slower.
-        const int64_t lim = a.Hq <= 16 ? 8 : D > 128 ? 7 : 6;
+        // One launch against ranges of cells and a merge launch, us a call: D 256 (step 64), 32 / 8 heads, 512 cells 12.7 / 14.2, 576 14.0 / 14.1, 1024
+        // 29 / 13.5; D 80 (step 128), 32 / 8 heads, 1024 cells 12.1 / 14.1; many kv heads, whose rows have no L2 in common: D 80, 32 / 32 heads,
+        // 768 cells 12.7 / 14, 896 15.1 / 14.0, 1024 16.8 / 13.9; D 256, 32 / 32 heads, 448 cells 12.8 / 14, 512 14.2 / 14.2, 576 17.3 / 14.0.
+        const int64_t lim = a.Hkv <= 24 ? 8 : D > 128 ? 7 : 6;
         if (quantized || a.Nkv <= lim * step || a.n_splits < 4) {
             a.n_splits = 1;
             a.cells_per_split = a.Nkv;

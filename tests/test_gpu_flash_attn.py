@@ -460,7 +460,7 @@ def test_prefill_ranges_of_cells(dev, D, Nkv, Nq, Hq, Hkv):
 
 
 @pytest.mark.parametrize("Nq", [1, 3])
-@pytest.mark.parametrize("D,Hq,Hkv,one", [(80, 32, 8, 768), (80, 16, 16, 1024), (112, 6, 3, 1024), (256, 32, 8, 448), (256, 16, 2, 512), (256, 33, 11, 448)])
+@pytest.mark.parametrize("D,Hq,Hkv,one", [(80, 32, 8, 1024), (80, 25, 25, 768), (80, 20, 20, 1024), (112, 6, 3, 1024), (256, 32, 8, 512), (256, 16, 2, 512), (256, 33, 11, 512), (256, 50, 25, 448)])
 def test_decode_ranges_of_cells(dev, D, Hq, Hkv, one, Nq):
     """few rows of a head size that only the vector kernel takes: one launch up to `one` cells, ranges as short as 64 cells and a merge
     beyond; ragged ends, ranges without a visible cell, masked cells that hold anything, and scratch memory for fewer ranges than the rule
