@@ -496,20 +496,27 @@ template <int TK, int TV>
 constexpr int fsq_waves() { return TK == MI355_Q8_0 && TV == MI355_Q8_0 ? 3 : (TK == MI355_Q4_0 && TV == MI355_Q4_0 ? 5 : 4); }
 static int fsq_waves_rt(int tk, int tv) { return tk == MI355_Q8_0 && tv == MI355_Q8_0 ? 3 : (tk == MI355_Q4_0 && tv == MI355_Q4_0 ? 5 : 4); }
 constexpr int FSQ_TOTAL_GROUPS = 256;
-
+// ONE: no wave has more than one tile.  A wave then keeps one stage, LDS holds more of them (of Q8_0 five at 26 KiB each, of Q4_0 eight at 18 KiB), and
+// the group's waves join their states, so that the merge launch reads one result per group.  In its place two waves walked two to four tiles
+// each: 8192 cells, 32 / 8 heads, Q8_0 16.9 -> 16.2 us, Q4_0 15.9 -> 14.7; 8 / 8 heads 15.7 -> 13.5 and 15.2 -> 13.2; 10240 cells of Q4_0 20.5 -> 16.8.  A result
+// per wave costs more than the chain it saves (Q8_0, 8192 cells, 32 / 8: 18.2 us); two waves with a tile or more each lose by joining (4096 cells 13.4 -> 14.3).
 template <int TK, int TV>
-__global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_stream_q(fattn_args a, fsq_src ksrc, fsq_src vsrc, int tiles_per_wave, int n_tiles, int R) {
+constexpr int fsq_waves_one() { return TK == MI355_Q8_0 && TV == MI355_Q8_0 ? 5 : (TK == MI355_Q4_0 && TV == MI355_Q4_0 ? 8 : 6); }
+static int fsq_waves_one_rt(int tk, int tv) { return tk == MI355_Q8_0 && tv == MI355_Q8_0 ? 5 : (tk == MI355_Q4_0 && tv == MI355_Q4_0 ? 8 : 6); }
+
+template <int TK, int TV, bool ONE>
+__global__ void __launch_bounds__(((ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK, TV>()) * 64), 1) k_fattn_dec_stream_q(fattn_args a, fsq_src ksrc, fsq_src vsrc, int tiles_per_wave, int n_tiles, int R) {
     typedef fsq_geo<TK> GK;
     typedef fsq_geo<TV> GV;
-    constexpr int NWV = fsq_waves<TK, TV>();
+    constexpr int NWV = ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK, TV>(), STAGES = ONE ? 1 : 2, MT = ONE ? 8 : FSQ_MAX_TILES;
     constexpr int K_LV = FS_TILE * GK::ROW, V_LV = FS_TILE * GV::ROW;
     constexpr int OFF_V = K_LV, OFF_KS = K_LV + V_LV, OFF_VS = OFF_KS + FSQ_SCALES;
     constexpr int STAGE = OFF_VS + FSQ_SCALES;
     constexpr int CK = GK::CNT, CV = GV::CNT;   // transfers of the K / V part of a tile
-    __shared__ __attribute__((aligned(1024))) uint8_t ring_buf[NWV * 2 * STAGE];
+    __shared__ __attribute__((aligned(1024))) uint8_t ring_buf[NWV * STAGES * STAGE];
     __shared__ __attribute__((aligned(1024))) uint8_t vf_buf[NWV * FSQ_VF];   // half of the wave's V tile as f16
     __shared__ __attribute__((aligned(16))) unsigned short pbuf[NWV][4][FS_TILE];
-    __shared__ __attribute__((aligned(16))) unsigned short mbuf[NWV][FSQ_MAX_TILES * FS_TILE];
+    __shared__ __attribute__((aligned(16))) unsigned short mbuf[NWV][MT * FS_TILE];
     asm volatile("" ::"v"((void *)ring_buf), "v"((void *)vf_buf) : "memory");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int split = (int)blockIdx.x * (int)(blockDim.x >> 6) + wave;   // the launch may give a group fewer than NWV waves
@@ -521,7 +528,7 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
 
     float slope[4];
     fs_slopes(a, hk * R, slope);
-    uint8_t *ring = ring_buf + wave * (2 * STAGE);
+    uint8_t *ring = ring_buf + wave * (STAGES * STAGE);
     const uint8_t *k_lv = ksrc.lv + hk * ksrc.head_lv, *k_sc = ksrc.sc + hk * ksrc.head_sc;
     const uint8_t *v_lv = vsrc.lv + hk * vsrc.head_lv, *v_sc = vsrc.sc + hk * vsrc.head_sc;
     // per-lane offsets of the transfers.  K levels: transfer i moves rows RPT i .. + RPT - 1, lane p -> row RPT i + p / CH, LDS position
@@ -592,7 +599,7 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
         issue(0, 0, 0);
         issue(0, 0, 1);
     }
-    if (n > 1) {
+    if (!ONE && n > 1) {
         issue(1, 1, 0);
         issue(1, 1, 1);
     }
@@ -618,9 +625,9 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
     {
         const unsigned short *mrow = (const unsigned short *)a.mask;
         const bool wide = ((uintptr_t)mrow & 15) == 0;
-        u32x4 mc[FSQ_MAX_TILES / 8];
+        u32x4 mc[MT / 8];
 #pragma unroll
-        for (int it = 0; it < FSQ_MAX_TILES / 8; it++) {
+        for (int it = 0; it < MT / 8; it++) {
             const int j = it * 64 + lane;
             const int64_t c = c_begin + (int64_t)j * 8;
             mc[it] = u32x4{0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u};   // -inf
@@ -637,7 +644,7 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
             }
         }
 #pragma unroll
-        for (int it = 0; it < FSQ_MAX_TILES / 8; it++) {
+        for (int it = 0; it < MT / 8; it++) {
             const int j = it * 64 + lane;
             if (j * 8 < n * FS_TILE) *(u32x4 *)(mw + j * 8) = mc[it];
         }
@@ -652,9 +659,9 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
     const unsigned p_wr = p_base + (unsigned)lane * 2, p_rd = p_base + (unsigned)hr * (FS_TILE * 2);
 
     for (int t = 0; t < n; t++) {
-        const int st = t & 1;
+        const int st = ONE ? 0 : t & 1;
         // K(t) has landed when at most V(t), K(t + 1), V(t + 1) are still on their way (transfers complete in the order issued)
-        if (t + 1 < n) FS_WAIT_VM(CV + CK + CV);
+        if (!ONE && t + 1 < n) FS_WAIT_VM(CV + CK + CV);
         else FS_WAIT_VM(CV);
         const unsigned sb = ring_lds + (unsigned)st * STAGE;
         u32x4 kc[GK::CH];
@@ -668,23 +675,68 @@ __global__ void __launch_bounds__((fsq_waves<TK, TV>() * 64), 1) k_fattn_dec_str
             asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(mbits), "+v"(ksc), "+v"(kc[0]), "+v"(kc[1]), "+v"(kc[2]), "+v"(kc[3]), "+v"(kc[4]), "+v"(kc[5]), "+v"(kc[6]), "+v"(kc[7]));
         else
             asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(mbits), "+v"(ksc), "+v"(kc[0]), "+v"(kc[1]), "+v"(kc[2]), "+v"(kc[3]));
-        if (t + 2 < n) issue(t + 2, st, 0);   // the K rows are in registers: their part of the stage is free
+        if (!ONE && t + 2 < n) issue(t + 2, st, 0);   // the K rows are in registers: their part of the stage is free
         float raw[4];
         fsq_scores<TK>(qw, dqa, qsa, kc, ksc, raw);
         fs_softmax(raw, half_bits_to_float((unsigned short)mbits), scale, a.softcap, slope, p_wr, S);
         // V(t) has landed when at most K(t + 1), V(t + 1), K(t + 2) are outstanding
-        if (t + 2 < n) FS_WAIT_VM(CK + CV + CK);
-        else if (t + 1 < n) FS_WAIT_VM(CK + CV);
+        if (!ONE && t + 2 < n) FS_WAIT_VM(CK + CV + CK);
+        else if (!ONE && t + 1 < n) FS_WAIT_VM(CK + CV);
         else FS_WAIT_VM(0);
         // the tile's V in two halves of 32 cells through the wave's 8 KiB of f16 rows
         fsq_convert_v<TV>(sb + (unsigned)OFF_V, sb + (unsigned)OFF_VS, vf_lds, lane);
         fs_output<8>(vf_lds + fs_v_lane(lane), p_rd, S);
         fsq_convert_v<TV>(sb + (unsigned)(OFF_V + 32 * GV::ROW), sb + (unsigned)(OFF_VS + 32 * 8), vf_lds, lane);
         // the levels are in registers or already converted: the V part of the stage may be overwritten
-        if (t + 2 < n) issue(t + 2, st, 1);
+        if (!ONE && t + 2 < n) issue(t + 2, st, 1);
         fs_output<8>(vf_lds + fs_v_lane(lane), p_rd + 64, S);
     }
 
+    if constexpr (ONE) {   // the states of the group's waves meet in LDS: one partial result per group
+        asm volatile("" ::: "memory");   // fs_output's reads of the V rows come first
+        float *mine = (float *)(vf_buf + wave * FSQ_VF);   // [4][FS_D], maxima, sums (the wave's V rows are consumed)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float L = wave_sum_dpp(S.lsum[r]);
+            mine[r * FS_D + lane] = S.o0[r];
+            mine[r * FS_D + 64 + lane] = S.o1[r];
+            if (lane == 0) {
+                mine[4 * FS_D + r] = S.m[r];
+                mine[4 * FS_D + 4 + r] = L;
+            }
+        }
+        __syncthreads();
+        const int n_waves = (int)(blockDim.x >> 6);
+        const float *all = (const float *)vf_buf;
+        for (int idx = wave; idx < 2 * R; idx += n_waves) {   // half a head per wave and turn
+            const int r = idx >> 1, d = 64 * (idx & 1) + lane;
+            float m[NWV], l[NWV], o[NWV];   // all requested before any is used; past the last wave its values again, left out below
+#pragma unroll
+            for (int w = 0; w < NWV; w++) {
+                const float *part = all + (w < n_waves ? w : n_waves - 1) * (FSQ_VF / 4);
+                m[w] = part[4 * FS_D + r];
+                l[w] = part[4 * FS_D + 4 + r];
+                o[w] = part[r * FS_D + d];
+            }
+            float M = m[0], L = 0.0f, O = 0.0f;
+#pragma unroll
+            for (int w = 1; w < NWV; w++) M = fmaxf(M, m[w]);
+#pragma unroll
+            for (int w = 0; w < NWV; w++) {
+                if (w >= n_waves) break;   // uniform
+                const float f = __expf(m[w] - M);
+                L += l[w] * f;
+                O += o[w] * f;
+            }
+            float *p = a.ws + (((int64_t)hk * R + r) * a.n_splits + blockIdx.x) * (FS_D + 2);
+            p[d] = O;
+            if (d == 0) {
+                p[FS_D] = M;
+                p[FS_D + 1] = L;
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         if (r < R) {
@@ -904,11 +956,26 @@ int launch_fattn_dec_stream_q(hipStream_t s, fattn_args &a, int64_t D, size_t ws
     if (tiles_per_wave > FSQ_MAX_TILES) return 1;
     int64_t n_splits = (n_tiles + tiles_per_wave - 1) / tiles_per_wave;
     n_splits = (n_splits + nwv - 1) / nwv * nwv;   // whole groups; a wave without tiles writes an empty partial
+    // A tile per wave where one group per compute unit holds them all.  Five waves of Q8_0 only for up to two query heads per kv head (10240 cells,
+    // 16 / 8 heads 19.4 -> 18.2 us, 32 / 8 heads 20.35 -> 20.45).
+    bool one = false;
+    const int64_t one_wv = (n_tiles * a.Hkv + FSQ_TOTAL_GROUPS - 1) / FSQ_TOTAL_GROUPS, one_groups = (n_tiles + one_wv - 1) / one_wv;
+    const int one_max = a.type_k == MI355_Q8_0 && a.type_v == MI355_Q8_0 && R > 2 ? 4 : fsq_waves_one_rt(a.type_k, a.type_v);
+    if (tiles_per_wave > 1 && one_wv <= one_max && one_groups <= n_splits) {
+        one = true;
+        nwv = (int)one_wv;
+        tiles_per_wave = 1;
+        n_splits = one_groups;
+    }
     if (n_splits > 256) return 1;
     if (ws_bytes < (size_t)a.Hq * (size_t)n_splits * (size_t)(FS_D + 2) * sizeof(float)) return 1;
     a.n_splits = (int)n_splits;
-    const dim3 grid((unsigned)(n_splits / nwv), (unsigned)a.Hkv), block((unsigned)nwv * 64);
-#define MI355_FSQ_LAUNCH(TK, TV) MI355_LAUNCH((k_fattn_dec_stream_q<TK, TV>), grid, block, 0, s, a, ks, vs, (int)tiles_per_wave, (int)n_tiles, (int)R)
+    const dim3 grid((unsigned)(one ? n_splits : n_splits / nwv), (unsigned)a.Hkv), block((unsigned)nwv * 64);
+#define MI355_FSQ_LAUNCH(TK, TV) \
+    do { \
+        if (one) MI355_LAUNCH((k_fattn_dec_stream_q<TK, TV, true>), grid, block, 0, s, a, ks, vs, 1, (int)n_tiles, (int)R); \
+        else MI355_LAUNCH((k_fattn_dec_stream_q<TK, TV, false>), grid, block, 0, s, a, ks, vs, (int)tiles_per_wave, (int)n_tiles, (int)R); \
+    } while (0)
     if (a.type_k == MI355_Q8_0 && a.type_v == MI355_Q8_0) MI355_FSQ_LAUNCH(MI355_Q8_0, MI355_Q8_0);
     else if (a.type_k == MI355_Q8_0) MI355_FSQ_LAUNCH(MI355_Q8_0, MI355_Q4_0);
     else if (a.type_v == MI355_Q8_0) MI355_FSQ_LAUNCH(MI355_Q4_0, MI355_Q8_0);
