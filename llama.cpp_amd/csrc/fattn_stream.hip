@@ -168,14 +168,66 @@ template <int H> __device__ __forceinline__ void fs_output_half(unsigned v_addr,
     for (int j = 0; j < NJ; j++) o = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pa[j]), __builtin_bit_cast(f16x4, v[j]), o, 0, 0, 0);
 }
 
-__global__ void __launch_bounds__(FS_WAVES * 64, 1) k_fattn_dec_stream(fattn_args a, int tiles_per_wave, int n_tiles, int R) {
-    __shared__ __attribute__((aligned(1024))) uint8_t ring_buf[FS_WAVES * 2 * FS_STAGE];
-    __shared__ __attribute__((aligned(16))) unsigned short pbuf[FS_WAVES][4][FS_TILE];
-    __shared__ __attribute__((aligned(16))) unsigned short mbuf[FS_WAVES][FS_MAX_TILES * FS_TILE];
+// The states of a group's waves (at most NWV) meet in LDS: one partial result per group.  all: `stride` floats per wave, whose LDS reads lie behind it; head r's
+// result goes to out + r * head_step.
+template <int NWV>
+__device__ __forceinline__ void fs_join(const fs_state &S, float *all, int stride, float *out, int64_t head_step, int R, int lane, int wave) {
+    asm volatile("" ::: "memory");   // the reads of fs_output come first
+    float *mine = all + wave * stride;   // [4][FS_D], maxima, sums
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const float L = wave_sum_dpp(S.lsum[r]);
+        mine[r * FS_D + lane] = S.o0[r];
+        mine[r * FS_D + 64 + lane] = S.o1[r];
+        if (lane == 0) {
+            mine[4 * FS_D + r] = S.m[r];
+            mine[4 * FS_D + 4 + r] = L;
+        }
+    }
+    __syncthreads();
+    const int n_waves = (int)(blockDim.x >> 6);
+    for (int idx = wave; idx < 2 * R; idx += n_waves) {   // half a head per wave and turn
+        const int r = idx >> 1, d = 64 * (idx & 1) + lane;
+        float m[NWV], l[NWV], o[NWV];   // all requested before any is used; past the last wave its values again, left out below
+#pragma unroll
+        for (int w = 0; w < NWV; w++) {
+            const float *part = all + (w < n_waves ? w : n_waves - 1) * stride;
+            m[w] = part[4 * FS_D + r];
+            l[w] = part[4 * FS_D + 4 + r];
+            o[w] = part[r * FS_D + d];
+        }
+        float M = m[0], L = 0.0f, O = 0.0f;
+#pragma unroll
+        for (int w = 1; w < NWV; w++) M = fmaxf(M, m[w]);
+#pragma unroll
+        for (int w = 0; w < NWV; w++) {
+            if (w >= n_waves) break;   // uniform
+            const float f = __expf(m[w] - M);
+            L += l[w] * f;
+            O += o[w] * f;
+        }
+        float *p = out + r * head_step;
+        p[d] = O;
+        if (d == 0) {
+            p[FS_D] = M;
+            p[FS_D + 1] = L;
+        }
+    }
+}
+
+// ONE: no wave has more than one tile; it keeps one stage, three or four waves fit where two walked two tiles each, and they join their states (us a call:
+// 32 / 8 heads, 5120 cells 14.5 -> 13.3, 6144 15.2 -> 14.2, 8192 16.2 -> 15.8; 16 / 4 heads, 12288 16.2 -> 14.6, 16384 17.6 -> 16.3; 4 / 4 heads, 16384 15.9 -> 13.5)
+constexpr int FS_WAVES_ONE = 4;
+template <bool ONE>
+__global__ void __launch_bounds__((ONE ? FS_WAVES_ONE : FS_WAVES) * 64, 1) k_fattn_dec_stream(fattn_args a, int tiles_per_wave, int n_tiles, int R) {
+    constexpr int NWV = ONE ? FS_WAVES_ONE : FS_WAVES, STAGES = ONE ? 1 : 2, MT = ONE ? 8 : FS_MAX_TILES;
+    __shared__ __attribute__((aligned(1024))) uint8_t ring_buf[NWV * STAGES * FS_STAGE];
+    __shared__ __attribute__((aligned(16))) unsigned short pbuf[NWV][4][FS_TILE];
+    __shared__ __attribute__((aligned(16))) unsigned short mbuf[NWV][MT * FS_TILE];
     // the ring is written by global-to-LDS transfers only
     asm volatile("" ::"v"((void *)ring_buf) : "memory");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int split = (int)blockIdx.x * FS_WAVES + wave;
+    const int split = (int)blockIdx.x * (ONE ? (int)(blockDim.x >> 6) : FS_WAVES) + wave;   // ONE: the launch may give a group fewer than four waves
     const int64_t hk = blockIdx.y;
     const int t_begin = split * tiles_per_wave;
     const int t_end = t_begin + tiles_per_wave < n_tiles ? t_begin + tiles_per_wave : n_tiles;
@@ -184,7 +236,7 @@ __global__ void __launch_bounds__(FS_WAVES * 64, 1) k_fattn_dec_stream(fattn_arg
 
     float slope[4];
     fs_slopes(a, hk * R, slope);
-    uint8_t *ring = ring_buf + wave * (2 * FS_STAGE);
+    uint8_t *ring = ring_buf + wave * (STAGES * FS_STAGE);
     // transfers of tile t into stage st: instruction i moves rows 4i .. 4i + 3; lane p -> row 4i + p / 16, chunk position p % 16.
     // A whole tile in range: scalar row addresses plus per-lane offsets that are the same for every tile; the last, partial tile
     // of the cache clamps its rows per lane (rows past the end repeat the last cell; their scores are discarded).
@@ -229,7 +281,7 @@ __global__ void __launch_bounds__(FS_WAVES * 64, 1) k_fattn_dec_stream(fattn_arg
         issue(0, 0, 0);
         issue(0, 0, 1);
     }
-    if (n > 1) {
+    if (!ONE && n > 1) {
         issue(1, 1, 0);
         issue(1, 1, 1);
     }
@@ -242,9 +294,9 @@ __global__ void __launch_bounds__(FS_WAVES * 64, 1) k_fattn_dec_stream(fattn_arg
     {
         const unsigned short *mrow = (const unsigned short *)a.mask;
         const bool wide = ((uintptr_t)mrow & 15) == 0;
-        u32x4 mc[FS_MAX_TILES / 8];
+        u32x4 mc[MT / 8];
 #pragma unroll
-        for (int it = 0; it < FS_MAX_TILES / 8; it++) {
+        for (int it = 0; it < MT / 8; it++) {
             const int j = it * 64 + lane;
             const int64_t c = c_begin + (int64_t)j * 8;
             mc[it] = u32x4{0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u};   // -inf
@@ -261,7 +313,7 @@ __global__ void __launch_bounds__(FS_WAVES * 64, 1) k_fattn_dec_stream(fattn_arg
             }
         }
 #pragma unroll
-        for (int it = 0; it < FS_MAX_TILES / 8; it++) {
+        for (int it = 0; it < MT / 8; it++) {
             const int j = it * 64 + lane;
             if (j * 8 < n * FS_TILE) *(u32x4 *)(mw + j * 8) = mc[it];
         }
@@ -278,9 +330,9 @@ __global__ void __launch_bounds__(FS_WAVES * 64, 1) k_fattn_dec_stream(fattn_arg
     const unsigned p_wr = p_base + (unsigned)lane * 2, p_rd = p_base + (unsigned)hr * (FS_TILE * 2);
 
     for (int t = 0; t < n; t++) {
-        const int st = t & 1;
+        const int st = ONE ? 0 : t & 1;
         // K(t) has landed when at most V(t), K(t + 1), V(t + 1) are still on their way (transfers complete in the order issued)
-        if (t + 1 < n) FS_WAIT_VM(48);
+        if (!ONE && t + 1 < n) FS_WAIT_VM(48);
         else FS_WAIT_VM(16);
         const unsigned sb = ring_lds + (unsigned)st * FS_STAGE;
 
@@ -293,17 +345,21 @@ __global__ void __launch_bounds__(FS_WAVES * 64, 1) k_fattn_dec_stream(fattn_arg
         asm volatile("s_waitcnt lgkmcnt(0)"
                      : "+v"(mbits), "+v"(kc[0]), "+v"(kc[1]), "+v"(kc[2]), "+v"(kc[3]), "+v"(kc[4]), "+v"(kc[5]), "+v"(kc[6]), "+v"(kc[7]), "+v"(kc[8]), "+v"(kc[9]),
                        "+v"(kc[10]), "+v"(kc[11]), "+v"(kc[12]), "+v"(kc[13]), "+v"(kc[14]), "+v"(kc[15]));
-        if (t + 2 < n) issue(t + 2, st, 0);   // the K rows are in registers: their half of the stage is free
+        if (!ONE && t + 2 < n) issue(t + 2, st, 0);   // the K rows are in registers: their half of the stage is free
         fs_scores(qv, kc, half_bits_to_float((unsigned short)mbits), scale, a.softcap, slope, p_wr, S);
         // V(t) has landed when at most K(t + 1), V(t + 1), K(t + 2) are outstanding
-        if (t + 2 < n) FS_WAIT_VM(48);
-        else if (t + 1 < n) FS_WAIT_VM(32);
+        if (!ONE && t + 2 < n) FS_WAIT_VM(48);
+        else if (!ONE && t + 1 < n) FS_WAIT_VM(32);
         else FS_WAIT_VM(0);
         fs_output(sb + v_lane, p_rd, S);
         // every LDS read of this stage has returned (the last wait above): the V half may be overwritten
-        if (t + 2 < n) issue(t + 2, st, 1);
+        if (!ONE && t + 2 < n) issue(t + 2, st, 1);
     }
 
+    if constexpr (ONE) {
+        fs_join<NWV>(S, (float *)ring_buf, FS_STAGE / 4, a.ws + ((int64_t)hk * R * a.n_splits + blockIdx.x) * (FS_D + 2), (int64_t)a.n_splits * (FS_D + 2), R, lane, wave);
+        return;
+    }
     // ---- partial result of this split: un-normalised outputs, running maximum, sum
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -692,49 +748,8 @@ __global__ void __launch_bounds__(((ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK
         fs_output<8>(vf_lds + fs_v_lane(lane), p_rd + 64, S);
     }
 
-    if constexpr (ONE) {   // the states of the group's waves meet in LDS: one partial result per group
-        asm volatile("" ::: "memory");   // fs_output's reads of the V rows come first
-        float *mine = (float *)(vf_buf + wave * FSQ_VF);   // [4][FS_D], maxima, sums (the wave's V rows are consumed)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float L = wave_sum_dpp(S.lsum[r]);
-            mine[r * FS_D + lane] = S.o0[r];
-            mine[r * FS_D + 64 + lane] = S.o1[r];
-            if (lane == 0) {
-                mine[4 * FS_D + r] = S.m[r];
-                mine[4 * FS_D + 4 + r] = L;
-            }
-        }
-        __syncthreads();
-        const int n_waves = (int)(blockDim.x >> 6);
-        const float *all = (const float *)vf_buf;
-        for (int idx = wave; idx < 2 * R; idx += n_waves) {   // half a head per wave and turn
-            const int r = idx >> 1, d = 64 * (idx & 1) + lane;
-            float m[NWV], l[NWV], o[NWV];   // all requested before any is used; past the last wave its values again, left out below
-#pragma unroll
-            for (int w = 0; w < NWV; w++) {
-                const float *part = all + (w < n_waves ? w : n_waves - 1) * (FSQ_VF / 4);
-                m[w] = part[4 * FS_D + r];
-                l[w] = part[4 * FS_D + 4 + r];
-                o[w] = part[r * FS_D + d];
-            }
-            float M = m[0], L = 0.0f, O = 0.0f;
-#pragma unroll
-            for (int w = 1; w < NWV; w++) M = fmaxf(M, m[w]);
-#pragma unroll
-            for (int w = 0; w < NWV; w++) {
-                if (w >= n_waves) break;   // uniform
-                const float f = __expf(m[w] - M);
-                L += l[w] * f;
-                O += o[w] * f;
-            }
-            float *p = a.ws + (((int64_t)hk * R + r) * a.n_splits + blockIdx.x) * (FS_D + 2);
-            p[d] = O;
-            if (d == 0) {
-                p[FS_D] = M;
-                p[FS_D + 1] = L;
-            }
-        }
+    if constexpr (ONE) {
+        fs_join<NWV>(S, (float *)vf_buf, FSQ_VF / 4, a.ws + ((int64_t)hk * R * a.n_splits + blockIdx.x) * (FS_D + 2), (int64_t)a.n_splits * (FS_D + 2), R, lane, wave);
         return;
     }
 #pragma unroll
@@ -911,9 +926,14 @@ int launch_fattn_dec_stream(hipStream_t s, fattn_args &a, int64_t D, size_t ws_b
     if (tiles_per_wave > FS_MAX_TILES) return 1;
     int64_t n_splits = (n_tiles + tiles_per_wave - 1) / tiles_per_wave;
     n_splits = (n_splits + FS_WAVES - 1) / FS_WAVES * FS_WAVES;   // whole groups; a wave without tiles writes an empty partial
+    // a tile per wave where one group of up to four waves per compute unit holds them all
+    const int64_t one_wv = (n_tiles * a.Hkv + FS_TOTAL_WAVES / FS_WAVES - 1) / (FS_TOTAL_WAVES / FS_WAVES), one_groups = (n_tiles + one_wv - 1) / one_wv;
+    const bool one = tiles_per_wave > 1 && one_wv <= FS_WAVES_ONE && one_groups <= n_splits;
+    if (one) n_splits = one_groups;
     if (ws_bytes < (size_t)a.Hq * (size_t)n_splits * (size_t)(FS_D + 2) * sizeof(float)) return 1;
     a.n_splits = (int)n_splits;
-    MI355_LAUNCH(k_fattn_dec_stream, dim3((unsigned)(n_splits / FS_WAVES), (unsigned)a.Hkv), dim3(FS_WAVES * 64), 0, s, a, (int)tiles_per_wave, (int)n_tiles, (int)R);
+    if (one) MI355_LAUNCH(k_fattn_dec_stream<true>, dim3((unsigned)n_splits, (unsigned)a.Hkv), dim3((unsigned)one_wv * 64), 0, s, a, 1, (int)n_tiles, (int)R);
+    else MI355_LAUNCH(k_fattn_dec_stream<false>, dim3((unsigned)(n_splits / FS_WAVES), (unsigned)a.Hkv), dim3(FS_WAVES * 64), 0, s, a, (int)tiles_per_wave, (int)n_tiles, (int)R);
     return launch_status("k_fattn_dec_stream");
 }
 
