@@ -25,7 +25,7 @@ struct fattn_args {
     float *dst;      // [D, Hq, Nq]
     int8_t *act_q;   // optional: Q8_1 of dst rows (Hq*D elements per query) in the split activation layout
     act_ds *act_s;
-    float *ws;       // partial results when n_splits > 1: [Nq][Hq][n_splits][D + 2]
+    float *ws;       // partial results when n_splits > 1: [Nq][Hq][n_splits][D + 2] (k_fattn_mma_half: [n_splits][Nq][Hq][D], then {max, sum} of each)
     const int32_t *kv_extent;   // prefill, optional: per tile of 32 queries, the number of leading cells after which every
                                 // mask entry of the tile's rows is -inf (see k_mask_extent); null = all Nkv cells
     int64_t Nq, Nkv, Hq, Hkv;

@@ -847,6 +847,12 @@ int launch_half(hipStream_t s, fattn_args a, size_t ws_bytes) {
     // at most one group per compute unit and a long cache: eight waves on 128-cell tiles (512 rows: 4096 cells 112 -> 103 us,
     // 512 cells 24.8 -> 26.2 us).  Head size 256: the eight waves' registers do not fit.
     const bool wide = D <= 128 && groups <= 256 && a.Nkv >= 1024;
+    // the groups read the mask extents, at the front of the scratch memory, while others write their states: those lie behind
+    if (a.kv_extent) {
+        const size_t used = ((size_t)((a.Nq + 31) / 32) * sizeof(int32_t) + 15) & ~(size_t)15;
+        a.ws += used / sizeof(float);
+        ws_bytes = ws_bytes > used ? ws_bytes - used : 0;
+    }
     const int64_t n = half_may_split(a, PX) ? plan_half(D, groups, rows, tiles, wide, ws_bytes).n : 1;
     a.cells_per_split = (tiles + n - 1) / n * 64;
     a.n_splits = (int)((a.Nkv + a.cells_per_split - 1) / a.cells_per_split);   // no empty range

@@ -416,9 +416,10 @@ def test_prefill_output_at_any_float_address(dev, D, quantized, floats):
         assert torch.equal(act, mi355.quantize_act(dst.clone().reshape(Nq, Hq * D)))
 
 
-@pytest.mark.parametrize("D,Nkv", [(64, 1100), (128, 1100), (128, 2049), (80, 2049), (112, 2500), (256, 2112)])
+@pytest.mark.parametrize("D,Nkv,quantized", [(64, 1100, False), (128, 1100, False), (128, 2049, False), (80, 2049, False), (112, 2500, False), (256, 2112, False),
+                                             (64, 2100, True), (128, 2049, True)])
 @pytest.mark.parametrize("Nq,Hq,Hkv", [(33, 8, 2), (64, 5, 5), (95, 12, 4), (40, 16, 2)])
-def test_prefill_ranges_of_cells(dev, D, Nkv, Nq, Hq, Hkv):
+def test_prefill_ranges_of_cells(dev, D, Nkv, quantized, Nq, Hq, Hkv):
     """few query tiles over many cells: ranges of cells side by side and a merge, against the textbook form and against one walk (no workspace);
     the last range is ragged, some queries see nothing of most ranges and two see nothing at all.  f16 probabilities leave some 2e-4 (NMSE
     4e-8), pairs of them 3e-7 (NMSE 1e-13)"""
@@ -426,8 +427,9 @@ def test_prefill_ranges_of_cells(dev, D, Nkv, Nq, Hq, Hkv):
     import mi355
     lib = mi355.load()
     rng = np.random.default_rng(D + Nq)
-    if D not in (64, 128):
-        Nq += 1152 // Hq                                   # below this many (query, head) pairs: the vector kernel
+    f16 = D in (64, 128) and not quantized
+    if not f16:
+        Nq += (1537 if D == 64 else 1152) // Hq            # below this many (query, head) pairs: the vector kernel
     q, k, v, mask = _inputs(rng, D, Nq, Nkv, Hq, Hkv, rand_mask=True)
     mask[3, 40:] = -np.inf
     mask[7, :Nkv - 700] = -np.inf
@@ -439,24 +441,70 @@ def test_prefill_ranges_of_cells(dev, D, Nkv, Nq, Hq, Hkv):
     scale = 1.0 / np.sqrt(D)
     args = [torch.from_numpy(a).to(dev) for a in (q, k, v, mask)]
     before = lib.mi355_launch_count()
-    got = mi355.flash_attn_ext(*args, scale)
-    assert lib.mi355_launch_count() - before == 2
+    got = mi355.flash_attn_ext(*args, scale, quantized=quantized)
+    assert lib.mi355_launch_count() - before == (3 if quantized else 2)      # ranges, merge, quantization of the output
     before = lib.mi355_launch_count()
-    whole = mi355.flash_attn_ext(*args, scale, workspace=False)
-    assert lib.mi355_launch_count() - before == 1
+    whole = mi355.flash_attn_ext(*args, scale, quantized=quantized, workspace=False)
+    assert lib.mi355_launch_count() - before == (2 if quantized else 1)
+    if quantized:
+        (got, act), (whole, _) = got, whole
+        seen_rows = torch.isfinite(got).all(dim=2).all(dim=1)
+        act, want_act = (a.reshape(-1)[:Nq * Hq * D].reshape(Nq, Hq * D)[seen_rows] for a in (act, mi355.quantize_act(got.reshape(Nq, Hq * D))))
+        assert torch.equal(act, want_act)
     got, whole = got.cpu().numpy(), whole.cpu().numpy()
     blind = [11, 32]
     seen = [i for i in range(Nq) if i not in blind]
-    if D in (64, 128):
+    if f16:
         assert np.all(got[blind] == 0.0) and np.all(whole[blind] == 0.0)
     else:
         assert np.isnan(got[blind]).all() and np.isnan(whole[blind]).all()     # 0 / 0, as in the vector kernel
     v[:, 900] = 0
     k[:, 901] = 0
     want = _textbook(q[:, seen], k, v, mask[seen], scale)
-    bound = 1e-6 if D in (64, 128) else 1e-12
+    bound = 1e-6 if f16 else 1e-12
     assert orc.nmse(whole[seen], want) < bound
     assert orc.nmse(got[seen], want) < bound
+
+
+@pytest.mark.parametrize("D,quantized,Nq,Nkv,Hq,Hkv", [(112, False, 1056, 6144, 64, 8), (128, True, 1056, 8192, 64, 8), (64, True, 2080, 6144, 32, 8)])
+def test_prefill_ranges_of_cells_behind_mask_extents(dev, D, quantized, Nq, Nkv, Hq, Hkv):
+    """more groups than the chip holds at once (so the extents of the mask's rows lie in the workspace) and ranges of cells (whose states lie
+    there too): groups that start late still find the extents.  Every query tile sees another number of cells, the first ones less than a
+    range.  Against the textbook form on two heads and against one walk over the cells (no workspace, or one that holds the extents alone)"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    rng = np.random.default_rng(D + Nq)
+    q, k, v, mask = _inputs(rng, D, Nq, Nkv, Hq, Hkv)
+    i = np.arange(Nq)[:, None]
+    mask[:Nq] = np.where(np.arange(Nkv)[None, :] <= i * (Nkv - 1) // (Nq - 1), 0.0, -np.inf).astype(np.float16)
+    scale = 1.0 / np.sqrt(D)
+    qd, kd, vd, md = (torch.from_numpy(a).to(dev) for a in (q, k, v, mask))
+
+    def call(ws_bytes):
+        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
+        dst = torch.empty((Nq, Hq, D), device=dev)
+        act = torch.empty(int(lib.mi355_act_bytes(Hq * D, Nq)), dtype=torch.uint8, device=dev) if quantized else None
+        before = lib.mi355_launch_count()
+        mi355.check(lib.mi355_flash_attn_ext_quant(torch.cuda.current_stream().cuda_stream, qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), md.data_ptr(), dst.data_ptr(), D, Nq,
+                                                   Nkv, Hq, Hkv, D * 4, Nq * D * 4, D * 2, Nkv * D * 2, D * 2, Nkv * D * 2, Nkv * 2, scale, 0.0, 0.0,
+                                                   ws.data_ptr() if ws_bytes else None, ws_bytes, act.data_ptr() if quantized else None))
+        launches = lib.mi355_launch_count() - before - quantized
+        if quantized:
+            assert torch.equal(act, mi355.quantize_act(dst.reshape(Nq, Hq * D)))
+        return dst.cpu().numpy(), launches
+
+    got, launches = call(1 << 28)
+    assert launches == 3                                   # extents, ranges, merge
+    whole, launches = call(0)
+    assert launches == 1
+    extents, launches = call((Nq + 31) // 32 * 4)
+    assert launches == 2
+    assert np.array_equal(whole, extents)
+    assert orc.nmse(got, whole) < 1e-12
+    for h in (1, Hq - 2):
+        kv = slice(h * Hkv // Hq, h * Hkv // Hq + 1)
+        assert orc.nmse(got[:, h:h + 1], _textbook(q[h:h + 1], k[kv], v[kv], mask, scale)) < 1e-12
 
 
 @pytest.mark.parametrize("Nq", [1, 3])
