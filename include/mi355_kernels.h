@@ -104,7 +104,7 @@ int mi355_quantize_act(void *stream, const float *x, void *act, int64_t k, int64
  * IQ4_XS (block_iq4_xs, ggml/src/ggml-common.h:406-412; ggml_vec_dot_iq4_xs_q8_K, ggml/src/ggml-cpu/ggml-cpu-quants.c:11381) runs on the
  * same three kernels as IQ4_NL, its block scales d * (ls - 32) taken from the super-block headers; from 256 rows on this entry point
  * runs it on mi355_mul_mat_q8k, and it has tile images for mi355_mul_mat_q8k_tiled.
- * `ws` is scratch of at least mi355_mul_mat_ws_bytes(K, B) bytes. */
+ * `ws` is scratch of at least mi355_mul_mat_ws_bytes(K, B) bytes, 16-byte aligned.  dst may overlap x: x is read before anything is written. */
 size_t mi355_mul_mat_ws_bytes(int64_t K, int64_t B);
 /* ... with the room that lets a product with few tiles run as slices along K, whatever the weight type. */
 size_t mi355_mul_mat_split_ws_bytes(int64_t N, int64_t K, int64_t B);
@@ -128,7 +128,8 @@ int mi355_mul_mat_static(void *stream, int type, const void *W, const float *x, 
 
 /* MUL_MAT of one to three f32 activation rows as one launch without a workspace: every group quantizes the rows to Q8_1 for itself
  * (quantize_row_q8_1_ref's bytes), so the result is mi355_mul_mat's bit for bit.  _supported: the product is one that this form serves
- * quicker than a quantization launch and a product launch; mi355_mul_mat asks it too.  x as for mi355_quantize_act. */
+ * quicker than a quantization launch and a product launch; mi355_mul_mat asks it too.  x as for mi355_quantize_act; unlike
+ * mi355_mul_mat's, dst may not overlap x (other groups still read x when the first write): such calls are refused. */
 int mi355_mul_mat_vec_f32_supported(int type, const void *W, int64_t N, int64_t K, int64_t B);
 int mi355_mul_mat_vec_f32(void *stream, int type, const void *W, const float *x, float *dst, int64_t N, int64_t K, int64_t B, int64_t x_stride,
                           int64_t dst_stride);

@@ -101,6 +101,16 @@ static bool gf_faster(int64_t N, int64_t K, int64_t B) {
     return B == 1 ? groups * K <= 256 * 16384 : groups <= 256 && B * K <= 12288;
 }
 
+// whether any of the B rows of x and any of those of dst have a float in common
+bool mul_mat_rows_overlap(const float *x, int64_t x_stride, int64_t K, const float *dst, int64_t dst_stride, int64_t N, int64_t B) {
+    for (int64_t i = 0; i < B; i++)
+        for (int64_t j = 0; j < B; j++) {
+            const uintptr_t a = (uintptr_t)(x + i * x_stride), b = (uintptr_t)(dst + j * dst_stride);
+            if (a < b + (uintptr_t)N * sizeof(float) && b < a + (uintptr_t)K * sizeof(float)) return true;
+        }
+    return false;
+}
+
 template <int TYPE, int NCOLS>
 static void launch_gf(hipStream_t s, const void *W, const float *x, float *dst, int64_t N, int K, int64_t x_stride, int64_t dst_stride) {
     const size_t lds = (size_t)NCOLS * (K + K / 4);
@@ -125,6 +135,7 @@ int mi355_mul_mat_vec_f32(void *stream, int type, const void *W, const float *x,
                   (long long)N, (long long)K, (long long)B);
     MI355_REQUIRE(x_stride >= K && x_stride % 4 == 0 && ((uintptr_t)x & 15) == 0, "mul_mat_vec_f32: x must be 16-byte aligned with a row stride that is a multiple of 4 floats");
     MI355_REQUIRE(dst_stride >= N, "mul_mat_vec_f32: dst_stride < N");
+    MI355_REQUIRE(!mul_mat_rows_overlap(x, x_stride, K, dst, dst_stride, N, B), "mul_mat_vec_f32: dst overlaps x, which other groups still read when the first write");
     hipStream_t s = (hipStream_t)stream;
 #define MI355_GF_LAUNCH(TY)                                                                 \
     if (B == 1) launch_gf<TY, 1>(s, W, x, dst, N, (int)K, x_stride, dst_stride);            \

@@ -41,6 +41,9 @@ int gemv_unaligned(hipStream_t s, int type, const void *W, const void *act, floa
     return launch_status("k_gemv_unaligned");
 }
 
+// one to three rows in one launch (gemv_f32.hip)
+bool mul_mat_rows_overlap(const float *x, int64_t x_stride, int64_t K, const float *dst, int64_t dst_stride, int64_t N, int64_t B);
+
 // Scratch of the allocation-free entry point: one array per GPU that loads this library, kept until the process ends.
 // Host code never uses the array's name as an address (it is only a host-side handle): the device address is looked up
 // once per device with hipGetSymbolAddress and kept in g_scratch_ptr.
@@ -114,7 +117,10 @@ int mi355_mul_mat(void *stream, int type, const void *W, const float *x, float *
         set_error("mul_mat: workspace of %zu bytes, need %zu", ws_bytes, mi355_mul_mat_ws_bytes(K, B));
         return MI355_ERR_WORKSPACE;
     }
-    if (mi355_mul_mat_vec_f32_supported(type, W, N, K, B)) return mi355_mul_mat_vec_f32(stream, type, W, x, dst, N, K, B, x_stride, dst_stride);
+    // (rows of x that dst overwrites go through the workspace, which holds all of them before the product's first write; so does a call whose
+    // workspace is not aligned, to be refused there)
+    if (mi355_mul_mat_vec_f32_supported(type, W, N, K, B) && ((uintptr_t)ws & 15) == 0 && !mul_mat_rows_overlap(x, x_stride, K, dst, dst_stride, N, B))
+        return mi355_mul_mat_vec_f32(stream, type, W, x, dst, N, K, B, x_stride, dst_stride);
     if (use_mid(type, W, K, B)) {
         int rc = mi355_quantize_act_q8k_tiled(stream, x, ws, K, B, x_stride);
         if (rc != MI355_OK) return rc;

@@ -834,6 +834,45 @@ def test_few_rows_in_one_launch(dev, name, t):
         mi355.check(lib.mi355_mul_mat_vec_f32(None, t, W.data_ptr(), x.data_ptr() + 4, guard.data_ptr(), N, K, 1, K, N))
 
 
+@pytest.mark.parametrize("name,t", [("q4_0", orc.Q4_0), ("q6_K", orc.Q6_K)])
+@pytest.mark.parametrize("B,offset", [(1, 0), (2, 0), (3, 0), (1, 1024), (3, 68), (1, -512), (40, 0)])
+def test_dst_over_x(dev, name, t, B, offset):
+    """a dst that overlaps x (in place, `offset` floats behind or before it) gives the bits of the same call on apart buffers, with a workspace
+    and on the library's own scratch; rows of dst between rows of x share nothing with them; a workspace at an odd address is refused"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    N = K = 2048
+    W = mi355.upload_weights(t, _to_dev(dev, _weights(np.random.default_rng(B), t, N, K)))
+    x = torch.randn(B, K, device=dev, generator=torch.Generator(device=dev).manual_seed(B))
+    want = mi355.mul_mat(t, W, x, split=False)
+    need = int(lib.mi355_mul_mat_ws_bytes(K, B))
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=dev)
+    for static in (False, True):
+        buf = torch.zeros(B * K + 4096, device=dev)
+        xv = buf[2048:2048 + B * K].reshape(B, K)
+        xv.copy_(x)
+        dst = buf[2048 + offset:2048 + offset + B * N].reshape(B, N)
+        if static:
+            mi355.mul_mat_static(t, W, xv, dst)
+        else:
+            mi355.check(lib.mi355_mul_mat(None, t, W.data_ptr(), xv.data_ptr(), dst.data_ptr(), N, K, B, K, N, ws.data_ptr(), need))
+        torch.cuda.synchronize()
+        assert torch.equal(dst, want) or (static and orc.nmse(dst.cpu().numpy(), want.cpu().numpy()) < 1e-12)   # the scratch has room for slices
+    if B > 3:
+        return
+    with pytest.raises(mi355.Mi355Error, match="overlap"):
+        mi355.check(lib.mi355_mul_mat_vec_f32(None, t, W.data_ptr(), xv.data_ptr(), dst.data_ptr(), N, K, B, K, N))
+    with pytest.raises(mi355.Mi355Error, match="aligned"):
+        mi355.check(lib.mi355_mul_mat(None, t, W.data_ptr(), x.data_ptr(), want.data_ptr(), N, K, B, K, N, ws.data_ptr() + 4, need))
+    both = torch.zeros(B, K + N, device=dev)
+    both[:, :K] = x
+    before = lib.mi355_launch_count()
+    mi355.check(lib.mi355_mul_mat(None, t, W.data_ptr(), both.data_ptr(), both[:, K:].data_ptr(), N, K, B, K + N, K + N, ws.data_ptr(), need))
+    assert lib.mi355_launch_count() - before == 1
+    assert torch.equal(both[:, K:], want)
+
+
 @pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t in (orc.Q4_K, orc.Q5_K, orc.Q6_K, orc.IQ4_XS)])
 @pytest.mark.parametrize("N", [129, 130, 131, 132])
 def test_slices_of_any_number_of_rows(dev, name, t, N):
