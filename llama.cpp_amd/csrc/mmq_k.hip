@@ -600,7 +600,7 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
     }
 
     // this thread's weight row (four threads each)
-    // offsets from the wave's first row: 16 rows stay below 4 GiB for any K whose activations do
+    // offsets from the wave's first row (kp_rows_fit)
     const int64_t wr = row0 + (tid >> 2) < N ? row0 + (tid >> 2) : N - 1, wr0 = row0 + 16 * wave < N ? row0 + 16 * wave : N - 1;
     const uint8_t *w_tile = W + wr0 * L.row_bytes;
     const kp_addr wa = kp_addr_of<TYPE>((u32)((wr - wr0) * L.row_bytes), L);
@@ -1219,13 +1219,78 @@ static void launch_split_sum(hipStream_t s, const float *part, float *dst, const
 // tiles of 64 rows fit on the chip at once
 static bool kp_one_round(int64_t N, int64_t cols) { return (N + 63) / 64 * cols <= 256; }
 
+// k_mmq_kp's loads have 32-bit offsets: from a wave's first weight row to the end of its sixteenth, and from the first activation row of a launch to
+// the end of its last.  Longer weight rows (Q6_K from 327 million elements on) go to k_mmq_k_long, more activations than 4 GiB run in several launches.
+static bool kp_rows_fit(const row_layout &L) { return 16 * L.row_bytes <= (int64_t)0xFFFFFFFF; }
+static int64_t kp_most_act_rows(int64_t K) { return (int64_t)0xFFFFFFFF / K; }   // at least 8 where kp_rows_fit
+static int64_t kp_act_run(int64_t K, int64_t B) {   // of a launch: all B, or whole column tiles where there are any
+    const int64_t most = kp_most_act_rows(K);
+    return B <= most ? B : most >= 128 ? most / 128 * 128 : most;
+}
+
+// Rows of any length: one group per (weight row, slot), plain 64-bit addresses.  Its four waves take super-blocks in turn, a lane four elements of each: more
+// and shorter f32 sums than k_mmq_kp's.
 template <int TYPE>
-static void launch_mmq_k(hipStream_t s, const void *W, const void *act, float *dst, const float *residual, int64_t N, int64_t K, int64_t B,
-                         int64_t dst_stride, void *ws, size_t ws_bytes) {
+__global__ void __launch_bounds__(256) k_mmq_k_long(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const float *__restrict__ ad8, float *dst, const float *residual,
+                                                    int64_t N, int64_t K, int64_t slots, int64_t dst_stride, row_layout L, const int32_t *__restrict__ ids, int64_t ids_stride,
+                                                    int64_t n_expert, int64_t n_used, int64_t nb1) {
+    __shared__ float s_part[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t nsb = K >> 8;
+    for (int64_t slot = blockIdx.y; slot < slots; slot += gridDim.y)
+        for (int64_t n = blockIdx.x; n < N; n += gridDim.x) {
+            int64_t row = n, arow = slot;
+            if (ids) {
+                const int64_t t = slot / n_used, e = slot % n_used;
+                int64_t ex = ids[t * ids_stride + e];
+                ex = ex < 0 ? 0 : (ex >= n_expert ? n_expert - 1 : ex);
+                row += ex * N;
+                arow = t * nb1 + e % nb1;
+            }
+            const uint8_t *wrow = W + row * L.row_bytes;
+            float acc = 0.0f;
+            for (int64_t sb = wave; sb < nsb; sb += 4) {
+                const int64_t e = sb * QKK + lane * 4;
+                const u32 q = *(const u32 *)(aq + arow * K + e);
+                float part = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 4; i++) part = fmaf(weight_value<TYPE>(wrow, L, e + i), (float)(int8_t)(q >> (8 * i)), part);
+                acc = fmaf(ad8[arow * nsb + sb], part, acc);
+            }
+            acc = wave_sum(acc);
+            if (lane == 0) s_part[wave] = acc;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                const int64_t o = slot * dst_stride + n;
+                const float sum = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+                dst[o] = residual ? sum + residual[o] : sum;
+            }
+            __syncthreads();
+        }
+}
+
+template <int TYPE>
+static void launch_mmq_k_long(hipStream_t s, const void *W, const int8_t *aq, const float *ad8, float *dst, const float *residual, int64_t N, int64_t K, int64_t slots,
+                              int64_t dst_stride, const row_layout &L, const int32_t *ids, int64_t ids_stride, int64_t n_expert, int64_t n_used, int64_t nb1) {
+    const dim3 grid((unsigned)(N < 65535 ? N : 65535), (unsigned)(slots < 65535 ? slots : 65535));
+    MI355_LAUNCH(k_mmq_k_long<TYPE>, grid, dim3(256), 0, s, (const uint8_t *)W, aq, ad8, dst, residual, N, K, slots, dst_stride, L, ids, ids_stride, n_expert, n_used, nb1);
+}
+
+template <int TYPE>
+static void launch_mmq_k(hipStream_t s, const void *W, const int8_t *aq, const float *ad8, const _Float16 *abs_, float *dst, const float *residual, int64_t N, int64_t K,
+                         int64_t B, int64_t dst_stride, void *ws, size_t ws_bytes) {
     const row_layout L = make_row_layout(TYPE, K);
-    const int8_t *aq = (const int8_t *)act;
-    const float *ad8 = (const float *)(aq + q8k_d_offset(K, B));
-    const _Float16 *abs_ = (const _Float16 *)(aq + q8k_bs_offset(K, B));
+    if (!kp_rows_fit(L)) {
+        launch_mmq_k_long<TYPE>(s, W, aq, ad8, dst, residual, N, K, B, dst_stride, L, nullptr, 0, 0, 0, 0);
+        return;
+    }
+    const int64_t run = kp_act_run(K, B), nsb = K >> 8;
+    if (run < B) {
+        for (int64_t b = 0; b < B; b += run)
+            launch_mmq_k<TYPE>(s, W, aq + b * K, ad8 + b * nsb, abs_ + b * nsb * 16, dst + b * dst_stride, residual ? residual + b * dst_stride : nullptr, N, K,
+                               B - b < run ? B - b : run, dst_stride, ws, ws_bytes);
+        return;
+    }
     const int n_col_tiles = (int)((B + 127) / 128);
     const int n_slices = usable_slices(N, K, B, ws, ws_bytes);
     float *out = n_slices > 1 ? (float *)ws : dst;
@@ -1312,18 +1377,27 @@ void launch_route_slots(hipStream_t s, const int32_t *ids, int64_t ids_stride, i
 }
 
 template <int TYPE>
-static void launch_mmq_k_id(hipStream_t s, const void *as, const void *act, int64_t act_rows, const int32_t *ids, int64_t ids_stride,
+static void launch_mmq_k_id(hipStream_t s, const void *as, const int8_t *aq, const float *ad8, const _Float16 *abs_, const int32_t *ids, int64_t ids_stride,
                             float *dst, int64_t N, int64_t K, int64_t n_expert, int64_t n_used, int64_t nb1, int64_t T, void *route_ws) {
     const int64_t S = T * n_used;
+    const row_layout L = make_row_layout(TYPE, K);
+    const int64_t run = kp_most_act_rows(K) / nb1;   // tokens whose activations stay below 4 GiB
+    if (!kp_rows_fit(L) || run == 0) {
+        launch_mmq_k_long<TYPE>(s, as, aq, ad8, dst, nullptr, N, K, S, N, L, ids, ids_stride, n_expert, n_used, nb1);
+        return;
+    }
+    if (T > run) {
+        const int64_t nsb = K >> 8;
+        for (int64_t t = 0; t < T; t += run)
+            launch_mmq_k_id<TYPE>(s, as, aq + t * nb1 * K, ad8 + t * nb1 * nsb, abs_ + t * nb1 * nsb * 16, ids + t * ids_stride, ids_stride, dst + t * n_used * N, N, K,
+                                  n_expert, n_used, nb1, T - t < run ? T - t : run, route_ws);
+        return;
+    }
     constexpr bool BOTH = TYPE == MI355_Q4_K || TYPE == MI355_Q6_K;   // the types the 64-column kernel unpacks too
     const int bn = BOTH ? route_bn(n_expert, S) : 128;
     const int max_tiles = (int)((S + bn - 1) / bn + n_expert);
     int32_t *act_row = (int32_t *)route_ws, *dst_row = act_row + S, *tiles = dst_row + S, *n_tiles = tiles + 4 * (int64_t)route_max_tiles(n_expert, S);
     MI355_LAUNCH(k_route_slots, dim3(1), dim3(1024), 0, s, ids, ids_stride, n_expert, n_used, nb1, T, bn, act_row, dst_row, tiles, n_tiles);
-    const row_layout L = make_row_layout(TYPE, K);
-    const int8_t *aq = (const int8_t *)act;
-    const float *ad8 = (const float *)(aq + q8k_d_offset(K, act_rows));
-    const _Float16 *abs_ = (const _Float16 *)(aq + q8k_bs_offset(K, act_rows));
     const mmq_route route = {act_row, dst_row, tiles, n_tiles, N * L.row_bytes};
     auto groups = [&](int bm) { return (int)((N + bm - 1) / bm) * max_tiles; };
     auto padded = [&](int bm) { return (groups(bm) + 7) & ~7; };
@@ -1389,10 +1463,13 @@ int mi355_mul_mat_id_q8k(void *stream, int type, const void *as, const void *act
         return MI355_ERR_WORKSPACE;
     }
     hipStream_t s = (hipStream_t)stream;
-    if (type == MI355_Q4_K) launch_mmq_k_id<MI355_Q4_K>(s, as, act, nb1 * T, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws);
-    else if (type == MI355_Q5_K) launch_mmq_k_id<MI355_Q5_K>(s, as, act, nb1 * T, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws);
-    else if (type == MI355_IQ4_XS) launch_mmq_k_id<MI355_IQ4_XS>(s, as, act, nb1 * T, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws);
-    else launch_mmq_k_id<MI355_Q6_K>(s, as, act, nb1 * T, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws);
+    const int8_t *aq = (const int8_t *)act;
+    const float *ad8 = (const float *)(aq + q8k_d_offset(K, nb1 * T));
+    const _Float16 *abs_ = (const _Float16 *)(aq + q8k_bs_offset(K, nb1 * T));
+    if (type == MI355_Q4_K) launch_mmq_k_id<MI355_Q4_K>(s, as, aq, ad8, abs_, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws);
+    else if (type == MI355_Q5_K) launch_mmq_k_id<MI355_Q5_K>(s, as, aq, ad8, abs_, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws);
+    else if (type == MI355_IQ4_XS) launch_mmq_k_id<MI355_IQ4_XS>(s, as, aq, ad8, abs_, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws);
+    else launch_mmq_k_id<MI355_Q6_K>(s, as, aq, ad8, abs_, ids, ids_stride, dst, N, K, n_expert, n_used, nb1, T, route_ws);
     return launch_status("k_mmq_k (routed)");
 }
 
@@ -1440,21 +1517,26 @@ int mi355_mul_mat_q8k_planes_ws(void *stream, int type, const void *planes, cons
     const int8_t *aq = (const int8_t *)act;
     const float *ad8 = (const float *)(aq + q8k_d_offset(K, B));
     const _Float16 *abs_ = (const _Float16 *)(aq + q8k_bs_offset(K, B));
-    const int n_row_tiles = (int)((N + 63) / 64), n_col_tiles = (int)((B + 127) / 128);
-    const int n_groups = n_row_tiles * n_col_tiles, n_groups_padded = (n_groups + 7) & ~7;
     hipStream_t s = (hipStream_t)stream;
-    const int n_slices = usable_slices(N, K, B, ws, ws_bytes);
-    const dim3 grid((unsigned)n_groups_padded, (unsigned)n_slices);
-    float *out = n_slices > 1 ? (float *)ws : dst;
-    const float *res = n_slices > 1 ? nullptr : residual;
-    const int64_t out_stride = n_slices > 1 ? slab_stride(N) : dst_stride;
-    if (type == MI355_Q4_K)
-        MI355_LAUNCH((k_mmq_pl<MI355_Q4_K, false>), grid, dim3(256), 0, s, (const int8_t *)planes, aq, ad8, abs_, out, res, N, K, B, out_stride, L,
-                           n_col_tiles, n_groups, n_groups_padded, mmq_route{}, N * K);
-    else
-        MI355_LAUNCH((k_mmq_pl<MI355_Q6_K, false>), grid, dim3(256), 0, s, (const int8_t *)planes, aq, ad8, abs_, out, res, N, K, B, out_stride, L,
-                           n_col_tiles, n_groups, n_groups_padded, mmq_route{}, N * K);
-    if (n_slices > 1) launch_split_sum(s, (const float *)ws, dst, residual, N, B, dst_stride, n_slices);
+    const int64_t run = kp_act_run(K, B), nsb = K >> 8;
+    for (int64_t b = 0; b < B; b += run, aq += run * K, ad8 += run * nsb, abs_ += run * nsb * 16, dst += run * dst_stride) {
+        const int64_t Br = B - b < run ? B - b : run;
+        const int n_row_tiles = (int)((N + 63) / 64), n_col_tiles = (int)((Br + 127) / 128);
+        const int n_groups = n_row_tiles * n_col_tiles, n_groups_padded = (n_groups + 7) & ~7;
+        const int n_slices = usable_slices(N, K, Br, ws, ws_bytes);
+        const dim3 grid((unsigned)n_groups_padded, (unsigned)n_slices);
+        float *out = n_slices > 1 ? (float *)ws : dst;
+        const float *res = n_slices > 1 ? nullptr : residual;
+        const int64_t out_stride = n_slices > 1 ? slab_stride(N) : dst_stride;
+        if (type == MI355_Q4_K)
+            MI355_LAUNCH((k_mmq_pl<MI355_Q4_K, false>), grid, dim3(256), 0, s, (const int8_t *)planes, aq, ad8, abs_, out, res, N, K, Br, out_stride, L,
+                               n_col_tiles, n_groups, n_groups_padded, mmq_route{}, N * K);
+        else
+            MI355_LAUNCH((k_mmq_pl<MI355_Q6_K, false>), grid, dim3(256), 0, s, (const int8_t *)planes, aq, ad8, abs_, out, res, N, K, Br, out_stride, L,
+                               n_col_tiles, n_groups, n_groups_padded, mmq_route{}, N * K);
+        if (n_slices > 1) launch_split_sum(s, (const float *)ws, dst, residual, N, Br, dst_stride, n_slices);
+        if (residual) residual += run * dst_stride;
+    }
     return launch_status("k_mmq_pl");
 }
 
@@ -1475,10 +1557,13 @@ int mi355_mul_mat_q8k_ws(void *stream, int type, const void *W, const void *act,
                   "mul_mat_q8k: activation workspace is not 16-byte aligned");
     MI355_REQUIRE((N + 63) / 64 * ((B + 63) / 64) < (1 << 30), "mul_mat_q8k: too many tiles");
     hipStream_t s = (hipStream_t)stream;
-    if (type == MI355_Q4_K) launch_mmq_k<MI355_Q4_K>(s, W, act, dst, residual, N, K, B, dst_stride, ws, ws_bytes);
-    else if (type == MI355_Q5_K) launch_mmq_k<MI355_Q5_K>(s, W, act, dst, residual, N, K, B, dst_stride, ws, ws_bytes);
-    else if (type == MI355_IQ4_XS) launch_mmq_k<MI355_IQ4_XS>(s, W, act, dst, residual, N, K, B, dst_stride, ws, ws_bytes);
-    else launch_mmq_k<MI355_Q6_K>(s, W, act, dst, residual, N, K, B, dst_stride, ws, ws_bytes);
+    const int8_t *aq = (const int8_t *)act;
+    const float *ad8 = (const float *)(aq + q8k_d_offset(K, B));
+    const _Float16 *abs_ = (const _Float16 *)(aq + q8k_bs_offset(K, B));
+    if (type == MI355_Q4_K) launch_mmq_k<MI355_Q4_K>(s, W, aq, ad8, abs_, dst, residual, N, K, B, dst_stride, ws, ws_bytes);
+    else if (type == MI355_Q5_K) launch_mmq_k<MI355_Q5_K>(s, W, aq, ad8, abs_, dst, residual, N, K, B, dst_stride, ws, ws_bytes);
+    else if (type == MI355_IQ4_XS) launch_mmq_k<MI355_IQ4_XS>(s, W, aq, ad8, abs_, dst, residual, N, K, B, dst_stride, ws, ws_bytes);
+    else launch_mmq_k<MI355_Q6_K>(s, W, aq, ad8, abs_, dst, residual, N, K, B, dst_stride, ws, ws_bytes);
     return launch_status("k_mmq_k");
 }
 

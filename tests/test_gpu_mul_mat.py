@@ -694,6 +694,55 @@ def test_batches_over_very_long_rows(dev, name, t, K):
     assert orc.nmse(got[..., 0].cpu().numpy(), want.gather(1, ids.long()).cpu().numpy()) < 1e-7
 
 
+@pytest.mark.parametrize("name,t,nb,rows,B", [("q6_K", orc.Q6_K, 1280000, 18, 3), ("iq4_xs", orc.IQ4_XS, 1974000, 18, 1), ("q4_K", orc.Q4_K, 1866240, 18, 2),   # 16 rows: more than 4 GiB
+                                              ("q4_K", orc.Q4_K, 420000, 4, 41), ("q6_K", orc.Q6_K, 420000, 4, 41)])                                           # activations: more than 4 GiB
+def test_super_block_tiles_beyond_32_bit_offsets(dev, name, t, nb, rows, B):
+    """mi355_mul_mat_q8k, its form on planes and its routed form where sixteen weight rows or the activation rows pass 4 GiB: all zeros but a few
+    super-blocks, against the oracle's product of those alone (f32 sums over six super-blocks: NMSE 1e-14)"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    K = nb * 256
+    at = [0, 1, 5, nb // 2 + 1, nb - 2, nb - 1]
+    rng = np.random.default_rng(t)
+    Wq = _weights(rng, t, rows, 256 * len(at))
+    part = mi355.upload_weights(t, _to_dev(dev, Wq))
+    W = torch.zeros(rows, nb * mi355.BLOCK[t][1], dtype=torch.uint8, device=dev)
+    o = o_big = 0
+    for size in {orc.Q6_K: (128, 64, 16, 2), orc.IQ4_XS: (128, 8), orc.Q4_K: (144,)}[t]:      # the pieces of a row in device layout
+        for j, a in enumerate(at):
+            W[:, o_big + a * size:o_big + (a + 1) * size] = part[:, o + j * size:o + (j + 1) * size]
+        o, o_big = o + len(at) * size, o_big + nb * size
+    xs = rng.standard_normal((B, 256 * len(at))).astype(np.float32)
+    x = torch.zeros(B, K, device=dev)
+    for j, a in enumerate(at):
+        x[:, a * 256:(a + 1) * 256] = _to_dev(dev, xs[:, j * 256:(j + 1) * 256])
+    act = mi355.quantize_act_q8k(x)
+    del x
+    want = orc.mul_mat("cpu", t, Wq, xs)
+    res = _to_dev(dev, rng.standard_normal((B, rows)).astype(np.float32))
+    dst = torch.empty(B, rows, device=dev)
+    mi355.check(lib.mi355_mul_mat_q8k(None, t, W.data_ptr(), act.data_ptr(), dst.data_ptr(), rows, K, B, rows))
+    assert orc.nmse(dst.cpu().numpy(), want) < 1e-11
+    need = int(lib.mi355_mul_mat_q8k_ws_bytes(rows, K, B))
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=dev)
+    mi355.check(lib.mi355_mul_mat_q8k_ws(None, t, W.data_ptr(), act.data_ptr(), dst.data_ptr(), res.data_ptr(), rows, K, B, rows, ws.data_ptr(), need))
+    assert orc.nmse(dst.cpu().numpy(), want + res.cpu().numpy()) < 1e-11
+    if rows * K < 1 << 32:
+        planes = torch.empty(int(lib.mi355_kq_planes_bytes(rows, K)), dtype=torch.uint8, device=dev)
+        mi355.check(lib.mi355_kq_unpack_planes(None, t, W.data_ptr(), planes.data_ptr(), rows, K))
+        mi355.check(lib.mi355_mul_mat_q8k_planes_ws(None, t, planes.data_ptr(), act.data_ptr(), dst.data_ptr(), res.data_ptr(), rows, K, B, rows, ws.data_ptr(), need))
+        assert orc.nmse(dst.cpu().numpy(), want + res.cpu().numpy()) < 1e-11
+        del planes
+    N = rows // 2                                          # the same rows as two experts
+    ids = torch.tensor([[b % 2, 1 - b % 2, 0] for b in range(B)], dtype=torch.int32, device=dev)
+    route = torch.empty(int(lib.mi355_mul_mat_id_q8k_route_bytes(2, 2, B)), dtype=torch.uint8, device=dev)
+    dst = torch.empty(B, 2, N, device=dev)
+    mi355.check(lib.mi355_mul_mat_id_q8k(None, t, W.data_ptr(), act.data_ptr(), ids.data_ptr(), 3, dst.data_ptr(), N, K, 2, 2, 1, B, route.data_ptr(), route.numel()))
+    routed = np.stack([np.stack([want[b, e * N:(e + 1) * N] for e in (b % 2, 1 - b % 2)]) for b in range(B)])
+    assert orc.nmse(dst.cpu().numpy(), routed) < 1e-11
+
+
 @pytest.mark.parametrize("name,t,bound", [("q8_0", orc.Q8_0, 1.04e-7), ("iq4_nl", orc.IQ4_NL, 1.04e-7), ("iq4_xs", orc.IQ4_XS, 1.04e-7), ("q4_0", orc.Q4_0, 1.04e-7),
                                           ("q5_0", orc.Q5_0, 1.04e-7)])
 def test_tile_kernel_sums_against_f64(dev, name, t, bound):
