@@ -159,11 +159,13 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
     // stage has landed, and no operand queues behind a weight stage that is wanted later than itself.  (With the stage two
     // super-blocks on requested at the start of a step, in front of the step's second half of activation operands, every step
     // waited for that stage's whole trip from HBM.)
-    if (s_lo < s_hi) {
+    if (s_lo < s_hi) {   // (fences: nothing else keeps the compiler from another order of the requests, on which the first step's wait rests)
         issue(s_lo, 0);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int g = 0; g < 4; g++) fetch_a(s_lo, g, A);
         fetch_s(s_lo, A);
+        __builtin_amdgcn_sched_barrier(0);
         issue(s_lo + 1 < s_hi ? s_lo + 1 : s_lo, 1);
     }
     // AHEAD: super-blocks of the wave that follow this one (2: two or more).  A request under a run-time condition would make the
