@@ -16,9 +16,8 @@
 // per 32.  The Q4_K min term is one v_mfma_f32_32x32x16_f16 per super-block on exact small
 // integers: k slots 0..7 carry (bsum & 63) x m_j, slots 8..15 carry (bsum >> 6) x 64*m_j.
 //
-// k_mmq_kp, the kernel of the full-width tile: a group owns 128 (weight rows) x 128 (activation rows) of dst, or 64 x 128 where the
-// launch has at most one such tile per compute unit; each wave a 32 x 64 sub-tile (1 x 2 MFMA tiles).  K is walked in stages of 128
-// elements, see there.  (Keeping the unpacked weights in the registers of the lane that feeds them to the matrix cores, with no LDS round
+// k_mmq_kp, the kernel of the full-width tile: a group of four waves owns 64 (weight rows) x 128 (activation rows) of dst, each wave a
+// 32 x 64 sub-tile (1 x 2 MFMA tiles).  K is walked in stages of 128 elements, see there.  (Keeping the unpacked weights in the registers of the lane that feeds them to the matrix cores, with no LDS round
 // trip, measured the same: the unpack is then repeated by the two waves that share rows.)  k_mmq_k is the single-buffered kernel (register
 // prefetch, two barriers per stage) of a 64 x 64 tile that sparse expert routing uses.
 //
@@ -388,16 +387,18 @@ __global__ void __launch_bounds__(256, OCC) k_mmq_k(const uint8_t *__restrict__ 
 
 // ---- pipelined kernel of the 128-column tile ----------------------------------------------------------------------------
 // Stage s works on 128 elements of K: the matrix cores read its weight planes and activations from LDS while the same waves unpack the
-// weight piece of stage s + 1 into the other pair of plane buffers; the activations of stage s + 3 start from memory to LDS (a ring of
-// four stages) and the weight piece of stage s + 3 to registers.  One barrier per stage, which waits for the next stage's transfers and
-// for nothing younger: a trip to L2 or HBM is longer than a stage.  LDS rows are 128 bytes without padding; the 16-byte chunk c of row r
-// lives at chunk c ^ ((r >> 1) & 7), which keeps every 16-lane group of a ds_read_b128 on distinct banks.
-// What bounds it (14336 x 4096, 512 rows, Q4_K): LDS is active 53 % of the compute units' busy time, the vector ALU 39 %, the matrix pipes
-// 34 %; two waves per SIMD do not overlap them further.  With two stages in flight, waits for everything in flight at every stage and two
-// groups of 64 rows per compute unit: whole calls, us, before / now: Q4_K 14336 x 4096 x 512 102.8 / 96.9, 4096 x 14336 x 512 104.7 / 97.2;
-// IQ4_XS 8192 x 4096 x 512 67.6 / 58.6; Q5_K 14336 x 4096 x 200 62.2 / 59.0; Q6_K 4096 x 4096 x 100 24.8 / 24.1; experts (8 of 14336 x 4096,
-// 1024 slots) Q4_K 284 / 264, Q6_K 399 / 333.  The 64-row tile: Q5_K 1024 x 4096 x 50 14.6 / 13.7, 16.1 on 128-row tiles (half the units idle).
-constexpr int KP_ROW = 128;
+// weight piece of stage s + 1 into the other pair of plane buffers; the activations of stage s + 1 go from memory to the other LDS buffer and the
+// weight piece of stage s + 3 to registers.  One barrier per stage, which waits for the next stage's transfers and for nothing younger: a
+// weight piece's trip from HBM is longer than a stage.  Two groups on a compute unit (78 KiB of LDS each) cover each other's barriers and waits.
+// LDS rows are 128 bytes without padding; the 16-byte chunk c of row r lives at chunk c ^ ((r >> 1) & 7), which keeps every 16-lane group
+// of a ds_read_b128 on distinct banks.
+// Against waits for everything in flight at every stage, weight pieces two stages ahead: whole calls, us, before / now: Q4_K 14336 x 4096 x 512
+// 100.4 / 95.4; IQ4_XS 8192 x 4096 x 512 65.5 / 59.4; Q5_K 14336 x 4096 x 200 58.9 / 56.1; experts (8 of 14336 x 4096, 1024 slots; the choices of
+// six seeds) Q4_K 294 .. 328 / 257 .. 260, Q6_K 358 .. 377 / 291 .. 322, Q5_K 316 .. 327 / 265 .. 296.
+// One group of 128 rows per compute unit, activations three stages ahead: 1 .. 5 % quicker where such groups fill all units of every XCD at once (Q4_K
+// 4096 x 14336 x 512 98.9 / 94.0), and up to a half slower elsewhere, as a launch has 256 places instead of 512: 300 tiles, Q4_K 7598 x 4608 x 564
+// 83.0 / 103.1; light column tiles that nothing is paired with, Q5_K 3108 x 5120 x 151 30.0 / 37.5; the experts above 258 / 268, 306 / 318, 285 / 301.
+constexpr int KP_ROW = 128, KP_BM = 64;
 __device__ __forceinline__ int kp_off(int row, int chunk) { return row * KP_ROW + ((chunk ^ ((row >> 1) & 7)) << 4); }
 
 template <int TYPE> struct kp_w;   // the 16-byte weight piece of one stage that this thread unpacks (row tid / 4, piece tid % 4)
@@ -551,18 +552,17 @@ __device__ __forceinline__ void kp_lds_wait(i32x4 &a, i32x4 &b, i32x4 &c, i32x4 
 }
 __device__ __forceinline__ void kp_lds_wait(i32x4 &a, i32x4 &b, i32x4 &c) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b), "+v"(c) : : "memory"); }
 
-template <int TYPE, bool ID, int BM>
-__global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const float *__restrict__ ad8,
+template <int TYPE, bool ID>
+__global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const float *__restrict__ ad8,
                                                    const _Float16 *__restrict__ abs_, float *dst, const float *residual,
                                                    int64_t N, int64_t K, int64_t B, int64_t dst_stride, row_layout L, int n_col_tiles,
                                                    int n_groups, int n_groups_padded, mmq_route route) {
     constexpr bool Q4 = kp_form<TYPE>::MIN;   // the form with a min term (Q4_K, Q5_K)
     constexpr int RADIX_SHIFT = kp_form<TYPE>::RADIX_SHIFT;
-    constexpr int BN = 128, WW = BM / 32;   // waves along the weight rows (two along the columns)
-    constexpr int CT = 4 * BM / BN;         // threads that share a column's scales
+    constexpr int BM = KP_BM, BN = 128;
     constexpr int W_BUF = BM * KP_ROW, A_BUF = BN * KP_ROW;
     __shared__ __attribute__((aligned(16))) int8_t sW[4 * W_BUF];   // [half][hi, lo plane]
-    __shared__ __attribute__((aligned(16))) int8_t sA[4 * A_BUF];   // ring of four stages
+    __shared__ __attribute__((aligned(16))) int8_t sA[2 * A_BUF];            // [half]
     __shared__ __attribute__((aligned(16))) float sWd[2][BM];
     __shared__ __attribute__((aligned(16))) float sWn[2][Q4 ? BM : 4];
     __shared__ __attribute__((aligned(16))) _Float16 sWm[2][Q4 ? BM * 16 : 8];
@@ -589,7 +589,7 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lhi = lane >> 5;
-    const int wrow0 = (wave % WW) * 32;    // weight rows of this wave inside the tile
+    const int wrow0 = (wave & 1) * 32;     // weight rows of this wave inside the tile
     const int64_t nsb = K >> 8;
     // split K: group y of gridDim.y walks super-blocks [sb_lo, sb_hi) and writes its sums to its own slice of `dst` (see launch)
     const int64_t sb_per = (nsb + gridDim.y - 1) / gridDim.y;
@@ -609,8 +609,8 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
     // for the whole group, so each form keeps a branch-free stage.
     auto walk = [&](auto ntb) __attribute__((always_inline)) {
         constexpr int NTB = decltype(ntb)::value;   // 32-column result tiles per wave
-        const int wcol0 = (wave / WW) * (32 * NTB); // activation rows of this wave inside the tile
-        constexpr int AI = NTB * 4 / WW;            // transfers of a wave per stage
+        const int wcol0 = (wave >> 1) * (32 * NTB); // activation rows of this wave inside the tile
+        constexpr int AI = 2 * NTB;                 // transfers of a wave per stage
         unsigned aofs[AI];
     #pragma unroll
         for (int it = 0; it < AI; it++) {
@@ -622,7 +622,7 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
         }
         int srow;
         {
-            const int64_t col = col0 + tid / CT;
+            const int64_t col = col0 + (tid >> 1);
             const int64_t cc = col < B ? col : B - 1;
             srow = ID ? route.act_row[cc] : (int)cc;
         }
@@ -642,16 +642,16 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
             for (int r = 0; r < 16; r++) acc[tb][r] = 0.0f;
 
         // per super-block scales of the weights come with the piece (Q4_K header / Q6_K d); those of the activations are fetched
-        // by two or four threads per column: the scale, and 16 bytes of the sub-block sums (threads 2, 3 the same as 0, 1)
+        // by two threads per column: the scale, and 16 bytes of the sub-block sums each
         const u32 d_off = (u32)srow * (u32)nsb * 4, s_off = (u32)srow * (u32)nsb * 32 + 16 * (tid & 1);
         auto fetch_scales = [&](int sb, float &d8, u32x4 &bs) {
             d8 = __builtin_bit_cast(float, buf_load4(ad8, d_off, (u32)sb * 4));
             if constexpr (Q4) bs = buf_load16(abs_, s_off, (u32)sb * 32);
         };
         auto store_scales = [&](int sbuf, float d8, const u32x4 &bs, const kp_h<TYPE> &H) {
-            sAd[sbuf][tid / CT] = d8;   // the threads of a column write the same value: an unconditional use keeps the load where it was issued
+            sAd[sbuf][tid >> 1] = d8;   // both threads of the column write the same value: an unconditional use keeps the load where it was issued
             if constexpr (Q4) {
-                *(u32x4 *)(sAs[sbuf] + (tid / CT) * 16 + 8 * (tid & 1)) = bs;
+                *(u32x4 *)(sAs[sbuf] + (tid >> 1) * 16 + 8 * (tid & 1)) = bs;
                 // the four threads of a row share the work (and all use the header, so its load stays where it was issued):
                 // each writes d, dmin (same values) and the mins of sub-blocks 2p, 2p + 1
                 const int r = tid >> 2, p2 = 2 * (tid & 3);
@@ -670,11 +670,11 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
             }
         };
 
-        // Requests of a stage, in this order: the activation transfers of the stage three on; the scales of the next super-block (first half)
+        // Requests of a stage, in this order: the activation transfers of the next stage; the scales of the next super-block (first half)
         // or the header of the one after it (second half); the weight piece of the stage three on.
         constexpr int LW = kp_loads<TYPE>::W, E0 = (Q4 ? 2 : 1) + LW, E1 = kp_loads<TYPE>::H + LW;
-        // End of a stage: the next stage's transfers of this wave, issued two stages ago, have landed - all but the YOUNGER requests behind
-        // them - and its LDS accesses are done; then the group's.
+        // End of a stage: the next stage's transfers of this wave have landed - all but the YOUNGER requests behind them - and its LDS accesses are done;
+        // then the group's.
         auto stage_end = [=](auto younger) {
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(younger)::value) : "memory");
             __builtin_amdgcn_s_barrier();
@@ -693,12 +693,8 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
         kp_fetch_h<TYPE>(H0, w_tile, wa, (u32)sb_lo);
         kp_fetch_w<TYPE>(R0, w_tile, wa, (u32)sb_lo, 0);
         __builtin_amdgcn_sched_barrier(0);
-        kp_dma_a<AI>(aq, (u32)sb_lo * QKK + 128, aofs, sA + A_BUF);
-        __builtin_amdgcn_sched_barrier(0);
         fetch_scales(sb_lo, d8n, bsn);
         kp_fetch_w<TYPE>(R1, w_tile, wa, (u32)sb_lo, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        kp_dma_a<AI>(aq, (u32)last(sb_lo + 1) * QKK, aofs, sA + 2 * A_BUF);
         __builtin_amdgcn_sched_barrier(0);
         kp_fetch_h<TYPE>(H1, w_tile, wa, (u32)last(sb_lo + 1));
         kp_fetch_w<TYPE>(R2, w_tile, wa, (u32)last(sb_lo + 1), 0);
@@ -713,7 +709,7 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
         stage_end(kp_int<0>{});
 
         i32x16 hi[NTB], lo[NTB];
-        // one stage; its position in the ring of four (0, 2: first half of a super-block) is known at compile time
+        // one stage; its number modulo 4 (0, 2: first half of a super-block) is known at compile time
         // LEFT: super-blocks from this one to the end, 3 for more than two.  The last stages request nothing that nobody uses (the compiler
         // would drop such loads, and stage_end's count with them).
         auto stage = [&](auto pos, auto left, const int sb) __attribute__((always_inline)) {
@@ -723,10 +719,12 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
             kp_w<TYPE> &Rf = POS == 0 ? R3 : POS == 1 ? R0 : POS == 2 ? R1 : R2;   // receives the piece of the stage three on
             kp_h<TYPE> &Hn = (half == 0) == (ODD == 0) ? H0 : H1;   // header of the piece being unpacked: this super-block's, then the next one's
             kp_h<TYPE> &Hf = ODD == 0 ? H0 : H1;                    // second half: this super-block's header is done with
+            if constexpr (NEXT) {
+                kp_dma_a<AI>(aq, (u32)sb * QKK + (half == 0 ? 128 : QKK), aofs, sA + (half ^ 1) * A_BUF);
+                __builtin_amdgcn_sched_barrier(0);   // the order of the requests is what stage_end counts on
+            }
             if constexpr (REQ) {
                 const int sb3 = last(half == 0 ? sb + 1 : sb + 2);
-                kp_dma_a<AI>(aq, (u32)sb3 * QKK + (half == 0 ? 128 : 0), aofs, sA + ((POS + 3) & 3) * A_BUF);
-                __builtin_amdgcn_sched_barrier(0);   // the order of the requests is what stage_end counts on
                 if constexpr (half == 0) fetch_scales(last(sb + 1), d8n, bsn);
                 else kp_fetch_h<TYPE>(Hf, w_tile, wa, (u32)sb3);
                 kp_fetch_w<TYPE>(Rf, w_tile, wa, (u32)sb3, half ^ 1);
@@ -735,11 +733,11 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
 
             kp_planes P;
             // Operand reads in inline assembly: for an LDS read it can see, the compiler waits for transfers in flight that may have written
-            // there, and it does not tell the stages of the ring apart.  A step waits for its operands, issues the next step's, computes.
+            // there, and it does not tell the two buffers apart.  A step waits for its operands, issues the next step's, computes.
             i32x4 af[2][NTB], b1[2], b0[2];
             auto load_frags = [&](int ks, int slot) {
-                af[slot][0] = kp_lds_request<POS * A_BUF>(a_rd[ks]);
-                if constexpr (NTB == 2) af[slot][NTB - 1] = kp_lds_request<POS * A_BUF + 32 * KP_ROW>(a_rd[ks]);
+                af[slot][0] = kp_lds_request<half * A_BUF>(a_rd[ks]);
+                if constexpr (NTB == 2) af[slot][NTB - 1] = kp_lds_request<half * A_BUF + 32 * KP_ROW>(a_rd[ks]);
                 b1[slot] = kp_lds_request<(2 * half) * W_BUF>(w_rd[ks]);
                 b0[slot] = kp_lds_request<(2 * half + 1) * W_BUF>(w_rd[ks]);
             };
@@ -800,8 +798,7 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (NEXT) store_scales(ODD ^ 1, d8n, bsn, ODD == 0 ? H1 : H0);
             }
-            if constexpr (REQ) stage_end(kp_int<2 * AI + (half == 0 ? 2 * E0 + E1 : 2 * E1 + E0)>{});
-            else if constexpr (LEFT == 2) stage_end(kp_int<AI + E0>{});
+            if constexpr (REQ) stage_end(kp_int<(half == 0 ? E0 : E1)>{});
             else if constexpr (NEXT) stage_end(kp_int<0>{});
         };
         int sb = sb_lo;
@@ -820,8 +817,6 @@ __global__ void __launch_bounds__(4 * BM, BM / 64) k_mmq_kp(const uint8_t *__res
             stage(kp_int<0>{}, kp_int<1>{}, sb);
             stage(kp_int<1>{}, kp_int<1>{}, sb);
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no transfer into this group's LDS outlives it
-
     #pragma unroll
         for (int tb = 0; tb < NTB; tb++) {
             const int64_t n = row0 + wrow0 + l32;
@@ -1216,9 +1211,6 @@ static void launch_split_sum(hipStream_t s, const float *part, float *dst, const
     MI355_LAUNCH(k_split_sum, dim3((unsigned)((slab_stride(N) * B / 4 + 255) / 256)), dim3(256), 0, s, part, dst, residual, N, B, dst_stride, n);
 }
 
-// tiles of 64 rows fit on the chip at once
-static bool kp_one_round(int64_t N, int64_t cols) { return (N + 63) / 64 * cols <= 256; }
-
 // k_mmq_kp's loads have 32-bit offsets: from a wave's first weight row to the end of its sixteenth, and from the first activation row of a launch to
 // the end of its last.  Longer weight rows (Q6_K from 327 million elements on) go to k_mmq_k_long, more activations than 4 GiB run in several launches.
 static bool kp_rows_fit(const row_layout &L) { return 16 * L.row_bytes <= (int64_t)0xFFFFFFFF; }
@@ -1296,15 +1288,9 @@ static void launch_mmq_k(hipStream_t s, const void *W, const int8_t *aq, const f
     float *out = n_slices > 1 ? (float *)ws : dst;
     const int64_t out_stride = n_slices > 1 ? slab_stride(N) : dst_stride;
     const float *add = n_slices > 1 ? nullptr : residual;
-    auto launch = [&](auto bm) {
-        constexpr int BM = decltype(bm)::value;
-        const int n_groups = (int)((N + BM - 1) / BM) * n_col_tiles, n_groups_padded = (n_groups + 7) & ~7;
-        MI355_LAUNCH((k_mmq_kp<TYPE, false, BM>), dim3((unsigned)n_groups_padded, (unsigned)n_slices), dim3(4 * BM), 0, s, (const uint8_t *)W, aq, ad8, abs_,
-                           out, add, N, K, B, out_stride, L, n_col_tiles, n_groups, n_groups_padded, mmq_route{});
-    };
-    // a group of 64 rows on every compute unit beats one of 128 on every second one
-    if (kp_one_round(N, n_col_tiles * n_slices)) launch(kp_int<64>{});
-    else launch(kp_int<128>{});
+    const int n_groups = (int)((N + KP_BM - 1) / KP_BM) * n_col_tiles, n_groups_padded = (n_groups + 7) & ~7;
+    MI355_LAUNCH((k_mmq_kp<TYPE, false>), dim3((unsigned)n_groups_padded, (unsigned)n_slices), dim3(256), 0, s, (const uint8_t *)W, aq, ad8, abs_, out, add, N, K, B,
+                       out_stride, L, n_col_tiles, n_groups, n_groups_padded, mmq_route{});
     if (n_slices > 1) launch_split_sum(s, (const float *)ws, dst, residual, N, B, dst_stride, n_slices);
 }
 
@@ -1399,21 +1385,18 @@ static void launch_mmq_k_id(hipStream_t s, const void *as, const int8_t *aq, con
     int32_t *act_row = (int32_t *)route_ws, *dst_row = act_row + S, *tiles = dst_row + S, *n_tiles = tiles + 4 * (int64_t)route_max_tiles(n_expert, S);
     MI355_LAUNCH(k_route_slots, dim3(1), dim3(1024), 0, s, ids, ids_stride, n_expert, n_used, nb1, T, bn, act_row, dst_row, tiles, n_tiles);
     const mmq_route route = {act_row, dst_row, tiles, n_tiles, N * L.row_bytes};
-    auto groups = [&](int bm) { return (int)((N + bm - 1) / bm) * max_tiles; };
-    auto padded = [&](int bm) { return (groups(bm) + 7) & ~7; };
+    const int n_groups = (int)((N + 63) / 64) * max_tiles;
     if constexpr (BOTH) {
         if (bn == 64) {
-            MI355_LAUNCH((k_mmq_k<TYPE, 1, 1, 2, true>), dim3((unsigned)padded(64)), dim3(256), 0, s, (const uint8_t *)as, aq, ad8, abs_,
-                               dst, nullptr, N, K, S, N, L, max_tiles, groups(64), padded(64), route);
+            const int padded = (n_groups + 7) & ~7;
+            MI355_LAUNCH((k_mmq_k<TYPE, 1, 1, 2, true>), dim3((unsigned)padded), dim3(256), 0, s, (const uint8_t *)as, aq, ad8, abs_,
+                               dst, nullptr, N, K, S, N, L, max_tiles, n_groups, padded, route);
             return;
         }
     }
-    if (kp_one_round(N, max_tiles))
-        MI355_LAUNCH((k_mmq_kp<TYPE, true, 64>), dim3((unsigned)groups(64)), dim3(256), 0, s, (const uint8_t *)as, aq, ad8, abs_, dst, nullptr, N, K,
-                               S, N, L, max_tiles, groups(64), groups(64), route);
-    else
-        MI355_LAUNCH((k_mmq_kp<TYPE, true, 128>), dim3((unsigned)groups(128)), dim3(512), 0, s, (const uint8_t *)as, aq, ad8, abs_, dst, nullptr, N, K,
-                               S, N, L, max_tiles, groups(128), groups(128), route);
+    static_assert(KP_BM == 64, "rows of both kernels' tiles");
+    MI355_LAUNCH((k_mmq_kp<TYPE, true>), dim3((unsigned)n_groups), dim3(256), 0, s, (const uint8_t *)as, aq, ad8, abs_, dst, nullptr, N, K, S, N, L, max_tiles, n_groups,
+                       n_groups, route);
 }
 
 }  // namespace mi355
