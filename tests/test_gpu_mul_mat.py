@@ -949,6 +949,26 @@ def test_slices_of_any_number_of_rows(dev, name, t, N):
     assert (dst[:, N:] == 7.0).all()
 
 
+@pytest.mark.parametrize("N,K,B,cut", [(1895, 1280, 606, False), (7263, 1024, 125, False), (2505, 2304, 68, True), (2026, 1792, 210, True), (1896, 1280, 606, True)])
+def test_short_rows_are_cut_only_where_the_sum_pays(dev, N, K, B, cut):
+    """few super-blocks per row and a number of rows that is no multiple of 4: one launch where the cut's sum costs more than it saves"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    rng = np.random.default_rng(N)
+    Wq = np.resize(_weights(rng, orc.Q5_K, 80, K), (N, orc.row_bytes(orc.Q5_K, K)))      # the rows repeat every 80
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    W, xd = mi355.upload_weights(orc.Q5_K, _to_dev(dev, Wq)), _to_dev(dev, x)
+    assert (int(lib.mi355_mul_mat_q8k_ws_bytes(N, K, B)) > 0) == cut
+    before = lib.mi355_launch_count()
+    got = mi355.mul_mat(orc.Q5_K, W, xd)
+    assert lib.mi355_launch_count() - before == (3 if cut else 2)
+    got = got.cpu().numpy()
+    for rows in (slice(0, 3), slice(B - 3, B)):
+        want = orc.mul_mat("cpu", orc.Q5_K, Wq[:80], x[rows])
+        assert orc.nmse(got[rows], np.tile(want, (1, N // 80 + 1))[:, :N]) < 1e-11
+
+
 @pytest.mark.parametrize("name,t", [(n, t) for n, t in TYPES if t not in (orc.Q4_K, orc.Q5_K)])
 @pytest.mark.parametrize("N,K,B", [(130, 5376, 65), (130, 1280, 40), (130, 4352, 130)])
 def test_tile_kernel_many_slices(dev, name, t, N, K, B):
