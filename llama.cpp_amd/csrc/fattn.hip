@@ -432,6 +432,8 @@ __global__ void __launch_bounds__(512) k_fattn_combine(const float *__restrict__
     }
 }
 
+constexpr int64_t ONE_HEAD_MAX = 1024;   // cells of an f16 cache up to which a group may serve one head (launch_vec_r)
+
 // query heads a group serves from one pass over the kv head's bytes
 static int heads_per_group(int64_t R) { return R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1; }
 
@@ -441,9 +443,12 @@ static int heads_per_group(int64_t R) { return R % 4 == 0 ? 4 : R % 2 == 0 ? 2 :
 // rule (n: ranges): 2048 cells 28.9 / 13.7 (32), 4096 29.7 / 18.4 (64; 20.0 with 32, 23.8 with 128); 64 / 8 heads, 4096 29.6 / 22.1 (32; 24.9 with 64);
 // 32 / 32 heads, 4096 28.5 either way (16; 32.4 with 64).  D 80 at 2048 and 4096 cells is the host's 13.5 us for two launches.  A Q8_0 cache, 64 / 8 heads of 128:
 // 512 cells 15.1 / 11.5, 1024 15.3 / 11.6, 2048 15.3 / 11.6.
-static int pick_splits(int64_t Nkv, int64_t Hkv, int64_t Hq, int64_t Nq) {
+// (launch_vec_r gives every head a group of its own over few cells: from 512 such groups on ranges of 256 cells alone; 62 rows over 96 cells,
+// 16 / 4 heads of 256, 18.5 us in two ranges, 10.7 in one; 21 rows over 256 cells, 32 / 8 heads 21.2 / 16.0)
+static int pick_splits(int64_t Nkv, int64_t Hkv, int64_t Hq, int64_t Nq, bool quantized) {
     const int64_t by_len = (Nkv + 255) / 256, by_fill = 2048 / (Hkv * Nq);
-    const int64_t fine_len = (Nkv + 63) / 64, fine_fill = 512 / (Hq / heads_per_group(Hq / Hkv) * Nq);
+    const int64_t groups = Nkv <= (quantized ? 256 : ONE_HEAD_MAX) && Nq * Hq > 512 ? Nq * Hq : Hq / heads_per_group(Hq / Hkv) * Nq;
+    const int64_t fine_len = (Nkv + 63) / 64, fine_fill = 512 / groups;
     int64_t n = by_len < by_fill ? by_len : by_fill;
     const int64_t fine = fine_len < fine_fill ? fine_len : fine_fill;
     if (n < fine) n = fine;
@@ -490,10 +495,9 @@ static int launch_vec_r(hipStream_t s, fattn_args &a, int R) {
     // instead of after it (one round trip less per step, but masked cells - rows of the cache that may never have been written - then
     // come from memory cold, and every lane waits for them) 1.91-1.96 ms; measured again with the mask entries requested together:
     // 6.6 us for 256 cells that are all in use, but a decoded token 1.87 ms against 1.83.
-    constexpr int64_t one_head_max = 1024;
     // (quantized operands cost more arithmetic per cell: from 257 cells on their cells are split over groups)
     const bool quantized = a.type_k != MI355_F16 || a.type_v != MI355_F16;
-    if (a.Nkv <= one_head_max && !(quantized && a.Nkv > 256 && a.n_splits > 1)) {
+    if (a.Nkv <= ONE_HEAD_MAX && !(quantized && a.Nkv > 256 && a.n_splits > 1)) {
         if (a.Nq * a.Hq > 512) return launch_vec<D, 1>(s, a);
         // few (token, head) pairs: the chip is far from full
         constexpr int64_t step = 8 * 4 * (D <= 64 ? 8 : D <= 128 ? 4 : 2);   // cells a group of eight waves takes per step
@@ -542,7 +546,7 @@ static int fattn_fill(fattn_args &a, const float *q, const void *k, const void *
     a.m1 = powf(2.0f, -(max_bias / 2.0f) / n2);
     const size_t per_split = (size_t)Nq * (size_t)Hq * (size_t)(D + 2) * sizeof(float);
     const int64_t fit = ws ? (int64_t)(ws_bytes / per_split) : 0;   // as many as the scratch holds; none: run unsplit
-    int64_t n = pick_splits(Nkv, Hkv, Hq, Nq);
+    int64_t n = pick_splits(Nkv, Hkv, Hq, Nq, !k_f16 || !v_f16);
     if (n > fit) n = fit > 1 ? fit : 1;
     a.cells_per_split = (Nkv + n - 1) / n;
     a.n_splits = (int)((Nkv + a.cells_per_split - 1) / a.cells_per_split);   // no empty range

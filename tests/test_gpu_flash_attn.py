@@ -507,6 +507,21 @@ def test_prefill_ranges_of_cells_behind_mask_extents(dev, D, quantized, Nq, Nkv,
         assert orc.nmse(got[:, h:h + 1], _textbook(q[h:h + 1], k[kv], v[kv], mask, scale)) < 1e-12
 
 
+@pytest.mark.parametrize("D,Nq,Nkv,Hq,Hkv,launches", [(256, 62, 96, 16, 4, 1), (256, 21, 256, 32, 8, 1), (80, 45, 256, 16, 4, 1), (80, 16, 256, 32, 8, 1), (80, 17, 257, 32, 8, 2),
+                                                       (256, 35, 1024, 32, 8, 2)])
+def test_many_heads_over_few_cells(dev, D, Nq, Nkv, Hq, Hkv, launches):
+    """the vector kernel with a group per head: one launch up to 256 cells once there are more than 512 groups"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    q, k, v, mask = _inputs(np.random.default_rng(D + Nq), D, Nq, Nkv, Hq, Hkv, rand_mask=True)
+    args = [torch.from_numpy(a).to(dev) for a in (q, k, v, mask)]
+    before = lib.mi355_launch_count()
+    got = mi355.flash_attn_ext(*args, 1.0 / np.sqrt(D))
+    assert lib.mi355_launch_count() - before == launches
+    assert orc.nmse(got.cpu().numpy(), _textbook(q, k, v, mask, 1.0 / np.sqrt(D))) < 1e-12
+
+
 @pytest.mark.parametrize("Nq", [1, 3])
 @pytest.mark.parametrize("D,Hq,Hkv,one", [(80, 32, 8, 1024), (80, 25, 25, 768), (80, 20, 20, 1024), (112, 6, 3, 1024), (256, 32, 8, 512), (256, 16, 2, 512), (256, 33, 11, 512), (256, 50, 25, 448)])
 def test_decode_ranges_of_cells(dev, D, Hq, Hkv, one, Nq):
