@@ -125,9 +125,11 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
     __shared__ float s_o[NW][R][D];
 
     const int split = blockIdx.x;
-    // neighbouring groups are different kv heads: workgroups go to the XCDs in turn, so the groups of one kv head (a multiple of 8 apart where there are
-    // 8 kv heads, or 16) share an L2 and its rows are fetched once (64 / 8 heads of 256, 448 cells: 15.5 -> 11.6 us; 32 / 8 heads of 80, 1024: 17.0 -> 12.1)
-    const int64_t hk = blockIdx.y % (unsigned)a.Hkv, hg = blockIdx.y / (unsigned)a.Hkv, iq = blockIdx.z;
+    // Neighbouring groups are different kv heads: workgroups go to the XCDs in turn, so the groups of one kv head (a multiple of 8 apart where there are
+    // 8 kv heads, or 16) share an L2 and its rows are fetched once (64 / 8 heads of 256, 448 cells: 15.5 -> 11.6 us; 32 / 8 heads of 80, 1024: 17.0 -> 12.1).
+    // far_apart: that many ranges of cells that they would not run at the same time; then the kv head's groups are neighbours (launch_vec)
+    const unsigned per = a.far_apart ? (unsigned)a.groups : (unsigned)a.Hkv, quot = blockIdx.y / per, rem = blockIdx.y - quot * per;
+    const int64_t hk = a.far_apart ? quot : rem, hg = a.far_apart ? rem : quot, iq = blockIdx.z;
     const int64_t head0 = (hk * a.groups + hg) * R;   // first of this group's R query heads
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sub = lane % LPR, slot = wave * CPW + lane / LPR;
@@ -461,6 +463,9 @@ template <int D, int R, int NW = 4>
 static int launch_vec(hipStream_t s, fattn_args &a) {
     const bool quant = a.type_k != MI355_F16 || a.type_v != MI355_F16;
     a.groups = (int)(a.Hq / a.Hkv) / R;
+    // One row, 49152 cells, device us, kv heads / a kv head's groups as neighbours: 64 / 8 heads of 256 187 / 164, of 112 94.5 / 90.2, 32 / 4 heads of 80 45.7 / 44.2;
+    // fewer ranges, 64 / 8 heads of 256 over 8192 cells 33.7 / 35.9, 32 / 4 over 16384 35.1 / 36.9
+    a.far_apart = a.n_splits > 1 && a.n_splits * a.Hkv >= 512;
     const dim3 grid((unsigned)a.n_splits, (unsigned)(a.Hkv * a.groups), (unsigned)a.Nq);
     if constexpr (D % 32 == 0) {
         const bool same = a.type_k == a.type_v && D == 128;   // the caches llama.cpp builds with -ctk / -ctv of one type

@@ -35,6 +35,7 @@ struct fattn_args {
     unsigned n_head_log2;
     int n_splits;
     int groups;      // head groups of R per kv head: Hq / Hkv == R * groups
+    bool far_apart = false;   // k_fattn_vec: blockIdx.y counts the groups of a kv head first, then the kv heads
     int64_t cells_per_split;
 };
 

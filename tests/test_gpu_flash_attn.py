@@ -522,6 +522,16 @@ def test_many_heads_over_few_cells(dev, D, Nq, Nkv, Hq, Hkv, launches):
     assert orc.nmse(got.cpu().numpy(), _textbook(q, k, v, mask, 1.0 / np.sqrt(D))) < 1e-12
 
 
+@pytest.mark.parametrize("D,Nq,Nkv,Hq,Hkv", [(80, 1, 16129, 64, 8), (80, 1, 16128, 64, 8), (112, 2, 22000, 30, 6), (256, 1, 33000, 16, 4), (256, 1, 5500, 72, 24)])
+def test_vector_kernel_order_of_groups(dev, D, Nq, Nkv, Hq, Hkv):
+    """both orders of the groups (ranges x kv heads on both sides of 512): every (kv head, head of its group) pair has its own result"""
+    import torch
+    import mi355
+    q, k, v, mask = _inputs(np.random.default_rng(D + Nkv), D, Nq, Nkv, Hq, Hkv, rand_mask=True)
+    got = mi355.flash_attn_ext(*[torch.from_numpy(a).to(dev) for a in (q, k, v, mask)], 1.0 / np.sqrt(D))
+    assert orc.nmse(got.cpu().numpy(), _textbook(q, k, v, mask, 1.0 / np.sqrt(D))) < 1e-12
+
+
 @pytest.mark.parametrize("Nq", [1, 3])
 @pytest.mark.parametrize("D,Hq,Hkv,one", [(80, 32, 8, 1024), (80, 25, 25, 768), (80, 20, 20, 1024), (112, 6, 3, 1024), (256, 32, 8, 512), (256, 16, 2, 512), (256, 33, 11, 512), (256, 50, 25, 448)])
 def test_decode_ranges_of_cells(dev, D, Hq, Hkv, one, Nq):
