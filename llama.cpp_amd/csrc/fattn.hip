@@ -447,10 +447,14 @@ static int heads_per_group(int64_t R) { return R % 4 == 0 ? 4 : R % 2 == 0 ? 2 :
 // 512 cells 15.1 / 11.5, 1024 15.3 / 11.6, 2048 15.3 / 11.6.
 // (launch_vec_r gives every head a group of its own over few cells: from 512 such groups on ranges of 256 cells alone; 62 rows over 96 cells,
 // 16 / 4 heads of 256, 18.5 us in two ranges, 10.7 in one; 21 rows over 256 cells, 32 / 8 heads 21.2 / 16.0)
-static int pick_splits(int64_t Nkv, int64_t Hkv, int64_t Hq, int64_t Nq, bool quantized) {
+static int pick_splits(int64_t D, int64_t Nkv, int64_t Hkv, int64_t Hq, int64_t Nq, bool quantized) {
     const int64_t by_len = (Nkv + 255) / 256, by_fill = 2048 / (Hkv * Nq);
     const int64_t groups = Nkv <= (quantized ? 256 : ONE_HEAD_MAX) && Nq * Hq > 512 ? Nq * Hq : Hq / heads_per_group(Hq / Hkv) * Nq;
-    const int64_t fine_len = (Nkv + 63) / 64, fine_fill = 512 / groups;
+    const int64_t fine_len = (Nkv + 63) / 64;
+    // Whole turns of the eight XCDs, so that a range of cells is on one of them whatever the head: with 21 or 42 ranges one row over 4096 cells, 24 / 24 heads of
+    // 112, took 16.4 us (device; 16 ranges 14.5), two over 2048, 12 / 12 heads 12.0 (16: 8.6), one over 8192 16.6 (40: 14.6).  Not head size 256, whose steps take
+    // longer than the fetches: three over 4096, 32 / 8 heads 30.4 (16: 32.6).
+    const int64_t fill = 512 / groups, fine_fill = D <= 128 && fill >= 8 ? fill & ~(int64_t)7 : fill;
     int64_t n = by_len < by_fill ? by_len : by_fill;
     const int64_t fine = fine_len < fine_fill ? fine_len : fine_fill;
     if (n < fine) n = fine;
@@ -551,7 +555,7 @@ static int fattn_fill(fattn_args &a, const float *q, const void *k, const void *
     a.m1 = powf(2.0f, -(max_bias / 2.0f) / n2);
     const size_t per_split = (size_t)Nq * (size_t)Hq * (size_t)(D + 2) * sizeof(float);
     const int64_t fit = ws ? (int64_t)(ws_bytes / per_split) : 0;   // as many as the scratch holds; none: run unsplit
-    int64_t n = pick_splits(Nkv, Hkv, Hq, Nq, !k_f16 || !v_f16);
+    int64_t n = pick_splits(D, Nkv, Hkv, Hq, Nq, !k_f16 || !v_f16);
     if (n > fit) n = fit > 1 ? fit : 1;
     a.cells_per_split = (Nkv + n - 1) / n;
     a.n_splits = (int)((Nkv + a.cells_per_split - 1) / a.cells_per_split);   // no empty range

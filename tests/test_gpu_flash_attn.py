@@ -522,9 +522,11 @@ def test_many_heads_over_few_cells(dev, D, Nq, Nkv, Hq, Hkv, launches):
     assert orc.nmse(got.cpu().numpy(), _textbook(q, k, v, mask, 1.0 / np.sqrt(D))) < 1e-12
 
 
-@pytest.mark.parametrize("D,Nq,Nkv,Hq,Hkv", [(80, 1, 16129, 64, 8), (80, 1, 16128, 64, 8), (112, 2, 22000, 30, 6), (256, 1, 33000, 16, 4), (256, 1, 5500, 72, 24)])
+@pytest.mark.parametrize("D,Nq,Nkv,Hq,Hkv", [(80, 1, 16129, 64, 8), (80, 1, 16128, 64, 8), (112, 2, 22000, 30, 6), (256, 1, 33000, 16, 4), (256, 1, 5500, 72, 24),
+                                              (112, 1, 4096, 24, 24), (112, 2, 2050, 12, 12), (80, 1, 8191, 12, 12), (256, 3, 4097, 32, 8)])
 def test_vector_kernel_order_of_groups(dev, D, Nq, Nkv, Hq, Hkv):
-    """both orders of the groups (ranges x kv heads on both sides of 512): every (kv head, head of its group) pair has its own result"""
+    """both orders of the groups (ranges x kv heads on both sides of 512), numbers of ranges that are whole turns of the XCDs and not: every (kv
+    head, head of its group) pair has its own result"""
     import torch
     import mi355
     q, k, v, mask = _inputs(np.random.default_rng(D + Nkv), D, Nq, Nkv, Hq, Hkv, rand_mask=True)
