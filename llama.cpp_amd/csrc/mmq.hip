@@ -681,7 +681,10 @@ static size_t mmq_slab_bytes(int n, int64_t rows, int64_t B) { return (size_t)n 
 // eight slices, at most two groups per compute unit; more of them, up to sixteen, where a model of the time in us says so, which a sweep of n = 1 .. 16 over
 // (1024 .. 21603 rows, 10 .. 112 stages, 50 .. 512 columns) meets within some 15 %: a stage takes 1.2 (64 columns) or 2.1 (128), Q6_K 1.7 times that; 1.4
 // times with a second group on the compute unit; the sum 4, and 8 bytes per value and slice at 4 TB/s.  A call, us: Q6_K 1135 x 7424, 65 rows
-// 41.2 -> 30.9 (16 slices instead of 8), Q5_1 3509 x 1216, 73 rows 23.6 -> 18.9 (5 instead of 2).  (Fewer slices than these would be quicker here
+// 41.2 -> 30.9 (16 slices instead of 8), Q5_1 3509 x 1216, 73 rows 23.6 -> 18.9 (5 instead of 2).  Groups are counted as an XCD gets them, padded to eighths: 18
+// tiles in 12 slices are 36 on the 32 units of one (Q4_0 1115 x 11776, 184 rows 42.0 us; in 8 slices 39.5).  From 600 tiles on, where the whole chip is busy
+// twice over, the model's steps no longer tell (Q4_0 28743 x 6400, 326 rows 231 us uncut, 264 in two; Q4_1 20630 x 5888, 481 rows 251 and 284; on the
+// other side of the line Q4_1 18629 x 7168, 415 rows 301 and 276).  (Fewer slices than these would be quicker here
 // and there, Q5_0 8491 x 2016, 316 rows 49.9 -> 44.5 with one instead of two, but make longer f32 sums.)
 // ws_bytes: what is there for the partial sums; none of them fits: one slice.
 static int mmq_slices(int type, int64_t row_tiles, int64_t K, int64_t B, int64_t rows, size_t ws_bytes) {
@@ -695,8 +698,9 @@ static int mmq_slices(int type, int64_t row_tiles, int64_t K, int64_t B, int64_t
     const float stage = (bn == 64 ? 1.2f : 2.1f) * (type == MI355_Q6_K ? 1.7f : 1.0f);
     int64_t best = 1;
     float best_us = 0.0f;
-    for (int64_t n = least; n <= 16 && n <= stages; n++) {
-        const int64_t per = (stages + n - 1) / n, g = groups * n;
+    const int64_t most = groups < 600 ? 16 : least;
+    for (int64_t n = least; n <= most && n <= stages; n++) {
+        const int64_t per = (stages + n - 1) / n, g = (groups + 7) / 8 * 8 * n;
         if (n > 1 && mmq_slab_bytes((int)n, rows, B) > ws_bytes) break;
         if ((stages + per - 1) / per != n) continue;
         const float busy = g <= 256 ? 1.0f : 1.4f * (float)((g + 511) / 512);

@@ -992,3 +992,11 @@ def test_tile_kernel_many_slices(dev, name, t, N, K, B):
         torch.cuda.synchronize()
         assert orc.nmse(got.cpu().numpy(), want) < 1e-11, room
         assert (ws[room:] == 255).all()
+
+
+def test_products_of_many_tiles_are_not_cut(dev):
+    """per-block tiles: from 600 tiles on the chip is busy without slices along K"""
+    import mi355
+    lib = mi355.load()
+    for N, K, B, cut in ((28743, 6400, 326, False), (20630, 5888, 481, False), (38400, 8192, 256, False), (18629, 7168, 415, True), (1115, 11776, 184, True)):
+        assert (int(lib.mi355_mul_mat_q_ws_bytes(N, K, B)) > 0) == cut, (N, K, B)
