@@ -955,6 +955,14 @@ static bool fsq_describe(int type, const kv_src &q, fsq_src &o) {
     return true;
 }
 
+// Groups per kv head of `waves` tiles each; with empty ones to whole turns of the eight XCDs where that leaves one group per compute unit, so that a group's range of
+// cells is on one XCD whatever the head: Q4_0, 32 / 8 heads, device us, 9216 cells 29 groups 20.1, 32 16.7 (two to four tiles per wave 18.4); 11776 cells 31
+// groups 21.9, 32 18.5 (21.2).  (Not over f16, whose rows are whole lines: 24 / 8 heads, 5120 cells 12.3 / 13.2.)  most: what the workspace rule allows
+static int64_t fsq_one_groups(int64_t n_tiles, int64_t waves, int64_t Hkv, int64_t most) {
+    const int64_t n = (n_tiles + waves - 1) / waves, whole = (n + 7) / 8 * 8;
+    return whole * Hkv <= FSQ_TOTAL_GROUPS && whole <= most ? whole : n;
+}
+
 // One query token over a long Q8_0 / Q4_0 cache in the device row layout (a.type_k, a.type_v, a.kq, a.vq filled in), head size 128,
 // R <= 4.  Sets a.n_splits; the caller merges the splits with k_fattn_combine.  Returns 1 when the shape is not served.
 int launch_fattn_dec_stream_q(hipStream_t s, fattn_args &a, int64_t D, size_t ws_bytes) {
@@ -979,7 +987,7 @@ int launch_fattn_dec_stream_q(hipStream_t s, fattn_args &a, int64_t D, size_t ws
     // A tile per wave where one group per compute unit holds them all.  Five waves of Q8_0 only for up to two query heads per kv head (10240 cells,
     // 16 / 8 heads 19.4 -> 18.2 us, 32 / 8 heads 20.35 -> 20.45).
     bool one = false;
-    const int64_t one_wv = (n_tiles * a.Hkv + FSQ_TOTAL_GROUPS - 1) / FSQ_TOTAL_GROUPS, one_groups = (n_tiles + one_wv - 1) / one_wv;
+    const int64_t one_wv = (n_tiles * a.Hkv + FSQ_TOTAL_GROUPS - 1) / FSQ_TOTAL_GROUPS, one_groups = fsq_one_groups(n_tiles, one_wv, a.Hkv, n_splits);
     const int one_max = a.type_k == MI355_Q8_0 && a.type_v == MI355_Q8_0 && R > 2 ? 4 : fsq_waves_one_rt(a.type_k, a.type_v);
     if (tiles_per_wave > 1 && one_wv <= one_max && one_groups <= n_splits) {
         one = true;
