@@ -173,6 +173,17 @@ def mul_mat(kind, t, W, x, n_threads=4):
     return out
 
 
+def mul_mat_all(t, W, x):
+    """every output of a large product: the reference CPU backend's, or where it is not built the dequantized weights times x in f32 (the
+    activations' quantization to 8 bits is then part of the difference: NMSE some 3e-5)"""
+    if ref is not None:
+        return mul_mat("ref", t, W, x, n_threads=16)
+    from concurrent.futures import ThreadPoolExecutor
+    x = f32(x)
+    with ThreadPoolExecutor(max_workers=16) as ex:   # the products themselves run on all cores
+        return np.concatenate([x @ w.T for w in ex.map(lambda i: dequantize("oracle", t, W[i:i + 2048], x.shape[1]), range(0, W.shape[0], 2048))], axis=1)
+
+
 def flash_attn(kind, q, k, v, mask, scale, max_bias=0.0, softcap=0.0, n_threads=4):
     """q f32 [Hq,Nq,D]; k,v f16-bits uint16 [Hkv,Nkv,D]; mask uint16 [Nq_pad,Nkv] or None -> f32 [Nq,Hq,D]"""
     Hq, Nq, D = q.shape
