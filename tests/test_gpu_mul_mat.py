@@ -12,7 +12,7 @@ TYPES = list(orc.WEIGHT_TYPES.items())
 
 def _weights(rng, t, N, K, kind="oracle"):
     Wf = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
-    return orc.quantize("ref" if (kind == "ref" and orc.ref is not None) else "oracle", t, Wf)
+    return orc.quantize_mt("ref" if (kind == "ref" and orc.ref is not None) else "oracle", t, Wf)
 
 
 def _to_dev(dev, a):
@@ -999,3 +999,11 @@ def test_products_of_many_tiles_are_not_cut(dev):
     lib = mi355.load()
     for N, K, B, cut in ((28743, 6400, 326, False), (20630, 5888, 481, False), (38400, 8192, 256, False), (18629, 7168, 415, True), (1115, 11776, 184, True)):
         assert (int(lib.mi355_mul_mat_q_ws_bytes(N, K, B)) > 0) == cut, (N, K, B)
+
+
+def test_a_short_last_slice_costs_no_round():
+    """per-block tiles: the fewest slices stay where only the groups of a short last slice exceed what the compute units hold at once"""
+    import mi355
+    lib = mi355.load()
+    for N, K, B, slices in ((2813, 2080, 287, 4), (4755, 2176, 144, 4), (5309, 3392, 231, 6), (10772, 4640, 65, 6)):
+        assert int(lib.mi355_mul_mat_q_ws_bytes(N, K, B)) == slices * N * B * 4, (N, K, B)
