@@ -813,14 +813,16 @@ __global__ void __launch_bounds__(256) k_fattn_half_merge(fattn_args a) {
 // (64 .. 256 head size, 24 .. 256 groups, 2 .. 256 tiles of 64 cells, n = 1 .. 16), which it meets within some 15 %: a tile step takes
 // 0.95 (D 64), 1.4 (up to 128) or 3.4 us (256: one group per compute unit), 1.34 times that with a second group on the compute unit; the merge 4
 // and 8 bytes per value and range at 4 TB/s.  Before / after, us: 64 rows over 8192 cells, 32 / 8 heads, D 128 146 -> 32; 343 x 3840, 4 / 4 heads, D 64
-// 51 -> 18; 268 x 3776, 32 / 8, D 128 77 -> 50; 512 x 4096 81 -> 72 (n = 2); 300 x 2500, 8 / 8, D 256 136 -> 41; not cut: 560 x 672, 16 / 4 (22.5; 27 in three).
-// (probabilities of f32 precision: one launch up to 2048 cells)
+// 51 -> 18; 268 x 3776, 32 / 8, D 128 77 -> 50; 512 x 4096 79.8 -> 69.2 (n = 2); 300 x 2500, 8 / 8, D 256 136 -> 41; not cut: 560 x 672, 16 / 4 (22.5; 27 in three).
+// Probabilities of f32 precision: one launch up to 2048 cells.  Shorter walks gain too, but over few cells the sum of ranges is in places further from 64 bits
+// than one walk; whole / in ranges, us and error: 300 rows x 512 cells, 8 / 8 heads, D 256 36.5 / 26.7 and 1.74e-7 / 1.76e-7, D 80 16.6 / 13.6 and 1.64e-7 /
+// 1.68e-7, x 1024 26.0 / 16.2 and 1.75e-7 / 1.77e-7.  At 2048 cells the errors are smaller in ranges (300 rows, D 256 109.8 / 39.5 us, 2.21e-7 / 2.02e-7;
+// 64 rows, 32 / 8 heads, D 80 43.6 / 16.7, 2.00e-7 / 1.97e-7; 512 rows are not cut): the line could lie there, it has not been looked for between 1024 and 2048.
 static bool half_may_split(const fattn_args &a, bool px) { return (!px || a.Nkv > 2048) && a.ws != nullptr && ((uintptr_t)a.ws & 15) == 0; }
-struct half_plan { int64_t n; float us; };
-static half_plan plan_half(int64_t D, int64_t groups, int64_t rows, int64_t tiles, bool wide, size_t ws_bytes) {
+static int64_t plan_half(int64_t D, int64_t groups, int64_t rows, int64_t tiles, bool wide, size_t ws_bytes) {
     const float step = D == 64 ? 0.95f : D <= 128 ? 1.4f : 3.4f;
-    half_plan best = {1, 0.0f};
-    float whole = 0.0f;
+    int64_t best = 1;
+    float best_us = 0.0f, whole = 0.0f;
     for (int64_t n = 1; n <= 64 && n <= tiles; n++) {
         if (n > 1 && ws_bytes < (size_t)n * (size_t)rows * (size_t)(D + 2) * sizeof(float)) break;
         const int64_t g = groups * n, slots = D <= 128 ? 512 : 256;
@@ -829,23 +831,22 @@ static half_plan plan_half(int64_t D, int64_t groups, int64_t rows, int64_t tile
         if (n == 1 && wide) us *= 0.9f;   // eight waves on 128-cell tiles
         if (n > 1) us += 4.0f + (float)(rows * n * D) * 8.0f / 4e6f;
         if (n == 1) whole = us;
-        if (n == 1 || (us < best.us && us < 0.9f * whole)) best = {n, us};
+        if (n == 1 || (us < best_us && us < 0.9f * whole)) {
+            best = n;
+            best_us = us;
+        }
     }
     return best;
 }
 
-// groups of the launch below
-static dim3 half_grid(const fattn_args &a, bool pq) {
-    const int64_t R = a.Hq / a.Hkv, n_tiles = (a.Nq + 31) / 32;
-    return dim3((unsigned)(pq ? (n_tiles + 1) / 2 : n_tiles), (unsigned)(a.Hkv * (pq ? R : R / 2)));
-}
-
 template <int D, bool PQ, bool PX>
 int launch_half(hipStream_t s, fattn_args a, size_t ws_bytes) {
-    dim3 grid = half_grid(a, PQ);
+    const int64_t R = a.Hq / a.Hkv, n_tiles = (a.Nq + 31) / 32;
+    dim3 grid((unsigned)(PQ ? (n_tiles + 1) / 2 : n_tiles), (unsigned)(a.Hkv * (PQ ? R : R / 2)));
     const int64_t groups = (int64_t)grid.x * grid.y, rows = a.Nq * a.Hq, tiles = (a.Nkv + 63) / 64;
-    // at most one group per compute unit and a long cache: eight waves on 128-cell tiles (512 rows: 4096 cells 112 -> 103 us,
-    // 512 cells 24.8 -> 26.2 us).  Head size 256: the eight waves' registers do not fit.
+    // at most one group per compute unit and a long cache: eight waves on 128-cell tiles (an earlier form of the kernel, 512 rows: 4096 cells 112 -> 103 us).
+    // Below 1024 cells four waves are quicker, four / eight, us: 512 rows, D 128, 32 / 8 heads, 512 cells 17.3 / 19.3, 768 22.2 / 23.3; D 80, 32 / 32, 512 17.5 / 18.5,
+    // 960 27.1 / 31.0; D 112, 32 / 8, 960 33.5 / 37.1; quantized output, D 64, 512 19.2 / 19.4.  Head size 256: the eight waves' registers do not fit.
     const bool wide = D <= 128 && groups <= 256 && a.Nkv >= 1024;
     // the groups read the mask extents, at the front of the scratch memory, while others write their states: those lie behind
     if (a.kv_extent) {
@@ -853,7 +854,7 @@ int launch_half(hipStream_t s, fattn_args a, size_t ws_bytes) {
         a.ws += used / sizeof(float);
         ws_bytes = ws_bytes > used ? ws_bytes - used : 0;
     }
-    const int64_t n = half_may_split(a, PX) ? plan_half(D, groups, rows, tiles, wide, ws_bytes).n : 1;
+    const int64_t n = half_may_split(a, PX) ? plan_half(D, groups, rows, tiles, wide, ws_bytes) : 1;
     a.cells_per_split = (tiles + n - 1) / n * 64;
     a.n_splits = (int)((a.Nkv + a.cells_per_split - 1) / a.cells_per_split);   // no empty range
     grid.z = (unsigned)a.n_splits;
