@@ -576,7 +576,11 @@ __global__ void __launch_bounds__(256, 2) k_mmq_kp(const uint8_t *__restrict__ W
         row0 = (int64_t)(lid / n_col_tiles) * BM;
         col0 = (int64_t)(lid % n_col_tiles) * BN;
     } else {
-        // column tile by column tile over the whole chip, in the order of their work (k_route_slots): the last groups are the short ones
+        // Column tile by column tile over the whole chip, in the order of their work (k_route_slots): the last groups are the short ones.  Experts of many column
+        // tiles gain less, row panel by row panel on an XCD / so, us: 8 experts of 12032 x 4608, 1040 slots Q4_K 255 / 237, IQ4_XS 283 / 271, 4160 slots Q4_K 820 / 763,
+        // 4 of 14336 x 4096, 4160 slots Q6_K 912 / 847; the order loses where a Q6_K panel is read eight times and more and the row tiles are no multiple of 8
+        // (2 of 6944 x 7936, 2080 slots 704 / 736; 8 of 12032 x 4608, 4160 slots 1436 / 1462).  Row tiles padded to multiples of 8, so that a panel stays on one
+        // XCD, take 2 .. 4 % off those and add up to a third elsewhere (8 of 1088 x 4096, 3200 slots).
         const int n_row_tiles = n_groups / n_col_tiles, ct = (int)blockIdx.x / n_row_tiles;
         row0 = (int64_t)((int)blockIdx.x - ct * n_row_tiles) * BM;
         if (ct >= *route.n_tiles) return;
