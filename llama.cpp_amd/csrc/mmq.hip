@@ -403,7 +403,9 @@ __global__ void __launch_bounds__(256, 2) k_mmq(mmq_mats mats, const int8_t *__r
     const int lid = ID ? (int)blockIdx.x : (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
     if (lid >= n_groups) return;   // uniform for the whole group
     // ID: column tile by column tile over the whole chip, in the order of their work (k_route_slots), so that the last groups are the short
-    // ones (8 experts of 14336 x 4096, 1024 slots: Q4_0 301 -> 238 us, Q8_0 342 -> 295; Q6_K 8 of 4096 x 2304, 600 slots 131 -> 95)
+    // ones (8 experts of 14336 x 4096, 1024 slots: Q4_0 301 -> 238 us, Q8_0 342 -> 295; Q6_K 8 of 4096 x 2304, 600 slots 131 -> 95).  With many column
+    // tiles per expert it is even: row panel by row panel on an XCD / so, 8 of 12032 x 4608, 1040 slots Q4_0 290 / 266, 4160 slots Q4_0 808 / 789, Q8_0 874 / 877;
+    // 2 of 6944 x 7936, 2080 slots Q8_0 420 / 426
     // (uniform: kept in scalar registers, although the division goes through the vector ALU)
     const int per_row = ID ? n_groups / n_col_tiles : n_col_tiles;
     const int first = __builtin_amdgcn_readfirstlane(lid / per_row), second = lid - first * per_row;
