@@ -687,7 +687,9 @@ static size_t mmq_slab_bytes(int n, int64_t rows, int64_t B) { return (size_t)n 
 // tiles in 12 slices are 36 on the 32 units of one (Q4_0 1115 x 11776, 184 rows 42.0 us; in 8 slices 39.5).  From 600 tiles on, where the whole chip is busy
 // twice over, the model's steps no longer tell (Q4_0 28743 x 6400, 326 rows 231 us uncut, 264 in two; Q4_1 20630 x 5888, 481 rows 251 and 284; on the
 // other side of the line Q4_1 18629 x 7168, 415 rows 301 and 276).  A short last slice of the fewest does not count: Q4_1 5309 x 3392, 231 rows in six slices (five
-// stages each, two in the last) 42.7 us, in seven 48.3; Q8_0 4755 x 2176, 144 rows in four 29.4, in six 32.4.  (Fewer slices than these would be quicker here
+// stages each, two in the last) 42.7 us, in seven 48.3; Q8_0 4755 x 2176, 144 rows in four 29.4, in six 32.4.  Up to two thirds of the others are short where the second
+// round is of padding only: Q4_0 2477 x 4096, 626 rows, 100 tiles in five slices (seven stages, four in the last) 49.1, in eight 53.4; with 20 of 22 stages in the last
+// Q5_1 2537 x 13792, 527 rows in five 149, in nine 124.  (Fewer slices than these would be quicker here
 // and there, Q5_0 8491 x 2016, 316 rows 49.9 -> 44.5 with one instead of two, but make longer f32 sums.)
 // ws_bytes: what is there for the partial sums; none of them fits: one slice.
 static int mmq_slices(int type, int64_t row_tiles, int64_t K, int64_t B, int64_t rows, size_t ws_bytes) {
@@ -707,7 +709,9 @@ static int mmq_slices(int type, int64_t row_tiles, int64_t K, int64_t B, int64_t
         if (n > 1 && mmq_slab_bytes((int)n, rows, B) > ws_bytes) break;
         if ((stages + per - 1) / per != n) continue;
         // the fewest slices, whose last one is short: its groups run beside or behind the others and do not count
-        const int64_t at_once = n == least && n > 1 && 2 * (stages - (n - 1) * per) <= per ? g / n * (n - 1) : g;
+        const int64_t last = stages - (n - 1) * per;
+        const bool is_short = 2 * last <= per || (3 * last <= 2 * per && groups * n <= 512 && g > 512);
+        const int64_t at_once = n == least && n > 1 && is_short ? g / n * (n - 1) : g;
         const float busy = at_once <= 256 ? 1.0f : 1.4f * (float)((at_once + 511) / 512);
         const float us = (float)per * stage * busy + (n > 1 ? 4.0f + (float)(n * rows * B) * 8.0f / 4e6f : 0.0f);
         if (n == least || us < 0.95f * best_us) {

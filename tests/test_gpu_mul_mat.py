@@ -1005,5 +1005,6 @@ def test_a_short_last_slice_costs_no_round():
     """per-block tiles: the fewest slices stay where only the groups of a short last slice exceed what the compute units hold at once"""
     import mi355
     lib = mi355.load()
-    for N, K, B, slices in ((2813, 2080, 287, 4), (4755, 2176, 144, 4), (5309, 3392, 231, 6), (10772, 4640, 65, 6)):
+    for N, K, B, slices in ((2813, 2080, 287, 4), (4755, 2176, 144, 4), (5309, 3392, 231, 6), (10772, 4640, 65, 6), (2477, 4096, 626, 5), (12317, 4096, 54, 5),
+                            (2537, 13792, 527, 9)):
         assert int(lib.mi355_mul_mat_q_ws_bytes(N, K, B)) == slices * N * B * 4, (N, K, B)
