@@ -95,6 +95,9 @@ static int gf_rpw(int64_t N) { return N <= 2048 ? 1 : 2; }
 // The quantization is paid once per group: from some four groups of 4096 elements per compute unit on (28672 x 8192: 22.8 / 22.5, 32768 x 2048
 // 11.1 / 11.2) and, for two or three rows, from the second group per unit on (8882 x 1056 Q4_0, 2 rows: 6.2 / 6.9) it costs what the
 // launch did.  Long rows are longer chains per wave here, with half of k_gemv_q's waves (4096 x 14336 Q4_0: 9.6 / 10.9).
+// Inside that line the device loses where a few units get a third group or two or three rows meet the types with the most arithmetic per byte: 8975 x 5120, 1 row
+// Q4_K 8.9 / 8.9, Q5_0 9.5 / 10.1, Q6_K 11.2 / 11.9, IQ4_XS 10.4 / 11.4, IQ4_NL 9.6 / 10.9; 2547 x 4096, 3 rows Q4_K 6.9 / 5.9, IQ4_NL 6.8 / 7.0, Q6_K 7.2 / 7.7.
+// They stay: a call that is not replayed from a graph takes 13.5 us of host time with two launches and 7 with one.
 static bool gf_faster(int64_t N, int64_t K, int64_t B) {
     if (B > 3 || K > 8192) return false;
     const int64_t groups = (N + GF_WAVES * gf_rpw(N) - 1) / (GF_WAVES * gf_rpw(N));
