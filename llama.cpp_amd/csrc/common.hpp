@@ -156,6 +156,29 @@ __device__ __forceinline__ float sub_rn(float a, float b) {
     return a - b;
 }
 
+// ---- Q8_0 / Q8_1 levels (quantize_row_q8_0_ref / _q8_1_ref, ggml/src/ggml-quants.c:194-253): d = amax / 127, id = d ? 1 / d : 0, level = roundf(v * id), bit for
+// bit, in a third of the instructions of the two divisions and the library's roundf (a launch whose groups each quantize the row for themselves is bound by them).
+// Both quotients are one multiplication by a reciprocal and one correction by the exact remainder: equal to the IEEE quotient for every mantissa (2^23 of a / 127
+// compared on the host, 1 / d for every mantissa and the exponents 20 .. 233 on gfx950).  Where a remainder could leave the normal range, and for infinities and NaN, the
+// divisions themselves run (no lane takes that branch in ordinary rows).
+__device__ __forceinline__ void q8_scale(float amax, float &d, float &id) {
+    constexpr float R127 = 0x1.020408p-7f;   // 1 / 127
+    const float q = mul_rn(amax, R127);
+    d = __builtin_fmaf(__builtin_fmaf(-127.0f, q, amax), R127, q);
+    const float r = __builtin_amdgcn_rcpf(d);
+    id = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+    id = d != 0.0f ? id : 0.0f;
+    if (!(amax >= 0x1p-90f && amax <= 0x1p90f) && amax != 0.0f) {
+        d = amax / 127.0f;
+        id = d != 0.0f ? 1.0f / d : 0.0f;
+    }
+}
+// roundf: the largest float below a half, added away from zero, carries exactly the fractions from a half on into the next integer (all floats up to 2^22 compared)
+__device__ __forceinline__ int q8_level(float v, float id) {
+    const float x = mul_rn(v, id);
+    return (int)add_rn(x, __builtin_copysignf(0x1.fffffep-2f, x));
+}
+
 // Sum over the 64 lanes with DPP row operations (no LDS round trips: a __shfl_xor butterfly is six ds_bpermute of about a hundred
 // cycles each), broadcast from lane 63 through a scalar register.  Every lane gets the same value.
 template <int CTRL, int ROWMASK>

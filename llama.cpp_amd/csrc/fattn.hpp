@@ -43,9 +43,9 @@ struct fattn_args {
 // ggml/src/ggml-quants.c:220-253); e = element index inside the query row of k elements
 __device__ __forceinline__ void quantize_lane32(float v, int8_t *__restrict__ qrow, act_ds *__restrict__ srow, int64_t e) {
     const float amax = lanes_max<32>(fabsf(v));
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    const int q = (int)roundf(v * id);
+    float d, id;
+    q8_scale(amax, d, id);
+    const int q = q8_level(v, id);
     const int sum = lanes_sum_i<32>(q);
     qrow[e] = (int8_t)q;
     if ((e & 31) == 0) {

@@ -1035,8 +1035,8 @@ __global__ void __launch_bounds__(256, 2) k_fattn_mma_dec(fattn_args a, int R, i
             for (int g = 0; g < 4; g++) *(f32x4 *)(dp + 32 * dt + 8 * g + 4 * lhi) = f32x4{w[4 * g], w[4 * g + 1], w[4 * g + 2], w[4 * g + 3]};
             if (a.act_q) {   // Q8_1 of this 32-element block of the head (quantize_row_q8_1_ref, ggml-quants.c:220-253)
                 amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-                const float d = amax / 127.0f;
-                const float id = d != 0.0f ? 1.0f / d : 0.0f;
+                float d, id;
+                q8_scale(amax, d, id);
                 int sum = 0;
                 const int64_t e0 = head * D + d_first + 32 * dt;   // first element of the block inside the activation row
                 int8_t *qrow = a.act_q + iq * a.Hq * D + e0;
@@ -1045,7 +1045,7 @@ __global__ void __launch_bounds__(256, 2) k_fattn_mma_dec(fattn_args a, int R, i
                     u32 packed = 0;
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        const int q = (int)roundf(w[4 * g + i] * id);
+                        const int q = q8_level(w[4 * g + i], id);
                         sum += q;
                         packed |= (u32)(q & 0xFF) << (8 * i);
                     }

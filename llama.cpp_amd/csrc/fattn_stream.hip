@@ -421,15 +421,15 @@ __device__ __forceinline__ void fsq_load_q(const fattn_args &a, int64_t head0, i
 #pragma unroll
             for (int j = 0; j < 4; j++) amax = fmaxf(amax, fabsf(x[i][j]));
         }
-        const float d = amax / 127.0f;
-        const float id = d != 0.0f ? 1.0f / d : 0.0f;
+        float d, id;
+        q8_scale(amax, d, id);
         int sum = 0;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             u32 w = 0;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int q = (int)roundf(x[i][j] * id);
+                const int q = q8_level(x[i][j], id);
                 sum += q;
                 w |= (u32)(q & 0xFF) << (8 * j);
             }

@@ -52,12 +52,12 @@ __device__ __forceinline__ void gate_up_blk_phase(const uint8_t *__restrict__ Wg
     const int c_first = lane < nchunks ? lane : nchunks - 1;
     int8_t *s_q = (int8_t *)s_act;
     act_ds *s_ds = (act_ds *)(s_act + NCOLS * K);
-    {
+    act_copy<NCOLS, 64 * WAVES> copy;
+    copy.request(aq, ads, K);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < 2 * R; r++) w_first[r] = T::load_w(rows[r], L, c_first);
-        for (int i = threadIdx.x * 16; i < NCOLS * K; i += 64 * WAVES * 16) *(u32x4 *)(s_q + i) = load16(aq + i);
-        for (int i = threadIdx.x; i < NCOLS * nblk; i += 64 * WAVES) s_ds[i] = ads[i];
-    }
+    for (int r = 0; r < 2 * R; r++) w_first[r] = T::load_w(rows[r], L, c_first);
+    copy.commit(s_act, aq, ads, K);
     __syncthreads();
 #pragma unroll
     for (int round = 0; round < RPM / R; round++) {

@@ -76,13 +76,13 @@ struct gemv_batch {
 // waves read it from there; otherwise every wave reads it from memory.  On the 14336 x 4096 Q4_K product the activation
 // reads of the 7168 waves (36 MB from L2) outweighed the 33 MB of weights and competed with them: 8.7 -> 7.9 us with the
 // copy in LDS.  The first step's weight loads are issued before the copy, so the copy's round trip hides behind them.
-template <int TYPE, int NCOLS, int RPW, bool QKV = false, bool COH = false, bool LDSA = false, bool NORM = false>
+template <int TYPE, int NCOLS, int RPW, bool QKV = false, bool COH = false, bool LDSA = false, bool NORM = false, int WAVES = 4>
 __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const int8_t *__restrict__ aq,
                                           const act_ds *__restrict__ ads, int K, const gemv_rope *rp = nullptr, uint8_t *s_act = nullptr) {
     typedef wq<TYPE> T;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t row0 = ((int64_t)group * 4 + wave) * RPW;
+    const int64_t row0 = ((int64_t)group * WAVES + wave) * RPW;
     const bool wave_live = row0 < m.N;   // uniform over the wave
     if (!LDSA && !wave_live) return;     // with the copy in LDS a wave without rows still takes its share of the copy
 
@@ -103,41 +103,52 @@ __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const i
 #pragma unroll
         for (int c = 0; c < NCOLS; c++) acc[r][c] = 0.0f;
 
-    // QKV: lane c finishes activation row c.  Its rotation and cache cell depend on nothing the product computes, so they are
-    // worked out here, while the weight loads of the first step are in flight (the empty asm keeps them from being moved
-    // behind the loop, next to their use).
+    // The order of the requests: a wave's loads return as they were issued, so the activation comes first (with what the QKV epilogue needs to know), the first step's
+    // weights behind it, and what can be computed without the weights is done while they are on their way.
+    typename T::chunk w_first[RPW];
     float rope_c = 1.0f, rope_s = 0.0f;
-    int cell = 0;
-    bool rotate = false;
+    int pos = 0, cell = 0;
     if constexpr (QKV) {
+        const int col = lane < NCOLS ? lane : NCOLS - 1;
+        if (rp->pos) pos = rp->pos[col];       // null where no matrix of the launch is rotated
+        if (rp->cells) cell = rp->cells[col];  // ... or goes to a cache
+    }
+    // QKV: lane c finishes activation row c.  Its rotation depends on nothing the product computes (the empty asm keeps it from being moved behind the loop, next
+    // to its use).
+    auto rotation = [&]() {
         if (lane < NCOLS) {
             const gemv_rope &R = *rp;
             const int d = (int)(row0 % R.D);
-            rotate = (m.epi == EPI_ROPE || m.epi == EPI_ROPE_CACHE) && d < R.n_dims;
-            if (rotate) rope_coeffs(R, R.pos[lane], d >> 1, rope_c, rope_s);
-            if (m.epi == EPI_ROPE_CACHE || m.epi == EPI_CACHE) cell = R.cells[lane];
+            if ((m.epi == EPI_ROPE || m.epi == EPI_ROPE_CACHE) && d < R.n_dims) rope_coeffs(R, pos, d >> 1, rope_c, rope_s);
         }
-        asm volatile("" : "+v"(rope_c), "+v"(rope_s), "+v"(cell));
-    }
-
-    typename T::chunk w_first[RPW];
+        asm volatile("" : "+v"(rope_c), "+v"(rope_s));
+    };
+    const int c_first = lane < nchunks ? lane : nchunks - 1;
     if constexpr (LDSA) {
-        const int c = lane < nchunks ? lane : nchunks - 1;
-#pragma unroll
-        for (int r = 0; r < RPW; r++) w_first[r] = T::load_w(rows[r], L, c);
-        int8_t *s_q = (int8_t *)s_act;
-        act_ds *s_ds = (act_ds *)(s_act + NCOLS * K);
         if constexpr (NORM) {   // RMS_NORM -> MUL -> Q8_1 of the one activation row straight into the group's LDS copy
             __shared__ float s_norm[4];
-            rms_norm_quant_row<4, false, false>(rp->nx, rp->nw, nullptr, s_act, 0, K, 1, rp->neps, s_norm);
+            norm_row<WAVES> row;
+            row.request(rp->nx, rp->nw, K);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < RPW; r++) w_first[r] = T::load_w(rows[r], L, c_first);
+            if constexpr (QKV) rotation();
+            row.finish(s_act, K, rp->neps, s_norm);
         } else {
-            for (int i = threadIdx.x * 16; i < NCOLS * K; i += 256 * 16) *(u32x4 *)(s_q + i) = load16(aq + i);
-            for (int i = threadIdx.x; i < NCOLS * nblk; i += 256) s_ds[i] = ads[i];
+            act_copy<NCOLS, 64 * WAVES> copy;
+            copy.request(aq, ads, K);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < RPW; r++) w_first[r] = T::load_w(rows[r], L, c_first);
+            if constexpr (QKV) rotation();
+            copy.commit(s_act, aq, ads, K);
         }
         __syncthreads();
         if (!wave_live) return;
-        aq = s_q;
-        ads = s_ds;
+        aq = (const int8_t *)s_act;
+        ads = (const act_ds *)(s_act + NCOLS * K);
+    } else if constexpr (QKV) {
+        rotation();
     }
 
     for (int c0 = 0; c0 < nchunks; c0 += 64) {
@@ -176,7 +187,7 @@ __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const i
             const int64_t head = row0 / R.D;
             const int d = (int)(row0 % R.D);
             float y0 = s0, y1 = s1;
-            if (rotate) rope_apply(rope_c, rope_s, s0, s1, y0, y1);
+            if ((m.epi == EPI_ROPE || m.epi == EPI_ROPE_CACHE) && d < R.n_dims) rope_apply(rope_c, rope_s, s0, s1, y0, y1);
             if (m.epi == EPI_ROPE || m.epi == EPI_STORE) {
                 float *o = m.dst + lane * m.dst_stride + row0;
                 o[0] = y0;
@@ -379,7 +390,8 @@ __global__ void __launch_bounds__(256) k_gemv_q(gemv_item m, const int8_t *__res
 }
 
 // ... with the RMS norm of the layer input computed by every group for itself (one activation row)
-__global__ void __launch_bounds__(256) k_gemv_qkv_norm(gemv_batch b, int K, gemv_rope rp) {
+constexpr int QN_WAVES = 8;
+__global__ void __launch_bounds__(64 * QN_WAVES) k_gemv_qkv_norm(gemv_batch b, int K, gemv_rope rp) {
     const int g = blockIdx.x;
     int i = 0;
 #pragma unroll
@@ -387,7 +399,7 @@ __global__ void __launch_bounds__(256) k_gemv_qkv_norm(gemv_batch b, int K, gemv
         if (g >= b.it[j].first_group) i = j;
     const gemv_item &m = b.it[i];
     const int group = g - m.first_group;
-#define MI355_BODY(TY) gemv_body<TY, 1, 2, true, false, true, true>(m, group, nullptr, nullptr, K, &rp, s_act_dyn);
+#define MI355_BODY(TY) gemv_body<TY, 1, 2, true, false, true, true, QN_WAVES>(m, group, nullptr, nullptr, K, &rp, s_act_dyn);
     MI355_WEIGHT_TYPE_SWITCH(m.type, MI355_BODY)
 #undef MI355_BODY
 }
@@ -775,6 +787,7 @@ static int vec_q_rope_impl(void *stream, int n_mats, const mi355_gemv_rope_mat *
     b.n = n_mats;
     int64_t groups = 0;
     bool needs_pos = false, needs_cells = false, any_qc = false;
+    const int64_t group_rows = nx ? 2 * QN_WAVES : 8;
     for (int i = 0; i < n_mats; i++) any_qc = any_qc || mats[i].epilogue == MI355_EPI_ROPE_QCACHE || mats[i].epilogue == MI355_EPI_QCACHE;
     // groups of 32 rows (quantized-cache epilogues) first in the grid, then the groups of 8: pass 0 places the former
     for (int pass = 0; pass < 2; pass++) {
@@ -817,7 +830,7 @@ static int vec_q_rope_impl(void *stream, int n_mats, const mi355_gemv_rope_mat *
                           : m.epilogue == MI355_EPI_ROPE_QCACHE ? EPI_ROPE_QCACHE
                                                                : EPI_QCACHE;
             b.it[i].first_group = i < n_mats ? (int)groups : 0x7fffffff;
-            if (i < n_mats) groups += any_qc ? (qc ? m.N / 32 : (m.N + 15) / 16) : (m.N + 7) / 8;   // 8 waves x 4 or 2 rows; without quantized stores 4 waves x 2 rows
+            if (i < n_mats) groups += any_qc ? (qc ? m.N / 32 : (m.N + 15) / 16) : (m.N + group_rows - 1) / group_rows;   // 8 waves x 4 or 2 rows; without quantized stores 4 or 8 waves x 2 rows
         }
     }
     MI355_REQUIRE(!needs_pos || rope->pos != nullptr, "mul_mat_vec_q_rope: rope positions missing");
@@ -843,7 +856,7 @@ static int vec_q_rope_impl(void *stream, int n_mats, const mi355_gemv_rope_mat *
             MI355_LAUNCH(k_gemv_qkv_norm_qc, dim3((unsigned)groups), dim3(512), (size_t)K + K / 4, s, b, (int)K, rp);
             return launch_status("k_gemv_qkv_norm_qc");
         }
-        MI355_LAUNCH(k_gemv_qkv_norm, dim3((unsigned)groups), dim3(256), (size_t)K + K / 4, s, b, (int)K, rp);
+        MI355_LAUNCH(k_gemv_qkv_norm, dim3((unsigned)groups), dim3(64 * QN_WAVES), (size_t)K + K / 4, s, b, (int)K, rp);
         return launch_status("k_gemv_qkv_norm");
     }
     rp.nx = rp.nw = nullptr; rp.neps = 0.0f;

@@ -24,7 +24,22 @@ __global__ void __launch_bounds__(GF_WAVES * 64) k_gemv_f32(const uint8_t *__res
     const row_layout L = make_row_layout(TYPE, K);
     const int nchunks = K / T::CHUNK, nblk = K >> 5;
 
-    // the first step's weights are requested before anything waits
+    int8_t *s_q = (int8_t *)s_gf;
+    act_ds *s_ds = (act_ds *)(s_gf + NCOLS * K);
+    constexpr int STEP = GF_WAVES * 64 * 4, PIECES = 2;
+    f32x4 v[NCOLS][PIECES];   // 4096 elements of every row in flight
+    auto request = [&](int k0) {
+#pragma unroll
+        for (int col = 0; col < NCOLS; col++)
+#pragma unroll
+            for (int i = 0; i < PIECES; i++) {
+                const int k = k0 + i * STEP + (int)threadIdx.x * 4;
+                v[col][i] = *(const f32x4 *)(x + col * x_stride + (k < K ? k : K - 4));
+            }
+    };
+    // x first, the first step's weights behind it: a wave's loads return in the order of their issue, and the rows are quantized while the weights arrive
+    request(0);
+    __builtin_amdgcn_sched_barrier(0);
     const uint8_t *rows[RPW];
     typename T::chunk w_first[RPW];
 #pragma unroll
@@ -33,27 +48,19 @@ __global__ void __launch_bounds__(GF_WAVES * 64) k_gemv_f32(const uint8_t *__res
         rows[r] = W + row * L.row_bytes;
         w_first[r] = T::load_w(rows[r], L, lane < nchunks ? lane : nchunks - 1);
     }
-    int8_t *s_q = (int8_t *)s_gf;
-    act_ds *s_ds = (act_ds *)(s_gf + NCOLS * K);
-    constexpr int STEP = GF_WAVES * 64 * 4, PIECES = 2;
-    for (int k0 = 0; k0 < K; k0 += PIECES * STEP) {   // 4096 elements of every row in flight
-        f32x4 v[NCOLS][PIECES];
+    auto quantize = [&](int k0) {
 #pragma unroll
         for (int col = 0; col < NCOLS; col++)
 #pragma unroll
             for (int i = 0; i < PIECES; i++) {
-                const int k = k0 + i * STEP + (int)threadIdx.x * 4;
-                v[col][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (k < K) v[col][i] = *(const f32x4 *)(x + col * x_stride + k);
-            }
-#pragma unroll
-        for (int col = 0; col < NCOLS; col++)
-#pragma unroll
-            for (int i = 0; i < PIECES; i++) {
-                if (k0 + i * STEP >= K) continue;   // uniform
                 const int k = k0 + i * STEP + (int)threadIdx.x * 4;
                 quantize_block_lane(v[col][i], k < K, s_q, s_ds, col, K, k);
             }
+    };
+    quantize(0);
+    for (int k0 = PIECES * STEP; k0 < K; k0 += PIECES * STEP) {
+        request(k0);
+        quantize(k0);
     }
     __syncthreads();
     if (row0 >= N) return;   // whole wave

@@ -35,9 +35,9 @@ __device__ __forceinline__ void kv_block_offsets(const kv_place &p, int64_t g, i
 // own 32 values: the exchanges stay inside a half).  quantize_row_q8_0_ref (ggml/src/ggml-quants.c:194-218) bit for bit.
 __device__ __forceinline__ void kv_store_q8_0_lane32(float v, int j, uint8_t *__restrict__ y, int64_t lv, int64_t sc, bool live) {
     const float amax = lanes_max<32>(fabsf(v));
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    const int q = (int)roundf(v * id);
+    float d, id;
+    q8_scale(amax, d, id);
+    const int q = q8_level(v, id);
     if (!live) return;
     y[lv + j] = (uint8_t)(q & 0xFF);
     if (j == 0) *(unsigned short *)(y + sc) = float_to_half_bits(d);
@@ -75,9 +75,9 @@ __device__ __forceinline__ void kv_store_q4_0_lane32(float v, int j, uint8_t *__
 // 2 * l16 and 2 * l16 + 1 (the rotation pairs of the adjacent-pair rope mode).
 __device__ __forceinline__ void kv_store_q8_0_pair16(float y0, float y1, int l16, uint8_t *__restrict__ y, int64_t lv, int64_t sc) {
     const float amax = lanes_max<16>(fmaxf(fabsf(y0), fabsf(y1)));
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    const int q0 = (int)roundf(y0 * id), q1 = (int)roundf(y1 * id);
+    float d, id;
+    q8_scale(amax, d, id);
+    const int q0 = q8_level(y0, id), q1 = q8_level(y1, id);
     *(unsigned short *)(y + lv + 2 * l16) = (unsigned short)((q0 & 0xFF) | ((q1 & 0xFF) << 8));
     if (l16 == 0) *(unsigned short *)(y + sc) = float_to_half_bits(d);
 }

@@ -39,15 +39,15 @@ __global__ void __launch_bounds__(256) k_cpy_f32_q8_0(const float *__restrict__ 
     float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
 #pragma unroll
     for (int off = 4; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    float d, id;
+    q8_scale(amax, d, id);
     if (!live) return;
     int64_t lv, sc;
     kv_block_offsets<MI355_Q8_0>(pl, pl.first_block + kv_view_block(vw, e0), lv, sc);
     const int sub = (int)((e0 >> 2) & 7);
     int q[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) q[i] = (int)roundf(v[i] * id);
+    for (int i = 0; i < 4; i++) q[i] = q8_level(v[i], id);
     // plain 34-byte blocks are 2-byte aligned only
     unsigned short *o = (unsigned short *)(y + lv + 4 * sub);
     o[0] = (unsigned short)((q[0] & 0xFF) | ((q[1] & 0xFF) << 8));

@@ -14,13 +14,13 @@ namespace mi355 {
 __device__ __forceinline__ void quantize_block_lane(const f32x4 &v, bool live, int8_t *__restrict__ qplane, act_ds *__restrict__ ds,
                                                     int64_t row, int64_t k, int64_t e0) {
     const float amax = lanes_max<8>(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    float d, id;
+    q8_scale(amax, d, id);
     int q[4];
     int sum = 0;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        q[i] = (int)roundf(v[i] * id);
+        q[i] = q8_level(v[i], id);
         sum += q[i];
     }
     sum = lanes_sum_i<8>(sum);
@@ -41,9 +41,9 @@ __device__ __forceinline__ void quantize_block_lane(const f32x4 &v, bool live, i
 template <bool COH = false>
 __device__ __forceinline__ void quantize_lane32(float v, int8_t *__restrict__ qrow, act_ds *__restrict__ srow, int64_t e) {
     const float amax = lanes_max<32>(fabsf(v));
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    const int q = (int)roundf(v * id);
+    float d, id;
+    q8_scale(amax, d, id);
+    const int q = q8_level(v, id);
     const int sum = lanes_sum_i<32>(q);
     act_ds o;
     o.d = half_bits_to_float(float_to_half_bits(d));
@@ -64,6 +64,64 @@ __device__ __forceinline__ void quantize_lane32(float v, int8_t *__restrict__ qr
     }
 }
 
+// Sum of squares of the thread's pieces -> the row's 1 / rms in every thread.  The first 256 threads' sums count (sh: 4 floats of LDS; the caller places a barrier
+// between two calls that share it).  Contains exactly one group barrier, which further waves of a larger group must match with a barrier of their own.
+template <int NV>
+__device__ __forceinline__ float rms_norm_scale(const f32x4 (&v)[NV], int64_t k, float eps, float *sh) {
+    const int tid = threadIdx.x;
+    float ss = 0.0f;
+#pragma unroll
+    for (int it = 0; it < NV; it++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) ss = __builtin_fmaf(v[it][i], v[it][i], ss);
+    ss = wave_sum_dpp(ss);
+    if ((tid & 63) == 0 && tid < 256) sh[tid >> 6] = ss;
+    __syncthreads();
+    ss = add_rn(add_rn(add_rn(sh[0], sh[1]), sh[2]), sh[3]);
+    return 1.0f / sqrtf(add_rn(ss / (float)k, eps));
+}
+
+// RMS_NORM -> MUL -> Q8_1 of one row of at most 4096 elements (a multiple of 1024) into a group's LDS copy, in two parts: request() ahead of the group's first weight
+// loads - a wave's loads return in the order of their issue - and finish() behind them.  Same bits as rms_norm_quant_row: 256 threads' sums of squares of sixteen
+// elements each (further waves repeat the first four's, their sums are not used), then every thread quantizes its share.  WAVES: 4 or 8.
+template <int WAVES>
+struct norm_row {
+    static constexpr int NQ = 16 / WAVES;   // pieces the thread quantizes
+    f32x4 v[4], w[NQ];
+    static __device__ __forceinline__ int element(int it) { return (it * 256 + (int)(threadIdx.x & 255)) * 4; }
+    static __device__ __forceinline__ int first() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)) * NQ; }
+    __device__ __forceinline__ void request(const float *__restrict__ x, const float *__restrict__ nw, int K) {
+        // pieces past the end repeat others, and nothing uses them: a branch around a load would let the compiler move it to where its value is needed
+#pragma unroll
+        for (int it = 0; it < 4; it++) v[it] = *(const f32x4 *)(x + (element(it) < K ? element(it) : element(0)));
+#pragma unroll
+        for (int j = 0; j < NQ; j++) {
+            const int e = element(first() + j);
+            w[j] = *(const f32x4 *)(nw + (e < K ? e : element(0)));
+        }
+    }
+    __device__ __forceinline__ void finish(uint8_t *s_act, int K, float eps, float *sh) {
+#pragma unroll
+        for (int it = 1; it < 4; it++)
+            if (it * 1024 >= K) v[it] = f32x4{0.f, 0.f, 0.f, 0.f};   // uniform
+        const float scale = rms_norm_scale<4>(v, K, eps, sh);
+        int8_t *qplane = (int8_t *)s_act;
+#pragma unroll
+        for (int j = 0; j < NQ; j++) {
+            const int it = first() + j;
+            if (it * 1024 >= K) break;   // uniform
+            f32x4 o;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float xv = first() ? v[(NQ & 3) + j][i] : v[j][i];   // four waves: always the thread's piece j
+                o[i] = xv * scale;
+                o[i] = o[i] * w[j][i];
+            }
+            quantize_block_lane(o, true, qplane, (act_ds *)(qplane + K), 0, K, element(it));
+        }
+    }
+};
+
 // One row: xr -> y row (optional) and row `row` of the activation workspace `act` (optional), which holds nrows rows of k.
 // Each thread keeps its NV float4 of the row in registers (k <= 1024 * NV).  COH: the row was written by other groups of the
 // same launch with device-scope stores and is read with device-scope loads.  sh: 4 floats of LDS; the caller places a
@@ -71,9 +129,9 @@ __device__ __forceinline__ void quantize_lane32(float v, int8_t *__restrict__ qr
 // FMT: activation format written to `act`: 0 Q8_1 (split layout), 1 per-super-block (q8k.hpp), 2 the same as tile images (tiles.hpp)
 // Called by the first 256 threads of a group; contains exactly one group barrier, which further waves of a larger group must
 // match with a barrier of their own.
-template <int NV, int FMT, bool COH>
 // keep: where the caller wants the thread's NV pieces of the normalised row (registers), or null
 // given: the thread's NV pieces of the row when the caller has just formed them (xr is not read then), or null
+template <int NV, int FMT, bool COH>
 __device__ __forceinline__ void rms_norm_quant_row(const float *__restrict__ xr, const float *__restrict__ w, float *__restrict__ yr,
                                                    void *__restrict__ act, int64_t row, int64_t k, int64_t nrows, float eps, float *sh,
                                                    f32x4 *keep = nullptr, const f32x4 *given = nullptr) {
@@ -97,16 +155,7 @@ __device__ __forceinline__ void rms_norm_quant_row(const float *__restrict__ xr,
             if (w) ww[it] = *(const f32x4 *)(w + e0);
         }
     }
-    float ss = 0.0f;
-#pragma unroll
-    for (int it = 0; it < NV; it++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) ss = __builtin_fmaf(v[it][i], v[it][i], ss);
-    ss = wave_sum_dpp(ss);
-    if ((tid & 63) == 0) sh[tid >> 6] = ss;
-    __syncthreads();
-    ss = add_rn(add_rn(add_rn(sh[0], sh[1]), sh[2]), sh[3]);
-    const float scale = 1.0f / sqrtf(add_rn(ss / (float)k, eps));
+    const float scale = rms_norm_scale<NV>(v, k, eps, sh);
     int8_t *qplane = (int8_t *)act;
     act_ds *ds = (act_ds *)(qplane + nrows * k);
 #pragma unroll

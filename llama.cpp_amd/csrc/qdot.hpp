@@ -484,6 +484,47 @@ template <> struct wq<MI355_Q6_K> {
     }
 };
 
+// The group's copy of a quantized activation (NCOLS rows of K levels, then their {d, sum} pairs) in LDS: request() before the first weight
+// loads, commit() behind them.  A wave's loads return in the order they were issued, so a copy requested behind the weights waits for all of
+// them, and no dot product starts before the last weight has arrived.
+template <int NCOLS, int THREADS>
+struct act_copy {
+    // pieces per thread requested up front (rows of 4096; longer ones take the rest behind the weights)
+    static constexpr int NQ = (NCOLS * 4096 / 16 + THREADS - 1) / THREADS, ND = (NCOLS * 4096 / 32 + THREADS - 1) / THREADS;
+    u32x4 q[NQ];
+    u32x2 d[ND];
+    __device__ __forceinline__ void request(const int8_t *aq, const act_ds *ads, int K) {
+        const int nq = NCOLS * (K >> 4), nd = NCOLS * (K >> 5);
+#pragma unroll
+        for (int p = 0; p < NQ; p++) {
+            const int i = (int)threadIdx.x + p * THREADS;
+            q[p] = load16(aq + (int64_t)(i < nq ? i : nq - 1) * 16);
+        }
+#pragma unroll
+        for (int p = 0; p < ND; p++) {
+            const int i = (int)threadIdx.x + p * THREADS;
+            d[p] = *(const u32x2 *)(ads + (i < nd ? i : nd - 1));
+        }
+    }
+    __device__ __forceinline__ void commit(uint8_t *s_act, const int8_t *aq, const act_ds *ads, int K) {
+        const int nq = NCOLS * (K >> 4), nd = NCOLS * (K >> 5);
+        uint8_t *s_ds = s_act + NCOLS * K;
+        // pieces past the end are the last one again, stored again: with a branch around the store the compiler moves the load into it
+#pragma unroll
+        for (int p = 0; p < NQ; p++) {
+            const int i = (int)threadIdx.x + p * THREADS;
+            *(u32x4 *)(s_act + (i < nq ? i : nq - 1) * 16) = q[p];
+        }
+#pragma unroll
+        for (int p = 0; p < ND; p++) {
+            const int i = (int)threadIdx.x + p * THREADS;
+            *(u32x2 *)(s_ds + (i < nd ? i : nd - 1) * 8) = d[p];
+        }
+        for (int i = (int)threadIdx.x + NQ * THREADS; i < nq; i += THREADS) *(u32x4 *)(s_act + i * 16) = load16(aq + (int64_t)i * 16);
+        for (int i = (int)threadIdx.x + ND * THREADS; i < nd; i += THREADS) *(u32x2 *)(s_ds + i * 8) = *(const u32x2 *)(ads + i);
+    }
+};
+
 // ---------------------------------------------------------------- scalar element access
 // Dequantized weight element e of a row stored in device layout.  Byte loads only, so it
 // works for rows at any address.  Semantics: dequantize_row_* of ggml/src/ggml-quants.c:255-347, 349-363,

@@ -25,8 +25,8 @@ void set_error(const char *fmt, ...) {
 // quantize_row_q8_1_ref, ggml/src/ggml-quants.c:220-253, bit for bit:
 //   d = amax / 127 ; id = d ? 1/d : 0 ; q = roundf(x * id) ; y.d = fp16(d) ; y.s = fp16(sum(q) * d)
 // Eight lanes share one 32-element block (one float4 each); a 256-thread group covers
-// 1024 consecutive elements of one row.  Division and roundf are the IEEE-correct ones
-// (no fast-math), so the levels agree with the host for every input.
+// 1024 consecutive elements of one row.  The quotients and the rounding are those of IEEE division and roundf (q8_scale,
+// q8_level), so the levels agree with the host for every input.
 //
 // STD = true : writes block_q8_1 (36 B: fp16 d, fp16 s, 32 x int8)
 // STD = false: writes the split layout of mi355_quantize_act (int8 plane + {float d; int sum})
@@ -42,13 +42,13 @@ __global__ void __launch_bounds__(256) k_quantize_q8_1(const float *__restrict__
 
     const float amax = lanes_max<8>(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
 
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    float d, id;
+    q8_scale(amax, d, id);
     int q[4];
     int sum = 0;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        q[i] = (int)roundf(v[i] * id);
+        q[i] = q8_level(v[i], id);
         sum += q[i];
     }
     sum = lanes_sum_i<8>(sum);

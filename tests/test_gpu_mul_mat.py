@@ -45,6 +45,22 @@ def test_quantize_q8_1_bit_exact(dev, K, dist):
         assert np.array_equal(got, orc.quantize("ref", orc.Q8_1, x))
 
 
+@pytest.mark.parametrize("seed", [0, 1])
+def test_quantize_q8_1_every_scale(dev, seed):
+    """block maxima of every magnitude whose reciprocal scale is finite: the quotients by correction step agree with IEEE division on both sides of the range (2^-90 .. 2^90)
+    they are used in, and levels that land on halves round away from zero"""
+    import mi355
+    rng = np.random.default_rng(seed)
+    amax = np.ldexp(rng.uniform(1, 2, (64, 246)), np.arange(-118, 128)).astype(np.float32)      # one per block
+    x = (rng.uniform(-1, 1, (64, 246, 32)) * amax[..., None]).astype(np.float32)
+    ties = (rng.integers(-127, 127, (64, 246, 32)) + 0.5).astype(np.float32) * (amax / np.float32(127))[..., None]
+    x = np.where(rng.random(x.shape) < 0.5, x, ties)
+    x[..., 7] = np.where(rng.random(amax.shape) < 0.5, amax, -amax)
+    x = np.clip(x, -amax[..., None], amax[..., None]).reshape(64, 246 * 32)
+    got = mi355.quantize_q8_1(_to_dev(dev, x)).cpu().numpy()
+    assert np.array_equal(got, orc.quantize("oracle", orc.Q8_1, x))
+
+
 @pytest.mark.parametrize("name,t", TYPES)
 @pytest.mark.parametrize("K", [256, 2048, 4096])
 def test_weight_layout_round_trip(dev, name, t, K):
