@@ -24,7 +24,7 @@ KERNEL_SOURCES = ["quantize.hip", "wquant.hip", "gemv.hip", "gemv_f32.hip", "ffn
 
 # -packed-fp32-ops: keep hipcc from forming packed-FP32 instructions out of scalar float code
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
-               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 
 def _hipcc():
