@@ -558,6 +558,12 @@ int mi355_rms_norm_qkv_rope_store(void *stream, const float *x, const float *nor
                                   size_t k_nb2, size_t v_nb1, size_t v_nb2, int n_dims, int mode, int n_ctx_orig, float freq_base,
                                   float freq_scale, float ext_factor, float attn_factor, float beta_fast, float beta_slow);
 
+/* The same with the rotations read from a table: {cos, sin} per pair of the token's position, D / 2 float pairs written by mi355_rope_table once per token - they
+ * do not depend on the layer, and working them out takes every wave of every layer's launch several hundred instructions.  Same bits.  8-byte aligned. */
+int mi355_rms_norm_qkv_rope_table_store(void *stream, const float *x, const float *norm_w, float eps, int type_q, const void *wq, int type_k, const void *wk,
+                                        int type_v, const void *wv, float *q, void *kcache, void *vcache, const void *table, const int32_t *cells, int64_t K,
+                                        int64_t H, int64_t HK, int64_t D, size_t k_nb1, size_t k_nb2, size_t v_nb1, size_t v_nb2, int n_dims);
+
 /* The gate and up projections of llm_build_ffn (LLM_FFN_SILU, LLM_FFN_PAR; src/llama.cpp:280-320) in ONE bandwidth-bound launch that
  * also performs UNARY(SILU)(gate), MUL by up and the Q8_1 quantization the ffn_down product needs (ggml-cpu.c:6646-6683, 5142-5211;
  * quantize_row_q8_1_ref).  gate/up: f32 [B][out_stride] receive the raw products; act_out: mi355_quantize_act layout of B rows of N.

@@ -28,6 +28,17 @@ __global__ void __launch_bounds__(256) k_rms_norm_mul_quant(const float *__restr
     rms_norm_quant_row<NV, FMT, false>(x + row * x_stride, w, y ? y + row * y_stride : nullptr, act, row, k, nrows, eps, sh);
 }
 
+// One 1024-thread group per row, up to 256 rows (one group per compute unit).  us, 256 threads / 1024: one row of 4096 2.96 / 2.43, 256 rows 3.46 / 3.13,
+// one of 8192 4.53 / 3.32; one row of 4096 to a Q8_K image 4.27 / 3.22
+template <int NV, int FMT>
+__global__ void __launch_bounds__(1024) k_rms_norm_mul_quant_wide(const float *__restrict__ x, int64_t x_stride, const float *__restrict__ w,
+                                                                  float *__restrict__ y, int64_t y_stride, void *__restrict__ act, int64_t k,
+                                                                  int64_t nrows, float eps) {
+    __shared__ float sh[4];
+    const int64_t row = blockIdx.x;
+    rms_norm_quant_row_wide<NV, FMT>(x + row * x_stride, w, y ? y + row * y_stride : nullptr, act, row, k, nrows, eps, sh);
+}
+
 // The FFN norm of a mixture-of-experts layer for a few tokens, continued with the router (llm_build_moe_ffn, src/llama.cpp:438-468):
 // logits[e] = W[e] . y for the row y the group has just normalised, then soft-max and the descending order.  A thread's pieces of y
 // are the pieces k_mul_mat_f (glue.hip) gives thread t of its 256-thread group - elements 4 t + 1024 i - and the sums are formed in
@@ -255,6 +266,8 @@ using namespace mi355;
 
 extern "C" {
 
+constexpr int64_t NORM_FEW_ROWS = 256;   // k_rms_norm_mul_quant_wide
+
 static int rms_norm_mul_quant(void *stream, const float *x, int64_t x_stride, const float *w, float *y, int64_t y_stride, void *act, int64_t k,
                               int64_t nrows, float eps, int fmt) {
     const bool q8k = fmt != 0;
@@ -266,17 +279,24 @@ static int rms_norm_mul_quant(void *stream, const float *x, int64_t x_stride, co
     MI355_REQUIRE(y != nullptr || act != nullptr, "rms_norm_mul_quant: no output requested");
     if (nrows == 0) return MI355_OK;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid((unsigned)nrows), block(256);
-#define MI355_LAUNCH_NORM(NV)                                                                                                        \
-    do {                                                                                                                              \
-        if (fmt == 2) MI355_LAUNCH((k_rms_norm_mul_quant<NV, 2>), grid, block, 0, s, x, x_stride, w, y, y_stride, act, k, nrows, eps);  \
-        else if (fmt == 1) MI355_LAUNCH((k_rms_norm_mul_quant<NV, 1>), grid, block, 0, s, x, x_stride, w, y, y_stride, act, k, nrows, eps);  \
-        else MI355_LAUNCH((k_rms_norm_mul_quant<NV, 0>), grid, block, 0, s, x, x_stride, w, y, y_stride, act, k, nrows, eps);     \
+    const bool wide = nrows <= NORM_FEW_ROWS;
+    const dim3 grid((unsigned)nrows), block(wide ? 1024 : 256);
+#define MI355_LAUNCH_NORM_FMT(KERNEL, NV)                                                                                         \
+    do {                                                                                                                          \
+        if (fmt == 2) MI355_LAUNCH((KERNEL<NV, 2>), grid, block, 0, s, x, x_stride, w, y, y_stride, act, k, nrows, eps);            \
+        else if (fmt == 1) MI355_LAUNCH((KERNEL<NV, 1>), grid, block, 0, s, x, x_stride, w, y, y_stride, act, k, nrows, eps);       \
+        else MI355_LAUNCH((KERNEL<NV, 0>), grid, block, 0, s, x, x_stride, w, y, y_stride, act, k, nrows, eps);                     \
+    } while (0)
+#define MI355_LAUNCH_NORM(NV)                                            \
+    do {                                                                 \
+        if (wide) MI355_LAUNCH_NORM_FMT(k_rms_norm_mul_quant_wide, NV);  \
+        else MI355_LAUNCH_NORM_FMT(k_rms_norm_mul_quant, NV);            \
     } while (0)
     if (k <= 4096) MI355_LAUNCH_NORM(4);
     else if (k <= 8192) MI355_LAUNCH_NORM(8);
     else MI355_LAUNCH_NORM(16);
 #undef MI355_LAUNCH_NORM
+#undef MI355_LAUNCH_NORM_FMT
     return launch_status("k_rms_norm_mul_quant");
 }
 

@@ -1,0 +1,264 @@
+// The Q/K/V launches of one to four tokens: the three projections, ROPE and the stores to the KV cache, with the attention norm of a single token where asked for
+// (gemv_body.hpp has the rows).
+#include "gemv_body.hpp"
+
+#include <math.h>
+
+namespace mi355 {
+
+// Q, K and V projections in one launch; finished rows are rotated and land in q (f32) or in the f16 KV cache
+template <int NCOLS, bool LDSA>
+__global__ void __launch_bounds__(256) k_gemv_qkv(gemv_batch b, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, int K, gemv_rope rp) {
+    const int g = blockIdx.x;
+    int i = 0;
+#pragma unroll
+    for (int j = 1; j < 3; j++)
+        if (g >= b.it[j].first_group) i = j;   // unused items start at INT_MAX
+    const gemv_item &m = b.it[i];
+    const int group = g - m.first_group;
+#define MI355_BODY(TY) gemv_body<TY, NCOLS, 2, true, false, LDSA>(m, group, aq, ads, K, &rp, s_act_dyn);
+    MI355_WEIGHT_TYPE_SWITCH(m.type, MI355_BODY)   // uniform over the group
+#undef MI355_BODY
+}
+
+// ... with the RMS norm of the layer input computed by every group for itself (one activation row).  Eight waves: half the groups that do so of four (8B shapes: a token
+// 1821 us with four, 1819 with eight).
+constexpr int QN_WAVES = 8;
+__global__ void __launch_bounds__(64 * QN_WAVES) k_gemv_qkv_norm(gemv_batch b, int K, gemv_rope rp) {
+    const int g = blockIdx.x;
+    int i = 0;
+#pragma unroll
+    for (int j = 1; j < 3; j++)
+        if (g >= b.it[j].first_group) i = j;
+    const gemv_item &m = b.it[i];
+    const int group = g - m.first_group;
+#define MI355_BODY(TY) gemv_body<TY, 1, 2, true, false, true, true, QN_WAVES>(m, group, nullptr, nullptr, K, &rp, s_act_dyn);
+    MI355_WEIGHT_TYPE_SWITCH(m.type, MI355_BODY)
+#undef MI355_BODY
+}
+
+// The same two launches with K and / or V going to a Q8_0 / Q4_0 cache (gemv_body_qc): 512 threads per group; the matrices with a
+// quantized destination have groups of 32 rows, one cache block per group, the others groups of 16.  The host lists the groups
+// of 32 rows first in the grid.
+__device__ __forceinline__ int qkv_item_of(const gemv_batch &b, int g) {
+    int i = 0, best = -1;
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+        if (g >= b.it[j].first_group && b.it[j].first_group > best) {   // unused items start at INT_MAX
+            i = j;
+            best = b.it[j].first_group;
+        }
+    return i;
+}
+
+template <int NCOLS>
+__global__ void __launch_bounds__(512, (NCOLS == 1 ? 4 : 2)) k_gemv_qkv_qc(gemv_batch b, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, int K, gemv_rope rp) {
+    const gemv_item &m = b.it[qkv_item_of(b, blockIdx.x)];
+    const int group = blockIdx.x - m.first_group;
+    if (m.epi >= EPI_ROPE_QCACHE) {   // uniform over the group
+#define MI355_BODY(TY) gemv_body_qc<TY, NCOLS, false, true>(m, group, aq, ads, K, rp, nullptr);
+        MI355_WEIGHT_TYPE_SWITCH(m.type, MI355_BODY)
+#undef MI355_BODY
+    } else {
+#define MI355_BODY(TY) gemv_body_qc<TY, NCOLS, false, false>(m, group, aq, ads, K, rp, nullptr);
+        MI355_WEIGHT_TYPE_SWITCH(m.type, MI355_BODY)
+#undef MI355_BODY
+    }
+}
+
+__global__ void __launch_bounds__(512, 4) k_gemv_qkv_norm_qc(gemv_batch b, int K, gemv_rope rp) {
+    const gemv_item &m = b.it[qkv_item_of(b, blockIdx.x)];
+    const int group = blockIdx.x - m.first_group;
+    if (m.epi >= EPI_ROPE_QCACHE) {
+#define MI355_BODY(TY) gemv_body_qc<TY, 1, true, true>(m, group, nullptr, nullptr, K, rp, s_act_dyn);
+        MI355_WEIGHT_TYPE_SWITCH(m.type, MI355_BODY)
+#undef MI355_BODY
+    } else {
+#define MI355_BODY(TY) gemv_body_qc<TY, 1, true, false>(m, group, nullptr, nullptr, K, rp, s_act_dyn);
+        MI355_WEIGHT_TYPE_SWITCH(m.type, MI355_BODY)
+#undef MI355_BODY
+    }
+}
+
+}  // namespace mi355
+
+using namespace mi355;
+
+extern "C" {
+
+// nx != null: one activation row that every group normalises and quantizes for itself (act is not read)
+static int vec_q_rope_impl(void *stream, int n_mats, const mi355_gemv_rope_mat *mats, const void *act, int64_t K, int64_t B,
+                             const mi355_rope_desc *rope, const float *nx, const float *nw, float neps, const void *table = nullptr) {
+    MI355_REQUIRE(n_mats >= 1 && n_mats <= 3 && mats != nullptr && rope != nullptr, "mul_mat_vec_q_rope: 1..3 matrices per launch");
+    MI355_REQUIRE(B >= 1 && B <= 4, "mul_mat_vec_q_rope: batch %lld outside 1..4", (long long)B);
+    const int64_t D = rope->head_dim;
+    const int n_dims = rope->n_dims;
+    MI355_REQUIRE(D > 0 && D % 2 == 0 && n_dims > 0 && n_dims <= D && n_dims % 2 == 0, "mul_mat_vec_q_rope: bad head geometry");
+    MI355_REQUIRE(rope->mode == 0, "mul_mat_vec_q_rope: only the adjacent-pair rope mode is fused (mode %d)", rope->mode);
+    MI355_REQUIRE(nx != nullptr || ((uintptr_t)act & 15) == 0, "mul_mat_vec_q_rope: activation workspace is not 16-byte aligned");
+    MI355_REQUIRE(nx == nullptr || (B == 1 && K <= 4096 && K % 1024 == 0 && ((uintptr_t)nx & 15) == 0 && ((uintptr_t)nw & 15) == 0),
+                  "rms_norm_qkv_rope_store: one row of K <= 4096 (a multiple of 1024), 16-byte aligned x and weights");
+    gemv_batch b;
+    b.n = n_mats;
+    int64_t groups = 0;
+    bool needs_pos = false, needs_cells = false, any_qc = false;
+    const int64_t group_rows = nx ? 2 * QN_WAVES : 8;
+    for (int i = 0; i < n_mats; i++) any_qc = any_qc || mats[i].epilogue == MI355_EPI_ROPE_QCACHE || mats[i].epilogue == MI355_EPI_QCACHE;
+    // groups of 32 rows (quantized-cache epilogues) first in the grid, then the groups of 8: pass 0 places the former
+    for (int pass = 0; pass < 2; pass++) {
+        for (int i = 0; i < 4; i++) {
+            const mi355_gemv_rope_mat &m = mats[i < n_mats ? i : 0];
+            const bool qc = m.epilogue == MI355_EPI_ROPE_QCACHE || m.epilogue == MI355_EPI_QCACHE;
+            if (i < n_mats && qc != (pass == 0)) continue;
+            if (i >= n_mats && pass == 0) continue;
+            if (i < n_mats) {
+                int rc = check_gemv_args("mul_mat_vec_q_rope", m.type, m.W, m.N, K, m.N);
+                if (rc != MI355_OK) return rc;
+                MI355_REQUIRE(m.epilogue >= MI355_EPI_STORE && m.epilogue <= MI355_EPI_QCACHE && m.dst != nullptr && m.N % 2 == 0,
+                              "mul_mat_vec_q_rope: bad epilogue %d, missing destination or odd row count", m.epilogue);
+                if (m.epilogue == MI355_EPI_STORE || m.epilogue == MI355_EPI_ROPE)
+                    MI355_REQUIRE(m.dst_stride >= m.N, "mul_mat_vec_q_rope: dst_stride < N");
+                else if (qc)
+                    MI355_REQUIRE(((uintptr_t)m.dst & 1) == 0 && (m.dst_stride == MI355_Q8_0 || m.dst_stride == MI355_Q4_0) && m.nb1 >= 0 && m.nb2 >= 0 &&
+                                      m.N % 32 == 0,
+                                  "mul_mat_vec_q_rope: a quantized cache takes whole Q8_0 / Q4_0 blocks (N a multiple of 32)");
+                else
+                    MI355_REQUIRE(((uintptr_t)m.dst & 1) == 0 && m.nb1 % 2 == 0 && m.nb2 % 2 == 0, "mul_mat_vec_q_rope: misaligned f16 destination");
+                if (m.epilogue != MI355_EPI_STORE) MI355_REQUIRE(m.N % D == 0, "mul_mat_vec_q_rope: N=%lld is not a whole number of heads", (long long)m.N);
+                needs_pos = needs_pos || m.epilogue == MI355_EPI_ROPE || m.epilogue == MI355_EPI_ROPE_CACHE || m.epilogue == MI355_EPI_ROPE_QCACHE;
+                needs_cells = needs_cells || m.epilogue == MI355_EPI_ROPE_CACHE || m.epilogue == MI355_EPI_CACHE || qc;
+            }
+            b.it[i].W = (const uint8_t *)m.W;
+            b.it[i].residual = nullptr;
+            b.it[i].N = m.N;
+            b.it[i].type = m.type;
+            b.it[i].dst = (float *)m.dst;
+            b.it[i].dst_stride = m.dst_stride;
+            b.it[i].nb1 = m.nb1;
+            b.it[i].nb2 = m.nb2;
+            b.it[i].ctype = qc ? (int)m.dst_stride : 0;
+            // the kernel's epilogue codes: plain rows take the rope path with no rotation applied to them
+            b.it[i].epi = m.epilogue == MI355_EPI_STORE        ? EPI_STORE
+                          : m.epilogue == MI355_EPI_ROPE       ? EPI_ROPE
+                          : m.epilogue == MI355_EPI_ROPE_CACHE ? EPI_ROPE_CACHE
+                          : m.epilogue == MI355_EPI_CACHE      ? EPI_CACHE
+                          : m.epilogue == MI355_EPI_ROPE_QCACHE ? EPI_ROPE_QCACHE
+                                                               : EPI_QCACHE;
+            b.it[i].first_group = i < n_mats ? (int)groups : 0x7fffffff;
+            if (i < n_mats) groups += any_qc ? (qc ? m.N / 32 : (m.N + 15) / 16) : (m.N + group_rows - 1) / group_rows;   // 8 waves x 4 or 2 rows; without quantized stores 4 or 8 waves x 2 rows
+        }
+    }
+    MI355_REQUIRE(!needs_pos || rope->pos != nullptr || table != nullptr, "mul_mat_vec_q_rope: rope positions missing");
+    MI355_REQUIRE(!needs_cells || rope->cells != nullptr, "mul_mat_vec_q_rope: cache cells missing");
+    MI355_REQUIRE(groups < 0x7fffffff, "mul_mat_vec_q_rope: too many rows for one launch");
+    gemv_rope rp;
+    rp.pos = needs_pos ? rope->pos : nullptr; rp.cells = needs_cells ? rope->cells : nullptr; rp.ff = rope->freq_factors;
+    rp.D = (int)D; rp.n_dims = n_dims;
+    rp.table = (const float2 *)table;
+    rp.theta_scale = rp.freq_scale = rp.ext_factor = rp.attn_factor = rp.corr0 = rp.corr1 = 0.0f;
+    if (!table) {
+        rp.theta_scale = powf(rope->freq_base, -2.0f / n_dims);
+        rp.freq_scale = rope->freq_scale; rp.ext_factor = rope->ext_factor; rp.attn_factor = rope->attn_factor;
+        const float pi = 3.14159265358979323846f;   // ggml_rope_yarn_corr_dims, ggml/src/ggml.c:3695-3707
+        const float c0 = floorf(n_dims * logf(rope->n_ctx_orig / (rope->beta_fast * 2 * pi)) / (2 * logf(rope->freq_base)));
+        const float c1 = ceilf(n_dims * logf(rope->n_ctx_orig / (rope->beta_slow * 2 * pi)) / (2 * logf(rope->freq_base)));
+        rp.corr0 = c0 > 0 ? c0 : 0;
+        rp.corr1 = c1 < n_dims - 1 ? c1 : (float)(n_dims - 1);
+    }
+    hipStream_t s = (hipStream_t)stream;
+    const int8_t *aq = (const int8_t *)act;
+    const act_ds *ads = (const act_ds *)(aq + B * K);
+    const size_t lds = act_lds_bytes((int)B, K, groups);
+    if (nx != nullptr) {
+        rp.nx = nx; rp.nw = nw; rp.neps = neps;
+        if (any_qc) {
+            MI355_LAUNCH(k_gemv_qkv_norm_qc, dim3((unsigned)groups), dim3(512), (size_t)K + K / 4, s, b, (int)K, rp);
+            return launch_status("k_gemv_qkv_norm_qc");
+        }
+        MI355_LAUNCH(k_gemv_qkv_norm, dim3((unsigned)groups), dim3(64 * QN_WAVES), (size_t)K + K / 4, s, b, (int)K, rp);
+        return launch_status("k_gemv_qkv_norm");
+    }
+    rp.nx = rp.nw = nullptr; rp.neps = 0.0f;
+    if (any_qc) {   // every wave reads the activation from memory (L2): these launches have too few groups for the copy in LDS to pay
+        switch (B) {
+            case 1: MI355_LAUNCH((k_gemv_qkv_qc<1>), dim3((unsigned)groups), dim3(512), 0, s, b, aq, ads, (int)K, rp); break;
+            case 2: MI355_LAUNCH((k_gemv_qkv_qc<2>), dim3((unsigned)groups), dim3(512), 0, s, b, aq, ads, (int)K, rp); break;
+            case 3: MI355_LAUNCH((k_gemv_qkv_qc<3>), dim3((unsigned)groups), dim3(512), 0, s, b, aq, ads, (int)K, rp); break;
+            default: MI355_LAUNCH((k_gemv_qkv_qc<4>), dim3((unsigned)groups), dim3(512), 0, s, b, aq, ads, (int)K, rp); break;
+        }
+        return launch_status("k_gemv_qkv_qc");
+    }
+    switch (B) {
+        case 1:
+            if (lds) MI355_LAUNCH((k_gemv_qkv<1, true>), dim3((unsigned)groups), dim3(256), lds, s, b, aq, ads, (int)K, rp);
+            else MI355_LAUNCH((k_gemv_qkv<1, false>), dim3((unsigned)groups), dim3(256), 0, s, b, aq, ads, (int)K, rp);
+            break;
+        case 2:
+            if (lds) MI355_LAUNCH((k_gemv_qkv<2, true>), dim3((unsigned)groups), dim3(256), lds, s, b, aq, ads, (int)K, rp);
+            else MI355_LAUNCH((k_gemv_qkv<2, false>), dim3((unsigned)groups), dim3(256), 0, s, b, aq, ads, (int)K, rp);
+            break;
+        case 3:
+            if (lds) MI355_LAUNCH((k_gemv_qkv<3, true>), dim3((unsigned)groups), dim3(256), lds, s, b, aq, ads, (int)K, rp);
+            else MI355_LAUNCH((k_gemv_qkv<3, false>), dim3((unsigned)groups), dim3(256), 0, s, b, aq, ads, (int)K, rp);
+            break;
+        default:
+            if (lds) MI355_LAUNCH((k_gemv_qkv<4, true>), dim3((unsigned)groups), dim3(256), lds, s, b, aq, ads, (int)K, rp);
+            else MI355_LAUNCH((k_gemv_qkv<4, false>), dim3((unsigned)groups), dim3(256), 0, s, b, aq, ads, (int)K, rp);
+            break;
+    }
+    return launch_status("k_gemv_qkv");
+}
+
+int mi355_mul_mat_vec_q_rope(void *stream, int n_mats, const mi355_gemv_rope_mat *mats, const void *act, int64_t K, int64_t B,
+                             const mi355_rope_desc *rope) {
+    return vec_q_rope_impl(stream, n_mats, mats, act, K, B, rope, nullptr, nullptr, 0.0f);
+}
+
+int mi355_rms_norm_mul_mat_vec_q_rope(void *stream, const float *x, const float *norm_w, float eps, int n_mats, const mi355_gemv_rope_mat *mats,
+                                      int64_t K, const mi355_rope_desc *rope) {
+    MI355_REQUIRE(x != nullptr && norm_w != nullptr, "rms_norm_mul_mat_vec_q_rope: missing operands");
+    return vec_q_rope_impl(stream, n_mats, mats, nullptr, K, 1, rope, x, norm_w, eps);
+}
+
+int mi355_rms_norm_qkv_rope_store(void *stream, const float *x, const float *norm_w, float eps, int type_q, const void *wq, int type_k,
+                                  const void *wk, int type_v, const void *wv, float *q, void *kcache, void *vcache, const int32_t *pos,
+                                  const int32_t *cells, const float *freq_factors, int64_t K, int64_t H, int64_t HK, int64_t D, size_t k_nb1,
+                                  size_t k_nb2, size_t v_nb1, size_t v_nb2, int n_dims, int mode, int n_ctx_orig, float freq_base,
+                                  float freq_scale, float ext_factor, float attn_factor, float beta_fast, float beta_slow) {
+    MI355_REQUIRE(H > 0 && HK > 0 && D > 0 && x != nullptr && norm_w != nullptr, "rms_norm_qkv_rope_store: bad head geometry or missing operands");
+    mi355_gemv_rope_mat m[3];
+    m[0] = mi355_gemv_rope_mat{type_q, wq, H * D, MI355_EPI_ROPE, q, H * D, 0, 0};
+    m[1] = mi355_gemv_rope_mat{type_k, wk, HK * D, MI355_EPI_ROPE_CACHE, kcache, 0, (int64_t)k_nb1, (int64_t)k_nb2};
+    m[2] = mi355_gemv_rope_mat{type_v, wv, HK * D, MI355_EPI_CACHE, vcache, 0, (int64_t)v_nb1, (int64_t)v_nb2};
+    mi355_rope_desc r = {pos, cells, freq_factors, D, n_dims, mode, n_ctx_orig, freq_base, freq_scale, ext_factor, attn_factor, beta_fast, beta_slow};
+    return vec_q_rope_impl(stream, 3, m, nullptr, K, 1, &r, x, norm_w, eps);
+}
+
+int mi355_rms_norm_qkv_rope_table_store(void *stream, const float *x, const float *norm_w, float eps, int type_q, const void *wq, int type_k, const void *wk,
+                                        int type_v, const void *wv, float *q, void *kcache, void *vcache, const void *table, const int32_t *cells, int64_t K,
+                                        int64_t H, int64_t HK, int64_t D, size_t k_nb1, size_t k_nb2, size_t v_nb1, size_t v_nb2, int n_dims) {
+    MI355_REQUIRE(H > 0 && HK > 0 && D > 0 && x != nullptr && norm_w != nullptr, "rms_norm_qkv_rope_table_store: bad head geometry or missing operands");
+    MI355_REQUIRE(table != nullptr && ((uintptr_t)table & 7) == 0, "rms_norm_qkv_rope_table_store: the table is missing or not 8-byte aligned");
+    mi355_gemv_rope_mat m[3];
+    m[0] = mi355_gemv_rope_mat{type_q, wq, H * D, MI355_EPI_ROPE, q, H * D, 0, 0};
+    m[1] = mi355_gemv_rope_mat{type_k, wk, HK * D, MI355_EPI_ROPE_CACHE, kcache, 0, (int64_t)k_nb1, (int64_t)k_nb2};
+    m[2] = mi355_gemv_rope_mat{type_v, wv, HK * D, MI355_EPI_CACHE, vcache, 0, (int64_t)v_nb1, (int64_t)v_nb2};
+    mi355_rope_desc r = {nullptr, cells, nullptr, D, n_dims, 0, 0, 1.0f, 1.0f, 0.0f, 1.0f, 1.0f, 1.0f};
+    return vec_q_rope_impl(stream, 3, m, nullptr, K, 1, &r, x, norm_w, eps, table);
+}
+
+int mi355_qkv_rope_store(void *stream, int type_q, const void *wq, int type_k, const void *wk, int type_v, const void *wv, const void *act,
+                         float *q, void *kcache, void *vcache, const int32_t *pos, const int32_t *cells, const float *freq_factors,
+                         int64_t K, int64_t B, int64_t H, int64_t HK, int64_t D, size_t k_nb1, size_t k_nb2, size_t v_nb1, size_t v_nb2,
+                         int n_dims, int mode, int n_ctx_orig, float freq_base, float freq_scale, float ext_factor, float attn_factor,
+                         float beta_fast, float beta_slow) {
+    MI355_REQUIRE(H > 0 && HK > 0 && D > 0, "qkv_rope_store: bad head geometry");
+    mi355_gemv_rope_mat m[3];
+    m[0] = mi355_gemv_rope_mat{type_q, wq, H * D, MI355_EPI_ROPE, q, H * D, 0, 0};
+    m[1] = mi355_gemv_rope_mat{type_k, wk, HK * D, MI355_EPI_ROPE_CACHE, kcache, 0, (int64_t)k_nb1, (int64_t)k_nb2};
+    m[2] = mi355_gemv_rope_mat{type_v, wv, HK * D, MI355_EPI_CACHE, vcache, 0, (int64_t)v_nb1, (int64_t)v_nb2};
+    mi355_rope_desc r = {pos, cells, freq_factors, D, n_dims, mode, n_ctx_orig, freq_base, freq_scale, ext_factor, attn_factor, beta_fast, beta_slow};
+    return mi355_mul_mat_vec_q_rope(stream, 3, m, act, K, B, &r);
+}
+
+}  // extern "C"

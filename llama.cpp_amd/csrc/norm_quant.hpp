@@ -122,6 +122,82 @@ struct norm_row {
     }
 };
 
+// Four elements of the row from e0 on, normalised (a wave's lanes hold 256 neighbouring ones) -> y row and activation, as rms_norm_quant_row
+template <int FMT>
+__device__ __forceinline__ f32x4 norm_piece(const f32x4 &v, const f32x4 &w, bool weighted, float scale, float *__restrict__ yr, void *__restrict__ act, int64_t row,
+                                            int64_t k, int64_t nrows, int64_t e0) {
+    const bool live = e0 < k;
+    int8_t *qplane = (int8_t *)act;
+    f32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = v[i] * scale;
+    if (weighted && live) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[i] = o[i] * w[i];
+    }
+    if (yr && live) *(f32x4 *)(yr + e0) = o;
+    if constexpr (FMT == 2) {
+        if (act && live) q8k_quantize_wave_tiled(o, threadIdx.x & 63, (uint8_t *)act, k, nrows, row, e0 >> 8);   // whole wave: k is a multiple of 256
+    } else if constexpr (FMT == 1) {
+        if (act && live) {   // whole wave: k is a multiple of 256
+            const int64_t nsb = k >> 8, sb = e0 >> 8;
+            float *d8 = (float *)(qplane + q8k_d_offset(k, nrows));
+            _Float16 *bs = (_Float16 *)(qplane + q8k_bs_offset(k, nrows));
+            q8k_quantize_wave(o, threadIdx.x & 63, qplane + row * k + sb * QKK, d8 + row * nsb + sb, bs + (row * nsb + sb) * 16);
+        }
+    } else {
+        if (act) quantize_block_lane(o, live, qplane, (act_ds *)(qplane + nrows * k), row, k, e0);
+    }
+    return o;
+}
+
+// One row by 1024 threads, for launches of a few rows: such a launch is one dependent chain per wave, some 2 ns per instruction, and with sixteen waves a thread of a
+// row of 4096 quantizes four elements instead of sixteen.  Same bits as rms_norm_quant_row: the first four waves form its sum in its order.  NV: pieces of a 256-thread
+// group (k <= 1024 * NV).  sh: 4 floats of LDS.
+template <int NV, int FMT>
+__device__ __forceinline__ void rms_norm_quant_row_wide(const float *__restrict__ xr, const float *__restrict__ w, float *__restrict__ yr, void *__restrict__ act, int64_t row,
+                                                        int64_t k, int64_t nrows, float eps, float *sh) {
+    constexpr int NP = NV / 4;
+    const int tid = threadIdx.x;
+    f32x4 own[NP], ww[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        const int64_t e0 = ((int64_t)p * 1024 + tid) * 4;
+        ww[p] = f32x4{1.f, 1.f, 1.f, 1.f};
+        if (w && e0 < k) ww[p] = *(const f32x4 *)(w + e0);
+    }
+    if (__builtin_amdgcn_readfirstlane(tid >> 8) == 0) {
+        f32x4 v[NV];
+#pragma unroll
+        for (int it = 0; it < NV; it++) {
+            const int64_t e0 = ((int64_t)it * 256 + tid) * 4;
+            v[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (e0 < k) v[it] = *(const f32x4 *)(xr + e0);
+        }
+        float ss = 0.0f;
+#pragma unroll
+        for (int it = 0; it < NV; it++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) ss = __builtin_fmaf(v[it][i], v[it][i], ss);
+        ss = wave_sum_dpp(ss);
+        if ((tid & 63) == 0) sh[tid >> 6] = ss;
+#pragma unroll
+        for (int p = 0; p < NP; p++) own[p] = v[4 * p];
+    } else {
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            const int64_t e0 = ((int64_t)p * 1024 + tid) * 4;
+            own[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (e0 < k) own[p] = *(const f32x4 *)(xr + e0);
+        }
+    }
+    __syncthreads();
+    const float total = add_rn(add_rn(add_rn(sh[0], sh[1]), sh[2]), sh[3]);
+    const float scale = 1.0f / sqrtf(add_rn(total / (float)k, eps));
+#pragma unroll
+    for (int p = 0; p < NP; p++) norm_piece<FMT>(own[p], ww[p], w != nullptr, scale, yr, act, row, k, nrows, ((int64_t)p * 1024 + tid) * 4);
+}
+
 // One row: xr -> y row (optional) and row `row` of the activation workspace `act` (optional), which holds nrows rows of k.
 // Each thread keeps its NV float4 of the row in registers (k <= 1024 * NV).  COH: the row was written by other groups of the
 // same launch with device-scope stores and is read with device-scope loads.  sh: 4 floats of LDS; the caller places a
@@ -156,33 +232,10 @@ __device__ __forceinline__ void rms_norm_quant_row(const float *__restrict__ xr,
         }
     }
     const float scale = rms_norm_scale<NV>(v, k, eps, sh);
-    int8_t *qplane = (int8_t *)act;
-    act_ds *ds = (act_ds *)(qplane + nrows * k);
 #pragma unroll
     for (int it = 0; it < NV; it++) {
-        const int64_t e0 = ((int64_t)it * 256 + tid) * 4;
-        const bool live = e0 < k;
-        f32x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; i++) o[i] = v[it][i] * scale;
-        if (w && live) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) o[i] = o[i] * ww[it][i];
-        }
-        if (yr && live) *(f32x4 *)(yr + e0) = o;
+        const f32x4 o = norm_piece<FMT>(v[it], ww[it], w != nullptr, scale, yr, act, row, k, nrows, ((int64_t)it * 256 + tid) * 4);
         if (keep) keep[it] = o;
-        if constexpr (FMT == 2) {
-            if (act && live) q8k_quantize_wave_tiled(o, tid & 63, (uint8_t *)act, k, nrows, row, e0 >> 8);   // whole wave: k is a multiple of 256
-        } else if constexpr (FMT == 1) {
-            if (act && live) {   // whole wave: k is a multiple of 256
-                const int64_t nsb = k >> 8, sb = e0 >> 8;
-                float *d8 = (float *)(qplane + q8k_d_offset(k, nrows));
-                _Float16 *bs = (_Float16 *)(qplane + q8k_bs_offset(k, nrows));
-                q8k_quantize_wave(o, tid & 63, qplane + row * k + sb * QKK, d8 + row * nsb + sb, bs + (row * nsb + sb) * 16);
-            }
-        } else {
-            if (act) quantize_block_lane(o, live, qplane, ds, row, k, e0);
-        }
     }
 }
 

@@ -126,7 +126,6 @@ class LlamaRunner:
         self.use_tiles = True
         self.tiles = {}
         self.fuse_qkv_rope = True   # prefill: ROPE and the KV-cache stores in the epilogue of the Q/K/V launch of the wide-tile GEMM
-        self.rope_table = None
         self.fuse_sum_norm = True   # prefill: a cut product's sum launch also normalises and quantizes its rows for the next products
         self.split_ws = None    # partial sums of tile products that are split along K (grown on first use, before any graph capture)
         # decode, T <= 4: SiLU*up + Q8_1 inside the gate/up launch (True: with both matrices of one type a group owns a whole 32-row
@@ -152,6 +151,7 @@ class LlamaRunner:
         self.kcache = [torch.zeros(cfg.n_ctx, HK, D, dtype=torch.float16, device=dev) for _ in range(cfg.n_layer)]
         self.vcache = [torch.zeros(cfg.n_ctx, HK, D, dtype=torch.float16, device=dev) for _ in range(cfg.n_layer)]
         self.pos = torch.zeros(T, dtype=torch.int32, device=dev)
+        self.rope_table = torch.empty(T * D, **f32)   # {cos, sin} per (token, pair), written once per pass
         self.mask = torch.zeros((T + 63) // 64 * 64, cfg.n_ctx, dtype=torch.float16, device=dev)
         kmax = max(E, F, H * D)
         self.act_a = torch.empty(max(int(self.lib.mi355_act_bytes(max(E, H * D), T)), int(self.lib.mi355_act_q8k_tiled_bytes(max(E, H * D), T))) + 256,
@@ -359,8 +359,6 @@ class LlamaRunner:
                 # wide-tile GEMM: the rotations and the cache stores ride in the epilogue of the Q/K/V launch; {cos, sin} per
                 # (token, pair) are the same for every layer and are written once per batch
                 if il == 0:
-                    if self.rope_table is None or self.rope_table.numel() < T * D:
-                        self.rope_table = torch.empty(T * D, dtype=torch.float32, device=self.dev)
                     check(lib.mi355_rope_table(_stream(), _ptr(self.pos), None, _ptr(self.rope_table), T, D, D, cfg.n_ctx, cfg.rope_theta, 1.0, 0.0, 1.0, 32.0, 1.0))
                 arr = (TiledMat * 3)()
                 for i, ((t, W), dst, N) in enumerate(((L["wq"], self.q, H * D), (L["wk"], kc, HK * D), (L["wv"], vc, HK * D))):
@@ -411,16 +409,17 @@ class LlamaRunner:
         x = self.x[:T]
         # one token: the attention norm is computed inside the Q/K/V launch (7 launches per layer)
         qkv_norm = self.fuse_qkv_norm and T == 1 and E <= 4096 and E % 1024 == 0
-        if not qkv_norm:
+        if qkv_norm:   # the rotations of the token's position are the same for every layer
+            check(lib.mi355_rope_table(_stream(), _ptr(self.pos), None, _ptr(self.rope_table), T, D, D, cfg.n_ctx, cfg.rope_theta, 1.0, 0.0, 1.0, 32.0, 1.0))
+        else:
             self._norm_quant(x, w.layers[0]["attn_norm"], self.act_a, T)
         for il, L in enumerate(w.layers):
             kc, vc = self.kcache[il], self.vcache[il]
             (tq, Wq), (tk, Wk), (tv, Wv) = L["wq"], L["wk"], L["wv"]
             if qkv_norm:
-                check(lib.mi355_rms_norm_qkv_rope_store(_stream(), _ptr(x), _ptr(L["attn_norm"]), cfg.rms_eps, tq, _ptr(Wq), tk, _ptr(Wk), tv, _ptr(Wv),
-                                                        _ptr(self.q), _ptr(kc), _ptr(vc), _ptr(self.pos), _ptr(self.pos), None, E, H, HK, D,
-                                                        kc.stride(0) * 2, kc.stride(1) * 2, vc.stride(0) * 2, vc.stride(1) * 2, D, 0, cfg.n_ctx,
-                                                        cfg.rope_theta, 1.0, 0.0, 1.0, 32.0, 1.0))
+                check(lib.mi355_rms_norm_qkv_rope_table_store(_stream(), _ptr(x), _ptr(L["attn_norm"]), cfg.rms_eps, tq, _ptr(Wq), tk, _ptr(Wk), tv, _ptr(Wv),
+                                                              _ptr(self.q), _ptr(kc), _ptr(vc), _ptr(self.rope_table), _ptr(self.pos), E, H, HK, D,
+                                                              kc.stride(0) * 2, kc.stride(1) * 2, vc.stride(0) * 2, vc.stride(1) * 2, D))
             else:
                 check(lib.mi355_qkv_rope_store(_stream(), tq, _ptr(Wq), tk, _ptr(Wk), tv, _ptr(Wv), _ptr(self.act_a), _ptr(self.q), _ptr(kc), _ptr(vc),
                                                _ptr(self.pos), _ptr(self.pos), None, E, T, H, HK, D, kc.stride(0) * 2, kc.stride(1) * 2,

@@ -50,6 +50,32 @@ def test_rms_norm_mul_quant(dev, K, nrows):
     _check_act_matches_q8_1(act, y, K, nrows)
 
 
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("K", [256, 2304, 4096, 8192, 12800, 16384])
+def test_rms_norm_mul_quant_few_rows_equal_many(dev, K, fmt):
+    """up to 256 rows have a group of 1024 threads each, more one of 256: same bits, row, weighted row and activation"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    rng = np.random.default_rng(K)
+    B = 257
+    x, w = _t(dev, (rng.standard_normal((B, K)) * rng.uniform(0.01, 100, (B, 1))).astype(np.float32)), _t(dev, rng.standard_normal(K).astype(np.float32))
+    fn = (lib.mi355_rms_norm_mul_quant, lib.mi355_rms_norm_mul_quant_q8k, lib.mi355_rms_norm_mul_quant_q8k_tiled)[fmt]
+    size = (lib.mi355_act_bytes, lib.mi355_act_q8k_bytes, lib.mi355_act_q8k_tiled_bytes)[fmt]
+    many = torch.zeros(B, K, device=dev)
+    act = torch.zeros(int(size(K, B)) + 256, dtype=torch.uint8, device=dev)
+    mi355.check(fn(None, x.data_ptr(), K, w.data_ptr(), many.data_ptr(), K, act.data_ptr(), K, B, 1e-5))
+    few = torch.zeros(B, K, device=dev)
+    mi355.check(fn(None, x.data_ptr(), K, w.data_ptr(), few.data_ptr(), K, None, K, 200, 1e-5))
+    mi355.check(fn(None, x[200:].data_ptr(), K, w.data_ptr(), few[200:].data_ptr(), K, None, K, B - 200, 1e-5))
+    assert torch.equal(few, many)
+    one, ref = torch.zeros_like(act), torch.zeros_like(act)
+    mi355.check(fn(None, x[:7].data_ptr(), K, w.data_ptr(), None, 0, one.data_ptr(), K, 7, 1e-5))
+    quant = (lib.mi355_quantize_act, lib.mi355_quantize_act_q8k, lib.mi355_quantize_act_q8k_tiled)[fmt]
+    mi355.check(quant(None, many.data_ptr(), ref.data_ptr(), K, 7, K))
+    assert torch.equal(one[:int(size(K, 7))], ref[:int(size(K, 7))])
+
+
 @pytest.mark.parametrize("K,nrows", [(14336, 1), (14336, 4), (1024, 7)])
 def test_swiglu_quant(dev, K, nrows):
     import torch
@@ -268,6 +294,34 @@ def test_qkv_rope_store_equals_three_launch_sequence(dev, B, tq, tk, tv):
     assert torch.equal(kc1, kc0)
     assert torch.equal(vc1, vc0)
     assert kc1.abs().sum().item() > 0 and vc1.abs().sum().item() > 0
+
+
+@pytest.mark.parametrize("K,H,HK,D,n_dims", [(1024, 4, 2, 64, 64), (3072, 5, 1, 128, 32), (4096, 32, 8, 128, 128)])
+def test_qkv_launch_with_norm_and_rope_table_equals_separate_launches(dev, K, H, HK, D, n_dims):
+    """one token: norm, projections, rotations from the table and the KV store in one launch, against the norm launch and the launch that works out its own rotations"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    rng = np.random.default_rng(K)
+    x, nw = _t(dev, rng.standard_normal((1, K)).astype(np.float32)), _t(dev, rng.standard_normal(K).astype(np.float32))
+    Ws = [mi355.upload_weights(t, _t(dev, orc.quantize("oracle", t, (rng.standard_normal((N, K)) * 0.05).astype(np.float32))))
+          for t, N in ((orc.Q4_K, H * D), (orc.Q8_0, HK * D), (orc.Q6_K if K % 2048 == 0 else orc.Q4_0, HK * D))]
+    types = (orc.Q4_K, orc.Q8_0, orc.Q6_K if K % 2048 == 0 else orc.Q4_0)
+    pos, cells = _t(dev, np.array([1234], dtype=np.int32)), _t(dev, np.array([3], dtype=np.int32))
+    rope = (4096, 500000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+    q = torch.zeros(2, H * D, device=dev)
+    kv = torch.zeros(2, 2, 8, HK, D, dtype=torch.float16, device=dev)
+    nb = (HK * D * 2, D * 2, HK * D * 2, D * 2)
+    act = torch.empty(int(lib.mi355_act_bytes(K, 1)) + 256, dtype=torch.uint8, device=dev)
+    mi355.check(lib.mi355_rms_norm_mul_quant(None, x.data_ptr(), K, nw.data_ptr(), None, 0, act.data_ptr(), K, 1, 1e-5))
+    w = [a for t, W in zip(types, Ws) for a in (t, W.data_ptr())]
+    mi355.check(lib.mi355_qkv_rope_store(None, *w, act.data_ptr(), q[0].data_ptr(), kv[0, 0].data_ptr(), kv[0, 1].data_ptr(), pos.data_ptr(), cells.data_ptr(), None,
+                                         K, 1, H, HK, D, *nb, n_dims, 0, *rope))
+    table = torch.empty(D, device=dev)
+    mi355.check(lib.mi355_rope_table(None, pos.data_ptr(), None, table.data_ptr(), 1, D, n_dims, *rope))
+    mi355.check(lib.mi355_rms_norm_qkv_rope_table_store(None, x.data_ptr(), nw.data_ptr(), 1e-5, *w, q[1].data_ptr(), kv[1, 0].data_ptr(), kv[1, 1].data_ptr(), table.data_ptr(),
+                                                        cells.data_ptr(), K, H, HK, D, *nb, n_dims))
+    assert torch.equal(q[0], q[1]) and torch.equal(kv[0], kv[1]) and bool(kv[0, :, 3].any())
 
 
 @pytest.mark.parametrize("B,norm", [(1, False), (1, True), (2, False), (4, False)])
