@@ -370,17 +370,23 @@ template <int D>
 __global__ void __launch_bounds__(512) k_fattn_combine(const float *__restrict__ ws, float *__restrict__ dst, int n_splits, int8_t *__restrict__ act_q,
                                                        act_ds *__restrict__ act_s, int64_t Hq) {
     constexpr int PARTS = 512 / D, U = 16;
-    __shared__ float s_w[256];
-    __shared__ float s_red[16];
+    __shared__ float s_weights[8][256];
     __shared__ float s_o[PARTS][D];
     const int64_t row = blockIdx.x;   // iq * Hq + head
     const float *p = ws + row * n_splits * (D + 2);
     const int tid = threadIdx.x, d = tid % D, part = tid / D;
     const bool live = part < PARTS;   // head sizes that do not divide 512 leave the last threads without an element
-    float ms = -FLT_MAX / 2, ls = 0.0f;
-    if (tid < n_splits) {
-        ms = p[tid * (D + 2) + D];
-        ls = p[tid * (D + 2) + D + 1];
+    // {max, sum} of split 64 c + lane, by every wave for itself: the weights need no exchange between waves
+    const int lane = tid & 63;
+    float ms[4], ls[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        ms[c] = -FLT_MAX / 2;
+        ls[c] = 0.0f;
+        if (64 * c + lane < n_splits) {
+            ms[c] = p[(64 * c + lane) * (D + 2) + D];
+            ls[c] = p[(64 * c + lane) * (D + 2) + D + 1];
+        }
     }
     float v[U];
 #pragma unroll
@@ -388,20 +394,17 @@ __global__ void __launch_bounds__(512) k_fattn_combine(const float *__restrict__
         const int sidx = part + PARTS * i;
         v[i] = live && sidx < n_splits ? p[sidx * (D + 2) + d] : 0.0f;
     }
-    float M = wave_max_dpp(ms);
-    if ((tid & 63) == 0) s_red[tid >> 6] = M;
-    __syncthreads();
-    M = s_red[0];
+    const float M = wave_max_dpp(fmaxf(fmaxf(ms[0], ms[1]), fmaxf(ms[2], ms[3])));
+    float *s_w = s_weights[__builtin_amdgcn_readfirstlane(tid >> 6)];   // the wave's own copy: LDS serves a wave's accesses in order
+    float L = 0.0f;
 #pragma unroll
-    for (int i = 1; i < 8; i++) M = fmaxf(M, s_red[i]);
-    const float w = tid < n_splits ? __expf(ms - M) : 0.0f;
-    if (tid < 256) s_w[tid] = w;
-    float L = wave_sum_dpp(ls * w);
-    if ((tid & 63) == 0) s_red[8 + (tid >> 6)] = L;
-    __syncthreads();
-    L = s_red[8];
-#pragma unroll
-    for (int i = 1; i < 8; i++) L += s_red[8 + i];
+    for (int c = 0; c < 4; c++) {
+        if (64 * c >= n_splits) break;   // uniform
+        const float w = 64 * c + lane < n_splits ? __expf(ms[c] - M) : 0.0f;
+        s_w[64 * c + lane] = w;
+        L = c == 0 ? wave_sum_dpp(ls[c] * w) : L + wave_sum_dpp(ls[c] * w);
+    }
+    asm volatile("" ::: "memory");   // other lanes' weights are read from here on
     float O = 0.0f;
 #pragma unroll
     for (int i = 0; i < U; i++) {

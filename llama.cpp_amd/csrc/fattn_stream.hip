@@ -53,19 +53,67 @@ __device__ __forceinline__ void fs_init(fs_state &S) {
     S.o0 = f32x4{0.f, 0.f, 0.f, 0.f};
     S.o1 = f32x4{0.f, 0.f, 0.f, 0.f};
 }
-// q of head head0 + lane % 4 (zeros past the R heads of the group) as f16 pairs, rounded as the reference rounds q to the K type
-// (ggml-cpu.c:11037-11040)
-__device__ __forceinline__ void fs_load_q(const fattn_args &a, int64_t head0, int R, int lane, u32 (&qv)[FS_D / 2]) {
-    const int hr = lane & 3;
-    const float *qp = (const float *)(a.q + (head0 + (hr < R ? hr : 0)) * a.q_nb2);
+// q of the group's four heads, 512 values, eight per lane (head lane / 16, elements 8 (lane % 16) .. + 7; zeros past the R heads): requested ahead of the transfers,
+// because a wave's loads return in the order of their issue.  (Every lane loading all 128 values of head lane % 4 behind the first tiles came to a third of a wave's
+// instructions over one tile, and none of them could run before those tiles had landed.)
+__device__ __forceinline__ void fs_request_q(const fattn_args &a, int64_t head0, int R, int lane, f32x4 (&x)[2]) {
+    const int h = lane >> 4;
+    const float *qp = (const float *)(a.q + (head0 + (h < R ? h : 0)) * a.q_nb2) + (lane & 15) * 8;
+    x[0] = *(const f32x4 *)qp;
+    x[1] = *(const f32x4 *)(qp + 4);
+}
+// ... as f16 pairs, rounded as the reference rounds q to the K type (ggml-cpu.c:11037-11040), through FS_QLDS bytes of the wave's LDS: qv = the 128 values of head
+// lane % 4.  Inline assembly, as all LDS accesses beside transfers in flight; heads FS_QROW bytes apart, so that the four of them lie in different banks.
+constexpr int FS_QROW = FS_ROW + 16, FS_QLDS = 4 * FS_QROW;
+__device__ __forceinline__ void fs_spread_q(f32x4 (&x)[2], int R, int lane, unsigned q_lds, u32 (&qv)[FS_D / 2]) {
+    u32x4 w;
 #pragma unroll
-    for (int i = 0; i < FS_D / 4; i++) {
-        f32x4 x = *(const f32x4 *)(qp + 4 * i);
-        if (hr >= R) x = f32x4{0.f, 0.f, 0.f, 0.f};
-        const f16x2 p0 = {(_Float16)x[0], (_Float16)x[1]}, p1 = {(_Float16)x[2], (_Float16)x[3]};
-        qv[2 * i] = __builtin_bit_cast(u32, p0);
-        qv[2 * i + 1] = __builtin_bit_cast(u32, p1);
+    for (int i = 0; i < 4; i++) {
+        const f16x2 p = {(_Float16)x[i >> 1][2 * (i & 1)], (_Float16)x[i >> 1][2 * (i & 1) + 1]};
+        w[i] = (lane >> 4) < R ? __builtin_bit_cast(u32, p) : 0u;
     }
+    asm volatile("ds_write_b128 %0, %1" ::"v"(q_lds + (unsigned)(lane >> 4) * FS_QROW + (unsigned)(lane & 15) * 16u), "v"(w) : "memory");
+    u32x4 t[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) asm volatile("ds_read_b128 %0, %1" : "=v"(t[i]) : "v"(q_lds + (unsigned)(lane & 3) * FS_QROW + (unsigned)i * 16u));
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]), "+v"(t[4]), "+v"(t[5]), "+v"(t[6]), "+v"(t[7]), "+v"(t[8]), "+v"(t[9]), "+v"(t[10]), "+v"(t[11]),
+                   "+v"(t[12]), "+v"(t[13]), "+v"(t[14]), "+v"(t[15]));
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        qv[4 * i] = t[i][0];
+        qv[4 * i + 1] = t[i][1];
+        qv[4 * i + 2] = t[i][2];
+        qv[4 * i + 3] = t[i][3];
+    }
+}
+// The mask values of a wave's cells, eight per lane and step (cells past the end count as masked): requested ahead of the transfers, then into the wave's LDS at m_lds
+template <int MT>   // tiles the wave has room for
+__device__ __forceinline__ void fs_request_mask(const fattn_args &a, int64_t c_begin, int n, int lane, u32x4 (&mc)[MT / 8]) {
+    const unsigned short *mrow = (const unsigned short *)a.mask;
+    const bool wide = ((uintptr_t)mrow & 15) == 0;
+#pragma unroll
+    for (int it = 0; it < MT / 8; it++) {
+        const int j = it * 64 + lane;
+        const int64_t c = c_begin + (int64_t)j * 8;
+        mc[it] = u32x4{0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u};   // -inf
+        if (j * 8 < n * FS_TILE) {
+            if (mrow && wide && c + 8 <= a.Nkv) {
+                mc[it] = load16(mrow + c);
+            } else {
+                unsigned short e[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) e[i] = c + i < a.Nkv ? (mrow ? mrow[c + i] : (unsigned short)0) : (unsigned short)0xFC00;
+#pragma unroll
+                for (int i = 0; i < 4; i++) mc[it][i] = (u32)e[2 * i] | ((u32)e[2 * i + 1] << 16);
+            }
+        }
+    }
+}
+template <int MT>
+__device__ __forceinline__ void fs_store_mask(u32x4 (&mc)[MT / 8], int lane, unsigned m_lds) {
+#pragma unroll
+    for (int it = 0; it < MT / 8; it++) asm volatile("ds_write_b128 %0, %1" ::"v"(m_lds + (unsigned)(it * 64 + lane) * 16u), "v"(mc[it]) : "memory");
 }
 // ALiBi slopes of the four heads (ggml-cpu.c:10998-11003), wave-uniform
 __device__ __forceinline__ void fs_slopes(const fattn_args &a, int64_t head0, float (&slope)[4]) {
@@ -224,6 +272,7 @@ __global__ void __launch_bounds__((ONE ? FS_WAVES_ONE : FS_WAVES) * 64, 1) k_fat
     __shared__ __attribute__((aligned(1024))) uint8_t ring_buf[NWV * STAGES * FS_STAGE];
     __shared__ __attribute__((aligned(16))) unsigned short pbuf[NWV][4][FS_TILE];
     __shared__ __attribute__((aligned(16))) unsigned short mbuf[NWV][MT * FS_TILE];
+    __shared__ __attribute__((aligned(16))) uint8_t qbuf[NWV][FS_QLDS];
     // the ring is written by global-to-LDS transfers only
     asm volatile("" ::"v"((void *)ring_buf) : "memory");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -247,28 +296,30 @@ __global__ void __launch_bounds__((ONE ? FS_WAVES_ONE : FS_WAVES) * 64, 1) k_fat
     voff = (unsigned)rsub * (unsigned)a.v_nb1 + (unsigned)(pos << 4);
     const uint8_t *k_head = a.k + hk * a.k_nb2, *v_head = a.v + hk * a.v_nb2;
     auto dma = [&](const uint8_t *g, unsigned off, uint8_t *l) {   // g, l: wave-uniform
-        asm volatile("" : "+v"(off));   // keeps the sum from being formed per lane ahead of the loop (two registers per source)
-        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(g + off), (void __attribute__((address_space(3))) *)l, 16, 0, 0);
+        buf_to_lds16(g, off, 0, l);
     };
-    // which = 0: the K half of the stage, 1: the V half (sixteen transfers each)
+    // which = 0: the K half of the stage, 1: the V half (sixteen transfers each).  The cell they start at; rows past the end of the cache repeat the last cell
+    auto issue_clamped = [&](int64_t c0, int st, int which) {
+        uint8_t *hb = ring + st * FS_STAGE + which * FS_KT;
+        const int64_t nb1 = which ? (int64_t)a.v_nb1 : (int64_t)a.k_nb1;
+        const uint8_t *g = (which ? v_head : k_head) + c0 * nb1;
+        const int last = a.Nkv - c0 < FS_TILE ? (int)(a.Nkv - 1 - c0) : FS_TILE - 1;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int row = 4 * i + rsub;
+            dma(g, (unsigned)(row < last ? row : last) * (unsigned)nb1 + (unsigned)((which ? pos : (pos ^ (row & 15))) << 4), hb + i * 1024);
+        }
+    };
     auto issue = [&](int t, int st, int which) {
         const int64_t c0 = c_begin + (int64_t)t * FS_TILE;
-        uint8_t *hb = ring + st * FS_STAGE + which * FS_KT;
-        const uint8_t *head = which ? v_head : k_head;
-        const int64_t nb1 = which ? (int64_t)a.v_nb1 : (int64_t)a.k_nb1;
         if (c0 + FS_TILE <= a.Nkv) {
-            const uint8_t *g = head + c0 * nb1;
+            uint8_t *hb = ring + st * FS_STAGE + which * FS_KT;
+            const int64_t nb1 = which ? (int64_t)a.v_nb1 : (int64_t)a.k_nb1;
+            const uint8_t *g = (which ? v_head : k_head) + c0 * nb1;
 #pragma unroll
             for (int i = 0; i < 16; i++) dma(g + (int64_t)(4 * i) * nb1, which ? voff : koff[i & 3], hb + i * 1024);
         } else {
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int row = 4 * i + rsub;
-                int64_t cell = c0 + row;
-                if (cell >= a.Nkv) cell = a.Nkv - 1;
-                const uint8_t *g = head + cell * nb1 + ((which ? pos : (pos ^ (row & 15))) << 4);
-                __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)g, (void __attribute__((address_space(3))) *)(hb + i * 1024), 16, 0, 0);
-            }
+            issue_clamped(c0, st, which);
         }
     };
 
@@ -276,51 +327,31 @@ __global__ void __launch_bounds__((ONE ? FS_WAVES_ONE : FS_WAVES) * 64, 1) k_fat
     fs_init(S);
     const float scale = a.softcap != 0.0f ? a.scale / a.softcap : a.scale;
 
-    // order of the transfers: K0 V0 K1 V1, then K(t + 2) once the scores of tile t are taken and V(t + 2) once its output is
-    if (n > 0) {
-        issue(0, 0, 0);
-        issue(0, 0, 1);
+    // q and this wave's mask values first, then the transfers in the order K0 V0, K1 V1 (when q is in place), then K(t + 2) once the scores of tile t are taken and V(t + 2) once its output
+    // is.  All are buffer accesses or ordinary loads: the compiler counts those exactly and waits for q with the transfers in flight.
+    const int hr = lane & 3;
+    f32x4 qx[2];
+    u32x4 mc[MT / 8];
+    fs_request_q(a, hk * R, R, lane, qx);
+    fs_request_mask<MT>(a, c_begin, n, lane, mc);
+    asm volatile("" ::: "memory");   // the loads are not to be moved behind the transfers
+    __builtin_amdgcn_sched_barrier(0);
+    {   // without a branch around them (a wave without tiles moves the last one): at a join of paths the compiler knows the smaller number of requests in flight only
+        const int64_t first = n > 0 ? c_begin : (int64_t)(n_tiles - 1) * FS_TILE;
+        issue_clamped(first, 0, 0);
+        issue_clamped(first, 0, 1);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    unsigned short *mw = mbuf[wave];
+    u32 qv[FS_D / 2];
+    fs_spread_q(qx, R, lane, (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)&qbuf[wave][0], qv);
+    fs_store_mask<MT>(mc, lane, (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned short *)mw);
     if (!ONE && n > 1) {
         issue(1, 1, 0);
         issue(1, 1, 1);
     }
-    // While the first two tiles travel: q and this wave's mask values (all requested before the first is used).
-    const int hr = lane & 3;
-    u32 qv[FS_D / 2];
-    fs_load_q(a, hk * R, R, lane, qv);
-    // ---- mask values of the wave's cells into LDS, eight cells per lane and step (cells past the end count as masked)
-    unsigned short *mw = mbuf[wave];
-    {
-        const unsigned short *mrow = (const unsigned short *)a.mask;
-        const bool wide = ((uintptr_t)mrow & 15) == 0;
-        u32x4 mc[MT / 8];
-#pragma unroll
-        for (int it = 0; it < MT / 8; it++) {
-            const int j = it * 64 + lane;
-            const int64_t c = c_begin + (int64_t)j * 8;
-            mc[it] = u32x4{0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u};   // -inf
-            if (j * 8 < n * FS_TILE) {
-                if (mrow && wide && c + 8 <= a.Nkv) {
-                    mc[it] = load16(mrow + c);
-                } else {
-                    unsigned short e[8];
-#pragma unroll
-                    for (int i = 0; i < 8; i++) e[i] = c + i < a.Nkv ? (mrow ? mrow[c + i] : (unsigned short)0) : (unsigned short)0xFC00;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) mc[it][i] = (u32)e[2 * i] | ((u32)e[2 * i + 1] << 16);
-                }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < MT / 8; it++) {
-            const int j = it * 64 + lane;
-            if (j * 8 < n * FS_TILE) *(u32x4 *)(mw + j * 8) = mc[it];
-        }
-    }
-    // From here on LDS is read and written through inline assembly with waits placed by hand: for an access it can see, the
+    // LDS is read and written through inline assembly with waits placed by hand: for an access it can see, the
     // compiler waits for every global-to-LDS transfer in flight, which would serialise the ring.
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     // LDS byte addresses of this lane's operands inside a stage
     const unsigned ring_lds = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)ring;
     const unsigned k_lane = (unsigned)lane * FS_ROW + ((unsigned)(lane & 15) << 4);                      // chunk c at k_lane ^ (c << 4)
@@ -402,41 +433,53 @@ struct fsq_geo {
 };
 constexpr int FSQ_SCALES = FS_TILE * 8;   // bytes of scales per tile and operand
 
-template <int R4>
-__device__ __forceinline__ int quad_bcast_i(int v) { return __builtin_amdgcn_update_dpp(0, v, R4 * 0x55, 0xF, 0xF, true); }
-
-// q of head head0 + lane % 4 as Q8_0 (quantize_row_q8_0_ref, ggml-quants.c:194-218): 32 words of levels, the f16-rounded scales of
-// the four blocks and the sums of their levels; zeros past the R heads of the group
-__device__ __forceinline__ void fsq_load_q(const fattn_args &a, int64_t head0, int R, int lane, u32 (&qw)[32], float (&dq)[4], int (&qs)[4]) {
-    const int hr = lane & 3;
-    const float *qp = (const float *)(a.q + (head0 + (hr < R ? hr : 0)) * a.q_nb2);
+// q of the group's four heads (fs_request_q's eight values per lane) as Q8_0 (quantize_row_q8_0_ref, ggml-quants.c:194-218): qw = the 32 words of levels of head lane % 4,
+// through FSQ_QLDS bytes of the wave's LDS; dqa / qsa [head][block] = the f16-rounded scales and the sums of the levels, the same in every lane; zeros past the R heads
+constexpr int FSQ_QROW = FS_D + 16, FSQ_QLDS = 4 * FSQ_QROW;
+static_assert(FSQ_QLDS <= 32 * FS_ROW, "taken from the room of half a V tile");
+__device__ __forceinline__ void fsq_spread_q(f32x4 (&x)[2], int R, int lane, unsigned q_lds, u32 (&qw)[32], float (&dqa)[4][4], int (&qsa)[4][4]) {
+    float amax = 0.0f;
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-        f32x4 x[8];
-        float amax = 0.0f;
+    for (int i = 0; i < 8; i++) {
+        x[i >> 2][i & 3] = (lane >> 4) < R ? x[i >> 2][i & 3] : 0.0f;
+        amax = fmaxf(amax, fabsf(x[i >> 2][i & 3]));
+    }
+    amax = lanes_max<4>(amax);   // four lanes hold a block
+    float d, id;
+    q8_scale(amax, d, id);
+    u32x2 w;
+    int sum = 0;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            x[i] = *(const f32x4 *)(qp + 32 * b + 4 * i);
-            if (hr >= R) x[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 2; i++) {
+        u32 t = 0;
 #pragma unroll
-            for (int j = 0; j < 4; j++) amax = fmaxf(amax, fabsf(x[i][j]));
+        for (int j = 0; j < 4; j++) {
+            const int q = q8_level(x[i][j], id);
+            sum += q;
+            t |= (u32)(q & 0xFF) << (8 * j);
         }
-        float d, id;
-        q8_scale(amax, d, id);
-        int sum = 0;
+        w[i] = t;
+    }
+    sum = lanes_sum_i<4>(sum);
+    const float dr = half_bits_to_float(float_to_half_bits(d));
+    asm volatile("ds_write_b64 %0, %1" ::"v"(q_lds + (unsigned)(lane >> 4) * FSQ_QROW + (unsigned)(lane & 15) * 8u), "v"(w) : "memory");
+    u32x4 t[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            u32 w = 0;
+    for (int i = 0; i < 8; i++) asm volatile("ds_read_b128 %0, %1" : "=v"(t[i]) : "v"(q_lds + (unsigned)(lane & 3) * FSQ_QROW + (unsigned)i * 16u));
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int q = q8_level(x[i][j], id);
-                sum += q;
-                w |= (u32)(q & 0xFF) << (8 * j);
-            }
-            qw[8 * b + i] = w;
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            dqa[r][b] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, dr), 16 * r + 4 * b));
+            qsa[r][b] = __builtin_amdgcn_readlane(sum, 16 * r + 4 * b);
         }
-        dq[b] = half_bits_to_float(float_to_half_bits(d));
-        qs[b] = sum;
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]), "+v"(t[4]), "+v"(t[5]), "+v"(t[6]), "+v"(t[7]));
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        qw[4 * i] = t[i][0];
+        qw[4 * i + 1] = t[i][1];
+        qw[4 * i + 2] = t[i][2];
+        qw[4 * i + 3] = t[i][3];
     }
 }
 
@@ -604,109 +647,77 @@ __global__ void __launch_bounds__(((ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK
         vsoff = (p >> 1) * (unsigned)vsrc.cell_sc + ((p & 1) << 2);
     }
     auto dma16 = [&](const uint8_t *g, unsigned off, uint8_t *l) {   // g, l: wave-uniform
-        asm volatile("" : "+v"(off));
-        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(g + off), (void __attribute__((address_space(3))) *)l, 16, 0, 0);
+        buf_to_lds16(g, off, 0, l);
     };
-    auto dma4 = [&](const uint8_t *g, unsigned off, uint8_t *l) {
-        asm volatile("" : "+v"(off));
-        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)(g + off), (void __attribute__((address_space(3))) *)l, 4, 0, 0);
-    };
-    // which = 0: K levels and scales of tile t into stage st (CK transfers), 1: V (CV transfers)
-    auto issue = [&](int t, int st, int which) {
-        const int64_t c0 = c_begin + (int64_t)t * FS_TILE;
+    auto dma4 = [&](const uint8_t *g, unsigned off, uint8_t *l) { buf_to_lds4(g, off, 0, l); };
+    // which = 0: K levels and scales into stage st (CK transfers), 1: V (CV transfers).  The cell they start at; rows past the end of the cache repeat the last cell (their
+    // scores are discarded)
+    auto issue_clamped = [&](int64_t c0, int st, int which) {
         uint8_t *sb = ring + st * STAGE;
         const int64_t nb_lv = which ? vsrc.cell_lv : ksrc.cell_lv, nb_sc = which ? vsrc.cell_sc : ksrc.cell_sc;
-        const uint8_t *lvp = which ? v_lv : k_lv, *scp = which ? v_sc : k_sc;
+        const uint8_t *g = (which ? v_lv : k_lv) + c0 * nb_lv, *gs = (which ? v_sc : k_sc) + c0 * nb_sc;
         uint8_t *l_lv = sb + (which ? OFF_V : 0), *l_sc = sb + (which ? OFF_VS : OFF_KS);
         const int NT = which ? GV::NT : GK::NT, RPT = which ? GV::RPT : GK::RPT, CH = which ? GV::CH : GK::CH;
+        const int last = a.Nkv - c0 < FS_TILE ? (int)(a.Nkv - 1 - c0) : FS_TILE - 1;
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (i < NT) {
+                const int row = RPT * i + lane / CH, pos = lane % CH;
+                const int swz = which ? 0 : (TK == MI355_Q8_0 ? (row >> 1) & 7 : (row >> 2) & 3);
+                dma16(g, (unsigned)(row < last ? row : last) * (unsigned)nb_lv + (unsigned)((pos ^ swz) << 4), l_lv + i * 1024);
+            }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int row = 32 * i + (lane >> 1);
+            dma4(gs, (unsigned)(row < last ? row : last) * (unsigned)nb_sc + (unsigned)((lane & 1) << 2), l_sc + i * 256);
+        }
+    };
+    auto issue = [&](int t, int st, int which) {
+        const int64_t c0 = c_begin + (int64_t)t * FS_TILE;
         if (c0 + FS_TILE <= a.Nkv) {
-            const uint8_t *g = lvp + c0 * nb_lv;
+            uint8_t *sb = ring + st * STAGE;
+            const int64_t nb_lv = which ? vsrc.cell_lv : ksrc.cell_lv, nb_sc = which ? vsrc.cell_sc : ksrc.cell_sc;
+            uint8_t *l_lv = sb + (which ? OFF_V : 0), *l_sc = sb + (which ? OFF_VS : OFF_KS);
+            const int NT = which ? GV::NT : GK::NT, RPT = which ? GV::RPT : GK::RPT;
+            const uint8_t *g = (which ? v_lv : k_lv) + c0 * nb_lv, *gs = (which ? v_sc : k_sc) + c0 * nb_sc;
 #pragma unroll
             for (int i = 0; i < 8; i++)
                 if (i < NT) dma16(g + (int64_t)(RPT * i) * nb_lv, which ? voff : koff[i & 1], l_lv + i * 1024);
-            const uint8_t *gs = scp + c0 * nb_sc;
             dma4(gs, which ? vsoff : ksoff, l_sc);
             dma4(gs + 32 * nb_sc, which ? vsoff : ksoff, l_sc + 256);
-        } else {   // the cache's last, partial tile: rows past the end repeat the last cell (their scores are discarded)
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (i < NT) {
-                    const int row = RPT * i + lane / CH, pos = lane % CH;
-                    int64_t cell = c0 + row;
-                    if (cell >= a.Nkv) cell = a.Nkv - 1;
-                    const int swz = which ? 0 : (TK == MI355_Q8_0 ? (row >> 1) & 7 : (row >> 2) & 3);
-                    const uint8_t *g = lvp + cell * nb_lv + ((pos ^ swz) << 4);
-                    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)g, (void __attribute__((address_space(3))) *)(l_lv + i * 1024), 16, 0, 0);
-                }
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                int64_t cell = c0 + 32 * i + (lane >> 1);
-                if (cell >= a.Nkv) cell = a.Nkv - 1;
-                const uint8_t *g = scp + cell * nb_sc + ((lane & 1) << 2);
-                __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)g, (void __attribute__((address_space(3))) *)(l_sc + i * 256), 4, 0, 0);
-            }
+        } else {
+            issue_clamped(c0, st, which);
         }
     };
 
     fs_state S;
     fs_init(S);
     const float scale = a.softcap != 0.0f ? a.scale / a.softcap : a.scale;
-    if (n > 0) {
-        issue(0, 0, 0);
-        issue(0, 0, 1);
+    // q and this wave's mask values first, the transfers of the first tile behind them (see k_fattn_dec_stream)
+    const int hr = lane & 3;
+    f32x4 qx[2];
+    u32x4 mc[MT / 8];
+    fs_request_q(a, hk * R, R, lane, qx);
+    fs_request_mask<MT>(a, c_begin, n, lane, mc);
+    asm volatile("" ::: "memory");   // the loads are not to be moved behind the transfers
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        const int64_t first = n > 0 ? c_begin : (int64_t)(n_tiles - 1) * FS_TILE;
+        issue_clamped(first, 0, 0);
+        issue_clamped(first, 0, 1);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    unsigned short *mw = mbuf[wave];
+    u32 qw[32];
+    float dqa[4][4];
+    int qsa[4][4];
+    fsq_spread_q(qx, R, lane, (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)(vf_buf + wave * FSQ_VF), qw, dqa, qsa);   // no V there yet
+    fs_store_mask<MT>(mc, lane, (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned short *)mw);
     if (!ONE && n > 1) {
         issue(1, 1, 0);
         issue(1, 1, 1);
     }
-    // While the first two tiles travel: q as Q8_0 and this wave's mask values.
-    const int hr = lane & 3;
-    u32 qw[32];
-    float dq[4], dqa[4][4];
-    int qs[4], qsa[4][4];
-    fsq_load_q(a, hk * R, R, lane, qw, dq, qs);
-#pragma unroll
-    for (int b = 0; b < 4; b++) {   // every lane needs the scales and sums of all four heads: lane r of its quad holds head r's
-        const int di = __builtin_bit_cast(int, dq[b]);
-        dqa[0][b] = __builtin_bit_cast(float, quad_bcast_i<0>(di));
-        dqa[1][b] = __builtin_bit_cast(float, quad_bcast_i<1>(di));
-        dqa[2][b] = __builtin_bit_cast(float, quad_bcast_i<2>(di));
-        dqa[3][b] = __builtin_bit_cast(float, quad_bcast_i<3>(di));
-        qsa[0][b] = quad_bcast_i<0>(qs[b]);
-        qsa[1][b] = quad_bcast_i<1>(qs[b]);
-        qsa[2][b] = quad_bcast_i<2>(qs[b]);
-        qsa[3][b] = quad_bcast_i<3>(qs[b]);
-    }
-    unsigned short *mw = mbuf[wave];
-    {
-        const unsigned short *mrow = (const unsigned short *)a.mask;
-        const bool wide = ((uintptr_t)mrow & 15) == 0;
-        u32x4 mc[MT / 8];
-#pragma unroll
-        for (int it = 0; it < MT / 8; it++) {
-            const int j = it * 64 + lane;
-            const int64_t c = c_begin + (int64_t)j * 8;
-            mc[it] = u32x4{0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u, 0xFC00FC00u};   // -inf
-            if (j * 8 < n * FS_TILE) {
-                if (mrow && wide && c + 8 <= a.Nkv) {
-                    mc[it] = load16(mrow + c);
-                } else {
-                    unsigned short e[8];
-#pragma unroll
-                    for (int i = 0; i < 8; i++) e[i] = c + i < a.Nkv ? (mrow ? mrow[c + i] : (unsigned short)0) : (unsigned short)0xFC00;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) mc[it][i] = (u32)e[2 * i] | ((u32)e[2 * i + 1] << 16);
-                }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < MT / 8; it++) {
-            const int j = it * 64 + lane;
-            if (j * 8 < n * FS_TILE) *(u32x4 *)(mw + j * 8) = mc[it];
-        }
-    }
-    // From here on LDS is read and written through inline assembly with waits placed by hand (see k_fattn_dec_stream).
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    // LDS is read and written through inline assembly with waits placed by hand (see k_fattn_dec_stream).
     const unsigned ring_lds = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)ring;
     const unsigned vf_lds = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)(vf_buf + wave * FSQ_VF);
     const unsigned k_lane = TK == MI355_Q8_0 ? (unsigned)lane * 128u + ((((unsigned)lane >> 1) & 7u) << 4) : (unsigned)lane * 64u + ((((unsigned)lane >> 2) & 3u) << 4);
@@ -918,6 +929,7 @@ int launch_fattn_dec_stream(hipStream_t s, fattn_args &a, int64_t D, size_t ws_b
     const int64_t R = a.Hq / a.Hkv;
     if (D != FS_D || a.Nq != 1 || R > 4 || a.Hkv > 65535 || a.ws == nullptr) return 1;
     if ((a.q_nb2 % 16) != 0 || (a.k_nb1 % 16) != 0 || (a.k_nb2 % 16) != 0 || (a.v_nb1 % 16) != 0 || (a.v_nb2 % 16) != 0) return 1;
+    if (a.k_nb1 >= ((size_t)1 << 26) || a.v_nb1 >= ((size_t)1 << 26)) return 1;   // the transfers' per-lane offsets are 32-bit
     const int64_t n_tiles = (a.Nkv + FS_TILE - 1) / FS_TILE;
     int64_t waves_per_head = FS_TOTAL_WAVES / a.Hkv;
     if (waves_per_head < FS_WAVES) waves_per_head = FS_WAVES;
