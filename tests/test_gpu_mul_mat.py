@@ -156,6 +156,26 @@ def test_quantize_q8k_bit_exact(dev, K, dist):
         assert bs[:, :, :8].min() >= 0 and bs[:, :, :8].max() <= 63
 
 
+@pytest.mark.parametrize("seed", [0, 1])
+def test_quantize_q8k_every_scale(dev, seed):
+    """block maxima of every magnitude whose reciprocal scale is finite, the largest value of either sign at any place and several times over: both quotients and the choice
+    of the first largest element agree with the host on both sides of the range (2^-90 .. 2^90) the correction steps are used in"""
+    import mi355
+    rng = np.random.default_rng(seed)
+    nsb, nrows = 236, 24
+    amax = np.ldexp(rng.uniform(1, 2, (nrows, nsb)), np.arange(-118, 118)).astype(np.float32)
+    x = (rng.uniform(-1, 1, (nrows, nsb, 256)) * amax[..., None]).astype(np.float32)
+    for _ in range(3):   # up to three elements of the largest magnitude
+        at, sign = rng.integers(0, 256, (nrows, nsb, 1)), rng.choice([-1, 1], (nrows, nsb, 1)).astype(np.float32)
+        np.put_along_axis(x, at, sign * amax[..., None], axis=2)
+    x = x.reshape(nrows, nsb * 256)
+    K = nsb * 256
+    got = mi355.quantize_act_q8k(_to_dev(dev, x)).cpu().numpy()
+    want = orc.quantize("oracle", orc.Q8_K, x).reshape(nrows, nsb, 292)
+    assert np.array_equal(got[nrows * K:nrows * K + nrows * nsb * 4].view(np.uint32).reshape(nrows, nsb), np.ascontiguousarray(want[:, :, :4]).view(np.uint32).reshape(nrows, nsb))
+    assert np.array_equal(got[:nrows * K].view(np.int8).reshape(nrows, nsb, 256), want[:, :, 4:260].view(np.int8))
+
+
 @pytest.mark.parametrize("name,t", TYPES)
 @pytest.mark.parametrize("N,K,B", [(512, 4096, 64), (384, 2048, 512), (130, 1024, 33), (4096, 4096, 9), (128, 14336, 100)])
 def test_mmq_matches_oracle(dev, name, t, N, K, B):
