@@ -800,7 +800,7 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
     __shared__ __attribute__((aligned(16))) unsigned short pbuf[FSS_MAX_WAVES][4][FS_TILE];
     __shared__ float s_m[FSS_MAX_WAVES][4], s_l[FSS_MAX_WAVES][4];
     __shared__ float s_o[FSS_MAX_WAVES][4][DO];
-    __shared__ __attribute__((aligned(16))) unsigned short qbuf[FSS_MAX_WAVES][4][FS_D];
+    __shared__ __attribute__((aligned(16))) uint8_t qbuf[FSS_MAX_WAVES][FS_QLDS];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int n_waves = (int)(blockDim.x >> 6);
@@ -809,6 +809,14 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
     const int64_t c0 = (int64_t)wave * FS_TILE;
     const int rsub = lane >> 4, pos = lane & 15;
 
+    // q of the group's four heads (two coalesced loads per lane) and the mask value first, K and V behind them: loads return in the order of their issue
+    f32x4 qx[2];
+    fs_request_q(a, hk * R, R, lane, qx);
+    const int64_t cell = c0 + lane;
+    // (without a mask some word of q is read in its place: at a join of two paths the compiler would wait for everything)
+    const unsigned short *mrow = (const unsigned short *)(a.mask ? a.mask : a.q);
+    unsigned short mbits = mrow[!a.mask ? 0 : cell < a.Nkv ? cell : a.Nkv - 1];
+    __builtin_amdgcn_sched_barrier(0);
     // load i: rows 4i .. 4i + 3, lane -> row 4i + lane / 16, chunk lane % 16 (rows past the end repeat the last cell; their weights are zero)
     // (half rows of V: rows 8i .. 8i + 7, lane -> row 8i + lane / 8, chunk lane % 8 of the half)
     const int vsub = lane / VCH, vpos = lane % VCH + VCH * part;
@@ -825,38 +833,14 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
         if (cell >= a.Nkv) cell = a.Nkv - 1;
         vraw[i] = load16(a.v + cell * a.v_nb1 + hk * a.v_nb2 + (vpos << 4));
     }
-    const int64_t cell = c0 + lane;
-    unsigned short mbits = 0xFC00;   // -inf
-    if (cell < a.Nkv) mbits = a.mask ? ((const unsigned short *)a.mask)[cell] : (unsigned short)0;
-    // q of the group's four heads: two coalesced loads per lane (chunk ch of 128: head ch / 32, floats 4 (ch % 32) .. + 3), rounded to
-    // f16 into the wave's 1 KiB of LDS; every lane then reads the 128 values of head lane % 4 (128 floats per lane in flight would
-    // not fit beside the K and V tiles)
-    f32x4 qraw[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int ch = lane + 64 * j, head = ch >> 5;
-        qraw[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (head < R) qraw[j] = *(const f32x4 *)(a.q + (hk * R + head) * a.q_nb2 + (size_t)(ch & 31) * 16);
-    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (!a.mask) mbits = 0;
+    if (cell >= a.Nkv) mbits = 0xFC00;   // -inf
     float slope[4];
     fs_slopes(a, hk * R, slope);
     const float scale = a.softcap != 0.0f ? a.scale / a.softcap : a.scale;
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int ch = lane + 64 * j;
-        const f16x2 p0 = {(_Float16)qraw[j][0], (_Float16)qraw[j][1]}, p1 = {(_Float16)qraw[j][2], (_Float16)qraw[j][3]};
-        const u32x2 packed = {__builtin_bit_cast(u32, p0), __builtin_bit_cast(u32, p1)};
-        *(u32x2 *)(&qbuf[wave][0][0] + ch * 4) = packed;
-    }
     u32 qv[FS_D / 2];
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const u32x4 t = *(const u32x4 *)(&qbuf[wave][lane & 3][0] + i * 8);
-        qv[4 * i] = t[0];
-        qv[4 * i + 1] = t[1];
-        qv[4 * i + 2] = t[2];
-        qv[4 * i + 3] = t[3];
-    }
+    fs_spread_q(qx, R, lane, (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)&qbuf[wave][0], qv);
 
     // K through LDS: chunk c of row r at position c ^ (r & 15); then each lane reads the row of its cell
     uint8_t *tb = tbuf + wave * FS_KT;
