@@ -136,24 +136,43 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
     const int d0 = sub * 8;
     const bool active = d0 < D;
 
+    const int64_t c_begin = (int64_t)split * a.cells_per_split;
+    const int64_t c_end = c_begin + a.cells_per_split < a.Nkv ? c_begin + a.cells_per_split : a.Nkv;
+    constexpr int U = 4;   // steps of SLOTS cells at a time, see the loop
+    // (us, one row over 1024 cells: 32 / 8 heads of 80 16.2 -> 12.5, of 256 12.9 -> 12.4 against masks requested when their round begins, behind q.)
+    // The mask entries of a round are requested together, from clamped addresses and without a branch per entry (a branch per entry makes each load wait for the one
+    // before it: U round trips instead of one); the first round's ahead of q, the others behind the rows of the round before.
+    unsigned mraw[U];   // (32-bit each: halves packed in pairs would be merged load by load, with a wait for each)
+    const unsigned short *mrow = a.mask ? (const unsigned short *)(a.mask + iq * a.mask_nb1) : (const unsigned short *)a.q;   // without a mask some word of q, not used
+    const int64_t mask_last = a.mask ? c_end - 1 : 0;   // (a choice of the index per entry becomes two paths, with a wait at their join)
+    auto request_mask = [&](int64_t cb) {
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int64_t c = cb + j * SLOTS + slot;
+            mraw[j] = mrow[c < mask_last ? c : mask_last];
+        }
+    };
     // q slices, rounded to f16 (ggml-cpu.c:11037-11040 converts q to the K type before the dot)
     u32x4 qh[R];
     float slope[R];
+    f32x4 qx[R][2];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const float *qp = (const float *)(a.q + iq * a.q_nb1 + (head0 + r) * a.q_nb2) + (active ? d0 : 0);
+        qx[r][0] = *(const f32x4 *)qp;
+        qx[r][1] = *(const f32x4 *)(qp + 4);
+    }
+    request_mask(c_begin);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const int64_t head = head0 + r;
-        const float *qp = (const float *)(a.q + iq * a.q_nb1 + head * a.q_nb2) + d0;
-        f32x4 x0 = {0, 0, 0, 0}, x1 = {0, 0, 0, 0};
-        if (active) {
-            x0 = *(const f32x4 *)qp;
-            x1 = *(const f32x4 *)(qp + 4);
-        }
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            f16x2 p0 = {(_Float16)x0[2 * i], (_Float16)x0[2 * i + 1]};
-            f16x2 p1 = {(_Float16)x1[2 * i], (_Float16)x1[2 * i + 1]};
-            qh[r][i] = __builtin_bit_cast(u32, p0);
-            qh[r][2 + i] = __builtin_bit_cast(u32, p1);
+            f16x2 p0 = {(_Float16)qx[r][0][2 * i], (_Float16)qx[r][0][2 * i + 1]};
+            f16x2 p1 = {(_Float16)qx[r][1][2 * i], (_Float16)qx[r][1][2 * i + 1]};
+            qh[r][i] = active ? __builtin_bit_cast(u32, p0) : 0u;
+            qh[r][2 + i] = active ? __builtin_bit_cast(u32, p1) : 0u;
         }
         // ALiBi slope of this head (ggml-cpu.c:10998-11003)
         slope[r] = 1.0f;
@@ -172,9 +191,6 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
         for (int i = 0; i < 8; i++) acc[r][i] = 0.0f;
     }
 
-    const int64_t c_begin = (int64_t)split * a.cells_per_split;
-    const int64_t c_end = c_begin + a.cells_per_split < a.Nkv ? c_begin + a.cells_per_split : a.Nkv;
-    const unsigned short *mrow = a.mask ? (const unsigned short *)(a.mask + iq * a.mask_nb1) : nullptr;
     const float scale = a.softcap != 0.0f ? a.scale / a.softcap : a.scale;
     // quantized operands (wave-uniform choice): this lane's place in the rows of kv head hk
     const bool k_f16 = !QUANT || type_k == MI355_F16, v_f16 = !QUANT || type_v == MI355_F16;
@@ -185,31 +201,16 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
     // U steps of SLOTS cells at a time: all mask entries, then all K/V rows of the U steps are requested before the first
     // is used, so a short context costs one round trip to memory instead of one per step.  Cells are still folded into a
     // slot's state in ascending order.
-    constexpr int U = 4;
     for (int64_t cb = c_begin; cb < c_end; cb += U * SLOTS) {
         float mv[U];
         bool valid[U];
-        {
-            // the U mask entries are requested together, from clamped addresses and without a branch per entry (a branch per entry
-            // makes each load wait for the one before it: U round trips instead of one)
-            unsigned mraw[U];   // (32-bit each: halves packed in pairs would be merged load by load, with a wait for each)
 #pragma unroll
-            for (int j = 0; j < U; j++) mraw[j] = 0;
-            if (mrow) {   // uniform
-#pragma unroll
-                for (int j = 0; j < U; j++) {
-                    const int64_t c = cb + j * SLOTS + slot;
-                    mraw[j] = mrow[c < c_end ? c : c_end - 1];
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);   // (or each load is moved down to its first use, and waited for there)
-#pragma unroll
-            for (int j = 0; j < U; j++) {
-                const int64_t c = cb + j * SLOTS + slot;
-                mv[j] = half_bits_to_float((unsigned short)mraw[j]);
-                valid[j] = c < c_end && mv[j] != -INFINITY;
-                if (c >= c_end) mv[j] = 0.0f;
-            }
+        for (int j = 0; j < U; j++) {
+            const int64_t c = cb + j * SLOTS + slot;
+            asm volatile("" : "+v"(mraw[j]));   // stays a register of its own from round to round
+            mv[j] = a.mask ? half_bits_to_float((unsigned short)mraw[j]) : 0.0f;
+            valid[j] = c < c_end && mv[j] != -INFINITY;
+            if (c >= c_end) mv[j] = 0.0f;
         }
         u32x4 kk[U], vv[U];
         if constexpr (!QUANT) {
@@ -249,6 +250,7 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
                 }
             }
         }
+        if (cb + U * SLOTS < c_end) request_mask(cb + U * SLOTS);   // uniform
         float kd[U];   // quantized K: the levels as exact f16 values; their dot with q takes the block's scale afterwards
 #pragma unroll
         for (int j = 0; j < U; j++) {

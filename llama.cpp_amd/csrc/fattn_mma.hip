@@ -236,19 +236,30 @@ __device__ __forceinline__ float finish_scores_dec(f32x16 &S, const u32x2 (&mw)[
     return mx;
 }
 
+// A query row's share of a lane (elements 16 kk + 8 lhi .. + 7), requested ahead of the first K/V tile - loads return in the order of their issue - and rounded to f16
+// (ggml-cpu.c:11037-11040) while that tile is on its way
 template <int D>
-__device__ __forceinline__ void load_q(f16x8 (&qf)[D / 16], const float *qp, int lhi) {
+struct q_row {
+    f32x4 x[D / 8];
+    __device__ __forceinline__ void request(const float *qp, int lhi) {
 #pragma unroll
-    for (int kk = 0; kk < D / 16; kk++) {   // rounded to f16 (ggml-cpu.c:11037-11040)
-        const f32x4 x0 = *(const f32x4 *)(qp + 16 * kk + 8 * lhi);
-        const f32x4 x1 = *(const f32x4 *)(qp + 16 * kk + 8 * lhi + 4);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            qf[kk][i] = (_Float16)x0[i];
-            qf[kk][4 + i] = (_Float16)x1[i];
+        for (int kk = 0; kk < D / 16; kk++) {
+            x[2 * kk] = *(const f32x4 *)(qp + 16 * kk + 8 * lhi);
+            x[2 * kk + 1] = *(const f32x4 *)(qp + 16 * kk + 8 * lhi + 4);
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
-}
+    __device__ __forceinline__ void convert(f16x8 (&qf)[D / 16]) const {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < D / 16; kk++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                qf[kk][i] = (_Float16)x[2 * kk][i];
+                qf[kk][4 + i] = (_Float16)x[2 * kk + 1][i];
+            }
+    }
+};
 __device__ __forceinline__ float alibi_slope(const fattn_args &a, int64_t head) {   // ggml-cpu.c:10998-11003
     if (a.max_bias <= 0.0f) return 1.0f;
     const unsigned h = (unsigned)head;
@@ -520,7 +531,8 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
     const int64_t iq = q0 + l32 < a.Nq ? q0 + l32 : a.Nq - 1;   // clamped: rows past Nq are computed and dropped
 
     f16x8 qf[D / 16];
-    load_q<D>(qf, (const float *)(a.q + iq * a.q_nb1 + head * a.q_nb2), lhi);
+    q_row<D> qr;
+    qr.request((const float *)(a.q + iq * a.q_nb1 + head * a.q_nb2), lhi);
     float slope = alibi_slope(a, head);
     asm volatile("" : "+v"(slope));   // kept in a vector register also where the head is uniform over the group: a scalar slope makes
                                       // the compiler build a second copy of the tile loop around "slope == 1", which then spills
@@ -549,13 +561,14 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
 
     stage_t st;
     u32x2 mnext[2][4];
-    auto prefetch = [&](int64_t kv0) {
-        st.fetch(a, hk, kv0, tid);
+    auto prefetch_mask = [&](int64_t kv0) {
         const bool vec_ok = mask_aligned && kv0 + FM_BC <= a.Nkv;
         fetch_mask<4>(mnext[0], mrow, vec_ok, kv0 + 4 * lhi, a.Nkv);
         fetch_mask<4>(mnext[1], mrow, vec_ok, kv0 + 32 + 4 * lhi, a.Nkv);
     };
-    if (kv_limit > 0) prefetch(0);
+    st.fetch(a, hk, 0, tid);   // also where the group will need no tile: behind a branch the compiler would wait for more than q
+    qr.convert(qf);
+    prefetch_mask(0);
     for (int64_t kv0 = 0; kv0 < kv_limit; kv0 += FM_BC) {
         __syncthreads();   // the previous tile has been consumed
         st.commit(sK, sVt, tid);
@@ -565,7 +578,10 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_fattn_mma(fattn_args a
 #pragma unroll
             for (int g = 0; g < 4; g++) mcur[u][g] = mnext[u][g];
         __syncthreads();
-        if (kv0 + FM_BC < kv_limit) prefetch(kv0 + FM_BC);
+        if (kv0 + FM_BC < kv_limit) {
+            st.fetch(a, hk, kv0 + FM_BC, tid);
+            prefetch_mask(kv0 + FM_BC);
+        }
 
         // scores of 64 cells for this lane's query: S[u][r] <-> cell kv0 + 32u + 8*(r/4) + 4*lhi + r%4
         f32x16 S[2];
@@ -643,7 +659,8 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
     const int64_t iq = q0 + l32 < a.Nq ? q0 + l32 : a.Nq - 1;   // clamped: rows past Nq are computed and dropped
 
     f16x8 qf[D / 16];
-    load_q<D>(qf, (const float *)(a.q + iq * a.q_nb1 + head * a.q_nb2), lhi);
+    q_row<D> qr;
+    qr.request((const float *)(a.q + iq * a.q_nb1 + head * a.q_nb2), lhi);
     const float slope = alibi_slope(a, head);
     const float scale = a.softcap != 0.0f ? a.scale / a.softcap : a.scale;
     const unsigned short *mrow = a.mask ? (const unsigned short *)(a.mask + iq * a.mask_nb1) : nullptr;
@@ -675,7 +692,9 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
         st.fetch(a, hk, kv0, tid);
         fetch_mask<4>(mnext, mrow, mask_aligned && kv0 + BC <= a.Nkv, kv0 + 32 * u + 4 * lhi, a.Nkv);
     };
-    if (!PX || kv_lo < kv_limit) prefetch(kv_lo);
+    st.fetch(a, hk, kv_lo, tid);   // also where the group will need no tile: behind a branch the compiler would wait for more than q
+    qr.convert(qf);
+    fetch_mask<4>(mnext, mrow, mask_aligned && kv_lo + BC <= a.Nkv, kv_lo + 32 * u + 4 * lhi, a.Nkv);
     for (int64_t kv0 = kv_lo; kv0 < kv_limit; kv0 += BC) {
         __syncthreads();   // the previous tile has been consumed
         st.commit(sK, sVt, tid);
@@ -929,7 +948,8 @@ __global__ void __launch_bounds__(256, 2) k_fattn_mma_dec(fattn_args a, int R, i
     const int64_t head = hk * R + (col_live ? col_head : 0);
 
     f16x8 qf[D / 16];
-    load_q<D>(qf, (const float *)(a.q + iq * a.q_nb1 + head * a.q_nb2), lhi);
+    q_row<D> qr;
+    qr.request((const float *)(a.q + iq * a.q_nb1 + head * a.q_nb2), lhi);
     const float slope = alibi_slope(a, head);
     const float scale = a.softcap != 0.0f ? a.scale / a.softcap : a.scale;
     const unsigned short *mrow = a.mask ? (const unsigned short *)(a.mask + iq * a.mask_nb1) : nullptr;
@@ -985,7 +1005,9 @@ __global__ void __launch_bounds__(256, 2) k_fattn_mma_dec(fattn_args a, int R, i
         }
         accumulate_pv<D, NDT>(o, S, sVt, h * NDT, u, l32, lhi);
     };
-    if (c_begin < c_end) prefetch(st0, mn0, c_begin);
+    st0.fetch(a, hk, c_begin, tid);   // (no range of cells is empty)
+    qr.convert(qf);
+    fetch_mask<4>(mn0, mrow, mask_aligned && c_begin + FM_BC <= a.Nkv, c_begin + 32 * u + 4 * lhi, a.Nkv);
     if (c_begin + FM_BC < c_end) prefetch(st1, mn1, c_begin + FM_BC);
     for (int64_t kv0 = c_begin; kv0 < c_end; kv0 += 2 * FM_BC) {
         tile(st0, mn0, kv0);
