@@ -11,6 +11,7 @@
 // into one long enough to fill the chip.  An optional residual is added in the epilogue.
 #include "ffn.hpp"
 #include "gemv_body.hpp"
+#include "gemv_row.hpp"
 
 #include <math.h>
 #include <stdlib.h>
@@ -301,6 +302,8 @@ int mi355_mul_mat_vec_q_multi(void *stream, int n_mats, const mi355_gemv_mat *ma
     hipStream_t s = (hipStream_t)stream;
     const int8_t *aq = (const int8_t *)act;
     const act_ds *ads = (const act_ds *)(aq + B * K);
+    if (n_mats == 1 && B == 1 && gemv_row_serves(mats[0].N, K))
+        return launch_gemv_row(s, mats[0].type, mats[0].W, aq, ads, mats[0].dst, mats[0].residual, mats[0].N, K);
     if (n_mats == 1) {
 #define MI355_SINGLE_LAUNCH(TY) launch_single_cols<TY>(rpw, B, s, b.it[0], (unsigned)groups, aq, ads, (int)K);
         MI355_WEIGHT_TYPE_SWITCH(mats[0].type, MI355_SINGLE_LAUNCH)

@@ -313,15 +313,25 @@ template <> struct wq<MI355_Q4_K> {
     static constexpr int CHUNK = 64;
     struct chunk { u32x4 q0, q1; float d, dmin, scA, mA, scB, mB; };
     struct act { u32x4 a0lo, a0hi, a1lo, a1hi; float d0, d1, ds0, ds1; };
-    static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &, int c) {
-        chunk w;
-        const int sb = c >> 2, g = c & 3;
-        const uint8_t *blk = row + sb * Q4_K_BYTES;
+    // what a chunk is loaded as: kept so while it is on its way, where decoding it at the load would wait for it
+    struct raw { u32x4 q0, q1, hdr; };
+    static __device__ __forceinline__ raw load_raw(const uint8_t *__restrict__ row, const row_layout &, int c) {
+        raw w;
+        const uint8_t *blk = row + (c >> 2) * Q4_K_BYTES;
+        const int g = c & 3;
         // header and both qs loads touch the same 128-byte lines from three instructions: ordinary
         // (temporal) loads, so the line is fetched from HBM once and the other two hit in cache
-        const u32x4 hdr = load16w(blk);   // d, dmin, 12 scale bytes: same address for the 4 lanes of a super-block
+        w.hdr = load16w(blk);   // d, dmin, 12 scale bytes: same address for the 4 lanes of a super-block
         w.q0 = load16w(blk + 16 + g * 32);
         w.q1 = load16w(blk + 32 + g * 32);
+        return w;
+    }
+    static __device__ __forceinline__ chunk decode(const raw &r, int c) {
+        chunk w;
+        const int g = c & 3;
+        const u32x4 hdr = r.hdr;
+        w.q0 = r.q0;
+        w.q1 = r.q1;
         w.d = half_bits_to_float((unsigned short)(hdr[0] & 0xFFFFu));
         w.dmin = half_bits_to_float((unsigned short)(hdr[0] >> 16));
         // all eight 6-bit (scale, min) pairs at once, branch-free (get_scale_min_k4, ggml-quants.c:631-638)
@@ -336,6 +346,7 @@ template <> struct wq<MI355_Q4_K> {
         w.mB = (float)((M >> (sh + 8)) & 0xFFu);
         return w;
     }
+    static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &L, int c) { return decode(load_raw(row, L, c), c); }
     static __device__ __forceinline__ act load_a(const int8_t *__restrict__ q, const act_ds *__restrict__ ds, int c) {
         act A;
         const int8_t *p = q + c * 64;      // activation blocks 2c (sub-block 2g) and 2c+1 (sub-block 2g+1)
@@ -432,20 +443,32 @@ template <> struct wq<MI355_Q6_K> {
     static constexpr int CHUNK = 32;
     struct chunk { u32x4 ql, qh; float d, scA, scB; int shA, shB; };
     struct act { u32x4 a0, a1; float d0, d1; int s0, s1; };
-    static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &L, int c) {
-        chunk w;
+    struct raw { u32x4 ql, qh; u32 scA, scB, d; };   // (see Q4_K)
+    static __device__ __forceinline__ raw load_raw(const uint8_t *__restrict__ row, const row_layout &L, int c) {
+        raw w;
         const int sb = c >> 3, cc = c & 7, hf = cc >> 2, r = cc & 3;
         const int l0 = 16 * (r & 1), qa = r >> 1;
         w.ql = load_stream16w(row + sb * 128 + cc * 16);
         w.qh = load_stream16w(row + L.off_b + sb * 64 + hf * 32 + l0);
-        const int8_t *sc = (const int8_t *)(row + L.off_c + sb * 16 + hf * 8 + (l0 >> 4));
-        w.scA = (float)sc[2 * qa];
-        w.scB = (float)sc[2 * qa + 4];
-        w.d = half_bits_to_float(*(const unsigned short *)(row + L.off_d + sb * 2));
+        const uint8_t *sc = row + L.off_c + sb * 16 + hf * 8 + (l0 >> 4);
+        w.scA = sc[2 * qa];
+        w.scB = sc[2 * qa + 4];
+        w.d = *(const unsigned short *)(row + L.off_d + sb * 2);
+        return w;
+    }
+    static __device__ __forceinline__ chunk decode(const raw &r, int c) {
+        chunk w;
+        const int qa = (c & 3) >> 1;
+        w.ql = r.ql;
+        w.qh = r.qh;
+        w.scA = (float)(int)(signed char)r.scA;
+        w.scB = (float)(int)(signed char)r.scB;
+        w.d = half_bits_to_float((unsigned short)r.d);
         w.shA = 2 * qa;
         w.shB = 2 * qa + 4;
         return w;
     }
+    static __device__ __forceinline__ chunk load_w(const uint8_t *__restrict__ row, const row_layout &L, int c) { return decode(load_raw(row, L, c), c); }
     static __device__ __forceinline__ act load_a(const int8_t *__restrict__ q, const act_ds *__restrict__ ds, int c) {
         act A;
         const int sb = c >> 3, cc = c & 7, hf = cc >> 2, r = cc & 3;
@@ -487,10 +510,11 @@ template <> struct wq<MI355_Q6_K> {
 // The group's copy of a quantized activation (NCOLS rows of K levels, then their {d, sum} pairs) in LDS: request() before the first weight
 // loads, commit() behind them.  A wave's loads return in the order they were issued, so a copy requested behind the weights waits for all of
 // them, and no dot product starts before the last weight has arrived.
-template <int NCOLS, int THREADS>
+// ALL: no row is longer than KMAX.
+template <int NCOLS, int THREADS, int KMAX = 4096, bool ALL = false>
 struct act_copy {
-    // pieces per thread requested up front (rows of 4096; longer ones take the rest behind the weights)
-    static constexpr int NQ = (NCOLS * 4096 / 16 + THREADS - 1) / THREADS, ND = (NCOLS * 4096 / 32 + THREADS - 1) / THREADS;
+    // pieces per thread requested up front (rows of KMAX; longer ones take the rest behind the weights)
+    static constexpr int NQ = (NCOLS * KMAX / 16 + THREADS - 1) / THREADS, ND = (NCOLS * KMAX / 32 + THREADS - 1) / THREADS;
     u32x4 q[NQ];
     u32x2 d[ND];
     __device__ __forceinline__ void request(const int8_t *aq, const act_ds *ads, int K) {
@@ -520,6 +544,7 @@ struct act_copy {
             const int i = (int)threadIdx.x + p * THREADS;
             *(u32x2 *)(s_ds + (i < nd ? i : nd - 1) * 8) = d[p];
         }
+        if constexpr (ALL) return;
         for (int i = (int)threadIdx.x + NQ * THREADS; i < nq; i += THREADS) *(u32x4 *)(s_act + i * 16) = load16(aq + (int64_t)i * 16);
         for (int i = (int)threadIdx.x + ND * THREADS; i < nd; i += THREADS) *(u32x2 *)(s_ds + i * 8) = *(const u32x2 *)(ads + i);
     }

@@ -1044,3 +1044,31 @@ def test_a_short_last_slice_costs_no_round():
     for N, K, B, slices in ((2813, 2080, 287, 4), (4755, 2176, 144, 4), (5309, 3392, 231, 6), (10772, 4640, 65, 6), (2477, 4096, 626, 5), (12317, 4096, 54, 5),
                             (2537, 13792, 527, 9)):
         assert int(lib.mi355_mul_mat_q_ws_bytes(N, K, B)) == slices * N * B * 4, (N, K, B)
+
+
+@pytest.mark.parametrize("name,t", list(orc.WEIGHT_TYPES.items()))
+@pytest.mark.parametrize("N,K", [(1, 256), (9, 4096 + 256), (2047, 1024), (2049, 2048), (33, 14336), (1030, 16384 + 512), (17, 32768), (8200, 4096)])
+def test_one_row_launch_has_the_bits_of_the_multi_matrix_one(dev, name, t, N, K):
+    """one row against one matrix (a wave per weight row, several steps of it in flight): the sums of the launch that walks it step by step, residual in place"""
+    import torch
+    import mi355
+    from mi355 import llama_graph as lg
+    lib = mi355.load()
+    if t in orc.WEIGHT_TYPES.values() and (K // 256) % 8 and name in ("q6_K", "iq4_xs"):
+        K = K // 2048 * 2048 or 2048      # rows of whole 16 bytes, as the launch of several matrices reads them
+    if name not in ("q4_K", "q5_K", "q6_K", "iq4_xs"):
+        K += 64                           # a last step of one or two blocks
+    gen = torch.Generator(device=dev).manual_seed(N + K)
+    W = mi355.upload_weights(t, lg.random_quantized(t, N, K, torch.device(dev), gen))
+    x = torch.randn(1, K, device=dev, generator=gen)
+    act = mi355.quantize_act(x)
+    res = torch.randn(N, device=dev, generator=gen)
+    for with_res in (False, True):
+        outs = [res.clone() for _ in range(3)]
+        arr = (mi355.GemvMat * 2)()
+        for i, o in enumerate(outs[:2]):
+            arr[i].type, arr[i].W, arr[i].N, arr[i].dst, arr[i].dst_stride, arr[i].residual = t, W.data_ptr(), N, o.data_ptr(), N, o.data_ptr() if with_res else None
+        mi355.check(lib.mi355_mul_mat_vec_q_multi(None, 2, arr, act.data_ptr(), K, 1))
+        arr[0].dst, arr[0].residual = outs[2].data_ptr(), outs[2].data_ptr() if with_res else None
+        mi355.check(lib.mi355_mul_mat_vec_q_multi(None, 1, arr, act.data_ptr(), K, 1))
+        assert bool(torch.isfinite(outs[2]).all()) and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
