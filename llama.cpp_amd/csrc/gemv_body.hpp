@@ -31,7 +31,7 @@ struct gemv_rope {
     int D, n_dims;
     float theta_scale, freq_scale, ext_factor, attn_factor, corr0, corr1;
     const float2 *table;     // {cos, sin} of every (activation row, pair) from k_rope_table (same bits), or null: each wave works out its own
-    const float *nx, *nw;    // NORM: the f32 row to normalise and the norm weights (the group quantizes it into its LDS copy itself)
+    const float *nx, *nw;    // the launches with the norm: the f32 row to normalise and the norm weights (the group quantizes it into its LDS copy itself)
     float neps;
 };
 
@@ -64,13 +64,13 @@ struct gemv_batch {
 // waves read it from there; otherwise every wave reads it from memory.  On the 14336 x 4096 Q4_K product the activation
 // reads of the 7168 waves (36 MB from L2) outweighed the 33 MB of weights and competed with them: 8.7 -> 7.9 us with the
 // copy in LDS.  The copy is requested ahead of the first step's weights: loads return in the order of their issue.
-template <int TYPE, int NCOLS, int RPW, bool QKV = false, bool COH = false, bool LDSA = false, bool NORM = false, int WAVES = 4>
+template <int TYPE, int NCOLS, int RPW, bool QKV = false, bool COH = false, bool LDSA = false>
 __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const int8_t *__restrict__ aq,
                                           const act_ds *__restrict__ ads, int K, const gemv_rope *rp = nullptr, uint8_t *s_act = nullptr) {
     typedef wq<TYPE> T;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t row0 = ((int64_t)group * WAVES + wave) * RPW;
+    const int64_t row0 = ((int64_t)group * 4 + wave) * RPW;
     const bool wave_live = row0 < m.N;   // uniform over the wave
     if (!LDSA && !wave_live) return;     // with the copy in LDS a wave without rows still takes its share of the copy
 
@@ -119,24 +119,13 @@ __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const i
     };
     const int c_first = lane < nchunks ? lane : nchunks - 1;
     if constexpr (LDSA) {
-        if constexpr (NORM) {   // RMS_NORM -> MUL -> Q8_1 of the one activation row straight into the group's LDS copy
-            __shared__ float s_norm[4];
-            norm_row<WAVES> row;
-            row.request(rp->nx, rp->nw, K);
-            __builtin_amdgcn_sched_barrier(0);
+        act_copy<NCOLS, 256> copy;
+        copy.request(aq, ads, K);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < RPW; r++) w_first[r] = T::load_w(rows[r], L, c_first);
-            if constexpr (QKV) rotation();
-            row.finish(s_act, K, rp->neps, s_norm);
-        } else {
-            act_copy<NCOLS, 64 * WAVES> copy;
-            copy.request(aq, ads, K);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int r = 0; r < RPW; r++) w_first[r] = T::load_w(rows[r], L, c_first);
-            if constexpr (QKV) rotation();
-            copy.commit(s_act, aq, ads, K);
-        }
+        for (int r = 0; r < RPW; r++) w_first[r] = T::load_w(rows[r], L, c_first);
+        if constexpr (QKV) rotation();
+        copy.commit(s_act, aq, ads, K);
         __syncthreads();
         if (!wave_live) return;
         aq = (const int8_t *)s_act;

@@ -21,19 +21,113 @@ __global__ void __launch_bounds__(256) k_gemv_qkv(gemv_batch b, const int8_t *__
 #undef MI355_BODY
 }
 
-// ... with the RMS norm of the layer input computed by every group for itself (one activation row).  Eight waves: half the groups that do so of four (8B shapes: a token
-// 1821 us with four, 1819 with eight).
-constexpr int QN_WAVES = 8;
-__global__ void __launch_bounds__(64 * QN_WAVES) k_gemv_qkv_norm(gemv_batch b, int K, gemv_rope rp) {
-    const int g = blockIdx.x;
-    int i = 0;
+// ... with the RMS norm of the layer input computed by every group for itself (one activation row of at most 4096 elements).
+//
+// A launch of 13 MB takes 4.6 us in a chain of launches with the row already quantized; what it takes beyond that is the norm's dependent instructions and trips to memory that a wave
+// makes one after the other.  So what the first requests need comes in arguments that are in registers when a wave starts (the first fourteen words), and where finished
+// rows go and how they are rotated is read behind the requests for the weights: left to itself the compiler moves all those reads - the matrix's entry by its
+// index, the rotation and the cell by what that holds - ahead of the branch over the types, and each waits for the one before it.  `late` is the index of the
+// matrix, opaque from where those reads may begin.  Four waves and eight rows per group: the 768 groups of 8B shapes are three to every compute unit (eight waves are
+// 384: two norms at a time on half of them, 7.2 us against 6.8; sixteen and 192 groups 9.2 against 8.4 in the previous form).
+// 8B shapes, us in the chain: 8.4 with everything read first, 64-bit divisions for the head and four elements per lane and block piece; 6.8 now (a token 1608 -> 1553).
+constexpr int QN_WAVES = 4;
+struct qkv_rest {
+    gemv_batch b;
+    gemv_rope rp[1];
+};
+template <int TYPE, bool TABLE>
+__device__ __forceinline__ void qkv_norm_body(const uint8_t *__restrict__ W, int64_t row0, int64_t last_row, const float *__restrict__ nx, const float *__restrict__ nw, int K,
+                                              const qkv_rest &rest, int item) {
+    typedef wq<TYPE> T;
+    typedef late_chunk<TYPE> G;
+    constexpr int STEPS = 64 / T::CHUNK;   // steps of 64 chunks in a row of 4096
+    const int lane = threadIdx.x & 63;
+    const row_layout L = make_row_layout(TYPE, K);
+    const int nchunks = K / T::CHUNK;
+    const uint8_t *rows[2];
 #pragma unroll
-    for (int j = 1; j < 3; j++)
-        if (g >= b.it[j].first_group) i = j;
-    const gemv_item &m = b.it[i];
-    const int group = g - m.first_group;
-#define MI355_BODY(TY) gemv_body<TY, 1, 2, true, false, true, true, QN_WAVES>(m, group, nullptr, nullptr, K, &rp, s_act_dyn);
-    MI355_WEIGHT_TYPE_SWITCH(m.type, MI355_BODY)
+    for (int r = 0; r < 2; r++) rows[r] = W + (row0 + r < last_row ? row0 + r : last_row) * L.row_bytes;   // rows past the end repeat the last one and are not stored
+    __shared__ float s_norm[4];
+    norm_row<QN_WAVES> row;
+    row.request(nx, nw, K);
+    __builtin_amdgcn_sched_barrier(0);
+    typename G::raw w[STEPS][2];
+#pragma unroll
+    for (int p = 0; p < STEPS; p++)
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int c = p * 64 + lane;
+            w[p][r] = G::load(rows[r], L, c < nchunks ? c : nchunks - 1);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    int late = item;
+    asm volatile("" : "+s"(late));
+    const gemv_item &m = rest.b.it[late];
+    const gemv_rope &R = rest.rp[late >> 2];   // (0)
+    // one trip for what the rotation and the cell are looked up with, one for them, behind the weights (neither is waited for ahead of the sums; where a launch
+    // has none of them some word of the row is read in their place)
+    const int D = R.D, n_dims = R.n_dims, epi = m.epi;
+    const int32_t *cells = R.cells;
+    const float2 *table = R.table;
+    const float eps = R.neps;
+    float *dst = m.dst;
+    const int64_t nb1 = m.nb1, nb2 = m.nb2;
+    asm volatile("" ::"s"(D), "s"(n_dims), "s"(epi), "s"(cells), "s"(table), "s"(eps), "s"(dst), "s"(nb1), "s"(nb2));
+    const u32 head = (u32)row0 / (u32)D;   // (2^31 rows of 1024 elements and more do not fit the memory)
+    const int d = (int)((u32)row0 - head * (u32)D);
+    const bool turned = (epi == EPI_ROPE || epi == EPI_ROPE_CACHE) && d < n_dims;
+    int zero;   // an offset the compiler does not know to be the same in all lanes: it would wait for a uniform value at once, to keep it in a scalar register
+    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+    float2 turn;
+    if constexpr (TABLE) turn = (turned ? table + (d >> 1) : (const float2 *)nx)[zero];
+    else if (turned) rope_coeffs(R, R.pos[0], d >> 1, turn.x, turn.y);
+    const int cell = (epi == EPI_ROPE_CACHE || epi == EPI_CACHE ? cells : (const int32_t *)nx)[zero];
+    __builtin_amdgcn_sched_barrier(0);
+    row.finish(s_act_dyn, K, eps, s_norm);
+    __syncthreads();
+    float acc[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int p = 0; p < STEPS; p++) {
+        const int c = p * 64 + lane;
+        if (p * 64 >= nchunks) break;   // uniform
+        const typename T::act A = T::load_a((const int8_t *)s_act_dyn, (const act_ds *)(s_act_dyn + K), c < nchunks ? c : nchunks - 1);
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const typename T::chunk now = G::decode(w[p][r], c);
+            const float sum = T::accumulate(acc[r], now, A, T::dots(now, A));
+            acc[r] = c < nchunks ? sum : acc[r];
+        }
+    }
+    const float s0 = wave_sum_dpp(acc[0]), s1 = wave_sum_dpp(acc[1]);
+    if (lane == 0 && row0 < last_row) {   // an even number of rows
+        float y0 = s0, y1 = s1;
+        if (turned) rope_apply(turn.x, turn.y, s0, s1, y0, y1);
+        if (epi == EPI_ROPE || epi == EPI_STORE) {
+            float *o = dst + row0;
+            o[0] = y0;
+            o[1] = y1;
+        } else {
+            _Float16 *o = (_Float16 *)((uint8_t *)dst + (int64_t)cell * nb1 + (int64_t)head * nb2) + d;
+            o[0] = (_Float16)y0;
+            o[1] = (_Float16)y1;
+        }
+    }
+}
+// first1, first2: first groups of the second and third matrix (`groups`, the number of all, where there is none); forms: five bits each for the types, from bit 15 three each for half
+// the rows of a matrix's last group less one, from bit 24 K / 1024
+template <bool TABLE>   // the rotations come from a table
+__global__ void __launch_bounds__(64 * QN_WAVES) k_gemv_qkv_norm(const uint8_t *__restrict__ W0, const uint8_t *__restrict__ W1, const uint8_t *__restrict__ W2,
+                                                                 const float *__restrict__ nx, const float *__restrict__ nw, int first1, int first2, int groups, u32 forms, qkv_rest rest) {
+    const int g = blockIdx.x;
+    const int item = g >= first2 ? 2 : g >= first1 ? 1 : 0;
+    const uint8_t *W = item == 0 ? W0 : item == 1 ? W1 : W2;
+    const int group = g - (item == 0 ? 0 : item == 1 ? first1 : first2);
+    const int left = (item == 0 ? first1 : item == 1 ? first2 : groups) - g;   // groups of the matrix from this one on
+    const int64_t row0 = ((int64_t)group * QN_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * 2;
+    const int64_t last_row = (int64_t)(group + left - 1) * (2 * QN_WAVES) + ((forms >> (15 + 3 * item)) & 7) * 2 + 1;
+    const int K = (int)(forms >> 24) << 10;
+#define MI355_BODY(TY) qkv_norm_body<TY, TABLE>(W, row0, last_row, nx, nw, K, rest, item);
+    MI355_WEIGHT_TYPE_SWITCH((int)((forms >> (5 * item)) & 31), MI355_BODY)   // uniform over the group
 #undef MI355_BODY
 }
 
@@ -175,7 +269,15 @@ static int vec_q_rope_impl(void *stream, int n_mats, const mi355_gemv_rope_mat *
             MI355_LAUNCH(k_gemv_qkv_norm_qc, dim3((unsigned)groups), dim3(512), (size_t)K + K / 4, s, b, (int)K, rp);
             return launch_status("k_gemv_qkv_norm_qc");
         }
-        MI355_LAUNCH(k_gemv_qkv_norm, dim3((unsigned)groups), dim3(64 * QN_WAVES), (size_t)K + K / 4, s, b, (int)K, rp);
+        u32 forms = 0;
+        for (int i = 0; i < n_mats; i++) forms |= (u32)b.it[i].type << (5 * i) | (u32)((b.it[i].N / 2 - 1) % QN_WAVES) << (15 + 3 * i);
+        forms |= (u32)(K / 1024) << 24;
+        const qkv_rest rest = {b, {rp}};
+        const int first1 = n_mats > 1 ? b.it[1].first_group : (int)groups, first2 = n_mats > 2 ? b.it[2].first_group : (int)groups;
+#define MI355_QN_ARGS dim3((unsigned)groups), dim3(64 * QN_WAVES), (size_t)K + K / 4, s, b.it[0].W, b.it[1].W, b.it[2].W, nx, nw, first1, first2, (int)groups, forms, rest
+        if (table) MI355_LAUNCH(k_gemv_qkv_norm<true>, MI355_QN_ARGS);
+        else MI355_LAUNCH(k_gemv_qkv_norm<false>, MI355_QN_ARGS);
+#undef MI355_QN_ARGS
         return launch_status("k_gemv_qkv_norm");
     }
     rp.nx = rp.nw = nullptr; rp.neps = 0.0f;

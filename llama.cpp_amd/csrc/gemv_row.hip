@@ -9,23 +9,10 @@
 #include "qdot.hpp"
 #include "gemv_row.hpp"
 
-#include <type_traits>
-
 namespace mi355 {
 
 extern __shared__ __attribute__((aligned(16))) uint8_t s_gr[];
 
-// a chunk as it is loaded, decoded where it is used (types whose scales take no arithmetic have one form)
-template <int TYPE, class = void> struct gr_chunk {
-    typedef typename wq<TYPE>::chunk raw;
-    static __device__ __forceinline__ raw load(const uint8_t *row, const row_layout &L, int c) { return wq<TYPE>::load_w(row, L, c); }
-    static __device__ __forceinline__ raw decode(const raw &r, int) { return r; }
-};
-template <int TYPE> struct gr_chunk<TYPE, std::void_t<typename wq<TYPE>::raw>> {
-    typedef typename wq<TYPE>::raw raw;
-    static __device__ __forceinline__ raw load(const uint8_t *row, const row_layout &L, int c) { return wq<TYPE>::load_raw(row, L, c); }
-    static __device__ __forceinline__ typename wq<TYPE>::chunk decode(const raw &r, int c) { return wq<TYPE>::decode(r, c); }
-};
 // steps in flight: four, two of the types whose chunks take the most registers or the most loads (4096 x 14336, four / two: Q5_K 14.3 / 10.9 us, IQ4_XS 10.6 / 9.2, Q6_K 10.8 / 10.9 alone
 // and 48.5 / 48.0 for the layer)
 template <int TYPE> constexpr int gr_steps() { return TYPE == MI355_Q6_K || TYPE == MI355_Q5_K || TYPE == MI355_IQ4_XS ? 2 : 4; }
@@ -45,7 +32,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_gemv_row(const uint8_t *__restri
     act_copy<1, 64 * WAVES, KMAX, true> copy;
     copy.request(aq, ads, K);
     __builtin_amdgcn_sched_barrier(0);
-    typedef gr_chunk<TYPE> G;
+    typedef late_chunk<TYPE> G;
     typename G::raw w[STEPS];
 #pragma unroll
     for (int p = 0; p < STEPS; p++) {

@@ -81,43 +81,77 @@ __device__ __forceinline__ float rms_norm_scale(const f32x4 (&v)[NV], int64_t k,
     return 1.0f / sqrtf(add_rn(ss / (float)k, eps));
 }
 
-// RMS_NORM -> MUL -> Q8_1 of one row of at most 4096 elements (a multiple of 1024) into a group's LDS copy, in two parts: request() ahead of the group's first weight
-// loads - a wave's loads return in the order of their issue - and finish() behind them.  Same bits as rms_norm_quant_row: 256 threads' sums of squares of sixteen
-// elements each (further waves repeat the first four's, their sums are not used), then every thread quantizes its share.  WAVES: 4 or 8.
+// Q8_1 of eight neighbouring values per lane over aligned groups of four lanes into a row's LDS copy (levels, then {d, sum} of every block); e0 = the lane's first element.
+// Same levels and scales as quantize_block_lane: of the work per block only the maximum and the sum are more than one lane's, and a third of the instructions per element
+// remain of four lanes doing what eight did twice.
+__device__ __forceinline__ void quantize_block_lane8(const f32x4 (&v)[2], int8_t *__restrict__ qrow, act_ds *__restrict__ srow, int e0) {
+    float amax = fmaxf(fabsf(v[0][0]), fabsf(v[1][0]));
+#pragma unroll
+    for (int i = 1; i < 4; i++) amax = fmaxf(amax, fmaxf(fabsf(v[0][i]), fabsf(v[1][i])));
+    amax = lanes_max<4>(amax);
+    float d, id;
+    q8_scale(amax, d, id);
+    u32x2 packed;
+    int sum = 0;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        u32 q[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) q[i] = (u32)q8_level(v[j][i], id);
+        packed[j] = __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u) | __builtin_amdgcn_perm(q[3], q[2], 0x04000c0cu);   // the low bytes in order
+        sum = dot4((int)packed[j], 0x01010101, sum);
+    }
+    sum = lanes_sum_i<4>(sum);
+    *(u32x2 *)(qrow + e0) = packed;
+    if ((e0 & 31) == 0) {
+        act_ds o;
+        o.d = half_bits_to_float(float_to_half_bits(d));
+        o.sum = sum;
+        srow[e0 >> 5] = o;
+    }
+}
+
+// RMS_NORM -> MUL -> Q8_1 of one row of at most 4096 elements (a multiple of 1024) into a group's LDS copy, in two parts: request() ahead of the group's
+// first weight loads - a wave's loads return in the order of their issue - and finish() behind them.  Same bits as rms_norm_quant_row: the first four waves form its
+// sum in its order, then every thread quantizes its share, eight elements at a time.  WAVES: 4 or 8.
 template <int WAVES>
 struct norm_row {
-    static constexpr int NQ = 16 / WAVES;   // pieces the thread quantizes
-    f32x4 v[4], w[NQ];
+    static constexpr int NP = 8 / WAVES;
+    f32x4 v[4], own[NP][2], w[NP][2];
     static __device__ __forceinline__ int element(int it) { return (it * 256 + (int)(threadIdx.x & 255)) * 4; }
-    static __device__ __forceinline__ int first() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)) * NQ; }
+    static __device__ __forceinline__ int first(int p) { return (p * 64 * WAVES + (int)threadIdx.x) * 8; }
     __device__ __forceinline__ void request(const float *__restrict__ x, const float *__restrict__ nw, int K) {
         // pieces past the end repeat others, and nothing uses them: a branch around a load would let the compiler move it to where its value is needed
 #pragma unroll
         for (int it = 0; it < 4; it++) v[it] = *(const f32x4 *)(x + (element(it) < K ? element(it) : element(0)));
 #pragma unroll
-        for (int j = 0; j < NQ; j++) {
-            const int e = element(first() + j);
-            w[j] = *(const f32x4 *)(nw + (e < K ? e : element(0)));
+        for (int p = 0; p < NP; p++) {
+            const int e0 = first(p), at = e0 < K ? e0 : 0;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                own[p][j] = *(const f32x4 *)(x + at + 4 * j);
+                w[p][j] = *(const f32x4 *)(nw + at + 4 * j);
+            }
         }
     }
     __device__ __forceinline__ void finish(uint8_t *s_act, int K, float eps, float *sh) {
 #pragma unroll
         for (int it = 1; it < 4; it++)
             if (it * 1024 >= K) v[it] = f32x4{0.f, 0.f, 0.f, 0.f};   // uniform
-        const float scale = rms_norm_scale<4>(v, K, eps, sh);
-        int8_t *qplane = (int8_t *)s_act;
+        const float scale = rms_norm_scale<4>(v, K, eps, sh);   // (further waves repeat the first four's sums, which are not used: a branch, see request())
 #pragma unroll
-        for (int j = 0; j < NQ; j++) {
-            const int it = first() + j;
-            if (it * 1024 >= K) break;   // uniform
-            f32x4 o;
+        for (int p = 0; p < NP; p++) {
+            const int e0 = first(p);
+            if (e0 >= K) return;   // uniform over the wave
+            f32x4 o[2];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float xv = first() ? v[(NQ & 3) + j][i] : v[j][i];   // four waves: always the thread's piece j
-                o[i] = xv * scale;
-                o[i] = o[i] * w[j][i];
-            }
-            quantize_block_lane(o, true, qplane, (act_ds *)(qplane + K), 0, K, element(it));
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    o[j][i] = own[p][j][i] * scale;
+                    o[j][i] = o[j][i] * w[p][j][i];
+                }
+            quantize_block_lane8(o, (int8_t *)s_act, (act_ds *)(s_act + K), e0);
         }
     }
 };

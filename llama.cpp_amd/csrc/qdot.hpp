@@ -13,6 +13,7 @@
 // integer dots, so what is checked bit-for-bit is what ships.
 #pragma once
 
+#include <type_traits>
 #include "common.hpp"
 
 namespace mi355 {
@@ -629,5 +630,18 @@ __device__ __forceinline__ float weight_value(const uint8_t *__restrict__ row, c
         return half_bits_to_float(dh) * (float)sc * (float)((nib | (hi << 4)) - 32);
     }
 }
+
+// A chunk as it is loaded, decoded where it is used: arithmetic on what was loaded, written beside the load, is moved ahead of the next barrier and waits there for the weights
+// (types whose scales take no arithmetic have one form)
+template <int TYPE, class = void> struct late_chunk {
+    typedef typename wq<TYPE>::chunk raw;
+    static __device__ __forceinline__ raw load(const uint8_t *row, const row_layout &L, int c) { return wq<TYPE>::load_w(row, L, c); }
+    static __device__ __forceinline__ raw decode(const raw &r, int) { return r; }
+};
+template <int TYPE> struct late_chunk<TYPE, std::void_t<typename wq<TYPE>::raw>> {
+    typedef typename wq<TYPE>::raw raw;
+    static __device__ __forceinline__ raw load(const uint8_t *row, const row_layout &L, int c) { return wq<TYPE>::load_raw(row, L, c); }
+    static __device__ __forceinline__ typename wq<TYPE>::chunk decode(const raw &r, int c) { return wq<TYPE>::decode(r, c); }
+};
 
 }  // namespace mi355

@@ -296,7 +296,7 @@ def test_qkv_rope_store_equals_three_launch_sequence(dev, B, tq, tk, tv):
     assert kc1.abs().sum().item() > 0 and vc1.abs().sum().item() > 0
 
 
-@pytest.mark.parametrize("K,H,HK,D,n_dims", [(1024, 4, 2, 64, 64), (3072, 5, 1, 128, 32), (4096, 32, 8, 128, 128)])
+@pytest.mark.parametrize("K,H,HK,D,n_dims", [(1024, 4, 2, 64, 64), (2048, 3, 1, 14, 10), (3072, 5, 1, 128, 32), (4096, 32, 8, 128, 128)])
 def test_qkv_launch_with_norm_and_rope_table_equals_separate_launches(dev, K, H, HK, D, n_dims):
     """one token: norm, projections, rotations from the table and the KV store in one launch, against the norm launch and the launch that works out its own rotations"""
     import torch
