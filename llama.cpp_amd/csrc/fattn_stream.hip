@@ -56,9 +56,9 @@ __device__ __forceinline__ void fs_init(fs_state &S) {
 // q of the group's four heads, 512 values, eight per lane (head lane / 16, elements 8 (lane % 16) .. + 7; zeros past the R heads): requested ahead of the transfers,
 // because a wave's loads return in the order of their issue.  (Every lane loading all 128 values of head lane % 4 behind the first tiles came to a third of a wave's
 // instructions over one tile, and none of them could run before those tiles had landed.)
-__device__ __forceinline__ void fs_request_q(const fattn_args &a, int64_t head0, int R, int lane, f32x4 (&x)[2]) {
+__device__ __forceinline__ void fs_request_q(const uint8_t *__restrict__ q, size_t q_nb2, int64_t head0, int R, int lane, f32x4 (&x)[2]) {
     const int h = lane >> 4;
-    const float *qp = (const float *)(a.q + (head0 + (h < R ? h : 0)) * a.q_nb2) + (lane & 15) * 8;
+    const float *qp = (const float *)(q + (head0 + (h < R ? h : 0)) * q_nb2) + (lane & 15) * 8;
     x[0] = *(const f32x4 *)qp;
     x[1] = *(const f32x4 *)(qp + 4);
 }
@@ -129,11 +129,12 @@ __device__ __forceinline__ void fs_slopes(const fattn_args &a, int64_t head0, fl
 // The soft-max update of the state with one tile's raw scores (q . k of this lane's cell and the four heads), and P^T (head, cell)
 // as f16 into the wave's 512 bytes of LDS at p_wr (= base + 2 * lane), where fs_output reads it back as the A operand.  LDS serves a
 // wave's operations in order: those reads see these writes, and the next tile's writes come after them.
+template <int NH = 4>   // heads the group has at most
 __device__ __forceinline__ void fs_softmax(const float (&raw)[4], float mv, float scale, float softcap, const float (&slope)[4], unsigned p_wr, fs_state &S) {
     constexpr float NEG = -FLT_MAX / 2;
     const bool valid = mv != -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
+    for (int r = 0; r < NH; r++) {
         float sc = raw[r] * scale;
         if (softcap != 0.0f) sc = softcap * tanhf(sc);
         sc += slope[r] * mv;
@@ -150,6 +151,7 @@ __device__ __forceinline__ void fs_softmax(const float (&raw)[4], float mv, floa
     }
 }
 // Scores of one tile (kc: the 16 chunks of this lane's K row), then fs_softmax.
+template <int NH = 4>
 __device__ __forceinline__ void fs_scores(const u32 (&qv)[FS_D / 2], const u32x4 (&kc)[16], float mv, float scale, float softcap, const float (&slope)[4],
                                           unsigned p_wr, fs_state &S) {
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
@@ -164,7 +166,7 @@ __device__ __forceinline__ void fs_scores(const u32 (&qv)[FS_D / 2], const u32x4
     float raw[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) raw[r] = s0[r] + s1[r];
-    fs_softmax(raw, mv, scale, softcap, slope, p_wr, S);
+    fs_softmax<NH>(raw, mv, scale, softcap, slope, p_wr, S);
 }
 // This lane's offset inside a row-major V tile for the transposing reads of fs_output: lane l' = lane % 16 of its 16-lane group
 // g points at row c0 + l' / 4, elements 16 g + 4 (l' % 4) .. + 3
@@ -332,7 +334,7 @@ __global__ void __launch_bounds__((ONE ? FS_WAVES_ONE : FS_WAVES) * 64, 1) k_fat
     const int hr = lane & 3;
     f32x4 qx[2];
     u32x4 mc[MT / 8];
-    fs_request_q(a, hk * R, R, lane, qx);
+    fs_request_q(a.q, a.q_nb2, hk * R, R, lane, qx);
     fs_request_mask<MT>(a, c_begin, n, lane, mc);
     asm volatile("" ::: "memory");   // the loads are not to be moved behind the transfers
     __builtin_amdgcn_sched_barrier(0);
@@ -697,7 +699,7 @@ __global__ void __launch_bounds__(((ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK
     const int hr = lane & 3;
     f32x4 qx[2];
     u32x4 mc[MT / 8];
-    fs_request_q(a, hk * R, R, lane, qx);
+    fs_request_q(a.q, a.q_nb2, hk * R, R, lane, qx);
     fs_request_mask<MT>(a, c_begin, n, lane, mc);
     asm volatile("" ::: "memory");   // the loads are not to be moved behind the transfers
     __builtin_amdgcn_sched_barrier(0);
@@ -779,65 +781,70 @@ __global__ void __launch_bounds__(((ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK
 }
 
 // ---- short caches: at most 512 cells, one launch -------------------------------------------------------------------------------
-// Two groups per kv head, one for each half of the output elements (PARTS), one wave per 64-cell tile (up to eight).  Nothing here is bound by bytes: the time is one trip to memory
-// plus the arithmetic of one tile, so a wave requests everything at once - its K and V tiles as coalesced 16-byte loads into
-// registers (four whole rows per instruction), q, its mask value - and then passes first K, then V through its own 16 KiB of
-// LDS to bring them into operand form: K rows with their chunks XOR-ed across the banks, so that each lane reads back the row of
-// its cell; V row-major for the transposing reads.  (A lane loading its own K row directly would touch 64 cache lines per
-// instruction: measured 2.8 us per wave of the group.)  The waves' states meet in LDS; the group normalises and writes the output
-// (and its Q8_1 form where the next product wants it), so no second launch merges anything.
-// Both groups of a kv head form the same scores; a group then reads only its half of every V row.  In a model the cache comes from HBM and a
-// compute unit's own requests are what takes the time: 512 cells are 256 KiB for one group per kv head (12.0 us per layer, 8B model),
-// 192 KiB for one of two (10.4 us; K reaches the second one through L2), with the same bits.  A group takes a compute unit's LDS: with
-// more than 128 kv heads two groups each would take a second round (256 kv heads, 512 cells: 16.4 us with one group per head, 23.9 with two).
+// One wave per 64-cell tile (up to eight).  Nothing here is bound by bytes: the time is one trip to memory plus the arithmetic of one tile, so a wave requests
+// everything at once - its K and V tiles as coalesced 16-byte loads into registers (four whole rows per instruction), q, its mask value - and then passes first K, then V
+// through its own 16 KiB of LDS to bring them into operand form: K rows with their chunks XOR-ed across the banks, so that each lane reads back the row of its
+// cell; V row-major for the transposing reads.  (A lane loading its own K row directly would touch 64 cache lines per instruction: measured 2.8 us per wave of the group.)
+// The waves' states meet in LDS; the group normalises and writes the output (and its Q8_1 form where the next product wants it), so no second launch merges anything.
+// As many groups per kv head as leave one on every compute unit (a group takes one's LDS), with the same bits: all form the scores of their heads over all cells.
+//   PARTS = 2: a group for each half of the output elements, which reads only its half of every V row.  In a model the cache comes from HBM and a compute unit's own requests take
+//     their time: 512 cells are 256 KiB for one group per kv head, 192 KiB for one of two (K reaches the second one through L2).
+//   NH: query heads of a group.  The soft-max of a head is some 90 instructions of each wave.
+// 32 / 8 heads, 512 cells, us: one group per kv head 7.6, two 6.3, four (NH = 2) 5.9, eight (NH = 1) 5.8; 288 cells 7.1, 5.7, 5.2, 5.1.  A group too many costs a second round: 160 / 40 heads,
+// 512 cells 11.1 with NH = 1, 6.8 with 2, 7.4 with 4; 256 / 64 heads 11.2, 6.8, 7.4.  With 32-bit offsets and arguments in registers, a layer of the 8B model 45.9 -> 45.2, with one
+// head per group 44.3 (a token 1553 -> 1508).
 constexpr int FSS_MAX_WAVES = 8;
 
-template <int PARTS>
-__global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn_args a, int R) {
+// The arguments ahead of `a` are all that the requests need, and in registers when a wave starts (fourteen words): read from `a` they are two trips to memory, the second
+// behind the mask's.  cells: Nkv and, from bit 16, R.  A tile's rows are less than 2^30 bytes apart: 32-bit offsets from one scalar address per wave.
+template <int PARTS, int NH>
+__global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(const uint8_t *__restrict__ q, const uint8_t *__restrict__ k, const uint8_t *__restrict__ v,
+                                                                           const uint8_t *__restrict__ mask, u32 q_nb2, u32 k_nb1, u32 k_nb2, u32 v_nb1, u32 v_nb2, u32 cells,
+                                                                           fattn_args a) {
     static_assert(PARTS == 1 || PARTS == 2, "whole rows of V or halves");
     constexpr int DO = FS_D / PARTS, VIT = 16 / PARTS, VCH = 16 / PARTS;   // output elements of the group; V loads; 16-byte chunks of V per row
     __shared__ __attribute__((aligned(1024))) uint8_t tbuf[FSS_MAX_WAVES * FS_KT];
     __shared__ __attribute__((aligned(16))) unsigned short pbuf[FSS_MAX_WAVES][4][FS_TILE];
-    __shared__ float s_m[FSS_MAX_WAVES][4], s_l[FSS_MAX_WAVES][4];
-    __shared__ float s_o[FSS_MAX_WAVES][4][DO];
+    __shared__ float s_m[FSS_MAX_WAVES][NH], s_l[FSS_MAX_WAVES][NH];
+    __shared__ float s_o[FSS_MAX_WAVES][NH][DO];
     __shared__ __attribute__((aligned(16))) uint8_t qbuf[FSS_MAX_WAVES][FS_QLDS];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int n_waves = (int)(blockDim.x >> 6);
     const int64_t hk = blockIdx.x;
     const int part = (int)blockIdx.y;   // PARTS == 2: elements 64 part .. + 63 of the output
-    const int64_t c0 = (int64_t)wave * FS_TILE;
+    const int Nkv = (int)(cells & 0xFFFF), HR = (int)(cells >> 16), n_waves = (Nkv + FS_TILE - 1) / FS_TILE;
+    const int64_t head0 = hk * HR + NH * (int)blockIdx.z;
+    const int R = HR - NH * (int)blockIdx.z < NH ? HR - NH * (int)blockIdx.z : NH;   // heads of the group
+    const int c0 = wave * FS_TILE, last = Nkv - 1 - c0;   // last: the last cell from the tile's first
     const int rsub = lane >> 4, pos = lane & 15;
 
-    // q of the group's four heads (two coalesced loads per lane) and the mask value first, K and V behind them: loads return in the order of their issue
+    // q of the group's heads (two coalesced loads per lane) and the mask value first, K and V behind them: loads return in the order of their issue
     f32x4 qx[2];
-    fs_request_q(a, hk * R, R, lane, qx);
-    const int64_t cell = c0 + lane;
+    fs_request_q(q, q_nb2, head0, R, lane, qx);
     // (without a mask some word of q is read in its place: at a join of two paths the compiler would wait for everything)
-    const unsigned short *mrow = (const unsigned short *)(a.mask ? a.mask : a.q);
-    unsigned short mbits = mrow[!a.mask ? 0 : cell < a.Nkv ? cell : a.Nkv - 1];
+    const unsigned short *mrow = (const unsigned short *)(mask ? mask : q);
+    unsigned short mbits = mrow[!mask ? 0 : c0 + (lane < last ? lane : last)];
     __builtin_amdgcn_sched_barrier(0);
     // load i: rows 4i .. 4i + 3, lane -> row 4i + lane / 16, chunk lane % 16 (rows past the end repeat the last cell; their weights are zero)
     // (half rows of V: rows 8i .. 8i + 7, lane -> row 8i + lane / 8, chunk lane % 8 of the half)
     const int vsub = lane / VCH, vpos = lane % VCH + VCH * part;
     u32x4 kraw[16], vraw[VIT];
+    const uint8_t *kt = k + hk * (uint64_t)k_nb2 + (uint64_t)c0 * k_nb1, *vt = v + hk * (uint64_t)v_nb2 + (uint64_t)c0 * v_nb1;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-        int64_t cell = c0 + 4 * i + rsub;
-        if (cell >= a.Nkv) cell = a.Nkv - 1;
-        kraw[i] = load16(a.k + cell * a.k_nb1 + hk * a.k_nb2 + (pos << 4));
+        const int row = 4 * i + rsub < last ? 4 * i + rsub : last;
+        kraw[i] = load16(kt + (__umul24((u32)row, k_nb1) + (u32)(pos << 4)));
     }
 #pragma unroll
     for (int i = 0; i < VIT; i++) {
-        int64_t cell = c0 + (64 / VIT) * i + vsub;
-        if (cell >= a.Nkv) cell = a.Nkv - 1;
-        vraw[i] = load16(a.v + cell * a.v_nb1 + hk * a.v_nb2 + (vpos << 4));
+        const int at = (64 / VIT) * i + vsub, row = at < last ? at : last;
+        vraw[i] = load16(vt + (__umul24((u32)row, v_nb1) + (u32)(vpos << 4)));
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (!a.mask) mbits = 0;
-    if (cell >= a.Nkv) mbits = 0xFC00;   // -inf
+    if (!mask) mbits = 0;
+    if (lane > last) mbits = 0xFC00;   // -inf
     float slope[4];
-    fs_slopes(a, hk * R, slope);
+    fs_slopes(a, head0, slope);
     const float scale = a.softcap != 0.0f ? a.scale / a.softcap : a.scale;
     u32 qv[FS_D / 2];
     fs_spread_q(qx, R, lane, (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)&qbuf[wave][0], qv);
@@ -856,7 +863,7 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
     fs_state S;
     fs_init(S);
     const unsigned p_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned short *)&pbuf[wave][0][0];
-    fs_scores(qv, kc, half_bits_to_float(mbits), scale, a.softcap, slope, p_base + (unsigned)lane * 2, S);
+    fs_scores<NH>(qv, kc, half_bits_to_float(mbits), scale, a.softcap, slope, p_base + (unsigned)lane * 2, S);
 
     // V through the same bytes, row-major (the K rows are in registers)
 #pragma unroll
@@ -869,7 +876,7 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
 
     // ---- the waves' states meet in LDS
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
+    for (int r = 0; r < NH; r++) {
         const float L = wave_sum_dpp(S.lsum[r]);
         if (lane == 0) {
             s_m[wave][r] = S.m[r];
@@ -879,7 +886,7 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
         if constexpr (PARTS == 1) s_o[wave][r][64 + lane] = S.o1[r];
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < R * DO; idx += (int)blockDim.x) {   // whole waves: R * DO and the group size are multiples of 64
+    for (int idx = threadIdx.x; idx < R * DO; idx += n_waves * 64) {   // whole waves: R * DO and the group size are multiples of 64
         const int r = idx / DO, d = idx % DO;
         float M = s_m[0][r];
         for (int w = 1; w < n_waves; w++) M = fmaxf(M, s_m[w][r]);
@@ -889,7 +896,7 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(fattn
             L += s_l[w][r] * f;
             O += s_o[w][r][d] * f;
         }
-        const int64_t head = hk * R + r;
+        const int64_t head = head0 + r;
         const float o = O / L;
         const int64_t at = head * FS_D + 64 * part + d;
         a.dst[at] = o;
@@ -901,9 +908,15 @@ int launch_fattn_dec_short(hipStream_t s, fattn_args &a, int64_t D) {
     const int64_t R = a.Hq / a.Hkv;
     if (D != FS_D || a.Nq != 1 || R > 4 || a.Hkv > 65535 || a.Nkv > FSS_MAX_WAVES * FS_TILE) return 1;
     if ((a.q_nb2 % 16) != 0 || (a.k_nb1 % 16) != 0 || (a.k_nb2 % 16) != 0 || (a.v_nb1 % 16) != 0 || (a.v_nb2 % 16) != 0) return 1;
+    if (a.k_nb1 >> 24 || a.v_nb1 >> 24 || a.q_nb2 >> 32 || a.k_nb2 >> 32 || a.v_nb2 >> 32) return 1;   // the kernel's offsets
+    constexpr int64_t CU = 256;   // compute units
     const int n_waves = (int)((a.Nkv + FS_TILE - 1) / FS_TILE);
-    if (a.Hkv <= 128) MI355_LAUNCH(k_fattn_dec_short<2>, dim3((unsigned)a.Hkv, 2), dim3((unsigned)n_waves * 64), 0, s, a, (int)R);
-    else MI355_LAUNCH(k_fattn_dec_short<1>, dim3((unsigned)a.Hkv), dim3((unsigned)n_waves * 64), 0, s, a, (int)R);
+#define MI355_FSS_ARGS dim3((unsigned)n_waves * 64), 0, s, a.q, a.k, a.v, a.mask, (u32)a.q_nb2, (u32)a.k_nb1, (u32)a.k_nb2, (u32)a.v_nb1, (u32)a.v_nb2, (u32)a.Nkv | (u32)R << 16, a
+    if (2 * a.Hq <= CU) MI355_LAUNCH((k_fattn_dec_short<2, 1>), dim3((unsigned)a.Hkv, 2, (unsigned)R), MI355_FSS_ARGS);
+    else if (2 * a.Hkv * ((R + 1) / 2) <= CU) MI355_LAUNCH((k_fattn_dec_short<2, 2>), dim3((unsigned)a.Hkv, 2, (unsigned)((R + 1) / 2)), MI355_FSS_ARGS);
+    else if (2 * a.Hkv <= CU) MI355_LAUNCH((k_fattn_dec_short<2, 4>), dim3((unsigned)a.Hkv, 2), MI355_FSS_ARGS);
+    else MI355_LAUNCH((k_fattn_dec_short<1, 4>), dim3((unsigned)a.Hkv), MI355_FSS_ARGS);
+#undef MI355_FSS_ARGS
     return launch_status("k_fattn_dec_short");
 }
 

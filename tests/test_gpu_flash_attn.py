@@ -320,6 +320,20 @@ def test_decode_short_cache_many_kv_heads(dev, Hq, Hkv, Nkv):
     assert torch.equal(act, mi355.quantize_act(dst.reshape(1, Hq * 128)))
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(160, 40), (129, 43), (195, 65), (258, 129)])
+@pytest.mark.parametrize("Nkv", [257, 512])
+def test_decode_short_cache_heads_per_group(dev, Hq, Hkv, Nkv):
+    """two, four heads per group and one group per kv head against a call with few enough heads for a group each: the same bits"""
+    rng = np.random.default_rng(Hq + Nkv)
+    q, k, v, mask = _inputs(rng, 128, 1, Nkv, Hq, Hkv, rand_mask=True)
+    R, few = Hq // Hkv, 7
+    got = _run(dev, q, k, v, mask, 128 ** -0.5)
+    for first in (0, Hkv - few):
+        sl, ql = slice(first, first + few), slice(first * R, (first + few) * R)
+        part = _run(dev, np.ascontiguousarray(q[ql]), np.ascontiguousarray(k[sl]), np.ascontiguousarray(v[sl]), mask, 128 ** -0.5)
+        assert np.array_equal(got[:, ql], part)
+
+
 @pytest.mark.parametrize("D,quantized", [(64, False), (80, False), (96, False), (112, False), (128, False), (256, False), (64, True), (128, True)])
 @pytest.mark.parametrize("Nq,Nkv,Hq,Hkv", [(300, 1100, 8, 2), (200, 520, 12, 12), (600, 640, 32, 8), (40, 600, 70, 70)])
 def test_prefill_non_finite_masked_cells(dev, D, quantized, Nq, Nkv, Hq, Hkv):
