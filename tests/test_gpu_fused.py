@@ -433,6 +433,14 @@ def test_tail_fused_launches_equal_separate_kernels(dev, B, tg, tu, K, N):
         assert int(tickets.abs().sum().item()) == 0
 
 
+@pytest.mark.parametrize("B", [1, 2, 3, 4])
+@pytest.mark.parametrize("t,K", [(orc.Q4_K, 256), (orc.Q4_K, 4352), (orc.Q4_K, 12544), (orc.Q5_K, 4096), (orc.Q5_K, 8448), (orc.Q6_K, 2048), (orc.Q6_K, 6144),
+                                 (orc.Q4_0, 2304), (orc.Q8_0, 4096), (orc.IQ4_XS, 5120)])
+def test_gate_up_ends_of_steps_and_rounds(dev, B, t, K):
+    """less than one step of 64 chunks, whole steps and a few chunks more, for types that walk a wave's rows in one, two and four rounds: the bits of the separate launches"""
+    test_tail_fused_launches_equal_separate_kernels(dev, B, t, t, K, 64)
+
+
 @pytest.mark.parametrize("K,nrows", [(4096, 40), (14336, 9), (2048, 512)])
 def test_q8k_outputs_of_fused_kernels_equal_separate_quantization(dev, K, nrows):
     """RMS_NORM+MUL and SiLU*up writing the per-super-block activation format directly: same bytes as quantizing their f32 output"""
