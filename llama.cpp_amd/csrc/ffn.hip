@@ -66,7 +66,10 @@ __device__ __forceinline__ void gate_up_blk_phase(const uint8_t *__restrict__ Wg
     copy.request(aq, ads, K);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 2 * R; r++) w[r] = G::load(rows[r], L, c_first);
+    for (int r = 0; r < 2 * R; r++) {
+        w[r] = G::load(rows[r], L, c_first);
+        if constexpr (AHEAD && G::ORDERED) __builtin_amdgcn_sched_barrier(0);   // a row must not wait for pieces of a later one
+    }
     copy.commit(s_act, aq, ads, K);
     __syncthreads();
     float acc[2 * R][NCOLS];

@@ -3,7 +3,7 @@
 // Such a launch is over when its slowest chain is: its groups are mostly resident at once, and a wave of k_gemv_q walked a row of 14336 in four steps, each a round trip for the
 // weights and, behind them, for the activation.  Here a group copies the activation to LDS first (a wave's loads return in the order of their issue), every wave has
 // gr_steps of its row on their way from the start - the 33 MB of a 4096 x 14336 Q4_K matrix all at once, 130 KB per compute unit - and the residual is requested ahead of everything.
-// 8B shapes in a chain of launches, us: wo 4.6 -> 3.8, ffn_down Q4_K 10.9 -> 8.2, Q6_K 11.4 -> 10.8 (figures over sizes and types: gemv_row.hpp).
+// 8B shapes in a chain of launches, us: wo 4.6 -> 3.8, ffn_down Q4_K 10.9 -> 8.0, Q6_K 11.4 -> 10.2 (8.2, 10.8 before the loads of a step were kept together; 8192 x 28672 Q4_K 25.3 -> 24.1; other figures: gemv_row.hpp).
 // Sums as in gemv_body: same lane-to-chunk mapping, same order of steps, same wave reduction.
 #include "common.hpp"
 #include "qdot.hpp"
@@ -38,6 +38,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_gemv_row(const uint8_t *__restri
     for (int p = 0; p < STEPS; p++) {
         const int c = p * 64 + lane;
         w[p] = G::load(wrow, L, c < nchunks ? c : nchunks - 1);
+        if constexpr (G::ORDERED) __builtin_amdgcn_sched_barrier(0);   // step by step, here and below: a step must not wait for pieces of a later one
     }
     copy.commit(s_gr, aq, ads, K);
     __syncthreads();
@@ -55,6 +56,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_gemv_row(const uint8_t *__restri
             const typename T::chunk now = G::decode(w[p], c);
             acc = T::accumulate(acc, now, A, T::dots(now, A));
             w[p] = G::load(wrow, L, next < nchunks ? next : nchunks - 1);
+            if constexpr (G::ORDERED) __builtin_amdgcn_sched_barrier(0);
         }
     }
 #pragma unroll

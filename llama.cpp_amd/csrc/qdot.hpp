@@ -632,13 +632,15 @@ __device__ __forceinline__ float weight_value(const uint8_t *__restrict__ row, c
 }
 
 // A chunk as it is loaded, decoded where it is used: arithmetic on what was loaded, written beside the load, is moved ahead of the next barrier and waits there for the weights
-// (types whose scales take no arithmetic have one form)
+// (the others have one form).  ORDERED: the loads of several chunks may be kept in order by a scheduling barrier behind each - no arithmetic is among them that would wait there.
 template <int TYPE, class = void> struct late_chunk {
+    static constexpr bool ORDERED = false;
     typedef typename wq<TYPE>::chunk raw;
     static __device__ __forceinline__ raw load(const uint8_t *row, const row_layout &L, int c) { return wq<TYPE>::load_w(row, L, c); }
     static __device__ __forceinline__ raw decode(const raw &r, int) { return r; }
 };
 template <int TYPE> struct late_chunk<TYPE, std::void_t<typename wq<TYPE>::raw>> {
+    static constexpr bool ORDERED = true;
     typedef typename wq<TYPE>::raw raw;
     static __device__ __forceinline__ raw load(const uint8_t *row, const row_layout &L, int c) { return wq<TYPE>::load_raw(row, L, c); }
     static __device__ __forceinline__ typename wq<TYPE>::chunk decode(const raw &r, int c) { return wq<TYPE>::decode(r, c); }
