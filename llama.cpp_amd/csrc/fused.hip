@@ -28,8 +28,8 @@ __global__ void __launch_bounds__(256) k_rms_norm_mul_quant(const float *__restr
     rms_norm_quant_row<NV, FMT, false>(x + row * x_stride, w, y ? y + row * y_stride : nullptr, act, row, k, nrows, eps, sh);
 }
 
-// One 1024-thread group per row, up to 256 rows (one group per compute unit).  us, 256 threads / 1024: one row of 4096 2.96 / 2.43, 256 rows 3.46 / 3.13,
-// one of 8192 4.53 / 3.32; one row of 4096 to a Q8_K image 4.27 / 3.22
+// One 1024-thread group per row, up to 256 rows (one group per compute unit).  us, 256 threads / 1024: one row of 4096 2.96 / 2.29, 256 rows 3.46 / 2.94,
+// one of 8192 4.53 / 3.04; one row of 4096 to a Q8_K image 4.27 / 2.71
 template <int NV, int FMT>
 __global__ void __launch_bounds__(1024) k_rms_norm_mul_quant_wide(const float *__restrict__ x, int64_t x_stride, const float *__restrict__ w,
                                                                   float *__restrict__ y, int64_t y_stride, void *__restrict__ act, int64_t k,

@@ -29,6 +29,7 @@
 // Group ids are remapped so that the groups sharing one weight panel run on the same XCD
 // (ids are dealt round-robin over the 8 XCDs) and hit its L2 instead of HBM.
 #include "common.hpp"
+#include "slices.hpp"
 #include "qdot.hpp"
 #include "tiles.hpp"
 
@@ -734,19 +735,60 @@ static size_t mmq_ws_bytes(int n_mats, const int64_t *Ns, int64_t K, int64_t B) 
     return n > 1 ? mmq_slab_bytes(n, rows, B) : 0;
 }
 
-// dst[b][n] of every matrix = sum of its slices in ascending order (+ residual).  part: [slice][B][rows of all matrices]
-__global__ void __launch_bounds__(256) k_mmq_split_sum(const float *__restrict__ part, mmq_mats mats, int64_t rows, int64_t B, int n_slices) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * B) return;
-    float acc = part[i];
-    for (int sl = 1; sl < n_slices; sl++) acc = add_rn(acc, part[(int64_t)sl * rows * B + i]);
-    const int64_t b = i / rows;
-    int64_t n = i % rows;
+// dst[b][n] of every matrix = sum of its slices in ascending order (+ residual).  part: [slice][B][rows of all matrices]; one activation row per blockIdx.y (rows beyond its range in turn)
+constexpr int64_t MMQ_SUM_ROWS = 65535;
+__device__ __forceinline__ const mmq_mat &mmq_mat_of(const mmq_mats &mats, int64_t &n) {
     int j = 0;
     while (j < MMQ_MATS - 1 && n >= mats.m[j].N) n -= mats.m[j++].N;
-    const mmq_mat &m = mats.m[j];
-    const int64_t o = b * m.dst_stride + n;
-    m.dst[o] = m.residual ? add_rn(acc, m.residual[o]) : acc;
+    return mats.m[j];
+}
+__global__ void __launch_bounds__(256) k_mmq_split_sum(const float *__restrict__ part, mmq_mats mats, int64_t rows, int64_t B, int n_slices) {
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= rows) return;
+    int64_t n = r;
+    const mmq_mat &m = mmq_mat_of(mats, n);
+    for (int64_t b = blockIdx.y; b < B; b += MMQ_SUM_ROWS) {
+        float acc = part[b * rows + r];
+        for (int sl = 1; sl < n_slices; sl++) acc = add_rn(acc, part[((int64_t)sl * B + b) * rows + r]);
+        const int64_t o = b * m.dst_stride + n;
+        m.dst[o] = m.residual ? add_rn(acc, m.residual[o]) : acc;
+    }
+}
+// ... four neighbouring elements per lane, for matrices of N % 4 == 0 with 16-byte aligned rows in dst and residual (4096 x 333, five slices: 9.3 -> 6.6 us)
+template <int SL>
+__global__ void __launch_bounds__(256) k_mmq_split_sum4(const float *__restrict__ part, mmq_mats mats, int64_t rows, int64_t B, int n_slices) {
+    const int64_t r = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (r >= rows) return;
+    int64_t n = r;
+    const mmq_mat &m = mmq_mat_of(mats, n);
+    for (int64_t b = blockIdx.y; b < B; b += MMQ_SUM_ROWS) {
+        slab_sum<SL> slabs;
+        slabs.request(part + b * rows + r, rows * B, n_slices);
+        const int64_t o = b * m.dst_stride + n;
+        f32x4 acc = slabs.sum(part + b * rows + r, rows * B, n_slices);
+        if (m.residual) {
+            const f32x4 t = *(const f32x4 *)(m.residual + o);
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[j] = add_rn(acc[j], t[j]);
+        }
+        *(f32x4 *)(m.dst + o) = acc;
+    }
+}
+static void launch_mmq_split_sum(hipStream_t s, const float *part, const mmq_mats &mats, int n_mats, int64_t rows, int64_t B, int n_slices) {
+    bool wide = true;
+    for (int i = 0; i < n_mats; i++) {
+        const mmq_mat &m = mats.m[i];
+        wide = wide && m.N % 4 == 0 && m.dst_stride % 4 == 0 && (((uintptr_t)m.dst | (uintptr_t)m.residual) & 15) == 0;
+    }
+    const int64_t per = wide ? 1024 : 256;
+    const dim3 grid((unsigned)((rows + per - 1) / per), (unsigned)(B < MMQ_SUM_ROWS ? B : MMQ_SUM_ROWS));
+    if (!wide) {
+        MI355_LAUNCH(k_mmq_split_sum, grid, dim3(256), 0, s, part, mats, rows, B, n_slices);
+        return;
+    }
+#define MI355_SUM_LAUNCH(SL) MI355_LAUNCH(k_mmq_split_sum4<SL>, grid, dim3(256), 0, s, part, mats, rows, B, n_slices)
+    MI355_SLAB_SWITCH(n_slices, MI355_SUM_LAUNCH)
+#undef MI355_SUM_LAUNCH
 }
 
 // The kernel reaches the 128 rows of a tile by 32-bit offsets from its first one: K up to some 2^25.  Longer rows run on the byte-load kernels.
@@ -784,7 +826,7 @@ static void launch_mmq(hipStream_t s, int n_mats, const mi355_gemv_mat *mats, co
     const int n_slices = mmq_slices(TYPE, row_tiles, K, B, rows, ws == nullptr || ((uintptr_t)ws & 15) != 0 ? 0 : ws_bytes);
     const dim3 grid((unsigned)n_groups_padded, (unsigned)n_slices);
     MI355_LAUNCH((k_mmq<TYPE, TN>), grid, dim3(256), 0, s, n_slices > 1 ? part : a, aq, ads, K, B, L, n_col_tiles, n_groups, n_groups_padded, rows * B, mmq32_route{});
-    if (n_slices > 1) MI355_LAUNCH(k_mmq_split_sum, dim3((unsigned)((rows * B + 255) / 256)), dim3(256), 0, s, (const float *)ws, a, rows, B, n_slices);
+    if (n_slices > 1) launch_mmq_split_sum(s, (const float *)ws, a, n_mats, rows, B, n_slices);
 }
 
 template <int TYPE>

@@ -193,41 +193,41 @@ __device__ __forceinline__ void rms_norm_quant_row_wide(const float *__restrict_
                                                         int64_t k, int64_t nrows, float eps, float *sh) {
     constexpr int NP = NV / 4;
     const int tid = threadIdx.x;
+    // Everything is requested before anything is waited for; pieces past the end repeat the first one, and nothing uses them (a branch around each load made three trips to memory of
+    // one: one row of 4096 2.43 us, now 2.29; to a Q8_K image 3.2, now 2.7).
     f32x4 own[NP], ww[NP];
+    const float *wr = w ? w : xr;
 #pragma unroll
     for (int p = 0; p < NP; p++) {
-        const int64_t e0 = ((int64_t)p * 1024 + tid) * 4;
-        ww[p] = f32x4{1.f, 1.f, 1.f, 1.f};
-        if (w && e0 < k) ww[p] = *(const f32x4 *)(w + e0);
+        const int64_t e0 = ((int64_t)p * 1024 + tid) * 4, at = e0 < k ? e0 : 0;
+        own[p] = *(const f32x4 *)(xr + at);
+        ww[p] = *(const f32x4 *)(wr + at);
     }
+    const float kf = (float)k;
+    asm volatile("" ::"s"(eps), "s"(kf), "s"(nrows));   // (arguments beyond the preloaded ones)
     if (__builtin_amdgcn_readfirstlane(tid >> 8) == 0) {
         f32x4 v[NV];
 #pragma unroll
         for (int it = 0; it < NV; it++) {
             const int64_t e0 = ((int64_t)it * 256 + tid) * 4;
-            v[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (e0 < k) v[it] = *(const f32x4 *)(xr + e0);
+            v[it] = *(const f32x4 *)(xr + (e0 < k ? e0 : 0));
         }
         float ss = 0.0f;
 #pragma unroll
-        for (int it = 0; it < NV; it++)
+        for (int it = 0; it < NV; it++) {
+            const bool live = ((int64_t)it * 256 + tid) * 4 < k;
 #pragma unroll
-            for (int i = 0; i < 4; i++) ss = __builtin_fmaf(v[it][i], v[it][i], ss);
+            for (int i = 0; i < 4; i++) {
+                const float t = live ? v[it][i] : 0.0f;
+                ss = __builtin_fmaf(t, t, ss);
+            }
+        }
         ss = wave_sum_dpp(ss);
         if ((tid & 63) == 0) sh[tid >> 6] = ss;
-#pragma unroll
-        for (int p = 0; p < NP; p++) own[p] = v[4 * p];
-    } else {
-#pragma unroll
-        for (int p = 0; p < NP; p++) {
-            const int64_t e0 = ((int64_t)p * 1024 + tid) * 4;
-            own[p] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (e0 < k) own[p] = *(const f32x4 *)(xr + e0);
-        }
     }
     __syncthreads();
     const float total = add_rn(add_rn(add_rn(sh[0], sh[1]), sh[2]), sh[3]);
-    const float scale = 1.0f / sqrtf(add_rn(total / (float)k, eps));
+    const float scale = 1.0f / sqrtf(add_rn(total / kf, eps));
 #pragma unroll
     for (int p = 0; p < NP; p++) norm_piece<FMT>(own[p], ww[p], w != nullptr, scale, yr, act, row, k, nrows, ((int64_t)p * 1024 + tid) * 4);
 }
@@ -240,31 +240,33 @@ __device__ __forceinline__ void rms_norm_quant_row_wide(const float *__restrict_
 // Called by the first 256 threads of a group; contains exactly one group barrier, which further waves of a larger group must
 // match with a barrier of their own.
 // keep: where the caller wants the thread's NV pieces of the normalised row (registers), or null
-// given: the thread's NV pieces of the row when the caller has just formed them (xr is not read then), or null
 template <int NV, int FMT, bool COH>
 __device__ __forceinline__ void rms_norm_quant_row(const float *__restrict__ xr, const float *__restrict__ w, float *__restrict__ yr,
                                                    void *__restrict__ act, int64_t row, int64_t k, int64_t nrows, float eps, float *sh,
-                                                   f32x4 *keep = nullptr, const f32x4 *given = nullptr) {
+                                                   f32x4 *keep = nullptr) {
     const int tid = threadIdx.x;
     f32x4 v[NV], ww[NV];
-    // the weight does not depend on the reduction: fetch it together with the row, one memory round trip instead of two
+    // the weight does not depend on the reduction: fetch it together with the row, one memory round trip instead of two; pieces past the end repeat the first one and are not used (a
+    // branch around every load makes a trip of each)
+    const float *wr = w ? w : xr;
+#pragma unroll
+    for (int it = 0; it < NV; it++) {
+        const int64_t e0 = ((int64_t)it * 256 + tid) * 4, at = e0 < k ? e0 : 0;
+        if constexpr (COH) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[it][i] = __hip_atomic_load(xr + at + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            v[it] = *(const f32x4 *)(xr + at);
+        }
+    }
 #pragma unroll
     for (int it = 0; it < NV; it++) {
         const int64_t e0 = ((int64_t)it * 256 + tid) * 4;
-        v[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-        ww[it] = f32x4{1.f, 1.f, 1.f, 1.f};
-        if (e0 < k) {
-            if (given) {
-                v[it] = given[it];
-            } else if constexpr (COH) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) v[it][i] = __hip_atomic_load(xr + e0 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                v[it] = *(const f32x4 *)(xr + e0);
-            }
-            if (w) ww[it] = *(const f32x4 *)(w + e0);
-        }
+        ww[it] = *(const f32x4 *)(wr + (e0 < k ? e0 : 0));
     }
+#pragma unroll
+    for (int it = 0; it < NV; it++)
+        if (((int64_t)it * 256 + tid) * 4 >= k) v[it] = f32x4{0.f, 0.f, 0.f, 0.f};
     const float scale = rms_norm_scale<NV>(v, k, eps, sh);
 #pragma unroll
     for (int it = 0; it < NV; it++) {

@@ -464,6 +464,36 @@ def _tile_off(row, k, K):
     return ((row >> 4) * (K >> 6) + (k >> 6)) * 1024 + r * 64 + ((c ^ ((r >> 2) & 3)) << 4) + (k & 15)
 
 
+@pytest.mark.parametrize("t,N,K,B", [(orc.Q4_0, 768, 8192, 70), (orc.Q4_0, 4096, 4096, 130), (orc.Q6_K, 4096, 11008, 140), (orc.Q6_K, 1024, 2048, 65), (orc.Q4_K, 4096, 4096, 256),
+                                     (orc.Q4_K, 1536, 4096, 300), (orc.Q6_K, 1024, 14336, 200)])
+def test_slab_sums_by_four_and_by_one(dev, t, N, K, B):
+    """products cut along K into dst rows that allow 16-byte stores and into rows one float apart from that: the same sums, the same bits (and nothing between the rows is touched)"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    rng = np.random.default_rng(N + K + B)
+    Wd = mi355.upload_weights(t, _to_dev(dev, orc.quantize("oracle", t, (rng.standard_normal((N, K)) * 0.05).astype(np.float32))))
+    x = _to_dev(dev, rng.standard_normal((B, K)).astype(np.float32))
+    wide, odd = torch.full((B, N + 4), 7.0, device=dev), torch.full((B, N + 5), 7.0, device=dev)
+    need = lib.mi355_mul_mat_split_ws_bytes(N, K, B)
+    for dst in (wide, odd):
+        ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+        mi355.check(lib.mi355_mul_mat(None, t, Wd.data_ptr(), x.data_ptr(), dst.data_ptr(), N, K, B, K, dst.stride(0), ws.data_ptr(), ws.numel()))
+    assert torch.equal(wide[:, :N], odd[:, :N]) and bool((wide[:, N:] == 7.0).all()) and bool((odd[:, N:] == 7.0).all())
+    assert bool(wide[:, :N].abs().sum() > 0)
+    if t == orc.Q4_0 or K % 2048 or not lib.mi355_mul_mat_q8k_tiled_ws_bytes(N, K, B): return
+    tiles = mi355.kq_unpack_tiles(t, Wd)
+    act = mi355.quantize_act_q8k_tiled(x)
+    res = [_to_dev(dev, rng.standard_normal((B, n)).astype(np.float32)) for n in (N + 4, N + 5)]
+    res[1][:, :N] = res[0][:, :N]
+    got = []
+    for r in res:   # in place: the residual is dst
+        ws = torch.zeros(lib.mi355_mul_mat_q8k_tiled_ws_bytes(N, K, B), dtype=torch.uint8, device=dev)
+        mi355.check(lib.mi355_mul_mat_q8k_tiled(None, t, tiles.data_ptr(), act.data_ptr(), r.data_ptr(), r.data_ptr(), N, K, B, r.stride(0), ws.data_ptr(), ws.numel()))
+        got.append(r[:, :N].cpu())
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("K,B", [(256, 5), (4096, 33), (14336, 130)])
 def test_quantize_q8k_tiled_bit_exact(dev, K, B):
     """the tile-image form holds the same levels, scales and sub-block sums as block_q8_K of the reference"""
