@@ -784,32 +784,37 @@ __global__ void __launch_bounds__(128 * NU, NU == 2 && D <= 128 ? 2 : 1) k_fattn
 // computed again by exact_row.
 template <int D, bool PX>
 __global__ void __launch_bounds__(256) k_fattn_half_merge(fattn_args a) {
-    constexpr int E = (D + 63) / 64;
+    constexpr int E = (D + 63) / 64;   // neighbouring elements of a lane (D is a multiple of E)
+    typedef float part __attribute__((ext_vector_type(E == 3 ? 4 : E), aligned(4 * E)));
+    static_assert(D % E == 0 && (E == 1 || E == 2 || E == 4), "elements of a lane");
     const int lane = threadIdx.x & 63;
     const int64_t rows = a.Nq * a.Hq, row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;   // whole wave
     const float2 *ml = (const float2 *)(a.ws + a.n_splits * rows * D);
-    const float2 mine = lane < a.n_splits ? ml[lane * rows + row] : float2{FM_NEG, 0.0f};
+    const bool live = E * lane < D;
+    const float *mine_at = a.ws + row * D + (live ? E * lane : 0);   // lanes past the end repeat the first one's and are not stored
+    // four ranges' values requested together, the first four ahead of the maxima; past the end the last range again, times 0
+    part v[4];
+    auto request = [&](int s0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = *(const part *)(mine_at + (s0 + j < a.n_splits ? s0 + j : a.n_splits - 1) * (rows * D));
+    };
+    const float2 state = ml[(lane < a.n_splits ? lane : a.n_splits - 1) * rows + row];
+    request(0);
+    const float2 mine = lane < a.n_splits ? state : float2{FM_NEG, 0.0f};
     const float f = merge_factor<PX>(mine.x, wave_max_dpp(mine.x));
     const float l = wave_sum_dpp(lane < a.n_splits ? mine.y * f : 0.0f);
-    float o[E];
-#pragma unroll
-    for (int e = 0; e < E; e++) o[e] = 0.0f;
-    for (int s0 = 0; s0 < a.n_splits; s0 += 4) {   // four ranges' values requested together; past the end the last one again, times 0
-        float v[4][E];
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int e = 0; e < E; e++) {
-                const int sp = s0 + j < a.n_splits ? s0 + j : a.n_splits - 1, d = 64 * e + lane;
-                v[j][e] = d < D ? a.ws[(sp * rows + row) * D + d] : 0.0f;
-            }
+    part o = 0.0f;
+    for (int s0 = 0;;) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const float fs = s0 + j < a.n_splits ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), s0 + j)) : 0.0f;
 #pragma unroll
             for (int e = 0; e < E; e++) o[e] = fmaf(v[j][e], fs, o[e]);
         }
+        s0 += 4;
+        if (s0 >= a.n_splits) break;   // uniform
+        request(s0);
     }
     float z = l * 0.0f;
 #pragma unroll
@@ -820,10 +825,9 @@ __global__ void __launch_bounds__(256) k_fattn_half_merge(fattn_args a) {
         return;
     }
     const float sum = sum_of<PX>(l), inv = reciprocal_of<PX>(sum);
+    if (live) {
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-        const int d = 64 * e + lane;
-        if (d < D) a.dst[row * D + d] = quotient<PX>(o[e], sum, inv);
+        for (int e = 0; e < E; e++) a.dst[row * D + E * lane + e] = quotient<PX>(o[e], sum, inv);
     }
 }
 
