@@ -53,25 +53,27 @@ template <int NB> struct mid_act {
 // act: tile images of B rows (mi355_quantize_act_q8k_tiled).
 // Up to three matrices that read the same activation go out in one launch, their 32-row tiles numbered one matrix after the other
 // (Q, K and V; gate and up: the small ones alone are a handful of groups each, and every launch costs its start-up).
+// What the first requests need comes in arguments that are in registers when a wave starts (the first fourteen words; first1, first2: first tiles of the second and third matrix, `tiles`,
+// the number of all, where there is none; rows: B and, from bit 8, five bits each for the rows of a matrix's last tile less one); destinations are read at the end.  Three trips for
+// them in a row ahead of the first request: 14336 x 4096, 64 rows 22.5 us a call, now 22.0, 128 rows 35.1, now 34.2.
 struct mid_mat {
     const uint8_t *W;
     float *dst;
     const float *residual;   // may be null; same shape and stride as dst; may be dst itself
     int64_t N, dst_stride;
-    int first_tile;          // index of the matrix's first 32-row tile in the launch (unused entries: INT_MAX)
+    int first_tile;          // index of the matrix's first 32-row tile in the launch
 };
 struct mid_launch {
     mid_mat m[3];
 };
 template <int NB, int NBW>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
-k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int steps_per_slice, int steps_per_wave) {
-    const int mi = ((int)blockIdx.x >= P.m[1].first_tile ? 1 : 0) + ((int)blockIdx.x >= P.m[2].first_tile ? 1 : 0);   // uniform
-    const uint8_t *__restrict__ W = P.m[mi].W;
-    float *__restrict__ dst = P.m[mi].dst;
-    const float *__restrict__ residual = P.m[mi].residual;
-    const int64_t N = P.m[mi].N, dst_stride = P.m[mi].dst_stride;
-    const int tile_x = (int)blockIdx.x - P.m[mi].first_tile;
+k_mm_mid_q4k(const uint8_t *__restrict__ W0, const uint8_t *__restrict__ W1, const uint8_t *__restrict__ W2, const uint8_t *__restrict__ act, int first1, int first2, int tiles, int K,
+             u32 rows, int steps_per_slice, mid_launch P) {
+    const int mi = ((int)blockIdx.x >= first1 ? 1 : 0) + ((int)blockIdx.x >= first2 ? 1 : 0);   // uniform
+    const uint8_t *__restrict__ W = mi == 0 ? W0 : mi == 1 ? W1 : W2;
+    const int first = mi == 0 ? 0 : mi == 1 ? first1 : first2, next = mi == 0 ? first1 : mi == 1 ? first2 : tiles;
+    const int tile_x = (int)blockIdx.x - first, last_row = 32 * (next - first - 1) + (int)((rows >> (8 + 5 * mi)) & 31), B = (int)(rows & 255);
     constexpr int KS = 4 / NBW;
     constexpr int WAVE_BYTES = MID_STAGES * MID_STAGE;
     constexpr int RED_BYTES = 4 * NB * 16 * 64 * 4;
@@ -85,6 +87,7 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
 
     const int64_t row0 = (int64_t)tile_x * 32;
     const int nsteps = K >> 8;
+    const int steps_per_wave = (steps_per_slice + KS - 1) / KS;
     const int slice_lo = blockIdx.y * steps_per_slice;
     const int slice_hi = slice_lo + steps_per_slice < nsteps ? slice_lo + steps_per_slice : nsteps;
     const int s_lo = slice_lo + part * steps_per_wave;
@@ -93,7 +96,6 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
     // sources of the transfers: 32-bit offsets from W (the launcher keeps matrices and images below 4 GiB), formed anew for every stage from the
     // lane number (registers); rows past the end repeat the last row and are not stored
     const u32 row_bytes = (u32)nsteps * Q4_K_BYTES;
-    const int last_row = (int)(N - 1);
     const int64_t b16 = ((int64_t)B + 15) & ~(int64_t)15;
     const int64_t cb_pad = wt_cb_pad(B);
     const int64_t aux0 = b16 * K;   // the records behind the activation image
@@ -282,6 +284,9 @@ k_mm_mid_q4k(mid_launch P, const uint8_t *__restrict__ act, int K, int B, int st
 #pragma unroll
         for (int i = 0; i < 16; i++) s_red[((wave * NB + nb) * 16 + i) * 64 + lane] = accf[nb][i];
     __syncthreads();
+    float *__restrict__ dst = P.m[mi].dst;
+    const float *__restrict__ residual = P.m[mi].residual;
+    const int64_t N = P.m[mi].N, dst_stride = P.m[mi].dst_stride;
     // value v = (set, tile of the set, i) is finished by wave v % 4
     for (int v = wave; v < NBW * NB * 16; v += 4) {
         const int tset = v / (NB * 16), tnb = (v / 16) % NB, i = v & 15;
@@ -400,7 +405,7 @@ static int mul_mat_mid_launch(void *stream, int type, int n_mats, const mi355_ge
         L.m[i].residual = m.residual;
         L.m[i].N = m.N;
         L.m[i].dst_stride = m.dst_stride;
-        L.m[i].first_tile = i < n_mats ? (int)tiles : 0x7fffffff;
+        L.m[i].first_tile = (int)tiles;
         if (i < n_mats) {
             tiles += (m.N + 31) / 32;
             n_sum += m.N;
@@ -412,8 +417,9 @@ static int mul_mat_mid_launch(void *stream, int type, int n_mats, const mi355_ge
     hipStream_t s = (hipStream_t)stream;
     const int nsteps = (int)(K >> 8);
     const int steps_per_slice = (nsteps + slices - 1) / slices;
-    const int nbw = mid_sets(B);
-    const int steps_per_wave = (steps_per_slice + 4 / nbw - 1) / (4 / nbw);
+    const int first1 = n_mats > 1 ? L.m[1].first_tile : (int)tiles, first2 = n_mats > 2 ? L.m[2].first_tile : (int)tiles;
+    u32 rows = (u32)B;
+    for (int i = 0; i < n_mats; i++) rows |= (u32)((mats[i].N - 1) & 31) << (8 + 5 * i);
     const dim3 grid((unsigned)tiles, (unsigned)slices);
     mid_sum S;
     int64_t n_max = 0;
@@ -435,7 +441,8 @@ static int mul_mat_mid_launch(void *stream, int type, int n_mats, const mi355_ge
             }
         }
     }
-#define MI355_MID_ARGS grid, dim3(256), 0, s, L, (const uint8_t *)act, (int)K, (int)B, steps_per_slice, steps_per_wave
+#define MI355_MID_ARGS \
+    grid, dim3(256), 0, s, L.m[0].W, L.m[1].W, L.m[2].W, (const uint8_t *)act, first1, first2, (int)tiles, (int)K, rows, steps_per_slice, L
     if (B <= 32) MI355_LAUNCH((k_mm_mid_q4k<1, 1>), MI355_MID_ARGS);
     else if (B <= 64) MI355_LAUNCH((k_mm_mid_q4k<2, 1>), MI355_MID_ARGS);
     else MI355_LAUNCH((k_mm_mid_q4k<2, 2>), MI355_MID_ARGS);
