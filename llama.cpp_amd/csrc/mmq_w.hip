@@ -302,14 +302,12 @@ constexpr int WT_A_AUX_TILE = (WT_BN / 16) * WT_A_AUX;       // 4608 bytes of ac
 // batch 512: 2 x 448 tiles = 3.5 rounds on 256 compute units instead of 2 x 2).  Cutting the last, partly empty round's tiles
 // along K so that short groups fill it was measured and dropped: 162 us against 160 us uncut for gate + up - with half of the
 // compute units idle the others run faster, so the uncut tail costs less than its group count suggests.
-// gridDim.y > 1 cuts every tile into gridDim.y slices (single matrices with few tiles; partial sums in dst, one N x B slab per
+// a grid of several rows cuts every tile into as many slices (single matrices with few tiles; partial sums in dst, one N x B slab per
 // slice, added by k_wt_split_sum).
 struct wt_mat {
-    const int8_t *w_img;
     float *dst;
     const float *residual;   // may be null; same shape and stride as dst; may be dst itself
     int64_t N, dst_stride;
-    int first_tile;          // index of this matrix's first tile in the launch (unused entries: INT_MAX)
     int shift;               // log2 of the radix between the matrix's two planes: 3 Q4_K, 4 Q5_K, 6 Q6_K
     int epi;                 // EPI launches: WT_EPI_*
     int64_t nb1, nb2;        // WT_EPI_*CACHE: dst = base of an f16 cache; byte strides of a cell and of a head inside it
@@ -324,17 +322,20 @@ struct wt_rope {
 };
 struct wt_launch {
     wt_mat m[3];
-    int n_col_tiles;
-    int n_tiles, n_tiles_padded;   // n_tiles_padded: rounded up to a multiple of 8
+    int sb_per_slice;        // super-blocks of a slice (all of them: not cut)
     wt_rope rope;
 };
 
+// The arguments ahead of P are what the first transfers need; they are in registers when a wave starts (fourteen words; first1, first2: first tiles of the second and third matrix,
+// INT_MAX where there is none; n_sb: super-blocks of a row; n_rows: B).  With five reads of the argument segment in a row and 64-bit divisions there, 512 rows, two slices: 4096 x 4096 and
+// 4096 x 14336 of Q4_K 41.3 -> 40.4 us on average, 4096 x 14336 of Q6_K 68.7 -> 67.4, gate and up (3.5 groups one after the other on a compute unit) 160.6 -> 159.5.
 // ID: MUL_MAT_ID.  The "matrix" is expert 0's images, the column tiles are those of the sorted slot list (rt), B the rows of the
 // activation image (128 per column tile); a tile's rows go to the dst rows of its slots.
 // TYPE: MI355_Q4_K = the form with the min term, the radix between the planes taken from the matrix (Q4_K, Q5_K, and Q6_K images,
 // whose minima are zeros, in a launch they share with the other two); MI355_Q6_K = launches of Q6_K matrices only: no min term.
 template <int TYPE, bool ID = false, bool EPI = false>
-__global__ void __launch_bounds__(512, 1) k_mmq_w(wt_launch P, const int8_t *__restrict__ a_img, int64_t K, int64_t B, wt_route rt) {
+__global__ void __launch_bounds__(512, 1) k_mmq_w(const int8_t *__restrict__ w_img0, const int8_t *__restrict__ w_img1, const int8_t *__restrict__ w_img2, const int8_t *__restrict__ a_img,
+                                                  int first1, int first2, int n_tiles, int n_col_tiles, int n_sb, int n_rows, wt_launch P, wt_route rt) {
     static_assert(TYPE == MI355_Q4_K || TYPE == MI355_Q6_K, "two forms");
     static_assert(!(ID && EPI), "one or the other");
     constexpr bool Q4 = TYPE == MI355_Q4_K;   // sub-block mins: the min term and its scale records
@@ -359,22 +360,23 @@ __global__ void __launch_bounds__(512, 1) k_mmq_w(wt_launch P, const int8_t *__r
     auto ring = [&](int i) -> int8_t * { return ring_buf + (i & (NBUF - 1)) * STAGE; };
 
     // groups of one XCD (every eighth group index) take consecutive tiles: the column tiles of a weight row tile meet in one L2
-    const int tile = (int)(blockIdx.x & 7) * (P.n_tiles_padded >> 3) + (int)(blockIdx.x >> 3);
-    if (tile >= P.n_tiles) return;
-    const int mi = (tile >= P.m[1].first_tile ? 1 : 0) + (tile >= P.m[2].first_tile ? 1 : 0);
-    const int8_t *__restrict__ w_img = P.m[mi].w_img;
+    const int tile = (int)(blockIdx.x & 7) * ((n_tiles + 7) >> 3) + (int)(blockIdx.x >> 3);
+    if (tile >= n_tiles) return;
+    const int mi = (tile >= first1 ? 1 : 0) + (tile >= first2 ? 1 : 0);
+    const int8_t *__restrict__ w_img = mi == 0 ? w_img0 : mi == 1 ? w_img1 : w_img2;
     float *dst = P.m[mi].dst;
     const float *residual = P.m[mi].residual;
     const int64_t N = P.m[mi].N;
     const int64_t dst_stride = P.m[mi].dst_stride;
     const int radix_shift = Q4 ? __builtin_amdgcn_readfirstlane(P.m[mi].shift) : 6;
-    const int n_col_tiles = P.n_col_tiles;
-    const int ltile = tile - P.m[mi].first_tile;
-    const int64_t row0 = (int64_t)(ltile / n_col_tiles) * WT_BM;
-    const int64_t col0 = (int64_t)(ltile % n_col_tiles) * WT_BN;
+    const int64_t K = (int64_t)n_sb * QKK, B = n_rows;
+    const int ltile = tile - (mi == 0 ? 0 : mi == 1 ? first1 : first2);
+    const u32 row_tile = (u32)ltile / (u32)n_col_tiles;
+    const int64_t row0 = (int64_t)row_tile * WT_BM;
+    const int64_t col0 = (int64_t)((u32)ltile - row_tile * (u32)n_col_tiles) * WT_BN;
     int slot_first = 0, slot_end = 0;   // ID: the tile's columns of the sorted slot list
     if constexpr (ID) {
-        const int ct = ltile % n_col_tiles;
+        const int ct = ltile - (int)row_tile * n_col_tiles;
         if (ct >= *rt.n_tiles) return;   // the whole group
         w_img += (int64_t)rt.tiles[4 * ct] * rt.expert_img_bytes;
         slot_first = rt.tiles[4 * ct + 1];
@@ -388,13 +390,13 @@ __global__ void __launch_bounds__(512, 1) k_mmq_w(wt_launch P, const int8_t *__r
     const int wrow0 = (wave & 3) * 32;    // weight rows of this wave inside the tile
     const int wcol0 = (wave >> 2) * 64;   // activation rows of this wave inside the tile
     const int64_t nsb = K >> 8, nkb = K >> 6;
-    // split K: group y of gridDim.y walks super-blocks [sb_lo, sb_hi) and writes its sums to its own slice of `dst`
-    const int64_t sb_per = (nsb + gridDim.y - 1) / gridDim.y;
+    // split K: group y walks super-blocks [sb_lo, sb_hi) and writes its sums to its own slice of `dst`
+    const int64_t sb_per = P.sb_per_slice;
     const int64_t sb_lo = (int64_t)blockIdx.y * sb_per, sb_hi = sb_lo + sb_per < nsb ? sb_lo + sb_per : nsb;
     // where the sums go: element (b, n) of the product at out[(b - col0) * dst_stride + (n - row0)]
     float *out = dst + col0 * dst_stride + row0;
     if (residual) residual += col0 * dst_stride + row0;
-    if (gridDim.y > 1) {
+    if (sb_per < nsb) {
         out += (int64_t)blockIdx.y * B * dst_stride;
         residual = nullptr;
     }
@@ -639,8 +641,8 @@ __global__ void __launch_bounds__(512, 1) k_mmq_w(wt_launch P, const int8_t *__r
         // element d of head n / D; its partner in the pair is the neighbouring lane.  Same roundings as k_rope_kv_store.
         const int kind = P.m[mi].epi;   // uniform over the group
         const int64_t n = row0 + wrow0 + l32;
-        const int D = P.rope.D, d = (int)(n % D);
-        const int64_t head = n / D;
+        const int D = P.rope.D, d = (int)((u32)n % (u32)D);   // (matrices of 2^32 rows do not fit the memory)
+        const int64_t head = (u32)n / (u32)D;
         const bool rot = kind != WT_EPI_CACHE && d < P.rope.n_dims;
         const float2 *cs = P.rope.cs + (d >> 1);
         uint8_t *cache = (uint8_t *)dst + head * P.m[mi].nb2 + 2 * d;
@@ -956,14 +958,14 @@ static int mul_mat_q8k_tiled_launch(void *stream, const int *types, int n_mats, 
     MI355_REQUIRE((int64_t)p.n_tiles + 8 < (1 << 30), "mul_mat_q8k_tiled: too many tiles");
     hipStream_t s = (hipStream_t)stream;
     wt_launch L;
+    const int8_t *images[3];
     for (int i = 0; i < 3; i++) {
         const int k = i < n_mats ? i : 0;
-        L.m[i].w_img = (const int8_t *)mats[k].tiles;
+        images[i] = (const int8_t *)mats[k].tiles;
         L.m[i].dst = mats[k].dst;
         L.m[i].residual = mats[k].residual;
         L.m[i].N = mats[k].N;
         L.m[i].dst_stride = mats[k].dst_stride;
-        L.m[i].first_tile = p.first_tile[i];
         L.m[i].shift = wt_radix_shift(types[k]);
         L.m[i].epi = 0;
         L.m[i].nb1 = L.m[i].nb2 = 0;
@@ -975,22 +977,25 @@ static int mul_mat_q8k_tiled_launch(void *stream, const int *types, int n_mats, 
         L.m[1].epi = WT_EPI_ROPE_CACHE; L.m[1].nb1 = qkv->k_nb1; L.m[1].nb2 = qkv->k_nb2;
         L.m[2].epi = WT_EPI_CACHE;      L.m[2].nb1 = qkv->v_nb1; L.m[2].nb2 = qkv->v_nb2;
     }
-    L.n_col_tiles = p.n_col_tiles;
-    L.n_tiles = p.n_tiles;
-    L.n_tiles_padded = (p.n_tiles + 7) & ~7;
+    const int64_t nsb = K / QKK;
+    MI355_REQUIRE(nsb < (int64_t(1) << 31) && B < (int64_t(1) << 31), "mul_mat_q8k_tiled: K=%lld or B=%lld out of range", (long long)K, (long long)B);
+    L.sb_per_slice = (int)((nsb + p.slices - 1) / p.slices);
     if (p.slices > 1) {   // partial sums: one N x B slab per slice in the workspace
         L.m[0].dst = (float *)ws;
         L.m[0].residual = nullptr;
         L.m[0].dst_stride = Ns[0];
     }
-    const dim3 grid((unsigned)L.n_tiles_padded, (unsigned)p.slices);
+    const dim3 grid((unsigned)((p.n_tiles + 7) & ~7), (unsigned)p.slices);
+#define MI355_WT_ARGS \
+    grid, dim3(512), 0, s, images[0], images[1], images[2], (const int8_t *)act, p.first_tile[1], p.first_tile[2], p.n_tiles, p.n_col_tiles, (int)nsb, (int)B, L, wt_route{}
     if (qkv) {
-        if (all_q6) MI355_LAUNCH((k_mmq_w<MI355_Q6_K, false, true>), grid, dim3(512), 0, s, L, (const int8_t *)act, K, B, wt_route{});
-        else MI355_LAUNCH((k_mmq_w<MI355_Q4_K, false, true>), grid, dim3(512), 0, s, L, (const int8_t *)act, K, B, wt_route{});
+        if (all_q6) MI355_LAUNCH((k_mmq_w<MI355_Q6_K, false, true>), MI355_WT_ARGS);
+        else MI355_LAUNCH((k_mmq_w<MI355_Q4_K, false, true>), MI355_WT_ARGS);
         return launch_status("k_mmq_w (Q/K/V)");
     }
-    if (all_q6) MI355_LAUNCH(k_mmq_w<MI355_Q6_K>, grid, dim3(512), 0, s, L, (const int8_t *)act, K, B, wt_route{});
-    else MI355_LAUNCH(k_mmq_w<MI355_Q4_K>, grid, dim3(512), 0, s, L, (const int8_t *)act, K, B, wt_route{});
+    if (all_q6) MI355_LAUNCH(k_mmq_w<MI355_Q6_K>, MI355_WT_ARGS);
+    else MI355_LAUNCH(k_mmq_w<MI355_Q4_K>, MI355_WT_ARGS);
+#undef MI355_WT_ARGS
     if (p.slices > 1 && norm && Ns[0] <= 4096 && mats[0].dst_stride % 4 == 0 && ((uintptr_t)mats[0].dst & 15) == 0 &&
         (mats[0].residual == nullptr || ((uintptr_t)mats[0].residual & 15) == 0)) {
         launch_split_sum_norm(s, (const float *)ws, mats[0].dst, mats[0].residual, Ns[0], B, mats[0].dst_stride, p.slices, norm->w, norm->eps, norm->y,
@@ -1068,25 +1073,24 @@ int mi355_mul_mat_id_q8k_tiled(void *stream, int type, const void *expert_tiles,
     wt_launch L;
     L.rope = wt_rope{nullptr, nullptr, 0, 0};
     for (int i = 0; i < 3; i++) {
-        L.m[i].w_img = (const int8_t *)expert_tiles;
         L.m[i].dst = dst;
         L.m[i].residual = nullptr;
         L.m[i].N = N;
         L.m[i].dst_stride = N;
-        L.m[i].first_tile = i == 0 ? 0 : 0x7fffffff;
         L.m[i].shift = wt_radix_shift(type);
         L.m[i].epi = 0;
         L.m[i].nb1 = L.m[i].nb2 = 0;
     }
     const int64_t n_row_tiles = (N + WT_BM - 1) / WT_BM;
     MI355_REQUIRE(n_row_tiles * max_tiles + 8 < (1 << 30), "mul_mat_id_q8k_tiled: too many tiles");
-    L.n_col_tiles = (int)max_tiles;
-    L.n_tiles = (int)(n_row_tiles * max_tiles);
-    L.n_tiles_padded = (L.n_tiles + 7) & ~7;
+    const int n_all = (int)(n_row_tiles * max_tiles);
+    MI355_REQUIRE(K / QKK < (int64_t(1) << 31) && B_img < (int64_t(1) << 31), "mul_mat_id_q8k_tiled: too many rows or too long ones");
+    L.sb_per_slice = (int)(K / QKK);
+    const int8_t *image = (const int8_t *)expert_tiles;
     const wt_route rt = {dst_row, tiles, n_tiles, (int64_t)expert_tiles_bytes};
-    const dim3 grid((unsigned)L.n_tiles_padded);
-    if (wt_radix_shift(type) == 6) MI355_LAUNCH((k_mmq_w<MI355_Q6_K, true>), grid, dim3(512), 0, s, L, (const int8_t *)img, K, B_img, rt);
-    else MI355_LAUNCH((k_mmq_w<MI355_Q4_K, true>), grid, dim3(512), 0, s, L, (const int8_t *)img, K, B_img, rt);
+    const dim3 grid((unsigned)((n_all + 7) & ~7));
+    if (wt_radix_shift(type) == 6) MI355_LAUNCH((k_mmq_w<MI355_Q6_K, true>), grid, dim3(512), 0, s, image, image, image, (const int8_t *)img, 0x7fffffff, 0x7fffffff, n_all, (int)max_tiles, (int)(K / QKK), (int)B_img, L, rt);
+    else MI355_LAUNCH((k_mmq_w<MI355_Q4_K, true>), grid, dim3(512), 0, s, image, image, image, (const int8_t *)img, 0x7fffffff, 0x7fffffff, n_all, (int)max_tiles, (int)(K / QKK), (int)B_img, L, rt);
     return launch_status("k_mmq_w (routed)");
 }
 
