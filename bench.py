@@ -72,7 +72,7 @@ def traffic_from(fetch_dir, write_dir):
     fetch_b = out["FETCH_SIZE"][0] * out["FETCH_SIZE"][5]
     write_b = out["WRITE_SIZE"][0] * out["WRITE_SIZE"][5]
     lines = [
-        "HBM traffic of the roofline kernel of bench.py: k_gemv_gate_up_blk<Q4_K, 1 column, 8 waves, 4 + 4 rows in flight> on the ffn_gate + ffn_up",
+        "HBM traffic of the roofline kernel of bench.py: k_gemv_gate_up_blk<Q4_K, 1 column, 8 waves, 2 + 2 rows in flight> on the ffn_gate + ffn_up",
         "matrices of one layer (2 x 14336 x 4096 Q4_K, SiLU * up + Q8_1 inside) - the launch a decoded token makes 32 times - on one MI355X",
         "",
         "commands (from /tmp, TMPDIR=/tmp; counters in their own runs, no trace domains):",
@@ -475,7 +475,7 @@ def main():
     alg_bytes = 2 * (N * K * 144 // 256) + (K + K // 4) + 2 * 4 * N + (N + N // 4)
     achieved = alg_bytes / us / 1e3                                       # GB/s
     traffic, traffic_commit = read_traffic()
-    roofline = {"kernel": "k_gemv_gate_up_blk<Q4_K, 1 column, 8 waves, 4 + 4 rows in flight> on ffn_gate + ffn_up with SiLU * up + Q8_1, 2 x 14336 x 4096 "
+    roofline = {"kernel": "k_gemv_gate_up_blk<Q4_K, 1 column, 8 waves, 2 + 2 rows in flight> on ffn_gate + ffn_up with SiLU * up + Q8_1, 2 x 14336 x 4096 "
                           "(the launch the timed step makes once per layer)", "bound": "hbm", "achieved": round(achieved, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                 "traffic_source": "profiles/%s, measured at commit %s" % (os.path.basename(TRAFFIC_FILE), traffic_commit) if traffic else None,

@@ -346,8 +346,8 @@ extern __shared__ __attribute__((aligned(16))) uint8_t s_act_dyn[];
 // bytes of LDS for the group's copy of the activation, or 0 when every wave reads it from memory.  The copy pays when the
 // launch has several generations of groups per compute unit (its round trip then hides behind other groups' loads, and the
 // activation reads it saves are the larger part of the launch's L2 traffic): output projection 98.9 -> 77.5 us (6.8 TB/s),
-// 14336 x 4096 8.6 -> 8.0 us.  A launch whose groups are all resident at once (wo, ffn_down, Q/K/V: ~1000 groups) is one
-// dependent chain per wave, and the copy's barrier lengthens it (+0.3 to +0.7 us measured).  Up to four activation rows, and
+// 14336 x 4096 8.6 -> 8.0 us.  One row against one matrix of few rows (wo, ffn_down) has a kernel of its own, gemv_row.hip; the launches of several rows or matrices
+// whose groups are all resident at once are one dependent chain per wave, and there the copy's barrier lengthened it (+0.3 to +0.7 us measured).  Up to four activation rows, and
 // small enough that eight groups still fit a compute unit.
 // Measured and not adopted: splitting K over the four waves of a group (each wave reads a quarter of the activation, partial
 // sums meet in LDS at the end) - Q4_K 4096 x 4096 4.9 -> 4.3 us and 14336 x 4096 8.2 -> 7.9 us, but Q6_K slower throughout
