@@ -129,7 +129,9 @@ __device__ __forceinline__ void fs_slopes(const fattn_args &a, int64_t head0, fl
 // The soft-max update of the state with one tile's raw scores (q . k of this lane's cell and the four heads), and P^T (head, cell)
 // as f16 into the wave's 512 bytes of LDS at p_wr (= base + 2 * lane), where fs_output reads it back as the A operand.  LDS serves a
 // wave's operations in order: those reads see these writes, and the next tile's writes come after them.
-template <int NH = 4>   // heads the group has at most
+// SPLIT: a second value per cell, 512 bytes on: what f16 leaves of p, times FS_LO (p to 22 bits, and as close below 2^-14, where f16 itself has fewer)
+constexpr float FS_LO = 2048.0f;
+template <int NH = 4, bool SPLIT = false>   // NH: heads the group has at most
 __device__ __forceinline__ void fs_softmax(const float (&raw)[4], float mv, float scale, float softcap, const float (&slope)[4], unsigned p_wr, fs_state &S) {
     constexpr float NEG = -FLT_MAX / 2;
     const bool valid = mv != -INFINITY;
@@ -148,25 +150,33 @@ __device__ __forceinline__ void fs_softmax(const float (&raw)[4], float mv, floa
         S.o1[r] *= f;
         const u32 ph = float_to_half_bits(p);
         asm volatile("ds_write_b16 %0, %1 offset:%2" ::"v"(p_wr), "v"(ph), "n"(r * FS_TILE * 2) : "memory");
+        if constexpr (SPLIT) {
+            const u32 pl = float_to_half_bits((p - half_bits_to_float((unsigned short)ph)) * FS_LO);
+            asm volatile("ds_write_b16 %0, %1 offset:%2" ::"v"(p_wr), "v"(pl), "n"((4 + r) * FS_TILE * 2) : "memory");
+        }
     }
 }
 // Scores of one tile (kc: the 16 chunks of this lane's K row), then fs_softmax.
-template <int NH = 4>
+template <int NH = 4, bool SPLIT = false>
 __device__ __forceinline__ void fs_scores(const u32 (&qv)[FS_D / 2], const u32x4 (&kc)[16], float mv, float scale, float softcap, const float (&slope)[4],
                                           unsigned p_wr, fs_state &S) {
-    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+    constexpr int CH = SPLIT ? 8 : 2;   // chains of matrix operations, added as a tree
+    f32x4 sc[CH];
+#pragma unroll
+    for (int i = 0; i < CH; i++) sc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < 16; c++) {
         const u32 a0 = qv[4 * c], a1 = qv[4 * c + 1], a2 = qv[4 * c + 2], a3 = qv[4 * c + 3];
         const u32 b0 = kc[c][0], b1 = kc[c][1], b2 = kc[c][2], b3 = kc[c][3];
         const u32x2 qa = {a0, a1}, qb = {a2, a3}, ka = {b0, b1}, kb2 = {b2, b3};
+        f32x4 &s0 = sc[2 * c % CH], &s1 = sc[(2 * c + 1) % CH];
         s0 = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, qa), __builtin_bit_cast(f16x4, ka), s0, 0, 0, 0);
         s1 = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, qb), __builtin_bit_cast(f16x4, kb2), s1, 0, 0, 0);
     }
     float raw[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++) raw[r] = s0[r] + s1[r];
-    fs_softmax<NH>(raw, mv, scale, softcap, slope, p_wr, S);
+    for (int r = 0; r < 4; r++) raw[r] = CH == 2 ? sc[0][r] + sc[1][r] : ((sc[0][r] + sc[1 % CH][r]) + (sc[2 % CH][r] + sc[3 % CH][r])) + ((sc[4 % CH][r] + sc[5 % CH][r]) + (sc[6 % CH][r] + sc[7 % CH][r]));
+    fs_softmax<NH, SPLIT>(raw, mv, scale, softcap, slope, p_wr, S);
 }
 // This lane's offset inside a row-major V tile for the transposing reads of fs_output: lane l' = lane % 16 of its 16-lane group
 // g points at row c0 + l' / 4, elements 16 g + 4 (l' % 4) .. + 3
@@ -198,24 +208,43 @@ __device__ __forceinline__ void fs_output(unsigned v_addr, unsigned p_rd, fs_sta
     }
 }
 
-// The same for one half of the elements (H = 0: lane, 1: 64 + lane), same sums
-template <int H> __device__ __forceinline__ void fs_output_half(unsigned v_addr, unsigned p_rd, f32x4 &o) {
+// The same for one half of the elements (H = 0: lane, 1: 64 + lane), same sums.  SPLIT: with fs_softmax's second values, in a sum of their own, and four chains for the first; o is written, not added to
+template <int H, bool SPLIT> __device__ __forceinline__ void fs_output_half(unsigned v_addr, unsigned p_rd, f32x4 &o) {
     constexpr int NJ = 16;
-    u32x2 v[NJ], pa[NJ];
+    u32x2 v[NJ], pa[NJ], pl[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const unsigned addr = v_addr + (unsigned)(j * 4 * FS_ROW);
         asm volatile("ds_read_b64 %0, %1" : "=v"(pa[j]) : "v"(p_rd + (unsigned)(j * 8)));
         if constexpr (H == 0) asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v[j]) : "v"(addr));
         else asm volatile("ds_read_b64_tr_b16 %0, %1 offset:128" : "=v"(v[j]) : "v"(addr));
+        if constexpr (SPLIT) asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(pl[j]) : "v"(p_rd + (unsigned)(j * 8)), "n"(4 * FS_TILE * 2));
     }
 #pragma unroll
     for (int jb = 0; jb < NJ; jb += 8)
         asm volatile("s_waitcnt lgkmcnt(0)"
                      : "+v"(v[jb]), "+v"(v[jb + 1]), "+v"(v[jb + 2]), "+v"(v[jb + 3]), "+v"(v[jb + 4]), "+v"(v[jb + 5]), "+v"(v[jb + 6]), "+v"(v[jb + 7]),
                        "+v"(pa[jb]), "+v"(pa[jb + 1]), "+v"(pa[jb + 2]), "+v"(pa[jb + 3]), "+v"(pa[jb + 4]), "+v"(pa[jb + 5]), "+v"(pa[jb + 6]), "+v"(pa[jb + 7]));
+    if constexpr (SPLIT) {
 #pragma unroll
-    for (int j = 0; j < NJ; j++) o = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pa[j]), __builtin_bit_cast(f16x4, v[j]), o, 0, 0, 0);
+        for (int jb = 0; jb < NJ; jb += 8)
+            asm volatile("" : "+v"(pl[jb]), "+v"(pl[jb + 1]), "+v"(pl[jb + 2]), "+v"(pl[jb + 3]), "+v"(pl[jb + 4]), "+v"(pl[jb + 5]), "+v"(pl[jb + 6]), "+v"(pl[jb + 7]));
+    }
+    if constexpr (!SPLIT) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) o = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pa[j]), __builtin_bit_cast(f16x4, v[j]), o, 0, 0, 0);
+    } else {
+        f32x4 hi[4], lo = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; i++) hi[i] = lo;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            hi[j % 4] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pa[j]), __builtin_bit_cast(f16x4, v[j]), hi[j % 4], 0, 0, 0);
+            lo = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pl[j]), __builtin_bit_cast(f16x4, v[j]), lo, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) o[r] = ((hi[0][r] + hi[1][r]) + (hi[2][r] + hi[3][r])) + lo[r] * (1.0f / FS_LO);
+    }
 }
 
 // The states of a group's waves (at most NWV) meet in LDS: one partial result per group.  all: `stride` floats per wave, whose LDS reads lie behind it; head r's
@@ -793,21 +822,26 @@ __global__ void __launch_bounds__(((ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK
 // 32 / 8 heads, 512 cells, us: one group per kv head 7.6, two 6.3, four (NH = 2) 5.9, eight (NH = 1) 5.8; 288 cells 7.1, 5.7, 5.2, 5.1.  A group too many costs a second round: 160 / 40 heads,
 // 512 cells 11.1 with NH = 1, 6.8 with 2, 7.4 with 4; 256 / 64 heads 11.2, 6.8, 7.4.  With 32-bit offsets and arguments in registers, a layer of the 8B model 45.9 -> 45.2, with one
 // head per group 44.3 (a token 1553 -> 1508).
-constexpr int FSS_MAX_WAVES = 8;
+//   SPLIT: up to FSS_SPLIT_CELLS cells, where the vector kernel, with f32 probabilities and masked cells not read, is the other choice: each probability as two f16 values, V of masked
+//     cells as zeros, sums in more and shorter chains.  Relative error against 64 bits (2-norm; scores of deviation 1 and 6) 1.7e-7 at 32 cells, 2.5e-7 at 256, the vector kernel's
+//     1.8e-7 and 2.6e-7 (3.8e-7 at 256 with the chains of the other form).  The vector kernel exchanges each score between sixteen lanes; 32 / 8 heads, 32 / 128 / 256 cells, us: 4.3, 4.3, 5.5
+//     there, 3.5, 3.8, 4.6 here; 512 / 128 heads 6.4, 6.7, 8.9 and 4.1, 4.9, 6.7; a token of the 8B model 1395 -> 1331.
+constexpr int FSS_MAX_WAVES = 8, FSS_SPLIT_WAVES = 4, FSS_SPLIT_CELLS = FSS_SPLIT_WAVES * FS_TILE;
 
 // The arguments ahead of `a` are all that the requests need, and in registers when a wave starts (fourteen words): read from `a` they are two trips to memory, the second
 // behind the mask's.  cells: Nkv and, from bit 16, R.  A tile's rows are less than 2^30 bytes apart: 32-bit offsets from one scalar address per wave.
-template <int PARTS, int NH>
-__global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(const uint8_t *__restrict__ q, const uint8_t *__restrict__ k, const uint8_t *__restrict__ v,
+template <int PARTS, int NH, bool SPLIT>
+__global__ void __launch_bounds__((SPLIT ? FSS_SPLIT_WAVES : FSS_MAX_WAVES) * 64, SPLIT ? 2 : 1) k_fattn_dec_short(const uint8_t *__restrict__ q, const uint8_t *__restrict__ k, const uint8_t *__restrict__ v,
                                                                            const uint8_t *__restrict__ mask, u32 q_nb2, u32 k_nb1, u32 k_nb2, u32 v_nb1, u32 v_nb2, u32 cells,
                                                                            fattn_args a) {
-    static_assert(PARTS == 1 || PARTS == 2, "whole rows of V or halves");
+    static_assert(PARTS == 2 || (PARTS == 1 && !SPLIT), "whole rows of V or halves");
+    constexpr int MAXW = SPLIT ? FSS_SPLIT_WAVES : FSS_MAX_WAVES;
     constexpr int DO = FS_D / PARTS, VIT = 16 / PARTS, VCH = 16 / PARTS;   // output elements of the group; V loads; 16-byte chunks of V per row
-    __shared__ __attribute__((aligned(1024))) uint8_t tbuf[FSS_MAX_WAVES * FS_KT];
-    __shared__ __attribute__((aligned(16))) unsigned short pbuf[FSS_MAX_WAVES][4][FS_TILE];
-    __shared__ float s_m[FSS_MAX_WAVES][NH], s_l[FSS_MAX_WAVES][NH];
-    __shared__ float s_o[FSS_MAX_WAVES][NH][DO];
-    __shared__ __attribute__((aligned(16))) uint8_t qbuf[FSS_MAX_WAVES][FS_QLDS];
+    __shared__ __attribute__((aligned(1024))) uint8_t tbuf[MAXW * FS_KT];
+    __shared__ __attribute__((aligned(16))) unsigned short pbuf[MAXW][SPLIT ? 8 : 4][FS_TILE];
+    __shared__ float s_m[MAXW][NH], s_l[MAXW][NH];
+    __shared__ float s_o[MAXW][NH][DO];
+    __shared__ __attribute__((aligned(16))) uint8_t qbuf[MAXW][FS_QLDS];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int64_t hk = blockIdx.x;
@@ -863,16 +897,21 @@ __global__ void __launch_bounds__(FSS_MAX_WAVES * 64, 1) k_fattn_dec_short(const
     fs_state S;
     fs_init(S);
     const unsigned p_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned short *)&pbuf[wave][0][0];
-    fs_scores<NH>(qv, kc, half_bits_to_float(mbits), scale, a.softcap, slope, p_base + (unsigned)lane * 2, S);
+    fs_scores<NH, SPLIT>(qv, kc, half_bits_to_float(mbits), scale, a.softcap, slope, p_base + (unsigned)lane * 2, S);
 
-    // V through the same bytes, row-major (the K rows are in registers)
+    // V through the same bytes, row-major (the K rows are in registers).  SPLIT: zeros for masked cells, whatever they hold: their weight of zero would not hide an infinity
+    const uint64_t in_use = __ballot(half_bits_to_float(mbits) != -INFINITY);
 #pragma unroll
-    for (int i = 0; i < VIT; i++) *(u32x4 *)(tb + ((64 / VIT) * i + vsub) * FS_ROW + (vpos << 4)) = vraw[i];
+    for (int i = 0; i < VIT; i++) {
+        if constexpr (SPLIT)
+            if (!((in_use >> ((64 / VIT) * i + vsub)) & 1)) vraw[i] = u32x4{0, 0, 0, 0};
+        *(u32x4 *)(tb + ((64 / VIT) * i + vsub) * FS_ROW + (vpos << 4)) = vraw[i];
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // fs_output reads LDS through inline assembly: nothing may be moved across
     const unsigned v_addr = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)tb + fs_v_lane(lane), p_rd = p_base + (unsigned)(lane & 3) * (FS_TILE * 2);
     if constexpr (PARTS == 1) fs_output(v_addr, p_rd, S);
-    else if (part == 0) fs_output_half<0>(v_addr, p_rd, S.o0);   // uniform
-    else fs_output_half<1>(v_addr, p_rd, S.o0);
+    else if (part == 0) fs_output_half<0, SPLIT>(v_addr, p_rd, S.o0);   // uniform
+    else fs_output_half<1, SPLIT>(v_addr, p_rd, S.o0);
 
     // ---- the waves' states meet in LDS
 #pragma unroll
@@ -912,10 +951,20 @@ int launch_fattn_dec_short(hipStream_t s, fattn_args &a, int64_t D) {
     constexpr int64_t CU = 256;   // compute units
     const int n_waves = (int)((a.Nkv + FS_TILE - 1) / FS_TILE);
 #define MI355_FSS_ARGS dim3((unsigned)n_waves * 64), 0, s, a.q, a.k, a.v, a.mask, (u32)a.q_nb2, (u32)a.k_nb1, (u32)a.k_nb2, (u32)a.v_nb1, (u32)a.v_nb2, (u32)a.Nkv | (u32)R << 16, a
-    if (2 * a.Hq <= CU) MI355_LAUNCH((k_fattn_dec_short<2, 1>), dim3((unsigned)a.Hkv, 2, (unsigned)R), MI355_FSS_ARGS);
-    else if (2 * a.Hkv * ((R + 1) / 2) <= CU) MI355_LAUNCH((k_fattn_dec_short<2, 2>), dim3((unsigned)a.Hkv, 2, (unsigned)((R + 1) / 2)), MI355_FSS_ARGS);
-    else if (2 * a.Hkv <= CU) MI355_LAUNCH((k_fattn_dec_short<2, 4>), dim3((unsigned)a.Hkv, 2), MI355_FSS_ARGS);
-    else MI355_LAUNCH((k_fattn_dec_short<1, 4>), dim3((unsigned)a.Hkv), MI355_FSS_ARGS);
+#define MI355_FSS_LAUNCH(SPLIT, RES)                                                                                                                                        \
+    if (2 * a.Hq <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 1, SPLIT>), dim3((unsigned)a.Hkv, 2, (unsigned)R), MI355_FSS_ARGS);                                              \
+    else if (2 * a.Hkv * ((R + 1) / 2) <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 2, SPLIT>), dim3((unsigned)a.Hkv, 2, (unsigned)((R + 1) / 2)), MI355_FSS_ARGS);            \
+    else if (2 * a.Hkv <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 4, SPLIT>), dim3((unsigned)a.Hkv, 2), MI355_FSS_ARGS);
+    if (a.Nkv <= FSS_SPLIT_CELLS) {
+        // two groups of this form share a compute unit's LDS, which pays for groups of one wave: 195 / 65 heads, 64 cells 4.6 -> 4.2 us, 512 / 128 heads 4.8 -> 4.1; with more waves not
+        // (160 / 40 heads, 128 cells 4.0 -> 4.4, 256 cells 4.8 -> 6.0)
+        MI355_FSS_LAUNCH(true, (a.Nkv <= FS_TILE ? 2 * CU : CU))
+        else return 1;
+    } else {
+        MI355_FSS_LAUNCH(false, CU)
+        else MI355_LAUNCH((k_fattn_dec_short<1, 4, false>), dim3((unsigned)a.Hkv), MI355_FSS_ARGS);
+    }
+#undef MI355_FSS_LAUNCH
 #undef MI355_FSS_ARGS
     return launch_status("k_fattn_dec_short");
 }
