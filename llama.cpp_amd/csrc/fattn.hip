@@ -646,7 +646,7 @@ int mi355_flash_attn_ext_quant(void *stream, const float *q, const void *k, cons
     // 3000 cells fewer than 512 of its 64-cell tiles exist and the kernel below is ahead (10.2 against 11.2 us at 2048).
     constexpr int64_t stream_min = 3072;
     // Up to 512 cells: one launch with a wave per 64 cells (32 / 8 heads, 288 / 512 cells 5.1 / 5.8 us, against 9.0 for the split form below with its merge
-    // launch; 256 cells 4.6, the vector kernel further down 5.5).  Up to 256 cells the vector kernel keeps calls whose groups would not all be resident at once
+    // launch; 256 cells 4.7, the vector kernel further down 5.6).  Up to 256 cells the vector kernel keeps calls whose groups would not all be resident at once
     constexpr int64_t short_max = 512;
     if (Nq == 1 && Nkv <= short_max && D == 128 && R <= 4) {
         const int rc = launch_fattn_dec_short(s, a, D);

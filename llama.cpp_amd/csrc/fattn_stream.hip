@@ -129,9 +129,8 @@ __device__ __forceinline__ void fs_slopes(const fattn_args &a, int64_t head0, fl
 // The soft-max update of the state with one tile's raw scores (q . k of this lane's cell and the four heads), and P^T (head, cell)
 // as f16 into the wave's 512 bytes of LDS at p_wr (= base + 2 * lane), where fs_output reads it back as the A operand.  LDS serves a
 // wave's operations in order: those reads see these writes, and the next tile's writes come after them.
-// SPLIT: a second value per cell, 512 bytes on: what f16 leaves of p, times FS_LO (p to 22 bits, and as close below 2^-14, where f16 itself has fewer)
-constexpr float FS_LO = 2048.0f;
-template <int NH = 4, bool SPLIT = false>   // NH: heads the group has at most
+// P32: as f32, 256 bytes per head, for fs_output_f32
+template <int NH = 4, bool P32 = false>   // NH: heads the group has at most
 __device__ __forceinline__ void fs_softmax(const float (&raw)[4], float mv, float scale, float softcap, const float (&slope)[4], unsigned p_wr, fs_state &S) {
     constexpr float NEG = -FLT_MAX / 2;
     const bool valid = mv != -INFINITY;
@@ -148,19 +147,19 @@ __device__ __forceinline__ void fs_softmax(const float (&raw)[4], float mv, floa
         S.lsum[r] = S.lsum[r] * f + p;
         S.o0[r] *= f;
         S.o1[r] *= f;
-        const u32 ph = float_to_half_bits(p);
-        asm volatile("ds_write_b16 %0, %1 offset:%2" ::"v"(p_wr), "v"(ph), "n"(r * FS_TILE * 2) : "memory");
-        if constexpr (SPLIT) {
-            const u32 pl = float_to_half_bits((p - half_bits_to_float((unsigned short)ph)) * FS_LO);
-            asm volatile("ds_write_b16 %0, %1 offset:%2" ::"v"(p_wr), "v"(pl), "n"((4 + r) * FS_TILE * 2) : "memory");
+        if constexpr (P32) {
+            *(float __attribute__((address_space(3))) *)(p_wr + (unsigned)(r * FS_TILE * 4)) = p;
+        } else {
+            const u32 ph = float_to_half_bits(p);
+            asm volatile("ds_write_b16 %0, %1 offset:%2" ::"v"(p_wr), "v"(ph), "n"(r * FS_TILE * 2) : "memory");
         }
     }
 }
 // Scores of one tile (kc: the 16 chunks of this lane's K row), then fs_softmax.
-template <int NH = 4, bool SPLIT = false>
+template <int NH = 4, bool P32 = false>
 __device__ __forceinline__ void fs_scores(const u32 (&qv)[FS_D / 2], const u32x4 (&kc)[16], float mv, float scale, float softcap, const float (&slope)[4],
                                           unsigned p_wr, fs_state &S) {
-    constexpr int CH = SPLIT ? 8 : 2;   // chains of matrix operations, added as a tree
+    constexpr int CH = P32 ? 8 : 2;   // chains of matrix operations, added as a tree
     f32x4 sc[CH];
 #pragma unroll
     for (int i = 0; i < CH; i++) sc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -176,7 +175,7 @@ __device__ __forceinline__ void fs_scores(const u32 (&qv)[FS_D / 2], const u32x4
     float raw[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) raw[r] = CH == 2 ? sc[0][r] + sc[1][r] : ((sc[0][r] + sc[1 % CH][r]) + (sc[2 % CH][r] + sc[3 % CH][r])) + ((sc[4 % CH][r] + sc[5 % CH][r]) + (sc[6 % CH][r] + sc[7 % CH][r]));
-    fs_softmax<NH, SPLIT>(raw, mv, scale, softcap, slope, p_wr, S);
+    fs_softmax<NH, P32>(raw, mv, scale, softcap, slope, p_wr, S);
 }
 // This lane's offset inside a row-major V tile for the transposing reads of fs_output: lane l' = lane % 16 of its 16-lane group
 // g points at row c0 + l' / 4, elements 16 g + 4 (l' % 4) .. + 3
@@ -208,42 +207,52 @@ __device__ __forceinline__ void fs_output(unsigned v_addr, unsigned p_rd, fs_sta
     }
 }
 
-// The same for one half of the elements (H = 0: lane, 1: 64 + lane), same sums.  SPLIT: with fs_softmax's second values, in a sum of their own, and four chains for the first; o is written, not added to
-template <int H, bool SPLIT> __device__ __forceinline__ void fs_output_half(unsigned v_addr, unsigned p_rd, f32x4 &o) {
+// The same for one half of the elements (H = 0: lane, 1: 64 + lane), same sums
+template <int H> __device__ __forceinline__ void fs_output_half(unsigned v_addr, unsigned p_rd, f32x4 &o) {
     constexpr int NJ = 16;
-    u32x2 v[NJ], pa[NJ], pl[NJ];
+    u32x2 v[NJ], pa[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const unsigned addr = v_addr + (unsigned)(j * 4 * FS_ROW);
         asm volatile("ds_read_b64 %0, %1" : "=v"(pa[j]) : "v"(p_rd + (unsigned)(j * 8)));
         if constexpr (H == 0) asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v[j]) : "v"(addr));
         else asm volatile("ds_read_b64_tr_b16 %0, %1 offset:128" : "=v"(v[j]) : "v"(addr));
-        if constexpr (SPLIT) asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(pl[j]) : "v"(p_rd + (unsigned)(j * 8)), "n"(4 * FS_TILE * 2));
     }
 #pragma unroll
     for (int jb = 0; jb < NJ; jb += 8)
         asm volatile("s_waitcnt lgkmcnt(0)"
                      : "+v"(v[jb]), "+v"(v[jb + 1]), "+v"(v[jb + 2]), "+v"(v[jb + 3]), "+v"(v[jb + 4]), "+v"(v[jb + 5]), "+v"(v[jb + 6]), "+v"(v[jb + 7]),
                        "+v"(pa[jb]), "+v"(pa[jb + 1]), "+v"(pa[jb + 2]), "+v"(pa[jb + 3]), "+v"(pa[jb + 4]), "+v"(pa[jb + 5]), "+v"(pa[jb + 6]), "+v"(pa[jb + 7]));
-    if constexpr (SPLIT) {
 #pragma unroll
-        for (int jb = 0; jb < NJ; jb += 8)
-            asm volatile("" : "+v"(pl[jb]), "+v"(pl[jb + 1]), "+v"(pl[jb + 2]), "+v"(pl[jb + 3]), "+v"(pl[jb + 4]), "+v"(pl[jb + 5]), "+v"(pl[jb + 6]), "+v"(pl[jb + 7]));
-    }
-    if constexpr (!SPLIT) {
+    for (int j = 0; j < NJ; j++) o = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pa[j]), __builtin_bit_cast(f16x4, v[j]), o, 0, 0, 0);
+}
+// One half of the elements (v_lane: that half of the row-major V tile + fs_v_lane) with the probabilities as f32: o[r] = sum over the tile's cells of p[r][cell] * V[cell] at the
+// lane's element, each product and sum rounded once, as the vector kernel does it.  V comes from the transposing reads, four cells each; p is NH x 64 floats.  Four chains of sixteen
+// cells, added as a tree.  One head: 64 multiply-adds that take V as f16, p read by all lanes at one address.  More: the matrix instruction for f32 (lane = row lane % 4 of P and column
+// lane % 4 of V, as in fs_output, one cell per step), which serves four heads at once.  Four heads with
+// multiply-adds: 512 / 128 heads, 256 cells 8.0 us, with the matrix instruction 7.5.
+template <int NH> __device__ __forceinline__ void fs_output_f32(const uint8_t __attribute__((address_space(3))) *v_lane, const float __attribute__((address_space(3))) *p, int lane, f32x4 &o) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    const float __attribute__((address_space(3))) *mine = p + (NH > 1 && (lane & 3) < NH ? lane & 3 : 0) * FS_TILE;   // rows past the group's heads repeat the first one and are not used
+    float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 acc[4];
 #pragma unroll
-        for (int j = 0; j < NJ; j++) o = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pa[j]), __builtin_bit_cast(f16x4, v[j]), o, 0, 0, 0);
-    } else {
-        f32x4 hi[4], lo = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 4; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; i++) hi[i] = lo;
+    for (int j = 0; j < FS_TILE / 4; j++) {
+        const f16x4 v = __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(v_lane + j * 4 * FS_ROW)));
+        const f32x4 pr = *(const f32x4 __attribute__((address_space(3))) *)(mine + 4 * j);
 #pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            hi[j % 4] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pa[j]), __builtin_bit_cast(f16x4, v[j]), hi[j % 4], 0, 0, 0);
-            lo = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, pl[j]), __builtin_bit_cast(f16x4, v[j]), lo, 0, 0, 0);
+        for (int i = 0; i < 4; i++) {
+            if constexpr (NH == 1) sum[i] = __builtin_fmaf(pr[i], (float)v[i], sum[i]);
+            else acc[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(pr[i], (float)v[i], acc[i], 0, 0, 0);
         }
+    }
+    if constexpr (NH == 1) {
+        o[0] = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++) o[r] = ((hi[0][r] + hi[1][r]) + (hi[2][r] + hi[3][r])) + lo[r] * (1.0f / FS_LO);
+        for (int r = 0; r < NH; r++) o[r] = (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
     }
 }
 
@@ -822,23 +831,24 @@ __global__ void __launch_bounds__(((ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK
 // 32 / 8 heads, 512 cells, us: one group per kv head 7.6, two 6.3, four (NH = 2) 5.9, eight (NH = 1) 5.8; 288 cells 7.1, 5.7, 5.2, 5.1.  A group too many costs a second round: 160 / 40 heads,
 // 512 cells 11.1 with NH = 1, 6.8 with 2, 7.4 with 4; 256 / 64 heads 11.2, 6.8, 7.4.  With 32-bit offsets and arguments in registers, a layer of the 8B model 45.9 -> 45.2, with one
 // head per group 44.3 (a token 1553 -> 1508).
-//   SPLIT: up to FSS_SPLIT_CELLS cells, where the vector kernel, with f32 probabilities and masked cells not read, is the other choice: each probability as two f16 values, V of masked
-//     cells as zeros, sums in more and shorter chains.  Relative error against 64 bits (2-norm; scores of deviation 1 and 6) 1.7e-7 at 32 cells, 2.5e-7 at 256, the vector kernel's
-//     1.8e-7 and 2.6e-7 (3.8e-7 at 256 with the chains of the other form).  The vector kernel exchanges each score between sixteen lanes; 32 / 8 heads, 32 / 128 / 256 cells, us: 4.3, 4.3, 5.5
-//     there, 3.5, 3.8, 4.6 here; 512 / 128 heads 6.4, 6.7, 8.9 and 4.1, 4.9, 6.7; a token of the 8B model 1395 -> 1331.
-constexpr int FSS_MAX_WAVES = 8, FSS_SPLIT_WAVES = 4, FSS_SPLIT_CELLS = FSS_SPLIT_WAVES * FS_TILE;
+//   P32: up to FSS_P32_CELLS cells, where the vector kernel, with f32 probabilities and masked cells not read, is the other choice: probabilities as f32 on the vector units (fs_output_f32),
+//     V of masked cells as zeros, scores in more and shorter chains.  (Probabilities as the sum of two f16 values on the f16 matrix instruction gave NaN for an infinite value of a visible
+//     cell - zero or a negative remainder times infinity - and lost the lower bits of weights below 2^-14: 1.6e-4 of an output that weights of 2^-20 .. 2^-30 make, 3e-6 as f32.)  Relative
+//     error against 64 bits, 2-norm, 32 .. 256 cells: 1.1e-7 .. 1.9e-7, the vector kernel's 1.2e-7 .. 1.9e-7.  The vector kernel exchanges each score between sixteen lanes; 32 / 8 heads,
+//     32 / 128 / 256 cells, us: 4.5, 4.7, 5.6 there, 3.7, 3.9, 4.7 here; 512 / 128 heads 7.1, 7.2, 10.8 and 4.7, 6.0, 7.5.
+constexpr int FSS_MAX_WAVES = 8, FSS_P32_WAVES = 4, FSS_P32_CELLS = FSS_P32_WAVES * FS_TILE;
 
 // The arguments ahead of `a` are all that the requests need, and in registers when a wave starts (fourteen words): read from `a` they are two trips to memory, the second
 // behind the mask's.  cells: Nkv and, from bit 16, R.  A tile's rows are less than 2^30 bytes apart: 32-bit offsets from one scalar address per wave.
-template <int PARTS, int NH, bool SPLIT>
-__global__ void __launch_bounds__((SPLIT ? FSS_SPLIT_WAVES : FSS_MAX_WAVES) * 64, SPLIT ? 2 : 1) k_fattn_dec_short(const uint8_t *__restrict__ q, const uint8_t *__restrict__ k, const uint8_t *__restrict__ v,
+template <int PARTS, int NH, bool P32>
+__global__ void __launch_bounds__((P32 ? FSS_P32_WAVES : FSS_MAX_WAVES) * 64, P32 ? 2 : 1) k_fattn_dec_short(const uint8_t *__restrict__ q, const uint8_t *__restrict__ k, const uint8_t *__restrict__ v,
                                                                            const uint8_t *__restrict__ mask, u32 q_nb2, u32 k_nb1, u32 k_nb2, u32 v_nb1, u32 v_nb2, u32 cells,
                                                                            fattn_args a) {
-    static_assert(PARTS == 2 || (PARTS == 1 && !SPLIT), "whole rows of V or halves");
-    constexpr int MAXW = SPLIT ? FSS_SPLIT_WAVES : FSS_MAX_WAVES;
+    static_assert(PARTS == 2 || (PARTS == 1 && !P32), "whole rows of V or halves");
+    constexpr int MAXW = P32 ? FSS_P32_WAVES : FSS_MAX_WAVES, PSZ = P32 ? NH * 4 : 4 * 2;   // PSZ: bytes of probabilities per cell
     constexpr int DO = FS_D / PARTS, VIT = 16 / PARTS, VCH = 16 / PARTS;   // output elements of the group; V loads; 16-byte chunks of V per row
     __shared__ __attribute__((aligned(1024))) uint8_t tbuf[MAXW * FS_KT];
-    __shared__ __attribute__((aligned(16))) unsigned short pbuf[MAXW][SPLIT ? 8 : 4][FS_TILE];
+    __shared__ __attribute__((aligned(16))) uint8_t pbuf[MAXW][FS_TILE * PSZ];
     __shared__ float s_m[MAXW][NH], s_l[MAXW][NH];
     __shared__ float s_o[MAXW][NH][DO];
     __shared__ __attribute__((aligned(16))) uint8_t qbuf[MAXW][FS_QLDS];
@@ -896,22 +906,24 @@ __global__ void __launch_bounds__((SPLIT ? FSS_SPLIT_WAVES : FSS_MAX_WAVES) * 64
 
     fs_state S;
     fs_init(S);
-    const unsigned p_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned short *)&pbuf[wave][0][0];
-    fs_scores<NH, SPLIT>(qv, kc, half_bits_to_float(mbits), scale, a.softcap, slope, p_base + (unsigned)lane * 2, S);
+    const unsigned p_base = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)&pbuf[wave][0];
+    fs_scores<NH, P32>(qv, kc, half_bits_to_float(mbits), scale, a.softcap, slope, p_base + (unsigned)lane * (P32 ? 4 : 2), S);
 
-    // V through the same bytes, row-major (the K rows are in registers).  SPLIT: zeros for masked cells, whatever they hold: their weight of zero would not hide an infinity
+    // V through the same bytes, row-major (the K rows are in registers).  P32: zeros for masked cells, whatever they hold: their weight of zero would not hide an infinity
     const uint64_t in_use = __ballot(half_bits_to_float(mbits) != -INFINITY);
 #pragma unroll
     for (int i = 0; i < VIT; i++) {
-        if constexpr (SPLIT)
+        if constexpr (P32)
             if (!((in_use >> ((64 / VIT) * i + vsub)) & 1)) vraw[i] = u32x4{0, 0, 0, 0};
         *(u32x4 *)(tb + ((64 / VIT) * i + vsub) * FS_ROW + (vpos << 4)) = vraw[i];
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // fs_output reads LDS through inline assembly: nothing may be moved across
     const unsigned v_addr = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)tb + fs_v_lane(lane), p_rd = p_base + (unsigned)(lane & 3) * (FS_TILE * 2);
-    if constexpr (PARTS == 1) fs_output(v_addr, p_rd, S);
-    else if (part == 0) fs_output_half<0, SPLIT>(v_addr, p_rd, S.o0);   // uniform
-    else fs_output_half<1, SPLIT>(v_addr, p_rd, S.o0);
+    if constexpr (P32)
+        fs_output_f32<NH>((const uint8_t __attribute__((address_space(3))) *)(v_addr + (unsigned)(part * 128)), (const float __attribute__((address_space(3))) *)p_base, lane, S.o0);
+    else if constexpr (PARTS == 1) fs_output(v_addr, p_rd, S);
+    else if (part == 0) fs_output_half<0>(v_addr, p_rd, S.o0);   // uniform
+    else fs_output_half<1>(v_addr, p_rd, S.o0);
 
     // ---- the waves' states meet in LDS
 #pragma unroll
@@ -951,13 +963,13 @@ int launch_fattn_dec_short(hipStream_t s, fattn_args &a, int64_t D) {
     constexpr int64_t CU = 256;   // compute units
     const int n_waves = (int)((a.Nkv + FS_TILE - 1) / FS_TILE);
 #define MI355_FSS_ARGS dim3((unsigned)n_waves * 64), 0, s, a.q, a.k, a.v, a.mask, (u32)a.q_nb2, (u32)a.k_nb1, (u32)a.k_nb2, (u32)a.v_nb1, (u32)a.v_nb2, (u32)a.Nkv | (u32)R << 16, a
-#define MI355_FSS_LAUNCH(SPLIT, RES)                                                                                                                                        \
-    if (2 * a.Hq <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 1, SPLIT>), dim3((unsigned)a.Hkv, 2, (unsigned)R), MI355_FSS_ARGS);                                              \
-    else if (2 * a.Hkv * ((R + 1) / 2) <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 2, SPLIT>), dim3((unsigned)a.Hkv, 2, (unsigned)((R + 1) / 2)), MI355_FSS_ARGS);            \
-    else if (2 * a.Hkv <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 4, SPLIT>), dim3((unsigned)a.Hkv, 2), MI355_FSS_ARGS);
-    if (a.Nkv <= FSS_SPLIT_CELLS) {
-        // two groups of this form share a compute unit's LDS, which pays for groups of one wave: 195 / 65 heads, 64 cells 4.6 -> 4.2 us, 512 / 128 heads 4.8 -> 4.1; with more waves not
-        // (160 / 40 heads, 128 cells 4.0 -> 4.4, 256 cells 4.8 -> 6.0)
+#define MI355_FSS_LAUNCH(P32, RES)                                                                                                                                        \
+    if (2 * a.Hq <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 1, P32>), dim3((unsigned)a.Hkv, 2, (unsigned)R), MI355_FSS_ARGS);                                              \
+    else if (2 * a.Hkv * ((R + 1) / 2) <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 2, P32>), dim3((unsigned)a.Hkv, 2, (unsigned)((R + 1) / 2)), MI355_FSS_ARGS);            \
+    else if (2 * a.Hkv <= RES) MI355_LAUNCH((k_fattn_dec_short<2, 4, P32>), dim3((unsigned)a.Hkv, 2), MI355_FSS_ARGS);
+    if (a.Nkv <= FSS_P32_CELLS) {
+        // two groups of this form share a compute unit's LDS, which pays for groups of one wave: 195 / 65 heads, 64 cells 5.2 -> 4.5 us, 512 / 128 heads 5.4 -> 4.8; with more waves not
+        // (160 / 40 heads, 128 cells 4.6 -> 4.8, 256 cells 5.6 -> 6.5)
         MI355_FSS_LAUNCH(true, (a.Nkv <= FS_TILE ? 2 * CU : CU))
         else return 1;
     } else {

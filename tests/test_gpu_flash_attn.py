@@ -357,6 +357,55 @@ def test_decode_up_to_256_cells(dev, Hq, Hkv, Nkv, max_bias, softcap, use_mask):
     assert orc.nmse(got, f64) < 1e-11
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (160, 40), (512, 128), (260, 260)])
+@pytest.mark.parametrize("Nkv", [1, 64, 200, 256])
+@pytest.mark.parametrize("use_mask", [True, False])
+def test_decode_up_to_256_cells_non_finite_visible(dev, Hq, Hkv, Nkv, use_mask):
+    """one token over up to 256 cells whose visible keys and values hold infinities and NaN: they come out as f64 arithmetic has them, and the other heads and elements are not touched"""
+    rng = np.random.default_rng(Nkv + Hq)
+    q, k, v, mask = _inputs(rng, 128, 1, Nkv, Hq, Hkv, causal=False, rand_mask=True)
+    q = q.astype(np.float16).astype(np.float32)   # the kernels round q to the K type
+    c, c2 = int(rng.integers(Nkv)), Nkv // 2
+    v[0, c, 3], v[0, c, 100] = np.inf, -np.inf
+    v[1, c2, 70], v[1, c, 5] = -np.inf, np.nan
+    v[2, c, 9], v[2, c2, 9] = np.inf, -np.inf     # NaN where they are two cells
+    v[2, :, 64] = np.inf
+    k[3, c, 7] = np.nan
+    k[4, c, 127] = np.inf                         # scores of either sign: a weight of zero, or NaN
+    v[5 % Hkv, 0, 127] = np.inf
+    g, m = Hq // Hkv, mask[0].astype(np.float64) if use_mask else np.zeros(Nkv)
+    got = _run(dev, q, k, v, mask if use_mask else None, 128 ** -0.5, llama_layout=True)[0]
+    with np.errstate(all="ignore"):
+        kk, vv = (np.repeat(a.astype(np.float64), g, 0) for a in (k, v))
+        s = np.einsum("hd,hcd->hc", q[:, 0].astype(np.float64), kk) * 128 ** -0.5 + m
+        p = np.exp(s - s.max(1, keepdims=True))
+        want = np.einsum("hc,hcd->hd", p, vv) / p.sum(1, keepdims=True)
+    assert np.isinf(want).any() and np.isnan(want).any()
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(kind(got), kind(want)), kind.__name__
+    fin = np.isfinite(want)
+    assert orc.nmse(got[fin], want[fin]) < 1e-11    # as test_decode_up_to_256_cells
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (160, 40), (512, 128), (260, 260)])
+@pytest.mark.parametrize("Nkv", [64, 200, 256])
+def test_decode_up_to_256_cells_small_weights(dev, Hq, Hkv, Nkv):
+    """the output is the work of cells whose weights are 2^-20 .. 2^-30 of the largest: weights of f32 precision have their share of it right.  The scores are exact, so per element
+    remain the rounding of score * log2 e (|score| < 21: 21 * 2^-24, and half of that for the constant), of the exponential (2^-23) and of some ten sums and products: 3e-6"""
+    rng = np.random.default_rng(Nkv + Hq)
+    q, k, v = np.zeros((Hq, 1, 128), np.float32), np.zeros((Hkv, Nkv, 128), np.float16), np.zeros((Hkv, Nkv, 128), np.float16)
+    q[:, 0, 17] = 1.0
+    faint = np.zeros((Hkv, Nkv), bool)
+    faint[:, 5::9] = True
+    k[:, :, 17] = np.where(faint, -rng.uniform(13.9, 20.8, faint.shape), -rng.uniform(0, 0.5, faint.shape))
+    v[faint] = rng.uniform(1000, 60000, (int(faint.sum()), 128))
+    got = _run(dev, q, k, v, None, 1.0, llama_layout=True)[0]
+    s = np.repeat(k[:, :, 17].astype(np.float64), Hq // Hkv, 0)
+    p = np.exp(s - s.max(1, keepdims=True))
+    want = np.einsum("hc,hcd->hd", p, np.repeat(v.astype(np.float64), Hq // Hkv, 0)) / p.sum(1, keepdims=True)
+    assert np.abs(got / want - 1).max() < 3e-6
+
+
 @pytest.mark.parametrize("D,quantized", [(64, False), (80, False), (96, False), (112, False), (128, False), (256, False), (64, True), (128, True)])
 @pytest.mark.parametrize("Nq,Nkv,Hq,Hkv", [(300, 1100, 8, 2), (200, 520, 12, 12), (600, 640, 32, 8), (40, 600, 70, 70)])
 def test_prefill_non_finite_masked_cells(dev, D, quantized, Nq, Nkv, Hq, Hkv):
