@@ -17,8 +17,13 @@ extern __shared__ __attribute__((aligned(16))) uint8_t s_gr[];
 // and 48.5 / 48.0 for the layer)
 template <int TYPE> constexpr int gr_steps() { return TYPE == MI355_Q6_K || TYPE == MI355_Q5_K || TYPE == MI355_IQ4_XS ? 2 : 4; }
 
+// Waves per SIMD the registers are to leave room for.  IQ4_XS would take 67 of them, three past eight waves: 8192 rows are 1024 groups, four to every compute unit, of which three fit then
+// and the last ones run alone.  us, k_gemv_q / this with 67 / with 64 registers: 8192 x 4096 6.6 / 6.4 / 5.9, x 6144 8.9 / 8.9 / 8.5, x 14336 16.1 / 16.6 / 15.2.  (IQ4_NL, 68 registers
+// with four steps: 64 of them spill, 8192 x 14336 12.8 % slower; as it is 8192 x 6144 is the one size of all types found slower than k_gemv_q beyond the noise, by 1 %.)
+template <int TYPE> constexpr int gr_min_waves() { return TYPE == MI355_IQ4_XS ? 8 : 1; }
+
 template <int TYPE, int STEPS, int WAVES, int KMAX>
-__global__ void __launch_bounds__(64 * WAVES) k_gemv_row(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, float *__restrict__ dst,
+__global__ void __launch_bounds__(64 * WAVES, gr_min_waves<TYPE>()) k_gemv_row(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, float *__restrict__ dst,
                                                          const float *__restrict__ residual, int N, int K) {
     typedef wq<TYPE> T;
     const int lane = threadIdx.x & 63;
