@@ -376,7 +376,7 @@ __global__ void __launch_bounds__((ONE ? FS_WAVES_ONE : FS_WAVES) * 64, 1) k_fat
     fs_request_mask<MT>(a, c_begin, n, lane, mc);
     asm volatile("" ::: "memory");   // the loads are not to be moved behind the transfers
     __builtin_amdgcn_sched_barrier(0);
-    {   // without a branch around them (a wave without tiles moves the last one): at a join of paths the compiler knows the smaller number of requests in flight only
+    {   // without a branch around them (a wave without tiles moves the last one, and waits for it behind the loop): at a join of paths the compiler knows the smaller number of requests in flight only
         const int64_t first = n > 0 ? c_begin : (int64_t)(n_tiles - 1) * FS_TILE;
         issue_clamped(first, 0, 0);
         issue_clamped(first, 0, 1);
@@ -426,6 +426,8 @@ __global__ void __launch_bounds__((ONE ? FS_WAVES_ONE : FS_WAVES) * 64, 1) k_fat
         // every LDS read of this stage has returned (the last wait above): the V half may be overwritten
         if (!ONE && t + 2 < n) issue(t + 2, st, 1);
     }
+    // a wave without tiles has not waited for its transfers: they must have landed before fs_join takes the ring, and before the wave gives its LDS back
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     if constexpr (ONE) {
         fs_join<NWV>(S, (float *)ring_buf, FS_STAGE / 4, a.ws + ((int64_t)hk * R * a.n_splits + blockIdx.x) * (FS_D + 2), (int64_t)a.n_splits * (FS_D + 2), R, lane, wave);
@@ -798,6 +800,7 @@ __global__ void __launch_bounds__(((ONE ? fsq_waves_one<TK, TV>() : fsq_waves<TK
         if (!ONE && t + 2 < n) issue(t + 2, st, 1);
         fs_output<8>(vf_lds + fs_v_lane(lane), p_rd + 64, S);
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the transfers of a wave without tiles (see k_fattn_dec_stream)
 
     if constexpr (ONE) {
         fs_join<NWV>(S, (float *)vf_buf, FSQ_VF / 4, a.ws + ((int64_t)hk * R * a.n_splits + blockIdx.x) * (FS_D + 2), (int64_t)a.n_splits * (FS_D + 2), R, lane, wave);
