@@ -23,8 +23,8 @@ template <int TYPE> constexpr int gr_steps() { return TYPE == MI355_Q6_K || TYPE
 template <int TYPE> constexpr int gr_min_waves() { return TYPE == MI355_IQ4_XS ? 8 : 1; }
 
 template <int TYPE, int STEPS, int WAVES, int KMAX>
-__global__ void __launch_bounds__(64 * WAVES, gr_min_waves<TYPE>()) k_gemv_row(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, float *__restrict__ dst,
-                                                         const float *__restrict__ residual, int N, int K) {
+__global__ void __launch_bounds__(64 * WAVES, gr_min_waves<TYPE>()) k_gemv_row(const uint8_t *__restrict__ W, const int8_t *__restrict__ aq, const act_ds *__restrict__ ads, float *dst,
+                                                         const float *residual, int N, int K) {   // residual may be dst: a row's is read by the wave that stores it
     typedef wq<TYPE> T;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
