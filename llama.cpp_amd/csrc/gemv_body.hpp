@@ -208,6 +208,7 @@ __device__ __forceinline__ void gemv_body_qc(const gemv_item &m, int group, cons
                                              const gemv_rope &R, uint8_t *s_act) {
     typedef wq<TYPE> T;
     constexpr int NW = 8, RPW = QUANT ? 4 : 2, NP = RPW / 2;
+    static_assert(!NORM || NCOLS == 1, "the norm is one row's");
     static_assert(NCOLS <= 4, "wave c quantizes activation row c");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -225,6 +226,37 @@ __device__ __forceinline__ void gemv_body_qc(const gemv_item &m, int group, cons
         rows[r] = m.W + row * L.row_bytes;
     }
 
+    // NORM.  Types whose row is two steps of 64 chunks: the row first, the weights behind it - a wave's loads return in the order of their issue - and the rotations worked out while both
+    // are on their way.  The second step of four rows per wave is requested when the registers of the normalised row are free; of the K-quants, whose chunks are the largest, it waits for
+    // the first one's.  Types of one step: rotations, weights, row.  8B shapes in a chain of launches, Q8_0 caches, us, every type's own matrices: the row behind the weights and the second
+    // step behind the sums of the first / this (the same before loads of the row were without branches): Q8_0 12.3 / 11.2 (11.7), Q4_0 9.2 / 8.5 (9.5), Q6_K 12.1 / 11.4 (12.3), Q5_K 13.2 / 11.9
+    // (13.7), IQ4_XS 10.9 / 10.4 (11.4), Q4_K 10.1 / 10.1 (10.7).  The row first for types of one step: Q5_K 13.5, Q4_K 10.0; both steps of four rows ahead: spills, Q6_K for V 14.1.
+    typedef late_chunk<TYPE> G;
+    constexpr int STEPS = 64 / T::CHUNK;   // steps of 64 chunks in a row of 4096
+    constexpr int FIRST = QUANT ? 1 : STEPS;
+    typename G::raw wn[STEPS][RPW];
+    auto request = [&](int from, int to) {
+#pragma unroll
+        for (int p = 0; p < STEPS; p++)
+#pragma unroll
+            for (int r = 0; r < RPW; r++) {
+                const int c = p * 64 + lane;
+                if (p >= from && p < to) wn[p][r] = G::load(rows[r], L, c < nchunks ? c : nchunks - 1);
+            }
+    };
+    norm_row<NW> row;
+    __shared__ float s_norm[4];
+    int pos = 0, cell = 0;
+    if constexpr (NORM) {
+        if (R.pos) pos = R.pos[0];       // null where no matrix of the launch is rotated
+        if (R.cells) cell = R.cells[0];  // ... or goes to a cache
+        if constexpr (STEPS > 1) {
+            row.request(R.nx, R.nw, K);
+            __builtin_amdgcn_sched_barrier(0);
+            request(0, FIRST);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
     float rope_c[NP], rope_s[NP];
     bool rotate[NP];
 #pragma unroll
@@ -233,29 +265,29 @@ __device__ __forceinline__ void gemv_body_qc(const gemv_item &m, int group, cons
         rope_s[p] = 0.0f;
         rotate[p] = false;
     }
-    int cell = 0;
     if (lane < NCOLS) {
         const bool rope_epi = m.epi == EPI_ROPE || m.epi == EPI_ROPE_CACHE || m.epi == EPI_ROPE_QCACHE;
 #pragma unroll
         for (int p = 0; p < NP; p++) {
             const int d = (int)((row0 + 2 * p) % R.D);
             rotate[p] = rope_epi && d < R.n_dims;
-            if (rotate[p]) rope_coeffs(R, R.pos[lane], d >> 1, rope_c[p], rope_s[p]);
+            if (rotate[p]) rope_coeffs(R, NORM ? pos : R.pos[lane], d >> 1, rope_c[p], rope_s[p]);
         }
-        if (m.epi == EPI_ROPE_CACHE || m.epi == EPI_CACHE) cell = R.cells[lane];
+        if (!NORM && (m.epi == EPI_ROPE_CACHE || m.epi == EPI_CACHE)) cell = R.cells[lane];
     }
 #pragma unroll
     for (int p = 0; p < NP; p++) asm volatile("" : "+v"(rope_c[p]), "+v"(rope_s[p]));
     asm volatile("" : "+v"(cell));
 
-    typename T::chunk w_first[RPW];
-    if constexpr (NORM) {   // as in gemv_body: the first step's weights are on their way while the group normalises and quantizes the row
-        const int c = lane < nchunks ? lane : nchunks - 1;
-#pragma unroll
-        for (int r = 0; r < RPW; r++) w_first[r] = T::load_w(rows[r], L, c);
-        __shared__ float s_norm[4];
-        if (threadIdx.x < 256) rms_norm_quant_row<4, false, false>(R.nx, R.nw, nullptr, s_act, 0, K, 1, R.neps, s_norm);
-        else __syncthreads();   // the one barrier inside the norm
+    if constexpr (NORM) {
+        if constexpr (STEPS == 1) {
+            request(0, FIRST);
+            __builtin_amdgcn_sched_barrier(0);
+            row.request(R.nx, R.nw, K);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        row.finish(s_act, K, R.neps, s_norm);
+        if constexpr (!G::ORDERED) request(FIRST, STEPS);
         __syncthreads();
         if (!wave_live) return;
         aq = (const int8_t *)s_act;
@@ -267,22 +299,35 @@ __device__ __forceinline__ void gemv_body_qc(const gemv_item &m, int group, cons
     for (int r = 0; r < RPW; r++)
 #pragma unroll
         for (int c = 0; c < NCOLS; c++) acc[r][c] = 0.0f;
-    for (int c0 = 0; c0 < nchunks; c0 += 64) {
-        const int c = c0 + lane;
-        if (c < nchunks) {
-            typename T::chunk w[RPW];
+    if constexpr (NORM) {
+#pragma unroll
+        for (int p = 0; p < STEPS; p++) {
+            const int c = p * 64 + lane;
+            if (p * 64 >= nchunks) break;   // uniform
+            if (G::ORDERED && p >= FIRST) request(p, p + 1);
+            const typename T::act A = T::load_a(aq, ads, c < nchunks ? c : nchunks - 1);
 #pragma unroll
             for (int r = 0; r < RPW; r++) {
-                if (NORM && c0 == 0) w[r] = w_first[r];
-                else w[r] = T::load_w(rows[r], L, c);
+                const typename T::chunk now = G::decode(wn[p][r], c);
+                const float sum = T::accumulate(acc[r][0], now, A, T::dots(now, A));
+                acc[r][0] = c < nchunks ? sum : acc[r][0];
             }
+        }
+    } else {
+        for (int c0 = 0; c0 < nchunks; c0 += 64) {
+            const int c = c0 + lane;
+            if (c < nchunks) {
+                typename T::chunk w[RPW];
 #pragma unroll
-            for (int col = 0; col < NCOLS; col++) {
-                const typename T::act A = T::load_a(aq + (int64_t)col * K, ads + col * nblk, c);
+                for (int r = 0; r < RPW; r++) w[r] = T::load_w(rows[r], L, c);
 #pragma unroll
-                for (int r = 0; r < RPW; r++) {
-                    const chunk_dots d = T::dots(w[r], A);
-                    acc[r][col] = T::accumulate(acc[r][col], w[r], A, d);
+                for (int col = 0; col < NCOLS; col++) {
+                    const typename T::act A = T::load_a(aq + (int64_t)col * K, ads + col * nblk, c);
+#pragma unroll
+                    for (int r = 0; r < RPW; r++) {
+                        const chunk_dots d = T::dots(w[r], A);
+                        acc[r][col] = T::accumulate(acc[r][col], w[r], A, d);
+                    }
                 }
             }
         }

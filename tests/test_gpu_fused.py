@@ -398,6 +398,40 @@ def test_qkv_rope_quantized_store_equals_separate_copies(dev, B, norm, ck, cv, d
     assert kc1.float().abs().sum().item() > 0 and vc1.float().abs().sum().item() > 0
 
 
+@pytest.mark.parametrize("name,t", list(orc.WEIGHT_TYPES.items()))
+@pytest.mark.parametrize("K", [1024, 2048, 3072, 4096])
+def test_qkv_norm_quantized_store_steps_of_a_row(dev, name, t, K):
+    """one token over quantized caches, rows of half a step of 64 chunks to two whole ones: norm, projections and stores in one launch against the norm launch and the launch behind it"""
+    import torch
+    import mi355
+    from mi355 import llama_graph as lg
+    if name in ("q6_K", "iq4_xs") and K % 2048:
+        pytest.skip("rows of whole 16 bytes")
+    lib = mi355.load()
+    H, HK, D, cells_n = 5, 2, 32, 8
+    N = HK * D
+    gen = torch.Generator(device=dev).manual_seed(K + t)
+    Ws = [mi355.upload_weights(t, lg.random_quantized(t, n, K, torch.device(dev), gen)) for n in (H * D, N, N)]
+    x, nw = torch.randn(1, K, device=dev, generator=gen), torch.randn(K, device=dev, generator=gen)
+    pos, cell = _t(dev, np.array([77], dtype=np.int32)), _t(dev, np.array([5], dtype=np.int32))
+    desc = mi355.RopeDesc(pos.data_ptr(), cell.data_ptr(), None, D, D, 0, 4096, 500000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+    act = torch.empty(int(lib.mi355_act_bytes(K, 1)) + 256, dtype=torch.uint8, device=dev)
+    mi355.check(lib.mi355_rms_norm_mul_quant(None, x.data_ptr(), K, nw.data_ptr(), None, 0, act.data_ptr(), K, 1, 1e-5))
+    got = []
+    for norm in (False, True):
+        q, kv = torch.zeros(H * D, device=dev), [torch.zeros(cells_n * N // 32 * mi355.BLOCK[c][1], dtype=torch.uint8, device=dev) for c in (orc.Q8_0, orc.Q4_0)]
+        arr = (mi355.GemvRopeMat * 3)(mi355.GemvRopeMat(t, Ws[0].data_ptr(), H * D, mi355.EPI_ROPE, q.data_ptr(), H * D, 0, 0),
+                                      mi355.GemvRopeMat(t, Ws[1].data_ptr(), N, mi355.EPI_ROPE_QCACHE, kv[0].data_ptr(), orc.Q8_0, 0, cells_n * N // 32),
+                                      mi355.GemvRopeMat(t, Ws[2].data_ptr(), N, mi355.EPI_QCACHE, kv[1].data_ptr(), orc.Q4_0, 0, cells_n * N // 32))
+        if norm:
+            mi355.check(lib.mi355_rms_norm_mul_mat_vec_q_rope(None, x.data_ptr(), nw.data_ptr(), 1e-5, 3, arr, K, C.byref(desc)))
+        else:
+            mi355.check(lib.mi355_mul_mat_vec_q_rope(None, 3, arr, act.data_ptr(), K, 1, C.byref(desc)))
+        got.append([q] + kv)
+    for a, b in zip(*got):
+        assert torch.equal(a, b) and bool(a.any())
+
+
 @pytest.mark.parametrize("B", [1, 2, 3, 4])
 @pytest.mark.parametrize("tg,tu,K,N", [(orc.Q4_K, orc.Q6_K, 2048, 1536),       # two types: groups of 8 rows, the last group of a 32-row block finishes it
                                        (orc.Q4_K, orc.Q4_K, 2048, 1536),       # one type: a group owns a 32-row block in both matrices
