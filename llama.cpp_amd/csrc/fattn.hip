@@ -46,7 +46,7 @@ __device__ __forceinline__ float dot8_f16(const u32x4 &a, const u32x4 &b) {
 
 
 
-// Where this lane's eight elements d0 .. d0 + 7 of the (cell 0, kv head hk) row of a quantized operand lie: their levels (Q4_0: the
+// Where this lane's eight elements d0 .. d0 + 7 of the (first_cell, kv head hk) row of a quantized operand lie: their levels (Q4_0: the
 // eight bytes whose low or high nibbles - shift 0 or 4 - they are) and the block's f16 scale; a cell further on they are lv_step /
 // sc_step bytes further on.
 struct kv_lane {
@@ -54,7 +54,7 @@ struct kv_lane {
     int shift;
     int64_t lv_step, sc_step;
 };
-__device__ __forceinline__ kv_lane kv_lane_of(const kv_src &s, int type, int64_t hk, int d0) {
+__device__ __forceinline__ kv_lane kv_lane_of(const kv_src &s, int type, int64_t hk, int d0, int64_t first_cell) {
     const int BB = type == MI355_Q8_0 ? Q8_0_BYTES : Q4_0_BYTES, LB = type == MI355_Q8_0 ? 32 : 16;
     const int64_t g = s.first_block + hk * s.head_blocks + (d0 >> 5);
     const int j = d0 & 31;
@@ -67,14 +67,15 @@ __device__ __forceinline__ kv_lane kv_lane_of(const kv_src &s, int type, int64_t
         lv = s.base + g * LB;
         o.sc = s.base + s.row_blocks * LB + g * 2;
     }
-    o.lv = lv + (type == MI355_Q8_0 ? j : (j & 15));
+    o.lv = lv + (type == MI355_Q8_0 ? j : (j & 15)) + first_cell * s.cell_lv;
+    o.sc += first_cell * s.cell_sc;
     o.shift = (type == MI355_Q4_0 && j >= 16) ? 4 : 0;
     o.lv_step = s.cell_lv;
     o.sc_step = s.cell_sc;
     return o;
 }
 // the raw bytes of one cell's eight elements: levels in words 0 and 1, the scale's bits in word 2 (plain blocks are 2-byte aligned)
-__device__ __forceinline__ u32x4 kv_load8(const kv_lane &p, int64_t cell) {
+__device__ __forceinline__ u32x4 kv_load8(const kv_lane &p, u32 cell) {
     u32x2 w;
     __builtin_memcpy(&w, p.lv + cell * p.lv_step, 8);
     return u32x4{w[0], w[1], (u32)*(const unsigned short *)(p.sc + cell * p.sc_step), 0u};
@@ -124,12 +125,24 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
     __shared__ float s_m[NW][R], s_l[NW][R];
     __shared__ float s_o[NW][R][D];
 
-    const int split = blockIdx.x;
     // Neighbouring groups are different kv heads: workgroups go to the XCDs in turn, so the groups of one kv head (a multiple of 8 apart where there are
     // 8 kv heads, or 16) share an L2 and its rows are fetched once (64 / 8 heads of 256, 448 cells: 15.5 -> 11.6 us; 32 / 8 heads of 80, 1024: 17.0 -> 12.1).
     // far_apart: that many ranges of cells that they would not run at the same time; then the kv head's groups are neighbours (launch_vec)
-    const unsigned per = a.far_apart ? (unsigned)a.groups : (unsigned)a.Hkv, quot = blockIdx.y / per, rem = blockIdx.y - quot * per;
-    const int64_t hk = a.far_apart ? quot : rem, hg = a.far_apart ? rem : quot, iq = blockIdx.z;
+    // sharers: see launch_vec.  Eighths of the grid are XCDs; a turn of one is a (range, kv head) pair's groups one after the other
+    unsigned split = blockIdx.x, hk_of, hg_of, iq_of = blockIdx.z;
+    if (a.sharers) {   // uniform
+        const unsigned turn = blockIdx.x >> 3, of_xcd = turn / (unsigned)a.sharers, member = turn - of_xcd * (unsigned)a.sharers, pair = (blockIdx.x & 7) + 8 * of_xcd;
+        if (pair >= (unsigned)(a.n_splits * a.Hkv)) return;   // the whole group
+        hk_of = pair / (unsigned)a.n_splits;
+        split = pair - hk_of * (unsigned)a.n_splits;
+        iq_of = member / (unsigned)a.groups;
+        hg_of = member - iq_of * (unsigned)a.groups;
+    } else {
+        const unsigned per = a.far_apart ? (unsigned)a.groups : (unsigned)a.Hkv, quot = blockIdx.y / per, rem = blockIdx.y - quot * per;
+        hk_of = a.far_apart ? quot : rem;
+        hg_of = a.far_apart ? rem : quot;
+    }
+    const int64_t hk = hk_of, hg = hg_of, iq = iq_of;
     const int64_t head0 = (hk * a.groups + hg) * R;   // first of this group's R query heads
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sub = lane % LPR, slot = wave * CPW + lane / LPR;
@@ -139,17 +152,19 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
     const int64_t c_begin = (int64_t)split * a.cells_per_split;
     const int64_t c_end = c_begin + a.cells_per_split < a.Nkv ? c_begin + a.cells_per_split : a.Nkv;
     constexpr int U = 4;   // steps of SLOTS cells at a time, see the loop
-    // (us, one row over 1024 cells: 32 / 8 heads of 80 16.2 -> 12.5, of 256 12.9 -> 12.4 against masks requested when their round begins, behind q.)
+    // (us, one row over 1024 cells: 32 / 8 heads of 80 12.1 -> 11.4, of 256 12.6 -> 12.0 against masks requested when their round begins, behind q.)
     // The mask entries of a round are requested together, from clamped addresses and without a branch per entry (a branch per entry makes each load wait for the one
-    // before it: U round trips instead of one); the first round's ahead of q, the others behind the rows of the round before.
+    // before it: U round trips instead of one); the first round's with q, the others ahead of the rows of the round before - behind them, the first use of a row would wait for them too.
+    // 32-bit cells and one base address per operand: seven groups of four waves on a compute unit instead of five (90 -> 70 registers; 16 / 16 heads of 80, 12 rows over 2048 cells 19.5 -> 17.3 us).
     unsigned mraw[U];   // (32-bit each: halves packed in pairs would be merged load by load, with a wait for each)
-    const unsigned short *mrow = a.mask ? (const unsigned short *)(a.mask + iq * a.mask_nb1) : (const unsigned short *)a.q;   // without a mask some word of q, not used
-    const int64_t mask_last = a.mask ? c_end - 1 : 0;   // (a choice of the index per entry becomes two paths, with a wait at their join)
-    auto request_mask = [&](int64_t cb) {
+    const int n_cells = (int)(c_end - c_begin);   // cells are counted from the range's first (2^31 cells of a range are more than the memory holds)
+    const unsigned short *mrow = a.mask ? (const unsigned short *)(a.mask + iq * a.mask_nb1) + c_begin : (const unsigned short *)a.q;   // without a mask some word of q, not used
+    const int mask_last = a.mask ? n_cells - 1 : 0;   // (a choice of the index per entry becomes two paths, with a wait at their join)
+    auto request_mask = [&](int cb) {
 #pragma unroll
         for (int j = 0; j < U; j++) {
-            const int64_t c = cb + j * SLOTS + slot;
-            mraw[j] = mrow[c < mask_last ? c : mask_last];
+            const int c = cb + j * SLOTS + slot;
+            mraw[j] = mrow[(unsigned)(c < mask_last ? c : mask_last)];
         }
     };
     // q slices, rounded to f16 (ggml-cpu.c:11037-11040 converts q to the K type before the dot)
@@ -162,7 +177,7 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
         qx[r][0] = *(const f32x4 *)qp;
         qx[r][1] = *(const f32x4 *)(qp + 4);
     }
-    request_mask(c_begin);
+    request_mask(0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -195,33 +210,36 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
     // quantized operands (wave-uniform choice): this lane's place in the rows of kv head hk
     const bool k_f16 = !QUANT || type_k == MI355_F16, v_f16 = !QUANT || type_v == MI355_F16;
     kv_lane kl = {nullptr, nullptr, 0, 0, 0}, vl = {nullptr, nullptr, 0, 0, 0};
-    if (!k_f16 && active) kl = kv_lane_of(a.kq, type_k, hk, d0);
-    if (!v_f16 && active) vl = kv_lane_of(a.vq, type_v, hk, d0);
+    if (!k_f16 && active) kl = kv_lane_of(a.kq, type_k, hk, d0, c_begin);
+    if (!v_f16 && active) vl = kv_lane_of(a.vq, type_v, hk, d0, c_begin);
 
     // U steps of SLOTS cells at a time: all mask entries, then all K/V rows of the U steps are requested before the first
     // is used, so a short context costs one round trip to memory instead of one per step.  Cells are still folded into a
     // slot's state in ascending order.
-    for (int64_t cb = c_begin; cb < c_end; cb += U * SLOTS) {
+    const uint8_t *k_rows = a.k + c_begin * a.k_nb1 + hk * a.k_nb2, *v_rows = a.v + c_begin * a.v_nb1 + hk * a.v_nb2;   // (f16 operands)
+    for (int cb = 0; cb < n_cells; cb += U * SLOTS) {
         float mv[U];
         bool valid[U];
 #pragma unroll
         for (int j = 0; j < U; j++) {
-            const int64_t c = cb + j * SLOTS + slot;
+            const int c = cb + j * SLOTS + slot;
             asm volatile("" : "+v"(mraw[j]));   // stays a register of its own from round to round
             mv[j] = a.mask ? half_bits_to_float((unsigned short)mraw[j]) : 0.0f;
-            valid[j] = c < c_end && mv[j] != -INFINITY;
-            if (c >= c_end) mv[j] = 0.0f;
+            valid[j] = c < n_cells && mv[j] != -INFINITY;
+            if (c >= n_cells) mv[j] = 0.0f;
         }
+        request_mask(cb + U * SLOTS);   // (behind the end: the last entry again)
+        __builtin_amdgcn_sched_barrier(0);
         u32x4 kk[U], vv[U];
         if constexpr (!QUANT) {
 #pragma unroll
             for (int j = 0; j < U; j++) {
-                const int64_t c = cb + j * SLOTS + slot;
+                const int c = cb + j * SLOTS + slot;
                 kk[j] = u32x4{0, 0, 0, 0};
                 vv[j] = u32x4{0, 0, 0, 0};
                 if (valid[j] && active) {   // masked cells cost no K/V traffic
-                    kk[j] = load16(a.k + c * a.k_nb1 + hk * a.k_nb2 + d0 * 2);
-                    vv[j] = load16(a.v + c * a.v_nb1 + hk * a.v_nb2 + d0 * 2);
+                    kk[j] = load16(k_rows + (unsigned)c * a.k_nb1 + d0 * 2);
+                    vv[j] = load16(v_rows + (unsigned)c * a.v_nb1 + d0 * 2);
                 }
             }
         } else if (!active) {
@@ -237,9 +255,9 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
             // from memory cold - and is zeroed afterwards.
 #pragma unroll
             for (int j = 0; j < U; j++) {
-                const int64_t c = valid[j] ? cb + j * SLOTS + slot : c_begin;
-                kk[j] = k_f16 ? load16(a.k + c * a.k_nb1 + hk * a.k_nb2 + d0 * 2) : kv_load8(kl, c);
-                vv[j] = v_f16 ? load16(a.v + c * a.v_nb1 + hk * a.v_nb2 + d0 * 2) : kv_load8(vl, c);
+                const int c = valid[j] ? cb + j * SLOTS + slot : 0;
+                kk[j] = k_f16 ? load16(k_rows + (unsigned)c * a.k_nb1 + d0 * 2) : kv_load8(kl, (u32)c);
+                vv[j] = v_f16 ? load16(v_rows + (unsigned)c * a.v_nb1 + d0 * 2) : kv_load8(vl, (u32)c);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -250,7 +268,6 @@ __global__ void __launch_bounds__(NW * 64) k_fattn_vec(fattn_args a) {
                 }
             }
         }
-        if (cb + U * SLOTS < c_end) request_mask(cb + U * SLOTS);   // uniform
         float kd[U];   // quantized K: the levels as exact f16 values; their dot with q takes the block's scale afterwards
 #pragma unroll
         for (int j = 0; j < U; j++) {
@@ -475,7 +492,15 @@ static int launch_vec(hipStream_t s, fattn_args &a) {
     // One row, 49152 cells, device us, kv heads / a kv head's groups as neighbours: 64 / 8 heads of 256 187 / 164, of 112 94.5 / 90.2, 32 / 4 heads of 80 45.7 / 44.2;
     // fewer ranges, 64 / 8 heads of 256 over 8192 cells 33.7 / 35.9, 32 / 4 over 16384 35.1 / 36.9
     a.far_apart = a.n_splits > 1 && a.n_splits * a.Hkv >= 512;
-    const dim3 grid((unsigned)a.n_splits, (unsigned)(a.Hkv * a.groups), (unsigned)a.Nq);
+    // Several rows over ranges of cells: every row reads what the others read.  Where their groups do not all run at once, or K and V come from memory at that, those of one (range, kv head) are
+    // numbered next to each other on one XCD, so that its L2 has what the first of them has fetched; in the order of the grid a kv head's rows are up to 2048 groups apart.  us, grid / this:
+    // 32 / 32 heads of 112, 4 rows over 16384 cells 161 / 65, of 256, 8 rows over 4096 128 / 65, 2 rows over 4096 39.4 / 30.9; 32 / 8 heads of 80, 6 rows over 16384 76.7 / 72.1.  Fewer groups
+    // or cells lose some per cent (the grid deals the kv heads out over the XCDs evenly): 32 / 4 heads of 256, 3 rows over 4096 28.4 / 33.8, 64 / 8 heads of 80, 15 rows over 1024 35.3 / 36.2.
+    // Quantized operands are bound by arithmetic: 32 / 8 heads of 96, Q4_0, 8 rows over 16384 cells 162 / 172 (Q8_0 of 128, 32 / 32 heads 181 / 161 is the one that gains).
+    const int64_t all = a.n_splits * a.Hkv * a.groups * a.Nq;
+    const bool together = !quant && a.n_splits > 1 && a.Nq > 1 && a.Nkv > 1024 && (all > 1024 || (all == 1024 && a.Nkv >= 4096));
+    a.sharers = together ? (int)(a.Nq * a.groups) : 0;
+    const dim3 grid = a.sharers ? dim3((unsigned)((a.n_splits * a.Hkv + 7) / 8 * 8 * a.sharers)) : dim3((unsigned)a.n_splits, (unsigned)(a.Hkv * a.groups), (unsigned)a.Nq);
     if constexpr (D % 32 == 0) {
         const bool same = a.type_k == a.type_v && D == 128;   // the caches llama.cpp builds with -ctk / -ctv of one type
         if (quant && same && a.type_k == MI355_Q8_0) MI355_LAUNCH((k_fattn_vec<D, R, NW, D == 128 ? 2 : 1>), grid, dim3(NW * 64), 0, s, a);

@@ -36,6 +36,7 @@ struct fattn_args {
     int n_splits;
     int groups;      // head groups of R per kv head: Hq / Hkv == R * groups
     bool far_apart = false;   // k_fattn_vec: blockIdx.y counts the groups of a kv head first, then the kv heads
+    int sharers = 0;          // k_fattn_vec: groups that read the same cells of the same kv head, numbered next to each other on one XCD; 0: the grid is (ranges, head groups, rows)
     int64_t cells_per_split;
 };
 

@@ -238,6 +238,21 @@ def _textbook(q, k, v, mask, scale):
     return np.matmul(p / p.sum(axis=-1, keepdims=True), vv).transpose(1, 0, 2)
 
 
+@pytest.mark.parametrize("D,Nq,Nkv,Hq,Hkv", [(80, 5, 2100, 35, 35),      # 9 ranges x 35 kv heads: 315 pairs, five past the last whole turn of eight XCDs
+                                             (112, 15, 5000, 40, 5),     # two groups of four heads per kv head: 30 groups share a pair's cells
+                                             (256, 2, 4096, 32, 32),     # 1024 groups: from 4096 cells on
+                                             (96, 2, 4095, 32, 32),      # ... and one cell fewer: the grid's order
+                                             (64, 7, 1025, 37, 37), (80, 7, 1024, 37, 37)])   # 1024 cells: one range
+def test_few_rows_whose_groups_share_cells(dev, D, Nq, Nkv, Hq, Hkv):
+    """two to fifteen rows over ranges of cells, the groups of one (range, kv head) numbered next to each other: every row, head and range once.  f32 probabilities: 1e-11 as
+    test_decode_up_to_256_cells (head size 64 may take the matrix-core form, whose probabilities are f16: 1e-6)"""
+    rng = np.random.default_rng(D + Nkv)
+    q, k, v, mask = _inputs(rng, D, Nq, Nkv, Hq, Hkv, rand_mask=True)
+    q = q.astype(np.float16).astype(np.float32)
+    got = _run(dev, q, k, v, mask, 1.0 / np.sqrt(D), llama_layout=True)
+    assert orc.nmse(got, _textbook(q, k, v, mask, 1.0 / np.sqrt(D))) < (1e-6 if D == 64 else 1e-11)
+
+
 @pytest.mark.parametrize("D", [80, 96, 112, 256])
 @pytest.mark.parametrize("Nq,Nkv,Hq,Hkv", [(16, 40, 4, 4), (33, 96, 6, 2), (65, 1090, 8, 2), (130, 1056, 3, 1), (545, 600, 64, 16), (545, 600, 66, 66)])
 def test_prefill_head_sizes(dev, D, Nq, Nkv, Hq, Hkv):

@@ -211,6 +211,18 @@ def test_flash_attn_quantized_kv(dev, kname, tk, vname, tv, D, Nq, Nkv, Hq, Hkv,
         assert orc.nmse(got, orc.flash_attn_kv("ref", q, k, tk, v, tv, mask.view(np.uint16), scale, n_threads=16)) <= 5e-4
 
 
+@pytest.mark.parametrize("kname,tk", KV_TYPES)
+@pytest.mark.parametrize("vname,tv", KV_TYPES)
+@pytest.mark.parametrize("D,Nq,Nkv,Hq,Hkv", [(128, 5, 2100, 35, 35), (96, 15, 2500, 40, 5)])
+def test_flash_attn_quantized_kv_few_rows_over_ranges(dev, kname, tk, vname, tv, D, Nq, Nkv, Hq, Hkv):
+    """a few rows over several ranges of cells, each read from its own first cell on; the bound of test_flash_attn_quantized_kv"""
+    rng = np.random.default_rng(D + Nkv + tk * 3 + tv)
+    q, kf, vf, mask = _case(rng, D, Nq, Nkv, Hq, Hkv)
+    k, v = orc.kv_rows(tk, kf), orc.kv_rows(tv, vf)
+    got = _run(dev, q, k, tk, v, tv, mask, 1.0 / np.sqrt(D), "1d" if tk != orc.F16 or tv != orc.F16 else False)
+    assert orc.nmse(got, _textbook(q, k, tk, v, tv, mask, 1.0 / np.sqrt(D))) < 1e-5
+
+
 @pytest.mark.parametrize("kname,tk", [kt for kt in KV_TYPES if kt[1] != orc.F16])
 @pytest.mark.parametrize("vname,tv", [kt for kt in KV_TYPES if kt[1] != orc.F16])
 @pytest.mark.parametrize("Nkv,Hq,Hkv", [(1024, 32, 8), (4096, 32, 8), (5000, 32, 8), (16421, 32, 8), (2048, 8, 8), (3000, 16, 8), (40000, 8, 2)])
