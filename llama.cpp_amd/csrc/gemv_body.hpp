@@ -30,7 +30,7 @@ struct gemv_rope {
     const float *ff;         // frequency factors [n_dims/2] or null
     int D, n_dims;
     float theta_scale, freq_scale, ext_factor, attn_factor, corr0, corr1;
-    const float2 *table;     // {cos, sin} of every (activation row, pair) from k_rope_table (same bits), or null: each wave works out its own
+    const float2 *table;     // k_gemv_qkv_norm<true>: {cos, sin} of every pair of the one activation row from k_rope_table; the other launches work out their own (same bits)
     const float *nx, *nw;    // the launches with the norm: the f32 row to normalise and the norm weights (the group quantizes it into its LDS copy itself)
     float neps;
 };
@@ -98,19 +98,13 @@ __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const i
     int pos = 0, cell = 0;
     if constexpr (QKV) {
         const int col = lane < NCOLS ? lane : NCOLS - 1;
-        if (rp->table) {
-            const float2 cs = rp->table[col * (rp->D >> 1) + ((int)(row0 % rp->D) >> 1)];
-            rope_c = cs.x;
-            rope_s = cs.y;
-        } else if (rp->pos) {   // null where no matrix of the launch is rotated
-            pos = rp->pos[col];
-        }
+        if (rp->pos) pos = rp->pos[col];       // null where no matrix of the launch is rotated
         if (rp->cells) cell = rp->cells[col];  // ... or goes to a cache
     }
     // QKV: lane c finishes activation row c.  Its rotation depends on nothing the product computes (the empty asm keeps it from being moved behind the loop, next
     // to its use).
     auto rotation = [&]() {
-        if (lane < NCOLS && !rp->table) {
+        if (lane < NCOLS) {
             const gemv_rope &R = *rp;
             const int d = (int)(row0 % R.D);
             if ((m.epi == EPI_ROPE || m.epi == EPI_ROPE_CACHE) && d < R.n_dims) rope_coeffs(R, pos, d >> 1, rope_c, rope_s);

@@ -242,6 +242,7 @@ static int vec_q_rope_impl(void *stream, int n_mats, const mi355_gemv_rope_mat *
             if (i < n_mats) groups += any_qc ? (qc ? m.N / 32 : (m.N + 15) / 16) : (m.N + group_rows - 1) / group_rows;   // 8 waves x 4 or 2 rows; without quantized stores 4 or 8 waves x 2 rows
         }
     }
+    MI355_REQUIRE(table == nullptr || (nx != nullptr && !any_qc), "mul_mat_vec_q_rope: only the launch with the norm and f16 destinations reads a table");
     MI355_REQUIRE(!needs_pos || rope->pos != nullptr || table != nullptr, "mul_mat_vec_q_rope: rope positions missing");
     MI355_REQUIRE(!needs_cells || rope->cells != nullptr, "mul_mat_vec_q_rope: cache cells missing");
     MI355_REQUIRE(groups < 0x7fffffff, "mul_mat_vec_q_rope: too many rows for one launch");
