@@ -93,6 +93,10 @@ __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const i
 
     // The order of the requests: a wave's loads return as they were issued, so the activation comes first (with what the QKV epilogue needs to know), the first step's
     // weights behind it, and what can be computed without the weights is done while they are on their way.
+    // Without the copy the Q/K/V launch requests the first step's weights ahead of the rotations too: of three and four tokens, of Q8_0, and of two tokens of the types whose chunks are the
+    // widest.  us, 32 / 8 heads, 4096 elements, weights behind the rotations / ahead: four tokens Q6_K 11.8 / 10.3, Q4_K with Q6_K for V 10.1 / 9.1, Q8_0 10.2 / 9.5, three Q4_K 8.8 / 7.4,
+    // one Q8_0 7.9 / 7.6, two Q4_K 7.4 / 6.7; but one of Q4_0 6.0 / 6.1, of Q4_K with Q6_K for V 6.6 / 7.0, two of Q6_K 8.1 / 8.7.
+    constexpr bool AHEAD = QKV && !LDSA && (NCOLS >= 3 || TYPE == MI355_Q8_0 || (T::CHUNK == 64 && NCOLS == 2));
     typename T::chunk w_first[RPW];
     float rope_c = 1.0f, rope_s = 0.0f;
     int pos = 0, cell = 0;
@@ -125,6 +129,11 @@ __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const i
         aq = (const int8_t *)s_act;
         ads = (const act_ds *)(s_act + NCOLS * K);
     } else if constexpr (QKV) {
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int r = 0; r < RPW; r++) w_first[r] = T::load_w(rows[r], L, c_first);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         rotation();
     }
 
@@ -134,7 +143,7 @@ __device__ __forceinline__ void gemv_body(const gemv_item &m, int group, const i
             typename T::chunk w[RPW];
 #pragma unroll
             for (int r = 0; r < RPW; r++) {
-                if (LDSA && c0 == 0) w[r] = w_first[r];
+                if ((LDSA || AHEAD) && c0 == 0) w[r] = w_first[r];
                 else w[r] = T::load_w(rows[r], L, c);
             }
 #pragma unroll
