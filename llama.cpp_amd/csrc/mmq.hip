@@ -780,6 +780,7 @@ static void launch_mmq_split_sum(hipStream_t s, const float *part, const mmq_mat
         const mmq_mat &m = mats.m[i];
         wide = wide && m.N % 4 == 0 && m.dst_stride % 4 == 0 && (((uintptr_t)m.dst | (uintptr_t)m.residual) & 15) == 0;
     }
+    wide = wide && (rows + 1023) / 1024 * B >= 256;   // a group per compute unit at least: 1024 rows, 64 activation rows, 16 slabs, the whole product 16.1 us by one, 16.6 by four elements per lane
     const int64_t per = wide ? 1024 : 256;
     const dim3 grid((unsigned)((rows + per - 1) / per), (unsigned)(B < MMQ_SUM_ROWS ? B : MMQ_SUM_ROWS));
     if (!wide) {
