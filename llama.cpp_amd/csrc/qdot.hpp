@@ -444,14 +444,14 @@ template <> struct wq<MI355_Q6_K> {
     static constexpr int CHUNK = 32;
     struct chunk { u32x4 ql, qh; float d, scA, scB; int shA, shB; };
     struct act { u32x4 a0, a1; float d0, d1; int s0, s1; };
-    struct raw { u32x4 ql, qh; int scA, scB; u32 d; };   // (see Q4_K)
+    struct raw { u32x4 ql, qh; u32 scA, scB, d; };   // (see Q4_K)
     static __device__ __forceinline__ raw load_raw(const uint8_t *__restrict__ row, const row_layout &L, int c) {
         raw w;
         const int sb = c >> 3, cc = c & 7, hf = cc >> 2, r = cc & 3;
         const int l0 = 16 * (r & 1), qa = r >> 1;
         w.ql = load_stream16w(row + sb * 128 + cc * 16);
         w.qh = load_stream16w(row + L.off_b + sb * 64 + hf * 32 + l0);
-        const int8_t *sc = (const int8_t *)(row + L.off_c + sb * 16 + hf * 8 + (l0 >> 4));
+        const uint8_t *sc = row + L.off_c + sb * 16 + hf * 8 + (l0 >> 4);
         w.scA = sc[2 * qa];
         w.scB = sc[2 * qa + 4];
         w.d = *(const unsigned short *)(row + L.off_d + sb * 2);
@@ -462,8 +462,8 @@ template <> struct wq<MI355_Q6_K> {
         const int qa = (c & 3) >> 1;
         w.ql = r.ql;
         w.qh = r.qh;
-        w.scA = (float)r.scA;
-        w.scB = (float)r.scB;
+        w.scA = (float)(int)(signed char)r.scA;
+        w.scB = (float)(int)(signed char)r.scB;
         w.d = half_bits_to_float((unsigned short)r.d);
         w.shA = 2 * qa;
         w.shB = 2 * qa + 4;
