@@ -464,34 +464,62 @@ def _tile_off(row, k, K):
     return ((row >> 4) * (K >> 6) + (k >> 6)) * 1024 + r * 64 + ((c ^ ((r >> 2) & 3)) << 4) + (k & 15)
 
 
-@pytest.mark.parametrize("t,N,K,B", [(orc.Q4_0, 768, 8192, 70), (orc.Q4_0, 4096, 4096, 130), (orc.Q6_K, 4096, 11008, 140), (orc.Q6_K, 1024, 2048, 65), (orc.Q4_K, 4096, 4096, 256),
-                                     (orc.Q4_K, 1536, 4096, 300), (orc.Q6_K, 1024, 14336, 200)])
-def test_slab_sums_by_four_and_by_one(dev, t, N, K, B):
-    """products cut along K into dst rows that allow 16-byte stores and into rows one float apart from that: the same sums, the same bits (and nothing between the rows is touched)"""
+def _slabs_written(ws, N, B):
+    """how many [B][N] slabs a product has left in a workspace that was NaN before"""
+    import torch
+    return int((~torch.isnan(ws)).sum().item()) / (N * B)
+
+
+@pytest.mark.parametrize("t,N,K,B,slabs", [(orc.Q4_0, 4096, 2048, 900, 2), (orc.Q6_K, 4096, 2048, 900, 2), (orc.Q4_0, 2688, 2048, 1000, 3), (orc.Q4_0, 4096, 2048, 130, 4),
+                                           (orc.Q4_0, 4096, 4096, 300, 5), (orc.Q4_0, 1028, 2048, 256, 8), (orc.Q6_K, 4096, 11008, 140, 8), (orc.Q4_0, 768, 8192, 70, 16),
+                                           (orc.Q6_K, 1024, 14336, 200, 16)])
+def test_slab_sums_by_four_and_by_one(dev, t, N, K, B, slabs):
+    """products cut along K into two, three, four and more slabs (counted), summed into dst rows that allow 16-byte stores and into rows one float apart from that (small ones by one
+    element per lane either way): the same bits, nothing between the rows is touched, and the values are the oracle's for these operands"""
     import torch
     import mi355
     lib = mi355.load()
     rng = np.random.default_rng(N + K + B)
-    Wd = mi355.upload_weights(t, _to_dev(dev, orc.quantize("oracle", t, (rng.standard_normal((N, K)) * 0.05).astype(np.float32))))
-    x = _to_dev(dev, rng.standard_normal((B, K)).astype(np.float32))
+    Wq = orc.quantize("oracle", t, (rng.standard_normal((N, K)) * 0.05).astype(np.float32))
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    Wd, act = mi355.upload_weights(t, _to_dev(dev, Wq)), mi355.quantize_act(_to_dev(dev, x))
     wide, odd = torch.full((B, N + 4), 7.0, device=dev), torch.full((B, N + 5), 7.0, device=dev)
-    need = lib.mi355_mul_mat_split_ws_bytes(N, K, B)
     for dst in (wide, odd):
-        ws = torch.zeros(need, dtype=torch.uint8, device=dev)
-        mi355.check(lib.mi355_mul_mat(None, t, Wd.data_ptr(), x.data_ptr(), dst.data_ptr(), N, K, B, K, dst.stride(0), ws.data_ptr(), ws.numel()))
+        ws = torch.full((20 * N * B,), float("nan"), device=dev)
+        mi355.check(lib.mi355_mul_mat_q_ws(None, t, Wd.data_ptr(), act.data_ptr(), dst.data_ptr(), N, K, B, dst.stride(0), ws.data_ptr(), ws.numel() * 4))
+        assert _slabs_written(ws, N, B) == slabs
     assert torch.equal(wide[:, :N], odd[:, :N]) and bool((wide[:, N:] == 7.0).all()) and bool((odd[:, N:] == 7.0).all())
-    assert bool(wide[:, :N].abs().sum() > 0)
-    if t == orc.Q4_0 or K % 2048 or not lib.mi355_mul_mat_q8k_tiled_ws_bytes(N, K, B): return
-    tiles = mi355.kq_unpack_tiles(t, Wd)
-    act = mi355.quantize_act_q8k_tiled(x)
-    res = [_to_dev(dev, rng.standard_normal((B, n)).astype(np.float32)) for n in (N + 4, N + 5)]
-    res[1][:, :N] = res[0][:, :N]
+    got = wide.cpu().numpy()
+    assert orc.nmse(got[:24, :64], orc.mul_mat("q8_1", t, Wq[:64], x[:24])) < 1e-11
+    assert orc.nmse(got[B - 3:, N - 9:N], orc.mul_mat("q8_1", t, Wq[N - 9:], x[B - 3:])) < 1e-11
+
+
+@pytest.mark.parametrize("t,N,K,B,slabs", [(orc.Q4_K, 4096, 4096, 300, 2), (orc.Q4_K, 3072, 2048, 300, 3), (orc.Q4_K, 1024, 2048, 65, 4), (orc.Q5_K, 3072, 8192, 130, 5),
+                                           (orc.Q4_K, 1536, 4096, 300, 6), (orc.Q6_K, 1024, 14336, 200, 8)])
+@pytest.mark.parametrize("add", [False, True])
+def test_slab_sums_of_tile_products(dev, t, N, K, B, slabs, add):
+    """the same for the products of tile images, with a residual that is dst itself and without"""
+    import torch
+    import mi355
+    lib = mi355.load()
+    assert lib.mi355_mul_mat_q8k_tiled_ws_bytes(N, K, B) == slabs * N * B * 4
+    rng = np.random.default_rng(N + K + B)
+    Wq = orc.quantize("oracle", t, (rng.standard_normal((N, K)) * 0.05).astype(np.float32))
+    x, res = (rng.standard_normal(shape).astype(np.float32) for shape in ((B, K), (B, N)))
+    tiles = mi355.kq_unpack_tiles(t, mi355.upload_weights(t, _to_dev(dev, Wq)))
+    act = mi355.quantize_act_q8k_tiled(_to_dev(dev, x))
     got = []
-    for r in res:   # in place: the residual is dst
-        ws = torch.zeros(lib.mi355_mul_mat_q8k_tiled_ws_bytes(N, K, B), dtype=torch.uint8, device=dev)
-        mi355.check(lib.mi355_mul_mat_q8k_tiled(None, t, tiles.data_ptr(), act.data_ptr(), r.data_ptr(), r.data_ptr(), N, K, B, r.stride(0), ws.data_ptr(), ws.numel()))
-        got.append(r[:, :N].cpu())
-    assert torch.equal(*got)
+    for pad in (4, 5):
+        dst = torch.full((B, N + pad), 7.0, device=dev)
+        dst[:, :N] = _to_dev(dev, res)
+        ws = torch.full((slabs * N * B,), float("nan"), device=dev)
+        mi355.check(lib.mi355_mul_mat_q8k_tiled(None, t, tiles.data_ptr(), act.data_ptr(), dst.data_ptr(), dst.data_ptr() if add else None, N, K, B, dst.stride(0), ws.data_ptr(),
+                                                ws.numel() * 4))
+        assert _slabs_written(ws, N, B) == slabs and bool((dst[:, N:] == 7.0).all())
+        got.append(dst[:, :N].cpu().numpy())
+    assert np.array_equal(*got)
+    for b, n in ((slice(0, 24), slice(0, 64)), (slice(B - 3, B), slice(N - 9, N))):
+        assert orc.nmse(got[0][b, n], orc.mul_mat("cpu", t, Wq[n], x[b]) + (res[b, n] if add else 0)) < 1e-9
 
 
 @pytest.mark.parametrize("K,B", [(256, 5), (4096, 33), (14336, 130)])
