@@ -57,11 +57,9 @@ template <int NB> struct mid_act {
 // the number of all, where there is none; rows: B and, from bit 8, five bits each for the rows of a matrix's last tile less one); destinations are read at the end.  Three trips for
 // them in a row ahead of the first request: 14336 x 4096, 64 rows 22.5 us a call, now 22.0, 128 rows 35.1, now 34.2.
 struct mid_mat {
-    const uint8_t *W;
     float *dst;
     const float *residual;   // may be null; same shape and stride as dst; may be dst itself
     int64_t N, dst_stride;
-    int first_tile;          // index of the matrix's first 32-row tile in the launch
 };
 struct mid_launch {
     mid_mat m[3];
@@ -392,6 +390,8 @@ static int mul_mat_mid_launch(void *stream, int type, int n_mats, const mi355_ge
     MI355_REQUIRE(mi355_act_q8k_tiled_bytes(K, B) < ((size_t)1 << 32), "mul_mat_mid: activation image of 4 GiB or more");
     int64_t n_sum = 0, tiles = 0;
     mid_launch L;
+    const uint8_t *Ws[3];
+    int64_t first[3];   // indices of the matrices' first 32-row tiles in the launch
     for (int i = 0; i < 3; i++) {
         const mi355_gemv_mat &m = mats[i < n_mats ? i : 0];
         if (i < n_mats) {
@@ -400,12 +400,12 @@ static int mul_mat_mid_launch(void *stream, int type, int n_mats, const mi355_ge
             MI355_REQUIRE(m.N > 0 && m.dst_stride >= m.N && m.N < (int64_t(1) << 31), "mul_mat_mid: bad shape N=%lld dst_stride=%lld", (long long)m.N, (long long)m.dst_stride);
             MI355_REQUIRE(m.N * (K / 256 * Q4_K_BYTES) < (int64_t(1) << 32), "mul_mat_mid: matrix of 4 GiB or more");
         }
-        L.m[i].W = (const uint8_t *)m.W;
+        Ws[i] = (const uint8_t *)m.W;
         L.m[i].dst = m.dst;
         L.m[i].residual = m.residual;
         L.m[i].N = m.N;
         L.m[i].dst_stride = m.dst_stride;
-        L.m[i].first_tile = (int)tiles;
+        first[i] = tiles;
         if (i < n_mats) {
             tiles += (m.N + 31) / 32;
             n_sum += m.N;
@@ -417,7 +417,7 @@ static int mul_mat_mid_launch(void *stream, int type, int n_mats, const mi355_ge
     hipStream_t s = (hipStream_t)stream;
     const int nsteps = (int)(K >> 8);
     const int steps_per_slice = (nsteps + slices - 1) / slices;
-    const int first1 = n_mats > 1 ? L.m[1].first_tile : (int)tiles, first2 = n_mats > 2 ? L.m[2].first_tile : (int)tiles;
+    const int first1 = (int)(n_mats > 1 ? first[1] : tiles), first2 = (int)(n_mats > 2 ? first[2] : tiles);
     u32 rows = (u32)B;
     for (int i = 0; i < n_mats; i++) rows |= (u32)((mats[i].N - 1) & 31) << (8 + 5 * i);
     const dim3 grid((unsigned)tiles, (unsigned)slices);
@@ -442,7 +442,7 @@ static int mul_mat_mid_launch(void *stream, int type, int n_mats, const mi355_ge
         }
     }
 #define MI355_MID_ARGS \
-    grid, dim3(256), 0, s, L.m[0].W, L.m[1].W, L.m[2].W, (const uint8_t *)act, first1, first2, (int)tiles, (int)K, rows, steps_per_slice, L
+    grid, dim3(256), 0, s, Ws[0], Ws[1], Ws[2], (const uint8_t *)act, first1, first2, (int)tiles, (int)K, rows, steps_per_slice, L
     if (B <= 32) MI355_LAUNCH((k_mm_mid_q4k<1, 1>), MI355_MID_ARGS);
     else if (B <= 64) MI355_LAUNCH((k_mm_mid_q4k<2, 1>), MI355_MID_ARGS);
     else MI355_LAUNCH((k_mm_mid_q4k<2, 2>), MI355_MID_ARGS);
