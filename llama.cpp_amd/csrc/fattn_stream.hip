@@ -148,7 +148,7 @@ __device__ __forceinline__ void fs_softmax(const float (&raw)[4], float mv, floa
         S.o0[r] *= f;
         S.o1[r] *= f;
         if constexpr (P32) {
-            *(float __attribute__((address_space(3))) *)(p_wr + (unsigned)(r * FS_TILE * 4)) = p;
+            *(float __attribute__((address_space(3))) *)(uintptr_t)(p_wr + (unsigned)(r * FS_TILE * 4)) = p;
         } else {
             const u32 ph = float_to_half_bits(p);
             asm volatile("ds_write_b16 %0, %1 offset:%2" ::"v"(p_wr), "v"(ph), "n"(r * FS_TILE * 2) : "memory");
@@ -923,7 +923,7 @@ __global__ void __launch_bounds__((P32 ? FSS_P32_WAVES : FSS_MAX_WAVES) * 64, P3
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // fs_output reads LDS through inline assembly: nothing may be moved across
     const unsigned v_addr = (unsigned)(uintptr_t)(void __attribute__((address_space(3))) *)tb + fs_v_lane(lane), p_rd = p_base + (unsigned)(lane & 3) * (FS_TILE * 2);
     if constexpr (P32)
-        fs_output_f32<NH>((const uint8_t __attribute__((address_space(3))) *)(v_addr + (unsigned)(part * 128)), (const float __attribute__((address_space(3))) *)p_base, lane, S.o0);
+        fs_output_f32<NH>((const uint8_t __attribute__((address_space(3))) *)(uintptr_t)(v_addr + (unsigned)(part * 128)), (const float __attribute__((address_space(3))) *)(uintptr_t)p_base, lane, S.o0);
     else if constexpr (PARTS == 1) fs_output(v_addr, p_rd, S);
     else if (part == 0) fs_output_half<0>(v_addr, p_rd, S.o0);   // uniform
     else fs_output_half<1>(v_addr, p_rd, S.o0);
