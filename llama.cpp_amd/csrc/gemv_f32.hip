@@ -53,7 +53,6 @@ __global__ void __launch_bounds__(GF_WAVES * 64) k_gemv_f32(const uint8_t *__res
         for (int col = 0; col < NCOLS; col++)
 #pragma unroll
             for (int i = 0; i < PIECES; i++) {
-                if (k0 + i * STEP >= K) continue;   // uniform
                 const int k = k0 + i * STEP + (int)threadIdx.x * 4;
                 quantize_block_lane(v[col][i], k < K, s_q, s_ds, col, K, k);
             }
