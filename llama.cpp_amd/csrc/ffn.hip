@@ -27,8 +27,8 @@ constexpr int gu_rows_in_flight(int type, int ncols) {
 }
 // Rows are used in the order their loads return, and a register goes to its row's next step or round as soon as it is used.  Not for one token of the other types, whose step is
 // some twenty instructions: requesting a step's rows together when the one before is done is as fast or faster there (28672 x 8192, us: Q4_0 41.4 against 42.4, Q8_0 84.9 against
-// 88.1, IQ4_XS 48.5 against 54.4), and for two of Q4_0 (14336 x 4096 14.9 against 15.3).
-constexpr bool gu_ahead(int type, int ncols) { return (ncols > 1 && !(type == MI355_Q4_0 && ncols == 2)) || type == MI355_Q4_K || type == MI355_Q5_K || type == MI355_Q6_K; }
+// 88.1, IQ4_XS 48.5 against 54.4).
+constexpr bool gu_ahead(int type, int ncols) { return ncols > 1 || type == MI355_Q4_K || type == MI355_Q5_K || type == MI355_Q6_K; }
 
 // Wave w of the group: rows 32 b + RPM w .. + RPM - 1 of gate and of up (RPM = 32 / WAVES), R rows of each in flight; the
 // block's 32 values of every activation row meet in s_g / s_u and are quantized by the group's first lanes.  The activation is
