@@ -270,10 +270,6 @@ __device__ __forceinline__ void rms_norm_quant_row(const float *__restrict__ xr,
     const float scale = rms_norm_scale<NV>(v, k, eps, sh);
 #pragma unroll
     for (int it = 0; it < NV; it++) {
-        if ((int64_t)it * 1024 >= k) {   // uniform
-            if (keep) keep[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-            continue;
-        }
         const f32x4 o = norm_piece<FMT>(v[it], ww[it], w != nullptr, scale, yr, act, row, k, nrows, ((int64_t)it * 256 + tid) * 4);
         if (keep) keep[it] = o;
     }
