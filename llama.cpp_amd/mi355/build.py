@@ -24,11 +24,7 @@ KERNEL_SOURCES = ["quantize.hip", "wquant.hip", "gemv.hip", "gemv_qkv.hip", "gem
 
 # -packed-fp32-ops: keep hipcc from forming packed-FP32 instructions out of scalar float code
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
-               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-# Arguments in scalar registers when a wave starts: one trip to memory less ahead of a kernel's first request.  Not where it was measured to cost more: the Q8_1 quantizer
-# (4096 elements, 1 .. 33 rows: 2.2 us in a chain of launches with it, 2.08 without) and the product of a few rows (quantizer included, 14336 x 4096, 5 rows: Q4_0 10.1 / 9.9, Q4_K 10.8 / 10.5).
-PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
-NO_PRELOAD = {"quantize.hip", "skinny.hip"}
+               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 
 def _hipcc():
@@ -58,7 +54,7 @@ def build_kernels(verbose=True):
 
     def compile_one(src):
         obj = os.path.join(OBJ, src.replace(".hip", ".o"))
-        _run([_hipcc()] + HIPCC_FLAGS + ([] if src in NO_PRELOAD else PRELOAD) + ["-I", os.path.join(ROOT, "include"), "-c", os.path.join(CSRC, src), "-o", obj])
+        _run([_hipcc()] + HIPCC_FLAGS + ["-I", os.path.join(ROOT, "include"), "-c", os.path.join(CSRC, src), "-o", obj])
         return obj
 
     with ThreadPoolExecutor(max_workers=min(8, len(KERNEL_SOURCES))) as ex:
